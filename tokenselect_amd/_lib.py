@@ -149,6 +149,26 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_bind = None
+
+
+def binding():
+    """The native host path of the layer objects (``csrc/bind/ts_bind.cpp``), connected to the
+    loaded library."""
+    global _bind
+    if _bind is None:
+        lib = load()
+        try:
+            from . import _ts_bind
+        except ImportError as e:
+            raise ImportError(f"the Python binding next to {LIB_PATH} is missing or does not load ({e}): "
+                              "build it with `python -m tokenselect_amd.build`") from e
+        _ts_bind.connect(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in
+                           ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step")))
+        _bind = _ts_bind
+    return _bind
+
+
 def check(code: int) -> None:
     if code != TS_OK:
         raise TokenSelectError(code, load().ts_last_error().decode("utf-8", "replace"))

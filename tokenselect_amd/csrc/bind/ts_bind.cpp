@@ -1,0 +1,486 @@
+// The per-call host work of ops.DecodeLayer and ops.PrefillChunk in native code: checks the
+// tensors, fills the structs of include/tokenselect.h and calls the library on the current
+// stream.
+//
+// A layer call is a few microseconds of kernel launches; the same checks and ctypes structs
+// in Python took 25 us around them, longer than the kernels of a short context run (8 layers
+// of a 2003-token request, 16 calls: 577 us a pass, of which the GPU was busy 290).  Nothing
+// is computed here and nothing is kept between calls but the buffers the object owns and the
+// shape its workspace was last left clean for.
+//
+// Built with the host compiler against PyTorch's headers; the library's entry points are
+// handed over as addresses by _lib.py, so that there is one loaded copy of it.
+#include <Python.h>
+
+#include <ATen/ops/empty_like.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+#include <exception>
+#include <string>
+
+#include "../../../include/tokenselect.h"
+
+namespace {
+
+// A Python exception is set; unwinds to the method's end.
+struct Raised {};
+[[noreturn]] void raise(PyObject* type, const std::string& text) {
+  PyErr_SetString(type, text.c_str());
+  throw Raised{};
+}
+[[noreturn]] void bad_value(const std::string& text) { raise(PyExc_ValueError, text); }
+
+// An owned reference.
+struct Ref {
+  PyObject* p;
+  explicit Ref(PyObject* o) : p(o) {
+    if (!p) throw Raised{};
+  }
+  ~Ref() { Py_XDECREF(p); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+};
+
+const char* dtype_name(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return "torch.bfloat16";
+    case at::kInt: return "torch.int32";
+    case at::kLong: return "torch.int64";
+    default: return at::toString(t);
+  }
+}
+
+std::string shape_text(const at::Tensor& t) {
+  std::string s = "(";
+  for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+  return s + (t.dim() == 1 ? ",)" : ")");
+}
+
+const at::Tensor& tensor(PyObject* o, const char* name) {
+  if (!THPVariable_Check(o)) raise(PyExc_TypeError, std::string(name) + " must be a torch.Tensor");
+  return THPVariable_Unpack(o);
+}
+
+// A tensor on the GPU of the given type; ndim < 0: any number of dims.
+const at::Tensor& need(PyObject* o, const char* name, at::ScalarType dtype, int ndim = -1) {
+  const at::Tensor& t = tensor(o, name);
+  if (t.scalar_type() != dtype)
+    raise(PyExc_TypeError, std::string(name) + " must be " + dtype_name(dtype) + ", got " + dtype_name(t.scalar_type()));
+  if (!t.is_cuda())
+    bad_value(std::string(name) + " must live on the GPU (got " + t.device().str() + "); there is no CPU path");
+  if (!t.is_contiguous()) bad_value(std::string(name) + " must be contiguous");
+  if (ndim >= 0 && t.dim() != ndim)
+    bad_value(std::string(name) + " must have " + std::to_string(ndim) + " dims, got shape " + shape_text(t));
+  return t;
+}
+
+// Attribute names of Batch, SelectionCache and PagePool, interned once.
+#define TS_NAMES(X)                                                                              \
+  X(seq_lens) X(table) X(max_seq_len) X(k_per_req) X(fault) X(host_seq_lens) X(hint)             \
+  X(separate_kernels) X(rerun) X(wait_us) X(absent_workgroups) X(workspace_clean)                \
+  X(q_cache) X(topk_cache) X(cache_len) X(counters) X(threshold)                                 \
+  X(free_pages) X(free_count) X(ticket)
+#define TS_DECLARE(n) PyObject* n_##n;
+TS_NAMES(TS_DECLARE)
+#undef TS_DECLARE
+
+bool intern_names() {
+#define TS_INTERN(n) \
+  if (!(n_##n = PyUnicode_InternFromString(#n))) return false;
+  TS_NAMES(TS_INTERN)
+#undef TS_INTERN
+  return true;
+}
+
+PyObject* attr(PyObject* o, PyObject* name) {
+  PyObject* v = PyObject_GetAttr(o, name);
+  if (!v) throw Raised{};
+  return v;
+}
+long as_long(PyObject* o) {
+  if (!PyLong_Check(o)) {  // (what int() takes: a numpy integer, a one-element tensor)
+    const Ref number(PyNumber_Long(o));
+    return as_long(number.p);
+  }
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw Raised{};
+  return v;
+}
+long long_attr(PyObject* o, PyObject* name) {
+  const Ref v(attr(o, name));
+  return as_long(v.p);
+}
+bool bool_attr(PyObject* o, PyObject* name) {
+  const Ref v(attr(o, name));
+  const int b = PyObject_IsTrue(v.p);
+  if (b < 0) throw Raised{};
+  return b != 0;
+}
+
+using StepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, const float*, const float*,
+                       void*, void*, int64_t, const ts_selcache*, void*, int32_t*, int32_t*, int64_t, int32_t*,
+                       void*, size_t, ts_stream_t);
+using LayerFn = int (*)(const ts_config*, const ts_batch*, const void*, const float*, const float*, const void*,
+                        const void*, int64_t, const ts_selcache*, void*, int32_t*, int32_t*, int64_t, int32_t*,
+                        void*, size_t, ts_stream_t);
+using ChunkStepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, int32_t, const float*,
+                            const float*, int64_t, void*, void*, int64_t, void*, int32_t*, int32_t*, int64_t,
+                            int32_t*, void*, size_t, ts_stream_t);
+using ChunkFn = int (*)(const ts_config*, const ts_batch*, const void*, int32_t, const float*, const float*, int64_t,
+                        const void*, const void*, int64_t, void*, int32_t*, int32_t*, int64_t, int32_t*, void*,
+                        size_t, ts_stream_t);
+StepFn decode_step;
+LayerFn decode_layer;
+ChunkStepFn prefill_step;
+ChunkFn prefill_chunk;
+
+// What a DecodeLayer (max_rows == 0) or a PrefillChunk owns.
+struct Owned {
+  ts_config cfg;
+  at::Tensor workspace, cos, sin, out, sel, sel_pos, sel_len, fault;
+  int64_t batch, max_seq_len, max_rows;
+  // (batch, max_seq_len) that the selection's counters in the workspace are clean for, -1: none.
+  int64_t clean_batch = -1, clean_len = -1;
+  // The outputs' rows of the last batch size: out, sel, sel_pos, sel_len.
+  int64_t rows_of = -1;
+  PyObject* rows[4] = {nullptr, nullptr, nullptr, nullptr};
+  void forget_rows() {
+    for (PyObject*& r : rows) Py_CLEAR(r);
+    rows_of = -1;
+  }
+};
+
+struct Runner {
+  PyObject_HEAD
+  Owned* own;
+};
+
+uint32_t fault_of(const Owned& o) { return *(const volatile uint32_t*)o.fault.data_ptr(); }
+
+const at::Tensor& check_pool(const ts_config& cfg, PyObject* o, const char* name) {
+  const at::Tensor& t = need(o, name, at::kBFloat16, 3);
+  if (t.size(1) != cfg.num_kv_heads || t.size(2) != cfg.head_dim)
+    bad_value(std::string(name) + " must be [rows, " + std::to_string(cfg.num_kv_heads) + ", " +
+              std::to_string(cfg.head_dim) + "], got " + shape_text(t));
+  return t;
+}
+
+// The options of a call, from a Batch and the object's own state.
+struct Call {
+  ts_batch bt{};
+  const at::Tensor* table = nullptr;
+};
+
+void fill_batch(const Owned& o, PyObject* b, bool separate, bool rerun, Call* call) {
+  ts_batch& c = call->bt;
+  const Ref lens_ref(attr(b, n_seq_lens)), table_ref(attr(b, n_table)), k_ref(attr(b, n_k_per_req)),
+      fault_ref(attr(b, n_fault)), host_ref(attr(b, n_host_seq_lens)), hint_ref(attr(b, n_hint));
+  // (the Batch holds the tensors: the references below outlive this function)
+  const at::Tensor& lens = need(lens_ref.p, "seq_lens", at::kInt, 1);
+  const at::Tensor& table = need(table_ref.p, "table", at::kInt, 2);
+  const int64_t B = lens.size(0);
+  const int64_t max_len = long_attr(b, n_max_seq_len);
+  if (table.size(0) != B) bad_value("table must have one row per request");
+  if (table.size(1) * o.cfg.page_size < max_len)
+    bad_value("table row of " + std::to_string(table.size(1)) + " pages (page_size " +
+              std::to_string(o.cfg.page_size) + ") cannot address max_seq_len " + std::to_string(max_len));
+  c.batch = (int32_t)B;
+  c.max_seq_len = (int32_t)max_len;
+  c.seq_lens = (const int32_t*)lens.data_ptr();
+  c.table = (const int32_t*)table.data_ptr();
+  c.table_stride = table.stride(0);
+  if (k_ref.p != Py_None) {
+    const at::Tensor& k = need(k_ref.p, "k_per_req", at::kInt, 1);
+    if (k.size(0) != B) bad_value("k_per_req must have one entry per request");
+    c.k_per_req = (const int32_t*)k.data_ptr();
+  }
+  if (fault_ref.p == Py_None) {
+    c.fault = (uint32_t*)o.fault.data_ptr();
+  } else {
+    const at::Tensor& f = tensor(fault_ref.p, "fault");
+    if (f.scalar_type() != at::kInt || f.numel() != 1 || !(f.is_cuda() || f.is_pinned()))
+      bad_value("fault must be one int32 word of device or pinned host memory");
+    c.fault = (uint32_t*)f.data_ptr();
+  }
+  if (host_ref.p != Py_None) {
+    const at::Tensor& h = tensor(host_ref.p, "host_seq_lens");
+    if (h.scalar_type() != at::kInt || h.is_cuda() || h.dim() != 1 || h.size(0) != B || !h.is_contiguous())
+      bad_value("host_seq_lens must be a contiguous [B] int32 tensor on the CPU");
+    c.host_seq_lens = (const int32_t*)h.data_ptr();
+  }
+  if (hint_ref.p != Py_None) {
+    const at::Tensor& h = need(hint_ref.p, "hint", at::kInt, 1);
+    if (h.size(0) != B) bad_value("hint must have one entry per request");
+    c.threshold_hint = (int32_t*)h.data_ptr();
+  }
+  c.separate_kernels = (separate || bool_attr(b, n_separate_kernels)) ? 1 : 0;
+  c.rerun = (rerun || bool_attr(b, n_rerun)) ? 1 : 0;
+  c.wait_us = (uint32_t)long_attr(b, n_wait_us);
+  c.absent_workgroups = rerun ? 0 : (int32_t)long_attr(b, n_absent_workgroups);
+  c.workspace_clean = bool_attr(b, n_workspace_clean) ? 1 : 0;
+  if (B > o.batch || max_len > o.max_seq_len) {
+    if (o.max_rows > 0) bad_value("one request, within the sizes this PrefillChunk was built for");
+    bad_value("batch / max_seq_len exceed what this DecodeLayer was sized for");
+  }
+  call->table = &table;
+}
+
+void fill_cache(const ts_config& cfg, PyObject* cache, int64_t B, ts_selcache* c) {
+  const Ref q_ref(attr(cache, n_q_cache)), top_ref(attr(cache, n_topk_cache)), len_ref(attr(cache, n_cache_len)),
+      cnt_ref(attr(cache, n_counters)), thr_ref(attr(cache, n_threshold));
+  const at::Tensor& q = need(q_ref.p, "q_cache", at::kBFloat16, 2);
+  const at::Tensor& top = need(top_ref.p, "topk_cache", at::kInt, 2);
+  const at::Tensor& len = need(len_ref.p, "cache_len", at::kInt, 1);
+  const at::Tensor& cnt = need(cnt_ref.p, "counters", at::kLong, 2);
+  if (q.size(0) != B || q.size(1) != (int64_t)cfg.num_heads * cfg.head_dim || top.size(0) != B ||
+      top.size(1) != cfg.top_k || len.size(0) != B || cnt.size(0) != B || cnt.size(1) != 2)
+    bad_value("selection cache arrays do not match batch / config");
+  const double threshold = PyFloat_AsDouble(thr_ref.p);
+  if (threshold == -1.0 && PyErr_Occurred()) throw Raised{};
+  *c = ts_selcache{q.data_ptr(), (int32_t*)top.data_ptr(), (int32_t*)len.data_ptr(), (int64_t*)cnt.data_ptr(),
+                   (float)threshold};
+}
+
+void fill_pages(PyObject* pages, ts_page_pool* c) {
+  const Ref list_ref(attr(pages, n_free_pages)), count_ref(attr(pages, n_free_count)), ticket_ref(attr(pages, n_ticket));
+  *c = ts_page_pool{(const int32_t*)need(list_ref.p, "free_pages", at::kInt, 1).data_ptr(),
+                    (int32_t*)need(count_ref.p, "free_count", at::kInt, 1).data_ptr(),
+                    (uint32_t*)need(ticket_ref.p, "ticket", at::kInt, 1).data_ptr()};
+}
+
+PyObject* row_view(const at::Tensor& t, int64_t B) {
+  PyObject* v = THPVariable_Wrap(t.narrow(0, 0, B));
+  if (!v) throw Raised{};
+  return v;
+}
+
+// run(q, k, v, out_cache_loc, k_pool, v_pool, bt, cache, out, pages, store, separate, rerun):
+// the layer (store false) or the step; None when an earlier call's selection gave up (not with
+// rerun), an error code of the library as an int, or (out, sel, sel_pos, sel_len).
+PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 13) raise(PyExc_TypeError, "run() takes 13 arguments");
+  Owned& o = *self->own;
+  PyObject *q_o = args[0], *k_o = args[1], *v_o = args[2], *loc_o = args[3], *kp_o = args[4], *vp_o = args[5],
+           *bt_o = args[6], *cache_o = args[7], *out_o = args[8], *pages_o = args[9];
+  const bool store = args[10] == Py_True, separate = args[11] == Py_True, rerun = args[12] == Py_True;
+  if (!rerun && fault_of(o) != 0) Py_RETURN_NONE;
+  const bool chunk = o.max_rows > 0;
+  const ts_config& cfg = o.cfg;
+  const int64_t width = (int64_t)cfg.num_heads * cfg.head_dim, row = (int64_t)cfg.num_kv_heads * cfg.head_dim;
+
+  Call call;
+  fill_batch(o, bt_o, separate, rerun, &call);
+  ts_batch& bt = call.bt;
+  const int64_t B = bt.batch;
+  const at::Tensor& q = need(q_o, "q", at::kBFloat16, chunk ? 2 : -1);
+  int64_t rows = B;
+  if (chunk) {
+    rows = q.size(0);
+    if (B != 1 || rows > o.max_rows) bad_value("one request, within the sizes this PrefillChunk was built for");
+    if (q.size(1) != width) bad_value("q must be [rows, H*D]");
+  } else if (q.numel() != B * width) {
+    bad_value("q must hold B*H*D elements");
+  }
+  const at::Tensor& k_pool = check_pool(cfg, kp_o, "k_pool");
+  const at::Tensor& v_pool = check_pool(cfg, vp_o, "v_pool");
+  if (!chunk && k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
+
+  ts_new_kv kv{};
+  ts_page_pool pool{};
+  if (store) {
+    const at::Tensor& k = need(k_o, "k", at::kBFloat16);
+    const at::Tensor& v = need(v_o, "v", at::kBFloat16);
+    int64_t slots = rows;
+    if (pages_o != Py_None) {
+      fill_pages(pages_o, &pool);
+      kv.pages = &pool;
+    } else {
+      if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
+      const at::Tensor& loc = need(loc_o, "out_cache_loc", at::kInt, 1);
+      slots = loc.size(0);
+      kv.out_cache_loc = (const int32_t*)loc.data_ptr();
+    }
+    if (k.numel() != rows * row || v.numel() != rows * row || slots != rows)
+      bad_value(chunk ? "k / v / out_cache_loc / table do not match the chunk"
+                      : "k / v / out_cache_loc / table do not match the batch");
+    kv.k = k.data_ptr();
+    kv.v = v.data_ptr();
+    kv.max_tokens = (int32_t)(call.table->size(1) * cfg.page_size);
+  }
+
+  ts_selcache cache{};
+  const bool cached = cache_o != Py_None;
+  if (cached) fill_cache(cfg, cache_o, B, &cache);
+
+  if (o.rows_of != B) {
+    o.forget_rows();
+    if (!chunk) o.rows[0] = row_view(o.out, B);
+    o.rows[1] = row_view(o.sel, B);
+    o.rows[2] = row_view(o.sel_pos, B);
+    o.rows[3] = row_view(o.sel_len, B);
+    o.rows_of = B;
+  }
+  PyObject* out_py;
+  void* out_ptr;
+  if (out_o != Py_None) {
+    const at::Tensor& t = need(out_o, "out", at::kBFloat16);
+    if (t.numel() != q.numel()) bad_value(chunk ? "out must hold rows*H*D elements" : "out must hold B*H*D elements");
+    out_ptr = t.data_ptr();
+    out_py = out_o;
+    Py_INCREF(out_py);
+  } else if (chunk) {
+    at::Tensor t = at::empty_like(q);
+    out_ptr = t.data_ptr();
+    out_py = THPVariable_Wrap(std::move(t));
+    if (!out_py) throw Raised{};
+  } else {
+    out_ptr = o.out.data_ptr();
+    out_py = o.rows[0];
+    Py_INCREF(out_py);
+  }
+  const Ref out_ref(out_py);
+
+  // The attention kernel of a plain call leaves the selection's counters zero for the next
+  // one of the same shape.
+  const bool plain = !chunk && !cached && !bt.separate_kernels && !rerun;
+  if (plain && o.clean_batch == B && o.clean_len == bt.max_seq_len) bt.workspace_clean = 1;
+  o.clean_batch = o.clean_len = -1;
+
+  const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
+  const float *cos = (const float*)o.cos.data_ptr(), *sin = (const float*)o.sin.data_ptr();
+  int32_t *sel = (int32_t*)o.sel.data_ptr(), *sel_pos = (int32_t*)o.sel_pos.data_ptr(),
+          *sel_len = (int32_t*)o.sel_len.data_ptr();
+  const int64_t sel_stride = o.sel.size(1), table_rows = o.cos.size(0), pool_rows = k_pool.size(0);
+  void *kp = k_pool.data_ptr(), *vp = v_pool.data_ptr(), *ws = o.workspace.data_ptr();
+  const void* qp = q.data_ptr();
+  const size_t ws_bytes = (size_t)o.workspace.numel();
+  const ts_selcache* cp = cached ? &cache : nullptr;
+  int code;
+  Py_BEGIN_ALLOW_THREADS
+  if (chunk)
+    code = store ? prefill_step(&cfg, &bt, &kv, qp, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out_ptr, sel,
+                                sel_pos, sel_stride, sel_len, ws, ws_bytes, stream)
+                 : prefill_chunk(&cfg, &bt, qp, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out_ptr, sel,
+                                 sel_pos, sel_stride, sel_len, ws, ws_bytes, stream);
+  else
+    code = store ? decode_step(&cfg, &bt, &kv, qp, cos, sin, kp, vp, pool_rows, cp, out_ptr, sel, sel_pos, sel_stride,
+                               sel_len, ws, ws_bytes, stream)
+                 : decode_layer(&cfg, &bt, qp, cos, sin, kp, vp, pool_rows, cp, out_ptr, sel, sel_pos, sel_stride,
+                                sel_len, ws, ws_bytes, stream);
+  Py_END_ALLOW_THREADS
+  if (code != TS_OK) return PyLong_FromLong(code);
+  if (plain) {
+    o.clean_batch = B;
+    o.clean_len = bt.max_seq_len;
+  }
+  return PyTuple_Pack(4, out_py, o.rows[1], o.rows[2], o.rows[3]);
+}
+
+// Runs `f`, with C++ exceptions turned into Python's.
+template <typename F>
+PyObject* guarded(F&& f) {
+  try {
+    return f();
+  } catch (const Raised&) {
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+  }
+  return nullptr;
+}
+
+PyObject* runner_run(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&] { return run((Runner*)self, args, nargs); });
+}
+
+PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  Py_buffer cfg;
+  PyObject *ws, *cos, *sin, *out, *sel, *sel_pos, *sel_len, *fault;
+  long long batch, max_seq_len, max_rows;
+  if (!PyArg_ParseTuple(args, "y*OOOOOOOOLLL", &cfg, &ws, &cos, &sin, &out, &sel, &sel_pos, &sel_len, &fault, &batch,
+                        &max_seq_len, &max_rows))
+    return nullptr;
+  PyObject* made = guarded([&]() -> PyObject* {
+    if (cfg.len != (Py_ssize_t)sizeof(ts_config)) bad_value("config of another size");
+    Ref self(type->tp_alloc(type, 0));
+    Owned* o = new Owned();
+    ((Runner*)self.p)->own = o;
+    memcpy(&o->cfg, cfg.buf, sizeof(ts_config));
+    o->workspace = tensor(ws, "workspace");
+    o->cos = tensor(cos, "cos");
+    o->sin = tensor(sin, "sin");
+    if (out != Py_None) o->out = tensor(out, "out");
+    o->sel = tensor(sel, "sel");
+    o->sel_pos = tensor(sel_pos, "sel_pos");
+    o->sel_len = tensor(sel_len, "sel_len");
+    o->fault = tensor(fault, "fault");
+    o->batch = batch;
+    o->max_seq_len = max_seq_len;
+    o->max_rows = max_rows;
+    Py_INCREF(self.p);
+    return self.p;
+  });
+  PyBuffer_Release(&cfg);
+  return made;
+}
+
+void runner_dealloc(PyObject* self) {
+  Owned* o = ((Runner*)self)->own;
+  if (o) {
+    o->forget_rows();
+    delete o;
+  }
+  PyTypeObject* type = Py_TYPE(self);
+  type->tp_free(self);
+  Py_DECREF(type);
+}
+
+PyObject* get_clean(PyObject* self, void*) {
+  const Owned& o = *((Runner*)self)->own;
+  if (o.clean_batch < 0) Py_RETURN_NONE;
+  return Py_BuildValue("(LL)", (long long)o.clean_batch, (long long)o.clean_len);
+}
+int set_clean(PyObject* self, PyObject* value, void*) {
+  Owned& o = *((Runner*)self)->own;
+  long long b = -1, n = -1;
+  if (value != Py_None && !(value && PyArg_ParseTuple(value, "LL", &b, &n))) return -1;
+  o.clean_batch = b;
+  o.clean_len = n;
+  return 0;
+}
+
+PyMethodDef runner_methods[] = {
+    {"run", (PyCFunction)(void (*)(void))runner_run, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyGetSetDef runner_getset[] = {{"clean", get_clean, set_clean, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyType_Slot runner_slots[] = {{Py_tp_new, (void*)runner_new}, {Py_tp_dealloc, (void*)runner_dealloc},
+                              {Py_tp_methods, runner_methods}, {Py_tp_getset, runner_getset}, {0, nullptr}};
+PyType_Spec runner_spec = {"_ts_bind.Runner", sizeof(Runner), 0, Py_TPFLAGS_DEFAULT, runner_slots};
+
+// connect(addresses): the library's entry points, in this order.
+PyObject* connect(PyObject*, PyObject* args) {
+  unsigned long long a, b, c, d;
+  if (!PyArg_ParseTuple(args, "KKKK", &a, &b, &c, &d)) return nullptr;
+  decode_layer = (LayerFn)(uintptr_t)a;
+  decode_step = (StepFn)(uintptr_t)b;
+  prefill_chunk = (ChunkFn)(uintptr_t)c;
+  prefill_step = (ChunkStepFn)(uintptr_t)d;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {{"connect", connect, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_ts_bind", nullptr, -1, module_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__ts_bind(void) {
+  if (!intern_names()) return nullptr;
+  PyObject* m = PyModule_Create(&module_def);
+  PyObject* type = m ? PyType_FromSpec(&runner_spec) : nullptr;
+  if (!type || PyModule_AddObject(m, "Runner", type) < 0) {
+    Py_XDECREF(type);
+    Py_XDECREF(m);
+    return nullptr;
+  }
+  return m;
+}

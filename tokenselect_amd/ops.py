@@ -150,16 +150,27 @@ class _GiveUpLatch:
             self._latch()
             raise SelectionGaveUp(_GAVE_UP_MESSAGE + "; this object now uses the separate kernels")
 
-    def _options(self, bt: "Batch", rerun: bool = False) -> "Batch":
+    def _options(self, bt: "Batch") -> "Batch":
         kw = {}
         if bt.fault is None:
             kw["fault"] = self.fault
         if self.separate and not bt.separate_kernels:
             kw["separate_kernels"] = True
-        if rerun:
-            kw["rerun"] = True
-            kw["absent_workgroups"] = 0
         return dataclasses.replace(bt, **kw) if kw else bt
+
+    def _init_native(self, cos, sin, out, batch: int, max_rows: int):
+        """The object's buffers handed to the native host path (``_lib.binding()``)."""
+        self._native = _lib.binding().Runner(bytes(self._c), self.workspace, cos, sin, out, self.sel,
+                                             self.sel_pos, self.sel_len, self.fault, batch,
+                                             self.max_seq_len, max_rows)
+
+    def _run(self, q, k, v, loc, k_pool, v_pool, bt, cache, out, pages, store: bool, rerun: bool = False):
+        got = self._native.run(q, k, v, loc, k_pool, v_pool, bt, cache, out, pages, store, self.separate, rerun)
+        if type(got) is tuple:
+            return got
+        if got is None:   # an earlier call gave up
+            self.check()
+        _lib.check(got)
 
 
 @dataclass
@@ -730,11 +741,19 @@ class DecodeLayer(_GiveUpLatch):
         self.sel_pos = torch.empty_like(self.sel)
         self.sel_len = torch.empty((batch,), dtype=torch.int32, device=device)
         self._init_latch()
-        # (batch, max_seq_len) of the last call when it was a plain layer call without a
-        # selection cache that raised nothing: that call's attention kernel has left the
-        # selection's counters zero, and the next call of the same shape says so
-        # (``ts_batch.workspace_clean``) and starts with the selection kernel.
-        self._clean_for = None
+        self._init_native(self.q_cos, self.q_sin, self.out, batch, 0)
+
+    @property
+    def _clean_for(self):
+        """(batch, max_seq_len) of the last call when it was a plain layer call without a
+        selection cache that raised nothing: that call's attention kernel has left the
+        selection's counters zero, and the next call of the same shape says so
+        (``ts_batch.workspace_clean``) and starts with the selection kernel."""
+        return self._native.clean
+
+    @_clean_for.setter
+    def _clean_for(self, shape):
+        self._native.clean = shape
 
     def recover(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                 cache: Optional[SelectionCache] = None, out: Optional[torch.Tensor] = None):
@@ -747,12 +766,11 @@ class DecodeLayer(_GiveUpLatch):
         if not self.gave_up():
             return None
         self._latch()
-        return self._run(q, k_pool, v_pool, bt, cache, out, rerun=True)
+        return self._run(q, None, None, None, k_pool, v_pool, bt, cache, out, None, False, rerun=True)
 
     def __call__(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                  cache: Optional[SelectionCache] = None, out: Optional[torch.Tensor] = None):
-        self.check()
-        return self._run(q, k_pool, v_pool, bt, cache, out)
+        return self._run(q, None, None, None, k_pool, v_pool, bt, cache, out, None, False)
 
     def step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_cache_loc: Optional[torch.Tensor],
              k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch, cache: Optional[SelectionCache] = None,
@@ -763,62 +781,7 @@ class DecodeLayer(_GiveUpLatch):
         the append, which ``bt.max_seq_len`` and ``bt.host_seq_lens`` must bound.  Same
         results as the two calls; with a selection cache the store rides in the layer's
         first launch."""
-        self.check()
-        cfg = self.cfg
-        _need(k, "k", torch.bfloat16)
-        _need(v, "v", torch.bfloat16)
-        loc, pool, _keep = _c_pages(cfg, out_cache_loc, pages)
-        _need(bt.table, "table", torch.int32, 2)
-        B = bt.batch
-        row = cfg.num_kv_heads * cfg.head_dim
-        if k.numel() != B * row or v.numel() != B * row or bt.table.shape[0] != B or \
-                (pages is None and out_cache_loc.shape[0] != B):
-            raise ValueError("k / v / out_cache_loc / table do not match the batch")
-        kv = _lib.TsNewKv(_p(k), _p(v), loc, ctypes.pointer(_keep) if pages is not None else None,
-                          bt.table.shape[1] * cfg.page_size)
-        kv._pool = _keep  # (the struct the pointer refers to lives as long as kv)
-        return self._run(q, k_pool, v_pool, bt, cache, out, new_kv=kv)
-
-    def _run(self, q, k_pool, v_pool, bt, cache, out, rerun: bool = False, new_kv=None):
-        cfg = self.cfg
-        bt = self._options(bt, rerun)
-        shape = (bt.batch, int(bt.max_seq_len))
-        plain = cache is None and not bt.separate_kernels and not rerun
-        if plain and self._clean_for == shape and not bt.workspace_clean:
-            bt = dataclasses.replace(bt, workspace_clean=True)
-        self._clean_for = None
-        cb = _c_batch(cfg, bt)
-        if bt.batch > self.batch or bt.max_seq_len > self.max_seq_len:
-            raise ValueError("batch / max_seq_len exceed what this DecodeLayer was sized for")
-        _need(q, "q", torch.bfloat16)
-        B = bt.batch
-        if q.numel() != B * cfg.num_heads * cfg.head_dim:
-            raise ValueError("q must hold B*H*D elements")
-        _check_pool(cfg, k_pool, "k_pool")
-        _check_pool(cfg, v_pool, "v_pool")
-        if k_pool.shape != v_pool.shape:
-            raise ValueError("k_pool and v_pool must have the same shape")
-        if out is None:
-            out = self.out[:B]
-        else:
-            _need(out, "out", torch.bfloat16)
-            if out.numel() != q.numel():
-                raise ValueError("out must hold B*H*D elements")
-        if new_kv is not None:
-            _lib.check(_lib.load().ts_decode_step(
-                ctypes.byref(self._c), ctypes.byref(cb), ctypes.byref(new_kv), _p(q), _p(self.q_cos),
-                _p(self.q_sin), _p(k_pool), _p(v_pool), k_pool.shape[0], _c_cache(cache, cfg, B), _p(out),
-                _p(self.sel), _p(self.sel_pos), cfg.max_sel, _p(self.sel_len), _p(self.workspace),
-                self.workspace.numel(), _stream()))
-        else:
-            _lib.check(_lib.load().ts_decode_layer(
-                ctypes.byref(self._c), ctypes.byref(cb), _p(q), _p(self.q_cos), _p(self.q_sin),
-                _p(k_pool), _p(v_pool), k_pool.shape[0], _c_cache(cache, cfg, B), _p(out),
-                _p(self.sel), _p(self.sel_pos), cfg.max_sel, _p(self.sel_len), _p(self.workspace),
-                self.workspace.numel(), _stream()))
-        if plain:
-            self._clean_for = shape
-        return out, self.sel[:B], self.sel_pos[:B], self.sel_len[:B]
+        return self._run(q, k, v, out_cache_loc, k_pool, v_pool, bt, cache, out, pages, True)
 
     # The layer split at the vote (tensor parallelism, tr.py:361-364): votes() leaves this
     # rank's partial votes, the caller adds the ranks' votes in place (all-reduce), attend()
@@ -968,6 +931,7 @@ class PrefillChunk(_GiveUpLatch):
         self.sel_pos = torch.empty_like(self.sel)
         self.sel_len = torch.empty((1,), dtype=torch.int32, device=device)
         self._init_latch()
+        self._init_native(self.cos, self.sin, None, 1, max_rows)
 
     def recover(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                 out: Optional[torch.Tensor] = None):
@@ -977,12 +941,11 @@ class PrefillChunk(_GiveUpLatch):
         if not self.gave_up():
             return None
         self._latch()
-        return self._run(q, k_pool, v_pool, bt, out, rerun=True)
+        return self._run(q, None, None, None, k_pool, v_pool, bt, None, out, None, False, rerun=True)
 
     def __call__(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                  out: Optional[torch.Tensor] = None):
-        self.check()
-        return self._run(q, k_pool, v_pool, bt, out)
+        return self._run(q, None, None, None, k_pool, v_pool, bt, None, out, None, False)
 
     def step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_cache_loc: Optional[torch.Tensor],
              k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch, out: Optional[torch.Tensor] = None,
@@ -992,53 +955,7 @@ class PrefillChunk(_GiveUpLatch):
         ``bt.seq_lens`` (both written), then the chunk on the length after the append, which
         ``bt.max_seq_len`` must bound.  Same results as the two calls; with caller-chosen
         slots the store rides in the chunk's first launch."""
-        self.check()
-        cfg = self.cfg
-        _need(k, "k", torch.bfloat16)
-        _need(v, "v", torch.bfloat16)
-        loc, pool, _keep = _c_pages(cfg, out_cache_loc, pages)
-        _need(bt.table, "table", torch.int32, 2)
-        row = cfg.num_kv_heads * cfg.head_dim
-        rows = q.shape[0]
-        if k.numel() != rows * row or v.numel() != rows * row or bt.table.shape[0] != 1 or \
-                (pages is None and out_cache_loc.shape[0] != rows):
-            raise ValueError("k / v / out_cache_loc / table do not match the chunk")
-        kv = _lib.TsNewKv(_p(k), _p(v), loc, ctypes.pointer(_keep) if pages is not None else None,
-                          bt.table.shape[1] * cfg.page_size)
-        kv._pool = _keep
-        return self._run(q, k_pool, v_pool, bt, out, new_kv=kv)
-
-    def _run(self, q, k_pool, v_pool, bt, out, rerun: bool = False, new_kv=None):
-        cfg = self.cfg
-        bt = self._options(bt, rerun)
-        cb = _c_batch(cfg, bt)
-        _need(q, "q", torch.bfloat16, 2)
-        rows = q.shape[0]
-        if bt.batch != 1 or bt.max_seq_len > self.max_seq_len or rows > self.max_rows:
-            raise ValueError("one request, within the sizes this PrefillChunk was built for")
-        if q.shape[1] != cfg.num_heads * cfg.head_dim:
-            raise ValueError("q must be [rows, H*D]")
-        _check_pool(cfg, k_pool, "k_pool")
-        _check_pool(cfg, v_pool, "v_pool")
-        if out is None:
-            out = torch.empty_like(q)
-        else:
-            _need(out, "out", torch.bfloat16)
-            if out.numel() != q.numel():
-                raise ValueError("out must hold rows*H*D elements")
-        if new_kv is not None:
-            _lib.check(_lib.load().ts_prefill_step(
-                ctypes.byref(self._c), ctypes.byref(cb), ctypes.byref(new_kv), _p(q), rows, _p(self.cos),
-                _p(self.sin), self.cos.shape[0], _p(k_pool), _p(v_pool), k_pool.shape[0], _p(out),
-                _p(self.sel), _p(self.sel_pos), cfg.max_sel, _p(self.sel_len), _p(self.workspace),
-                self.workspace.numel(), _stream()))
-        else:
-            _lib.check(_lib.load().ts_prefill_chunk(
-                ctypes.byref(self._c), ctypes.byref(cb), _p(q), rows, _p(self.cos), _p(self.sin),
-                self.cos.shape[0], _p(k_pool), _p(v_pool), k_pool.shape[0], _p(out), _p(self.sel),
-                _p(self.sel_pos), cfg.max_sel, _p(self.sel_len), _p(self.workspace),
-                self.workspace.numel(), _stream()))
-        return out, self.sel, self.sel_pos, self.sel_len
+        return self._run(q, k, v, out_cache_loc, k_pool, v_pool, bt, None, out, pages, True)
 
 
 def sparse_decode_attention_static(cfg: LayerConfig, q: torch.Tensor, k_pool: torch.Tensor,
