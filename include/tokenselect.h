@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define TS_VERSION 100
+#define TS_VERSION 101
 
 #define TS_OK 0
 #define TS_EINVAL (-1)     /* null pointer or scalar out of range            */
@@ -141,6 +141,9 @@ typedef struct ts_batch {
                                where the selection is the single ts_select launch and no
                                selection cache is used; ignored otherwise.  A wrong
                                statement gives wrong selections or waits that give up */
+  int32_t q_row_stride;     /* layer, chunk and step calls: elements between the query
+                               rows (>= H*D, a multiple of 8), 0 = H*D: the query part
+                               of a fused QKV projection is read where it lies          */
 } ts_batch;
 
 /* Default bound of a grid-wide wait: a selection that has the device to itself
@@ -404,6 +407,8 @@ typedef struct ts_new_kv {
   const int32_t* out_cache_loc;  /* [batch] slots, or NULL with pages */
   const ts_page_pool* pages;     /* or NULL */
   int32_t max_tokens;            /* as for ts_kv_store */
+  int32_t row_stride;            /* elements between rows of k, and of v (>= Hkv*D, a
+                                    multiple of 8), 0 = Hkv*D */
 } ts_new_kv;
 int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
                    const float* q_cos, const float* q_sin, void* k_pool, void* v_pool,

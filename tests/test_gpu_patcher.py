@@ -301,3 +301,50 @@ def test_patched_decode_forward_for_a_batch(dev):
             attns[0].forward(torch.zeros(3, H * D, dtype=torch.bfloat16, device=dev), None, None, meta)
     finally:
         tr.PREFILL_CHUNK_SIZE = 512
+
+
+def test_fused_projection_rows_are_read_where_they_lie(dev):
+    """q, k and v as a split of one projection leaves them (rows of one stride, not contiguous),
+    whole or from a misaligned column on, against the same rows made contiguous: prompts of
+    one row, one chunk and a ragged second chunk, then decode steps, alone and as a batch."""
+    say("strided projection rows")
+    H, Hkv, D, chunk = 8, 2, 128, 32
+    tr.patch(rope_base=1e4, rope_scale=1, rope_model="ROPE_LLAMA", max_n_tokens=256, top_k=24, n_init=4,
+             n_local=16)
+    tr.PREFILL_CHUNK_SIZE = chunk
+    try:
+        for pad in (0, 1):                                     # 1: rows start at an odd column
+            g = torch.Generator(device=dev).manual_seed(31)
+            sizes = (H * D, Hkv * D, Hkv * D)
+            slots = torch.randperm(512, generator=g, device=dev).to(torch.int32)
+            prompts = [torch.randn(T, sum(sizes) + 8, generator=g, device=dev).bfloat16() for T in (1, 32, 77)]
+            steps = [torch.randn(3, sum(sizes) + 8, generator=g, device=dev).bfloat16() for _ in range(3)]
+            outs = []
+            for contiguous in (True, False):
+                def parts(x):
+                    q, k, v = x[:, pad:pad + sum(sizes)].split(sizes, dim=-1)
+                    return tuple(t.contiguous() if contiguous else t for t in (q, k, v))
+                pool = sg.TokenToKVPool(512, torch.bfloat16, Hkv, D, 1, dev)
+                runner = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool,
+                                        dtype=torch.bfloat16)
+                owner = runner.req_to_token_retriever
+                attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
+                got, used, singles = [], 0, []
+                for x in prompts:
+                    r = owner.new_token_retriever()
+                    singles.append(r)
+                    for mode, rows in ((sg.ForwardMode.EXTEND, x), (sg.ForwardMode.DECODE, steps[0][:1])):
+                        n = rows.shape[0]
+                        meta = sg.InputMetadata(mode, r, pool, slots[used:used + n])
+                        used += n
+                        got.append(attn.forward(*parts(rows), meta))
+                batch = owner.get_batch_token_retriever(("a", "b", "c"), singles)
+                for x in steps:
+                    meta = sg.InputMetadata(sg.ForwardMode.DECODE, batch, pool, slots[used:used + 3], batch_size=3)
+                    used += 3
+                    got.append(attn.forward(*parts(x), meta))
+                outs.append(got + [pool.k_buffer[0], pool.v_buffer[0]])
+            for i, (a, b) in enumerate(zip(*outs)):
+                assert torch.equal(a, b), f"pad {pad}, output {i}"
+    finally:
+        tr.PREFILL_CHUNK_SIZE = 512

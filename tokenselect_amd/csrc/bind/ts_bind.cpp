@@ -12,12 +12,14 @@
 // handed over as addresses by _lib.py, so that there is one loaded copy of it.
 #include <Python.h>
 
+#include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
 #include <exception>
+#include <optional>
 #include <string>
 
 #include "../../../include/tokenselect.h"
@@ -143,12 +145,12 @@ struct Owned {
   int64_t batch, max_seq_len, max_rows;
   // (batch, max_seq_len) that the selection's counters in the workspace are clean for, -1: none.
   int64_t clean_batch = -1, clean_len = -1;
-  // The outputs' rows of the last batch size: out, sel, sel_pos, sel_len.
-  int64_t rows_of = -1;
-  PyObject* rows[4] = {nullptr, nullptr, nullptr, nullptr};
-  void forget_rows() {
-    for (PyObject*& r : rows) Py_CLEAR(r);
-    rows_of = -1;
+  // The outputs' first rows, for the last batch size: out, sel, sel_pos, sel_len.
+  int64_t views_of = -1;
+  PyObject* views[4] = {nullptr, nullptr, nullptr, nullptr};
+  void forget_views() {
+    for (PyObject*& r : views) Py_CLEAR(r);
+    views_of = -1;
   }
 };
 
@@ -170,7 +172,7 @@ const at::Tensor& check_pool(const ts_config& cfg, PyObject* o, const char* name
 // The options of a call, from a Batch and the object's own state.
 struct Call {
   ts_batch bt{};
-  const at::Tensor* table = nullptr;
+  int64_t table_tokens = 0;
 };
 
 void fill_batch(const Owned& o, PyObject* b, bool separate, bool rerun, Call* call) {
@@ -224,7 +226,7 @@ void fill_batch(const Owned& o, PyObject* b, bool separate, bool rerun, Call* ca
     if (o.max_rows > 0) bad_value("one request, within the sizes this PrefillChunk was built for");
     bad_value("batch / max_seq_len exceed what this DecodeLayer was sized for");
   }
-  call->table = &table;
+  call->table_tokens = table.size(1) * o.cfg.page_size;
 }
 
 void fill_cache(const ts_config& cfg, PyObject* cache, int64_t B, ts_selcache* c) {
@@ -250,10 +252,75 @@ void fill_pages(PyObject* pages, ts_page_pool* c) {
                     (uint32_t*)need(ticket_ref.p, "ticket", at::kInt, 1).data_ptr()};
 }
 
+// Rows of bf16 as the library takes them: at `ptr`, `stride` elements apart.
+struct Rows {
+  const void* ptr;
+  int64_t stride;
+  std::optional<at::Tensor> copy;  // of rows that do not lie so
+};
+// `count` rows of `width` elements, rows [from, from + count) of `t` (the part of a fused QKV
+// projection, as a split leaves it: read where it lies).
+Rows rows_of(PyObject* obj, const char* name, int64_t from, int64_t count, int64_t width, bool packed) {
+  const at::Tensor& t = tensor(obj, name);
+  if (t.scalar_type() != at::kBFloat16 || !t.is_cuda()) need(obj, name, at::kBFloat16);  // (raises)
+  if (t.dim() < 2 || t.numel() != t.size(0) * width || from + count > t.size(0))
+    bad_value(std::string(name) + " must hold rows of " + std::to_string(width) + " elements, got shape " + shape_text(t));
+  bool dense = true;  // within a row
+  int64_t step = 1;
+  for (int64_t d = t.dim() - 1; d > 0; --d) {
+    dense = dense && (t.size(d) == 1 || t.stride(d) == step);
+    step *= t.size(d);
+  }
+  const int64_t stride = t.size(0) > 1 ? t.stride(0) : width;
+  if (dense && !packed && stride >= width && stride <= INT32_MAX && stride % 8 == 0 && (uintptr_t)t.data_ptr() % 16 == 0)
+    return Rows{(const char*)t.data_ptr() + 2 * from * stride, stride, std::nullopt};
+  at::Tensor c = t.narrow(0, from, count).contiguous();
+  if ((uintptr_t)c.data_ptr() % 16 != 0) c = c.clone();
+  const void* at = c.data_ptr();
+  return Rows{at, width, std::move(c)};
+}
+
 PyObject* row_view(const at::Tensor& t, int64_t B) {
   PyObject* v = THPVariable_Wrap(t.narrow(0, 0, B));
   if (!v) throw Raised{};
   return v;
+}
+
+// The library's call on the current stream, with the object's buffers.  kv: the tokens to store
+// first, or NULL.  rows: of the chunk.
+int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int64_t rows, const at::Tensor& k_pool,
+                 const at::Tensor& v_pool, const ts_selcache* cache, void* out, bool rerun = false) {
+  // The attention kernel of a plain call leaves the selection's counters zero for the next
+  // one of the same shape.
+  const bool chunk = o.max_rows > 0, plain = !chunk && !cache && !bt->separate_kernels && !rerun;
+  if (plain && o.clean_batch == bt->batch && o.clean_len == bt->max_seq_len) bt->workspace_clean = 1;
+  o.clean_batch = o.clean_len = -1;
+  const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
+  const float *cos = (const float*)o.cos.data_ptr(), *sin = (const float*)o.sin.data_ptr();
+  int32_t *sel = (int32_t*)o.sel.data_ptr(), *sel_pos = (int32_t*)o.sel_pos.data_ptr(),
+          *sel_len = (int32_t*)o.sel_len.data_ptr();
+  const int64_t sel_stride = o.sel.size(1), table_rows = o.cos.size(0), pool_rows = k_pool.size(0);
+  void *kp = k_pool.data_ptr(), *vp = v_pool.data_ptr(), *ws = o.workspace.data_ptr();
+  const size_t ws_bytes = (size_t)o.workspace.numel();
+  const ts_config* cfg = &o.cfg;
+  int code;
+  Py_BEGIN_ALLOW_THREADS
+  if (chunk)
+    code = kv ? prefill_step(cfg, bt, kv, q, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out, sel, sel_pos,
+                             sel_stride, sel_len, ws, ws_bytes, stream)
+              : prefill_chunk(cfg, bt, q, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out, sel, sel_pos,
+                              sel_stride, sel_len, ws, ws_bytes, stream);
+  else
+    code = kv ? decode_step(cfg, bt, kv, q, cos, sin, kp, vp, pool_rows, cache, out, sel, sel_pos, sel_stride, sel_len,
+                            ws, ws_bytes, stream)
+              : decode_layer(cfg, bt, q, cos, sin, kp, vp, pool_rows, cache, out, sel, sel_pos, sel_stride, sel_len, ws,
+                             ws_bytes, stream);
+  Py_END_ALLOW_THREADS
+  if (code == TS_OK && plain) {
+    o.clean_batch = bt->batch;
+    o.clean_len = bt->max_seq_len;
+  }
+  return code;
 }
 
 // run(q, k, v, out_cache_loc, k_pool, v_pool, bt, cache, out, pages, store, separate, rerun):
@@ -307,20 +374,20 @@ PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
                       : "k / v / out_cache_loc / table do not match the batch");
     kv.k = k.data_ptr();
     kv.v = v.data_ptr();
-    kv.max_tokens = (int32_t)(call.table->size(1) * cfg.page_size);
+    kv.max_tokens = (int32_t)call.table_tokens;
   }
 
   ts_selcache cache{};
   const bool cached = cache_o != Py_None;
   if (cached) fill_cache(cfg, cache_o, B, &cache);
 
-  if (o.rows_of != B) {
-    o.forget_rows();
-    if (!chunk) o.rows[0] = row_view(o.out, B);
-    o.rows[1] = row_view(o.sel, B);
-    o.rows[2] = row_view(o.sel_pos, B);
-    o.rows[3] = row_view(o.sel_len, B);
-    o.rows_of = B;
+  if (o.views_of != B) {
+    o.forget_views();
+    if (!chunk) o.views[0] = row_view(o.out, B);
+    o.views[1] = row_view(o.sel, B);
+    o.views[2] = row_view(o.sel_pos, B);
+    o.views[3] = row_view(o.sel_len, B);
+    o.views_of = B;
   }
   PyObject* out_py;
   void* out_ptr;
@@ -337,45 +404,72 @@ PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
     if (!out_py) throw Raised{};
   } else {
     out_ptr = o.out.data_ptr();
-    out_py = o.rows[0];
+    out_py = o.views[0];
     Py_INCREF(out_py);
   }
   const Ref out_ref(out_py);
 
-  // The attention kernel of a plain call leaves the selection's counters zero for the next
-  // one of the same shape.
-  const bool plain = !chunk && !cached && !bt.separate_kernels && !rerun;
-  if (plain && o.clean_batch == B && o.clean_len == bt.max_seq_len) bt.workspace_clean = 1;
-  o.clean_batch = o.clean_len = -1;
-
-  const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
-  const float *cos = (const float*)o.cos.data_ptr(), *sin = (const float*)o.sin.data_ptr();
-  int32_t *sel = (int32_t*)o.sel.data_ptr(), *sel_pos = (int32_t*)o.sel_pos.data_ptr(),
-          *sel_len = (int32_t*)o.sel_len.data_ptr();
-  const int64_t sel_stride = o.sel.size(1), table_rows = o.cos.size(0), pool_rows = k_pool.size(0);
-  void *kp = k_pool.data_ptr(), *vp = v_pool.data_ptr(), *ws = o.workspace.data_ptr();
-  const void* qp = q.data_ptr();
-  const size_t ws_bytes = (size_t)o.workspace.numel();
-  const ts_selcache* cp = cached ? &cache : nullptr;
-  int code;
-  Py_BEGIN_ALLOW_THREADS
-  if (chunk)
-    code = store ? prefill_step(&cfg, &bt, &kv, qp, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out_ptr, sel,
-                                sel_pos, sel_stride, sel_len, ws, ws_bytes, stream)
-                 : prefill_chunk(&cfg, &bt, qp, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out_ptr, sel,
-                                 sel_pos, sel_stride, sel_len, ws, ws_bytes, stream);
-  else
-    code = store ? decode_step(&cfg, &bt, &kv, qp, cos, sin, kp, vp, pool_rows, cp, out_ptr, sel, sel_pos, sel_stride,
-                               sel_len, ws, ws_bytes, stream)
-                 : decode_layer(&cfg, &bt, qp, cos, sin, kp, vp, pool_rows, cp, out_ptr, sel, sel_pos, sel_stride,
-                                sel_len, ws, ws_bytes, stream);
-  Py_END_ALLOW_THREADS
+  const int code = call_library(o, &bt, store ? &kv : nullptr, q.data_ptr(), rows, k_pool, v_pool,
+                                cached ? &cache : nullptr, out_ptr, rerun);
   if (code != TS_OK) return PyLong_FromLong(code);
-  if (plain) {
-    o.clean_batch = B;
-    o.clean_len = bt.max_seq_len;
+  return PyTuple_Pack(4, out_py, o.views[1], o.views[2], o.views[3]);
+}
+
+// serve(q, k, v, out_cache_loc, k_pool, v_pool, bt, cache, out, from, rows, separate): the step of a
+// serving stack whose q, k and v are parts of one projection.  A DecodeLayer: one row per
+// request, the output a fresh tensor.  A PrefillChunk: `rows` rows of the prompt part from
+// `from` on, written to the same rows of `out`.  Returns as run() does, but the output alone.
+PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 12) raise(PyExc_TypeError, "serve() takes 12 arguments");
+  Owned& o = *self->own;
+  if (fault_of(o) != 0) Py_RETURN_NONE;
+  const bool chunk = o.max_rows > 0, separate = args[11] == Py_True;
+  const ts_config& cfg = o.cfg;
+  const int64_t width = (int64_t)cfg.num_heads * cfg.head_dim, row = (int64_t)cfg.num_kv_heads * cfg.head_dim;
+  Call call;
+  fill_batch(o, args[6], separate, false, &call);
+  ts_batch& bt = call.bt;
+  const int64_t from = chunk ? as_long(args[9]) : 0;
+  int64_t rows = bt.batch;
+  if (chunk) {
+    rows = as_long(args[10]);
+    if (bt.batch != 1 || rows > o.max_rows) bad_value("one request, within the sizes this PrefillChunk was built for");
+    if (from < 0 || rows < 1) bad_value("a chunk has at least one row");
   }
-  return PyTuple_Pack(4, out_py, o.rows[1], o.rows[2], o.rows[3]);
+  const Rows q = rows_of(args[0], "q", from, rows, width, false);
+  Rows k = rows_of(args[1], "k", from, rows, row, false), v = rows_of(args[2], "v", from, rows, row, false);
+  if (k.stride != v.stride) {
+    if (k.stride != row) k = rows_of(args[1], "k", from, rows, row, true);
+    if (v.stride != row) v = rows_of(args[2], "v", from, rows, row, true);
+  }
+  bt.q_row_stride = (int32_t)q.stride;
+  const at::Tensor& k_pool = check_pool(cfg, args[4], "k_pool");
+  const at::Tensor& v_pool = check_pool(cfg, args[5], "v_pool");
+  if (k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
+  if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
+  const at::Tensor& loc = need(args[3], "out_cache_loc", at::kInt, 1);
+  if (loc.size(0) < from + rows) bad_value("out_cache_loc does not match the rows");
+  ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.data_ptr() + from, nullptr,
+               (int32_t)call.table_tokens, (int32_t)k.stride};
+  ts_selcache cache{};
+  const bool cached = args[7] != Py_None;
+  if (cached) fill_cache(cfg, args[7], bt.batch, &cache);
+  at::Tensor out;
+  if (chunk) {
+    out = need(args[8], "out", at::kBFloat16);
+    if (out.dim() < 1 || out.numel() != out.size(0) * width || out.size(0) < from + rows)
+      bad_value("out must hold the rows of q");
+  } else {
+    out = at::empty({rows, width}, o.out.options());
+  }
+  const int code = call_library(o, &bt, &kv, q.ptr, rows, k_pool, v_pool, cached ? &cache : nullptr,
+                                (char*)out.data_ptr() + 2 * from * width);
+  if (code != TS_OK) return PyLong_FromLong(code);
+  if (chunk) {
+    Py_INCREF(args[8]);
+    return args[8];
+  }
+  return THPVariable_Wrap(std::move(out));
 }
 
 // Runs `f`, with C++ exceptions turned into Python's.
@@ -392,6 +486,10 @@ PyObject* guarded(F&& f) {
 
 PyObject* runner_run(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&] { return run((Runner*)self, args, nargs); });
+}
+
+PyObject* runner_serve(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&] { return serve((Runner*)self, args, nargs); });
 }
 
 PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
@@ -428,7 +526,7 @@ PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
 void runner_dealloc(PyObject* self) {
   Owned* o = ((Runner*)self)->own;
   if (o) {
-    o->forget_rows();
+    o->forget_views();
     delete o;
   }
   PyTypeObject* type = Py_TYPE(self);
@@ -451,7 +549,9 @@ int set_clean(PyObject* self, PyObject* value, void*) {
 }
 
 PyMethodDef runner_methods[] = {
-    {"run", (PyCFunction)(void (*)(void))runner_run, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+    {"run", (PyCFunction)(void (*)(void))runner_run, METH_FASTCALL, nullptr},
+    {"serve", (PyCFunction)(void (*)(void))runner_serve, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
 PyGetSetDef runner_getset[] = {{"clean", get_clean, set_clean, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyType_Slot runner_slots[] = {{Py_tp_new, (void*)runner_new}, {Py_tp_dealloc, (void*)runner_dealloc},
                               {Py_tp_methods, runner_methods}, {Py_tp_getset, runner_getset}, {0, nullptr}};

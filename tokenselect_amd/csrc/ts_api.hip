@@ -56,6 +56,13 @@ int validate_config(const ts_config* cfg) {
   return TS_OK;
 }
 
+int check_row_stride(int64_t stride, int64_t width, const char* who) {
+  TS_REQUIRE(stride == 0 || (stride >= width && stride % 8 == 0), TS_EINVAL,
+             "%s: row stride %lld is neither 0 nor a multiple of 8 of at least %lld", who, (long long)stride,
+             (long long)width);
+  return TS_OK;
+}
+
 int validate_batch(const ts_config* cfg, const ts_batch* bt) {
   (void)cfg;
   TS_REQUIRE(bt != nullptr, TS_EINVAL, "batch is NULL");
@@ -66,12 +73,18 @@ int validate_batch(const ts_config* cfg, const ts_batch* bt) {
   TS_REQUIRE(bt->batch == 1 || bt->table_stride * (int64_t)cfg->page_size >= bt->max_seq_len,
              TS_EINVAL, "table_stride %lld too small for max_seq_len %d at page_size %d",
              (long long)bt->table_stride, bt->max_seq_len, cfg->page_size);
+  TS_TRY(check_row_stride(bt->q_row_stride, (int64_t)cfg->num_heads * cfg->head_dim, "query"));
   if (bt->host_seq_lens)
     for (int b = 0; b < bt->batch; ++b)
       TS_REQUIRE(bt->host_seq_lens[b] >= 0 && bt->host_seq_lens[b] <= bt->max_seq_len, TS_EINVAL,
                  "host_seq_lens[%d] = %d outside [0, max_seq_len %d]", b, bt->host_seq_lens[b],
                  bt->max_seq_len);
   return TS_OK;
+}
+
+// Elements between the query rows of a call.
+static int query_stride(const ts_config* cfg, const ts_batch* bt) {
+  return bt->q_row_stride ? bt->q_row_stride : cfg->num_heads * cfg->head_dim;
 }
 
 int score_tokens_per_block(int64_t total_candidates, int num_heads) {
@@ -209,6 +222,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
              "internal: a chunk's store rides in the fingerprint launch only");
   TS_REQUIRE(pool_rows >= 1 && pool_rows <= 0x7fffffffLL, TS_EINVAL, "pool_rows %lld out of range",
              (long long)pool_rows);
+  const int q_stride = query_stride(cfg, bt);
   LayerWorkspace w = layer_workspace(cfg, bt->batch, bt->max_seq_len);
   TS_REQUIRE_ALIGNED(workspace, 256, "workspace");
   TS_REQUIRE_ALIGNED(q, 16, "q");
@@ -265,18 +279,18 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   if (starts_with_selection) {
   } else if (chunk_rows > 0) {
     // Chunk fingerprint: row i rotated to n_local + i, mean over the rows (tr.py:380-392).
-    TS_TRY(launch_fingerprint(cfg, q, chunk_rows, q_cos, q_sin, table_rows, qf, zero,
+    TS_TRY(launch_fingerprint(cfg, q, q_stride, chunk_rows, q_cos, q_sin, table_rows, qf, zero,
                               (hipStream_t)stream, chunk_store));
   } else if (cache) {  // rotation and cache decision in one launch
-    TS_TRY(launch_rope_selcache(cfg, bt, q, qf, q_cos, q_sin, cache, hit, bt->rerun ? sel_len : nullptr,
+    TS_TRY(launch_rope_selcache(cfg, bt, q, q_stride, qf, q_cos, q_sin, cache, hit, bt->rerun ? sel_len : nullptr,
                                 zero, (hipStream_t)stream, store));
   } else {
-    TS_TRY(launch_rope(q, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
+    TS_TRY(launch_rope(q, q_stride, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
                        zero, (hipStream_t)stream));
   }
   if (cache && chunk_rows > 0)
     TS_TRY(launch_selcache(cfg, bt, qf, cache, hit, bt->rerun ? sel_len : nullptr, (hipStream_t)stream));
-  const UnrotatedQuery unrotated{q, q_cos, q_sin};
+  const UnrotatedQuery unrotated{q, q_stride, q_cos, q_sin};
   if (one_launch) {
     TS_TRY(launch_select(cfg, bt, qf, k_pool, pool_rows, hit, cache, sel, sel_pos, sel_stride, sel_len,
                          nullptr, 0, ws + w.select_ws, tickets, attn_tickets_per_request(cfg),
@@ -304,9 +318,9 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                        zeroed && cfg->pool_kernel <= 0));
   }
   if (chunk_rows > 0)
-    return ts_sparse_prefill_attn(cfg, q, chunk_rows, k_pool, v_pool, pool_rows, sel, sel_len,
-                                  w.max_sel, out, ws + w.attn_ws, w.total - w.attn_ws, stream);
-  return launch_attn(cfg, q, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch,
+    return launch_prefill_attn(cfg, q, q_stride, chunk_rows, k_pool, v_pool, pool_rows, sel, sel_len,
+                               w.max_sel, out, ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream);
+  return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch,
                      w.max_sel, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream,
                      plain_decode ? &zero : nullptr);
 }
@@ -338,8 +352,9 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
   const bool rides = cache != nullptr && bt->rerun == 0;
   if (!rides) {
     if (bt->rerun == 0)
-      TS_TRY(ts_kv_store(cfg, kv->k, kv->v, kv->out_cache_loc, kv->pages, k_pool, v_pool, pool_rows, table,
-                         bt->table_stride, seq_lens, bt->batch, kv->max_tokens, stream));
+      TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
+                             pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
+                             (hipStream_t)stream));
     return run_layer(cfg, bt, q, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
                      sel_stride, sel_len, workspace, workspace_bytes, stream);
   }
@@ -375,6 +390,8 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
   st.table_stride = bt->table_stride;
   st.seq_lens = seq_lens;
   st.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  TS_TRY(check_row_stride(kv->row_stride, st.row_vec * 8, "ts_decode_step"));
+  st.kv_stride = kv->row_stride ? kv->row_stride / 8 : st.row_vec;
   st.max_tokens = kv->max_tokens;
   if (kv->pages) {
     st.free_pages = kv->pages->free_pages;
@@ -412,6 +429,7 @@ int ts_decode_layer_votes(const ts_config* cfg, const ts_batch* bt, const void* 
   if (cache)
     TS_REQUIRE(cache->q_cache && cache->topk_cache && cache->cache_len && cache->counters, TS_EINVAL,
                "selection cache has a NULL array");
+  const int q_stride = query_stride(cfg, bt);
   ts_config plain = *cfg;  // the max-pool comes after the ranks' votes are added up
   plain.pool_kernel = -1;
   char* ws = (char*)workspace;
@@ -421,7 +439,7 @@ int ts_decode_layer_votes(const ts_config* cfg, const ts_batch* bt, const void* 
   const int group = vote_launches_planned(&plain, bt) ? 1 : 0;
   ZeroSet zero;
   if (group > 0) score_votes_zero_regions(&plain, bt, fused, ws + w.select_ws, &zero);
-  TS_TRY(launch_rope(q, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
+  TS_TRY(launch_rope(q, q_stride, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
                      zero, (hipStream_t)stream));
   if (cache) TS_TRY(ts_selcache_step(cfg, bt, qf, cache, hit, stream));
   if (max_n <= 0) return TS_OK;
@@ -482,7 +500,7 @@ int ts_decode_layer_attend(const ts_config* cfg, const ts_batch* bt, const void*
   if (vote_launches_planned(&plain, bt))
     topk.fault = score_votes_fault_word(&plain, bt->batch, bt->max_seq_len, ws + w.select_ws);
   TS_TRY(launch_topk(topk, bt->batch, max_n, (hipStream_t)stream));
-  return launch_attn(cfg, q, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch, w.max_sel,
+  return launch_attn(cfg, q, query_stride(cfg, bt), k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch, w.max_sel,
                      out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream);
 }
 
@@ -517,8 +535,8 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
                      rows <= 1023 * 32;
   if (!rides) {
     if (bt->rerun == 0)  // (a call that repeats a chunk after a give-up does not append again)
-      TS_TRY(ts_kv_store_chunk(cfg, kv->k, kv->v, kv->out_cache_loc, kv->pages, rows, k_pool, v_pool, pool_rows,
-                               table, seq_len, kv->max_tokens, stream));
+      TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
+                                   v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream));
     return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                      out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
   }
@@ -544,6 +562,8 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
   cs.seq_len = seq_len;
   cs.rows = rows;
   cs.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  TS_TRY(check_row_stride(kv->row_stride, cs.row_vec * 8, "ts_prefill_step"));
+  cs.kv_stride = kv->row_stride ? kv->row_stride / 8 : cs.row_vec;
   cs.max_tokens = kv->max_tokens;
   return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                    out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, &cs);

@@ -18,7 +18,8 @@
 namespace ts {
 
 struct AttnArgs {
-  const uint16_t* q;  // [B,H,128] bf16, un-rotated
+  const uint16_t* q;  // [B,H,128] bf16, un-rotated, rows q_stride elements apart
+  int q_stride;
   const uint16_t* k_pool;
   const uint16_t* v_pool;
   uint32_t pool_rows;
@@ -253,7 +254,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, qd = lane >> 4;
-  const int H = a.num_heads;
   const int chunk = attn_chunk(a.max_sel_len, a.nsplit);
   const int wlen = chunk / 4;
   const int32_t* sel = a.sel + (int64_t)b * a.sel_stride;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // for every load that either side may have issued.)
   uint4 q_raw[2];
   {
-    const uint16_t* qrow = a.q + ((size_t)b * H + head) * kHeadDim + 32 * (wave & 1) + 8 * qd;
+    const uint16_t* qrow = a.q + (size_t)b * a.q_stride + head * kHeadDim + 32 * (wave & 1) + 8 * qd;
     q_raw[0] = *(const uint4*)qrow;
     q_raw[1] = *(const uint4*)(qrow + 64);
   }
@@ -583,7 +583,7 @@ uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* w
   return (uint32_t*)((char*)workspace + attn_workspace(cfg, batch, max_sel_len).tickets);
 }
 
-int launch_attn(const ts_config* cfg, const void* q, const void* k_pool, const void* v_pool,
+int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
                 hipStream_t st, const ZeroSet* clear_after) {
@@ -595,6 +595,7 @@ int launch_attn(const ts_config* cfg, const void* q, const void* k_pool, const v
     a.zero = *clear_after;
   }
   a.q = (const uint16_t*)q;
+  a.q_stride = q_stride;
   a.k_pool = (const uint16_t*)k_pool;
   a.v_pool = (const uint16_t*)v_pool;
   a.pool_rows = (uint32_t)pool_rows;
@@ -713,7 +714,7 @@ int ts_sparse_decode_attn(const ts_config* cfg, const void* q, const void* k_poo
   TS_REQUIRE_ALIGNED(k_pool, 16, "k_pool");
   TS_REQUIRE_ALIGNED(v_pool, 16, "v_pool");
   TS_REQUIRE_ALIGNED(out, 16, "out");
-  return launch_attn(cfg, q, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, batch, max_sel_len,
+  return launch_attn(cfg, q, cfg->num_heads * cfg->head_dim, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, batch, max_sel_len,
                      out, workspace, /*tickets_clear=*/false, (hipStream_t)stream);
 }
 
@@ -753,7 +754,7 @@ int ts_sparse_decode_attn_static(const ts_config* cfg, const void* q, const void
   if (ptr == nullptr) return TS_EHIP;
   // The tickets are cleared by a fill kernel on the caller's stream (the previous call
   // may have been interrupted), so the call can be captured into a HIP graph.
-  return launch_attn(cfg, q, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, batch, max_sel_len,
+  return launch_attn(cfg, q, cfg->num_heads * cfg->head_dim, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, batch, max_sel_len,
                      out, ptr, /*tickets_clear=*/false, (hipStream_t)stream);
 }
 

@@ -13,6 +13,8 @@ int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
 int validate_config(const ts_config* cfg);
 int validate_batch(const ts_config* cfg, const ts_batch* bt);
+// A row stride in elements: 0 (contiguous rows of `width`), or a multiple of 8 of at least `width`.
+int check_row_stride(int64_t stride, int64_t width, const char* who);
 bool group_supported(int num_kv_heads, int group);
 
 #define TS_REQUIRE(cond, code, ...)                     \
@@ -91,12 +93,14 @@ struct ChunkStore {
   int32_t* table;    // the request's row
   int32_t* seq_len;  // the request's length word
   int rows, row_vec, max_tokens;
+  int kv_stride;     // 16-byte pieces between rows of k, and of v
   int workgroups;    // of the launch that store (set by the launcher)
 };
-int launch_fingerprint(const ts_config* cfg, const void* q, int32_t rows, const float* cos_table,
+int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
                        const float* sin_table, int64_t table_rows, void* qf, const ZeroSet& zero,
                        hipStream_t stream, const ChunkStore* store = nullptr);
-int launch_rope(const void* x, void* out, const float* cos_table, const float* sin_table,
+// x_stride: elements between the rows of x (out is contiguous).
+int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
                 const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
                 const ZeroSet& zero, hipStream_t stream);
 
@@ -121,6 +125,7 @@ struct StepStore {
   int64_t table_stride;
   int32_t* seq_lens;
   int row_vec;     // 16-byte pieces per row
+  int kv_stride;   // 16-byte pieces between rows of k, and of v
   int max_tokens;
   // With a page pool (free_pages != NULL; loc is not read): the slots come from the table and
   // the pool as kv_store_paged_kernel takes them.
@@ -129,10 +134,24 @@ struct StepStore {
   uint32_t* ticket;
   int page_shift;
 };
-int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q, void* qf,
+int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q, int q_stride, void* qf,
                          const float* q_cos, const float* q_sin, const ts_selcache* cache, int32_t* hit,
                          const int32_t* gave_up_len, const ZeroSet& zero, hipStream_t stream,
                          const StepStore* store = nullptr);
+
+// ts_kv_store and ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
+int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
+                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
+                    int32_t max_tokens, hipStream_t stream);
+int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                          const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
+                          void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
+                          hipStream_t stream);
+// ts_sparse_prefill_attn for query rows that lie q_stride elements apart.
+int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
+                        const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
+                        int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 // Sparse decode attention (ts_attn.hip).  The kernel counts its workgroups in per
 // (request, KV head) tickets inside the workspace, which must be zero at launch:
@@ -143,7 +162,7 @@ uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* w
 int attn_tickets_per_request(const ts_config* cfg);
 // clear_after: regions that the kernel clears on the side (the counters of the stream's
 // next selection), or NULL.
-int launch_attn(const ts_config* cfg, const void* q, const void* k_pool, const void* v_pool,
+int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
                 hipStream_t stream, const ZeroSet* clear_after = nullptr);

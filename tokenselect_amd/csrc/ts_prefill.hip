@@ -25,7 +25,7 @@ constexpr int kFpVec = 4;       // rotation pairs per thread
 constexpr int kFpSplit = 2;     // workgroups per head
 
 __global__ __launch_bounds__(1024) void fingerprint_kernel(
-    const uint16_t* __restrict__ q, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
+    const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
     const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int heads,
     ZeroSet zero, ChunkStore cs) {
 #pragma clang fp contract(off)
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(1024) void fingerprint_kernel(
       pos = pos < table_rows ? pos : table_rows - 1;
       const float* c = cos_table + pos * kHeadDim;
       const float* s = sin_table + pos * kHeadDim;
-      const size_t base = ((size_t)r * heads + h) * kHeadDim;
+      const size_t base = (size_t)r * q_stride + h * kHeadDim;
       x1[j] = *(const uint2*)(q + base + i);
       x2[j] = *(const uint2*)(q + base + i + half);
       c1[j] = *(const float4*)(c + i);
@@ -169,7 +169,8 @@ __global__ __launch_bounds__(1024) void fingerprint_kernel(
 // stream: two wavefronts per SIMD cover each other only partly.  Four wavefronts per SIMD
 // with one head each double the LDS reads and came out the same.
 struct PrefillArgs {
-  const uint16_t* q;  // [rows, H, 128] bf16, un-rotated
+  const uint16_t* q;  // [rows, H, 128] bf16, un-rotated, rows q_stride elements apart
+  int q_stride;
   const uint16_t* k_pool;
   const uint16_t* v_pool;
   uint32_t pool_rows;
@@ -398,7 +399,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint4 q_raw[HEADS][4];
 #pragma unroll
   for (int rb = 0; rb < HEADS; ++rb) {
-    const uint16_t* qrow = a.q + ((size_t)q_row * H + head[rb]) * kHeadDim;
+    const uint16_t* qrow = a.q + (size_t)q_row * a.q_stride + head[rb] * kHeadDim;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) q_raw[rb][ks] = *(const uint4*)(qrow + 32 * ks + 8 * g4);
   }
@@ -746,7 +747,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-int launch_fingerprint(const ts_config* cfg, const void* q, int32_t rows, const float* cos_table,
+int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
                        const float* sin_table, int64_t table_rows, void* qf, const ZeroSet& zero,
                        hipStream_t stream, const ChunkStore* store) {
   TS_TRY(validate_config(cfg));
@@ -769,34 +770,17 @@ int launch_fingerprint(const ts_config* cfg, const void* q, int32_t rows, const 
     grid_y += (unsigned)ceil_div(cs.workgroups, cfg->num_heads);
   }
   hipLaunchKernelGGL(fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y), dim3(1024), 0, stream,
-                     (const uint16_t*)q, (uint16_t*)qf, cos_table, sin_table, table_rows,
+                     (const uint16_t*)q, q_stride, (uint16_t*)qf, cos_table, sin_table, table_rows,
                      cfg->n_local, rows, cfg->num_heads, zero, cs);
   return check_launch("fingerprint_kernel");
 }
 
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }
 
-}  // namespace ts
-
-using namespace ts;
-
-extern "C" {
-
-int ts_fingerprint(const ts_config* cfg, const void* q, int32_t rows, const float* cos_table,
-                   const float* sin_table, int64_t table_rows, void* qf, ts_stream_t stream) {
-  return launch_fingerprint(cfg, q, rows, cos_table, sin_table, table_rows, qf, ZeroSet{},
-                            (hipStream_t)stream);
-}
-
-size_t ts_prefill_attn_workspace_bytes(const ts_config* cfg, int32_t max_sel_len) {
-  if (validate_config(cfg) != TS_OK || max_sel_len < 1) return 0;
-  return 2 * align_up((size_t)cfg->num_kv_heads * prefill_s_pad(max_sel_len) * kHeadDim * 2, 256);
-}
-
-int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, const void* k_pool,
-                           const void* v_pool, int64_t pool_rows, const int32_t* sel,
-                           const int32_t* sel_len, int32_t max_sel_len, void* out, void* workspace,
-                           size_t workspace_bytes, ts_stream_t stream) {
+int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
+                        const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
+                        int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes,
+                        hipStream_t stream) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(q && k_pool && v_pool && sel && sel_len && out, TS_EINVAL,
              "ts_sparse_prefill_attn: NULL tensor argument");
@@ -813,6 +797,7 @@ int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, co
   TS_REQUIRE_ALIGNED(out, 16, "out");
   PrefillArgs a;
   a.q = (const uint16_t*)q;
+  a.q_stride = q_stride;
   a.k_pool = (const uint16_t*)k_pool;
   a.v_pool = (const uint16_t*)v_pool;
   a.pool_rows = (uint32_t)pool_rows;
@@ -831,7 +816,7 @@ int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, co
   a.kr = (uint16_t*)workspace;
   a.vt = (uint16_t*)((char*)workspace + need / 2);
   a.out = (uint16_t*)out;
-  hipStream_t st = (hipStream_t)stream;
+  hipStream_t st = stream;
   hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)(a.s_pad / kPfKeys), (unsigned)cfg->num_kv_heads),
                      dim3(256), 0, st, a);
   TS_TRY(check_launch("prefill_gather_kernel"));
@@ -866,6 +851,31 @@ int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, co
 #undef TS_PF_CASE
 #undef TS_PF_LAUNCH
   return check_launch("prefill_attn_kernel");
+}
+
+}  // namespace ts
+
+using namespace ts;
+
+extern "C" {
+
+int ts_fingerprint(const ts_config* cfg, const void* q, int32_t rows, const float* cos_table,
+                   const float* sin_table, int64_t table_rows, void* qf, ts_stream_t stream) {
+  return launch_fingerprint(cfg, q, cfg ? cfg->num_heads * cfg->head_dim : 0, rows, cos_table, sin_table, table_rows, qf, ZeroSet{},
+                            (hipStream_t)stream);
+}
+
+size_t ts_prefill_attn_workspace_bytes(const ts_config* cfg, int32_t max_sel_len) {
+  if (validate_config(cfg) != TS_OK || max_sel_len < 1) return 0;
+  return 2 * align_up((size_t)cfg->num_kv_heads * prefill_s_pad(max_sel_len) * kHeadDim * 2, 256);
+}
+
+int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, const void* k_pool,
+                           const void* v_pool, int64_t pool_rows, const int32_t* sel,
+                           const int32_t* sel_len, int32_t max_sel_len, void* out, void* workspace,
+                           size_t workspace_bytes, ts_stream_t stream) {
+  return launch_prefill_attn(cfg, q, cfg ? cfg->num_heads * cfg->head_dim : 0, rows, k_pool, v_pool, pool_rows, sel,
+                             sel_len, max_sel_len, out, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -10,6 +10,7 @@ namespace ts {
 // what the reference's elementwise torch expression does, so that the result is
 // bit-identical for identical tables.
 __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restrict__ x,
+                                                         int64_t x_stride,
                                                          uint16_t* __restrict__ out,
                                                          const float* __restrict__ cos_table,
                                                          const float* __restrict__ sin_table,
@@ -32,15 +33,16 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
   const float* c = cos_table + pos * dim;
   const float* s = sin_table + pos * dim;
   const int64_t base = rh * dim;
-  const float x1 = bf16_to_f32(x[base + i]);
-  const float x2 = bf16_to_f32(x[base + i + half]);
+  const int64_t from = row * x_stride + (rh - row * heads) * dim;
+  const float x1 = bf16_to_f32(x[from + i]);
+  const float x2 = bf16_to_f32(x[from + i + half]);
   const float lo = rotate_element(x1, x2, c[i], s[i], true);
   const float hi = rotate_element(x2, x1, c[i + half], s[i + half], false);
   out[base + i] = f32_to_bf16(lo);
   out[base + i + half] = f32_to_bf16(hi);
 }
 
-int launch_rope(const void* x, void* out, const float* cos_table, const float* sin_table,
+int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
                 const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
                 const ZeroSet& zero, hipStream_t stream) {
   TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);
@@ -50,7 +52,7 @@ int launch_rope(const void* x, void* out, const float* cos_table, const float* s
   const int64_t blocks = std::max(ceil_div(pairs, 256), ceil_div(to_clear, 1024));
   TS_REQUIRE(blocks <= 0x7fffffff, TS_EINVAL, "ts_rope_apply: too many rows");
   hipLaunchKernelGGL(rope_apply_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     (const uint16_t*)x, (uint16_t*)out, cos_table, sin_table, position_ids,
+                     (const uint16_t*)x, x_stride, (uint16_t*)out, cos_table, sin_table, position_ids,
                      table_rows, rows, heads, dim, zero);
   return check_launch("rope_apply_kernel");
 }
@@ -69,6 +71,6 @@ extern "C" int ts_rope_apply(const void* x, void* out, const float* cos_table,
              (long long)table_rows);
   TS_REQUIRE(dim >= 2 && dim % 2 == 0, TS_ESHAPE, "ts_rope_apply: dim %d must be even", dim);
   if (rows == 0) return TS_OK;
-  return launch_rope(x, out, cos_table, sin_table, position_ids, table_rows, rows, heads, dim,
+  return launch_rope(x, (int64_t)heads * dim, out, cos_table, sin_table, position_ids, table_rows, rows, heads, dim,
                      ZeroSet{}, (hipStream_t)stream);
 }

@@ -24,6 +24,7 @@ struct ScoreArgs {
   // q_raw [B,H,128] (un-rotated bf16) itself with the [128] rows q_cos / q_sin, bit-identical
   // to what the rotation kernel would have written to qf.
   const uint16_t* q_raw;
+  int q_stride;            // elements between its rows
   const float* q_cos;
   const float* q_sin;
   const uint16_t* k_pool;  // [pool_rows,Hkv,128] bf16
@@ -203,6 +204,7 @@ const uint32_t* score_votes_fault_word(const ts_config* cfg, int batch, int max_
 // A query that the selection kernel rotates itself (see ScoreArgs::q_raw).
 struct UnrotatedQuery {
   const void* q;
+  int stride;
   const float* cos;
   const float* sin;
 };

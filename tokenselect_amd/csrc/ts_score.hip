@@ -578,7 +578,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         // back), rotated as the rotation kernel does it.
         const bool lower = rg < 2;
         const uint32_t other_off = lower ? lane_off + 128u : lane_off - 128u;
-        const char* qrow = (const char*)(a.q_raw + ((size_t)b * H + h) * kHeadDim);
+        const char* qrow = (const char*)(a.q_raw + (size_t)b * a.q_stride + h * kHeadDim);
         const uint4 own = *(const uint4*)(qrow + lane_off), other = *(const uint4*)(qrow + other_off);
         const float4 c0 = *(const float4*)((const char*)a.q_cos + 2 * lane_off);
         const float4 c1 = *(const float4*)((const char*)a.q_cos + 2 * lane_off + 16);
@@ -1819,6 +1819,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
   a.nchunks = kSelMaxChunks;  // the row of a (request, head) pair in the statistics' table
   if (unrotated) {
     a.q_raw = (const uint16_t*)unrotated->q;
+    a.q_stride = unrotated->stride;
     a.q_cos = unrotated->cos;
     a.q_sin = unrotated->sin;
   }

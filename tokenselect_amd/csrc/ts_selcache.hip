@@ -105,6 +105,7 @@ __global__ __launch_bounds__(256) void selcache_kernel(SelCacheArgs a) {
 // A thread owns units of two 16-byte pieces: dims [8u, 8u + 8) of a head and their rotation
 // partners 64 dims further on.
 __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __restrict__ x,
+                                                           int x_stride,
                                                            uint16_t* __restrict__ qf_out,
                                                            const float* __restrict__ cos_row,
                                                            const float* __restrict__ sin_row,
@@ -135,8 +136,8 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
   const PagePool pool{st.free_pages, st.free_count, st.ticket};
   if (st.k != nullptr) {
     if (first < st.row_vec) {
-      k0 = st.k[(size_t)b * st.row_vec + first];
-      v0 = st.v[(size_t)b * st.row_vec + first];
+      k0 = st.k[(size_t)b * st.kv_stride + first];
+      v0 = st.v[(size_t)b * st.kv_stride + first];
     }
     if (paged) {
       // The plan of the whole batch from the snapshot that no workgroup modifies before the
@@ -171,8 +172,8 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
         st.v_pool[(size_t)store_slot * st.row_vec + first] = v0;
       }
       for (int i = first + 256; i < st.row_vec; i += 256) {
-        st.k_pool[(size_t)store_slot * st.row_vec + i] = st.k[(size_t)b * st.row_vec + i];
-        st.v_pool[(size_t)store_slot * st.row_vec + i] = st.v[(size_t)b * st.row_vec + i];
+        st.k_pool[(size_t)store_slot * st.row_vec + i] = st.k[(size_t)b * st.kv_stride + i];
+        st.v_pool[(size_t)store_slot * st.row_vec + i] = st.v[(size_t)b * st.kv_stride + i];
       }
     }
     // (the workgroups of the requests are the launch that stores: the last of them commits)
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
     geo.dense = (a.n_init + geo.k + a.n_local >= geo.seq_len);
     geo.n = geo.dense ? 0 : geo.seq_len - a.n_init - a.n_local;
   }
-  const uint16_t* q = x + (size_t)b * a.dim;
+  const uint16_t* q = x + (size_t)b * x_stride;
   uint16_t* qo = qf_out + (size_t)b * a.dim;
   uint16_t* qc = a.q_cache + (size_t)b * a.dim;
   const bool have = !geo.dense && a.cache_len[b] > 0 && !(a.gave_up_len && a.gave_up_len[b] < 0);
@@ -342,7 +343,7 @@ int launch_selcache(const ts_config* cfg, const ts_batch* bt, const void* qf, co
   return check_launch("selcache_kernel");
 }
 
-int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q, void* qf,
+int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q, int q_stride, void* qf,
                          const float* q_cos, const float* q_sin, const ts_selcache* cache, int32_t* hit,
                          const int32_t* gave_up_len, const ZeroSet& zero, hipStream_t stream,
                          const StepStore* store) {
@@ -355,7 +356,7 @@ int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q
   TS_REQUIRE_ALIGNED(q_sin, 16, "q_sin");
   const int64_t blocks = bt->batch + std::max<int64_t>(1, ceil_div(zero.total(), 1024));
   hipLaunchKernelGGL(rope_selcache_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     (const uint16_t*)q, (uint16_t*)qf, q_cos, q_sin, a, bt->batch, zero, st);
+                     (const uint16_t*)q, q_stride, (uint16_t*)qf, q_cos, q_sin, a, bt->batch, zero, st);
   return check_launch("rope_selcache_kernel");
 }
 

@@ -31,8 +31,8 @@ __device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, i
     int64_t slot = cs.loc[r];
     slot = slot < 0 ? 0 : (slot >= cs.pool_rows ? cs.pool_rows - 1 : slot);
     for (int i = t; i < cs.row_vec; i += kChunkThreadsPerRow) {
-      cs.k_pool[(size_t)slot * cs.row_vec + i] = cs.k[(size_t)r * cs.row_vec + i];
-      cs.v_pool[(size_t)slot * cs.row_vec + i] = cs.v[(size_t)r * cs.row_vec + i];
+      cs.k_pool[(size_t)slot * cs.row_vec + i] = cs.k[(size_t)r * cs.kv_stride + i];
+      cs.v_pool[(size_t)slot * cs.row_vec + i] = cs.v[(size_t)r * cs.kv_stride + i];
     }
     if (t == 0) cs.table[at] = (int32_t)slot;
   }

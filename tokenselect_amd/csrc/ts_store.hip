@@ -17,15 +17,15 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const uint4* __restrict__
                                                        int32_t* __restrict__ table,
                                                        int64_t table_stride,
                                                        int32_t* __restrict__ seq_lens,
-                                                       int row_vec, int max_tokens) {
+                                                       int row_vec, int kv_stride, int max_tokens) {
   const int b = blockIdx.x;
   // The new rows are asked for together with the slot and the length, not after them: the
   // kernel is two memory round trips long instead of three.
   const int first = threadIdx.x;
   uint4 k0 = make_uint4(0u, 0u, 0u, 0u), v0 = k0;
   if (first < row_vec) {
-    k0 = k[(size_t)b * row_vec + first];
-    v0 = v[(size_t)b * row_vec + first];
+    k0 = k[(size_t)b * kv_stride + first];
+    v0 = v[(size_t)b * kv_stride + first];
   }
   const int slot = loc[b];
   const int len = seq_lens[b];
@@ -35,8 +35,8 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const uint4* __restrict__
     v_pool[(size_t)slot * row_vec + first] = v0;
   }
   for (int i = first + blockDim.x; i < row_vec; i += blockDim.x) {
-    k_pool[(size_t)slot * row_vec + i] = k[(size_t)b * row_vec + i];
-    v_pool[(size_t)slot * row_vec + i] = v[(size_t)b * row_vec + i];
+    k_pool[(size_t)slot * row_vec + i] = k[(size_t)b * kv_stride + i];
+    v_pool[(size_t)slot * row_vec + i] = v[(size_t)b * kv_stride + i];
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -53,8 +53,8 @@ template <bool COUNTED>
 __global__ __launch_bounds__(256) void kv_store_chunk_kernel(
     const uint4* __restrict__ k, const uint4* __restrict__ v, const int32_t* __restrict__ loc,
     uint4* __restrict__ k_pool, uint4* __restrict__ v_pool, int64_t pool_rows,
-    int32_t* __restrict__ table, int32_t* seq_len, int rows, int row_vec, int max_tokens) {
-  ChunkStore cs{k, v, loc, k_pool, v_pool, pool_rows, table, seq_len, rows, row_vec, max_tokens, (int)gridDim.x};
+    int32_t* __restrict__ table, int32_t* seq_len, int rows, int row_vec, int kv_stride, int max_tokens) {
+  ChunkStore cs{k, v, loc, k_pool, v_pool, pool_rows, table, seq_len, rows, row_vec, max_tokens, kv_stride, (int)gridDim.x};
   store_chunk_rows<COUNTED>(cs, (int)blockIdx.x, 256);
 }
 
@@ -71,15 +71,15 @@ __global__ void seq_len_add_kernel(int32_t* seq_len, int rows, int max_tokens) {
 __global__ __launch_bounds__(256) void kv_store_paged_kernel(
     const uint4* __restrict__ k, const uint4* __restrict__ v, uint4* __restrict__ k_pool,
     uint4* __restrict__ v_pool, uint32_t pool_rows, int32_t* table, int64_t table_stride,
-    int32_t* seq_lens, int batch, int row_vec, int max_tokens, int page_shift, PagePool pool) {
+    int32_t* seq_lens, int batch, int row_vec, int kv_stride, int max_tokens, int page_shift, PagePool pool) {
   __shared__ uint32_t plan_slot, plan_ok;
   const int b = blockIdx.x, lane = threadIdx.x & 63;
   // (the new rows are asked for before the plan is made, not after)
   const int first = threadIdx.x;
   uint4 k0 = make_uint4(0u, 0u, 0u, 0u), v0 = k0;
   if (first < row_vec) {
-    k0 = k[(size_t)b * row_vec + first];
-    v0 = v[(size_t)b * row_vec + first];
+    k0 = k[(size_t)b * kv_stride + first];
+    v0 = v[(size_t)b * kv_stride + first];
   }
   if (threadIdx.x < 64)
     for_each_append(seq_lens, table, table_stride, batch, pool, page_shift, max_tokens, pool_rows,
@@ -97,8 +97,8 @@ __global__ __launch_bounds__(256) void kv_store_paged_kernel(
       v_pool[slot * row_vec + first] = v0;
     }
     for (int i = first + blockDim.x; i < row_vec; i += blockDim.x) {
-      k_pool[slot * row_vec + i] = k[(size_t)b * row_vec + i];
-      v_pool[slot * row_vec + i] = v[(size_t)b * row_vec + i];
+      k_pool[slot * row_vec + i] = k[(size_t)b * kv_stride + i];
+      v_pool[slot * row_vec + i] = v[(size_t)b * kv_stride + i];
     }
   }
   __syncthreads();
@@ -135,7 +135,7 @@ __device__ __forceinline__ ChunkPlan make_chunk_plan(const int32_t* seq_len, con
 __global__ __launch_bounds__(256) void kv_store_chunk_paged_kernel(
     const uint4* __restrict__ k, const uint4* __restrict__ v, uint4* __restrict__ k_pool,
     uint4* __restrict__ v_pool, uint32_t pool_rows, int32_t* table, int32_t* seq_len, int rows,
-    int row_vec, int max_tokens, int page_shift, PagePool pool) {
+    int row_vec, int kv_stride, int max_tokens, int page_shift, PagePool pool) {
   const int r = blockIdx.x;
   const ChunkPlan c = make_chunk_plan(seq_len, pool, rows, max_tokens, page_shift);
   if (r < c.stored) {
@@ -146,8 +146,8 @@ __global__ __launch_bounds__(256) void kv_store_chunk_paged_kernel(
     uint32_t slot = ((uint32_t)page << page_shift) + (uint32_t)(at & ((1 << page_shift) - 1));
     slot = slot < pool_rows ? slot : pool_rows - 1;
     for (int i = threadIdx.x; i < row_vec; i += blockDim.x) {
-      k_pool[(size_t)slot * row_vec + i] = k[(size_t)r * row_vec + i];
-      v_pool[(size_t)slot * row_vec + i] = v[(size_t)r * row_vec + i];
+      k_pool[(size_t)slot * row_vec + i] = k[(size_t)r * kv_stride + i];
+      v_pool[(size_t)slot * row_vec + i] = v[(size_t)r * kv_stride + i];
     }
   }
   __syncthreads();
@@ -160,10 +160,6 @@ __global__ __launch_bounds__(256) void kv_store_chunk_paged_kernel(
     __hip_atomic_store(pool.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
-
-}  // namespace ts
-
-using namespace ts;
 
 static int check_pool_arg(const ts_config* cfg, const int32_t* out_cache_loc, const ts_page_pool* pages,
                           const char* who) {
@@ -180,11 +176,10 @@ static int check_pool_arg(const ts_config* cfg, const int32_t* out_cache_loc, co
   return TS_OK;
 }
 
-extern "C" int ts_kv_store(const ts_config* cfg, const void* k, const void* v,
-                           const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool,
-                           void* v_pool, int64_t pool_rows, int32_t* table, int64_t table_stride,
-                           int32_t* seq_lens, int32_t batch, int32_t max_tokens,
-                           ts_stream_t stream) {
+int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
+                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
+                    int32_t max_tokens, hipStream_t stream) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_lens, TS_EINVAL,
              "ts_kv_store: NULL tensor argument");
@@ -200,23 +195,25 @@ extern "C" int ts_kv_store(const ts_config* cfg, const void* k, const void* v,
              "ts_kv_store: table_stride %lld x page_size %d < max_tokens %d", (long long)table_stride,
              cfg->page_size, max_tokens);
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store"));
+  const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
   if (pages) {
-    hipLaunchKernelGGL(kv_store_paged_kernel, dim3((unsigned)batch), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(kv_store_paged_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
                        (const uint4*)k, (const uint4*)v, (uint4*)k_pool, (uint4*)v_pool,
-                       (uint32_t)pool_rows, table, table_stride, seq_lens, batch, row_vec, max_tokens,
+                       (uint32_t)pool_rows, table, table_stride, seq_lens, batch, row_vec, kv_stride, max_tokens,
                        page_shift_of(cfg->page_size), page_pool_of(pages));
     return check_launch("kv_store_paged_kernel");
   }
-  hipLaunchKernelGGL(kv_store_kernel, dim3((unsigned)batch), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(kv_store_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
                      (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                     pool_rows, table, table_stride, seq_lens, row_vec, max_tokens);
+                     pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens);
   return check_launch("kv_store_kernel");
 }
 
-extern "C" int ts_kv_store_chunk(const ts_config* cfg, const void* k, const void* v,
-                                 const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows,
-                                 void* k_pool, void* v_pool, int64_t pool_rows, int32_t* table,
-                                 int32_t* seq_len, int32_t max_tokens, ts_stream_t stream) {
+int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                          const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
+                          void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
+                          hipStream_t stream) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_len, TS_EINVAL,
              "ts_kv_store_chunk: NULL tensor argument");
@@ -230,25 +227,49 @@ extern "C" int ts_kv_store_chunk(const ts_config* cfg, const void* k, const void
              (long long)pool_rows, max_tokens);
   if (rows == 0) return TS_OK;
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store_chunk"));
+  const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
   if (pages) {
     hipLaunchKernelGGL(kv_store_chunk_paged_kernel, dim3((unsigned)rows), dim3(256), 0,
-                       (hipStream_t)stream, (const uint4*)k, (const uint4*)v, (uint4*)k_pool,
-                       (uint4*)v_pool, (uint32_t)pool_rows, table, seq_len, rows, row_vec, max_tokens,
+                       stream, (const uint4*)k, (const uint4*)v, (uint4*)k_pool,
+                       (uint4*)v_pool, (uint32_t)pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens,
                        page_shift_of(cfg->page_size), page_pool_of(pages));
     return check_launch("kv_store_chunk_paged_kernel");
   }
   const unsigned wgs = (unsigned)ceil_div(rows, kChunkRowsPerWg);
   if (wgs <= (unsigned)kChunkCountedWgs && max_tokens <= kLenMask) {
-    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs), dim3(256), 0, stream,
                        (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                       pool_rows, table, seq_len, rows, row_vec, max_tokens);
+                       pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens);
     return check_launch("kv_store_chunk_kernel");
   }
-  hipLaunchKernelGGL(kv_store_chunk_kernel<false>, dim3(wgs), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(kv_store_chunk_kernel<false>, dim3(wgs), dim3(256), 0, stream,
                      (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                     pool_rows, table, seq_len, rows, row_vec, max_tokens);
+                     pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens);
   TS_TRY(check_launch("kv_store_chunk_kernel"));
-  hipLaunchKernelGGL(seq_len_add_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, seq_len, rows,
+  hipLaunchKernelGGL(seq_len_add_kernel, dim3(1), dim3(1), 0, stream, seq_len, rows,
                      max_tokens);
   return check_launch("seq_len_add_kernel");
 }
+
+}  // namespace ts
+
+using namespace ts;
+
+extern "C" {
+
+int ts_kv_store(const ts_config* cfg, const void* k, const void* v, const int32_t* out_cache_loc,
+                const ts_page_pool* pages, void* k_pool, void* v_pool, int64_t pool_rows, int32_t* table,
+                int64_t table_stride, int32_t* seq_lens, int32_t batch, int32_t max_tokens, ts_stream_t stream) {
+  return launch_kv_store(cfg, k, v, 0, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride,
+                         seq_lens, batch, max_tokens, (hipStream_t)stream);
+}
+
+int ts_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, const int32_t* out_cache_loc,
+                      const ts_page_pool* pages, int32_t rows, void* k_pool, void* v_pool, int64_t pool_rows,
+                      int32_t* table, int32_t* seq_len, int32_t max_tokens, ts_stream_t stream) {
+  return launch_kv_store_chunk(cfg, k, v, 0, out_cache_loc, pages, rows, k_pool, v_pool, pool_rows, table, seq_len,
+                               max_tokens, (hipStream_t)stream);
+}
+
+}  // extern "C"

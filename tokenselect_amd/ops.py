@@ -164,6 +164,19 @@ class _GiveUpLatch:
                                              self.sel_pos, self.sel_len, self.fault, batch,
                                              self.max_seq_len, max_rows)
 
+    def _serve(self, q, k, v, loc, k_pool, v_pool, bt, cache=None, out=None, start: int = 0,
+               rows: int = 0) -> torch.Tensor:
+        """:meth:`step` for a serving stack whose q, k and v are parts of one projection (rows
+        of any stride are read where they lie), with slots chosen by the stack: a decode
+        step's output as a fresh tensor, or the chunk of ``rows`` rows of a prompt from row
+        ``start`` on, written to the same rows of ``out``."""
+        got = self._native.serve(q, k, v, loc, k_pool, v_pool, bt, cache, out, start, rows, self.separate)
+        if got is None:   # an earlier call gave up
+            self.check()
+        if type(got) is int:
+            _lib.check(got)
+        return got
+
     def _run(self, q, k, v, loc, k_pool, v_pool, bt, cache, out, pages, store: bool, rerun: bool = False):
         got = self._native.run(q, k, v, loc, k_pool, v_pool, bt, cache, out, pages, store, self.separate, rerun)
         if type(got) is tuple:
@@ -726,15 +739,20 @@ class DecodeLayer(_GiveUpLatch):
     step's selection and attention with the separate kernels (the KV store before the
     layer is not repeated) and keeps the object on them."""
 
-    def __init__(self, cfg: LayerConfig, batch: int, max_seq_len: int, device):
+    def __init__(self, cfg: LayerConfig, batch: int, max_seq_len: int, device, tables=None):
+        """``tables``: the ``(cos, sin)`` of :func:`rope_tables` with at least
+        ``n_local + 1`` rows, where the caller has them already."""
         self.cfg, self.batch, self.max_seq_len = cfg, batch, max_seq_len
         self._c = cfg.to_c()
         lib = _lib.load()
         _lib.check(lib.ts_check_config(ctypes.byref(self._c)))
         nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(self._c), batch, max_seq_len)
         self.workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
-        self.q_cos, self.q_sin = scoring_cos_sin(cfg.head_dim, cfg.rope_theta, cfg.rope_scale,
-                                                 cfg.n_local, device)
+        if tables is not None:
+            self.q_cos, self.q_sin = (t[cfg.n_local:cfg.n_local + 1] for t in tables)
+        else:
+            self.q_cos, self.q_sin = scoring_cos_sin(cfg.head_dim, cfg.rope_theta, cfg.rope_scale,
+                                                     cfg.n_local, device)
         self.out = torch.empty((batch, cfg.num_heads * cfg.head_dim), dtype=torch.bfloat16,
                                device=device)
         self.sel = torch.empty((batch, cfg.max_sel), dtype=torch.int32, device=device)
@@ -918,15 +936,17 @@ class PrefillChunk(_GiveUpLatch):
     single library call, for one request; buffers are allocated once.  :meth:`recover`
     as for :class:`DecodeLayer`."""
 
-    def __init__(self, cfg: LayerConfig, max_seq_len: int, device, max_rows: int = 512):
+    def __init__(self, cfg: LayerConfig, max_seq_len: int, device, max_rows: int = 512, tables=None):
+        """``tables``: the ``(cos, sin)`` of :func:`rope_tables` with ``n_local + max_rows``
+        rows, where the caller has them already."""
         self.cfg, self.max_seq_len, self.max_rows = cfg, max_seq_len, max_rows
         self._c = cfg.to_c()
         lib = _lib.load()
         _lib.check(lib.ts_check_config(ctypes.byref(self._c)))
         nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(self._c), 1, max_seq_len)
         self.workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
-        self.cos, self.sin = rope_tables(cfg.head_dim, cfg.rope_theta, cfg.rope_scale,
-                                         cfg.n_local + max_rows, device)
+        self.cos, self.sin = tables if tables is not None else rope_tables(
+            cfg.head_dim, cfg.rope_theta, cfg.rope_scale, cfg.n_local + max_rows, device)
         self.sel = torch.empty((1, cfg.max_sel), dtype=torch.int32, device=device)
         self.sel_pos = torch.empty_like(self.sel)
         self.sel_len = torch.empty((1,), dtype=torch.int32, device=device)

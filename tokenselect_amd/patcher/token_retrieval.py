@@ -29,7 +29,7 @@ classes of :mod:`tokenselect_amd.patcher.sglang_standins` are patched.
 """
 
 from contextlib import contextmanager
-from math import ceil
+from functools import cached_property
 from typing import Optional
 
 import torch
@@ -98,6 +98,16 @@ class RotaryEmbedding(torch.nn.Module):
             angles = torch.cat((angles, angles), dim=-1)
             self._cos_table = angles.cos().unsqueeze(1).to(self.device)
             self._sin_table = angles.sin().unsqueeze(1).to(self.device)
+
+    def layer_tables(self, rows: int):
+        """``(cos, sin)`` tables [>= rows, dim] of ``ops.rope_tables``, built once for all the
+        retrievers that share this embedding: on the host and copied, they took 230 us of
+        every new request (None without the patched globals' base and scale)."""
+        held = getattr(self, "_layer_tables", None)
+        if held is None or held[0].shape[0] < rows:
+            held = ops.rope_tables(self.dim, float(self.base), float(self.distance_scale), rows, self.device)
+            self._layer_tables = held
+        return held
 
     def apply_rotary_pos_emb(self, x: torch.Tensor, position_ids: torch.Tensor,
                              max_position: Optional[int] = None) -> torch.Tensor:
@@ -188,7 +198,9 @@ class BatchTokenRetriever:
         self.num_tokens = [[r.num_tokens[l] for r in retrievers] for l in range(self.num_layers)]
         self._num_tokens_dev = torch.stack([r._num_tokens_dev for r in retrievers], dim=1).contiguous()
         self._threshold_hints = torch.stack([r._threshold_hints for r in retrievers], dim=1).contiguous()
+        self.rope_embedding = first.rope_embedding
         self._layers = {}
+        self._batches = {}
         self._caches = None
         if QUERY_CACHE:
             self._caches = [ops.SelectionCache(
@@ -219,23 +231,37 @@ class BatchTokenRetriever:
                      self.token_indices[layer], self._num_tokens_dev[layer])
         self._note_appended(layer, loc.shape[0])
 
+    def _batch_of(self, layer_id, lens) -> ops.Batch:
+        """The layer's ``Batch`` for the lengths ``lens``.  They go along on the host too: a
+        batch that is too large for one selection launch is then scored in phases packed by
+        what the requests hold."""
+        bt = self._batches.get(layer_id)
+        if bt is None:
+            bt = ops.Batch(self._num_tokens_dev[layer_id], self.token_indices[layer_id], 0,
+                           hint=self._threshold_hints[layer_id])
+            self._batches[layer_id] = bt
+        bt.max_seq_len = max(lens)
+        bt.host_seq_lens = torch.tensor(lens, dtype=torch.int32)
+        return bt
+
     def decode_attention(self, attn, q, k_buffer, v_buffer):
         """One fused library call for a decode layer of the whole batch (tr.py:791-825 per request)."""
         layer_id = attn.layer_id
-        cfg = self._config(N_INIT, N_Local, TOP_K, attn.scaling, attn.logit_cap)
-        key = (attn.scaling, attn.logit_cap)
-        runner = self._layers.get(key)
-        if runner is None:
-            runner = ops.DecodeLayer(cfg, self.batch, self.max_num_tokens, self.device)
-            self._layers[key] = runner
-        # The lengths go along on the host too: a batch that is too large for one selection
-        # launch is then scored in phases packed by what the requests hold.
-        bt = ops.Batch(self._num_tokens_dev[layer_id], self.token_indices[layer_id],
-                       max(self.num_tokens[layer_id]),
-                       host_seq_lens=torch.tensor(self.num_tokens[layer_id], dtype=torch.int32),
-                       hint=self._threshold_hints[layer_id])
+        bt = self._batch_of(layer_id, self.num_tokens[layer_id])
         out = torch.empty((self.batch, self.num_heads * self.head_dim), dtype=q.dtype, device=q.device)
-        runner(q, k_buffer, v_buffer, bt, self._caches[layer_id] if self._caches else None, out=out)
+        _decode_layer(self, attn, self.batch)(q, k_buffer, v_buffer, bt,
+                                              self._caches[layer_id] if self._caches else None, out=out)
+        return out
+
+    def decode_step(self, attn, q, k, v, loc, k_buffer, v_buffer):
+        """Store and :meth:`decode_attention` in one library call (tr.py:777-825)."""
+        layer_id = attn.layer_id
+        lens = [n + 1 for n in self.num_tokens[layer_id]]
+        assert max(lens) <= self.max_num_tokens   # tr.py:334
+        out = _decode_layer(self, attn, self.batch)._serve(
+            q, k, v, loc, k_buffer, v_buffer, self._batch_of(layer_id, lens),
+            self._caches[layer_id] if self._caches else None)
+        self.num_tokens[layer_id] = lens
         return out
 
 
@@ -245,6 +271,27 @@ def paged_matmul(query, token, indices, scores, num_relevant_tokens, num_heads, 
     ignored (the HIP kernel chooses its own tiling)."""
     ops.paged_matmul(query, token, indices, scores, num_relevant_tokens, num_heads, num_kv_heads,
                      head_dim)
+
+
+def _layer_tables(retriever, rows):
+    """The rotation tables of a retriever's layer objects, where it shares an embedding."""
+    rotary = retriever.rope_embedding
+    if rotary is None or rotary.base != ROPE_BASE or rotary.distance_scale != ROPE_SCALE \
+            or rotary.dim != retriever.head_dim:
+        return None
+    return rotary.layer_tables(rows)
+
+
+def _decode_layer(retriever, attn, batch) -> ops.DecodeLayer:
+    """The retriever's layer object for attention modules of this scaling and cap."""
+    key = (attn.scaling, attn.logit_cap)
+    runner = retriever._layers.get(key)
+    if runner is None:
+        cfg = retriever._config(N_INIT, N_Local, TOP_K, attn.scaling, attn.logit_cap)
+        runner = ops.DecodeLayer(cfg, batch, retriever.max_num_tokens, retriever.device,
+                                 tables=_layer_tables(retriever, int(N_Local) + max(PREFILL_CHUNK_SIZE, 1)))
+        retriever._layers[key] = runner
+    return runner
 
 
 class TokenRetriever:
@@ -267,36 +314,49 @@ class TokenRetriever:
         self.token_indices = torch.empty((num_layers, max_num_tokens), device=device,
                                          dtype=torch.int32)
         self.rope_embedding = rotary_embedding
-        top_k = max(int(TOP_K), 1)
-        self.query_fingerprints_cache = torch.zeros((num_layers, num_heads * head_dim),
-                                                    device=device, dtype=dtype)
-        # int32 here (the reference keeps int64, tr.py:307-311): positions fit and
-        # the library's tables are 32-bit.
-        self.topk_indices_cache = torch.zeros((num_layers, top_k), device=device, dtype=torch.int32)
-        self.similarity_threshold = torch.tensor([0.9] * num_layers, device=device, dtype=dtype)
-        self._threshold_host = float(torch.tensor(0.9, dtype=dtype))  # 0.8984375 in bf16
+        self._top_k = max(int(TOP_K), 1)
         self.skip_count = 0
         self.retrieval_count = 0
-        self.is_first_query = [True] * num_layers
-        # Device-side twins of the host bookkeeping, read by the kernels.
-        self._num_tokens_dev = torch.zeros((num_layers,), device=device, dtype=torch.int32)
-        self._cache_len_dev = torch.zeros((num_layers,), device=device, dtype=torch.int32)
-        self._counters_dev = torch.zeros((num_layers, 2), device=device, dtype=torch.int64)
-        # Where the k-th vote of a layer's last selection lay: the single-launch selection's
-        # guess for the next step (ts_batch.threshold_hint), one word per layer.
-        self._threshold_hints = torch.zeros((num_layers,), device=device, dtype=torch.int32)
+        # Device-side twins of the host bookkeeping, read by the kernels, all in one
+        # allocation that one launch clears: [L, 2] int64 counters, then [L] int32 each of the
+        # lengths, the selection cache's fill and where the k-th vote of a layer's last
+        # selection lay (the single-launch selection's guess for the next step,
+        # ts_batch.threshold_hint).
+        self._words = torch.zeros((7 * num_layers,), device=device, dtype=torch.int32)
+        self._counters_dev = self._words[:4 * num_layers].view(torch.int64).view(num_layers, 2)
+        self._num_tokens_dev, self._cache_len_dev, self._threshold_hints = \
+            self._words[4 * num_layers:].view(3, num_layers).unbind(0)
         self._layers = {}
-        self.clear()
+        self._batches = {}
+        self.num_tokens = [0] * num_layers
+        self.is_first_query = [True] * num_layers
+
+    # The selection cache's arrays (tr.py:301-316) exist from their first use on.
+    @cached_property
+    def query_fingerprints_cache(self):
+        return torch.zeros((self.num_layers, self.num_heads * self.head_dim), device=self.device,
+                           dtype=self.dtype)
+
+    @cached_property
+    def topk_indices_cache(self):
+        # int32 here (the reference keeps int64, tr.py:307-311): positions fit and
+        # the library's tables are 32-bit.
+        return torch.zeros((self.num_layers, self._top_k), device=self.device, dtype=torch.int32)
+
+    @cached_property
+    def similarity_threshold(self):
+        return torch.tensor([0.9] * self.num_layers, device=self.device, dtype=self.dtype)
+
+    @cached_property
+    def _threshold_host(self):
+        return float(torch.tensor(0.9, dtype=self.dtype))  # 0.8984375 in bf16
 
     # ------------------------------------------------------------ bookkeeping
     def clear(self):
         self.num_tokens = [0] * self.num_layers
         self.is_first_query = [True] * self.num_layers
         self.skip_count = 0
-        self._num_tokens_dev.zero_()
-        self._cache_len_dev.zero_()
-        self._counters_dev.zero_()
-        self._threshold_hints.zero_()
+        self._words.zero_()
 
     def get_all_tokens(self, layer_id):
         return self.token_indices[layer_id, : self.num_tokens[layer_id]]
@@ -436,43 +496,78 @@ class TokenRetriever:
         return sel[0, : n_init + topk + n_local]
 
     # ------------------------------------------------------- fused decode step
+    def _batch_of(self, layer_id, length) -> ops.Batch:
+        """The layer's one-request ``Batch`` for a length."""
+        bt = self._batches.get(layer_id)
+        if bt is None:
+            bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
+                           self.token_indices[layer_id:layer_id + 1], 0,
+                           hint=self._threshold_hints[layer_id:layer_id + 1])
+            self._batches[layer_id] = bt
+        bt.max_seq_len = length
+        return bt
+
     def decode_attention(self, attn, q, k_buffer, v_buffer):
         """One fused library call for a decode layer: selection (or the dense
         fallback) and the attention over the result (tr.py:791-825)."""
         layer_id = attn.layer_id
-        cfg = self._config(N_INIT, N_Local, TOP_K, attn.scaling, attn.logit_cap)
-        key = (attn.scaling, attn.logit_cap)
-        runner = self._layers.get(key)
-        if runner is None:
-            runner = ops.DecodeLayer(cfg, 1, self.max_num_tokens, self.device)
-            self._layers[key] = runner
-        bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
-                       self.token_indices[layer_id:layer_id + 1], self.num_tokens[layer_id],
-                       hint=self._threshold_hints[layer_id:layer_id + 1])
+        bt = self._batch_of(layer_id, self.num_tokens[layer_id])
         out = torch.empty((1, self.num_heads * self.head_dim), dtype=q.dtype, device=q.device)
         cache = self._cache(layer_id)
-        runner(q, k_buffer, v_buffer, bt, cache, out=out)
+        _decode_layer(self, attn, 1)(q, k_buffer, v_buffer, bt, cache, out=out)
         if cache is not None:
             self.is_first_query[layer_id] = False
         return out
 
+    def decode_step(self, attn, q, k, v, loc, k_buffer, v_buffer):
+        """Store and :meth:`decode_attention` in one library call (tr.py:777-825)."""
+        layer_id = attn.layer_id
+        length = self.num_tokens[layer_id] + 1
+        assert length <= self.max_num_tokens   # tr.py:334
+        cache = self._cache(layer_id)
+        out = _decode_layer(self, attn, 1)._serve(q, k, v, loc, k_buffer, v_buffer,
+                                                  self._batch_of(layer_id, length), cache)
+        self.num_tokens[layer_id] = length
+        if cache is not None:
+            self.is_first_query[layer_id] = False
+        return out
 
     # ------------------------------------------------------ fused prefill chunk
+    def _prefill_chunk(self, attn) -> ops.PrefillChunk:
+        key = ("prefill", attn.scaling, attn.logit_cap)
+        runner = self._layers.get(key)
+        if runner is None:
+            cfg = self._config(N_INIT, N_Local, TOP_K, attn.scaling, attn.logit_cap)
+            rows = max(PREFILL_CHUNK_SIZE, 1)
+            runner = ops.PrefillChunk(cfg, self.max_num_tokens, self.device, max_rows=rows,
+                                      tables=_layer_tables(self, int(N_Local) + rows))
+            self._layers[key] = runner
+        return runner
+
     def prefill_attention(self, attn, q, k_buffer, v_buffer):
         """One fused library call for a prefill chunk after its KV store: chunk
         fingerprint, selection (or the dense fallback) and the causal attention of the
         chunk's rows over the result (tr.py:735-773)."""
         layer_id = attn.layer_id
-        cfg = self._config(N_INIT, N_Local, TOP_K, attn.scaling, attn.logit_cap)
-        key = ("prefill", attn.scaling, attn.logit_cap)
-        runner = self._layers.get(key)
-        if runner is None:
-            runner = ops.PrefillChunk(cfg, self.max_num_tokens, self.device,
-                                      max_rows=max(PREFILL_CHUNK_SIZE, 1))
-            self._layers[key] = runner
         bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
                        self.token_indices[layer_id:layer_id + 1], self.num_tokens[layer_id])
-        out, _, _, _ = runner(q, k_buffer, v_buffer, bt)
+        out, _, _, _ = self._prefill_chunk(attn)(q, k_buffer, v_buffer, bt)
+        return out
+
+    def prefill_step(self, attn, q, k, v, loc, k_buffer, v_buffer, out):
+        """The whole prompt part in chunks (tr.py:716-773), each one library call: its store,
+        then :meth:`prefill_attention`, the rows of ``out`` written in place."""
+        layer_id, rows = attn.layer_id, q.shape[0]
+        runner = self._prefill_chunk(attn)
+        bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
+                       self.token_indices[layer_id:layer_id + 1], 0)
+        for start in range(0, rows, PREFILL_CHUNK_SIZE):
+            here = min(PREFILL_CHUNK_SIZE, rows - start)
+            length = self.num_tokens[layer_id] + here
+            assert length <= self.max_num_tokens   # tr.py:334
+            bt.max_seq_len = length
+            runner._serve(q, k, v, loc, k_buffer, v_buffer, bt, None, out, start, here)
+            self.num_tokens[layer_id] = length
         return out
 
 
@@ -507,14 +602,25 @@ def patched_radix_attention_store_kv_cache(self, cache_k, cache_v, input_metadat
     retriever.add_k_cache(loc, self.layer_id)
 
 
+def _one_call(attn, loc, rows) -> bool:
+    """Whether the store of ``rows`` new tokens can be left to the library's step calls: 32-bit
+    slots, one per row, and a store that is the patched one."""
+    return loc.dtype == torch.int32 and loc.dim() == 1 and loc.shape[0] == rows and \
+        getattr(attn.store_kv_cache, "__func__", None) is patched_radix_attention_store_kv_cache
+
+
 def patched_radix_attention_decode_forward_flashinfer(self, q, k, v, input_metadata):
     """tr.py:777-825 without FlashInfer: store, select, attend."""
     if self.sliding_window_size != -1:
         raise NotImplementedError("Sliding window not supported yet")
+    retriever, loc = input_metadata.token_retriever, input_metadata.out_cache_loc
+    batched = isinstance(retriever, BatchTokenRetriever)
     if k is not None:
         assert v is not None
+        if q.shape[0] == (retriever.batch if batched else 1) and _one_call(self, loc, q.shape[0]):
+            k_buffer, v_buffer = input_metadata.token_to_kv_pool.get_kv_buffer(self.layer_id)
+            return retriever.decode_step(self, q, k, v, loc, k_buffer, v_buffer)
         self.store_kv_cache(k, v, input_metadata)
-    batched = isinstance(input_metadata.token_retriever, BatchTokenRetriever)
     if q.shape[0] != (input_metadata.token_retriever.batch if batched else 1):
         raise NotImplementedError(
             "the patched decode forward serves one running request, as the reference does "
@@ -531,12 +637,14 @@ def patched_radix_attention_extend_forward_flashinfer(self, q, k, v, input_metad
     if self.sliding_window_size != -1:
         raise NotImplementedError("Sliding window not supported yet")
     assert not getattr(input_metadata, "flashinfer_use_ragged", False)  # not supported yet
-    num_chunks = ceil(q.shape[0] / PREFILL_CHUNK_SIZE)
-    outputs = torch.empty_like(q)
+    outputs = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     k_buffer, v_buffer = input_metadata.token_to_kv_pool.get_kv_buffer(self.layer_id)
-    for chunk_idx in range(num_chunks):
-        start = chunk_idx * PREFILL_CHUNK_SIZE
-        end = min((chunk_idx + 1) * PREFILL_CHUNK_SIZE, q.shape[0])
+    retriever, loc = input_metadata.token_retriever, input_metadata.out_cache_loc
+    if k is not None and v is not None and isinstance(retriever, TokenRetriever) and q.dim() == 2 \
+            and _one_call(self, loc, q.shape[0]):
+        return retriever.prefill_step(self, q, k, v, loc, k_buffer, v_buffer, outputs)
+    for start in range(0, q.shape[0], PREFILL_CHUNK_SIZE):
+        end = min(start + PREFILL_CHUNK_SIZE, q.shape[0])
         if k is not None:
             assert v is not None
             self.store_kv_cache(k, v, input_metadata, start=start, end=end)
