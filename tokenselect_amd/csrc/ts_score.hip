@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 #include <vector>
 
 #include "ts_score.h"
@@ -141,8 +142,8 @@ __device__ __forceinline__ void merge_request_stats(const ScoreArgs& a, const La
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int c = base + 64 * i + lane;
-          v[i] = c < chunks ? load_coherent(part + c) : make_float2(kNegBig, 1.f);
-          there = there && __float_as_uint(v[i].y) != 0u;
+          v[i] = c < chunks ? load_coherent(part + c) : make_float2(kNegBig, 0.f);
+          there = there && (c >= chunks || __float_as_uint(v[i].y) != 0u);
         }
         if (__all(there) || lost) break;
         if ((polls & 7u) == 0) {
@@ -153,23 +154,35 @@ __device__ __forceinline__ void merge_request_stats(const ScoreArgs& a, const La
             lost = true;
           }
         }
-        __builtin_amdgcn_s_sleep(8);  // some 0.2 us between the polls of a few dozen wavefronts
+        __builtin_amdgcn_s_sleep(2);  // (a few dozen wavefronts poll)
       }
+      // The maximum first, then every sum scaled to it: one exponential per entry, none of
+      // them waiting for another.  (An entry past the last chunk has the weight zero.)
+      float top = m;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int c = base + 64 * i + lane;
-        if (c < chunks) softmax_merge(m, l, v[i].x, v[i].y);
-      }
+      for (int i = 0; i < 8; ++i) top = fmaxf(top, v[i].x);
+      top = fmaxf(top, dpp_move<kRowRor8>(top));
+      top = fmaxf(top, dpp_move<kRowRor4>(top));
+      top = fmaxf(top, dpp_move<kRowRor2>(top));
+      top = fmaxf(top, dpp_move<kRowRor1>(top));
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      float add = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (base + 64 * i < chunks) add += v[i].y * __expf(v[i].x - top);
+      add = row16_sum(add);
+      add += __shfl_xor(add, 16);
+      add += __shfl_xor(add, 32);
+      l = l * __expf(m - top) + add;
+      m = top;
     }
-    row16_softmax_merge(m, l);
-    softmax_merge(m, l, __shfl_xor(m, 16), __shfl_xor(l, 16));
-    softmax_merge(m, l, __shfl_xor(m, 32), __shfl_xor(l, 32));
     store_coherent((float2*)(a.stats + (size_t)lane * a.stats_stride) + (size_t)b * H + h, m, l);
   }
 }
 
-constexpr int kStatsPollSleep = 12;     // x 64 clocks between a workgroup's polls for the merged statistics
-constexpr uint32_t kSelectRounds = 4;  // rendezvous of the fused kernel at most (without the max-pool's)
+constexpr int kStatsPollSleep = 4;     // x 64 clocks between a workgroup's polls for the merged statistics
+constexpr uint32_t kSelectRounds = 5;  // rendezvous of the fused kernel at most (without the max-pool's)
 
 #ifdef TS_TRACE  // development builds only: per-workgroup phase timestamps of the fused kernel
 #include "ts_trace.h"
@@ -223,6 +236,7 @@ struct Deal {
   int tokens_per_block;  // of every selecting request of this launch
   int req;               // this workgroup's request (within the launch), -1: none
   int chunk, chunks;     // its chunk of that request, and the request's chunks
+  int n;                 // the request's candidates
   uint32_t team_size, team_index;
 };
 constexpr int kDealPerLane = 8;  // requests per lane of the dealing wavefront: batches of up to 512
@@ -237,12 +251,13 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int B = a.batch, T = (int)gridDim.x, w = (int)blockIdx.x;
   if (B == 1) {  // one request: every thread works it out for itself, no exchange
-    Deal d{a.tokens_per_block, -1, 0, 0, a.absent, (uint32_t)w};
+    Deal d{a.tokens_per_block, -1, 0, 0, 0, a.absent, (uint32_t)w};
     int n = 0;
     if (!(a.skip && a.skip[a.batch_offset]))
       n = request_geometry(a.seq_lens, a.k_per_req, a.batch_offset, a.n_init, a.n_local, a.top_k,
                            a.max_seq_len).n;
     if (n <= 0) return d;
+    d.n = n;
     int tpb = max((n + T * 64 - 1) / (T * 64) * 64, 64);
     while ((n + tpb - 1) / tpb > T && tpb < a.tokens_per_block) tpb += 64;
     d.tokens_per_block = tpb;
@@ -262,7 +277,8 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
     for (int j = 0; j < kDealPerLane; ++j) {
       const int b = lane + 64 * j;
       n[j] = 0;
-      if (64 * j < B && b < B && !(a.skip && a.skip[a.batch_offset + b]))
+      if (64 * j >= B) continue;
+      if (b < B && !(a.skip && a.skip[a.batch_offset + b]))
         n[j] = request_geometry(a.seq_lens, a.k_per_req, a.batch_offset + b, a.n_init, a.n_local, a.top_k,
                                 a.max_seq_len).n;
       all += n[j];
@@ -278,13 +294,15 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
       int mine = 0;
 #pragma unroll
       for (int j = 0; j < kDealPerLane; ++j) {
-        chunks[j] = 64 * j < B ? (n[j] + tpb - 1) / tpb : 0;
+        chunks[j] = 0;
+        if (64 * j >= B) continue;
+        chunks[j] = (n[j] + tpb - 1) / tpb;
         mine += chunks[j];
       }
       if (wave_sum(mine) <= T || tpb >= a.tokens_per_block) break;
     }
     // First workgroup of every request, in request order (lane + 64 j: j by j).
-    int base = 0, req = -1, chunk = 0, req_chunks = 0;
+    int base = 0, req = -1, chunk = 0, req_chunks = 0, req_n = 0;
 #pragma unroll
     for (int j = 0; j < kDealPerLane; ++j) {
       if (64 * j >= B) break;
@@ -302,6 +320,7 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
         req = 64 * j + src;
         chunk = w - __shfl(first, src);
         req_chunks = __shfl(chunks[j], src);
+        req_n = __shfl(n[j], src);
       }
       base += __shfl(incl, 63);
     }
@@ -311,6 +330,7 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
       lds[2] = chunk;
       lds[3] = req_chunks;
       lds[4] = base;  // workgroups with tokens: the team
+      lds[5] = req_n;
     }
   }
   __syncthreads();
@@ -319,13 +339,14 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
   d.req = lds[1];
   d.chunk = lds[2];
   d.chunks = lds[3];
+  d.n = lds[5];
   d.team_size = (uint32_t)lds[4] + a.absent;
   d.team_index = (uint32_t)w;
   __syncthreads();
   return d;
 }
 
-// The parts of the output that need no votes, written while the keys stream: a
+// The parts of the output that need no votes, written while the statistics are on their way: a
 // dense request gets all its positions and a selection-cache hit its cached ones
 // (both spread over the request's workgroups); workgroup 0 of a request writes the
 // length, the sink and the local window, and clears the words the next kernel of
@@ -366,6 +387,28 @@ __device__ __forceinline__ void fixed_segments(const ScoreArgs& a, int b, int x,
   }
   for (int i = threadIdx.x; i < a.n_init; i += 256) emit(i, i);
   for (int i = threadIdx.x; i < a.n_local; i += 256) emit(a.n_init + k + i, L - a.n_local + i);
+}
+
+// Sum over the wavefront, in every lane.
+__device__ __forceinline__ uint32_t wave_total(uint32_t x) {
+  auto ror = [](uint32_t v, auto ctrl) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+  };
+  x += ror(x, std::integral_constant<int, kRowRor8>{});
+  x += ror(x, std::integral_constant<int, kRowRor4>{});
+  x += ror(x, std::integral_constant<int, kRowRor2>{});
+  x += ror(x, std::integral_constant<int, kRowRor1>{});
+  return (uint32_t)(__builtin_amdgcn_readlane((int)x, 0) + __builtin_amdgcn_readlane((int)x, 16) +
+                    __builtin_amdgcn_readlane((int)x, 32) + __builtin_amdgcn_readlane((int)x, 48));
+}
+
+// This workgroup's share of the launch's parts that need no votes: counted from the last
+// workgroup down, those of request w % B, as one of the workgroups w % B, w % B + B, ...
+// (The first workgroups of the team merge the statistics, and everybody waits for those; the
+// last ones often have no candidates.)
+__device__ __forceinline__ void fixed_parts(const ScoreArgs& a) {
+  const int B = a.batch, T = (int)gridDim.x, w = T - 1 - (int)blockIdx.x;
+  fixed_segments(a, a.batch_offset + w % B, w / B, (T - w % B + B - 1) / B);
 }
 
 // Adds the wavefront's candidates to a histogram in memory with one fetch-add per
@@ -498,6 +541,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   LaunchPart lp{a.tokens_per_block, a.batch_offset, 0, nullptr, (int)blockIdx.x, a.sync};
   int req = blockIdx.y, chunk = blockIdx.x;
   int req_chunks = (int)gridDim.x;  // chunks of this workgroup's request (the single launch: dealt)
+  int dealt_n = 0;
   GridTeam team{0u, 0u};
   if (PACKED) {
     TS_MARK(0);
@@ -514,22 +558,24 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   if constexpr (FUSED && !PACKED) {
     __shared__ int deal_lds[8];
     TS_MARK(0);
-    // The parts of the output that need no votes: request w % B by workgroup w / B of its share.
-    {
-      const int B = a.batch, w = (int)blockIdx.x, T = (int)gridDim.x;
-      fixed_segments(a, a.batch_offset + w % B, w / B, (T - w % B + B - 1) / B);
-    }
     const Deal deal = deal_workgroups(a, deal_lds);
-    if (deal.req < 0) return;  // no chunk left for this workgroup
+    if (deal.req < 0) {  // no chunk left for this workgroup
+      fixed_parts(a);
+      return;
+    }
     lp.tokens_per_block = deal.tokens_per_block;
     req = deal.req;
     chunk = deal.chunk;
     req_chunks = deal.chunks;
+    dealt_n = deal.n;
     team = GridTeam{deal.team_size, deal.team_index};
   }
   const int b = req + lp.batch_offset;
   int n, first_pos;
-  if (a.direct_n >= 0) {
+  if (FUSED && !PACKED) {
+    n = dealt_n;
+    first_pos = a.n_init;
+  } else if (a.direct_n >= 0) {
     n = (int)a.direct_n;
     first_pos = 0;
   } else {
@@ -564,29 +610,51 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   const int tile_stride = FUSED ? 16 * H + 16 : 16 * H;
   const int32_t* tab = a.table + (int64_t)b * a.table_stride;
 
-  // A operands: query 4*na + t4 of each KV head, same byte offsets as the keys.
-  bf16x8_t qa[HKV][NA];
+  // A operands: query 4*na + t4 of each KV head, same byte offsets as the keys.  The four
+  // wavefronts share the work of preparing them: wavefront w loads the operands w, w + 4, ...
+  // (one of which is also rotated where the kernel does that itself: the 8 dims 64 further on
+  // and the rotation's rows are loaded too) and hands them over in LDS.  Only the table
+  // entries stand before the first keys; the queries arrive and are rotated while the keys
+  // travel (every wavefront preparing all operands first, the first key was asked for 3.3 us
+  // into a selection from 32K tokens that takes 27).
+  constexpr bool RAW = FUSED && !PACKED;  // the query may be un-rotated (a.q_raw)
+  constexpr int OPS = HKV * NA, MINE = (OPS + 3) / 4;
+  // The histogram of the selection below takes the same place.
+  __shared__ __attribute__((aligned(16))) uint32_t lh[FUSED && kTopkBins > OPS * 256 ? kTopkBins : OPS * 256];
+  const bool raw = RAW && a.q_raw != nullptr;
+  const bool lower = rg < 2;
+  uint4 q_own[MINE], q_other[MINE];
+  float4 q_cs[2], q_sn[2];
+  auto load_queries = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int kvh = 0; kvh < HKV; ++kvh)
-#pragma unroll
-    for (int na = 0; na < NA; ++na) {
-      const int g = 4 * na + t4;
+    for (int i = 0; i < MINE; ++i) {
+      const int op = min(wave + 4 * i, OPS - 1), kvh = op / NA, g = 4 * (op % NA) + t4;
       const int h = head_of<HKV, G>(kvh, g < G ? g : 0, a.head_map);
-      uint4 v;
-      if (FUSED && !PACKED && a.q_raw != nullptr) {
+      const char* qrow = raw ? (const char*)(a.q_raw + (size_t)b * a.q_stride + h * kHeadDim)
+                             : (const char*)(a.qf + ((size_t)b * H + h) * kHeadDim);
+      q_own[i] = *(const uint4*)(qrow + lane_off);
+      if (RAW) q_other[i] = *(const uint4*)(qrow + (lower ? lane_off + 128u : lane_off - 128u));
+    }
+    if (RAW) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {  // (q_cos and q_sin are readable whether or not they are used)
+        q_cs[i] = *(const float4*)((const char*)a.q_cos + 2 * lane_off + 16 * i);
+        q_sn[i] = *(const float4*)((const char*)a.q_sin + 2 * lane_off + 16 * i);
+      }
+    }
+  };
+  auto share_queries = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) {
+      const int op = wave + 4 * i, g = 4 * (op % NA) + t4;
+      uint4 v = q_own[i];
+      if (RAW && raw) {
         // The caller's un-rotated query: this lane's 8 dims and the 8 dims 64 further on (or
         // back), rotated as the rotation kernel does it.
-        const bool lower = rg < 2;
-        const uint32_t other_off = lower ? lane_off + 128u : lane_off - 128u;
-        const char* qrow = (const char*)(a.q_raw + (size_t)b * a.q_stride + h * kHeadDim);
-        const uint4 own = *(const uint4*)(qrow + lane_off), other = *(const uint4*)(qrow + other_off);
-        const float4 c0 = *(const float4*)((const char*)a.q_cos + 2 * lane_off);
-        const float4 c1 = *(const float4*)((const char*)a.q_cos + 2 * lane_off + 16);
-        const float4 s0 = *(const float4*)((const char*)a.q_sin + 2 * lane_off);
-        const float4 s1 = *(const float4*)((const char*)a.q_sin + 2 * lane_off + 16);
-        const uint32_t ow[4] = {own.x, own.y, own.z, own.w}, th[4] = {other.x, other.y, other.z, other.w};
-        const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+        const uint32_t ow[4] = {v.x, v.y, v.z, v.w};
+        const uint32_t th[4] = {q_other[i].x, q_other[i].y, q_other[i].z, q_other[i].w};
+        const float cs[8] = {q_cs[0].x, q_cs[0].y, q_cs[0].z, q_cs[0].w, q_cs[1].x, q_cs[1].y, q_cs[1].z, q_cs[1].w};
+        const float sn[8] = {q_sn[0].x, q_sn[0].y, q_sn[0].z, q_sn[0].w, q_sn[1].x, q_sn[1].y, q_sn[1].z, q_sn[1].w};
         uint32_t r[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -595,13 +663,13 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
           r[e] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
         }
         v = make_uint4(r[0], r[1], r[2], r[3]);
-      } else {
-        v = *(const uint4*)((const char*)(a.qf + ((size_t)b * H + h) * kHeadDim) + lane_off);
       }
       if (g >= G) v = make_uint4(0u, 0u, 0u, 0u);
-      qa[kvh][na] = __builtin_bit_cast(bf16x8_t, v);
+      if (op < OPS) *(uint4*)&lh[op * 256 + lane * 4] = v;
     }
+  };
 
+  bf16x8_t qa[HKV][NA];
   float run_m[HKV][NA], run_l[HKV][NA];
 #pragma unroll
   for (int kvh = 0; kvh < HKV; ++kvh)
@@ -686,16 +754,29 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
 
   size_t rows_cur[TG][4];
   size_t rows_next[TG][4];
-  if (wave_lo < wave_hi) {
+  {
+    // (a wavefront without tokens asks too, for its request's last ones: behind a branch the
+    // compiler would wait for all of these loads where it joins)
+    int32_t entry_first[TG][4];
 #pragma unroll
     for (int t = 0; t < TG; ++t)
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int tok = wave_lo + 16 * t + 4 * m + t4;
-        rows_cur[t][m] = row_off(table_entry(tok), tok);
-      }
+      for (int m = 0; m < 4; ++m) entry_first[t][m] = table_entry(wave_lo + 16 * t + 4 * m + t4);
+    load_queries();  // (in flight together with the table entries)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) rows_cur[t][m] = row_off(entry_first[t][m], wave_lo + 16 * t + 4 * m + t4);
     issue(buf0, rows_cur, 0);
   }
+  share_queries();
+  __syncthreads();
+#pragma unroll
+  for (int kvh = 0; kvh < HKV; ++kvh)
+#pragma unroll
+    for (int na = 0; na < NA; ++na)
+      qa[kvh][na] = __builtin_bit_cast(bf16x8_t, *(const uint4*)&lh[(kvh * NA + na) * 256 + lane * 4]);
 
   for (int base = wave_lo; base < wave_hi; base += ITER) {
     int32_t entry_next[TG][4];
@@ -800,28 +881,36 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
 
   if constexpr (FUSED) {
     __shared__ float s_rz[kMaxHeads];
-    __shared__ uint32_t lh[kTopkBins];
     __shared__ uint32_t scratch[16];
     const int tid = threadIdx.x;
     static_assert(kBandSlots == 4, "a workgroup's candidates of a bin are one 16-byte piece");
     __shared__ uint32_t band_lds[kBandBins][kBandSlots];
     __shared__ uint32_t band_count[kBandBins + 1];  // per bin; [kBandBins]: tokens above the band
+    __shared__ uint32_t band_sum[kBandBins + 2];    // the same over all workgroups; a bin's candidates do not fit
     for (int i = tid; i < kTopkBins; i += 256) lh[i] = 0u;
     if (tid < 16) scratch[tid] = 0u;
     if (tid < kBandBins * kBandSlots) band_lds[tid / kBandSlots][tid % kBandSlots] = 0u;
     if (tid <= kBandBins) band_count[tid] = 0u;
+    if (tid < kBandBins + 2) band_sum[tid] = 0u;
     TS_MARK(1);
     __syncthreads();  // scores, own maxima and the cleared histogram are in LDS for all
     TS_MARK(2);
-    merge_request_stats<PACKED>(a, lp, team, lane, wave);
-    TS_MARK(3);
+    // The votes-only form merges first: its workgroups hold up to twice the tokens, all of them
+    // stream to the phase's end, and the next phase waits for them (4 x 256K: 420 us, 425 with
+    // the exponentials first).
+    if constexpr (PACKED) {
+      merge_request_stats<PACKED>(a, lp, team, lane, wave);
+      TS_MARK(3);
+    } else {
+      fixed_parts(a);
+    }
     uint32_t ahead[kAheadLoads];
 #pragma unroll
     for (int i = 0; i < kAheadLoads; ++i) ahead[i] = 0u;
     if constexpr (PACKED) {
       if (wave != 0) touch_successor_keys<HKV>(a, wave, lane, ahead);  // (wavefront 0 polls)
     }
-    // While the merged statistics are on their way: the exponentials, relative to this
+    // While the statistics are on their way: the exponentials, relative to this
     // workgroup's own maxima; exp(s - max) / sum = exp(s - own max) * exp(own max - max) / sum.
     const ReqGeom geo =
         request_geometry(a.seq_lens, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len);
@@ -841,6 +930,11 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         for (int j = 0; j < 8; ++j)
           if (s0 + j < HKV * G) sc[(s0 + j) * 16] = __expf(x[j] - local_max[s0 + j]);
       }
+    }
+    // (after the exponentials: the workgroups that merge are among those that wait for the last one's)
+    if constexpr (!PACKED) {
+      merge_request_stats<PACKED>(a, lp, team, lane, wave);
+      TS_MARK(3);
     }
     if (tid < H) {  // H <= kMaxHeads < 256
       const int h = head_of<HKV, G>(tid / G, tid % G, a.head_map);
@@ -936,52 +1030,58 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     uint32_t slot_ahead[kEmitAhead];
 #pragma unroll
     for (int it = 0; it < kEmitAhead; ++it) {
+      slot_ahead[it] = 0u;
+      if (it * 256 >= count) continue;
       const int i = min(it * 256 + tid, count - 1);
       slot_ahead[it] = lookup_slot(tab, a.n_init + block_lo + i, a.page_size, a.page_shift, a.pool_rows);
     }
-    // Local histogram: one LDS atomic per candidate (lanes that hit the same bin are
+    // With a hint, what the band around it needs: the candidates of each band bin go to slots
+    // in LDS (published below), and the tokens above the band are counted.  Without one, the
+    // local histogram: one LDS atomic per candidate (lanes that hit the same bin are
     // performed one after the other, which for 256 candidates is a few hundred cycles).
-    // With a hint, also what the band around it needs: the candidates of each band bin go
-    // to slots in LDS (published below), and the tokens above the band are counted.
     const int hint_bin = hint_word - 1;
     const bool banded = hint_bin >= 0 && hint_bin < kTopkBins && lp.tokens_per_block <= kBandMaxTokens &&
                         req_chunks <= kSelMaxChunks / 2;
     const int band_lo = hint_bin - kBandBelow;  // (bins outside [0, kTopkBins) hold nothing)
-    uint32_t over_band = 0;  // this thread's tokens above the band
-    uint32_t top = 0;        // this thread's highest bin
-    for (int base = 0; base < count; base += 256) {
-      const bool have = base + tid < count;
-      const uint32_t key = have ? key_of(base + tid) : 0u;
-      const uint32_t bin = have ? key_bin0(key) : 0u;
-      if (have) atomicAdd(&lh[bin], 1u);
-      top = max(top, bin);
-      if (banded) {
-        const int d = (int)bin - band_lo;
-        if (have && d >= 0 && d < kBandBins) {
-          const uint32_t at = atomicAdd(&band_count[d], 1u);
-          if (at < (uint32_t)kBandSlots)
-            band_lds[d][at] = 0x80000000u | ((key & 0x1fffffu) << 10) | (uint32_t)(base + tid);
-        }
-        over_band += (have && d >= kBandBins) ? 1u : 0u;
-      }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
-    if (lane == 0) atomicMax(&scratch[8], top);
     if (banded) {
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) over_band += __shfl_xor(over_band, off);
+      uint32_t over_band = 0;  // this thread's tokens above the band
+      for (int i = tid; i < count; i += 256) {
+        const uint32_t key = key_of(i);
+        const int d = (int)key_bin0(key) - band_lo;
+        if (d >= 0 && d < kBandBins) {
+          const uint32_t at = atomicAdd(&band_count[d], 1u);
+          if (at < (uint32_t)kBandSlots) band_lds[d][at] = 0x80000000u | ((key & 0x1fffffu) << 10) | (uint32_t)i;
+        }
+        over_band += d >= kBandBins ? 1u : 0u;
+      }
+      over_band = wave_total(over_band);
       if (lane == 0 && over_band) atomicAdd(&band_count[kBandBins], over_band);
     }
-    __syncthreads();
+    uint32_t top = 0;  // this thread's highest bin
+    auto count_bins = [&]() {
+      for (int i = tid; i < count; i += 256) {
+        const uint32_t bin = key_bin0(key_of(i));
+        atomicAdd(&lh[bin], 1u);
+        top = max(top, bin);
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+      if (lane == 0) atomicMax(&scratch[8], top);
+      __syncthreads();
+    };
+    if (!banded) count_bins();
+    else __syncthreads();
 
     TS_MARK(6);
     // First level: top 11 key bits.  The workgroups add their local histograms to one
     // of the copies and note the highest occupied bin; afterwards each searches
     // downwards from that bin, 256 bins at a time (one is enough unless the votes
-    // span more than 64 binades).
+    // span more than 64 binades).  With a hint the band's counts go out instead, and the
+    // histogram only follows, a rendezvous later, when the threshold turns out to lie outside
+    // the band: some 40 of a workgroup's 70 read-modify-writes, which the device serves at
+    // 10-15 thousand a microsecond.
     uint32_t* hist0 = ctr + kSelHist0 + (chunk % kSelHistCopies) * kTopkBins;
-    {
+    auto publish_histogram = [&]() {
       // Two adjacent bins per 64-bit add (their counts cannot carry into each other):
       // half as many read-modify-writes on the few hot lines.
       uint64_t done = 0;  // old values: waited for once, after all are on their way
@@ -995,33 +1095,40 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       }
       if (tid == 0)
         done += fetch_max_coherent(&ctr[kSelMaxBin + (chunk % kSelHistCopies) * 32], scratch[8]);
-      if (banded && wave == 1) {
-        // The band.  Lane l holds the count of band bin l (lane kBandBins: of the bins above
-        // the band); the tokens above bin l are the sum over the lanes after it.
-        uint4* slots = a.band_slots + (size_t)b * kBandBins * kSelMaxChunks;
-        uint32_t* above = a.band_above + (size_t)b * kBandBins * kSelMaxChunks;
-        const uint32_t here = lane <= kBandBins ? band_count[lane] : 0u;
-        uint32_t run = here;  // becomes the sum over lanes l .. l + 15
+      await(done);
+    };
+    if (!banded) {
+      publish_histogram();
+    } else if (wave < 2) {
+      // The band, its words by one wavefront and its histogram by another.  Lane l holds the count of band bin l (lane kBandBins: of the bins above
+      // the band); the tokens above bin l are the sum over the lanes after it.
+      uint64_t done = 0;
+      uint4* slots = a.band_slots + (size_t)b * kBandBins * kSelMaxChunks;
+      uint32_t* above = a.band_above + (size_t)b * kBandBins * kSelMaxChunks;
+      const uint32_t here = lane <= kBandBins ? band_count[lane] : 0u;
+      if (wave == 1) {
+        if (here) done += fetch_add_coherent(&ctr[kSelBandHist + (chunk % kBandHistCopies) * 32 + lane], here);
+      } else {
+      uint32_t run = here;  // becomes the sum over lanes l .. l + 15
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-          const uint32_t up = (uint32_t)__shfl_down((int)run, off);
-          run += lane + off < 64 ? up : 0u;
-        }
-        static_assert(kBandBins + 1 <= 16, "the sum spans the band");
-        if (lane < kBandBins) {
-          done += __hip_atomic_exchange(&above[(size_t)lane * kSelMaxChunks + chunk], ((run - here) << 16) | here,
+      for (int off = 1; off < 16; off <<= 1) {
+        const uint32_t up = (uint32_t)__shfl_down((int)run, off);
+        run += lane + off < 64 ? up : 0u;
+      }
+      static_assert(kBandBins + 1 <= 16, "the sum spans the band");
+      if (lane < kBandBins) {
+        done += __hip_atomic_exchange(&above[(size_t)lane * kSelMaxChunks + chunk], ((run - here) << 16) | here,
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (the candidates: the first 8-byte half of the piece, the second only if used; none
+        // when they do not fit, since the bin is then not ranked from the band)
+        uint64_t* piece = (uint64_t*)&slots[(size_t)lane * kSelMaxChunks + chunk];
+        if (here >= 1 && here <= (uint32_t)kBandSlots)
+          done += __hip_atomic_exchange(piece, (uint64_t)band_lds[lane][0] | ((uint64_t)band_lds[lane][1] << 32),
                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          // (the candidates: the first 8-byte half of the piece, the second only if used)
-          uint64_t* piece = (uint64_t*)&slots[(size_t)lane * kSelMaxChunks + chunk];
-          if (here >= 1)
-            done += __hip_atomic_exchange(piece, (uint64_t)band_lds[lane][0] | ((uint64_t)band_lds[lane][1] << 32),
-                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (here >= 3)
-            done += __hip_atomic_exchange(piece + 1, (uint64_t)band_lds[lane][2] | ((uint64_t)band_lds[lane][3] << 32),
-                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane <= kBandBins && here)
-          done += fetch_add_coherent(&ctr[kSelBandHist + (chunk % kBandHistCopies) * 32 + lane], here);
+        if (here >= 3 && here <= (uint32_t)kBandSlots)
+          done += __hip_atomic_exchange(piece + 1, (uint64_t)band_lds[lane][2] | ((uint64_t)band_lds[lane][3] << 32),
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       }
       await(done);
     }
@@ -1053,12 +1160,43 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       }
     };
     bool found = false;     // the threshold bin is known
-    bool from_band = false; // and the band's slots hold its candidates
+    bool from_band = false; // and its candidates are in `entries`
+    // The candidates that the last step ranks, in any order (in the place of the histogram's
+    // last bins: with a hint it has not been counted yet, else it has been searched by then).
+    uint2* const entries = (uint2*)(lh + kTopkBins - 2 * kSelListCap);
+    // Appends the band's candidates of the loaded bin and counts the tokens above it in the
+    // workgroups before this one; a workgroup with more candidates than slots is noted.
+    auto gather_band = [&](uint32_t bin) {
+      uint32_t before = 0;
+#pragma unroll
+      for (int r = 0; r < kBandLoads; ++r) {
+        const uint32_t packed[4] = {band_piece[r].x, band_piece[r].y, band_piece[r].z, band_piece[r].w};
+        const uint32_t from = (uint32_t)(tid + 256 * r) * (uint32_t)lp.tokens_per_block;  // that workgroup's first token
+        uint32_t have = band_word[r] & 0xffffu;  // (zero where the load was skipped)
+        if (tid + 256 * r < chunk) before += band_word[r] >> 16;
+        if (have > (uint32_t)kBandSlots) {
+          band_sum[kBandBins + 1] = 1u;
+          have = 0u;
+        }
+        // Places for the wavefront's candidates with one addition (each lane adding its own
+        // count to the one word would be performed lane after lane).
+        const uint64_t b0 = __ballot(have & 1u), b1 = __ballot(have & 2u), b2 = __ballot(have & 4u);
+        if ((b0 | b1 | b2) == 0ull) continue;
+        const uint64_t low = (1ull << lane) - 1ull;
+        uint32_t at = 0;
+        if (lane == 0)
+          at = atomicAdd(&scratch[15], (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2)));
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) +
+             (uint32_t)(__popcll(b0 & low) + 2 * __popcll(b1 & low) + 4 * __popcll(b2 & low));
+#pragma unroll
+        for (uint32_t h2 = 0; h2 < 4; ++h2)
+          if (h2 < have && at + h2 < (uint32_t)kSelListCap)
+            entries[at + h2] = make_uint2((bin << 21) | ((packed[h2] >> 10) & 0x1fffffu), from + (packed[h2] & 1023u));
+      }
+      before = wave_total(before);
+      if (lane == 0 && before) atomicAdd(&scratch[10], before);
+    };
     if (banded) {
-      uint32_t* band_hist = lh + 1960;   // [kBandBins + 1] (the histogram array is free again)
-      if (tid <= kBandBins) band_hist[tid] = 0u;
-      if (tid == 32) lh[2000] = 0u;      // a workgroup with more candidates in the bin than slots
-      __syncthreads();
       constexpr int kWords = kBandHistCopies * (kBandBins + 1);
       constexpr int kPerThread = (kWords + 255) / 256;
       uint32_t part[kPerThread];
@@ -1072,37 +1210,51 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       load_band(kBandBelow);
 #pragma unroll
       for (int r = 0; r < kPerThread; ++r)
-        if (part[r]) atomicAdd(&band_hist[(tid + 256 * r) % (kBandBins + 1)], part[r]);
+        if (part[r]) atomicAdd(&band_sum[(tid + 256 * r) % (kBandBins + 1)], part[r]);
+      gather_band((uint32_t)hint_bin);
       __syncthreads();
       // Downwards from the bins above the band: the bin in which the count reaches k.
-      uint32_t run = band_hist[kBandBins];
+      uint32_t sums[kBandBins + 1];
+#pragma unroll
+      for (int d = 0; d <= kBandBins; ++d) sums[d] = band_sum[d];
+      uint32_t run = sums[kBandBins];
       int d0 = -1;
-      if (run < k) {
-        for (int d = kBandBins - 1; d >= 0; --d) {
-          const uint32_t here = band_hist[d];
-          if (run + here >= k) {
-            d0 = d;
-            in_bin0 = here;
-            break;
-          }
-          run += here;
+#pragma unroll
+      for (int d = kBandBins - 1; d >= 0; --d) {
+        const bool here = d0 < 0 && run < k && run + sums[d] >= k;
+        if (here) {
+          d0 = d;
+          in_bin0 = sums[d];
         }
+        if (d0 < 0) run += sums[d];
       }
       if (d0 >= 0 && band_lo + d0 >= 0) {
         found = true;
         t0 = (uint32_t)(band_lo + d0);
         above0 = run;
         if (in_bin0 <= (uint32_t)kSelListCap) {
-          if (d0 != kBandBelow) load_band(d0);
-          bool fits = true;
-#pragma unroll
-          for (int r = 0; r < kBandLoads; ++r) fits = fits && (band_word[r] & 0xffffu) <= (uint32_t)kBandSlots;
-          if (!fits) lh[2000] = 1u;
-          __syncthreads();
-          from_band = lh[2000] == 0u;
+          if (d0 != kBandBelow) {  // another bin of the band: once more, with its words
+            __syncthreads();
+            if (tid == 0) scratch[10] = scratch[15] = band_sum[kBandBins + 1] = 0u;
+            load_band(d0);
+            __syncthreads();
+            gather_band(t0);
+            __syncthreads();
+          }
+          from_band = band_sum[kBandBins + 1] == 0u;
+          // (every candidate of the bin is in a slot: the count is that of the histogram)
+          if (from_band && scratch[15] != in_bin0 && tid == 0)
+            __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
+    }
+    if (banded && !found) {  // the hint was of no use: the histogram is needed after all
       __syncthreads();
+      for (int i = tid; i < 2 * kSelListCap; i += 256) lh[kTopkBins - 2 * kSelListCap + i] = 0u;  // (the entries)
+      __syncthreads();
+      count_bins();
+      publish_histogram();
+      grid_arrive(lp.sync, ++round, a.spin_ticks, team.size, team.index);
     }
     if (!found) {
     // The search starts at the highest occupied bin of the request.  Together with the
@@ -1197,43 +1349,16 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
 
     uint2* counts = a.block_counts + (size_t)b * kSelMaxChunks;
     const bool listed = in_bin <= (uint32_t)kSelListCap;
-    uint32_t kth, need_eq = 0, pos_thr = 0;
-    if (tid < 8) scratch[8 + tid] = 0u;
-    __syncthreads();
+    uint32_t kth, need_eq = 0, pos_thr = 0, lower_taken = 0;
     // With a hint whose band holds the threshold bin, everything the ranking needs was
     // published before the first rendezvous: no list round.  The test was the same for every
     // workgroup of the request (the band's histogram, the flags), so all take the same way.
-    bool has = false;
-    uint2 e = make_uint2(0u, 0u);
-    if (from_band) {
-      uint2* entries_lds = (uint2*)(lh + 1024);  // [kSelListCap]
-      uint32_t band_sure = 0;  // tokens above the bin in the workgroups before this one
-#pragma unroll
-      for (int r = 0; r < kBandLoads; ++r) {
-        const uint32_t packed[4] = {band_piece[r].x, band_piece[r].y, band_piece[r].z, band_piece[r].w};
-        const uint32_t from = (uint32_t)(tid + 256 * r) * (uint32_t)lp.tokens_per_block;  // that workgroup's first token
-        const uint32_t have = band_word[r] & 0xffffu;  // (zero where the load was skipped)
-        if (tid + 256 * r < chunk) band_sure += band_word[r] >> 16;
-#pragma unroll
-        for (int h2 = 0; h2 < 4; ++h2)
-          if ((uint32_t)h2 < have) {
-            const uint32_t at = atomicAdd(&scratch[15], 1u);
-            if (at < (uint32_t)kSelListCap)
-              entries_lds[at] = make_uint2((t0 << 21) | ((packed[h2] >> 10) & 0x1fffffu), from + (packed[h2] & 1023u));
-          }
-      }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) band_sure += __shfl_xor(band_sure, off);
-      if (lane == 0) atomicAdd(&scratch[10], band_sure);
+    if (!from_band) {
       __syncthreads();
-      // (every candidate of the bin is in a slot: the count is that of the histogram)
-      if (scratch[15] != in_bin && tid == 0)
-        __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      has = (uint32_t)tid < min(scratch[15], (uint32_t)kSelListCap);
-      if (has) e = entries_lds[tid];
+      if (tid < 8) scratch[8 + tid] = 0u;
       __syncthreads();
-      TS_MARK(10);
-    } else if (listed) {
+    }
+    if (listed && !from_band) {
       // Last round, short form: the candidates of the threshold bin are appended to
       // the list (in kSelListParts parts with a counter each, a wavefront reserving
       // its entries with one add), and every workgroup publishes how many of its
@@ -1259,91 +1384,82 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
             store_coherent(&list[part * kSelListCap + slot], key, (uint32_t)(block_lo + i));
         }
       }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) above += __shfl_xor(above, off);
+      above = wave_total(above);
       if (lane == 0) atomicAdd(&scratch[8], above);
       __syncthreads();
       if (tid == 0) store_coherent(&counts[chunk], scratch[8], 0u);
       TS_MARK(10);
       grid_arrive(lp.sync, ++round, a.spin_ticks, team.size, team.index);
       TS_MARK(11);
-
-      // Every workgroup ranks the list on its own, one entry per thread, in the order
-      // (key descending, position ascending) packed into one 64-bit word.  The fill
-      // counters, the entries (thread t guesses entry t / parts of part t % parts,
-      // which is right unless a part holds more than 256 / parts) and the counts of
-      // the workgroups before this one are fetched together.
-      constexpr uint32_t kPerPart = kSelListCap / kSelListParts;
-      const uint32_t fill =
-          tid < kSelListParts ? load_coherent(&ctr[kSelListCount + tid * 32]) : 0u;
-      e = load_coherent(&list[(tid % kSelListParts) * kSelListCap + tid / kSelListParts]);
-      {
-        uint32_t sure = 0;
-        for (int j = tid; j < chunk; j += 256) sure += load_coherent(&counts[j]).x;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) sure += __shfl_xor(sure, off);
-        if (lane == 0) atomicAdd(&scratch[10], sure);
-      }
-      if (tid < kSelListParts) scratch[tid] = min(fill, (uint32_t)kSelListCap);
+      // The fill counters, the entries (a thread asks for two of a part, which covers all
+      // unless a part holds more than a quarter of the list) and the counts of the
+      // workgroups before this one are fetched together.
+      constexpr uint32_t kPerPart = 2 * 256 / kSelListParts;
+      const int my_part = tid % kSelListParts;
+      const uint32_t first = (uint32_t)(tid / kSelListParts), second = first + 256u / kSelListParts;
+      const uint32_t fill = load_coherent(&ctr[kSelListCount + my_part * 32]);
+      const uint2 e0 = load_coherent(&list[my_part * kSelListCap + first]);
+      const uint2 e1 = load_coherent(&list[my_part * kSelListCap + second]);
+      uint32_t sure = 0;
+      for (int j = tid; j < chunk; j += 256) sure += load_coherent(&counts[j]).x;
+      auto append = [&](const uint2& e) {
+        const uint32_t at = atomicAdd(&scratch[15], 1u);
+        if (at < (uint32_t)kSelListCap) entries[at] = e;
+      };
+      if (first < fill) append(e0);
+      if (second < fill) append(e1);
+      for (uint32_t at = kPerPart + first; at < min(fill, (uint32_t)kSelListCap); at += 256u / kSelListParts)
+        append(load_coherent(&list[my_part * kSelListCap + at]));
+      sure = wave_total(sure);
+      if (lane == 0 && sure) atomicAdd(&scratch[10], sure);
       __syncthreads();
-      uint32_t entries = 0, longest = 0;
-#pragma unroll
-      for (int p = 0; p < kSelListParts; ++p) {
-        entries += scratch[p];
-        longest = max(longest, scratch[p]);
-      }
-      if (longest <= kPerPart) {
-        has = (uint32_t)tid / kSelListParts < scratch[tid % kSelListParts];
-      } else {  // uneven parts: entry t of the concatenation
-        uint32_t at = (uint32_t)tid, from = 0;
-        has = false;
-#pragma unroll
-        for (int p = 0; p < kSelListParts; ++p) {
-          if (!has && at < scratch[p]) {
-            has = true;
-            from = (uint32_t)p;
-          } else if (!has) {
-            at -= scratch[p];
-          }
-        }
-        has = has && (uint32_t)tid < min(entries, (uint32_t)kSelListCap);
-        if (has) e = load_coherent(&list[from * kSelListCap + at]);
-      }
+    } else {
+      TS_MARK(10);
     }
     if (listed) {
-      const uint64_t mine = has ? ((uint64_t)e.x << 32) | (uint64_t)(0xffffffffu - e.y) : 0ull;
-      const uint32_t my_pos = e.y;
-      // The need-th largest entry: one more histogram level, over the next 8 key bits
-      // and in LDS, leaves the entries of one digit, which rank themselves against
-      // each other (ranking all entries against all would cost 64 K comparisons).
-      uint32_t* digits = lh;                    // [256]
-      uint64_t* peers = (uint64_t*)(lh + 256);  // [kSelListCap] entries of the threshold digit
-      const uint32_t digit = (e.x >> (shift - 8)) & 255u;
-      digits[tid] = 0u;
-      __syncthreads();
-      if (has) atomicAdd(&digits[digit], 1u);
-      __syncthreads();
-      uint32_t above_digit, all_digits, in_digit;
-      const int down = block_threshold_scan(digits[255 - tid], need, scratch, above_digit,
-                                            all_digits, in_digit);
-      const uint32_t threshold_digit = 255u - (uint32_t)down;  // down >= 0: the bin holds the k-th
-      const bool peer = has && digit == threshold_digit;
-      if (peer) peers[atomicAdd(&scratch[14], 1u)] = mine;
-      __syncthreads();
-      uint32_t rank = 0;
-      if (peer)
-        for (uint32_t u = 0; u < in_digit; ++u) rank += peers[u] > mine ? 1u : 0u;
-      const uint32_t need_here = need - above_digit;
-      const bool taken = has && (digit > threshold_digit || (peer && rank < need_here));
-      if (peer && rank + 1 == need_here) {  // the k-th of the request
-        scratch[9] = e.x;
-        scratch[12] = my_pos;
+      // Every wavefront finds the last candidate taken on its own, in the order (key
+      // descending, position ascending): it holds all of them, four to a lane, and the
+      // need-th largest key is built bit by bit from how many keys reach it, until as many do
+      // as are needed: some ten steps, and no barrier (narrowing the entries down by one
+      // more digit in LDS took seven of them, and counting the larger keys for every entry
+      // 2-6 us).
+      constexpr int kHeld = kSelListCap / 64;
+      const uint32_t total = min(scratch[15], (uint32_t)kSelListCap);
+      uint2 e[kHeld];
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i)
+        e[i] = (uint32_t)(64 * i + lane) < total ? entries[64 * i + lane] : make_uint2(0u, 0xffffffffu);
+      auto count = [&](auto&& pred) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) sum += (uint32_t)__popcll(__ballot(pred(e[i])));
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)sum);
+      };
+      uint32_t floor = (uint32_t)__builtin_amdgcn_readfirstlane((int)(prefix << shift)), reach = total;
+      const uint32_t wanted = (uint32_t)__builtin_amdgcn_readfirstlane((int)need);
+      for (int bit = __builtin_amdgcn_readfirstlane(shift) - 1; bit >= 0 && reach != wanted; --bit) {
+        const uint32_t trial = floor | (1u << bit);
+        const uint32_t with = count([&](const uint2& x) { return x.x >= trial; });
+        if (with >= wanted) {
+          floor = trial;
+          reach = with;
+        }
       }
-      const uint64_t lower = __ballot(taken && my_pos < (uint32_t)block_lo);
-      if (lane == 0 && lower) atomicAdd(&scratch[13], (uint32_t)__popcll(lower));
-      __syncthreads();
-      kth = scratch[9];
-      pos_thr = scratch[12];
+      kth = floor;
+      pos_thr = 0xffffffffu;
+      if (reach > need) {
+        // More ties at the k-th key than places: those at the lowest positions are taken.  The
+        // largest position with which the ties up to it still fit, from the top bit down.
+        const uint32_t places = need - count([&](const uint2& x) { return x.x > kth; });
+        pos_thr = 0u;
+        for (int bit = 31; bit >= 0; --bit) {
+          const uint32_t trial = pos_thr | (1u << bit);
+          if (count([&](const uint2& x) { return x.x == kth && x.y < trial; }) < places) pos_thr = trial;
+        }
+      }
+      lower_taken = count([&](const uint2& x) {
+        return (x.x > kth || (x.x == kth && x.y <= pos_thr)) && x.y < (uint32_t)block_lo;
+      });
       TS_MARK(12);
     } else {
       // Third level: last 10 bits of the candidates inside (t0, t1).
@@ -1424,7 +1540,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     TS_MARK(13);
     uint32_t tie_run = scratch[11];  // ties at lower positions
     // selected at lower positions
-    uint32_t out_run = scratch[10] + (listed ? scratch[13] : min(tie_run, need_eq));
+    uint32_t out_run = scratch[10] + (listed ? lower_taken : min(tie_run, need_eq));
     __syncthreads();
 
     // Emission in position order.
@@ -1623,7 +1739,7 @@ int fused_tokens_per_block(const ts_config* cfg, int batch, int max_seq_len, boo
   auto plan = [&](bool large) {
     const int capacity = fused_capacity(cfg, false, large);
     if (capacity <= 0) return 0;
-    int tpb = score_tokens_per_block((int64_t)batch * max_seq_len, cfg->num_heads);
+    int tpb = score_tokens_per_block((int64_t)batch * max_n, cfg->num_heads);
     while ((int64_t)ceil_div(max_n, tpb) * batch > capacity) tpb += 64;
     if (fused_lds_bytes(tpb, cfg->num_heads) > fused_stage_bytes(large) || tpb > pooling_tokens_cap(cfg))
       return 0;
@@ -1817,6 +1933,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
   ScoreArgs a = selection_args(cfg, bt, qf, k_pool, pool_rows, hit, (float*)(ws + w.partials),
                                w.tokens_per_block);
   a.nchunks = kSelMaxChunks;  // the row of a (request, head) pair in the statistics' table
+  a.q_cos = a.q_sin = (const float*)(ws + w.counters);  // (readable, not used)
   if (unrotated) {
     a.q_raw = (const uint16_t*)unrotated->q;
     a.q_stride = unrotated->stride;
