@@ -145,6 +145,33 @@ def test_sparse_prefill_attention_short_selections(dev, m, S):
     assert err <= 2e-2, err
 
 
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[3], SHAPES[4], SHAPES[7]],
+                         ids=[IDS[0], IDS[3], IDS[4], IDS[7]])
+@pytest.mark.parametrize("m,S", [(15, 140), (16, 128), (63, 190), (64, 64), (65, 257)])
+def test_sparse_prefill_attention_query_block_edges(dev, shape, m, S):
+    """A workgroup's 64 query columns are 16, 32 or 64 rows, by the query heads per KV head
+    (4, 2, 1 and 5 here): rows just short of, at and past such a block, and keys for which the
+    causal mask falls on the only tile of a key stream, on a last one and on none.  The keys'
+    norms grow, so that rows move to new maxima on the way.  (Tolerance: that of this file,
+    2^-8 of outputs below 4 and the rounding of queries, keys and weights to bf16.)"""
+    say(f"prefill attention query block edges H={shape['num_heads']} m={m} S={S}")
+    wl = workloads.build("pf", shape, [S + 8], [8], 1, dev, seed=31, n_init=1, n_local=m)
+    c = wl.cfg
+    g = torch.Generator(device=dev).manual_seed(32)
+    q = torch.randn((m, c.num_heads * 128), generator=g, device=dev).bfloat16()
+    sel = wl.table[0, :S].contiguous()
+    growth = torch.linspace(0.2, 2.0, S, device=dev).view(S, 1, 1)
+    rows = wl.k_pool.view(-1, c.num_kv_heads, 128)
+    rows[sel.long()] = (rows[sel.long()].float() * growth).bfloat16()
+    sel_len = torch.tensor([S], dtype=torch.int32, device=dev)
+    out = ops.sparse_prefill_attention(c, q, wl.k_pool, wl.v_pool, sel, sel_len)
+    torch.cuda.synchronize()
+    ref = oracle.prefill.sparse_prefill_attention(q.cpu().view(m, c.num_heads, 128), wl.k_pool.cpu(),
+                                                  wl.v_pool.cpu(), sel.cpu(), _sm(c), c.rope_theta)
+    err = (out.cpu().float() - ref.reshape(m, -1).float()).abs().max().item()
+    assert err <= 2e-2, err
+
+
 @pytest.mark.parametrize("direction", ["growing", "shrinking"])
 def test_sparse_prefill_attention_moving_maximum(dev, direction):
     """Logits that grow (or fall) steadily along the selected list, by far more than the

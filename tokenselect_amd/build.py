@@ -29,6 +29,9 @@ CXXFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# Matrix instructions write to the vector registers, as the vector instructions that follow on
+# their results want them; accumulators that are to live in the others are placed by hand.
+SOURCE_FLAGS = {"ts_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def sources():
@@ -37,7 +40,7 @@ def sources():
 
 def _compile(src: str, extra) -> str:
     obj = os.path.join(BUILD_DIR, os.path.basename(src)[:-4] + ".o")
-    cmd = [HIPCC, *CXXFLAGS, *extra, "-c", src, "-o", obj]
+    cmd = [HIPCC, *CXXFLAGS, *SOURCE_FLAGS.get(os.path.basename(src), ()), *extra, "-c", src, "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{res.stdout}\n{res.stderr}")

@@ -125,49 +125,44 @@ __global__ __launch_bounds__(1024) void fingerprint_kernel(
 //
 // prefill_gather_kernel: the selected rows are gathered once per chunk into a
 // contiguous staging area, K rotated to its index in the selected list (in fp32,
-// rounded to bf16 like the queries) as kr[kvh][j][128] and V transposed as
-// vt[kvh][128][S_pad], so that the attention kernel, whose 32 query tiles would
-// otherwise each repeat the gather, the rotation and the transposition, only copies
-// tiles.  Within every block of 32 keys a V^T row is stored in the order in which the
-// attention kernel's matrix instructions want the keys (see kv_pos below).
+// rounded to bf16 like the queries) and V transposed, so that the attention kernel, whose
+// query tiles would otherwise each repeat the gather, the rotation and the transposition,
+// only loads operands: per KV head and tile of 32 keys kr and vt hold the eight A operands
+// of the tile one after the other, 1 KB each, 16 bytes per lane in lane order.  The keys of
+// a V^T operand are in the order in which the logits' product leaves them (kv_pos below).
 //
-// prefill_attn_kernel<G>: grid (KV heads, 16-row query tiles, quads of the G query
-// heads of a KV head); 512 threads = four key groups of two wavefronts.  Key group g
-// takes the 32-key tiles g, g + 4, g + 8, ...; its two wavefronts serve two query heads
-// each (two 16 x 128 query blocks held in registers), so that every K and V^T operand
-// read from LDS feeds two matrix instructions.  The four groups' (max, sum, acc) are
-// merged through LDS at the end.
+// prefill_attn_kernel<G>: grid (KV heads, query tiles, head blocks); 256 threads = four
+// wavefronts, one per SIMD, each a key group of its own: group g takes the 32-key tiles
+// g, g + 4, g + 8, ... for all 64 query columns of the workgroup (kPfBlocks column blocks of
+// 16 query rows of one head: four heads x 16 rows, two x 32 or one x 64, whatever divides G
+// with the least waste), held in registers.  The four groups' (max, sum, acc) are merged
+// through LDS at the end, a column block per wavefront.
 //
-// Staging: a group's 128 threads bring the next tile of their group (8 KB of kr, 8 KB
-// of vt) from global memory straight into LDS (global_load_lds_dwordx4: 16 bytes per
-// lane, a wavefront fills 1 KB of consecutive LDS; no registers, no LDS store
-// instructions) while the group computes on the tiles that arrived during the previous
-// step; two LDS buffers per group, and two counters in LDS per group instead of a
-// workgroup barrier per step (see the loop).  Rows are not padded in LDS;
-// instead the 16-byte pieces of a row are permuted (XOR with row bits) so that the 16
-// lanes the hardware serves together when a wavefront reads a matrix operand fall on
-// distinct banks: which global piece a lane fetches is free, where it lands is not.
+// Why one wavefront per SIMD with 64 columns: every K and V^T operand that a wavefront
+// fetches feeds four matrix instructions, and nobody shares its tiles, so that they go from
+// L2 straight into the operand registers.  With two wavefronts per SIMD of 32 columns the
+// tiles went through LDS (written once, read by two wavefronts): 192 KB of LDS traffic per
+// round and counters in LDS to hand buffers over, which a wavefront, issuing in order,
+// waited for.  The staging area is laid out so that an operand is 1 KB in a row, lane l's 16
+// bytes at 16 l; an operand's registers are refilled for the next tile as soon as its last
+// product is issued, so that a load has a whole round (some 1400 cycles) to arrive.
 //
-// A wavefront computes S^T = K Q^T with v_mfma_f32_16x16x32_bf16 (A = 16 keys x 32 dims
-// from LDS, B = 16 rotated queries of one head, pre-multiplied by the softmax scale and
-// log2 e), which leaves lane (query l%16, key group l/16) with base-2 logits of 8 keys of
-// the tile.  The accumulator starts at minus the running maximum of the row, so the
-// products come out already shifted; the running maximum is only raised when a logit
-// exceeds it by more than 8 (the weights then stay below 2^8, harmless in fp32 sums
-// and invisible after the final division), so the common path per logit is one
-// maximum, one exp2 and half a conversion.  The 8 probabilities, rounded to bf16, are
-// directly the B operand of O^T += V^T P^T (A = 16 dims x 32 keys from the V^T tile);
-// a ninth product with an all-ones A operand accumulates the row sums.  fp32
-// accumulation throughout.
+// A wavefront computes S^T = K Q^T with v_mfma_f32_16x16x32_bf16 (A = 16 keys x 32 dims,
+// B = 16 rotated queries of one head, pre-multiplied by the softmax scale and log2 e), which
+// leaves lane (query l%16, key group l/16) with base-2 logits of 8 keys of the tile.  The
+// accumulator starts at minus the running maximum of the row, so the products come out
+// already shifted; the running maximum is only raised when a logit exceeds it by more than 8
+// (the weights then stay below 2^8, harmless in fp32 sums and invisible after the final
+// division), so the common path per logit is one maximum, one exp2 and half a conversion.
+// The 8 probabilities, rounded to bf16, are directly the B operand of O^T += V^T P^T
+// (A = 16 dims x 32 keys from the V^T tile); a ninth product with an all-ones A operand
+// accumulates the row sums.  fp32 accumulation throughout.
 //
-// Where the time goes (512 rows over 2688 selected keys, 36.5 us): 4.6 us until the
-// queries are rotated and the first tile is there, 2 us for the merge and the output, the
-// rest in some 19 rounds of 2100 cycles per wavefront, of which the matrix unit of a SIMD
-// is busy 1090 (its two wavefronts' 68 instructions of 16 cycles).  A round is some 250
-// instructions, a wavefront issues one per four cycles at best, and every wait (for LDS
-// data, for a matrix result, for the partner's counter) stalls the wavefront's whole
-// stream: two wavefronts per SIMD cover each other only partly.  Four wavefronts per SIMD
-// with one head each double the LDS reads and came out the same.
+// Measured, 512 rows over 2688 selected keys: 32 heads on 8 KV heads 37.3 -> 28.8 us, 28 on 4
+// 32.8 -> 25.4 us (68 matrix instructions of 7 ns per tile: 10 us; the 1.4 MB of tiles per
+// CU at the 110 GB/s that L2 delivers to one: 13 us).  What is left over is mostly the
+// loads' latency: 64 KB per CU in flight, 0.6 to 0.85 us from L2 under this load.
+// Alternating products and exp2 in the source order of the logits' steps changed nothing.
 struct PrefillArgs {
   const uint16_t* q;  // [rows, H, 128] bf16, un-rotated, rows q_stride elements apart
   int q_stride;
@@ -177,12 +172,12 @@ struct PrefillArgs {
   const int32_t* sel;      // [S] selected slots in attention order
   const int32_t* sel_len;  // device scalar S
   int max_sel_len;
-  int s_pad;               // columns of a vt row: max_sel_len rounded up to kPfPadKeys
+  int s_pad;               // keys in kr and vt per KV head: max_sel_len rounded up to kPfPadKeys
   int rows;
   int num_heads, num_kv_heads, rope_mode;
   float log2_theta, rope_rcp_scale, sm_scale, logit_cap;
-  uint16_t* kr;   // [Hkv, s_pad, 128] bf16 rotated keys
-  uint16_t* vt;   // [Hkv, 128, s_pad] bf16 transposed values, keys permuted within blocks of 32
+  uint16_t* kr;   // [Hkv, s_pad / 32, operand 4 kb + ks, lane, 8] bf16 rotated keys
+  uint16_t* vt;   // [Hkv, s_pad / 32, operand db, lane, 8] bf16 transposed values
   uint16_t* out;  // [rows, H, 128] bf16
 };
 
@@ -193,11 +188,14 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kPfKeys = 32;            // keys per tile: of the gather kernel and of the attention kernel
 constexpr int kPfVRow = kPfKeys + 8;   // halfwords per V^T row in the gather kernel's LDS (80 B)
 constexpr int kPfPadKeys = 64;         // the staging area holds whole multiples of this many keys
-constexpr int kPfGroups = 4;           // key groups of an attention workgroup
-constexpr int kPfTileBytes = kPfKeys * kHeadDim * 2;  // 8 KB: a K tile; a V^T tile is as large
-constexpr int kPfBufBytes = 2 * kPfTileBytes;         // K tile, then V^T tile
-constexpr size_t kPfLdsBytes = (size_t)kPfGroups * 2 * kPfBufBytes;  // 128 KB
-constexpr int kPfHeads = 2;            // query heads per wavefront of the attention kernel
+constexpr int kPfGroups = 4;           // key groups of an attention workgroup: its wavefronts
+constexpr int kPfBlocks = 4;           // column blocks (16 query rows of one head) of a wavefront
+constexpr int kPfTileElems = kPfKeys * kHeadDim;      // a K tile; a V^T tile is as large
+constexpr int kPfOperands = kPfTileElems / (64 * 8);  // operands of a tile: 16 bytes per lane each
+// The merge area: per group and column block eight vectors of accumulators and (max, sum),
+// four floats per lane each.  (The rotated queries pass through the same space at the start.)
+constexpr size_t kPfLdsBytes = (size_t)kPfGroups * kPfBlocks * 9 * 64 * 16;  // 144 KB
+static_assert(kPfOperands == 8, "a tile has eight operands");
 constexpr float kPfRaise = 8.0f;       // a row's maximum is raised when a logit exceeds it by this much
 
 // Position of key kk (0..31 within its block) in a V^T row: the matrix instruction
@@ -252,13 +250,16 @@ __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
       lo[e] = l2;
     }
   }
-  uint16_t* krow = a.kr + ((size_t)kvh * a.s_pad + j) * kHeadDim;
-  *(uint4*)(krow + 8 * c8) = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]),
+  // key kk = 16 kb + qc, dims 32 ks + 8 g4: operand 4 kb + ks, lane 16 g4 + qc
+  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)blockIdx.x * kPfKeys) * kHeadDim;
+  uint16_t* kout = a.kr + tile_at + ((4 * (kk >> 4) + (c8 >> 2)) * 64 + 16 * (c8 & 3) + (kk & 15)) * 8;
+  *(uint4*)kout = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]),
                                         pack_bf16(lo[4], lo[5]), pack_bf16(lo[6], lo[7]));
-  *(uint4*)(krow + 64 + 8 * c8) = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
+  *(uint4*)(kout + 2 * 64 * 8) = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
                                              pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
-  // transpose the 32 x 128 V tile through LDS (key kk to column kv_pos(kk)), then write
-  // 128 rows of 64 bytes
+  // transpose the 32 x 128 V tile through LDS (key kk to column kv_pos(kk)), then write its
+  // eight operands: piece p is lane p % 64 of operand p / 64, dim 16 (p / 64) + p % 16,
+  // columns [8 g4, +8) with g4 = p % 64 / 16
   const uint32_t vlo[4] = {vraw[0].x, vraw[0].y, vraw[0].z, vraw[0].w};
   const uint32_t vhi[4] = {vraw[1].x, vraw[1].y, vraw[1].z, vraw[1].w};
   const int col = kv_pos(kk);
@@ -270,48 +271,12 @@ __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
     vt_lds[(64 + 8 * c8 + 2 * e + 1) * kPfVRow + col] = (uint16_t)(vhi[e] >> 16);
   }
   __syncthreads();
-  const int d = tid >> 1, half = tid & 1;
-  uint16_t* vrow = a.vt + ((size_t)kvh * kHeadDim + d) * a.s_pad + blockIdx.x * kPfKeys + 16 * half;
-  const uint4* src = (const uint4*)(vt_lds + d * kPfVRow + 16 * half);
-  ((uint4*)vrow)[0] = src[0];
-  ((uint4*)vrow)[1] = src[1];
-}
-
-typedef void __attribute__((address_space(3)))* pf_lds_ptr;
-
-// 16 bytes per lane from global memory straight into LDS: lane l's piece lands at LDS
-// byte address lds_dst + 16 l (lds_dst the same for the whole wavefront, passed in M0).
-// Written as assembly and not through the compiler's builtin on purpose: the compiler
-// makes every later LDS read wait for all such loads (it cannot tell that they fill the
-// other buffer), which serialises exactly what is meant to overlap.  The waits are
-// explicit instead: s_waitcnt vmcnt(0) before the barrier that hands a buffer over.
-// The source is base (the same for the whole wavefront) + offset (per lane).  Four pieces per
-// lane with one write of M0: the instruction's offset field moves both addresses, so piece
-// i lands 1 KB after piece i - 1, and its source offset is passed 1024 i too small.
-// A wavefront issues one instruction per four cycles at best, whatever its kind, and
-// the loop around these loads is bound by exactly that: every scalar instruction counts.
-__device__ __forceinline__ void load_to_lds16(const void* base, const uint32_t (&offset)[4], uint32_t lds_dst) {
-  uint32_t saved_m0;  // M0 is the compiler's; it gets it back
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-      "global_load_lds_dwordx4 %2, %6\n\t"
-      "global_load_lds_dwordx4 %3, %6 offset:1024\n\t"
-      "global_load_lds_dwordx4 %4, %6 offset:2048\n\t"
-      "global_load_lds_dwordx4 %5, %6 offset:3072\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved_m0)
-      : "s"(lds_dst), "v"(offset[0]), "v"(offset[1]), "v"(offset[2]), "v"(offset[3]), "s"(base)
-      : "memory");
-}
-
-// One lane adds 1 to a counter in LDS.  LDS instructions of a wavefront are carried out in
-// order, so the reads before it have been served when the addition is.
-__device__ __forceinline__ void lds_count(uint32_t lds_at_vgpr, uint32_t one_vgpr) {
-  uint64_t saved_exec;
-  asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 1\n\tds_add_u32 %1, %2\n\ts_mov_b64 exec, %0"
-               : "=&s"(saved_exec)
-               : "v"(lds_at_vgpr), "v"(one_vgpr)
-               : "memory");
+  uint4* vout = (uint4*)(a.vt + tile_at);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int p = tid + 256 * i;
+    vout[p] = *(const uint4*)(vt_lds + (16 * (p >> 6) + (p & 15)) * kPfVRow + 8 * ((p >> 4) & 3));
+  }
 }
 
 // Largest of three, without the NaN-quieting copies fmaxf brings along.
@@ -321,430 +286,399 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return d;
 }
 
-// Two wavefronts per SIMD by construction (8 per workgroup, one workgroup per CU): saying
-// so lets the compiler use 256 registers.
+// The products, with their registers in the half of the register file that suits them: the
+// accumulators of the output and the queries in the accumulation registers, the logits,
+// which vector instructions read, in the others.  Written as assembly because the compiler,
+// left to choose, moves accumulators to and fro around every product (480 moves per tile).
+// What it does not see it does not keep apart: the caller leaves at least eleven cycles of
+// instruction issue between a product and any use of its result other than as the same
+// product's next accumulator, and two between a vector instruction and a product that reads
+// its result.
+__device__ __forceinline__ void mfma_acc(pf_f32x4& acc, const pf_bf16x8& a, const pf_bf16x8& b) {
+  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ pf_f32x4 mfma_logits(const pf_f32x4& s, const uint4& k, const pf_bf16x8& q) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, k), q, s, 0, 0, 0);
+}
+// Says that acc lives in the accumulation registers here, so that where paths join it stays there.
+template <typename V>
+__device__ __forceinline__ void keep_acc(V& acc) { asm("" : "+a"(acc)); }
+// Eleven instructions and more: between the last product and another use of its accumulators.
+__device__ __forceinline__ void mfma_settled() { asm volatile("s_nop 15" ::: "memory"); }
+
+// Heads of a workgroup's column blocks; the kPfBlocks / heads blocks of a head are
+// consecutive query tiles.  The choice that leaves the fewest columns of the last head block
+// without a head, and of those the one with the most heads (which share a row's rotation).
+constexpr int prefill_heads(int group) { return group % 4 == 0 || group % 4 == 3 ? 4 : group % 2 == 0 ? 2 : 1; }
+
+// One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
+// LDS): saying so lets the compiler use all 512 registers.
 template <int G, bool CAP>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_kernel(
+__global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
     PrefillArgs a) {
-  constexpr int HEADS = kPfHeads;        // query heads per wavefront
-  constexpr int kWaves = 4 / HEADS;      // wavefronts of a key group
-  constexpr int kBlocks = 8 / kWaves;    // 1 KB blocks of a K tile (and of a V^T tile) a wavefront brings in
-  static_assert(HEADS == 2 && kBlocks == 4, "the staging loads come four per wavefront");
-  // Dynamic LDS: per key group two buffers, each a K tile [32 keys][256 B] followed by a
-  // V^T tile [128 dims][64 B]; the merge of the groups at the end reuses the space.
+  constexpr int CB = kPfBlocks;
+  constexpr int NH = prefill_heads(G);   // heads of the workgroup
+  constexpr int RT = CB / NH;            // query tiles of 16 rows
+  constexpr int kRows = 16 * RT;
+  // Column block cb: head cb % NH of the workgroup's, query tile cb / NH.
   extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int group = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // wavefront = key group
   const int lane = threadIdx.x & 63;
-  const int group = wave / kWaves;  // which of the four tile streams this wavefront follows
-  const int hp = wave % kWaves;     // which HEADS of the quad's heads it serves
   const int qc = lane & 15, g4 = lane >> 4;  // query column / key group of the matrix layouts
   // The KV head is the fastest-moving workgroup index: consecutive workgroups go to
   // consecutive XCDs, so with eight KV heads each XCD's L2 holds the keys and values of one
   // head (1.4 MB of 11 MB) and every query tile of that head finds them there.  The last
   // query tiles, which see the most keys, start first.
   const int kvh = blockIdx.x;
-  const int q_row0 = (int)(gridDim.y - 1 - blockIdx.y) * 16;
+  const int q_row0 = (int)(gridDim.y - 1 - blockIdx.y) * kRows;
   const int H = a.num_heads;
-  char* const group_lds = (char*)pf_lds + group * (2 * kPfBufBytes);
-  const uint32_t group_lds_at = (uint32_t)(uintptr_t)(pf_lds_ptr)pf_lds + (uint32_t)(group * (2 * kPfBufBytes));
-
-  // ---- staging role.  K tile: wavefront hp of the group fills the 1 KB blocks kBlocks hp + i
-  // (i < kBlocks; a block is 4 keys), lane l the piece (key l/16 of the block, slot l%16), which
-  // holds the dims [8 c, 8 c + 8) with c = slot ^ (key & 15).  V^T tile: blocks of 16 dims,
-  // lane l the piece (dim l/4 of the block, slot l%4) = keys [8 c, +8) of the tile in vt's
-  // order, c = slot ^ ((dim / 4) & 3).
-  uint32_t k_src[kBlocks], v_src[kBlocks];
-  {
-    const int key_in_block = lane >> 4, slot = lane & 15;
-#pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const int key = 4 * (kBlocks * hp + i) + key_in_block;
-      k_src[i] = (uint32_t)(key * kHeadDim + 8 * (slot ^ (key & 15))) * 2u - (uint32_t)(i * 1024);
-    }
-    const int dim_in_block = lane >> 2, vslot = lane & 3;
-#pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const int dim = 16 * (kBlocks * hp + i) + dim_in_block;
-      v_src[i] = (uint32_t)(dim * a.s_pad + 8 * (vslot ^ ((dim >> 2) & 3))) * 2u - (uint32_t)(i * 1024);
-    }
-  }
-  const char* const k_base = (const char*)(a.kr + (size_t)kvh * a.s_pad * kHeadDim);
-  const char* const v_base = (const char*)(a.vt + (size_t)kvh * kHeadDim * a.s_pad);
-  // Tile t of this group holds the keys [(t kPfGroups + group) kPfKeys, + kPfKeys); K tile t
-  // lives in K buffer t % 2, V^T tile t in V buffer t % 2.
-  auto request_k = [&](int t) __attribute__((always_inline)) {
-    // past the end: a harmless repeat of the last tile
-    const int tile = min((t * kPfGroups + group) * kPfKeys, a.s_pad - kPfKeys);
-    const uint32_t dst = group_lds_at + (uint32_t)((t & 1) * kPfBufBytes + (kBlocks * hp) * 1024);
-    load_to_lds16(k_base + (size_t)tile * (kHeadDim * 2), k_src, dst);
-  };
-  auto request_v = [&](int t) __attribute__((always_inline)) {
-    const int tile = min((t * kPfGroups + group) * kPfKeys, a.s_pad - kPfKeys);
-    const uint32_t dst = group_lds_at + (uint32_t)((t & 1) * kPfBufBytes + kPfTileBytes + (kBlocks * hp) * 1024);
-    load_to_lds16(v_base + (size_t)tile * 2, v_src, dst);
-  };
-  request_k(0);  // on its way while the queries are prepared
-
   const int m = a.rows;
-  int head[HEADS];
-  bool head_active[HEADS];
+  auto head_in_group = [&](int cb) { return (int)blockIdx.z * NH + cb % NH; };
+  auto head_of = [&](int cb) { return kvh * G + min(head_in_group(cb), G - 1); };
+  auto row_of = [&](int cb) { return q_row0 + 16 * (cb / NH) + qc; };
+
+  // Tile t of this group holds the keys [(t kPfGroups + group) kPfKeys, + kPfKeys).  A tile
+  // past the staging area (asked for ahead, never used) is replaced by the last one.
+  const uint16_t* const k_base = a.kr + (size_t)kvh * a.s_pad * kHeadDim;
+  const uint16_t* const v_base = a.vt + (size_t)kvh * a.s_pad * kHeadDim;
+  const int last_tile = a.s_pad / kPfKeys - 1;
+  auto tile_at = [&](const uint16_t* base, int t) __attribute__((always_inline)) {
+    return (const uint4*)(base + (size_t)min(t * kPfGroups + group, last_tile) * kPfTileElems);
+  };
+  uint4 kw[kPfOperands], vw[kPfOperands];  // the operands of the next K tile and of the current V^T tile
+  {
+    const uint4* const k0 = tile_at(k_base, 0);
 #pragma unroll
-  for (int rb = 0; rb < HEADS; ++rb) {
-    const int head_in_group = blockIdx.z * 4 + HEADS * hp + rb;
-    head_active[rb] = head_in_group < G;
-    head[rb] = kvh * G + (head_active[rb] ? head_in_group : 0);
+    for (int i = 0; i < kPfOperands; ++i) kw[i] = k0[64 * i + lane];
   }
+
+  // ---- queries: B operand, lane (qc, g4) holds dims [32 ks + 8 g4, +8) of its column block's
+  // row, rotated to position shift + row (partner dims d and d + 64 are k-steps ks and ks + 2).
+  // All wavefronts need all of them; each prepares a quarter, four dims of every eight of one
+  // k-step and their partners, and they meet in LDS.
   // The queries' loads do not wait for the selection's length.
-  const int q_row = min(q_row0 + qc, m - 1);
-  uint4 q_raw[HEADS][4];
+  const int my_ks = group >> 1, my_half = 4 * (group & 1);
+  uint2 q_raw[CB][2];
 #pragma unroll
-  for (int rb = 0; rb < HEADS; ++rb) {
-    const uint16_t* qrow = a.q + (size_t)q_row * a.q_stride + head[rb] * kHeadDim;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) q_raw[rb][ks] = *(const uint4*)(qrow + 32 * ks + 8 * g4);
+  for (int cb = 0; cb < CB; ++cb) {
+    const uint16_t* qrow = a.q + (size_t)min(row_of(cb), m - 1) * a.q_stride + head_of(cb) * kHeadDim +
+                           32 * my_ks + 8 * g4 + my_half;
+    q_raw[cb][0] = *(const uint2*)qrow;
+    q_raw[cb][1] = *(const uint2*)(qrow + 64);
   }
   const int S = min(max(*a.sel_len, 0), a.max_sel_len);
   const int shift = S - m;  // query row i sits at position shift + i and sees keys <= that
-  const bool rope = a.rope_mode == TS_ROPE_LLAMA;
-  const bool wave_active = head_active[0];
   if (S <= 0) {
     // No keys (a selection that reported a fault): the rows attend to nothing and the
     // output is defined as zero.  (With fewer keys than rows, 0 < S < m, the rows whose
     // position S - m + i is negative see no key either: every tile is masked for them,
     // their sums stay zero and so does their output; the others attend as usual.)
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb)
-      if (head_active[rb])
-        for (int i = lane; i < 16 * (kHeadDim / 8); i += 64) {
-          const int row = q_row0 + i / (kHeadDim / 8);
-          if (row < m)
-            *(uint4*)(a.out + ((size_t)row * H + head[rb]) * kHeadDim + 8 * (i % (kHeadDim / 8))) =
-                make_uint4(0u, 0u, 0u, 0u);
-        }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile on its way lands before the LDS is given up
+    const int cb = group;  // a column block per wavefront
+    if (head_in_group(cb) < G)
+      for (int i = lane; i < 16 * (kHeadDim / 8); i += 64) {
+        const int row = q_row0 + 16 * (cb / NH) + i / (kHeadDim / 8);
+        if (row < m)
+          *(uint4*)(a.out + ((size_t)row * H + head_of(cb)) * kHeadDim + 8 * (i % (kHeadDim / 8))) =
+              make_uint4(0u, 0u, 0u, 0u);
+      }
     return;
   }
-
-  // ---- queries: B operand, lane (qc, g4) holds dims [32 ks + 8 g4, +8) of row q_row0 + qc
-  // of each of its two heads, rotated to position shift + row (partner dims d and d + 64 are
-  // k-steps ks and ks + 2; the angles are the same for both heads).
-  pf_bf16x8 qb[HEADS][4];
   {
-    float x[HEADS][4][8];
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const uint4 w = q_raw[rb][ks];
-        const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[rb][ks][2 * e] = bf16_lo(ww[e]);
-          x[rb][ks][2 * e + 1] = bf16_hi(ww[e]);
-        }
-      }
-    }
-    if (rope) {
-      const float pos = (float)(shift + q_row);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int pair = 32 * ks + 8 * g4 + e;
-          const float freq = a.rope_rcp_scale * exp2f(-(float)pair * (2.0f / kHeadDim) * a.log2_theta);
-          float sn, cs;
-          sincos_reduced(pos * freq, sn, cs);
-#pragma unroll
-          for (int rb = 0; rb < HEADS; ++rb) {
-            const float lo = x[rb][ks][e], hi = x[rb][ks + 2][e];
-            x[rb][ks][e] = lo * cs - hi * sn;
-            x[rb][ks + 2][e] = hi * cs + lo * sn;
-          }
-        }
-    }
+    const bool rope = a.rope_mode == TS_ROPE_LLAMA;
     // Without a soft cap the softmax scale and log2(e) go into the query, so that the
     // products come out as base-2 logits and every key costs one exp2 and no multiply.
     const float qs = CAP ? 1.0f : a.sm_scale * kLog2e;
+    float freq[4];
 #pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb)
+    for (int e = 0; e < 4; ++e) {
+      const int pair = 32 * my_ks + 8 * g4 + my_half + e;
+      freq[e] = a.rope_rcp_scale * exp2f(-(float)pair * (2.0f / kHeadDim) * a.log2_theta);
+    }
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+    for (int rt = 0; rt < RT; ++rt) {
+      float sn[4], cs[4];
+      if (rope) {
+        const float pos = (float)(shift + min(q_row0 + 16 * rt + qc, m - 1));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[rb][ks][e] *= qs;
-        const uint4 w = make_uint4(pack_bf16(x[rb][ks][0], x[rb][ks][1]), pack_bf16(x[rb][ks][2], x[rb][ks][3]),
-                                   pack_bf16(x[rb][ks][4], x[rb][ks][5]), pack_bf16(x[rb][ks][6], x[rb][ks][7]));
-        qb[rb][ks] = __builtin_bit_cast(pf_bf16x8, w);
+        for (int e = 0; e < 4; ++e) sincos_reduced(pos * freq[e], sn[e], cs[e]);
       }
-  }
-
-  // ---- reading role: where this lane's operands sit in a buffer.  K operand (kb, ks): key
-  // 16 kb + qc, dims [32 ks + 8 g4, +8) = piece 4 ks + g4, in slot (4 ks + g4) ^ qc.  V^T
-  // operand db: dim 16 db + qc, piece g4, in slot g4 ^ ((qc / 4) & 3).
-  uint32_t k_at[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) k_at[ks] = (uint32_t)(qc * (kHeadDim * 2) + 16 * ((4 * ks + g4) ^ qc));
-  const uint32_t v_at = (uint32_t)(kPfTileBytes + qc * (kPfKeys * 2) + 16 * (g4 ^ ((qc >> 2) & 3)));
+      for (int hh = 0; hh < NH; ++hh) {
+        const int cb = rt * NH + hh;
+        float lo[4] = {bf16_lo(q_raw[cb][0].x), bf16_hi(q_raw[cb][0].x), bf16_lo(q_raw[cb][0].y),
+                       bf16_hi(q_raw[cb][0].y)};
+        float hi[4] = {bf16_lo(q_raw[cb][1].x), bf16_hi(q_raw[cb][1].x), bf16_lo(q_raw[cb][1].y),
+                       bf16_hi(q_raw[cb][1].y)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (rope) {
+            const float l2 = lo[e] * cs[e] - hi[e] * sn[e];
+            hi[e] = hi[e] * cs[e] + lo[e] * sn[e];
+            lo[e] = l2;
+          }
+          lo[e] *= qs;
+          hi[e] *= qs;
+        }
+        uint16_t* const to = pf_lds + ((cb * 4 + my_ks) * 64 + lane) * 8 + my_half;
+        *(uint2*)to = make_uint2(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]));
+        *(uint2*)(to + 2 * 64 * 8) = make_uint2(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]));
+      }
+    }
+  }
+  __syncthreads();
+  pf_bf16x8 qb[CB][4];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      qb[cb][ks] = __builtin_bit_cast(pf_bf16x8, *(const uint4*)(pf_lds + ((cb * 4 + ks) * 64 + lane) * 8));
+      keep_acc(qb[cb][ks]);
+    }
+  __syncthreads();  // (the space is the merge area from here on)
 
-  // ---- main loop over the tiles any row of this query tile can see
-  const int last_visible = min(S - 1, shift + min(q_row0 + 15, m - 1));
-  const int my_limit = shift + q_row;  // last key this lane's query sees
+  // ---- main loop over the tiles any row of this workgroup can see
+  const int last_visible = min(S - 1, shift + min(q_row0 + kRows - 1, m - 1));
   // tiles of this group that hold a visible key
   const int n_tiles = last_visible >= group * kPfKeys
                           ? (last_visible - group * kPfKeys) / (kPfGroups * kPfKeys) + 1
                           : 0;
-  // Running maximum of each head's row: m_run (kNegBig: none yet), minus that as the
+  // Running maximum of each column's row: m_run (kNegBig: none yet), minus that as the
   // four-register start value of the logits' accumulators (0 while there is none), and the
   // excess over it that makes the row move (-inf while there is none: any finite logit does).
-  float m_run[HEADS], raise_at[HEADS];
-  pf_f32x4 minus_m[HEADS];
-  pf_f32x4 o[HEADS][8], row_sum[HEADS];
+  float m_run[CB], raise_at[CB];
+  pf_f32x4 minus_m[CB];  // (all zero with a soft cap, whose logits are shifted afterwards)
+  pf_f32x4 o[CB][8], row_sum[CB];
 #pragma unroll
-  for (int rb = 0; rb < HEADS; ++rb) {
-    m_run[rb] = kNegBig;
-    raise_at[rb] = -INFINITY;
-    minus_m[rb] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
-    row_sum[rb] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int cb = 0; cb < CB; ++cb) {
+    m_run[cb] = kNegBig;
+    raise_at[cb] = -INFINITY;
+    minus_m[cb] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+    row_sum[cb] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int db = 0; db < 8; ++db) o[rb][db] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < 8; ++db) {
+      o[cb][db] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+      keep_acc(o[cb][db]);
+    }
   }
   const pf_bf16x8 ones = __builtin_bit_cast(pf_bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 
-  // The work on a tile comes in three parts, and the loop below is a software pipeline
-  // over them, because a wavefront issues in order and the matrix unit and the vector
-  // ALU only run side by side when their instructions alternate in one stream (two
-  // wavefronts of a SIMD, each doing first one kind and then the other, were measured to
-  // overlap in 15 % of the matrix cycles):
-  //   logits(t):  S^T = K_t Q^T for both heads (16 matrix instructions), shifted by the
-  //               running maximum through the accumulator's start value;
-  //   settle(t):  the causal mask on the diagonal, the largest logit of a row, and, when
-  //               a row outgrew its maximum by kPfRaise, the move to a new one (vector);
-  //   output(t):  P = exp2 (vector, 16 exp2), O^T += V_t^T P^T and the row sums (18 matrix).
-  // Iteration t runs logits(t + 1) with the exp2 of tile t in between, then output(t),
-  // then settle(t + 1).
-  pf_f32x4 s_cur[HEADS][2];  // logits of the tile whose output comes next: [head][key block]
+  // The loop is a software pipeline, because a wavefront issues in order and the matrix unit
+  // and the vector ALU only run side by side when their instructions alternate in one stream.
+  // Iteration t:
+  //   logits(t + 1): S^T = K_{t+1} Q^T (32 matrix instructions in eight steps, one per K
+  //                  operand), shifted by the running maximum through the accumulators' start
+  //                  values; in between, a step's share of the exp2 of tile t, and the
+  //                  operand's registers are filled with tile t + 2's;
+  //   output(t):     O^T += V_t^T P^T and the row sums (36 matrix instructions); in between the
+  //                  largest logit of each row of tile t + 1, and the V^T operands of tile t + 1
+  //                  are asked for;
+  //   settle(t + 1): when a row outgrew its maximum by kPfRaise, the move to a new one.
+  // Only the last tile of a group can hold keys that some row must not see (a group's tiles
+  // are 128 keys apart, and a workgroup has at most 64 rows): the mask is on that one alone.
+  pf_f32x4 s_cur[CB][2];  // logits of the tile whose output comes next: [column block][key block]
 
-  auto logits = [&](int t, pf_f32x4 (&s)[HEADS][2]) __attribute__((always_inline)) {
-    const char* const base = group_lds + (t & 1) * kPfBufBytes;
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
-      s[rb][0] = CAP ? pf_f32x4{0.f, 0.f, 0.f, 0.f} : minus_m[rb];
-      s[rb][1] = s[rb][0];
-    }
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const uint4 kw = *(const uint4*)(base + kb * (16 * kHeadDim * 2) + k_at[ks]);
-#pragma unroll
-        for (int rb = 0; rb < HEADS; ++rb)
-          s[rb][kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, kw), qb[rb][ks],
-                                                             s[rb][kb], 0, 0, 0);
-      }
-  };
-
-  auto settle = [&](int t, pf_f32x4 (&s)[HEADS][2]) __attribute__((always_inline)) {
-    const int tile = (t * kPfGroups + group) * kPfKeys;
-    // Only the tiles on the diagonal hold keys that some query of the tile must not see.
-    const bool diagonal = tile + kPfKeys - 1 > shift + q_row0;
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
-      if (CAP) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            s[rb][kb][r] = a.logit_cap * tanhf(s[rb][kb][r] * a.sm_scale / a.logit_cap) * kLog2e + minus_m[rb][0];
-      }
-      if (diagonal) {
-        // Masked logits are -inf: exp2 makes them 0 without a branch.  (The tile's
-        // number passes through an empty asm so that the comparisons stay in here: the
-        // compiler otherwise computes all of them before the branch, on every tile.)
-        int tile_here = tile;
-        asm volatile("" : "+s"(tile_here));
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (tile_here + 16 * kb + 4 * g4 + r > my_limit) s[rb][kb][r] = -INFINITY;
-      }
-      float mx = max3(s[rb][0][0], s[rb][0][1], s[rb][0][2]);
-      mx = max3(mx, s[rb][0][3], s[rb][1][0]);
-      mx = max3(mx, s[rb][1][1], s[rb][1][2]);
-      mx = fmaxf(mx, s[rb][1][3]);
-      if (__ballot(mx > raise_at[rb]) != 0ull) {
-        // Some row of this head has no maximum yet, or outgrew it: agree on the row's
-        // maximum over the four key groups of lanes and move to it.
-        const bool unset = m_run[rb] == kNegBig;
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool take = unset ? mx > -INFINITY : mx > kPfRaise;
-        const float delta = take ? mx : 0.f;
-        // (a row without a maximum has only zeros in its accumulators)
-        const float scale = unset ? 1.0f : __builtin_amdgcn_exp2f(-delta);
-        if (take) {
-          m_run[rb] = delta - minus_m[rb][0];
-          raise_at[rb] = kPfRaise;
-          const float nm = -m_run[rb];
-          minus_m[rb] = pf_f32x4{nm, nm, nm, nm};
-        }
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[rb][kb][r] -= delta;
-#pragma unroll
-        for (int db = 0; db < 8; ++db)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[rb][db][r] *= scale;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) row_sum[rb][r] *= scale;
-      }
-    }
-  };
-
-  // One iteration of the pipeline: NEXT = there is a tile t + 1.
-  auto iteration = [&](int t, auto next) __attribute__((always_inline)) {
-    constexpr bool NEXT = decltype(next)::value;
-    const char* const vbase = group_lds + (t & 1) * kPfBufBytes;
-    pf_f32x4 s_next[HEADS][2];
-    // The V^T operands are asked for first: they arrive under the logits' products.
-    uint4 vw[8];
-#pragma unroll
-    for (int db = 0; db < 8; ++db) vw[db] = *(const uint4*)(vbase + db * (16 * kPfKeys * 2) + v_at);
-    if (NEXT) logits(t + 1, s_next);
-    pf_bf16x8 pb[HEADS];
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
-      float p[2][4];
+  // The soft cap, and the mask of the last tile; the largest logit of the lane's eight.
+  auto largest = [&](int t, pf_f32x4 (&s)[2], int cb, bool last) __attribute__((always_inline)) {
+    if (CAP) {
+      const float shift_by = m_run[cb] == kNegBig ? 0.f : m_run[cb];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[kb][r] = __builtin_amdgcn_exp2f(s_cur[rb][kb][r]);
-      const uint4 pw = make_uint4(pack_bf16(p[0][0], p[0][1]), pack_bf16(p[0][2], p[0][3]),
-                                  pack_bf16(p[1][0], p[1][1]), pack_bf16(p[1][2], p[1][3]));
-      pb[rb] = __builtin_bit_cast(pf_bf16x8, pw);
+        for (int r = 0; r < 4; ++r)
+          s[kb][r] = a.logit_cap * tanhf(s[kb][r] * a.sm_scale / a.logit_cap) * kLog2e - shift_by;
     }
+    if (last) {
+      // Masked logits are -inf: exp2 makes them 0 without a branch.
+      const int limit = shift + min(row_of(cb), m - 1) - ((t * kPfGroups + group) * kPfKeys + 4 * g4);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * kb + r > limit) s[kb][r] = -INFINITY;
+    }
+    float mx = max3(s[0][0], s[0][1], s[0][2]);
+    mx = max3(mx, s[0][3], s[1][0]);
+    mx = max3(mx, s[1][1], s[1][2]);
+    return fmaxf(mx, s[1][3]);
+  };
+  auto settle = [&](pf_f32x4 (&s)[CB][2], const float (&mx_lane)[CB]) __attribute__((always_inline)) {
+    bool any = false;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) any = any || mx_lane[cb] > raise_at[cb];
+    if (__ballot(any) == 0ull) return;
+    // Some row has no maximum yet, or outgrew it: agree on the row's maximum over the four
+    // key groups of lanes and move to it.  (All column blocks, and one vector at a time: a
+    // row that stays where it is is multiplied by one, and a branch per block or more
+    // vectors at once would cost the loop around this its registers.)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      const bool unset = m_run[cb] == kNegBig;
+      float mx = mx_lane[cb];
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const bool take = mx > raise_at[cb];
+      const float delta = take ? mx : 0.f;
+      // (a row without a maximum has only zeros in its accumulators)
+      const float scale = unset ? 1.0f : __builtin_amdgcn_exp2f(-delta);
+      if (take) {
+        m_run[cb] = unset ? delta : delta + m_run[cb];
+        raise_at[cb] = kPfRaise;
+        if (!CAP) {
+          const float nm = -m_run[cb];
+          minus_m[cb] = pf_f32x4{nm, nm, nm, nm};
+        }
+      }
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[cb][kb][r] -= delta;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[cb][db][r] *= scale;
+        keep_acc(o[cb][db]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) row_sum[cb][r] *= scale;
+    }
+  };
+
+  // NEXT: there is a tile t + 1; LAST: that one is the group's last.
+  auto iteration = [&](int t, auto next, auto last) __attribute__((always_inline)) {
+    constexpr bool NEXT = decltype(next)::value, LAST = decltype(last)::value;
+    const uint4* const k2 = tile_at(k_base, t + 2);
+    const uint4* const v1 = tile_at(v_base, t + 1);
+    pf_f32x4 s_next[CB][2];
+    uint32_t pw[CB][4];
+#pragma unroll
+    for (int i = 0; i < kPfOperands; ++i) {
+      const int kb = i >> 2, ks = i & 3;
+      // this step's share of the weights: column block i / 2, key block i % 2
+      const int pcb = i >> 1, pkb = i & 1;
+      float p[4];
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
+        if (NEXT) s_next[cb][kb] = mfma_logits(ks == 0 ? minus_m[cb] : s_next[cb][kb], kw[i], qb[cb][ks]);
+        p[cb] = __builtin_amdgcn_exp2f(s_cur[pcb][pkb][cb]);
+      }
+      if (NEXT && !LAST) kw[i] = k2[64 * i + lane];
+      pw[pcb][2 * pkb] = pack_bf16(p[0], p[1]);
+      pw[pcb][2 * pkb + 1] = pack_bf16(p[2], p[3]);
+      if (NEXT) {  // in the order: product, exp2, product, exp2, ...
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // matrix
+          __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);  // transcendental
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    pf_bf16x8 pb[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+      pb[cb] = __builtin_bit_cast(pf_bf16x8, make_uint4(pw[cb][0], pw[cb][1], pw[cb][2], pw[cb][3]));
+    // (the row sums first: between the packing of the weights and the products whose
+    // registers the compiler does not see)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+      row_sum[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[cb], row_sum[cb], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    float mx[CB];
 #pragma unroll
     for (int db = 0; db < 8; ++db) {
 #pragma unroll
-      for (int rb = 0; rb < HEADS; ++rb)
-        o[rb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, vw[db]), pb[rb],
-                                                           o[rb][db], 0, 0, 0);
+      for (int cb = 0; cb < CB; ++cb) mfma_acc(o[cb][db], __builtin_bit_cast(pf_bf16x8, vw[db]), pb[cb]);
+      if (NEXT) {
+        vw[db] = v1[64 * db + lane];
+        if (db >= 3 && db < 3 + CB) mx[db - 3] = largest(t + 1, s_next[db - 3], db - 3, LAST);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb)
-      row_sum[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[rb], row_sum[rb], 0, 0, 0);
+    mfma_settled();
+    __builtin_amdgcn_sched_barrier(0);
     if (NEXT) {
-      settle(t + 1, s_next);
+      settle(s_next, mx);
 #pragma unroll
-      for (int rb = 0; rb < HEADS; ++rb) {
-        s_cur[rb][0] = s_next[rb][0];
-        s_cur[rb][1] = s_next[rb][1];
+      for (int cb = 0; cb < CB; ++cb) {
+        s_cur[cb][0] = s_next[cb][0];
+        s_cur[cb][1] = s_next[cb][1];
       }
     }
   };
 
-  // The wavefronts of a key group keep in step through two counters in LDS and no
-  // barrier, so that the four groups drift apart.  landed = requests that have arrived
-  // (after each round of requests a wavefront waits for its own pieces and counts once),
-  // done = rounds of reading a wavefront has finished.  Round -1 brings K tile 0 and reads
-  // nothing; round t >= 0 is iteration t: it needs K tile t + 1 and V tile t, requested in
-  // round t - 1, and requests K tile t + 2 and V tile t + 1 into the buffers that round
-  // t - 1 read (K tile t, V tile t - 1): so it starts when landed >= kWaves (t + 2) and
-  // done >= kWaves (t + 1).  Neither wait can last: a partner is at most one round behind.
-  // The waits are bounded all the same, so that a mistake here would show as a wrong
-  // result and not as a hang.
-  __shared__ __attribute__((aligned(8))) uint32_t pf_sync[kPfGroups][2];
-  if (threadIdx.x < 2 * kPfGroups) (&pf_sync[0][0])[threadIdx.x] = 0u;
-  __syncthreads();
-  const uint64_t* const both = (const uint64_t*)&pf_sync[group][0];  // one read for the two
-  const uint32_t landed_at = (uint32_t)(uintptr_t)(pf_lds_ptr)&pf_sync[group][0], done_at = landed_at + 4u;
-  const uint32_t one = 1u;
-  auto await = [&](uint32_t need_landed, uint32_t need_done) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_count(landed_at, one);
-    for (int spin = 0; spin < (1 << 20); ++spin) {
-      const uint64_t counters = __hip_atomic_load(both, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if ((uint32_t)counters >= need_landed && (uint32_t)(counters >> 32) >= need_done) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-  };
-  auto finish_round = [&]() __attribute__((always_inline)) {
-    lds_count(done_at, one);
-  };
   if (n_tiles > 0) {
-    await((uint32_t)kWaves, 0u);
-    if (1 < n_tiles) request_k(1);
-    request_v(0);
-    if (wave_active) {
-      logits(0, s_cur);
-      settle(0, s_cur);
+    // the first tile's logits: nothing comes before them
+    const uint4* const k1 = tile_at(k_base, 1);
+    const uint4* const v0 = tile_at(v_base, 0);
+#pragma unroll
+    for (int i = 0; i < kPfOperands; ++i) {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+        s_cur[cb][i >> 2] = mfma_logits((i & 3) == 0 ? minus_m[cb] : s_cur[cb][i >> 2], kw[i], qb[cb][i & 3]);
+      kw[i] = k1[64 * i + lane];
+      __builtin_amdgcn_sched_barrier(0);
     }
-    finish_round();
-    for (int t = 0; t + 1 < n_tiles; ++t) {
-      await((uint32_t)(kWaves * (t + 2)), (uint32_t)(kWaves * (t + 1)));
-      if (t + 2 < n_tiles) request_k(t + 2);
-      request_v(t + 1);
-      if (wave_active) iteration(t, std::true_type{});
-      finish_round();
-    }
-    // the last tile: nothing follows it
-    await((uint32_t)(kWaves * (n_tiles + 1)), (uint32_t)(kWaves * n_tiles));
-    if (wave_active) iteration(n_tiles - 1, std::false_type{});
+    // (after the second K tile, in the order of the loop: loads return in order, and at the
+    // loop's head the compiler waits for the later of the two orders it may have come from)
+#pragma unroll
+    for (int i = 0; i < kPfOperands; ++i) vw[i] = v0[64 * i + lane];
+    __builtin_amdgcn_sched_barrier(0);
+    mfma_settled();
+    __builtin_amdgcn_sched_barrier(0);
+    float mx[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) mx[cb] = largest(0, s_cur[cb], cb, n_tiles == 1);
+    settle(s_cur, mx);
+    for (int t = 0; t + 2 < n_tiles; ++t) iteration(t, std::true_type{}, std::false_type{});
+    if (n_tiles > 1) iteration(n_tiles - 2, std::true_type{}, std::true_type{});
+    iteration(n_tiles - 1, std::false_type{}, std::false_type{});
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
 
-  // ---- merge of the four key groups (the barrier that ended the last step also freed
-  // the tiles' space): groups 1..3 hand their partial results to group 0 (same heads,
-  // same lane), per head 9 vectors of four floats per lane: 8 of acc and (max, sum).
-  constexpr int kVecs = 9 * HEADS;
-  pf_f32x4* const merge = (pf_f32x4*)pf_lds;  // [(group - 1) * kWaves + hp][kVecs][64 lanes]
-  static_assert(3 * kWaves * kVecs * 64 * 16 <= kPfLdsBytes, "the merge area fits the tiles");
-  if (group != 0) {
-    pf_f32x4* const mine = merge + ((group - 1) * kWaves + hp) * (kVecs * 64) + lane;
+  // ---- merge of the four key groups: every wavefront hands all its column blocks over (per
+  // lane 8 vectors of acc and one of (max, sum)) and merges one of them.
+  pf_f32x4* const merge = (pf_f32x4*)pf_lds;  // [group][column block][9][64 lanes]
 #pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
+  for (int cb = 0; cb < CB; ++cb) {
+    pf_f32x4* const mine = merge + (group * CB + cb) * (9 * 64) + lane;
 #pragma unroll
-      for (int db = 0; db < 8; ++db) mine[(9 * rb + db) * 64] = o[rb][db];
-      mine[(9 * rb + 8) * 64] = pf_f32x4{m_run[rb], row_sum[rb][0], 0.f, 0.f};
-    }
+    for (int db = 0; db < 8; ++db) mine[db * 64] = o[cb][db];
+    mine[8 * 64] = pf_f32x4{m_run[cb], row_sum[cb][0], 0.f, 0.f};
   }
   __syncthreads();
-  if (group != 0 || !wave_active) return;
-  float l_run[HEADS];
+  static_assert(CB == kPfGroups, "a column block per wavefront");
+  const int cb = group;
+  const pf_f32x4* const all = merge + cb * (9 * 64) + lane;
+  pf_f32x4 ml = all[8 * 64];
+  float m_all = ml[0], l_all = ml[1];
+  pf_f32x4 sum[8];
 #pragma unroll
-  for (int rb = 0; rb < HEADS; ++rb) l_run[rb] = row_sum[rb][0];
+  for (int db = 0; db < 8; ++db) sum[db] = all[db * 64];
 #pragma unroll
   for (int g = 1; g < kPfGroups; ++g) {
-    const pf_f32x4* const other = merge + ((g - 1) * kWaves + hp) * (kVecs * 64) + lane;
+    const pf_f32x4* const other = all + g * CB * (9 * 64);
+    ml = other[8 * 64];
+    const float m_new = fmaxf(m_all, ml[0]);
+    const float e0 = __builtin_amdgcn_exp2f(m_all - m_new), e1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
+    m_all = m_new;
+    l_all = l_all * e0 + ml[1] * e1;
 #pragma unroll
-    for (int rb = 0; rb < HEADS; ++rb) {
-      const pf_f32x4 ml = other[(9 * rb + 8) * 64];
-      const float m_new = fmaxf(m_run[rb], ml[0]);
-      const float e0 = __builtin_amdgcn_exp2f(m_run[rb] - m_new), e1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
-      m_run[rb] = m_new;
-      l_run[rb] = l_run[rb] * e0 + ml[1] * e1;
+    for (int db = 0; db < 8; ++db) {
+      const pf_f32x4 od = other[db * 64];
 #pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        const pf_f32x4 od = other[(9 * rb + db) * 64];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[rb][db][r] = o[rb][db][r] * e0 + od[r] * e1;
-      }
+      for (int r = 0; r < 4; ++r) sum[db][r] = sum[db][r] * e0 + od[r] * e1;
     }
   }
 
-  // o[rb][db][r] = O[query qc][dim 16 db + 4 g4 + r] of head rb; the row sum is complete in every lane.
-  if (q_row0 + qc >= m) return;
+  // sum[db][r] = O[query qc][dim 16 db + 4 g4 + r]; the row sum is complete in every lane.
+  const int row = row_of(cb);
+  if (row >= m || head_in_group(cb) >= G) return;
+  const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
+  uint16_t* orow = a.out + ((size_t)row * H + head_of(cb)) * kHeadDim;
 #pragma unroll
-  for (int rb = 0; rb < HEADS; ++rb) {
-    if (!head_active[rb]) continue;
-    const float inv = l_run[rb] > 0.f ? 1.0f / l_run[rb] : 0.f;
-    uint16_t* orow = a.out + ((size_t)(q_row0 + qc) * H + head[rb]) * kHeadDim;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-      *(uint2*)(orow + 16 * db + 4 * g4) = make_uint2(pack_bf16(o[rb][db][0] * inv, o[rb][db][1] * inv),
-                                                      pack_bf16(o[rb][db][2] * inv, o[rb][db][3] * inv));
-  }
+  for (int db = 0; db < 8; ++db)
+    *(uint2*)(orow + 16 * db + 4 * g4) = make_uint2(pack_bf16(sum[db][0] * inv, sum[db][1] * inv),
+                                                    pack_bf16(sum[db][2] * inv, sum[db][3] * inv));
 }
 
 int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
@@ -821,8 +755,9 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
                      dim3(256), 0, st, a);
   TS_TRY(check_launch("prefill_gather_kernel"));
   const int group = cfg->num_heads / cfg->num_kv_heads;
-  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(rows, 16),
-                  (unsigned)ceil_div(group, 4));
+  const int heads = prefill_heads(group);
+  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(rows, 16 * (kPfBlocks / heads)),
+                  (unsigned)ceil_div(group, heads));
   const bool cap = cfg->logit_cap > 0.f;
 #define TS_PF_LAUNCH(G_, C_)                                                                  \
   {                                                                                           \
@@ -830,7 +765,7 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
         (const void*)prefill_attn_kernel<G_, C_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
         (int)kPfLdsBytes);                                                                    \
     if (lds_ok != hipSuccess) return fail(TS_EHIP, "prefill attention: %zu bytes of LDS refused", kPfLdsBytes); \
-    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_>), grid, dim3(512), kPfLdsBytes, st, a); \
+    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_>), grid, dim3(64 * kPfGroups), kPfLdsBytes, st, a); \
   }
 #define TS_PF_CASE(G_)               \
   case G_:                           \
