@@ -1,0 +1,83 @@
+"""Steps whose every request is known to attend to all its tokens: the store writes the selection
+and nothing is scored.  Compared with the general path, which a call takes when its requests have
+a k of their own (the same k here)."""
+
+import pytest
+import torch
+
+from tokenselect_amd import ops
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+MAX_TOKENS = 5000
+
+
+def _state(cfg, lengths, extra, dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    total = sum(lengths) + extra + 8
+    order = torch.randperm(total, generator=g, device=dev).to(torch.int32)
+    table = torch.zeros((len(lengths), MAX_TOKENS), dtype=torch.int32, device=dev)
+    at = 0
+    for b, n in enumerate(lengths):
+        table[b, :n] = order[at:at + n]
+        at += n
+    pools = [torch.randn((total, cfg.num_kv_heads, 128), generator=g, device=dev).bfloat16() for _ in range(2)]
+    return g, pools, table, torch.tensor(lengths, dtype=torch.int32, device=dev), order[at:].contiguous()
+
+
+def _same(got, ref):
+    """Lists, tables, lengths and stored rows are copies: equal.  The outputs are the same fp32 sums
+    over another number of splits, rounded to bf16: one ulp of the larger."""
+    assert torch.equal(got["lens"], ref["lens"]) and torch.equal(got["table"], ref["table"])
+    assert torch.equal(got["k"], ref["k"]) and torch.equal(got["v"], ref["v"])
+    assert torch.equal(got["sel_len"], ref["sel_len"])
+    for b, n in enumerate(ref["sel_len"].tolist()):
+        assert torch.equal(got["sel"][b, :n], ref["sel"][b, :n])
+        assert torch.equal(got["sel_pos"][b, :n], ref["sel_pos"][b, :n])
+    a, b = got["out"].float(), ref["out"].float()
+    assert bool(((a - b).abs() <= b.abs() * 2.0 ** -7 + 1e-6).all())
+
+
+@pytest.mark.parametrize("lengths,top_k", [([0], 2048), ([1], 2048), ([127], 2048), ([128, 1023, 1024], 2048),
+                                           ([2687], 2048), ([2687, 640, 5, 4095 - 1408] , 2048),
+                                           ([4095, 4096], 4096), ([4735], 4096)])
+def test_dense_step_matches_the_general_path(dev, lengths, top_k):
+    say(f"dense step lengths={lengths} k={top_k}")
+    cfg = ops.LayerConfig(num_heads=8, num_kv_heads=2, n_init=128, n_local=512, top_k=top_k, rope_theta=5e5)
+    B, got = len(lengths), []
+    for own_k in (False, True):
+        g, (k_pool, v_pool), table, lens, slots = _state(cfg, lengths, B, dev, 5)
+        loc = slots[:B].clone()
+        if B == 3:
+            loc[1] = k_pool.shape[0]  # a slot outside the pool: the request is left untouched
+        q, k, v = (torch.randn((B, n * 128), generator=g, device=dev).bfloat16() for n in (8, 2, 2))
+        layer = ops.DecodeLayer(cfg, B, max(lengths) + 1, dev)
+        for _ in range(2):  # the second call finds the counters that the first one left
+            kpr = torch.full((B,), top_k, dtype=torch.int32, device=dev) if own_k else None
+            lens.copy_(torch.tensor(lengths))
+            bt = ops.Batch(lens, table, max(lengths) + 1, k_per_req=kpr)
+            out, sel, sel_pos, sel_len = layer.step(q, k, v, loc, k_pool, v_pool, bt)
+        got.append(dict(out=out.clone(), sel=sel.clone(), sel_pos=sel_pos.clone(), sel_len=sel_len.clone(), lens=lens,
+                        table=table, k=k_pool, v=v_pool))
+    torch.cuda.synchronize()
+    _same(*got)
+
+
+@pytest.mark.parametrize("length,rows", [(0, 1), (0, 300), (255, 1), (256, 8), (700, 9), (2176, 512), (2687, 1)])
+def test_dense_chunk_matches_the_general_path(dev, length, rows):
+    say(f"dense chunk length={length} rows={rows}")
+    cfg = ops.LayerConfig(num_heads=8, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5)
+    got = []
+    for own_k in (False, True):
+        g, (k_pool, v_pool), table, lens, slots = _state(cfg, [length], rows, dev, 6)
+        loc = slots[:rows].clone()
+        q, k, v = (torch.randn((rows, n * 128), generator=g, device=dev).bfloat16() for n in (8, 2, 2))
+        chunk = ops.PrefillChunk(cfg, length + rows, dev, max_rows=512)
+        kpr = torch.full((1,), 2048, dtype=torch.int32, device=dev) if own_k else None
+        bt = ops.Batch(lens, table, length + rows, k_per_req=kpr)
+        out, sel, sel_pos, sel_len = chunk.step(q, k, v, loc, k_pool, v_pool, bt)
+        got.append(dict(out=out.clone(), sel=sel.view(1, -1).clone(), sel_pos=sel_pos.view(1, -1).clone(),
+                        sel_len=sel_len.view(-1).clone(), lens=lens, table=table, k=k_pool, v=v_pool))
+    torch.cuda.synchronize()
+    _same(*got)

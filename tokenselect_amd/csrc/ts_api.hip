@@ -201,6 +201,49 @@ static int layer_selection_form(const ts_config* cfg, int32_t batch, int32_t max
   return layer_selection_form(cfg, &bt);
 }
 
+// Whether every request of a call attends to all its tokens, by what the host knows: no
+// length exceeds max_seq_len (the kernels clamp to it) and no request has a k of its own.
+// There is nothing to score then (tr.py:377-378), so the launches that prepare a selection are
+// left out, and the attention is laid out for the lengths at hand.  With a selection cache the
+// general path keeps the cache's books.
+static bool known_dense(const ts_config* cfg, const ts_batch* bt, const ts_selcache* cache) {
+  return cache == nullptr && bt->k_per_req == nullptr &&
+         (int64_t)cfg->n_init + cfg->top_k + cfg->n_local >= bt->max_seq_len;
+}
+
+// The longest list of a call, as its attention is laid out: where every request is known to be
+// dense no list is longer than max_seq_len (300 tokens: 3 workgroups per KV head instead of 21
+// that mostly find nothing).  Never a layout that needs more than the one the workspace is
+// sized for: splits do not shrink with the list in every case.
+static int32_t attn_list_bound(const ts_config* cfg, const ts_batch* bt, const ts_selcache* cache, int32_t max_sel) {
+  if (!known_dense(cfg, bt, cache) || bt->max_seq_len >= max_sel) return max_sel;
+  return attn_workspace_bytes(cfg, bt->batch, bt->max_seq_len) <= attn_workspace_bytes(cfg, bt->batch, max_sel)
+             ? bt->max_seq_len
+             : max_sel;
+}
+
+// The list that a step's store writes, or sel == NULL where the step is not known to be dense,
+// or where run_layer is going to refuse the call.
+static DenseList step_list(const ts_config* cfg, const ts_batch* bt, const ts_selcache* cache, const void* q,
+                           const float* q_cos, const float* q_sin, const void* out, int32_t* sel, int32_t* sel_pos,
+                           int64_t sel_stride, int32_t* sel_len, void* workspace, size_t workspace_bytes) {
+  DenseList list{};
+  if (validate_config(cfg) != TS_OK || validate_batch(cfg, bt) != TS_OK || !known_dense(cfg, bt, cache) ||
+      cfg->page_size != 1 || !q || !q_cos || !q_sin || !out || !sel || !sel_pos || !sel_len || !workspace ||
+      (uintptr_t)q % 16 || (uintptr_t)out % 16 || (uintptr_t)workspace % 256)
+    return list;
+  const LayerWorkspace w = layer_workspace(cfg, bt->batch, bt->max_seq_len);
+  if (sel_stride < w.max_sel || workspace_bytes < w.total) return list;
+  list.sel = sel;
+  list.sel_pos = sel_pos;
+  list.sel_stride = sel_stride;
+  list.sel_len = sel_len;
+  list.clear = attn_tickets(cfg, bt->batch, attn_list_bound(cfg, bt, cache, w.max_sel), (char*)workspace + w.attn_ws);
+  list.clear_per_req = attn_tickets_per_request(cfg);
+  list.max_seq_len = bt->max_seq_len;
+  return list;
+}
+
 // Decode (chunk_rows == 0: one query row per request, q_cos / q_sin are the [D] rows
 // of position n_local) or one prefill chunk of a single request (chunk_rows > 0:
 // q_cos / q_sin are the whole [table_rows, D] tables).
@@ -210,7 +253,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                      const ts_selcache* cache, void* out, int32_t* sel, int32_t* sel_pos,
                      int64_t sel_stride, int32_t* sel_len, void* workspace, size_t workspace_bytes,
                      ts_stream_t stream, const StepStore* store = nullptr,
-                     const ChunkStore* chunk_store = nullptr) {
+                     const ChunkStore* chunk_store = nullptr, bool listed = false) {
   TS_TRY(validate_config(cfg));
   TS_TRY(validate_batch(cfg, bt));
   SeparateKernelsScope separate(bt->separate_kernels != 0);
@@ -250,7 +293,9 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
 
   const int max_n = bt->max_seq_len - cfg->n_init - cfg->n_local;
   const SelectWorkspace fused = select_workspace(cfg, bt->batch, bt->max_seq_len);
-  uint32_t* tickets = attn_tickets(cfg, bt->batch, w.max_sel, ws + w.attn_ws);
+  const bool dense = known_dense(cfg, bt, cache) && chunk_store == nullptr;
+  const int32_t longest = dense ? attn_list_bound(cfg, bt, cache, w.max_sel) : w.max_sel;
+  uint32_t* tickets = attn_tickets(cfg, bt->batch, longest, ws + w.attn_ws);
 
   // Fingerprint: every request's single decode row is rotated to n_local
   // (tr.py:381-388); the mean over one row is the row itself (tr.py:392).  The same
@@ -276,6 +321,18 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   // the query itself; this call's attention kernel clears the counters again.
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;
+  if (dense) {
+    // (listed: the store has written the selection; otherwise the last of the top-k kernels,
+    // which writes a dense request's list, is all that is left of the selection)
+    if (chunk_rows > 0) TS_TRY(check_fingerprint(q, chunk_rows, q_cos, q_sin, table_rows, qf, cfg->n_local));
+    if (!listed) TS_TRY(launch_topk(topk, bt->batch, 0, (hipStream_t)stream));
+    if (chunk_rows > 0)
+      return launch_prefill_attn(cfg, q, q_stride, chunk_rows, k_pool, v_pool, pool_rows, sel, sel_len, longest, out,
+                                 ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream);
+    return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch, longest,
+                       out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream,
+                       plain_decode && !starts_with_selection ? &zero : nullptr);
+  }
   if (starts_with_selection) {
   } else if (chunk_rows > 0) {
     // Chunk fingerprint: row i rotated to n_local + i, mean over the rows (tr.py:380-392).
@@ -351,12 +408,17 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
   // (a call that repeats a step after a give-up does not append again: it is the layer alone)
   const bool rides = cache != nullptr && bt->rerun == 0;
   if (!rides) {
-    if (bt->rerun == 0)
+    DenseList list{};
+    if (bt->rerun == 0) {
+      if (kv->pages == nullptr)
+        list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
+                         workspace_bytes);
       TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
                              pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
-                             (hipStream_t)stream));
+                             (hipStream_t)stream, list.sel ? &list : nullptr));
+    }
     return run_layer(cfg, bt, q, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
-                     sel_stride, sel_len, workspace, workspace_bytes, stream);
+                     sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, list.sel != nullptr);
   }
   // The checks ts_kv_store makes.
   TS_TRY(validate_config(cfg));
@@ -531,6 +593,22 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
   TS_REQUIRE(bt->table != nullptr && bt->seq_lens != nullptr, TS_EINVAL, "ts_prefill_step: NULL table / seq_lens");
   int32_t* table = const_cast<int32_t*>(bt->table);
   int32_t* seq_len = const_cast<int32_t*>(bt->seq_lens);
+  // A chunk that is known to be dense has no fingerprint to ride in: its store writes the
+  // selection instead.
+  DenseList list{};
+  if (kv->pages == nullptr && bt->rerun == 0 &&
+      chunk_store_takes_list(rows, kv->max_tokens, bt->max_seq_len) &&
+      table_rows >= (int64_t)(cfg ? cfg->n_local : 0) + rows && (uintptr_t)cos_table % 16 == 0 &&
+      (uintptr_t)sin_table % 16 == 0)
+    list = step_list(cfg, bt, nullptr, q, cos_table, sin_table, out, sel, sel_pos, sel_stride, sel_len, workspace,
+                     workspace_bytes);
+  if (list.sel) {
+    TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
+                                 v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream, &list));
+    return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr, out,
+                     sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr,
+                     /*listed=*/true);
+  }
   const bool rides = kv->pages == nullptr && bt->rerun == 0 && kv->max_tokens <= 0x1fffff &&
                      rows <= 1023 * 32;
   if (!rides) {

@@ -583,6 +583,10 @@ uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* w
   return (uint32_t*)((char*)workspace + attn_workspace(cfg, batch, max_sel_len).tickets);
 }
 
+size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
+  return attn_workspace(cfg, batch, max_sel_len).total;
+}
+
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,

@@ -139,15 +139,33 @@ int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q
                          const int32_t* gave_up_len, const ZeroSet& zero, hipStream_t stream,
                          const StepStore* store = nullptr);
 
+// The selection of a call whose every request attends to all its tokens, written by the store
+// that precedes it (per-token tables only): sel and sel_pos of all positions, the new ones
+// included, and sel_len; and the attention's tickets cleared.
+struct DenseList {
+  int32_t* sel;  // NULL: no list
+  int32_t* sel_pos;
+  int64_t sel_stride;
+  int32_t* sel_len;
+  uint32_t* clear;
+  int clear_per_req;
+  int max_seq_len;
+};
+
 // ts_kv_store and ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
 int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                     const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
                     int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
-                    int32_t max_tokens, hipStream_t stream);
+                    int32_t max_tokens, hipStream_t stream, const DenseList* list = nullptr);
+// (list: only where chunk_store_takes_list says so)
+bool chunk_store_takes_list(int32_t rows, int32_t max_tokens, int32_t max_seq_len);
 int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                           const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
                           void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
-                          hipStream_t stream);
+                          hipStream_t stream, const DenseList* list = nullptr);
+// What launch_fingerprint requires of its arguments.
+int check_fingerprint(const void* q, int32_t rows, const float* cos_table, const float* sin_table,
+                      int64_t table_rows, const void* qf, int32_t n_local);
 // ts_sparse_prefill_attn for query rows that lie q_stride elements apart.
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
@@ -158,6 +176,7 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
 // tickets_clear = false makes the launcher clear them first, true says an earlier
 // kernel of the stream already did (attn_tickets() tells it where they are).
 uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* workspace);
+size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len);
 // Tickets per request (the words to clear): one per KV head.
 int attn_tickets_per_request(const ts_config* cfg);
 // clear_after: regions that the kernel clears on the side (the counters of the stream's

@@ -681,19 +681,25 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
                                                     pack_bf16(sum[db][2] * inv, sum[db][3] * inv));
 }
 
-int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
-                       const float* sin_table, int64_t table_rows, void* qf, const ZeroSet& zero,
-                       hipStream_t stream, const ChunkStore* store) {
-  TS_TRY(validate_config(cfg));
-  TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);
+int check_fingerprint(const void* q, int32_t rows, const float* cos_table, const float* sin_table,
+                      int64_t table_rows, const void* qf, int32_t n_local) {
   TS_REQUIRE(q && cos_table && sin_table && qf, TS_EINVAL, "ts_fingerprint: NULL tensor argument");
   TS_REQUIRE_ALIGNED(q, 16, "q");
   TS_REQUIRE_ALIGNED(cos_table, 16, "cos_table");
   TS_REQUIRE_ALIGNED(sin_table, 16, "sin_table");
   TS_REQUIRE(rows >= 1, TS_EINVAL, "ts_fingerprint: rows %d < 1", rows);
-  TS_REQUIRE(table_rows >= (int64_t)cfg->n_local + rows, TS_EINVAL,
+  TS_REQUIRE(table_rows >= (int64_t)n_local + rows, TS_EINVAL,
              "ts_fingerprint: cos/sin tables have %lld rows, need n_local + rows = %lld",
-             (long long)table_rows, (long long)cfg->n_local + rows);
+             (long long)table_rows, (long long)n_local + rows);
+  return TS_OK;
+}
+
+int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
+                       const float* sin_table, int64_t table_rows, void* qf, const ZeroSet& zero,
+                       hipStream_t stream, const ChunkStore* store) {
+  TS_TRY(validate_config(cfg));
+  TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);
+  TS_TRY(check_fingerprint(q, rows, cos_table, sin_table, table_rows, qf, cfg->n_local));
   ChunkStore cs{};
   unsigned grid_y = kFpSplit;
   if (store) {  // rows of 32 threads: 32 rows per workgroup of 1024

@@ -18,12 +18,29 @@ constexpr int kLenMask = (1 << kLenBits) - 1;
 constexpr int kChunkThreadsPerRow = 32;
 constexpr int kChunkCountedWgs = 1023;  // more workgroups take the two-launch form
 
+// A workgroup counts itself in when all its wavefronts have read the length, at its end,
+// where nobody waits for the answer; whoever completes the count knows that every workgroup
+// has read the old length, and writes the new one.
+__device__ __forceinline__ void count_chunk_workgroup(const ChunkStore& cs, int len) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int before = __hip_atomic_fetch_add(cs.seq_len, 1 << kLenBits, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+    if ((before >> kLenBits) + 1 == cs.workgroups)
+      __hip_atomic_store(cs.seq_len, min(len + cs.rows, cs.max_tokens), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The old length: the upper bits may already hold other workgroups' counts.
+__device__ __forceinline__ int counted_length(const ChunkStore& cs) {
+  return __hip_atomic_load(cs.seq_len, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLenMask;
+}
+
 // wg: this workgroup among the cs.workgroups that store; threads: its size.
 template <bool COUNTED>
 __device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, int threads) {
-  // Counted: the upper bits may already hold other workgroups' counts.
-  const int len = COUNTED ? (__hip_atomic_load(cs.seq_len, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLenMask)
-                          : *cs.seq_len;
+  const int len = COUNTED ? counted_length(cs) : *cs.seq_len;
   const int r = wg * (threads / kChunkThreadsPerRow) + (int)threadIdx.x / kChunkThreadsPerRow;
   const int t = threadIdx.x % kChunkThreadsPerRow;
   const int at = len + r;
@@ -36,19 +53,7 @@ __device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, i
     }
     if (t == 0) cs.table[at] = (int32_t)slot;
   }
-  if (COUNTED) {
-    // A workgroup counts itself in when all its wavefronts have read the length, at its
-    // end, where nobody waits for the answer; whoever completes the count knows that
-    // every workgroup has read the old length, and writes the new one.
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int before = __hip_atomic_fetch_add(cs.seq_len, 1 << kLenBits, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-      if ((before >> kLenBits) + 1 == cs.workgroups)
-        __hip_atomic_store(cs.seq_len, min(len + cs.rows, cs.max_tokens), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+  if (COUNTED) count_chunk_workgroup(cs, len);
 }
 
 }  // namespace ts

@@ -9,15 +9,21 @@ namespace ts {
 // pool slot out_cache_loc[b], appends the slot to the request's table and bumps
 // its length.  A full table (tr.py:334 asserts) or a slot outside the pool
 // leaves the request untouched.
-__global__ __launch_bounds__(256) void kv_store_kernel(const uint4* __restrict__ k,
-                                                       const uint4* __restrict__ v,
-                                                       const int32_t* __restrict__ loc,
-                                                       uint4* __restrict__ k_pool,
-                                                       uint4* __restrict__ v_pool, int64_t pool_rows,
-                                                       int32_t* __restrict__ table,
-                                                       int64_t table_stride,
-                                                       int32_t* __restrict__ seq_lens,
-                                                       int row_vec, int kv_stride, int max_tokens) {
+// LIST: every request of the step attends to all its tokens, and the workgroup also writes
+// the request's selection (list), the table itself.  Bound by three dependent memory round
+// trips (length and slot, stores, the length's store); the table entries are asked for with the
+// first.  A dense step then has two launches, this (2.2 us) and the attention, where it had
+// a store (1.7), a selection kernel or a rotation and a list (3.3 to 4.6) and the attention:
+// 8 layers of a 2003-token request, two steps, 320 -> 261 us; 2 layers of a 300-token prompt
+// with 8 tokens 430 -> 368 us.
+constexpr int kListThreads = 1024;  // one request's few thousand entries in a handful of steps
+constexpr int kListAhead = 4;       // table entries a thread asks for before it knows the length
+
+template <bool LIST>
+__global__ __launch_bounds__(LIST ? kListThreads : 256) void kv_store_kernel(
+    const uint4* __restrict__ k, const uint4* __restrict__ v, const int32_t* __restrict__ loc,
+    uint4* __restrict__ k_pool, uint4* __restrict__ v_pool, int64_t pool_rows, int32_t* table,
+    int64_t table_stride, int32_t* seq_lens, int row_vec, int kv_stride, int max_tokens, DenseList list) {
   const int b = blockIdx.x;
   // The new rows are asked for together with the slot and the length, not after them: the
   // kernel is two memory round trips long instead of three.
@@ -29,18 +35,52 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const uint4* __restrict__
   }
   const int slot = loc[b];
   const int len = seq_lens[b];
-  if (slot < 0 || slot >= pool_rows || len >= max_tokens) return;
-  if (first < row_vec) {
-    k_pool[(size_t)slot * row_vec + first] = k0;
-    v_pool[(size_t)slot * row_vec + first] = v0;
+  int32_t* const tab = table + (int64_t)b * table_stride;
+  int32_t ahead[kListAhead];
+  int64_t known = 0;  // entries that are there to be read, whatever the length
+  if (LIST) {
+    known = min((int64_t)list.max_seq_len, table_stride);
+#pragma unroll
+    for (int i = 0; i < kListAhead; ++i) {
+      const int pos = first + i * kListThreads;
+      ahead[i] = pos < known ? tab[pos] : 0;
+    }
   }
-  for (int i = first + blockDim.x; i < row_vec; i += blockDim.x) {
-    k_pool[(size_t)slot * row_vec + i] = k[(size_t)b * kv_stride + i];
-    v_pool[(size_t)slot * row_vec + i] = v[(size_t)b * kv_stride + i];
+  const bool ok = slot >= 0 && slot < pool_rows && len < max_tokens;
+  if (!LIST && !ok) return;
+  if (ok) {
+    if (first < row_vec) {
+      k_pool[(size_t)slot * row_vec + first] = k0;
+      v_pool[(size_t)slot * row_vec + first] = v0;
+    }
+    for (int i = first + blockDim.x; i < row_vec; i += blockDim.x) {
+      k_pool[(size_t)slot * row_vec + i] = k[(size_t)b * kv_stride + i];
+      v_pool[(size_t)slot * row_vec + i] = v[(size_t)b * kv_stride + i];
+    }
+  }
+  if (LIST) {
+    const int L = min(max(ok ? len + 1 : len, 0), list.max_seq_len);
+    int32_t* const sel = list.sel + (int64_t)b * list.sel_stride;
+    int32_t* const sel_pos = list.sel_pos + (int64_t)b * list.sel_stride;
+    auto emit = [&](int pos, int32_t entry) {
+      const uint32_t s = (uint32_t)(ok && pos == len ? slot : entry);
+      sel_pos[pos] = pos;
+      sel[pos] = (int32_t)(s < (uint32_t)pool_rows ? s : (uint32_t)pool_rows - 1);
+    };
+#pragma unroll
+    for (int i = 0; i < kListAhead; ++i) {
+      const int pos = first + i * kListThreads;
+      if (pos < L) emit(pos, pos < known ? ahead[i] : (ok && pos == len ? slot : tab[pos]));
+    }
+    for (int pos = first + kListAhead * kListThreads; pos < L; pos += kListThreads)
+      emit(pos, ok && pos == len ? slot : tab[pos]);
+    for (int i = first; i < list.clear_per_req; i += kListThreads)
+      list.clear[(size_t)b * list.clear_per_req + i] = 0u;
+    if (first == 0) list.sel_len[b] = L;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    table[(int64_t)b * table_stride + len] = slot;
+  if (threadIdx.x == 0 && ok) {
+    tab[len] = slot;
     seq_lens[b] = len + 1;
   }
 }
@@ -49,13 +89,32 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const uint4* __restrict__
 // fingerprint launch of a chunk can also run on the side.
 constexpr int kChunkRowsPerWg = 256 / kChunkThreadsPerRow;  // few workgroups, few counts on one word
 
+// The workgroups past the first cs_wgs write the chunk's dense selection (list): entries
+// before the chunk from the table, those of the chunk from the caller's slots.
 template <bool COUNTED>
 __global__ __launch_bounds__(256) void kv_store_chunk_kernel(
     const uint4* __restrict__ k, const uint4* __restrict__ v, const int32_t* __restrict__ loc,
     uint4* __restrict__ k_pool, uint4* __restrict__ v_pool, int64_t pool_rows,
-    int32_t* __restrict__ table, int32_t* seq_len, int rows, int row_vec, int kv_stride, int max_tokens) {
+    int32_t* table, int32_t* seq_len, int rows, int row_vec, int kv_stride, int max_tokens, int cs_wgs,
+    DenseList list) {
   ChunkStore cs{k, v, loc, k_pool, v_pool, pool_rows, table, seq_len, rows, row_vec, max_tokens, kv_stride, (int)gridDim.x};
-  store_chunk_rows<COUNTED>(cs, (int)blockIdx.x, 256);
+  if (!COUNTED || (int)blockIdx.x < cs_wgs) {
+    store_chunk_rows<COUNTED>(cs, (int)blockIdx.x, 256);
+    return;
+  }
+  const int len = counted_length(cs);
+  const int L = min(max(min(len + rows, max_tokens), 0), list.max_seq_len);
+  const int pos = ((int)blockIdx.x - cs_wgs) * 256 + (int)threadIdx.x;
+  if (pos < L) {
+    // (a slot of the chunk is clamped to the pool as it is stored, an entry as it is looked up)
+    const int32_t at = pos < len ? table[pos] : loc[pos - len];
+    const uint32_t s = pos >= len && at < 0 ? 0u : (uint32_t)at;
+    list.sel_pos[pos] = pos;
+    list.sel[pos] = (int32_t)(s < (uint32_t)pool_rows ? s : (uint32_t)pool_rows - 1);
+  }
+  if (pos == 0) *list.sel_len = L;
+  if (pos < list.clear_per_req) list.clear[pos] = 0u;
+  count_chunk_workgroup(cs, len);
 }
 
 __global__ void seq_len_add_kernel(int32_t* seq_len, int rows, int max_tokens) {
@@ -179,7 +238,7 @@ static int check_pool_arg(const ts_config* cfg, const int32_t* out_cache_loc, co
 int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                     const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
                     int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
-                    int32_t max_tokens, hipStream_t stream) {
+                    int32_t max_tokens, hipStream_t stream, const DenseList* list) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_lens, TS_EINVAL,
              "ts_kv_store: NULL tensor argument");
@@ -197,6 +256,7 @@ int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t 
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
   TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store"));
   const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
+  TS_REQUIRE(list == nullptr || pages == nullptr, TS_EINVAL, "internal: a list needs a per-token table");
   if (pages) {
     hipLaunchKernelGGL(kv_store_paged_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
                        (const uint4*)k, (const uint4*)v, (uint4*)k_pool, (uint4*)v_pool,
@@ -204,16 +264,28 @@ int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t 
                        page_shift_of(cfg->page_size), page_pool_of(pages));
     return check_launch("kv_store_paged_kernel");
   }
-  hipLaunchKernelGGL(kv_store_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
-                     (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                     pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens);
+  if (list)
+    hipLaunchKernelGGL(kv_store_kernel<true>, dim3((unsigned)batch), dim3(kListThreads), 0, stream,
+                       (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
+                       pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens, *list);
+  else
+    hipLaunchKernelGGL(kv_store_kernel<false>, dim3((unsigned)batch), dim3(256), 0, stream,
+                       (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
+                       pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens, DenseList{});
   return check_launch("kv_store_kernel");
+}
+
+static int chunk_list_workgroups(int32_t max_seq_len) { return (int)ceil_div(max_seq_len, 256); }
+
+bool chunk_store_takes_list(int32_t rows, int32_t max_tokens, int32_t max_seq_len) {
+  return max_tokens <= kLenMask &&
+         ceil_div(rows, kChunkRowsPerWg) + chunk_list_workgroups(max_seq_len) <= kChunkCountedWgs;
 }
 
 int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                           const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
                           void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
-                          hipStream_t stream) {
+                          hipStream_t stream, const DenseList* list) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_len, TS_EINVAL,
              "ts_kv_store_chunk: NULL tensor argument");
@@ -229,6 +301,8 @@ int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, in
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
   TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store_chunk"));
   const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
+  TS_REQUIRE(list == nullptr || (pages == nullptr && chunk_store_takes_list(rows, max_tokens, list->max_seq_len)),
+             TS_EINVAL, "internal: a list of %d rows does not ride in the chunk's store", rows);
   if (pages) {
     hipLaunchKernelGGL(kv_store_chunk_paged_kernel, dim3((unsigned)rows), dim3(256), 0,
                        stream, (const uint4*)k, (const uint4*)v, (uint4*)k_pool,
@@ -238,14 +312,16 @@ int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, in
   }
   const unsigned wgs = (unsigned)ceil_div(rows, kChunkRowsPerWg);
   if (wgs <= (unsigned)kChunkCountedWgs && max_tokens <= kLenMask) {
-    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs), dim3(256), 0, stream,
+    const unsigned list_wgs = list ? (unsigned)chunk_list_workgroups(list->max_seq_len) : 0u;
+    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs + list_wgs), dim3(256), 0, stream,
                        (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                       pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens);
+                       pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens, (int)wgs,
+                       list ? *list : DenseList{});
     return check_launch("kv_store_chunk_kernel");
   }
   hipLaunchKernelGGL(kv_store_chunk_kernel<false>, dim3(wgs), dim3(256), 0, stream,
                      (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                     pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens);
+                     pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens, (int)wgs, DenseList{});
   TS_TRY(check_launch("kv_store_chunk_kernel"));
   hipLaunchKernelGGL(seq_len_add_kernel, dim3(1), dim3(1), 0, stream, seq_len, rows,
                      max_tokens);
