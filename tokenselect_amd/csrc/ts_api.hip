@@ -610,7 +610,7 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
                      /*listed=*/true);
   }
   const bool rides = kv->pages == nullptr && bt->rerun == 0 && kv->max_tokens <= 0x1fffff &&
-                     rows <= 1023 * 32;
+                     rows <= 1023 * 16;
   if (!rides) {
     if (bt->rerun == 0)  // (a call that repeats a chunk after a give-up does not append again)
       TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,

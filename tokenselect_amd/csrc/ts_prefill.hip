@@ -12,7 +12,7 @@
 namespace ts {
 
 // ------------------------------------------------------------------ fingerprint
-// Two workgroups per head (32 rotation pairs each), 1024 threads = 8 quads of pairs
+// Four workgroups per head (16 rotation pairs each), 512 threads = 4 quads of pairs
 // x 128 row groups, so that a chunk of 512 rows is one step of four independent rows
 // per thread (the kernel is bound by the latency of its loads).  Row r
 // is rotated with table row first_pos + r exactly like the rotation kernel (every
@@ -22,9 +22,10 @@ namespace ts {
 constexpr int kFpRowGroups = 128;
 constexpr int kFpInFlight = 4;  // rows per step of a row group
 constexpr int kFpVec = 4;       // rotation pairs per thread
-constexpr int kFpSplit = 2;     // workgroups per head
+constexpr int kFpSplit = 4;     // workgroups per head
+constexpr int kFpThreads = kHeadDim / 2 / kFpSplit / kFpVec * kFpRowGroups;
 
-__global__ __launch_bounds__(1024) void fingerprint_kernel(
+__global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
     const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
     const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int heads,
     ZeroSet zero, ChunkStore cs) {
@@ -32,14 +33,15 @@ __global__ __launch_bounds__(1024) void fingerprint_kernel(
   constexpr int half = kHeadDim / 2;
   constexpr int kPairs = half / kFpSplit;   // rotation pairs of this workgroup
   constexpr int kLanes = kPairs / kFpVec;   // threads per row
-  static_assert(kLanes * kFpRowGroups == 1024, "1024 threads per workgroup");
+  static_assert(kFpThreads == kLanes * kFpRowGroups && kFpThreads == 2 * kPairs * kFpRowGroups / 8,
+                "a thread per row group and four pairs, and per eight row groups and column");
   const int h = blockIdx.x;
   const int first_pair = blockIdx.y * kPairs;
   const int i = first_pair + (threadIdx.x % kLanes) * kFpVec, rg = threadIdx.x / kLanes;
   // On the side: clear the words the selection kernel after this one counts into.
   {
-    const int64_t gid = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 1024 + threadIdx.x;
-    const int64_t step = (int64_t)gridDim.x * gridDim.y * 1024;
+    const int64_t gid = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kFpThreads + threadIdx.x;
+    const int64_t step = (int64_t)gridDim.x * gridDim.y * kFpThreads;
     clear_regions(zero, gid, step);
   }
   // Also on the side: the workgroups past the fingerprint's own store the chunk's K/V
@@ -47,7 +49,7 @@ __global__ __launch_bounds__(1024) void fingerprint_kernel(
   // done, riding here instead of in a launch of its own).
   if ((int)blockIdx.y >= kFpSplit) {
     const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
-    if (cs.k != nullptr && wg < cs.workgroups) store_chunk_rows<true>(cs, wg, 1024);
+    if (cs.k != nullptr && wg < cs.workgroups) store_chunk_rows<true>(cs, wg, kFpThreads);
     return;
   }
   float lo_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f}, hi_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f};
@@ -702,14 +704,14 @@ int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_
   TS_TRY(check_fingerprint(q, rows, cos_table, sin_table, table_rows, qf, cfg->n_local));
   ChunkStore cs{};
   unsigned grid_y = kFpSplit;
-  if (store) {  // rows of 32 threads: 32 rows per workgroup of 1024
+  if (store) {  // 32 threads per row
     cs = *store;
-    cs.workgroups = (int)ceil_div(cs.rows, 1024 / kChunkThreadsPerRow);
+    cs.workgroups = (int)ceil_div(cs.rows, kFpThreads / kChunkThreadsPerRow);
     TS_REQUIRE(cs.workgroups <= kChunkCountedWgs && cs.max_tokens <= kLenMask, TS_EINVAL,
                "internal: a chunk store of %d rows does not ride in the fingerprint launch", cs.rows);
     grid_y += (unsigned)ceil_div(cs.workgroups, cfg->num_heads);
   }
-  hipLaunchKernelGGL(fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y), dim3(1024), 0, stream,
+  hipLaunchKernelGGL(fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y), dim3(kFpThreads), 0, stream,
                      (const uint16_t*)q, q_stride, (uint16_t*)qf, cos_table, sin_table, table_rows,
                      cfg->n_local, rows, cfg->num_heads, zero, cs);
   return check_launch("fingerprint_kernel");
