@@ -131,7 +131,8 @@ typedef struct ts_batch {
                                after wait_us while all kernels still exit        */
   int32_t workspace_clean;  /* ts_decode_layer only.  1: the caller states that this
                                workspace was last used by a ts_decode_layer call with
-                               the same cfg, batch, max_seq_len and cache == NULL that
+                               the same cfg, batch, max_seq_len (or one of the same
+                               ts_decode_layer_layout) and cache == NULL that
                                completed without a give-up, and by nothing since (every
                                such call leaves the selection's counters zero again:
                                its attention kernel clears them on the side).  The
@@ -531,6 +532,12 @@ int ts_set_fused_select(int enable);
  * same answer: host_seq_lens changes how the phases are packed, not the form). */
 int ts_decode_layer_selection(const ts_config* cfg, int32_t batch, int32_t max_seq_len);
 int ts_decode_layer_selection_of(const ts_config* cfg, const ts_batch* bt);
+
+/* Where a ts_decode_layer call of this shape without a selection cache keeps the counters of its
+ * selection, as one number: calls whose numbers are equal (and not negative) keep the same
+ * counters in the same places, so that the one may state workspace_clean after the other
+ * though their max_seq_len differ.  -1: the selection is not the single ts_select launch. */
+int64_t ts_decode_layer_layout(const ts_config* cfg, int32_t batch, int32_t max_seq_len);
 size_t ts_decode_layer_workspace_bytes(const ts_config* cfg, int32_t batch, int32_t max_seq_len);
 int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, const float* q_cos,
                     const float* q_sin, const void* k_pool, const void* v_pool,

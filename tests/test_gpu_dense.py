@@ -1,6 +1,7 @@
 """Steps whose every request is known to attend to all its tokens: the store writes the selection
 and nothing is scored.  Compared with the general path, which a call takes when its requests have
-a k of their own (the same k here)."""
+a k of their own (the same k here).  And steps of a growing context, which start with the selection
+as long as the workspace's layout stays what the step before left clean."""
 
 import pytest
 import torch
@@ -81,3 +82,29 @@ def test_dense_chunk_matches_the_general_path(dev, length, rows):
                         sel_len=sel_len.view(-1).clone(), lens=lens, table=table, k=k_pool, v=v_pool))
     torch.cuda.synchronize()
     _same(*got)
+
+
+@pytest.mark.parametrize("first,steps,B,pool", [(2640, 80, 1, -1), (3180, 40, 3, -1), (3000, 70, 1, 9)])
+def test_growing_context_on_one_workspace(dev, first, steps, B, pool):
+    """Lengths that grow past dense, past 64-token and past workgroup boundaries, one object for
+    all steps against a fresh one (whose first call clears everything) at each: the same
+    selections and outputs, bit for bit."""
+    say(f"growing context from {first}, {steps} steps, B={B} pool={pool}")
+    cfg = ops.LayerConfig(num_heads=8, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5,
+                          pool_kernel=pool)
+    last = first + steps
+    g, (k_pool, v_pool), table, lens, _ = _state(cfg, [last] * B, 0, dev, 8)
+    layer = ops.DecodeLayer(cfg, B, last, dev)
+    layer.workspace.fill_(0xa5)
+    for n in range(first, last):
+        q = torch.randn((B, 8 * 128), generator=g, device=dev).bfloat16()
+        lens.copy_(torch.tensor([n - 300 * b for b in range(B)]))
+        bt = ops.Batch(lens, table, n)
+        got = [t.clone() for t in layer(q, k_pool, v_pool, bt)]
+        fresh = ops.DecodeLayer(cfg, B, last, dev)
+        want = fresh(q, k_pool, v_pool, bt)
+        torch.cuda.synchronize()
+        assert not layer.gave_up() and torch.equal(got[3], want[3]), n
+        for b, s in enumerate(want[3].tolist()):
+            assert torch.equal(got[1][b, :s], want[1][b, :s]) and torch.equal(got[2][b, :s], want[2][b, :s]), (n, b)
+        assert torch.equal(got[0], want[0]), n

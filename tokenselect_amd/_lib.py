@@ -110,6 +110,7 @@ SIGNATURES = {
     "ts_set_fused_select": (_i32, [_i32]),
     "ts_decode_layer_selection": (_i32, [_CFG, _i32, _i32]),
     "ts_decode_layer_selection_of": (_i32, [_CFG, _BT]),
+    "ts_decode_layer_layout": (_i64, [_CFG, _i32, _i32]),
     "ts_decode_layer_workspace_bytes": (_size, [_CFG, _i32, _i32]),
     "ts_decode_layer_votes": (_i32, [_CFG, _BT, _ptr, _ptr, _ptr, _ptr, _i64, _SC, _ptr, _i64, _ptr,
                                      _size, _ptr]),
@@ -164,7 +165,8 @@ def binding():
             raise ImportError(f"the Python binding next to {LIB_PATH} is missing or does not load ({e}): "
                               "build it with `python -m tokenselect_amd.build`") from e
         _ts_bind.connect(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in
-                           ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step")))
+                           ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step",
+                            "ts_decode_layer_layout")))
         _bind = _ts_bind
     return _bind
 

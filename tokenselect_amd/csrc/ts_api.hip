@@ -168,6 +168,19 @@ int ts_decode_layer_selection_of(const ts_config* cfg, const ts_batch* bt) {
   return layer_selection_form(cfg, bt);
 }
 
+int64_t ts_decode_layer_layout(const ts_config* cfg, int32_t batch, int32_t max_seq_len) {
+  if (validate_config(cfg) != TS_OK || batch < 1 || max_seq_len < 1) return -1;
+  const SelectWorkspace s = select_workspace(cfg, batch, max_seq_len);
+  if (s.tokens_per_block <= 0) return -1;
+  // The regions select_zero_regions names follow from the batch, the head count, where the
+  // selection's workspace starts, where its last piece does and how many statistics per head
+  // are cleared (at most kSelMaxChunks); the offsets are multiples of 256.
+  const int64_t at = (int64_t)(layer_workspace(cfg, batch, max_seq_len).select_ws / 256);
+  const int64_t sync = (int64_t)(s.sync / 256);
+  if (at >= (int64_t)1 << 26 || sync >= (int64_t)1 << 26 || s.clear_chunks >= 1 << 11) return -1;
+  return (at << 37) | (sync << 11) | s.clear_chunks;
+}
+
 size_t ts_decode_layer_workspace_bytes(const ts_config* cfg, int32_t batch, int32_t max_seq_len) {
   if (validate_config(cfg) != TS_OK || batch < 1 || max_seq_len < 1) return 0;
   // A workspace sized for `batch` serves every smaller batch and both settings of
