@@ -12,6 +12,8 @@
 // them with the matching pieces of x from LDS (bf16, staged once per workgroup of
 // eight wavefronts) and the wavefront reduces its sums (rows x B) on its own: no
 // exchange between wavefronts.
+#include <type_traits>
+
 #include "ts_pages.h"
 
 namespace ts {
@@ -20,6 +22,7 @@ constexpr int kQkvMaxBatch = 8;      // rows of x
 constexpr int kQkvWaves = 8;         // wavefronts per workgroup
 constexpr int kQkvPieces = 8;        // 16-byte pieces of a row per lane
 constexpr int kQkvMaxHidden = 4096;  // 64 lanes x kQkvPieces x 8 elements
+static_assert(kQkvMaxHidden / 8 <= 64 * kQkvWaves, "a piece of each row of x per thread");
 
 struct QkvArgs {
   const uint16_t* x;     // [B, hidden] bf16
@@ -54,25 +57,38 @@ __device__ __forceinline__ uint4 load_streaming(const uint4* p) {
 
 // kQkvRows: rows of W per wavefront (two or three, whichever spreads the rows more evenly
 // over the CUs).
-template <int B, int kQkvRows>
+// FULL: rows of W have kQkvMaxHidden elements, a piece for every lane and j.
+template <int B, int kQkvRows, bool FULL>
 __global__ __launch_bounds__(64 * kQkvWaves) void qkv_store_kernel(QkvArgs a) {
   extern __shared__ uint4 lds_x[];  // [B][hidden / 8]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kvec = a.hidden >> 3;  // 16-byte pieces per row
   const int n0 = (blockIdx.x * kQkvWaves + wave) * kQkvRows;
 
-  // The wavefront's rows first: they do not depend on the copy of x.
+  // x first, then the wavefront's rows, piece by piece: loads return in order, so that x can be
+  // staged while the rows are still travelling, and the products below take the pieces in the
+  // order in which they come.  (With x asked for last and the rows one after the other the
+  // products, 4 us with eight rows of x, began when the whole stream was through.)  No load
+  // sits behind a branch: where one joins the compiler waits for every load under way.
+  u32x4_t xr[B];  // (kvec is at most the workgroup's size)
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    xr[i] = ((const u32x4_t*)a.x)[min(tid + i * 64 * kQkvWaves, B * kvec - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
   uint4 wv[kQkvRows][kQkvPieces];
 #pragma unroll
-  for (int r = 0; r < kQkvRows; ++r) {
-    const uint4* row = (const uint4*)(a.w + (size_t)min(n0 + r, a.n_out - 1) * a.hidden);
+  for (int j = 0; j < kQkvPieces; ++j) {
+    const int v = min(lane + 64 * j, kvec - 1);
 #pragma unroll
-    for (int j = 0; j < kQkvPieces; ++j) {
-      const int v = lane + 64 * j;
-      wv[r][j] = v < kvec ? load_streaming(row + v) : make_uint4(0u, 0u, 0u, 0u);
-    }
+    for (int r = 0; r < kQkvRows; ++r)
+      wv[r][j] = load_streaming((const uint4*)(a.w + (size_t)min(n0 + r, a.n_out - 1) * a.hidden) + v);
   }
-  for (int i = tid; i < B * kvec; i += 64 * kQkvWaves) lds_x[i] = ((const uint4*)a.x)[i];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    ((u32x4_t*)lds_x)[min(tid + i * 64 * kQkvWaves, B * kvec - 1)] = xr[i];  // (past the end: the last piece again)
+  }
   __syncthreads();
 
   float acc[kQkvRows][B];
@@ -84,7 +100,18 @@ __global__ __launch_bounds__(64 * kQkvWaves) void qkv_store_kernel(QkvArgs a) {
   // stay packed as they were loaded, nothing is unpacked.
 #pragma unroll
   for (int j = 0; j < kQkvPieces; ++j) {
-    const int v = min(lane + 64 * j, kvec - 1);  // past the row: W piece is zero
+    const int v = min(lane + 64 * j, kvec - 1);
+    if (!FULL) {  // past the row: the piece of W is zero
+      const uint32_t keep = lane + 64 * j < kvec ? 0xffffffffu : 0u;
+#pragma unroll
+      for (int r = 0; r < kQkvRows; ++r) {
+        wv[r][j].x &= keep;
+        wv[r][j].y &= keep;
+        wv[r][j].z &= keep;
+        wv[r][j].w &= keep;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const uint4 xv = lds_x[b * kvec + v];
@@ -187,6 +214,8 @@ static int launch_qkv(const QkvArgs& a, hipStream_t stream) {
   // The kernel is one burst of loads per wavefront, and the slowest CU decides: 6144 rows
   // (Llama-3-8B) in 16-row workgroups are 384 workgroups, one and a half per CU, 16.3 us;
   // in 24-row workgroups 256, one per CU, 14.5 us; in 32-row workgroups 192: 16.8 us.
+  // (Measured before the loads were put in the order of their use, which took eight rows of x
+  // from 17.4 to 15.2 us; 50 MB of W are 9 to 10 us at the rate of a large copy.)
   static thread_local int cus_of[64] = {};  // by device, asked once per thread
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) {
@@ -200,13 +229,19 @@ static int launch_qkv(const QkvArgs& a, hipStream_t stream) {
     cus = 256;
   }
   auto rounds = [&](int rows) { return ceil_div(ceil_div(a.n_out, rows * kQkvWaves), cus) * rows; };
-  if (rounds(3) < rounds(2)) {
-    hipLaunchKernelGGL((qkv_store_kernel<B, 3>), dim3((unsigned)ceil_div(a.n_out, 3 * kQkvWaves)),
-                       dim3(64 * kQkvWaves), lds, stream, a);
-  } else {
-    hipLaunchKernelGGL((qkv_store_kernel<B, 2>), dim3((unsigned)ceil_div(a.n_out, 2 * kQkvWaves)),
-                       dim3(64 * kQkvWaves), lds, stream, a);
-  }
+  const bool full = a.hidden == kQkvMaxHidden;
+  auto launch = [&](auto rows) {
+    constexpr int R = decltype(rows)::value;
+    const dim3 grid((unsigned)ceil_div(a.n_out, R * kQkvWaves)), block(64 * kQkvWaves);
+    if (full)
+      hipLaunchKernelGGL((qkv_store_kernel<B, R, true>), grid, block, lds, stream, a);
+    else
+      hipLaunchKernelGGL((qkv_store_kernel<B, R, false>), grid, block, lds, stream, a);
+  };
+  if (rounds(3) < rounds(2))
+    launch(std::integral_constant<int, 3>{});
+  else
+    launch(std::integral_constant<int, 2>{});
   return check_launch("qkv_store_kernel");
 }
 
