@@ -37,9 +37,9 @@ __global__ __launch_bounds__(LIST ? kListThreads : 256) void kv_store_kernel(
   const int len = seq_lens[b];
   int32_t* const tab = table + (int64_t)b * table_stride;
   int32_t ahead[kListAhead];
-  int64_t known = 0;  // entries that are there to be read, whatever the length
+  int known = 0;  // entries that are there to be read, whatever the length: a table holds max_tokens
   if (LIST) {
-    known = min((int64_t)list.max_seq_len, table_stride);
+    known = min(list.max_seq_len, max_tokens);
 #pragma unroll
     for (int i = 0; i < kListAhead; ++i) {
       const int pos = first + i * kListThreads;
