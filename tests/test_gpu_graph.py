@@ -4,11 +4,14 @@ kernels too), so a captured call replays with new queries, new lengths and new t
 contents in the same buffers.  Every replay is checked against an eager call of a second
 layer object on the same inputs, with eager work and synchronisations in between."""
 
+import ctypes
+import dataclasses
+
 import pytest
 import torch
 
 from helpers import say
-from tokenselect_amd import ops, workloads
+from tokenselect_amd import _lib, ops, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -27,7 +30,7 @@ def _capture(layer, q, k_pool, v_pool, bt):
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):  # the first calls load code objects and size the grids
         for _ in range(2):
-            layer(q, k_pool, v_pool, bt)
+            layer(q, k_pool, v_pool, dataclasses.replace(bt, workspace_clean=False))
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
@@ -71,3 +74,93 @@ def test_decode_layer_replays_in_a_graph(dev, fused_select, pool_kernel):
         assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16)), f"replay {replay}: out"
     # and the replays moved with their inputs: the last lengths are the shortened ones
     assert sel_len.tolist() == [16 + 256 + 32, 100, 16 + 200 + 32, 16 + 256 + 32]
+
+
+@pytest.fixture
+def stated(monkeypatch):
+    """The layer calls reach a function that notes what they state of the workspace and launches
+    nothing."""
+    lib, flags = _lib.load(), []
+
+    def note(cfg, bt, *rest):
+        flags.append(bt.contents.workspace_clean)
+        return _lib.TS_OK
+
+    restype, argtypes = _lib.SIGNATURES["ts_decode_layer"]
+    layer = ctypes.CFUNCTYPE(restype, *argtypes)(note)
+    names = ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step", "ts_decode_layer_layout")
+    real = [ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names]
+    bind = _lib.binding()
+    bind.connect(ctypes.cast(layer, ctypes.c_void_p).value, *real[1:])
+    yield flags
+    bind.connect(*real)
+
+
+def test_no_call_vouches_for_a_workspace_that_a_graph_uses(dev, stated):
+    """What the object says of its workspace: nothing in a captured call, whatever ran before it,
+    and nothing after one, since the object does not see the replays.  The caller may."""
+    wl = workloads.build("small", SHAPE, [2048, 901], [256, 256], 16, dev, 63, n_init=16, n_local=32, top_k=256)
+    bt = wl.batch
+    longer = dataclasses.replace(bt, max_seq_len=bt.max_seq_len - 1)   # (of the same layout)
+    some = torch.zeros(8, device=dev)
+
+    def capture(layer, b, call=True):
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            some.add_(1)
+            if call:
+                layer(wl.q, wl.k_pool, wl.v_pool, b)
+            else:
+                layer._clean_for = None   # (what votes() and attend() do)
+
+    for call in (True, False):
+        layer = ops.DecodeLayer(wl.cfg, 2, 2048, dev)
+        del stated[:]
+        for b in (longer, longer, bt):
+            layer(wl.q, wl.k_pool, wl.v_pool, b)
+        assert stated == [0, 1, 1] and layer._clean_for == (2, 2048)
+        del stated[:]
+        capture(layer, bt, call)
+        for _ in range(3):
+            layer(wl.q, wl.k_pool, wl.v_pool, bt)
+        assert stated == ([0] if call else []) + [0, 0, 0] and layer._clean_for is None
+        layer(wl.q, wl.k_pool, wl.v_pool, dataclasses.replace(bt, workspace_clean=True))
+        assert stated[-1] == 1
+
+
+@pytest.mark.parametrize("said", [False, True], ids=["full", "caller says clean"])
+def test_replays_and_eager_steps_share_a_workspace(dev, said):
+    """A captured step and eager steps of two other shapes on one object, in turn; where the
+    caller says that the captured call finds its counters clean, only calls of its layout run
+    between the replays."""
+    say(f"replays and eager steps in turn: said={said}")
+    wl = workloads.build("small", SHAPE, [5000, 100, 2048, 901], [256] * 4, 16, dev, 64, n_init=16, n_local=32,
+                         top_k=256)
+    bt, q = wl.batch, wl.q.clone()
+    steps = [bt, dataclasses.replace(bt, max_seq_len=5001)]
+    if not said:
+        pair = ops.Batch(bt.seq_lens[2:], bt.table[2:].contiguous(), 2048)
+        steps += [pair, pair, bt]
+    layer = ops.DecodeLayer(wl.cfg, 4, 5001, dev)
+    layout = {_lib.load().ts_decode_layer_layout(ctypes.byref(layer._c), 4, n) for n in (5000, 5001)}
+    assert len(layout) == 1
+
+    def check(got, b):
+        fresh = ops.DecodeLayer(wl.cfg, 4, 5001, dev)
+        want = fresh(q if b.batch == 4 else q[2:].contiguous(), wl.k_pool, wl.v_pool, b)
+        torch.cuda.synchronize()
+        layer.check()
+        assert torch.equal(got[3], want[3])
+        for r in range(b.batch):
+            S = int(want[3][r])
+            assert torch.equal(got[1][r, :S], want[1][r, :S]) and torch.equal(got[2][r, :S], want[2][r, :S])
+        assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16))
+
+    graph, outputs = _capture(layer, q, wl.k_pool, wl.v_pool, dataclasses.replace(bt, workspace_clean=said))
+    gen = torch.Generator(device=dev).manual_seed(65)
+    for replay in range(4):
+        q.copy_(torch.randn(q.shape, device=dev, generator=gen).to(q.dtype))
+        graph.replay()
+        check([t.clone() for t in outputs], bt)
+        for b in steps:
+            mine = q if b.batch == 4 else q[2:].contiguous()
+            check([t.clone() for t in layer(mine, wl.k_pool, wl.v_pool, b)], b)

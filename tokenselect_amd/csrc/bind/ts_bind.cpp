@@ -148,6 +148,10 @@ struct Owned {
   // (batch, max_seq_len) that the selection's counters in the workspace are clean for, -1: none.
   int64_t clean_batch = -1, clean_len = -1;
   int64_t clean_layout = -1;  // ts_decode_layer_layout of that call
+  // A call on this workspace was recorded into a graph: a replay, which the object does not
+  // see, may have used it since any call it remembers.  From then on nothing is remembered.
+  bool captured = false;
+  void forget_clean() { clean_batch = clean_len = clean_layout = -1; }
   // The outputs' first rows, for the last batch size: out, sel, sel_pos, sel_len.
   int64_t views_of = -1;
   PyObject* views[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -283,6 +287,16 @@ Rows rows_of(PyObject* obj, const char* name, int64_t from, int64_t count, int64
   return Rows{at, width, std::move(c)};
 }
 
+// Whether what is launched on the current stream is recorded into a graph instead of run.
+bool capturing() {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &status) != hipSuccess) {
+    (void)hipGetLastError();  // (the legacy stream beside a capture on another one)
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 PyObject* row_view(const at::Tensor& t, int64_t B) {
   PyObject* v = THPVariable_Wrap(t.narrow(0, 0, B));
   if (!v) throw Raised{};
@@ -295,14 +309,18 @@ int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int
                  const at::Tensor& v_pool, const ts_selcache* cache, void* out, bool rerun = false) {
   // The attention kernel of a plain call leaves the selection's counters zero for the next
   // one of the same shape.
-  const bool chunk = o.max_rows > 0, plain = !chunk && !cache && !bt->separate_kernels && !rerun;
+  const bool chunk = o.max_rows > 0;
+  // (While a graph is captured the object states nothing: the recorded flag would hold for
+  // every replay, whatever used the workspace before it.)
+  if (!chunk && !o.captured) o.captured = capturing();
+  const bool plain = !chunk && !cache && !bt->separate_kernels && !rerun && !o.captured;
   // (By the layout and not by the length, which grows with every token: it is the same for
   // some 64 steps, and each of them starts with the selection instead of with a launch that
   // rotates and clears: 2 layers of a 128K request, two steps, 296 -> 292 us; a 31599-token
   // prompt with 16 tokens 4615 -> 4513.)
   const int64_t layout = plain ? decode_layer_layout(&o.cfg, bt->batch, bt->max_seq_len) : -1;
   if (layout >= 0 && o.clean_batch == bt->batch && o.clean_layout == layout) bt->workspace_clean = 1;
-  o.clean_batch = o.clean_len = o.clean_layout = -1;
+  o.forget_clean();
   const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
   const float *cos = (const float*)o.cos.data_ptr(), *sin = (const float*)o.sin.data_ptr();
   int32_t *sel = (int32_t*)o.sel.data_ptr(), *sel_pos = (int32_t*)o.sel_pos.data_ptr(),
@@ -552,6 +570,11 @@ int set_clean(PyObject* self, PyObject* value, void*) {
   Owned& o = *((Runner*)self)->own;
   long long b = -1, n = -1;
   if (value != Py_None && !(value && PyArg_ParseTuple(value, "LL", &b, &n))) return -1;
+  if (value == Py_None) {  // other calls use the workspace from here on
+    o.captured = o.captured || capturing();
+    o.forget_clean();
+    return 0;
+  }
   o.clean_batch = b;
   o.clean_len = n;
   o.clean_layout = b >= 1 && n >= 1 ? decode_layer_layout(&o.cfg, (int32_t)b, (int32_t)n) : -1;

@@ -82,7 +82,8 @@ class Batch:
     wait_us: int = 0
     absent_workgroups: int = 0
     # ``ts_batch.workspace_clean``: the workspace was left by a completed call of the same
-    # shape without a selection cache (set by :class:`DecodeLayer`, which knows).
+    # shape without a selection cache.  :class:`DecodeLayer` states it by itself where it
+    # knows; never in a call that is captured into a graph, where only the caller can.
     workspace_clean: bool = False
 
     @property
@@ -766,7 +767,10 @@ class DecodeLayer(_GiveUpLatch):
         """(batch, max_seq_len) of the last call when it was a plain layer call without a
         selection cache that raised nothing: that call's attention kernel has left the
         selection's counters zero, and the next call of the same shape says so
-        (``ts_batch.workspace_clean``) and starts with the selection kernel."""
+        (``ts_batch.workspace_clean``) and starts with the selection kernel.  ``None`` for
+        good once a call of this object was captured into a graph, whose replays use the
+        workspace without its knowledge; a caller who knows what uses the workspace between
+        the replays sets ``Batch.workspace_clean``."""
         return self._native.clean
 
     @_clean_for.setter
