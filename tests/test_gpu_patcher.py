@@ -348,3 +348,52 @@ def test_fused_projection_rows_are_read_where_they_lie(dev):
                 assert torch.equal(a, b), f"pad {pad}, output {i}"
     finally:
         tr.PREFILL_CHUNK_SIZE = 512
+
+
+def _requests(dev, rows, like=lambda x: x, chunk=32):
+    """Prompts of one row, one chunk and a ragged third chunk with a decode step each, then the
+    three decoded together: the outputs and the pools.  `like` makes the slots of a call."""
+    H, Hkv, D = 8, 2, 128
+    tr.patch(rope_base=1e4, rope_scale=1, rope_model="ROPE_LLAMA", max_n_tokens=256, top_k=24, n_init=4, n_local=16)
+    tr.PREFILL_CHUNK_SIZE = chunk
+    try:
+        g = torch.Generator(device=dev).manual_seed(rows)
+        slots = torch.randperm(512, generator=g, device=dev).to(torch.int32)
+        pool = sg.TokenToKVPool(512, torch.bfloat16, Hkv, D, 1, dev)
+        owner = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool,
+                               dtype=torch.bfloat16).req_to_token_retriever
+        attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
+        got, used, singles = [], 0, []
+
+        def forward(mode, retriever, n):
+            nonlocal used
+            q, k, v = (torch.randn(n, h * D, generator=g, device=dev).bfloat16() for h in (H, Hkv, Hkv))
+            meta = sg.InputMetadata(mode, retriever, pool, like(slots[used:used + n]))
+            used += n
+            got.append(attn.forward(q, k, v, meta))
+
+        for n in (1, chunk, rows):
+            singles.append(owner.new_token_retriever())
+            forward(sg.ForwardMode.EXTEND, singles[-1], n)
+            forward(sg.ForwardMode.DECODE, singles[-1], 1)
+        batch = owner.get_batch_token_retriever(("a", "b", "c"), singles)
+        for _ in range(2):
+            forward(sg.ForwardMode.DECODE, batch, 3)
+        return got + [pool.k_buffer[0], pool.v_buffer[0]]
+    finally:
+        tr.PREFILL_CHUNK_SIZE = 512
+
+
+@pytest.mark.parametrize("stride", [2, 3])
+def test_slots_of_any_stride(dev, stride):
+    """out_cache_loc as a column of a larger tensor: the results are those of the same slots made
+    contiguous."""
+    say(f"out_cache_loc with stride {stride}")
+
+    def spread(loc):
+        wide = torch.full((loc.shape[0], stride), -1, dtype=torch.int32, device=dev)
+        wide[:, 1] = loc
+        return wide[:, 1]
+
+    for a, b in zip(_requests(dev, 77), _requests(dev, 77, spread)):
+        assert torch.equal(a, b)

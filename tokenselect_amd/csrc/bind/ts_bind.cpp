@@ -287,6 +287,18 @@ Rows rows_of(PyObject* obj, const char* name, int64_t from, int64_t count, int64
   return Rows{at, width, std::move(c)};
 }
 
+// The slots of rows [from, from + count), next to each other: a part of a strided tensor is
+// copied together.
+Rows slots_of(PyObject* obj, int64_t from, int64_t count) {
+  const at::Tensor& t = tensor(obj, "out_cache_loc");
+  if (t.scalar_type() != at::kInt || !t.is_cuda() || t.dim() != 1) need(obj, "out_cache_loc", at::kInt, 1);  // (raises)
+  if (t.size(0) < from + count) bad_value("out_cache_loc does not match the rows");
+  if (t.is_contiguous()) return Rows{(const int32_t*)t.data_ptr() + from, 1, std::nullopt};
+  at::Tensor c = t.narrow(0, from, count).contiguous();
+  const void* at = c.data_ptr();
+  return Rows{at, 1, std::move(c)};
+}
+
 // Whether what is launched on the current stream is recorded into a graph instead of run.
 bool capturing() {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -474,9 +486,8 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor& v_pool = check_pool(cfg, args[5], "v_pool");
   if (k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
   if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
-  const at::Tensor& loc = need(args[3], "out_cache_loc", at::kInt, 1);
-  if (loc.size(0) < from + rows) bad_value("out_cache_loc does not match the rows");
-  ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.data_ptr() + from, nullptr,
+  const Rows loc = slots_of(args[3], from, rows);
+  ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.ptr, nullptr,
                (int32_t)call.table_tokens, (int32_t)k.stride};
   ts_selcache cache{};
   const bool cached = args[7] != Py_None;
