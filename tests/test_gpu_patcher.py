@@ -397,3 +397,24 @@ def test_slots_of_any_stride(dev, stride):
 
     for a, b in zip(_requests(dev, 77), _requests(dev, 77, spread)):
         assert torch.equal(a, b)
+
+
+def test_rows_of_k_and_v_match_the_step(dev):
+    """A decode step whose k or v has another number of rows than there are requests is refused,
+    and stores nothing."""
+    say("decode step with too many rows of k / v")
+    H, Hkv, D = 8, 2, 128
+    tr.patch(rope_base=1e4, rope_scale=1, rope_model="ROPE_LLAMA", max_n_tokens=64, top_k=24, n_init=4, n_local=16)
+    pool = sg.TokenToKVPool(64, torch.bfloat16, Hkv, D, 1, dev)
+    retriever = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool,
+                               dtype=torch.bfloat16).req_to_token_retriever.get_token_retriever("a")
+    attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
+    meta = sg.InputMetadata(sg.ForwardMode.DECODE, retriever, pool, torch.tensor([3], dtype=torch.int32, device=dev))
+    q = torch.ones(1, H * D, dtype=torch.bfloat16, device=dev)
+    rows = {n: torch.ones(n, Hkv * D, dtype=torch.bfloat16, device=dev) for n in (1, 2)}
+    for nk, nv in ((2, 2), (2, 1), (1, 2)):
+        with pytest.raises(ValueError):
+            attn.forward(q, rows[nk], rows[nv], meta)
+    assert retriever.num_tokens == [0] and not pool.k_buffer[0].any() and not pool.v_buffer[0].any()
+    attn.forward(q, rows[1], rows[1], meta)
+    assert retriever.num_tokens == [1] and bool((pool.k_buffer[0][3] == 1).all())

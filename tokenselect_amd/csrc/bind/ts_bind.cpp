@@ -475,6 +475,9 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
     if (bt.batch != 1 || rows > o.max_rows) bad_value("one request, within the sizes this PrefillChunk was built for");
     if (from < 0 || rows < 1) bad_value("a chunk has at least one row");
   }
+  // (a prompt's k and v may have rows after those of q, which are not read)
+  if (!chunk && (tensor(args[1], "k").numel() != rows * row || tensor(args[2], "v").numel() != rows * row))
+    bad_value("k / v do not match the batch");
   const Rows q = rows_of(args[0], "q", from, rows, width, false);
   Rows k = rows_of(args[1], "k", from, rows, row, false), v = rows_of(args[2], "v", from, rows, row, false);
   if (k.stride != v.stride) {
