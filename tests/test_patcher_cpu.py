@@ -116,6 +116,50 @@ def test_forward_dispatch_and_unsupported_modes():
         attn.forward(q, torch.zeros(1, 256, dtype=torch.bfloat16), None, meta)
 
 
+@pytest.mark.parametrize("how", ["subclass", "object", "class"])
+def test_replaced_retriever_methods_are_called(monkeypatch, how):
+    """A retriever whose attention or store somebody has replaced: the patched forwards store and
+    call the replacements, and no step in one library call goes past them."""
+    req, pool = make_retriever()
+    monkeypatch.setattr(tr.ops, "kv_store", lambda *a, **k: None)
+    monkeypatch.setattr(tr.ops, "kv_store_chunk", lambda *a, **k: None)
+    calls = []
+
+    def attention(name):
+        def replacement(self, attn, q, *rest):
+            calls.append(name)
+            return torch.zeros_like(q)
+        return replacement
+
+    def replaced(retriever, names):
+        if how == "object":
+            for n in names:
+                monkeypatch.setattr(retriever, n, attention(n).__get__(retriever))
+        elif how == "class":
+            for n in names:
+                monkeypatch.setattr(type(retriever), n, attention(n))
+        else:
+            retriever.__class__ = type("Mine", (type(retriever),), {n: attention(n) for n in names})
+        return retriever
+
+    attn = sg.RadixAttention(4, 128, 128 ** -0.5, 2, layer_id=0)
+
+    def forward(mode, retriever, rows):
+        del calls[:]
+        q, k, v = (torch.zeros(rows, n * 128, dtype=torch.bfloat16) for n in (4, 2, 2))
+        out = attn.forward(q, k, v, sg.InputMetadata(mode, retriever, pool, torch.arange(rows, dtype=torch.int32)))
+        assert out.shape == q.shape
+        return calls
+
+    r = replaced(req.new_token_retriever(), ("decode_attention", "prefill_attention"))
+    assert forward(sg.ForwardMode.EXTEND, r, 3) == ["prefill_attention"]
+    assert forward(sg.ForwardMode.DECODE, r, 1) == ["decode_attention"] and r.num_tokens[0] == 4
+    batch = replaced(tr.BatchTokenRetriever([r, req.new_token_retriever()], pool), ("decode_attention",))
+    assert forward(sg.ForwardMode.DECODE, batch, 2) == ["decode_attention"] and batch.num_tokens[0] == [5, 1]
+    batch = replaced(batch, ("store", "decode_attention"))
+    assert forward(sg.ForwardMode.DECODE, batch, 2) == ["store", "decode_attention"]
+
+
 def test_rotary_tables_follow_the_reference_expressions():
     rot = tr.RotaryEmbedding(128, 5e5, 1.0, device="cpu")
     rot._update_cos_sin_tables(600)
