@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define TS_VERSION 101
+#define TS_VERSION 102
 
 #define TS_OK 0
 #define TS_EINVAL (-1)     /* null pointer or scalar out of range            */
@@ -142,9 +142,6 @@ typedef struct ts_batch {
                                where the selection is the single ts_select launch and no
                                selection cache is used; ignored otherwise.  A wrong
                                statement gives wrong selections or waits that give up */
-  int32_t q_row_stride;     /* layer, chunk and step calls: elements between the query
-                               rows (>= H*D, a multiple of 8), 0 = H*D: the query part
-                               of a fused QKV projection is read where it lies          */
 } ts_batch;
 
 /* Default bound of a grid-wide wait: a selection that has the device to itself
@@ -408,14 +405,22 @@ typedef struct ts_new_kv {
   const int32_t* out_cache_loc;  /* [batch] slots, or NULL with pages */
   const ts_page_pool* pages;     /* or NULL */
   int32_t max_tokens;            /* as for ts_kv_store */
-  int32_t row_stride;            /* elements between rows of k, and of v (>= Hkv*D, a
-                                    multiple of 8), 0 = Hkv*D */
 } ts_new_kv;
 int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
                    const float* q_cos, const float* q_sin, void* k_pool, void* v_pool,
                    int64_t pool_rows, const ts_selcache* cache, void* out, int32_t* sel,
                    int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
                    size_t workspace_bytes, ts_stream_t stream);
+
+/* ts_decode_step with rows that lie further apart than they are long, as a split of a fused
+ * QKV projection leaves them: elements between the rows of q (>= H*D), and between those of
+ * k and of v (>= Hkv*D), multiples of 8; 0 = next to each other. */
+int ts_decode_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                           int32_t q_row_stride, int32_t kv_row_stride, const float* q_cos,
+                           const float* q_sin, void* k_pool, void* v_pool, int64_t pool_rows,
+                           const ts_selcache* cache, void* out, int32_t* sel, int32_t* sel_pos,
+                           int64_t sel_stride, int32_t* sel_len, void* workspace,
+                           size_t workspace_bytes, ts_stream_t stream);
 
 /* The QKV projection of a decode step with the KV store as its epilogue: what the
  * serving stack does in two places, qkv = x W^T (+ bias) in the model's attention
@@ -508,6 +513,13 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
                     void* k_pool, void* v_pool, int64_t pool_rows, void* out, int32_t* sel,
                     int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
                     size_t workspace_bytes, ts_stream_t stream);
+/* ts_prefill_step with row strides, as for ts_decode_step_strided. */
+int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                            int32_t q_row_stride, int32_t kv_row_stride, int32_t rows,
+                            const float* cos_table, const float* sin_table, int64_t table_rows,
+                            void* k_pool, void* v_pool, int64_t pool_rows, void* out, int32_t* sel,
+                            int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
+                            size_t workspace_bytes, ts_stream_t stream);
 
 /* One layer of patched_radix_attention_decode_forward_flashinfer after the KV
  * store (tr.py:791-825): fingerprint (q rotated with q_cos/q_sin, the [D] table

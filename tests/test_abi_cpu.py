@@ -57,6 +57,45 @@ def test_struct_layouts_match_the_header():
     assert ctypes.sizeof(_lib.TsNewKv) == 4 * 8 + 8 and _lib.TsNewKv.max_tokens.offset == 32
 
 
+def test_padding_of_the_structs_is_not_read(lib):
+    """ts_batch and ts_new_kv end in four bytes of padding, in which a caller may leave anything:
+    what is reported is what is wrong with the call (here its workspace)."""
+    c, one = cfg(), ctypes.c_void_p(0x1000)  # never dereferenced: validation fails first
+
+    def padded(struct):
+        raw = bytearray(struct)
+        assert len(raw) == ctypes.sizeof(struct) and not any(raw[-4:])
+        raw[-4:] = (12345).to_bytes(4, "little")
+        return type(struct).from_buffer(raw)
+
+    bt = padded(_lib.TsBatch(1, 4096, one, one, 4096, None))
+    kv = padded(_lib.TsNewKv(one, one, one, None, 4096))
+    cache = _lib.TsSelCache(one, one, one, one, 0.9)
+    tail = (one, one, one, 4096, one, one, 64, None)
+    assert lib.ts_decode_layer(ctypes.byref(c), ctypes.byref(bt), one, one, one, one, one, 10, None,
+                               *tail) == _lib.TS_EWORKSPACE, err(lib)
+    assert lib.ts_decode_step(ctypes.byref(c), ctypes.byref(bt), ctypes.byref(kv), one, one, one, one, one, 10,
+                              ctypes.byref(cache), *tail) == _lib.TS_EWORKSPACE, err(lib)
+    assert lib.ts_prefill_step(ctypes.byref(c), ctypes.byref(bt), ctypes.byref(kv), one, 8, one, one, 4096, one, one,
+                               10, *tail) == _lib.TS_EWORKSPACE, err(lib)
+
+
+def test_row_strides_are_checked_before_anything_is_launched(lib):
+    """The strided steps: rows at least as far apart as they are long, in whole 16-byte pieces."""
+    c, one = cfg(), ctypes.c_void_p(0x1000)
+    bt = _lib.TsBatch(1, 4096, one, one, 4096, None)
+    kv = _lib.TsNewKv(one, one, one, None, 4096)
+    cache = _lib.TsSelCache(one, one, one, one, 0.9)
+    tail = (one, one, one, 4096, one, one, 64, None)
+    for q, rows, code in ((0, 0, _lib.TS_EWORKSPACE), (6144, 6144, _lib.TS_EWORKSPACE), (4096, 1024, _lib.TS_EWORKSPACE),
+                          (4088, 1024, _lib.TS_EINVAL), (4100, 1024, _lib.TS_EINVAL), (-4096, 1024, _lib.TS_EINVAL),
+                          (4096, 1016, _lib.TS_EINVAL), (4096, 1028, _lib.TS_EINVAL)):
+        assert lib.ts_decode_step_strided(ctypes.byref(c), ctypes.byref(bt), ctypes.byref(kv), one, q, rows, one, one,
+                                          one, one, 10, ctypes.byref(cache), *tail) == code, (q, rows, err(lib))
+        assert lib.ts_prefill_step_strided(ctypes.byref(c), ctypes.byref(bt), ctypes.byref(kv), one, q, rows, 8, one,
+                                           one, 4096, one, one, 10, *tail) == code, (q, rows, err(lib))
+
+
 def test_config_validation(lib):
     assert lib.ts_check_config(ctypes.byref(cfg())) == _lib.TS_OK
     assert lib.ts_check_config(None) == _lib.TS_EINVAL
@@ -220,21 +259,27 @@ def test_header_is_plain_c_and_agrees_with_the_ctypes_mirror(tmp_path):
     gcc = shutil.which("gcc")
     if gcc is None:
         pytest.skip("no C compiler")
+    include = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include")
+    # The mirror has the header's fields, all of them and in their order.
+    header = re.sub(r"/\*.*?\*/", "", open(os.path.join(include, "tokenselect.h")).read(), flags=re.S)
+    mirrors = {"ts_config": _lib.TsConfig, "ts_batch": _lib.TsBatch, "ts_selcache": _lib.TsSelCache,
+               "ts_page_pool": _lib.TsPagePool, "ts_new_kv": _lib.TsNewKv}
+    structs = dict(re.findall(r"typedef struct (\w+) \{(.*?)\}", header, flags=re.S))
+    assert set(structs) == set(mirrors)
+    for name, mirror in mirrors.items():
+        assert re.findall(r"(\w+)\s*;", structs[name]) == [f[0] for f in mirror._fields_], name
     src = tmp_path / "layout.c"
     src.write_text(
         '#include <stddef.h>\n#include <stdio.h>\n#include "tokenselect.h"\n'
         'int main(void) {\n'
-        '  printf("%zu %zu %zu %zu %zu %zu %zu %zu %zu\\n", sizeof(ts_config), sizeof(ts_batch), sizeof(ts_selcache),\n'
-        '         offsetof(ts_batch, threshold_hint), offsetof(ts_batch, wait_us),\n'
-        '         offsetof(ts_batch, workspace_clean), offsetof(ts_batch, host_seq_lens),\n'
-        '         sizeof(ts_new_kv), offsetof(ts_new_kv, max_tokens));\n'
+        + "".join(f'  printf("%zu\\n", sizeof({name}));\n' + "".join(
+            f'  printf("%zu\\n", offsetof({name}, {field[0]}));\n' for field in mirror._fields_)
+            for name, mirror in mirrors.items()) +
         '  return 0;\n}\n')
     exe = tmp_path / "layout"
-    include = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include")
     subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-Werror", "-pedantic", "-I", include, str(src),
                     "-o", str(exe)], check=True)
     got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
-    assert got == [ctypes.sizeof(_lib.TsConfig), ctypes.sizeof(_lib.TsBatch), ctypes.sizeof(_lib.TsSelCache),
-                   _lib.TsBatch.threshold_hint.offset, _lib.TsBatch.wait_us.offset,
-                   _lib.TsBatch.workspace_clean.offset, _lib.TsBatch.host_seq_lens.offset,
-                   ctypes.sizeof(_lib.TsNewKv), _lib.TsNewKv.max_tokens.offset]
+    want = [n for mirror in mirrors.values() for n in
+            (ctypes.sizeof(mirror), *(getattr(mirror, field[0]).offset for field in mirror._fields_))]
+    assert got == want

@@ -88,7 +88,8 @@ def stated(monkeypatch):
 
     restype, argtypes = _lib.SIGNATURES["ts_decode_layer"]
     layer = ctypes.CFUNCTYPE(restype, *argtypes)(note)
-    names = ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step", "ts_decode_layer_layout")
+    names = ("ts_decode_layer", "ts_decode_step_strided", "ts_prefill_chunk", "ts_prefill_step_strided",
+             "ts_decode_layer_layout")
     real = [ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names]
     bind = _lib.binding()
     bind.connect(ctypes.cast(layer, ctypes.c_void_p).value, *real[1:])

@@ -37,7 +37,7 @@ class TsBatch(ctypes.Structure):
         ("batch", _i32), ("max_seq_len", _i32), ("seq_lens", _ptr), ("table", _ptr),
         ("table_stride", _i64), ("k_per_req", _ptr), ("fault", _ptr), ("host_seq_lens", _ptr),
         ("threshold_hint", _ptr), ("separate_kernels", _i32), ("rerun", _i32), ("wait_us", ctypes.c_uint32),
-        ("absent_workgroups", _i32), ("workspace_clean", _i32), ("q_row_stride", _i32),
+        ("absent_workgroups", _i32), ("workspace_clean", _i32),
     ]
 
 
@@ -54,7 +54,7 @@ class TsPagePool(ctypes.Structure):
 
 class TsNewKv(ctypes.Structure):
     _fields_ = [("k", _ptr), ("v", _ptr), ("out_cache_loc", _ptr), ("pages", ctypes.POINTER(TsPagePool)),
-                ("max_tokens", _i32), ("row_stride", _i32)]
+                ("max_tokens", _i32)]
 
 
 _CFG, _BT, _SC = ctypes.POINTER(TsConfig), ctypes.POINTER(TsBatch), ctypes.POINTER(TsSelCache)
@@ -107,6 +107,8 @@ SIGNATURES = {
                                 _ptr, _i64, _ptr, _ptr, _size, _ptr]),
     "ts_prefill_step": (_i32, [_CFG, _BT, _KV, _ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _ptr,
                                _ptr, _i64, _ptr, _ptr, _size, _ptr]),
+    "ts_prefill_step_strided": (_i32, [_CFG, _BT, _KV, _ptr, _i32, _i32, _i32, _ptr, _ptr, _i64, _ptr, _ptr,
+                                       _i64, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _size, _ptr]),
     "ts_set_fused_select": (_i32, [_i32]),
     "ts_decode_layer_selection": (_i32, [_CFG, _i32, _i32]),
     "ts_decode_layer_selection_of": (_i32, [_CFG, _BT]),
@@ -120,6 +122,8 @@ SIGNATURES = {
                                _ptr, _i64, _ptr, _ptr, _size, _ptr]),
     "ts_decode_step": (_i32, [_CFG, _BT, _KV, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _SC, _ptr, _ptr,
                               _ptr, _i64, _ptr, _ptr, _size, _ptr]),
+    "ts_decode_step_strided": (_i32, [_CFG, _BT, _KV, _ptr, _i32, _i32, _ptr, _ptr, _ptr, _ptr, _i64, _SC,
+                                      _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _size, _ptr]),
 }
 
 _lib = None
@@ -165,7 +169,7 @@ def binding():
             raise ImportError(f"the Python binding next to {LIB_PATH} is missing or does not load ({e}): "
                               "build it with `python -m tokenselect_amd.build`") from e
         _ts_bind.connect(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in
-                           ("ts_decode_layer", "ts_decode_step", "ts_prefill_chunk", "ts_prefill_step",
+                           ("ts_decode_layer", "ts_decode_step_strided", "ts_prefill_chunk", "ts_prefill_step_strided",
                             "ts_decode_layer_layout")))
         _bind = _ts_bind
     return _bind

@@ -121,14 +121,14 @@ bool bool_attr(PyObject* o, PyObject* name) {
   return b != 0;
 }
 
-using StepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, const float*, const float*,
-                       void*, void*, int64_t, const ts_selcache*, void*, int32_t*, int32_t*, int64_t, int32_t*,
+using StepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, int32_t, int32_t,
+                       const float*, const float*, void*, void*, int64_t, const ts_selcache*, void*, int32_t*, int32_t*, int64_t, int32_t*,
                        void*, size_t, ts_stream_t);
 using LayerFn = int (*)(const ts_config*, const ts_batch*, const void*, const float*, const float*, const void*,
                         const void*, int64_t, const ts_selcache*, void*, int32_t*, int32_t*, int64_t, int32_t*,
                         void*, size_t, ts_stream_t);
-using ChunkStepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, int32_t, const float*,
-                            const float*, int64_t, void*, void*, int64_t, void*, int32_t*, int32_t*, int64_t,
+using ChunkStepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, int32_t, int32_t,
+                            int32_t, const float*, const float*, int64_t, void*, void*, int64_t, void*, int32_t*, int32_t*, int64_t,
                             int32_t*, void*, size_t, ts_stream_t);
 using ChunkFn = int (*)(const ts_config*, const ts_batch*, const void*, int32_t, const float*, const float*, int64_t,
                         const void*, const void*, int64_t, void*, int32_t*, int32_t*, int64_t, int32_t*, void*,
@@ -316,9 +316,11 @@ PyObject* row_view(const at::Tensor& t, int64_t B) {
 }
 
 // The library's call on the current stream, with the object's buffers.  kv: the tokens to store
-// first, or NULL.  rows: of the chunk.
-int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int64_t rows, const at::Tensor& k_pool,
-                 const at::Tensor& v_pool, const ts_selcache* cache, void* out, bool rerun = false) {
+// first, or NULL.  q_stride, kv_stride: elements between the rows of a step (0: next to each
+// other).  rows: of the chunk.
+int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int32_t q_stride, int32_t kv_stride,
+                 int64_t rows, const at::Tensor& k_pool, const at::Tensor& v_pool, const ts_selcache* cache, void* out,
+                 bool rerun = false) {
   // The attention kernel of a plain call leaves the selection's counters zero for the next
   // one of the same shape.
   const bool chunk = o.max_rows > 0;
@@ -344,12 +346,12 @@ int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int
   int code;
   Py_BEGIN_ALLOW_THREADS
   if (chunk)
-    code = kv ? prefill_step(cfg, bt, kv, q, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out, sel, sel_pos,
-                             sel_stride, sel_len, ws, ws_bytes, stream)
+    code = kv ? prefill_step(cfg, bt, kv, q, q_stride, kv_stride, (int32_t)rows, cos, sin, table_rows, kp, vp,
+                             pool_rows, out, sel, sel_pos, sel_stride, sel_len, ws, ws_bytes, stream)
               : prefill_chunk(cfg, bt, q, (int32_t)rows, cos, sin, table_rows, kp, vp, pool_rows, out, sel, sel_pos,
                               sel_stride, sel_len, ws, ws_bytes, stream);
   else
-    code = kv ? decode_step(cfg, bt, kv, q, cos, sin, kp, vp, pool_rows, cache, out, sel, sel_pos, sel_stride, sel_len,
+    code = kv ? decode_step(cfg, bt, kv, q, q_stride, kv_stride, cos, sin, kp, vp, pool_rows, cache, out, sel, sel_pos, sel_stride, sel_len,
                             ws, ws_bytes, stream)
               : decode_layer(cfg, bt, q, cos, sin, kp, vp, pool_rows, cache, out, sel, sel_pos, sel_stride, sel_len, ws,
                              ws_bytes, stream);
@@ -448,7 +450,7 @@ PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   }
   const Ref out_ref(out_py);
 
-  const int code = call_library(o, &bt, store ? &kv : nullptr, q.data_ptr(), rows, k_pool, v_pool,
+  const int code = call_library(o, &bt, store ? &kv : nullptr, q.data_ptr(), 0, 0, rows, k_pool, v_pool,
                                 cached ? &cache : nullptr, out_ptr, rerun);
   if (code != TS_OK) return PyLong_FromLong(code);
   return PyTuple_Pack(4, out_py, o.views[1], o.views[2], o.views[3]);
@@ -484,14 +486,13 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
     if (k.stride != row) k = rows_of(args[1], "k", from, rows, row, true);
     if (v.stride != row) v = rows_of(args[2], "v", from, rows, row, true);
   }
-  bt.q_row_stride = (int32_t)q.stride;
   const at::Tensor& k_pool = check_pool(cfg, args[4], "k_pool");
   const at::Tensor& v_pool = check_pool(cfg, args[5], "v_pool");
   if (k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
   if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
   const Rows loc = slots_of(args[3], from, rows);
   ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.ptr, nullptr,
-               (int32_t)call.table_tokens, (int32_t)k.stride};
+               (int32_t)call.table_tokens};
   ts_selcache cache{};
   const bool cached = args[7] != Py_None;
   if (cached) fill_cache(cfg, args[7], bt.batch, &cache);
@@ -503,7 +504,7 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   } else {
     out = at::empty({rows, width}, o.out.options());
   }
-  const int code = call_library(o, &bt, &kv, q.ptr, rows, k_pool, v_pool, cached ? &cache : nullptr,
+  const int code = call_library(o, &bt, &kv, q.ptr, (int32_t)q.stride, (int32_t)k.stride, rows, k_pool, v_pool, cached ? &cache : nullptr,
                                 (char*)out.data_ptr() + 2 * from * width);
   if (code != TS_OK) return PyLong_FromLong(code);
   if (chunk) {

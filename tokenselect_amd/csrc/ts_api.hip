@@ -73,7 +73,6 @@ int validate_batch(const ts_config* cfg, const ts_batch* bt) {
   TS_REQUIRE(bt->batch == 1 || bt->table_stride * (int64_t)cfg->page_size >= bt->max_seq_len,
              TS_EINVAL, "table_stride %lld too small for max_seq_len %d at page_size %d",
              (long long)bt->table_stride, bt->max_seq_len, cfg->page_size);
-  TS_TRY(check_row_stride(bt->q_row_stride, (int64_t)cfg->num_heads * cfg->head_dim, "query"));
   if (bt->host_seq_lens)
     for (int b = 0; b < bt->batch; ++b)
       TS_REQUIRE(bt->host_seq_lens[b] >= 0 && bt->host_seq_lens[b] <= bt->max_seq_len, TS_EINVAL,
@@ -82,9 +81,12 @@ int validate_batch(const ts_config* cfg, const ts_batch* bt) {
   return TS_OK;
 }
 
-// Elements between the query rows of a call.
-static int query_stride(const ts_config* cfg, const ts_batch* bt) {
-  return bt->q_row_stride ? bt->q_row_stride : cfg->num_heads * cfg->head_dim;
+// The configuration, and the elements between the rows of a step's q and of its k and v (0:
+// next to each other), before anything is launched.
+static int check_strides(const ts_config* cfg, int32_t q_row_stride, int32_t kv_row_stride, const char* who) {
+  TS_TRY(validate_config(cfg));
+  TS_TRY(check_row_stride(q_row_stride, (int64_t)cfg->num_heads * cfg->head_dim, who));
+  return check_row_stride(kv_row_stride, (int64_t)cfg->num_kv_heads * cfg->head_dim, who);
 }
 
 int score_tokens_per_block(int64_t total_candidates, int num_heads) {
@@ -259,8 +261,8 @@ static DenseList step_list(const ts_config* cfg, const ts_batch* bt, const ts_se
 
 // Decode (chunk_rows == 0: one query row per request, q_cos / q_sin are the [D] rows
 // of position n_local) or one prefill chunk of a single request (chunk_rows > 0:
-// q_cos / q_sin are the whole [table_rows, D] tables).
-static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, int32_t chunk_rows,
+// q_cos / q_sin are the whole [table_rows, D] tables).  q_row_stride: checked by the caller.
+static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, int32_t q_row_stride, int32_t chunk_rows,
                      const float* q_cos, const float* q_sin, int64_t table_rows,
                      const void* k_pool, const void* v_pool, int64_t pool_rows,
                      const ts_selcache* cache, void* out, int32_t* sel, int32_t* sel_pos,
@@ -278,7 +280,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
              "internal: a chunk's store rides in the fingerprint launch only");
   TS_REQUIRE(pool_rows >= 1 && pool_rows <= 0x7fffffffLL, TS_EINVAL, "pool_rows %lld out of range",
              (long long)pool_rows);
-  const int q_stride = query_stride(cfg, bt);
+  const int q_stride = q_row_stride ? q_row_stride : cfg->num_heads * cfg->head_dim;
   LayerWorkspace w = layer_workspace(cfg, bt->batch, bt->max_seq_len);
   TS_REQUIRE_ALIGNED(workspace, 256, "workspace");
   TS_REQUIRE_ALIGNED(q, 16, "q");
@@ -400,7 +402,7 @@ int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, con
                     int64_t pool_rows, const ts_selcache* cache, void* out, int32_t* sel,
                     int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
                     size_t workspace_bytes, ts_stream_t stream) {
-  return run_layer(cfg, bt, q, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel,
+  return run_layer(cfg, bt, q, 0, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel,
                    sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
 }
 
@@ -409,11 +411,13 @@ int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, con
 // store rides in the layer's first launch (the rotation and the cache decision, whose
 // workgroup of a request stores that request's rows first); otherwise the two calls follow
 // each other.
-int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
-                   const float* q_cos, const float* q_sin, void* k_pool, void* v_pool,
-                   int64_t pool_rows, const ts_selcache* cache, void* out, int32_t* sel,
-                   int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
-                   size_t workspace_bytes, ts_stream_t stream) {
+int ts_decode_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                           int32_t q_row_stride, int32_t kv_row_stride, const float* q_cos,
+                           const float* q_sin, void* k_pool, void* v_pool, int64_t pool_rows,
+                           const ts_selcache* cache, void* out, int32_t* sel, int32_t* sel_pos,
+                           int64_t sel_stride, int32_t* sel_len, void* workspace,
+                           size_t workspace_bytes, ts_stream_t stream) {
+  TS_TRY(check_strides(cfg, q_row_stride, kv_row_stride, "ts_decode_step"));
   TS_REQUIRE(bt != nullptr && kv != nullptr, TS_EINVAL, "ts_decode_step: NULL batch / new K,V");
   TS_REQUIRE(bt->table != nullptr && bt->seq_lens != nullptr, TS_EINVAL, "ts_decode_step: NULL table / seq_lens");
   int32_t* table = const_cast<int32_t*>(bt->table);
@@ -426,15 +430,14 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
       if (kv->pages == nullptr)
         list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
                          workspace_bytes);
-      TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
+      TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
                              pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
                              (hipStream_t)stream, list.sel ? &list : nullptr));
     }
-    return run_layer(cfg, bt, q, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
+    return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
                      sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, list.sel != nullptr);
   }
   // The checks ts_kv_store makes.
-  TS_TRY(validate_config(cfg));
   TS_REQUIRE(kv->k && kv->v && k_pool && v_pool, TS_EINVAL, "ts_decode_step: NULL tensor argument");
   TS_REQUIRE_ALIGNED(kv->k, 16, "k");
   TS_REQUIRE_ALIGNED(kv->v, 16, "v");
@@ -465,8 +468,7 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
   st.table_stride = bt->table_stride;
   st.seq_lens = seq_lens;
   st.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  TS_TRY(check_row_stride(kv->row_stride, st.row_vec * 8, "ts_decode_step"));
-  st.kv_stride = kv->row_stride ? kv->row_stride / 8 : st.row_vec;
+  st.kv_stride = kv_row_stride ? kv_row_stride / 8 : st.row_vec;
   st.max_tokens = kv->max_tokens;
   if (kv->pages) {
     st.free_pages = kv->pages->free_pages;
@@ -474,8 +476,17 @@ int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv
     st.ticket = kv->pages->ticket;
     st.page_shift = page_shift_of(cfg->page_size);
   }
-  return run_layer(cfg, bt, q, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
+  return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
                    sel_stride, sel_len, workspace, workspace_bytes, stream, &st);
+}
+
+int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                   const float* q_cos, const float* q_sin, void* k_pool, void* v_pool,
+                   int64_t pool_rows, const ts_selcache* cache, void* out, int32_t* sel,
+                   int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
+                   size_t workspace_bytes, ts_stream_t stream) {
+  return ts_decode_step_strided(cfg, bt, kv, q, 0, 0, q_cos, q_sin, k_pool, v_pool, pool_rows, cache, out, sel,
+                                sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
 }
 
 // The layer split at the vote, for tensor parallelism (tr.py:361-364): every rank scores
@@ -504,7 +515,7 @@ int ts_decode_layer_votes(const ts_config* cfg, const ts_batch* bt, const void* 
   if (cache)
     TS_REQUIRE(cache->q_cache && cache->topk_cache && cache->cache_len && cache->counters, TS_EINVAL,
                "selection cache has a NULL array");
-  const int q_stride = query_stride(cfg, bt);
+  const int q_stride = cfg->num_heads * cfg->head_dim;
   ts_config plain = *cfg;  // the max-pool comes after the ranks' votes are added up
   plain.pool_kernel = -1;
   char* ws = (char*)workspace;
@@ -575,7 +586,7 @@ int ts_decode_layer_attend(const ts_config* cfg, const ts_batch* bt, const void*
   if (vote_launches_planned(&plain, bt))
     topk.fault = score_votes_fault_word(&plain, bt->batch, bt->max_seq_len, ws + w.select_ws);
   TS_TRY(launch_topk(topk, bt->batch, max_n, (hipStream_t)stream));
-  return launch_attn(cfg, q, query_stride(cfg, bt), k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch, w.max_sel,
+  return launch_attn(cfg, q, cfg->num_heads * cfg->head_dim, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch, w.max_sel,
                      out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream);
 }
 
@@ -587,7 +598,7 @@ int ts_prefill_chunk(const ts_config* cfg, const ts_batch* bt, const void* q, in
   TS_REQUIRE(bt != nullptr && bt->batch == 1, TS_EINVAL,
              "ts_prefill_chunk serves one request at a time (batch must be 1)");
   TS_REQUIRE(rows >= 1, TS_EINVAL, "ts_prefill_chunk: rows %d < 1", rows);
-  return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows,
+  return run_layer(cfg, bt, q, 0, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows,
                    nullptr, out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes,
                    stream);
 }
@@ -595,11 +606,13 @@ int ts_prefill_chunk(const ts_config* cfg, const ts_batch* bt, const void* q, in
 // One chunk of the reference's extend forward in one call (tr.py:725-773): the chunk's K/V
 // stored and appended (ts_kv_store_chunk), then ts_prefill_chunk.  With slots chosen by the
 // caller the store rides in the chunk's first launch, the fingerprint, as spare workgroups.
-int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
-                    int32_t rows, const float* cos_table, const float* sin_table, int64_t table_rows,
-                    void* k_pool, void* v_pool, int64_t pool_rows, void* out, int32_t* sel,
-                    int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
-                    size_t workspace_bytes, ts_stream_t stream) {
+int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                            int32_t q_row_stride, int32_t kv_row_stride, int32_t rows,
+                            const float* cos_table, const float* sin_table, int64_t table_rows,
+                            void* k_pool, void* v_pool, int64_t pool_rows, void* out, int32_t* sel,
+                            int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
+                            size_t workspace_bytes, ts_stream_t stream) {
+  TS_TRY(check_strides(cfg, q_row_stride, kv_row_stride, "ts_prefill_step"));
   TS_REQUIRE(bt != nullptr && bt->batch == 1 && kv != nullptr, TS_EINVAL,
              "ts_prefill_step serves one request at a time (batch must be 1) and needs the chunk's K/V");
   TS_REQUIRE(rows >= 1, TS_EINVAL, "ts_prefill_step: rows %d < 1", rows);
@@ -611,14 +624,14 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
   DenseList list{};
   if (kv->pages == nullptr && bt->rerun == 0 &&
       chunk_store_takes_list(rows, kv->max_tokens, bt->max_seq_len) &&
-      table_rows >= (int64_t)(cfg ? cfg->n_local : 0) + rows && (uintptr_t)cos_table % 16 == 0 &&
+      table_rows >= (int64_t)cfg->n_local + rows && (uintptr_t)cos_table % 16 == 0 &&
       (uintptr_t)sin_table % 16 == 0)
     list = step_list(cfg, bt, nullptr, q, cos_table, sin_table, out, sel, sel_pos, sel_stride, sel_len, workspace,
                      workspace_bytes);
   if (list.sel) {
-    TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
+    TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
                                  v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream, &list));
-    return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr, out,
+    return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr, out,
                      sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr,
                      /*listed=*/true);
   }
@@ -626,13 +639,12 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
                      rows <= 1023 * 16;
   if (!rides) {
     if (bt->rerun == 0)  // (a call that repeats a chunk after a give-up does not append again)
-      TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv->row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
+      TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
                                    v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream));
-    return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
+    return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                      out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
   }
   // The checks ts_kv_store_chunk makes.
-  TS_TRY(validate_config(cfg));
   TS_REQUIRE(kv->k && kv->v && kv->out_cache_loc && k_pool && v_pool, TS_EINVAL,
              "ts_prefill_step: NULL tensor argument");
   TS_REQUIRE_ALIGNED(kv->k, 16, "k");
@@ -653,11 +665,19 @@ int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* k
   cs.seq_len = seq_len;
   cs.rows = rows;
   cs.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  TS_TRY(check_row_stride(kv->row_stride, cs.row_vec * 8, "ts_prefill_step"));
-  cs.kv_stride = kv->row_stride ? kv->row_stride / 8 : cs.row_vec;
+  cs.kv_stride = kv_row_stride ? kv_row_stride / 8 : cs.row_vec;
   cs.max_tokens = kv->max_tokens;
-  return run_layer(cfg, bt, q, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
+  return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                    out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, &cs);
+}
+
+int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                    int32_t rows, const float* cos_table, const float* sin_table, int64_t table_rows,
+                    void* k_pool, void* v_pool, int64_t pool_rows, void* out, int32_t* sel,
+                    int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
+                    size_t workspace_bytes, ts_stream_t stream) {
+  return ts_prefill_step_strided(cfg, bt, kv, q, 0, 0, rows, cos_table, sin_table, table_rows, k_pool, v_pool,
+                                 pool_rows, out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"
