@@ -887,6 +887,26 @@ def fused_select(request):
     ops.set_fused_select(previous)
 
 
+def test_a_call_returns_tensors_of_its_own(dev):
+    """What a caller does in place to the shape of the returned tensors stays with those."""
+    say("layer and chunk: returned tensors reshaped in place")
+    wl = small(dev, SHAPES[0], seed=73, lens=[900, 400], ks=[64] * 2)
+    one = ops.Batch(wl.batch.seq_lens[:1], wl.batch.table[:1], 900)
+    layer = ops.DecodeLayer(wl.cfg, 2, 900, dev)
+    chunk = ops.PrefillChunk(wl.cfg, 900, dev)
+    q = wl.q.view(2, -1)
+    for call, rows in ((lambda: layer(wl.q, wl.k_pool, wl.v_pool, wl.batch), 2),
+                       (lambda: chunk(q, wl.k_pool, wl.v_pool, one), 1)):
+        want = [t.clone() for t in call()]
+        for t in call():
+            t.unsqueeze_(0)
+        got = call()
+        assert [t.shape for t in got] == [t.shape for t in want] and got[1].shape == (rows, wl.cfg.max_sel)
+        n = int(want[3][0])
+        assert torch.equal(got[3], want[3]) and torch.equal(got[1][0, :n], want[1][0, :n])
+        assert torch.equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"H{s['num_heads']}kv{s['num_kv_heads']}")
 @pytest.mark.parametrize("lens", [[3000], [2500, 700, 3000]], ids=["B1", "B3"])
 def test_layer_starts_with_the_selection_on_a_clean_workspace(dev, shape, lens):

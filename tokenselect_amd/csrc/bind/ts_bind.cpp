@@ -152,13 +152,6 @@ struct Owned {
   // see, may have used it since any call it remembers.  From then on nothing is remembered.
   bool captured = false;
   void forget_clean() { clean_batch = clean_len = clean_layout = -1; }
-  // The outputs' first rows, for the last batch size: out, sel, sel_pos, sel_len.
-  int64_t views_of = -1;
-  PyObject* views[4] = {nullptr, nullptr, nullptr, nullptr};
-  void forget_views() {
-    for (PyObject*& r : views) Py_CLEAR(r);
-    views_of = -1;
-  }
 };
 
 struct Runner {
@@ -309,8 +302,16 @@ bool capturing() {
   return status != hipStreamCaptureStatusNone;
 }
 
+// The first B rows, as a tensor of its own.  (As narrow() makes it, without the dispatcher: four
+// of them are made per call, 2 us of the 17 that a dense step of 2003 tokens takes.)
 PyObject* row_view(const at::Tensor& t, int64_t B) {
-  PyObject* v = THPVariable_Wrap(t.narrow(0, 0, B));
+  at::Tensor rows = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(t.storage()),
+                                                             t.key_set(), t.dtype());
+  c10::SmallVector<int64_t, 4> sizes(t.sizes().begin(), t.sizes().end());
+  sizes[0] = B;
+  rows.unsafeGetTensorImpl()->set_storage_offset(t.storage_offset());
+  rows.unsafeGetTensorImpl()->set_sizes_and_strides(sizes, t.strides());
+  PyObject* v = THPVariable_Wrap(std::move(rows));
   if (!v) throw Raised{};
   return v;
 }
@@ -422,14 +423,6 @@ PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   const bool cached = cache_o != Py_None;
   if (cached) fill_cache(cfg, cache_o, B, &cache);
 
-  if (o.views_of != B) {
-    o.forget_views();
-    if (!chunk) o.views[0] = row_view(o.out, B);
-    o.views[1] = row_view(o.sel, B);
-    o.views[2] = row_view(o.sel_pos, B);
-    o.views[3] = row_view(o.sel_len, B);
-    o.views_of = B;
-  }
   PyObject* out_py;
   void* out_ptr;
   if (out_o != Py_None) {
@@ -445,15 +438,16 @@ PyObject* run(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
     if (!out_py) throw Raised{};
   } else {
     out_ptr = o.out.data_ptr();
-    out_py = o.views[0];
-    Py_INCREF(out_py);
+    out_py = row_view(o.out, B);
   }
   const Ref out_ref(out_py);
 
   const int code = call_library(o, &bt, store ? &kv : nullptr, q.data_ptr(), 0, 0, rows, k_pool, v_pool,
                                 cached ? &cache : nullptr, out_ptr, rerun);
   if (code != TS_OK) return PyLong_FromLong(code);
-  return PyTuple_Pack(4, out_py, o.views[1], o.views[2], o.views[3]);
+  // (tensors of the call's own: a caller may reshape or resize them in place)
+  const Ref sel(row_view(o.sel, B)), sel_pos(row_view(o.sel_pos, B)), sel_len(row_view(o.sel_len, B));
+  return PyTuple_Pack(4, out_py, sel.p, sel_pos.p, sel_len.p);
 }
 
 // serve(q, k, v, out_cache_loc, k_pool, v_pool, bt, cache, out, from, rows, separate): the step of a
@@ -567,10 +561,7 @@ PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
 
 void runner_dealloc(PyObject* self) {
   Owned* o = ((Runner*)self)->own;
-  if (o) {
-    o->forget_views();
-    delete o;
-  }
+  delete o;
   PyTypeObject* type = Py_TYPE(self);
   type->tp_free(self);
   Py_DECREF(type);
