@@ -602,18 +602,22 @@ def patched_radix_attention_store_kv_cache(self, cache_k, cache_v, input_metadat
     retriever.add_k_cache(loc, self.layer_id)
 
 
-# What a step in one call takes the place of, as defined here.
-_STEP_PARTS = {"decode_attention": (TokenRetriever.decode_attention, BatchTokenRetriever.decode_attention),
-               "prefill_attention": (TokenRetriever.prefill_attention,), "store": (BatchTokenRetriever.store,)}
+# What a step in one call takes the place of, as defined here: the retrievers' attention and store.
+_decode_attention, _prefill_attention = TokenRetriever.decode_attention, TokenRetriever.prefill_attention
+_batch_attention, _batch_store = BatchTokenRetriever.decode_attention, BatchTokenRetriever.store
 
 
-def _one_call(attn, retriever, parts, loc, rows) -> bool:
-    """Whether ``rows`` new tokens can be left to the library's step calls: 32-bit slots, one per
-    row, a store that is the patched one, and a retriever whose methods ``parts`` nobody has
-    replaced (a subclass's, or one set on the object or the class, is called as ever)."""
+def _function(method):
+    return getattr(method, "__func__", None)
+
+
+def _one_call(attn, loc, rows) -> bool:
+    """Whether the store of ``rows`` new tokens can be left to the library's step calls: 32-bit
+    slots, one per row, and a store that is the patched one.  (The callers also look whether the
+    retriever's methods are those above: one that a subclass, the object or the class replaces
+    is called as ever.)"""
     return loc.dtype == torch.int32 and loc.dim() == 1 and loc.shape[0] == rows and \
-        getattr(attn.store_kv_cache, "__func__", None) is patched_radix_attention_store_kv_cache and \
-        all(getattr(getattr(retriever, name, None), "__func__", None) in _STEP_PARTS[name] for name in parts)
+        _function(attn.store_kv_cache) is patched_radix_attention_store_kv_cache
 
 
 def patched_radix_attention_decode_forward_flashinfer(self, q, k, v, input_metadata):
@@ -624,8 +628,12 @@ def patched_radix_attention_decode_forward_flashinfer(self, q, k, v, input_metad
     batched = isinstance(retriever, BatchTokenRetriever)
     if k is not None:
         assert v is not None
-        if q.shape[0] == (retriever.batch if batched else 1) and _one_call(
-                self, retriever, ("decode_attention", "store") if batched else ("decode_attention",), loc, q.shape[0]):
+        if batched:
+            own = _function(retriever.decode_attention) is _batch_attention and \
+                _function(retriever.store) is _batch_store
+        else:
+            own = _function(retriever.decode_attention) is _decode_attention
+        if own and q.shape[0] == (retriever.batch if batched else 1) and _one_call(self, loc, q.shape[0]):
             k_buffer, v_buffer = input_metadata.token_to_kv_pool.get_kv_buffer(self.layer_id)
             return retriever.decode_step(self, q, k, v, loc, k_buffer, v_buffer)
         self.store_kv_cache(k, v, input_metadata)
@@ -649,7 +657,7 @@ def patched_radix_attention_extend_forward_flashinfer(self, q, k, v, input_metad
     k_buffer, v_buffer = input_metadata.token_to_kv_pool.get_kv_buffer(self.layer_id)
     retriever, loc = input_metadata.token_retriever, input_metadata.out_cache_loc
     if k is not None and v is not None and isinstance(retriever, TokenRetriever) and q.dim() == 2 \
-            and _one_call(self, retriever, ("prefill_attention",), loc, q.shape[0]):
+            and _function(retriever.prefill_attention) is _prefill_attention and _one_call(self, loc, q.shape[0]):
         return retriever.prefill_step(self, q, k, v, loc, k_buffer, v_buffer, outputs)
     for start in range(0, q.shape[0], PREFILL_CHUNK_SIZE):
         end = min(start + PREFILL_CHUNK_SIZE, q.shape[0])
