@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle
-from tokenselect_amd import ops, workloads
+from tokenselect_amd import _lib, ops, workloads
 from helpers import (assert_attention_close, assert_index_sets_match, assert_scores_close, cpu_tabs,
                      oracle_layer, say)
 
@@ -885,6 +885,71 @@ def fused_select(request):
     previous = ops.set_fused_select(request.param)
     yield request.param
     ops.set_fused_select(previous)
+
+
+def test_replaced_buffers_and_copies(dev):
+    """A buffer assigned to a layer object is the one that its calls use from then on (one that
+    does not fit is refused and changes nothing), and copies are objects of their own."""
+    import copy
+    say("layer: buffers replaced, object copied")
+    wl = small(dev, SHAPES[0], seed=74, lens=[900, 400], ks=[64] * 2)
+    args = (wl.q, wl.k_pool, wl.v_pool, wl.batch)
+    layer = ops.DecodeLayer(wl.cfg, 2, 900, dev)
+    want = [t.clone() for t in layer(*args)]
+    lists = [int(n) for n in want[3]]
+
+    def same(got):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[3], want[3])
+        for b, n in enumerate(lists):
+            assert torch.equal(got[1][b, :n], want[1][b, :n]) and torch.equal(got[2][b, :n], want[2][b, :n])
+
+    for name in ("out", "sel", "sel_len", "workspace"):
+        mine = torch.full_like(getattr(layer, name), 7)
+        setattr(layer, name, mine)
+        assert layer._clean_for is None
+        same(layer(*args))
+        torch.cuda.synchronize()
+        assert getattr(layer, name) is mine and bool((mine != 7).any()), name
+    assert layer(*args)[0].data_ptr() == layer.out.data_ptr()
+    word = ops.fault_word()
+    layer.fault = word
+    word[0] = 1                                   # (as a selection that gave up leaves it)
+    with pytest.raises(ops.SelectionGaveUp):
+        layer(*args)
+    layer.separate = False
+    for name, bad in (("out", layer.out.float()), ("out", layer.out[:1]), ("sel", layer.sel[:, 1:]),
+                      ("sel_pos", layer.sel_pos[:1].contiguous()), ("sel_len", layer.sel_len.cpu()),
+                      ("workspace", layer.workspace.int()), ("fault", torch.zeros(1, dtype=torch.int32))):
+        before = getattr(layer, name)
+        with pytest.raises((ValueError, TypeError)):
+            setattr(layer, name, bad)
+        assert getattr(layer, name) is before
+    same(layer(*args))
+    whole = layer.workspace
+    layer.workspace = whole[:256].clone()
+    with pytest.raises(_lib.TokenSelectError):    # too small: the library's own check
+        layer(*args)
+    layer.workspace = whole
+
+    deep, twin = copy.deepcopy(layer), copy.copy(layer)
+    assert deep.out.data_ptr() != layer.out.data_ptr() and twin.out.data_ptr() == layer.out.data_ptr()
+    one = ops.Batch(wl.batch.seq_lens[:1], wl.batch.table[:1], 900)
+    for i in range(3):
+        same(layer(*args))
+        twin(wl.q[:1].contiguous(), wl.k_pool, wl.v_pool, one)   # (another shape on the same workspace)
+        same(deep(*args))
+    assert deep._clean_for == (2, 900) and twin._clean_for is None and layer._clean_for is None
+    assert not layer.gave_up() and not deep.gave_up() and not twin.gave_up()
+
+    chunk = ops.PrefillChunk(wl.cfg, 900, dev)
+    q = wl.q.view(2, -1)
+    want_chunk = [t.clone() for t in chunk(q, wl.k_pool, wl.v_pool, one)]
+    chunk.sel = torch.full_like(chunk.sel, 7)
+    for c in (chunk, copy.deepcopy(chunk)):
+        got = c(q, wl.k_pool, wl.v_pool, one)
+        n = int(want_chunk[3][0])
+        assert torch.equal(got[0], want_chunk[0]) and torch.equal(got[1][0, :n], want_chunk[1][0, :n])
+    assert bool((chunk.sel != 7).any())
 
 
 def test_a_call_returns_tensors_of_its_own(dev):

@@ -148,9 +148,10 @@ struct Owned {
   // (batch, max_seq_len) that the selection's counters in the workspace are clean for, -1: none.
   int64_t clean_batch = -1, clean_len = -1;
   int64_t clean_layout = -1;  // ts_decode_layer_layout of that call
-  // A call on this workspace was recorded into a graph: a replay, which the object does not
-  // see, may have used it since any call it remembers.  From then on nothing is remembered.
-  bool captured = false;
+  // The workspace has users that the object does not see: the replays of a graph into which a
+  // call on it was recorded, or a shallow copy of the object.  They may have used it since any
+  // call that is remembered, so from then on none is.
+  bool shared = false;
   void forget_clean() { clean_batch = clean_len = clean_layout = -1; }
 };
 
@@ -327,8 +328,8 @@ int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int
   const bool chunk = o.max_rows > 0;
   // (While a graph is captured the object states nothing: the recorded flag would hold for
   // every replay, whatever used the workspace before it.)
-  if (!chunk && !o.captured) o.captured = capturing();
-  const bool plain = !chunk && !cache && !bt->separate_kernels && !rerun && !o.captured;
+  if (!chunk && !o.shared) o.shared = capturing();
+  const bool plain = !chunk && !cache && !bt->separate_kernels && !rerun && !o.shared;
   // (By the layout and not by the length, which grows with every token: it is the same for
   // some 64 steps, and each of them starts with the selection instead of with a launch that
   // rotates and clears: 2 layers of a 128K request, two steps, 296 -> 292 us; a 31599-token
@@ -541,14 +542,26 @@ PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
     Owned* o = new Owned();
     ((Runner*)self.p)->own = o;
     memcpy(&o->cfg, cfg.buf, sizeof(ts_config));
-    o->workspace = tensor(ws, "workspace");
-    o->cos = tensor(cos, "cos");
-    o->sin = tensor(sin, "sin");
-    if (out != Py_None) o->out = tensor(out, "out");
-    o->sel = tensor(sel, "sel");
-    o->sel_pos = tensor(sel_pos, "sel_pos");
-    o->sel_len = tensor(sel_len, "sel_len");
+    const ts_config& c = o->cfg;
+    const int64_t width = (int64_t)c.num_heads * c.head_dim, max_sel = (int64_t)c.n_init + c.top_k + c.n_local;
+    o->workspace = need(ws, "workspace", at::kByte);
+    o->cos = need(cos, "cos", at::kFloat, 2);
+    o->sin = need(sin, "sin", at::kFloat, 2);
+    if (o->cos.sizes() != o->sin.sizes() || o->cos.size(0) < 1 || o->cos.size(1) != c.head_dim)
+      bad_value("cos / sin must both be [rows, head_dim]");
+    if (out != Py_None) {
+      o->out = need(out, "out", at::kBFloat16, 2);
+      if (o->out.size(0) < batch || o->out.size(1) != width) bad_value("out must hold the batch's rows of H*D elements");
+    }
+    o->sel = need(sel, "sel", at::kInt, 2);
+    o->sel_pos = need(sel_pos, "sel_pos", at::kInt, 2);
+    o->sel_len = need(sel_len, "sel_len", at::kInt, 1);
+    if (o->sel.size(0) < batch || o->sel.size(1) < max_sel || o->sel_pos.sizes() != o->sel.sizes() ||
+        o->sel_len.size(0) < batch)
+      bad_value("sel / sel_pos / sel_len must hold the batch's lists of " + std::to_string(max_sel));
     o->fault = tensor(fault, "fault");
+    if (o->fault.scalar_type() != at::kInt || o->fault.numel() != 1 || !o->fault.is_pinned())
+      bad_value("fault must be one int32 word of pinned host memory");
     o->batch = batch;
     o->max_seq_len = max_seq_len;
     o->max_rows = max_rows;
@@ -577,7 +590,7 @@ int set_clean(PyObject* self, PyObject* value, void*) {
   long long b = -1, n = -1;
   if (value != Py_None && !(value && PyArg_ParseTuple(value, "LL", &b, &n))) return -1;
   if (value == Py_None) {  // other calls use the workspace from here on
-    o.captured = o.captured || capturing();
+    o.shared = o.shared || capturing();
     o.forget_clean();
     return 0;
   }
@@ -587,11 +600,21 @@ int set_clean(PyObject* self, PyObject* value, void*) {
   return 0;
 }
 
+PyObject* get_shared(PyObject* self, void*) { return PyBool_FromLong(((Runner*)self)->own->shared); }
+int set_shared(PyObject* self, PyObject* value, void*) {
+  const int yes = value ? PyObject_IsTrue(value) : 0;
+  if (yes < 0) return -1;
+  ((Runner*)self)->own->shared = yes != 0;
+  return 0;
+}
+
 PyMethodDef runner_methods[] = {
     {"run", (PyCFunction)(void (*)(void))runner_run, METH_FASTCALL, nullptr},
     {"serve", (PyCFunction)(void (*)(void))runner_serve, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
-PyGetSetDef runner_getset[] = {{"clean", get_clean, set_clean, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyGetSetDef runner_getset[] = {{"clean", get_clean, set_clean, nullptr, nullptr},
+                               {"shared", get_shared, set_shared, nullptr, nullptr},
+                               {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyType_Slot runner_slots[] = {{Py_tp_new, (void*)runner_new}, {Py_tp_dealloc, (void*)runner_dealloc},
                               {Py_tp_methods, runner_methods}, {Py_tp_getset, runner_getset}, {0, nullptr}};
 PyType_Spec runner_spec = {"_ts_bind.Runner", sizeof(Runner), 0, Py_TPFLAGS_DEFAULT, runner_slots};

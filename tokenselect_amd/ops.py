@@ -129,9 +129,11 @@ class _GiveUpLatch:
     """What DecodeLayer and PrefillChunk share: the pinned fault word, the switch to the
     separate kernels that a give-up latches for the object, and the options of a call."""
 
-    def _init_latch(self):
-        self.fault = fault_word()
-        self.separate = False  # latched by a give-up: the separate kernels from then on
+    def _init_latch(self, **own):
+        # (past __setattr__: a patched forward builds two of these objects per request)
+        vars(self).update(own, fault=fault_word(),
+                          separate=False)  # latched by a give-up: the separate kernels from then on
+        self._connect()
 
     def gave_up(self) -> bool:
         """Whether a selection of this object gave up since the last check (a host memory
@@ -159,11 +161,47 @@ class _GiveUpLatch:
             kw["separate_kernels"] = True
         return dataclasses.replace(bt, **kw) if kw else bt
 
-    def _init_native(self, cos, sin, out, batch: int, max_rows: int):
-        """The object's buffers handed to the native host path (``_lib.binding()``)."""
-        self._native = _lib.binding().Runner(bytes(self._c), self.workspace, cos, sin, out, self.sel,
-                                             self.sel_pos, self.sel_len, self.fault, batch,
-                                             self.max_seq_len, max_rows)
+    def _connect(self):
+        """Hands the object's buffers to the native host path (``_lib.binding()``)."""
+        cos, sin, out, batch, max_rows = self._shapes()
+        native = _lib.binding().Runner(bytes(self._c), self.workspace, cos, sin, out, self.sel, self.sel_pos,
+                                       self.sel_len, self.fault, batch, self.max_seq_len, max_rows)
+        if "_native" in self.__dict__:
+            native.shared = self._native.shared
+        vars(self)["_native"] = native
+
+    # What the native host path holds of the object: assigning one hands it over again.
+    _HELD = frozenset(("_c", "workspace", "q_cos", "q_sin", "cos", "sin", "out", "sel", "sel_pos", "sel_len", "fault",
+                       "batch", "max_seq_len", "max_rows"))
+
+    def __setattr__(self, name, value):
+        if name not in self._HELD or "_native" not in self.__dict__:
+            object.__setattr__(self, name, value)
+            return
+        before = self.__dict__.get(name)
+        object.__setattr__(self, name, value)
+        try:
+            self._connect()
+        except Exception:
+            object.__setattr__(self, name, before)
+            raise
+
+    # A copy has a fault word and a native half of its own; a deep copy also its own buffers.
+    def __getstate__(self):
+        return {name: value for name, value in self.__dict__.items() if name != "_native"}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        set_already = int(self.fault[0])
+        self.fault = fault_word()
+        self.fault[0] = set_already
+        self._connect()
+
+    def __copy__(self):
+        twin = type(self).__new__(type(self))
+        twin.__setstate__(self.__getstate__())
+        self._native.shared = twin._native.shared = True   # (one workspace, two objects that use it)
+        return twin
 
     def _serve(self, q, k, v, loc, k_pool, v_pool, bt, cache=None, out=None, start: int = 0,
                rows: int = 0) -> torch.Tensor:
@@ -732,7 +770,10 @@ def scoring_cos_sin(head_dim: int, rope_base: float, rope_scale, n_local: int, d
 
 class DecodeLayer(_GiveUpLatch):
     """One layer of the patched decode forward after the KV store
-    (tr.py:791-825) as a single library call; buffers are allocated once.
+    (tr.py:791-825) as a single library call; buffers are allocated once (a caller may
+    assign others: ``workspace``, ``out``, ``sel``, ``sel_pos``, ``sel_len``, ``fault``).
+    What a call returns are new tensors over the first rows of these buffers, which the
+    next call writes again.
 
     A fused selection kernel that gave up (``SelectionGaveUp``) has left ``sel_len[b] = -1``
     and an output attended over nothing.  A caller that synchronises before the output is
@@ -743,24 +784,23 @@ class DecodeLayer(_GiveUpLatch):
     def __init__(self, cfg: LayerConfig, batch: int, max_seq_len: int, device, tables=None):
         """``tables``: the ``(cos, sin)`` of :func:`rope_tables` with at least
         ``n_local + 1`` rows, where the caller has them already."""
-        self.cfg, self.batch, self.max_seq_len = cfg, batch, max_seq_len
-        self._c = cfg.to_c()
-        lib = _lib.load()
-        _lib.check(lib.ts_check_config(ctypes.byref(self._c)))
-        nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(self._c), batch, max_seq_len)
-        self.workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
+        c, lib = cfg.to_c(), _lib.load()
+        _lib.check(lib.ts_check_config(ctypes.byref(c)))
+        nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(c), batch, max_seq_len)
+        workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
         if tables is not None:
-            self.q_cos, self.q_sin = (t[cfg.n_local:cfg.n_local + 1] for t in tables)
+            q_cos, q_sin = (t[cfg.n_local:cfg.n_local + 1] for t in tables)
         else:
-            self.q_cos, self.q_sin = scoring_cos_sin(cfg.head_dim, cfg.rope_theta, cfg.rope_scale,
-                                                     cfg.n_local, device)
-        self.out = torch.empty((batch, cfg.num_heads * cfg.head_dim), dtype=torch.bfloat16,
-                               device=device)
-        self.sel = torch.empty((batch, cfg.max_sel), dtype=torch.int32, device=device)
-        self.sel_pos = torch.empty_like(self.sel)
-        self.sel_len = torch.empty((batch,), dtype=torch.int32, device=device)
-        self._init_latch()
-        self._init_native(self.q_cos, self.q_sin, self.out, batch, 0)
+            q_cos, q_sin = scoring_cos_sin(cfg.head_dim, cfg.rope_theta, cfg.rope_scale, cfg.n_local, device)
+        out = torch.empty((batch, cfg.num_heads * cfg.head_dim), dtype=torch.bfloat16, device=device)
+        sel = torch.empty((batch, cfg.max_sel), dtype=torch.int32, device=device)
+        sel_pos = torch.empty_like(sel)
+        sel_len = torch.empty((batch,), dtype=torch.int32, device=device)
+        self._init_latch(cfg=cfg, _c=c, batch=batch, max_seq_len=max_seq_len, workspace=workspace, q_cos=q_cos,
+                         q_sin=q_sin, out=out, sel=sel, sel_pos=sel_pos, sel_len=sel_len)
+
+    def _shapes(self):
+        return self.q_cos, self.q_sin, self.out, self.batch, 0
 
     @property
     def _clean_for(self):
@@ -943,19 +983,20 @@ class PrefillChunk(_GiveUpLatch):
     def __init__(self, cfg: LayerConfig, max_seq_len: int, device, max_rows: int = 512, tables=None):
         """``tables``: the ``(cos, sin)`` of :func:`rope_tables` with ``n_local + max_rows``
         rows, where the caller has them already."""
-        self.cfg, self.max_seq_len, self.max_rows = cfg, max_seq_len, max_rows
-        self._c = cfg.to_c()
-        lib = _lib.load()
-        _lib.check(lib.ts_check_config(ctypes.byref(self._c)))
-        nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(self._c), 1, max_seq_len)
-        self.workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
-        self.cos, self.sin = tables if tables is not None else rope_tables(
+        c, lib = cfg.to_c(), _lib.load()
+        _lib.check(lib.ts_check_config(ctypes.byref(c)))
+        nbytes = lib.ts_decode_layer_workspace_bytes(ctypes.byref(c), 1, max_seq_len)
+        workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
+        cos, sin = tables if tables is not None else rope_tables(
             cfg.head_dim, cfg.rope_theta, cfg.rope_scale, cfg.n_local + max_rows, device)
-        self.sel = torch.empty((1, cfg.max_sel), dtype=torch.int32, device=device)
-        self.sel_pos = torch.empty_like(self.sel)
-        self.sel_len = torch.empty((1,), dtype=torch.int32, device=device)
-        self._init_latch()
-        self._init_native(self.cos, self.sin, None, 1, max_rows)
+        sel = torch.empty((1, cfg.max_sel), dtype=torch.int32, device=device)
+        sel_pos = torch.empty_like(sel)
+        sel_len = torch.empty((1,), dtype=torch.int32, device=device)
+        self._init_latch(cfg=cfg, _c=c, max_seq_len=max_seq_len, max_rows=max_rows, workspace=workspace, cos=cos,
+                         sin=sin, sel=sel, sel_pos=sel_pos, sel_len=sel_len)
+
+    def _shapes(self):
+        return self.cos, self.sin, None, 1, self.max_rows
 
     def recover(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                 out: Optional[torch.Tensor] = None):
