@@ -31,6 +31,9 @@ CXXFLAGS = [
 ]
 # Matrix instructions write to the vector registers, as the vector instructions that follow on
 # their results want them; accumulators that are to live in the others are placed by hand.
+# (An internal option of the compiler: one that does not know it refuses it, and the build stops
+# there.  Without it the kernel is as correct and moves its logits between the two halves of the
+# register file.)
 SOURCE_FLAGS = {"ts_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 

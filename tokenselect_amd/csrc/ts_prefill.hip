@@ -292,10 +292,11 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 // accumulators of the output and the queries in the accumulation registers, the logits,
 // which vector instructions read, in the others.  Written as assembly because the compiler,
 // left to choose, moves accumulators to and fro around every product (480 moves per tile).
-// What it does not see it does not keep apart: the caller leaves at least eleven cycles of
-// instruction issue between a product and any use of its result other than as the same
-// product's next accumulator, and two between a vector instruction and a product that reads
-// its result.
+// What it does not see it does not keep apart: between a product and any use of its result other
+// than as the same product's next accumulator there must be eight instructions' issue, and two
+// between a vector instruction and a product that reads its result.  The two fences below make
+// that order a dependency of the values themselves; tests/test_prefill_hazards_cpu.py looks
+// through the compiler's listing for what register copies could still have put in between.
 __device__ __forceinline__ void mfma_acc(pf_f32x4& acc, const pf_bf16x8& a, const pf_bf16x8& b) {
   asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
@@ -305,8 +306,24 @@ __device__ __forceinline__ pf_f32x4 mfma_logits(const pf_f32x4& s, const uint4& 
 // Says that acc lives in the accumulation registers here, so that where paths join it stays there.
 template <typename V>
 __device__ __forceinline__ void keep_acc(V& acc) { asm("" : "+a"(acc)); }
-// Eleven instructions and more: between the last product and another use of its accumulators.
-__device__ __forceinline__ void mfma_settled() { asm volatile("s_nop 15" ::: "memory"); }
+// The accumulators behind this are those before it, sixteen idle instructions later: no use of
+// one can come before the idling, and no product that makes one after it.
+template <int CB>
+__device__ __forceinline__ void mfma_settled(pf_f32x4 (&o)[CB][8]) {
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int db = 0; db < 8; ++db) asm volatile("" : "+a"(o[cb][db]));
+  asm volatile("s_nop 15" ::: "memory");
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int db = 0; db < 8; ++db) asm volatile("" : "+a"(o[cb][db]));
+}
+// The weights behind this are those before it, two idle instructions later.
+__device__ __forceinline__ void packed_settled(pf_bf16x8 (&pb)[4]) {
+  asm("s_nop 1" : "+v"(pb[0]), "+v"(pb[1]), "+v"(pb[2]), "+v"(pb[3]));
+}
 
 // Heads of a workgroup's column blocks; the kPfBlocks / heads blocks of a head are
 // consecutive query tiles.  The choice that leaves the fewest columns of the last head block
@@ -580,8 +597,7 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
       pb[cb] = __builtin_bit_cast(pf_bf16x8, make_uint4(pw[cb][0], pw[cb][1], pw[cb][2], pw[cb][3]));
-    // (the row sums first: between the packing of the weights and the products whose
-    // registers the compiler does not see)
+    packed_settled(pb);
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
       row_sum[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[cb], row_sum[cb], 0, 0, 0);
@@ -597,7 +613,7 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    mfma_settled();
+    mfma_settled(o);
     __builtin_amdgcn_sched_barrier(0);
     if (NEXT) {
       settle(s_next, mx);
@@ -625,8 +641,6 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
     // loop's head the compiler waits for the later of the two orders it may have come from)
 #pragma unroll
     for (int i = 0; i < kPfOperands; ++i) vw[i] = v0[64 * i + lane];
-    __builtin_amdgcn_sched_barrier(0);
-    mfma_settled();
     __builtin_amdgcn_sched_barrier(0);
     float mx[CB];
 #pragma unroll
