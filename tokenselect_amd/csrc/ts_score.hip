@@ -610,17 +610,26 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   const int tile_stride = FUSED ? 16 * H + 16 : 16 * H;
   const int32_t* tab = a.table + (int64_t)b * a.table_stride;
 
-  // A operands: query 4*na + t4 of each KV head, same byte offsets as the keys.  The four
-  // wavefronts share the work of preparing them: wavefront w loads the operands w, w + 4, ...
-  // (one of which is also rotated where the kernel does that itself: the 8 dims 64 further on
-  // and the rotation's rows are loaded too) and hands them over in LDS.  Only the table
+  // A operands: query 4*na + t4 of each KV head, same byte offsets as the keys.  In the single
+  // launch the four wavefronts share the work of preparing them: wavefront w loads the operands w,
+  // w + 4, ... (one of which is also rotated where the kernel does that itself: the 8 dims 64
+  // further on and the rotation's rows are loaded too) and hands them over in LDS.  Only the table
   // entries stand before the first keys; the queries arrive and are rotated while the keys
   // travel (every wavefront preparing all operands first, the first key was asked for 3.3 us
   // into a selection from 32K tokens that takes 27).
-  constexpr bool RAW = FUSED && !PACKED;  // the query may be un-rotated (a.q_raw)
+  // The other forms have rotated queries, and workgroups that follow each other on a CU: a
+  // wavefront loads its own, and one without tokens asks for no keys.  Shared in LDS they cost
+  // a barrier between every workgroup's first keys and its first product, and keys asked for
+  // by wavefronts without tokens are bytes.  Votes of 9 x 60K tokens, seven heads per KV head:
+  // 159.4 us shared, 155.4 without the barrier, 149.1 without those keys either; 18 x 20K 97.3,
+  // 95.8 and 93.4; scores alone of 8 x 20K 54.0, 52.9 and 50.5; with four heads per KV head (16 x
+  // 68K, 4 x 256K) all within the spread.
+  constexpr bool SHARED_QUERY = FUSED && !PACKED;
+  constexpr bool RAW = SHARED_QUERY;  // the query may be un-rotated (a.q_raw)
   constexpr int OPS = HKV * NA, MINE = (OPS + 3) / 4;
   // The histogram of the selection below takes the same place.
-  __shared__ __attribute__((aligned(16))) uint32_t lh[FUSED && kTopkBins > OPS * 256 ? kTopkBins : OPS * 256];
+  constexpr int LH = SHARED_QUERY && OPS * 256 > kTopkBins ? OPS * 256 : kTopkBins;
+  __shared__ __attribute__((aligned(16))) uint32_t lh[FUSED ? LH : 4];
   const bool raw = RAW && a.q_raw != nullptr;
   const bool lower = rg < 2;
   uint4 q_own[MINE], q_other[MINE];
@@ -754,29 +763,45 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
 
   size_t rows_cur[TG][4];
   size_t rows_next[TG][4];
-  {
-    // (a wavefront without tokens asks too, for its request's last ones: behind a branch the
-    // compiler would wait for all of these loads where it joins)
+  if constexpr (!SHARED_QUERY) {
+#pragma unroll
+    for (int kvh = 0; kvh < HKV; ++kvh)
+#pragma unroll
+      for (int na = 0; na < NA; ++na) {
+        const int g = 4 * na + t4;
+        const int h = head_of<HKV, G>(kvh, g < G ? g : 0, a.head_map);
+        uint4 v = *(const uint4*)((const char*)(a.qf + ((size_t)b * H + h) * kHeadDim) + lane_off);
+        if (g >= G) v = make_uint4(0u, 0u, 0u, 0u);
+        qa[kvh][na] = __builtin_bit_cast(bf16x8_t, v);
+      }
+  }
+  if (SHARED_QUERY || wave_lo < wave_hi) {
+    // (in the single launch a wavefront without tokens asks too, for its request's last ones:
+    // behind a branch the compiler would wait for the queries' loads where it joins)
     int32_t entry_first[TG][4];
 #pragma unroll
     for (int t = 0; t < TG; ++t)
 #pragma unroll
       for (int m = 0; m < 4; ++m) entry_first[t][m] = table_entry(wave_lo + 16 * t + 4 * m + t4);
-    load_queries();  // (in flight together with the table entries)
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SHARED_QUERY) {
+      load_queries();  // (in flight together with the table entries)
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int t = 0; t < TG; ++t)
 #pragma unroll
       for (int m = 0; m < 4; ++m) rows_cur[t][m] = row_off(entry_first[t][m], wave_lo + 16 * t + 4 * m + t4);
     issue(buf0, rows_cur, 0);
   }
-  share_queries();
-  __syncthreads();
+  if constexpr (SHARED_QUERY) {
+    share_queries();
+    __syncthreads();
 #pragma unroll
-  for (int kvh = 0; kvh < HKV; ++kvh)
+    for (int kvh = 0; kvh < HKV; ++kvh)
 #pragma unroll
-    for (int na = 0; na < NA; ++na)
-      qa[kvh][na] = __builtin_bit_cast(bf16x8_t, *(const uint4*)&lh[(kvh * NA + na) * 256 + lane * 4]);
+      for (int na = 0; na < NA; ++na)
+        qa[kvh][na] = __builtin_bit_cast(bf16x8_t, *(const uint4*)&lh[(kvh * NA + na) * 256 + lane * 4]);
+  }
 
   for (int base = wave_lo; base < wave_hi; base += ITER) {
     int32_t entry_next[TG][4];
