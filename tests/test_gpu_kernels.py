@@ -248,6 +248,41 @@ def test_fused_select_ties(dev):
         assert torch.equal(sel_pos[0, :int(sel_len[0])], pos_sep[0, :int(sel_len[0])])
 
 
+@pytest.mark.parametrize("where", ["adjacent", "spread", "ends", "powers"])
+@pytest.mark.parametrize("group", [2, 3, 64, 65, 255])
+def test_fused_select_ties_in_the_list(dev, group, where):
+    """A group of equal votes at the top, alone and among close ones, cut after its first, in its
+    middle and before its last: its lowest positions are taken, wherever it lies."""
+    L, n_init, n_local = 40000, 8, 16
+    n = L - n_init - n_local
+    at = {"adjacent": lambda m: 8190 + torch.arange(m), "spread": lambda m: torch.arange(m) * ((n - 1) // (m - 1)),
+          "ends": lambda m: torch.cat([torch.arange(m // 2), n - m + m // 2 + torch.arange(m - m // 2)]),
+          "powers": lambda m: torch.cat([2 ** torch.arange(15), 20000 + torch.arange(max(m - 15, 0))])[:m]}[where](group)
+    for k in sorted({1, max(group // 2, 1), group - 1}):
+        say(f"ties in the list: {group} {where}, k={k}")
+        wl = small(dev, SHAPES[0], seed=85, lens=[L], ks=[k], page=1, top_k=k, n_init=n_init, n_local=n_local)
+        c = wl.cfg
+        tab, group_at = wl.table[0].long(), at.to(dev)
+        qf = fingerprint(wl, dev)
+        heads = qf.view(c.num_heads, c.head_dim).float()
+        row = torch.stack([heads[kv::c.num_kv_heads].mean(0) for kv in range(c.num_kv_heads)])
+        row = (row / row.norm(dim=-1, keepdim=True) * 16).bfloat16()
+        for close in (0, 100):
+            pool = wl.k_pool.clone()
+            near = torch.randperm(n, generator=torch.Generator().manual_seed(close))[:close].to(dev)
+            pool[tab[n_init + near]] = (row.float() * torch.linspace(0.95, 0.985, max(close, 1), device=dev)[:close, None, None]
+                                        ).bfloat16()
+            pool[tab[n_init + group_at]] = row
+            _, sel_pos, sel_len, votes, space = ops.select(c, wl.batch, qf, pool, want_votes=True)
+            torch.cuda.synchronize()
+            assert not ops.select_fault(c, wl.batch, space)
+            v = votes[0, :n]
+            assert torch.unique(v[group_at]).numel() == 1 and int((v >= v[group_at[0]]).sum()) == group
+            mid = sel_pos[0, n_init:n_init + k].long() - n_init
+            order = torch.sort(v, descending=True, stable=True).indices[:k]   # (stable: lowest position first)
+            assert torch.equal(mid, order.sort().values), f"k={k} close={close}"
+
+
 @pytest.mark.parametrize("fused_select", [True, False], indirect=True, ids=["fused", "separate"])
 def test_select_with_all_votes_equal(dev, fused_select):
     """A zero query makes every vote H/n: one histogram bin at every level, every

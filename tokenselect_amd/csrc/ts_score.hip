@@ -402,6 +402,19 @@ __device__ __forceinline__ uint32_t wave_total(uint32_t x) {
                     __builtin_amdgcn_readlane((int)x, 32) + __builtin_amdgcn_readlane((int)x, 48));
 }
 
+// Bits set in any lane of the wavefront, in every lane.
+__device__ __forceinline__ uint32_t wave_or(uint32_t x) {
+  auto ror = [](uint32_t v, auto ctrl) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+  };
+  x |= ror(x, std::integral_constant<int, kRowRor8>{});
+  x |= ror(x, std::integral_constant<int, kRowRor4>{});
+  x |= ror(x, std::integral_constant<int, kRowRor2>{});
+  x |= ror(x, std::integral_constant<int, kRowRor1>{});
+  return (uint32_t)(__builtin_amdgcn_readlane((int)x, 0) | __builtin_amdgcn_readlane((int)x, 16) |
+                    __builtin_amdgcn_readlane((int)x, 32) | __builtin_amdgcn_readlane((int)x, 48));
+}
+
 // This workgroup's share of the launch's parts that need no votes: counted from the last
 // workgroup down, those of request w % B, as one of the workgroups w % B, w % B + B, ...
 // (The first workgroups of the team merge the statistics, and everybody waits for those; the
@@ -1447,7 +1460,10 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       // need-th largest key is built bit by bit from how many keys reach it, until as many do
       // as are needed: some ten steps, and no barrier (narrowing the entries down by one
       // more digit in LDS took seven of them, and counting the larger keys for every entry
-      // 2-6 us).
+      // 2-6 us).  Equal keys, which a max-pool makes of every peak, are never told apart that
+      // way: after twelve steps it is looked whether the keys that are left are all one (128K
+      // tokens, windows of 15: 5.9 us with a step for every bit of key and position, 3.2 so; one
+      // request of 100K tokens 71.5 -> 69.3 us a layer.  Votes without ties are through before).
       constexpr int kHeld = kSelListCap / 64;
       const uint32_t total = min(scratch[15], (uint32_t)kSelListCap);
       uint2 e[kHeld];
@@ -1460,24 +1476,59 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         for (int i = 0; i < kHeld; ++i) sum += (uint32_t)__popcll(__ballot(pred(e[i])));
         return (uint32_t)__builtin_amdgcn_readfirstlane((int)sum);
       };
+      // The first entry (of the lowest lane that has one) for which `pred` holds.
+      auto first = [&](auto&& pred) {
+        uint2 got = make_uint2(0u, 0u);
+#pragma unroll
+        for (int i = kHeld - 1; i >= 0; --i) {
+          const uint64_t lanes = __ballot(pred(e[i]));
+          if (lanes != 0ull) {
+            const int at = __builtin_ctzll(lanes);
+            got = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)e[i].x, at),
+                             (uint32_t)__builtin_amdgcn_readlane((int)e[i].y, at));
+          }
+        }
+        return got;
+      };
+      // `reach` keys are at least `floor`, and fewer than are wanted are past its next 2 << bit.
       uint32_t floor = (uint32_t)__builtin_amdgcn_readfirstlane((int)(prefix << shift)), reach = total;
       const uint32_t wanted = (uint32_t)__builtin_amdgcn_readfirstlane((int)need);
-      for (int bit = __builtin_amdgcn_readfirstlane(shift) - 1; bit >= 0 && reach != wanted; --bit) {
-        const uint32_t trial = floor | (1u << bit);
-        const uint32_t with = count([&](const uint2& x) { return x.x >= trial; });
-        if (with >= wanted) {
-          floor = trial;
-          reach = with;
+      const int bits = __builtin_amdgcn_readfirstlane(shift);
+      int bit = bits - 1;
+      auto narrow = [&](int last) {
+        for (; bit >= last && reach != wanted; --bit) {
+          const uint32_t trial = floor | (1u << bit);
+          const uint32_t with = count([&](const uint2& x) { return x.x >= trial; });
+          if (with >= wanted) {
+            floor = trial;
+            reach = with;
+          }
         }
+      };
+      narrow(max(bits - 12, 0));
+      if (bit >= 0 && reach != wanted) {
+        const uint32_t one = first([&](const uint2& x) { return x.x - floor < (2u << bit); }).x;
+        if (count([&](const uint2& x) { return x.x == one; }) ==
+            count([&](const uint2& x) { return x.x - floor < (2u << bit); })) {
+          floor = one;
+          bit = -1;
+        }
+        narrow(0);
       }
       kth = floor;
       pos_thr = 0xffffffffu;
-      if (reach > need) {
+      if (reach > wanted) {
         // More ties at the k-th key than places: those at the lowest positions are taken.  The
-        // largest position with which the ties up to it still fit, from the top bit down.
-        const uint32_t places = need - count([&](const uint2& x) { return x.x > kth; });
-        pos_thr = 0u;
-        for (int bit = 31; bit >= 0; --bit) {
+        // largest position with which the ties up to it still fit, from the highest bit in which
+        // the ties' positions differ (there are two at least) down.
+        const uint32_t places = wanted - count([&](const uint2& x) { return x.x > kth; });
+        const uint32_t any = first([&](const uint2& x) { return x.x == kth; }).y;
+        uint32_t differ = 0u;
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) differ |= e[i].x == kth ? e[i].y ^ any : 0u;
+        int bit = 31 - __builtin_clz(wave_or(differ) | 1u);
+        pos_thr = any & ~((2u << bit) - 1u);
+        for (; bit >= 0; --bit) {
           const uint32_t trial = pos_thr | (1u << bit);
           if (count([&](const uint2& x) { return x.x == kth && x.y < trial; }) < places) pos_thr = trial;
         }
