@@ -109,9 +109,9 @@ typedef struct ts_batch {
                                the previous step's as a guess: while the votes of a
                                layer drift slowly from step to step, as the queries
                                do, the selection is then through after one meeting of
-                               its workgroups instead of two (C2: 4 us of 62).  Only
-                               ever a guess: a wrong or stale value costs the saving,
-                               never the result, which is exact either way          */
+                               its workgroups instead of two (C2: 5 us of 60).  Only
+                               ever a guess: a wrong or stale value costs the saving
+                               and some 4 us, never the result, which is exact          */
   /* Per-call options; all zero = the defaults. */
   int32_t separate_kernels; /* 1: this call selects with ts_score + ts_vote +
                                ts_topk_ragged's kernels, whose workgroups never wait
@@ -268,12 +268,14 @@ int ts_topk_ragged(const ts_config* cfg, const ts_batch* bt, const float* votes,
  * The scores stay in LDS.  The softmax statistics need no meeting (the
  * per-workgroup partials and the merged statistics are polled for: the data
  * is its own flag); the workgroups of the launch then meet two to four times:
- * histogram rounds over the 11 + 11 + 10 bits of the vote keys until at most 256 candidates are left around the k-th
- * vote, which are listed and ranked by every workgroup in a last round together
- * with the per-workgroup counts that place its selected positions in the output
- * (masses of exact ties take all three histogram rounds and a count round; one
- * more round with cfg->pool_kernel > 0: the max-pool of tr.py:366-369 needs the
- * votes of the neighbouring workgroups).  Outputs and the hit / cache arguments are those of
+ * histogram rounds over the 11 + 11 + 10 bits of the vote keys until at most 256
+ * candidates are left around the k-th vote, which are listed and ranked by every
+ * workgroup in a last round together with the per-workgroup counts that place its
+ * selected positions in the output (masses of exact ties take all three histogram
+ * rounds and a count round).  With bt->threshold_hint they meet once when the k-th
+ * vote lies near the hint, and once more than without when it does not; with
+ * cfg->pool_kernel > 0 once more in any case: the max-pool of tr.py:366-369 needs
+ * the votes of the neighbouring workgroups.  Outputs and the hit / cache arguments are those of
  * ts_topk_ragged (same tie rule: lowest position first); votes, when not NULL,
  * also receives the [B, vote_stride] fp32 votes (pooled when pool_kernel > 0).
  * Usable when ts_select_supported() returns 1: pool_kernel at most 256 and batch x

@@ -128,6 +128,38 @@ def test_no_call_vouches_for_a_workspace_that_a_graph_uses(dev, stated):
         assert stated[-1] == 1
 
 
+def test_what_ends_the_memory_of_a_clean_workspace(dev, stated):
+    """A call of the same layout states that the workspace is clean; the one after a call of another
+    layout, with a selection cache, with the separate kernels or split at the vote does not."""
+    wl = workloads.build("small", SHAPE, [2048, 901], [256, 256], 16, dev, 63, n_init=16, n_local=32, top_k=256)
+    bt, args = wl.batch, (wl.q, wl.k_pool, wl.v_pool)
+    layer = ops.DecodeLayer(wl.cfg, 2, 2048, dev)
+    one = ops.Batch(bt.seq_lens[:1], bt.table[:1], 2048)
+    short = dataclasses.replace(bt, max_seq_len=1000)
+    cache = ops.SelectionCache.allocate(wl.cfg, 2, dev)
+
+    def split():
+        layer.attend(wl.q, layer.votes(wl.q, wl.k_pool, bt), wl.k_pool, wl.v_pool, bt)
+
+    def refused():
+        with pytest.raises(ValueError):
+            layer(wl.q[:, 1:], wl.k_pool, wl.v_pool, bt)
+
+    between = {"nothing": (lambda: None, 1),
+               "same layout": (lambda: layer(*args, dataclasses.replace(bt, max_seq_len=2047)), 1),
+               "batch": (lambda: layer(wl.q[:1], *args[1:], one), 0), "length": (lambda: layer(*args, short), 0),
+               "cache": (lambda: layer(*args, bt, cache=cache), 0), "split": (split, 0),
+               "separate": (lambda: layer(*args, dataclasses.replace(bt, separate_kernels=True)), 0),
+               "refused before anything ran": (refused, 1)}
+    for name, (call, after) in between.items():
+        layer(*args, bt)
+        layer(*args, bt)
+        assert stated[-1] == 1, name
+        call()
+        layer(*args, bt)
+        assert stated[-1] == after, name
+
+
 @pytest.mark.parametrize("said", [False, True], ids=["full", "caller says clean"])
 def test_replays_and_eager_steps_share_a_workspace(dev, said):
     """A captured step and eager steps of two other shapes on one object, in turn; where the

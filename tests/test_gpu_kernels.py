@@ -1014,8 +1014,8 @@ def test_layer_starts_with_the_selection_on_a_clean_workspace(dev, shape, lens):
     library that its workspace is clean (the attention kernel of the call before cleared the
     selection's counters) and the call starts with the selection kernel, which rotates the
     query itself: selections and outputs bit-identical to those of a fresh object, whose first
-    call runs the rotation kernel, step after step with new queries; a call of another shape,
-    with a selection cache or split at the vote in between makes the next call a full one."""
+    call runs the rotation kernel, step after step with new queries; a call with a selection cache
+    in between makes the next call a full one (what else does: tests/test_gpu_graph.py)."""
     say(f"layer on a clean workspace H={shape['num_heads']} kv={shape['num_kv_heads']} B={len(lens)}")
     wl = small(dev, shape, seed=71, lens=lens, ks=[64] * len(lens))
     c, B = wl.cfg, len(lens)

@@ -103,9 +103,9 @@ __device__ __forceinline__ void grid_poll(uint32_t* sync, uint32_t round, uint64
 }
 
 // Every participating workgroup arrives exactly once per round and waits for the round to
-// complete (a workgroup that needs no more rounds arrives at the rest with grid_arrive_rest).  Each thread first waits for its
-// outstanding memory operations (what it published has been performed by then);
-// thread 0 then counts the workgroup in.  Arrivals are counted in 16 groups:
+// complete (a workgroup that needs no more rounds arrives at the rest with
+// grid_arrive_rest).  Each thread first waits for its outstanding memory operations (what it
+// published has been performed by then); thread 0 then counts the workgroup in.  Arrivals are counted in 16 groups:
 // read-modify-writes of one address are performed one after the other, some 10 ns each, so
 // that a single counter would cost 5 us per round with 500 workgroups.  The workgroup
 // that completes its group's count says so in that group's word of every replica, and
