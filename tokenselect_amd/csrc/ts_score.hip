@@ -1471,9 +1471,15 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       for (int i = 0; i < kHeld; ++i)
         e[i] = (uint32_t)(64 * i + lane) < total ? entries[64 * i + lane] : make_uint2(0u, 0xffffffffu);
       auto count = [&](auto&& pred) {
+        uint64_t lanes[kHeld];
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) lanes[i] = __ballot(pred(e[i]));
+        // (all compared before the first is counted: in turn, through the one VCC, a step takes
+        // half as long again)
+        __builtin_amdgcn_sched_barrier(0);
         uint32_t sum = 0;
 #pragma unroll
-        for (int i = 0; i < kHeld; ++i) sum += (uint32_t)__popcll(__ballot(pred(e[i])));
+        for (int i = 0; i < kHeld; ++i) sum += (uint32_t)__popcll(lanes[i]);
         return (uint32_t)__builtin_amdgcn_readfirstlane((int)sum);
       };
       // The first entry (of the lowest lane that has one) for which `pred` holds.
@@ -1506,7 +1512,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         }
       };
       narrow(max(bits - 12, 0));
-      if (bit >= 0 && reach != wanted) {
+      // (both ways for ties out of line: in the path of the calls without any, their instructions
+      // cost 0.5 us, which is 1 % of three requests' prompts and 8 tokens)
+      if (__builtin_expect(bit >= 0 && reach != wanted, 0)) {
         const uint32_t one = first([&](const uint2& x) { return x.x - floor < (2u << bit); }).x;
         if (count([&](const uint2& x) { return x.x == one; }) ==
             count([&](const uint2& x) { return x.x - floor < (2u << bit); })) {
@@ -1517,7 +1525,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       }
       kth = floor;
       pos_thr = 0xffffffffu;
-      if (reach > wanted) {
+      if (__builtin_expect(reach > wanted, 0)) {
         // More ties at the k-th key than places: those at the lowest positions are taken.  The
         // largest position with which the ties up to it still fit, from the highest bit in which
         // the ties' positions differ (there are two at least) down.
