@@ -129,8 +129,8 @@ typedef struct ts_batch {
                                workgroups counted as members of every rendezvous
                                that never arrive, so that every wait gives up
                                after wait_us while all kernels still exit        */
-  int32_t workspace_clean;  /* ts_decode_layer only.  1: the caller states that this
-                               workspace was last used by a ts_decode_layer call with
+  int32_t workspace_clean;  /* ts_decode_layer and ts_decode_step.  1: the caller states that
+                               this workspace was last used by one of these calls with
                                the same cfg, batch, max_seq_len (or one of the same
                                ts_decode_layer_layout) and cache == NULL that
                                completed without a give-up, and by nothing since (every
@@ -141,7 +141,8 @@ typedef struct ts_batch {
                                the launch that rotates and clears is not needed.  Honoured
                                where the selection is the single ts_select launch and no
                                selection cache is used; ignored otherwise.  A wrong
-                               statement gives wrong selections or waits that give up */
+                               statement gives wrong selections or waits that give up;
+                               one in a call captured into a graph holds for every replay */
 } ts_batch;
 
 /* Default bound of a grid-wide wait: a selection that has the device to itself

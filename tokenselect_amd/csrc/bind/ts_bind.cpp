@@ -6,7 +6,7 @@
 // in Python took 25 us around them, longer than the kernels of a short context run (8 layers
 // of a 2003-token request, 16 calls: 577 us a pass, of which the GPU was busy 290).  Nothing
 // is computed here and nothing is kept between calls but the buffers the object owns and the
-// shape its workspace was last left clean for.
+// layout its workspace was last left clean for.
 //
 // Built with the host compiler against PyTorch's headers; the library's entry points are
 // handed over as addresses by _lib.py, so that there is one loaded copy of it.
@@ -324,7 +324,7 @@ int call_library(Owned& o, ts_batch* bt, const ts_new_kv* kv, const void* q, int
                  int64_t rows, const at::Tensor& k_pool, const at::Tensor& v_pool, const ts_selcache* cache, void* out,
                  bool rerun = false) {
   // The attention kernel of a plain call leaves the selection's counters zero for the next
-  // one of the same shape.
+  // one of the same layout.
   const bool chunk = o.max_rows > 0;
   // (While a graph is captured the object states nothing: the recorded flag would hold for
   // every replay, whatever used the workspace before it.)

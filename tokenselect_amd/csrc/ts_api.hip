@@ -332,7 +332,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   }
   // A decode step without a selection cache whose single-launch selection finds its
   // counters zero (the caller says so: the attention kernel of its previous call, of the
-  // same shape, cleared them on the side) starts with the selection kernel, which rotates
+  // same layout, cleared them on the side) starts with the selection kernel, which rotates
   // the query itself; this call's attention kernel clears the counters again.
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;

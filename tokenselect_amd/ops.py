@@ -806,7 +806,7 @@ class DecodeLayer(_GiveUpLatch):
     def _clean_for(self):
         """(batch, max_seq_len) of the last call when it was a plain layer call without a
         selection cache that raised nothing: that call's attention kernel has left the
-        selection's counters zero, and the next call of the same shape says so
+        selection's counters zero, and the next call of the same layout says so
         (``ts_batch.workspace_clean``) and starts with the selection kernel.  ``None`` for
         good once a call of this object was captured into a graph, whose replays use the
         workspace without its knowledge; a caller who knows what uses the workspace between
