@@ -23,6 +23,7 @@ constexpr int kFpRowGroups = 128;
 constexpr int kFpInFlight = 4;  // rows per step of a row group
 constexpr int kFpVec = 4;       // rotation pairs per thread
 constexpr int kFpSplit = 4;     // workgroups per head
+constexpr int kFpClear = 16;    // workgroups that clear
 constexpr int kFpThreads = kHeadDim / 2 / kFpSplit / kFpVec * kFpRowGroups;
 
 __global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
@@ -38,18 +39,18 @@ __global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
   const int h = blockIdx.x;
   const int first_pair = blockIdx.y * kPairs;
   const int i = first_pair + (threadIdx.x % kLanes) * kFpVec, rg = threadIdx.x / kLanes;
-  // On the side: clear the words the selection kernel after this one counts into.
-  {
-    const int64_t gid = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kFpThreads + threadIdx.x;
-    const int64_t step = (int64_t)gridDim.x * gridDim.y * kFpThreads;
-    clear_regions(zero, gid, step);
-  }
-  // Also on the side: the workgroups past the fingerprint's own store the chunk's K/V
-  // rows (the caller's store of the chunk, which the selection after this launch must find
-  // done, riding here instead of in a launch of its own).
+  // On the side: the workgroups past the fingerprint's own store the chunk's K/V rows (the
+  // caller's store of the chunk, which the selection after this launch must find done, riding here
+  // instead of in a launch of its own), and the last kFpClear of them clear the words that the
+  // selection counts into.
   if ((int)blockIdx.y >= kFpSplit) {
     const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
-    if (cs.k != nullptr && wg < cs.workgroups) store_chunk_rows<true>(cs, wg, kFpThreads);
+    const int stores = cs.k != nullptr ? cs.workgroups : 0;
+    if (wg < stores)
+      store_chunk_rows<true>(cs, wg, kFpThreads);
+    else if (wg < stores + kFpClear)
+      clear_regions(zero, (uint32_t)(wg - stores) * (kFpThreads / 64) + (threadIdx.x >> 6),
+                    kFpClear * (kFpThreads / 64));
     return;
   }
   float lo_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f}, hi_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f};
@@ -717,14 +718,14 @@ int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_
   TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);
   TS_TRY(check_fingerprint(q, rows, cos_table, sin_table, table_rows, qf, cfg->n_local));
   ChunkStore cs{};
-  unsigned grid_y = kFpSplit;
   if (store) {  // 32 threads per row
     cs = *store;
     cs.workgroups = (int)ceil_div(cs.rows, kFpThreads / kChunkThreadsPerRow);
     TS_REQUIRE(cs.workgroups <= kChunkCountedWgs && cs.max_tokens <= kLenMask, TS_EINVAL,
                "internal: a chunk store of %d rows does not ride in the fingerprint launch", cs.rows);
-    grid_y += (unsigned)ceil_div(cs.workgroups, cfg->num_heads);
   }
+  const unsigned grid_y =
+      kFpSplit + (unsigned)ceil_div(cs.workgroups + (zero.used ? kFpClear : 0), cfg->num_heads);
   hipLaunchKernelGGL(fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y), dim3(kFpThreads), 0, stream,
                      (const uint16_t*)q, q_stride, (uint16_t*)qf, cos_table, sin_table, table_rows,
                      cfg->n_local, rows, cfg->num_heads, zero, cs);

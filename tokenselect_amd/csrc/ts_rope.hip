@@ -21,11 +21,11 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
   const int half = dim >> 1;
   const int64_t pairs = rows * heads * half;
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  // Counters the later kernels of a decode step accumulate into.
-  clear_regions(zero, gid, (int64_t)gridDim.x * blockDim.x);
-  if (gid >= pairs) return;
-  const int i = (int)(gid % half);
-  const int64_t rh = gid / half;
+  // (the loads of a thread past the last pair are the last pair's: none of them behind a branch,
+  // and the clearing in between while they travel)
+  const int64_t pair = min(gid, pairs - 1);
+  const int i = (int)(pair % half);
+  const int64_t rh = pair / half;
   const int64_t row = rh / heads;
   int64_t pos = position_ids ? position_ids[row] : 0;
   if (pos < 0) pos = 0;
@@ -36,8 +36,12 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
   const int64_t from = row * x_stride + (rh - row * heads) * dim;
   const float x1 = bf16_to_f32(x[from + i]);
   const float x2 = bf16_to_f32(x[from + i + half]);
-  const float lo = rotate_element(x1, x2, c[i], s[i], true);
-  const float hi = rotate_element(x2, x1, c[i + half], s[i + half], false);
+  const float c1 = c[i], s1 = s[i], c2 = c[i + half], s2 = s[i + half];
+  // Counters the later kernels of a decode step accumulate into.
+  clear_regions(zero, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), gridDim.x * (blockDim.x >> 6));
+  if (gid >= pairs) return;
+  const float lo = rotate_element(x1, x2, c1, s1, true);
+  const float hi = rotate_element(x2, x1, c2, s2, false);
   out[base + i] = f32_to_bf16(lo);
   out[base + i + half] = f32_to_bf16(hi);
 }

@@ -1968,7 +1968,7 @@ const uint32_t* score_votes_fault_word(const ts_config* cfg, int batch, int max_
 }
 
 __global__ __launch_bounds__(256) void select_zero_kernel(ZeroSet zero) {
-  clear_regions(zero, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+  clear_regions(zero, blockIdx.x * 4 + (threadIdx.x >> 6), gridDim.x * 4);
 }
 int launch_select_zero(const ZeroSet& zero, hipStream_t stream) {
   TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
 #pragma clang fp contract(off)
   const int b = blockIdx.x;
   if (b >= batch) {  // the clearing is the other workgroups' job: the decision is a chain of its own
-    clear_regions(zero, (int64_t)(b - batch) * 256 + threadIdx.x, (int64_t)((int)gridDim.x - batch) * 256);
+    clear_regions(zero, (uint32_t)(b - batch) * 4 + (threadIdx.x >> 6), (gridDim.x - (uint32_t)batch) * 4);
     return;
   }
   constexpr int kMaxUnits = kSelCacheMaxVec / 2;
