@@ -140,7 +140,10 @@ typedef struct ts_batch {
                                rotates the query itself (bit-identical to ts_rope_apply);
                                the launch that rotates and clears is not needed.  Honoured
                                where the selection is the single ts_select launch and no
-                               selection cache is used; ignored otherwise.  A wrong
+                               selection cache is used, and by a ts_decode_step whose
+                               requests all attend to everything (its attention kernel's
+                               counters are then known to be zero, and it stores the new
+                               tokens itself); ignored otherwise.  A wrong
                                statement gives wrong selections or waits that give up;
                                one in a call captured into a graph holds for every replay */
 } ts_batch;
@@ -551,7 +554,8 @@ int ts_decode_layer_selection_of(const ts_config* cfg, const ts_batch* bt);
 /* Where a ts_decode_layer call of this shape without a selection cache keeps the counters of its
  * selection, as one number: calls whose numbers are equal (and not negative) keep the same
  * counters in the same places, so that the one may state workspace_clean after the other
- * though their max_seq_len differ.  -1: the selection is not the single ts_select launch. */
+ * though their max_seq_len differ.  -1: neither is the selection the single ts_select launch,
+ * nor is there none (max_seq_len <= n_init + n_local). */
 int64_t ts_decode_layer_layout(const ts_config* cfg, int32_t batch, int32_t max_seq_len);
 size_t ts_decode_layer_workspace_bytes(const ts_config* cfg, int32_t batch, int32_t max_seq_len);
 int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, const float* q_cos,

@@ -108,3 +108,54 @@ def test_growing_context_on_one_workspace(dev, first, steps, B, pool):
         for b, s in enumerate(want[3].tolist()):
             assert torch.equal(got[1][b, :s], want[1][b, :s]) and torch.equal(got[2][b, :s], want[2][b, :s]), (n, b)
         assert torch.equal(got[0], want[0]), n
+
+
+@pytest.mark.parametrize("page", [1, 16], ids=["tokens", "pages"])
+@pytest.mark.parametrize("first,steps", [(0, 3), (126, 4), (637, 8), (2684, 8)])
+def test_steps_on_one_workspace(dev, first, steps, page):
+    """Steps that store their own tokens, over the ends of the sinks, of sinks and window (where a
+    selection's counters begin) and of dense, one object for all against a fresh one at each, whose
+    first call clears everything and stores in a launch of its own: the same bit for bit, the
+    attention apart (other splits: one ulp of the output's rounding).  Request 1 is shorter, and its
+    table is full for the last steps."""
+    say(f"steps from {first}, pages of {page}")
+    cfg = ops.LayerConfig(num_heads=14, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5,
+                          page_size=page)
+    last, B = first + steps, 2
+    room = -(-last // page) * page
+    lengths = [first, max(room - 2 - steps // 2, 0)]
+    g = torch.Generator(device=dev).manual_seed(9)
+    pages = 2 * (room // page) + 2 * steps
+    order = torch.randperm(pages, generator=g, device=dev).to(torch.int32)
+    table = torch.zeros((B, room // page), dtype=torch.int32, device=dev)
+    at = 0
+    for b, n in enumerate(lengths):
+        held = -(-n // page)
+        table[b, :held] = order[at:at + held]
+        at += held
+    free = order[at:].contiguous()
+    start = [torch.randn((pages * page, 2, 128), generator=g, device=dev).bfloat16() for _ in range(2)]
+    sides = []
+    for _ in range(2):
+        count = torch.tensor([free.shape[0]], dtype=torch.int32, device=dev)
+        sides.append(dict(k=start[0].clone(), v=start[1].clone(), table=table.clone(),
+                          lens=torch.tensor(lengths, dtype=torch.int32, device=dev),
+                          pages=ops.PagePool(free.clone(), count, torch.zeros(1, dtype=torch.int32, device=dev))))
+    one = ops.DecodeLayer(cfg, B, max(room, lengths[1]) + 1, dev)
+    one.workspace.fill_(0xa5)
+    for t in range(steps):
+        q, kv = (torch.randn((B, n * 128), generator=g, device=dev).bfloat16() for n in (14, 4))
+        loc = free[2 * t:2 * t + 2].clone()
+        got = []
+        for s, layer in zip(sides, (one, ops.DecodeLayer(cfg, B, max(room, lengths[1]) + 1, dev))):
+            bt = ops.Batch(s["lens"], s["table"], min(max(first, lengths[1]) + t + 1, room))
+            out, sel, sel_pos, sel_len = layer.step(q, kv[:, :256].contiguous(), kv[:, 256:].contiguous(),
+                                                    loc if page == 1 else None, s["k"], s["v"], bt,
+                                                    pages=None if page == 1 else s["pages"])
+            got.append(dict(out=out.clone(), sel=sel, sel_pos=sel_pos, sel_len=sel_len, lens=s["lens"],
+                            table=s["table"], k=s["k"], v=s["v"]))
+        torch.cuda.synchronize()
+        assert not one.gave_up()
+        _same(*got)
+        assert torch.equal(sides[0]["pages"].free_count, sides[1]["pages"].free_count)
+    assert sides[0]["lens"].tolist() == [last, min(lengths[1] + steps, room)]

@@ -172,8 +172,10 @@ int ts_decode_layer_selection_of(const ts_config* cfg, const ts_batch* bt) {
 
 int64_t ts_decode_layer_layout(const ts_config* cfg, int32_t batch, int32_t max_seq_len) {
   if (validate_config(cfg) != TS_OK || batch < 1 || max_seq_len < 1) return -1;
+  // (Lengths of sinks and local window alone have no selection, and its counters no words that are
+  // cleared; what their calls leave zero are the attention's tickets, which lie behind.)
   const SelectWorkspace s = select_workspace(cfg, batch, max_seq_len);
-  if (s.tokens_per_block <= 0) return -1;
+  if (s.tokens_per_block <= 0 && max_seq_len > cfg->n_init + cfg->n_local) return -1;
   // The regions select_zero_regions names follow from the batch, the head count, where the
   // selection's workspace starts, where its last piece does and how many statistics per head
   // are cleared (at most kSelMaxChunks); the offsets are multiples of 256.
@@ -237,14 +239,14 @@ static int32_t attn_list_bound(const ts_config* cfg, const ts_batch* bt, const t
              : max_sel;
 }
 
-// The list that a step's store writes, or sel == NULL where the step is not known to be dense,
-// or where run_layer is going to refuse the call.
+// The list of a step that is known to be dense, for whoever writes it, or sel == NULL where the
+// step is not, or where run_layer is going to refuse the call.
 static DenseList step_list(const ts_config* cfg, const ts_batch* bt, const ts_selcache* cache, const void* q,
                            const float* q_cos, const float* q_sin, const void* out, int32_t* sel, int32_t* sel_pos,
                            int64_t sel_stride, int32_t* sel_len, void* workspace, size_t workspace_bytes) {
   DenseList list{};
   if (validate_config(cfg) != TS_OK || validate_batch(cfg, bt) != TS_OK || !known_dense(cfg, bt, cache) ||
-      cfg->page_size != 1 || !q || !q_cos || !q_sin || !out || !sel || !sel_pos || !sel_len || !workspace ||
+      !q || !q_cos || !q_sin || !out || !sel || !sel_pos || !sel_len || !workspace ||
       (uintptr_t)q % 16 || (uintptr_t)out % 16 || (uintptr_t)workspace % 256)
     return list;
   const LayerWorkspace w = layer_workspace(cfg, bt->batch, bt->max_seq_len);
@@ -253,7 +255,7 @@ static DenseList step_list(const ts_config* cfg, const ts_batch* bt, const ts_se
   list.sel_pos = sel_pos;
   list.sel_stride = sel_stride;
   list.sel_len = sel_len;
-  list.clear = attn_tickets(cfg, bt->batch, attn_list_bound(cfg, bt, cache, w.max_sel), (char*)workspace + w.attn_ws);
+  list.clear = attn_tickets((char*)workspace + w.attn_ws);
   list.clear_per_req = attn_tickets_per_request(cfg);
   list.max_seq_len = bt->max_seq_len;
   return list;
@@ -268,7 +270,8 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                      const ts_selcache* cache, void* out, int32_t* sel, int32_t* sel_pos,
                      int64_t sel_stride, int32_t* sel_len, void* workspace, size_t workspace_bytes,
                      ts_stream_t stream, const StepStore* store = nullptr,
-                     const ChunkStore* chunk_store = nullptr, bool listed = false) {
+                     const ChunkStore* chunk_store = nullptr, bool listed = false,
+                     const AttnDense* dense_step = nullptr) {
   TS_TRY(validate_config(cfg));
   TS_TRY(validate_batch(cfg, bt));
   SeparateKernelsScope separate(bt->separate_kernels != 0);
@@ -310,7 +313,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   const SelectWorkspace fused = select_workspace(cfg, bt->batch, bt->max_seq_len);
   const bool dense = known_dense(cfg, bt, cache) && chunk_store == nullptr;
   const int32_t longest = dense ? attn_list_bound(cfg, bt, cache, w.max_sel) : w.max_sel;
-  uint32_t* tickets = attn_tickets(cfg, bt->batch, longest, ws + w.attn_ws);
+  uint32_t* tickets = attn_tickets(ws + w.attn_ws);
 
   // Fingerprint: every request's single decode row is rotated to n_local
   // (tr.py:381-388); the mean over one row is the row itself (tr.py:392).  The same
@@ -337,6 +340,10 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;
   if (dense) {
+    if (dense_step)  // the attention reads the table, and leaves the list (and the new tokens) itself
+      return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, bt->table, bt->table_stride, bt->seq_lens,
+                         bt->batch, longest, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream, nullptr,
+                         dense_step);
     // (listed: the store has written the selection; otherwise the last of the top-k kernels,
     // which writes a dense request's list, is all that is left of the selection)
     if (chunk_rows > 0) TS_TRY(check_fingerprint(q, chunk_rows, q_cos, q_sin, table_rows, qf, cfg->n_local));
@@ -427,9 +434,41 @@ int ts_decode_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_ne
   if (!rides) {
     DenseList list{};
     if (bt->rerun == 0) {
-      if (kv->pages == nullptr)
-        list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
-                         workspace_bytes);
+      list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
+                       workspace_bytes);
+      if (list.sel && bt->workspace_clean != 0) {
+        // The attention alone (its tickets are zero, as any such call leaves them): the list of a
+        // dense request is its table, and the new row can be read where the caller has it.  With a
+        // page pool the store goes first, since a page is taken in the order of the requests.
+        // 8 layers of a 2003-token request, two steps: 273 -> 215-224 us; 2 layers of a 300-token
+        // prompt with 8 tokens 380 -> 320-350.
+        TS_TRY(check_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool, pool_rows,
+                              table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens));
+        AttnDense step{};
+        step.sel = sel;
+        step.sel_pos = sel_pos;
+        step.sel_stride = sel_stride;
+        step.sel_len = sel_len;
+        step.list_bound = bt->max_seq_len < kv->max_tokens ? bt->max_seq_len : kv->max_tokens;
+        if (kv->pages) {
+          TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
+                                 pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
+                                 (hipStream_t)stream));
+        } else {
+          step.loc = kv->out_cache_loc;
+          step.k = (const uint16_t*)kv->k;
+          step.v = (const uint16_t*)kv->v;
+          step.k_from_pool = ((intptr_t)kv->k - (intptr_t)k_pool) / 2;  // (both aligned to 16 bytes)
+          step.v_from_pool = ((intptr_t)kv->v - (intptr_t)v_pool) / 2;
+          step.kv_stride = kv_row_stride ? kv_row_stride : cfg->num_kv_heads * cfg->head_dim;
+          step.table = table;
+          step.seq_lens = seq_lens;
+          step.max_tokens = kv->max_tokens;
+        }
+        return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
+                         sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, true, &step);
+      }
+      if (kv->pages) list = DenseList{};  // (a paged store writes no list)
       TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
                              pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
                              (hipStream_t)stream, list.sel ? &list : nullptr));
@@ -579,7 +618,7 @@ int ts_decode_layer_attend(const ts_config* cfg, const ts_batch* bt, const void*
   }
   TopkArgs topk = make_topk_args(cfg, bt, ranked, ranked_stride, hit, cache, sel, sel_pos, sel_stride,
                                  sel_len, (uint32_t*)(ws + w.topk_ws));
-  topk.clear = attn_tickets(cfg, bt->batch, w.max_sel, ws + w.attn_ws);
+  topk.clear = attn_tickets(ws + w.attn_ws);
   topk.clear_per_req = attn_tickets_per_request(cfg);
   ts_config plain = *cfg;
   plain.pool_kernel = -1;
@@ -624,7 +663,7 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
   DenseList list{};
   if (kv->pages == nullptr && bt->rerun == 0 &&
       chunk_store_takes_list(rows, kv->max_tokens, bt->max_seq_len) &&
-      table_rows >= (int64_t)cfg->n_local + rows && (uintptr_t)cos_table % 16 == 0 &&
+      cfg->page_size == 1 && table_rows >= (int64_t)cfg->n_local + rows && (uintptr_t)cos_table % 16 == 0 &&
       (uintptr_t)sin_table % 16 == 0)
     list = step_list(cfg, bt, nullptr, q, cos_table, sin_table, out, sel, sel_pos, sel_stride, sel_len, workspace,
                      workspace_bytes);

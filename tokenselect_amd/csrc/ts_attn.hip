@@ -5,7 +5,8 @@
 // the request's selected list for one KV head and all G = H/Hkv query heads that read it;
 // its four wavefronts walk a quarter of the range each, in tiles of 32 tokens, on the
 // matrix cores (see attn_kernel).  Keys are rotated to their index in the selected list,
-// the query to S-1; softmax is online in fp32.  Partial (max, sum, acc) triples are merged
+// the query to S-1; softmax is online in fp32.  A dense decode step on a per-token or paged
+// table is this one launch (AttnDense): the list is the table itself.  Partial (max, sum, acc) triples are merged
 // across the wavefronts, written with device-coherent stores, and the workgroup that draws
 // the last ticket of its (request, KV head) merges the splits and writes the bf16 output.
 #include <math.h>
@@ -33,9 +34,13 @@ struct AttnArgs {
   int nsplit, max_sel_len;
   float* part_acc;    // [B,H,nsplit,128]
   float* part_ml;     // [B,H,nsplit,2]
-  uint32_t* tickets;  // [B,Hkv], zero at launch and again when the kernel ends
+  uint32_t* tickets;  // [B][Hkv + 1], zero at launch and again when the kernel ends
   uint16_t* out;      // [B,H,128] bf16
   ZeroSet zero;       // cleared on the side (counters of the stream's next selection)
+  // A dense step (AttnDense): sel is the table, in pages of 1 << list_shift, sel_len the lengths;
+  // list_bound: positions whose entries are there to be read.
+  int list_shift, list_bound;
+  AttnDense step;
 };
 
 // The last three wavefronts' share of the regions to clear.
@@ -59,12 +64,57 @@ __device__ __forceinline__ void store_coherent2(float* p, float x, float y) {
   __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Whether a request's new token is stored: what the store kernels ask (ts_store.hip).
+__device__ __forceinline__ bool attn_appends(const AttnArgs& a, int slot, int len) {
+  return a.step.loc != nullptr && (uint32_t)slot < a.pool_rows && len >= 0 && len < a.step.max_tokens;
+}
+
+// What a dense step leaves behind besides the output, after a workgroup's share of the attention:
+// the new token's row of this KV head in the pool (by the workgroup whose range holds it), the
+// list (by the workgroups of the first KV head), and, by the last workgroup of the request's last
+// KV head (`last`), when all of them have read the length, the table's entry and the length.
+// Nobody waits for any of it in this launch: the new row was read where the caller has it.
+__device__ __forceinline__ void attn_dense_epilogue(const AttnArgs& a, int b, int kvh, int lo, int hi, int S,
+                                                    int slot, int len, bool ok, bool last) {
+  const int tid = threadIdx.x;
+  if (ok && lo <= len && len < hi && tid < 2 * (kHeadDim / 8)) {
+    const bool is_v = tid >= kHeadDim / 8;
+    const int at = 8 * (tid % (kHeadDim / 8));
+    const uint16_t* row = (is_v ? a.step.v : a.step.k) + (size_t)b * a.step.kv_stride + kvh * kHeadDim + at;
+    uint16_t* to = (uint16_t*)(is_v ? a.v_pool : a.k_pool) + ((size_t)slot * a.num_kv_heads + kvh) * kHeadDim + at;
+    *(uint4*)to = *(const uint4*)row;
+  }
+  if (kvh == 0) {
+    const int32_t* tab = a.sel + (int64_t)b * a.sel_stride;
+    int32_t* const sel = a.step.sel + (int64_t)b * a.step.sel_stride;
+    int32_t* const sel_pos = a.step.sel_pos + (int64_t)b * a.step.sel_stride;
+    for (int pos = lo + tid; pos < min(hi, S); pos += 256) {
+      const uint32_t entry = ((uint32_t)tab[min(pos, a.list_bound - 1) >> a.list_shift] << a.list_shift) +
+                             (uint32_t)(pos & ((1 << a.list_shift) - 1));
+      sel_pos[pos] = pos;
+      sel[pos] = ok && pos == len ? slot : (int32_t)min(entry, a.pool_rows - 1);
+    }
+  }
+  if (last && tid == 0) {
+    uint32_t* const heads = a.tickets + (size_t)b * (a.num_kv_heads + 1) + a.num_kv_heads;
+    if (__hip_atomic_fetch_add(heads, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
+        (uint32_t)a.num_kv_heads) {
+      __hip_atomic_store(heads, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      a.step.sel_len[b] = S;
+      if (ok) {
+        a.step.table[(int64_t)b * a.sel_stride + len] = slot;
+        a.step.seq_lens[b] = len + 1;
+      }
+    }
+  }
+}
+
 // The end of an attention workgroup: its four wavefronts' partial (max, sum, acc) triples
 // of G head slots lie in LDS; they are merged, written with device-coherent stores, and the
 // workgroup that draws the last ticket of its (request, KV head) merges the splits and
-// writes the bf16 output.
+// writes the bf16 output.  Whether this was that workgroup.
 template <int G>
-__device__ __forceinline__ void attn_finish(const AttnArgs& a, int b, int kvh, int split,
+__device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, int split,
                                             float (*sm_acc)[G][kHeadDim], float (*sm_m)[G],
                                             float (*sm_l)[G], uint32_t* s_last_ptr) {
   const int tid = threadIdx.x, lane = tid & 63;
@@ -94,7 +144,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int b, int kvh, i
   // Ticket: the stores above are acknowledged before the workgroup is counted.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  uint32_t* ticket = a.tickets + (size_t)b * a.num_kv_heads + kvh;
+  uint32_t* ticket = a.tickets + (size_t)b * (a.num_kv_heads + 1) + kvh;
   if (tid == 0) {
     const uint32_t before =
         __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -105,7 +155,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int b, int kvh, i
     attn_clear_on_the_side(a);
   }
   __syncthreads();
-  if (!s_last) return;
+  if (!s_last) return false;
 
   // out[b,h,:] = sum_s exp(m_s - M) acc_s / sum_s exp(m_s - M) l_s, rounded to bf16.
   // A wavefront per head slot (a thread owns two adjacent dims, and a head has 64 such
@@ -174,10 +224,11 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int b, int kvh, i
     }
   }
   if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
 }
 
 // ---------------------------------------------------------------------------------------
-// attn_kernel<G, ROPE, CAP>: G = H / Hkv query heads per workgroup (1 to 8), on the matrix
+// attn_kernel<G, ROPE, CAP, DENSE>: G = H / Hkv query heads per workgroup (1 to 8), on the matrix
 // cores.  A wavefront walks a contiguous quarter of the workgroup's range in tiles of 32
 // tokens.  v_mfma_f32_16x16x32_bf16 three times over:
 //   logits   S[token][head] = K' Q'^T : A = 16 rotated keys x 32 dims (lane (token l%16,
@@ -206,6 +257,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int b, int kvh, i
 typedef __attribute__((ext_vector_type(8))) __bf16 at_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float at_f32x4;
 constexpr float kAttnLog2e = 1.4426950408889634f, kAttnLn2 = 0.6931471805599453f;
+constexpr uint32_t kNewRow = 0xffffffffu;  // the slot of a row that is not in the pool (no pool has as many)
 constexpr int kAttnTile = 32;        // tokens per step of a wavefront
 constexpr int kAttnChunkUnit = 64;   // a workgroup's range is a multiple of this (16 per wavefront)
 
@@ -251,7 +303,9 @@ __device__ __forceinline__ int opaque_zero(uint32_t after) {
   return z;
 }
 
-template <int G, bool ROPE, bool CAP>
+// DENSE (AttnDense) is an instantiation of its own: with its few instructions in the one kernel the
+// attention over a list took 1 us more.
+template <int G, bool ROPE, bool CAP, bool DENSE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_kernel(AttnArgs a) {
   static_assert(G >= 1 && G <= 8, "the query heads of a KV head are columns of one tile");
   const int split = blockIdx.x, b = blockIdx.z, kvh = blockIdx.y;
@@ -289,31 +343,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // An entry past the wavefront's range (its token gets the weight zero) is replaced by the
   // slot of the range's first token: its row must still be one that holds numbers.
   const int wlo = split * chunk + wave * wlen;
-  auto raw_slot = [&](int j) { return (uint32_t)sel[min(j, a.max_sel_len - 1)]; };
+  auto raw_slot = [&](int j) {
+    if (!DENSE) return (uint32_t)sel[min(j, a.max_sel_len - 1)];
+    return ((uint32_t)sel[min(j, a.list_bound - 1) >> a.list_shift] << a.list_shift) +
+           (uint32_t)(j & ((1 << a.list_shift) - 1));
+  };
   uint32_t slot_cur[2] = {raw_slot(wlo + n), raw_slot(wlo + 16 + n)};
   uint32_t slot_next[2] = {raw_slot(wlo + kAttnTile + n), raw_slot(wlo + kAttnTile + 16 + n)};
-  const int S = min(max(a.sel_len[b], 0), a.max_sel_len);
+  // A dense step's list is the table and, at the end, the new token, whose row is not in the pool
+  // yet: it is read where the caller has it, as slot kNewRow.  (With no new token some word that can
+  // be read is loaded in place of its slot.)
+  const int length = a.sel_len[b];
+  const int new_slot = DENSE ? (a.step.loc ? a.step.loc : a.sel_len)[b] : -1;
+  const bool appends = DENSE && attn_appends(a, new_slot, length);
+  const int new_pos = appends ? length : -1;
+  const int S = min(max(length + (appends ? 1 : 0), 0), DENSE ? a.list_bound : a.max_sel_len);
   const int whi = min(S, wlo + wlen);
-  const uint32_t first_slot =
+  uint32_t first_slot =
       min((uint32_t)__builtin_amdgcn_readfirstlane((int)slot_cur[0]), a.pool_rows - 1);
-  auto checked = [&](uint32_t slot, int j) { return j < whi && slot < a.pool_rows ? slot : first_slot; };
+  if (DENSE && wlo == new_pos) first_slot = kNewRow;
+  auto checked = [&](uint32_t slot, int j) {
+    if (!DENSE) return j < whi && slot < a.pool_rows ? slot : first_slot;
+    if (j == new_pos) return kNewRow;
+    return j < whi ? min(slot, a.pool_rows - 1) : first_slot;  // (an entry that is no slot: as it is listed)
+  };
   slot_cur[0] = checked(slot_cur[0], wlo + n);
   slot_cur[1] = checked(slot_cur[1], wlo + 16 + n);
   slot_next[0] = checked(slot_next[0], wlo + kAttnTile + n);
   slot_next[1] = checked(slot_next[1], wlo + kAttnTile + 16 + n);
   // ... and the first tile's rows before the set-up below, which then runs while they travel.
   uint4 kr[2][4], vr[2][4];
-  auto request = [&](const uint16_t* pool, const uint32_t* slots, uint4 (&dst)[2][4]) {
+  // (from_new: elements from the pool to the new token's row)
+  auto request = [&](const uint16_t* pool, int64_t from_new, const uint32_t* slots, uint4 (&dst)[2][4]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const uint16_t* row = pool + (size_t)slots[t] * row_elems + (size_t)kvh * kHeadDim + 8 * qd;
+      size_t at = (size_t)slots[t] * row_elems;
+      if (DENSE && slots[t] == kNewRow) at = (size_t)from_new;
+      const uint16_t* row = pool + at + (size_t)kvh * kHeadDim + 8 * qd;
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) dst[t][kb] = *(const uint4*)(row + 32 * kb);
     }
   };
+  const int64_t new_k = a.step.k_from_pool + (int64_t)b * a.step.kv_stride;
+  const int64_t new_v = a.step.v_from_pool + (int64_t)b * a.step.kv_stride;
   // (a wavefront without tokens asks too: rows of some entry of the list, never used)
-  request(a.k_pool, slot_cur, kr);
-  request(a.v_pool, slot_cur, vr);
+  request(a.k_pool, new_k, slot_cur, kr);
+  request(a.v_pool, new_v, slot_cur, vr);
 
   if (tid < kHeadDim / 2) {
     float sn = 0.f, cs = 1.f;
@@ -458,7 +533,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       }
       // the next tile's keys, into the registers just read
-      if (more) request(a.k_pool, slot_next, kr);
+      if (more) request(a.k_pool, new_k, slot_next, kr);
       __builtin_amdgcn_sched_barrier(0);
       // ---- weights of 32 tokens x 16 head columns
       float p[8];
@@ -518,7 +593,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       __builtin_amdgcn_sched_barrier(0);
       if (more) {
-        request(a.v_pool, slot_next, vr);
+        request(a.v_pool, new_v, slot_next, vr);
         slot_next[0] = checked(slot_after[0], j0 + 2 * kAttnTile + n);
         slot_next[1] = checked(slot_after[1], j0 + 2 * kAttnTile + 16 + n);
       }
@@ -546,15 +621,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       sm_l[wave][n] = l;
     }
   }
-  attn_finish<G>(a, b, kvh, split, sm_acc, sm_m, sm_l, &s_last);
+  const bool last = attn_finish<G>(a, b, kvh, split, sm_acc, sm_m, sm_l, &s_last);
+  if (DENSE) attn_dense_epilogue(a, b, kvh, split * chunk, (split + 1) * chunk, S, new_slot, length, appends, last);
 }
 
 __global__ __launch_bounds__(256) void attn_zero_kernel(uint32_t* tickets, int count) {
   for (int i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) tickets[i] = 0u;
 }
 
-// Tickets per request (the words to clear): one per KV head.
-int attn_tickets_per_request(const ts_config* cfg) { return cfg->num_kv_heads; }
+// Tickets per request (the words to clear): one per KV head, and one for the heads of a dense step.
+int attn_tickets_per_request(const ts_config* cfg) { return cfg->num_kv_heads + 1; }
 
 constexpr int kAttnRange = 128;  // list entries per workgroup as long as the device has room
 static int attn_splits(int batch, int num_kv_heads, int max_sel_len) {
@@ -569,23 +645,23 @@ static int attn_splits(int batch, int num_kv_heads, int max_sel_len) {
   return (int)ceil_div(max_sel_len, attn_chunk(max_sel_len, (int)want));
 }
 
+// The tickets come first, where they lie whatever the length of the lists: a completed call of any
+// of them leaves the words of the next one zero.
 struct AttnWorkspace {
-  size_t acc, ml, tickets, total;
+  size_t tickets, acc, ml, total;
 };
 static AttnWorkspace attn_workspace(const ts_config* cfg, int batch, int max_sel_len) {
-  const size_t ns = (size_t)attn_splits(batch, attn_tickets_per_request(cfg), max_sel_len);
+  const size_t ns = (size_t)attn_splits(batch, cfg->num_kv_heads, max_sel_len);
   const size_t heads = (size_t)batch * cfg->num_heads;
   AttnWorkspace w;
-  w.acc = 0;
+  w.tickets = 0;
+  w.acc = align_up((size_t)batch * attn_tickets_per_request(cfg) * 4, 256);
   w.ml = w.acc + align_up(heads * ns * kHeadDim * 4, 256);
-  w.tickets = w.ml + align_up(heads * ns * 2 * 4, 256);
-  w.total = w.tickets + align_up((size_t)batch * attn_tickets_per_request(cfg) * 4, 256);
+  w.total = w.ml + align_up(heads * ns * 2 * 4, 256);
   return w;
 }
 
-uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* workspace) {
-  return (uint32_t*)((char*)workspace + attn_workspace(cfg, batch, max_sel_len).tickets);
-}
+uint32_t* attn_tickets(void* workspace) { return (uint32_t*)workspace; }
 
 size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
   return attn_workspace(cfg, batch, max_sel_len).total;
@@ -594,9 +670,17 @@ size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
-                hipStream_t st, const ZeroSet* clear_after) {
+                hipStream_t st, const ZeroSet* clear_after, const AttnDense* dense) {
   const AttnWorkspace w = attn_workspace(cfg, batch, max_sel_len);
   AttnArgs a;
+  a.step = AttnDense{};
+  a.list_shift = a.list_bound = 0;
+  if (dense) {
+    a.step = *dense;
+    a.list_shift = page_shift_of(cfg->page_size);
+    a.list_bound = dense->list_bound;
+    TS_REQUIRE(!dense->loc || a.list_shift == 0, TS_EINVAL, "internal: a dense step appends to per-token tables only");
+  }
   if (clear_after) {
     TS_REQUIRE(!clear_after->overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch",
                kZeroRegions);
@@ -618,7 +702,7 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
   a.rope_rcp_scale = cfg->rope_mode == TS_ROPE_LLAMA ? 1.0f / cfg->rope_scale : 1.0f;
   a.sm_scale = cfg->sm_scale;
   a.logit_cap = cfg->logit_cap;
-  a.nsplit = attn_splits(batch, attn_tickets_per_request(cfg), max_sel_len);
+  a.nsplit = attn_splits(batch, cfg->num_kv_heads, max_sel_len);
   a.max_sel_len = max_sel_len;
   a.part_acc = (float*)((char*)workspace + w.acc);
   a.part_ml = (float*)((char*)workspace + w.ml);
@@ -631,9 +715,13 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
                        a.tickets, count);
     TS_TRY(check_launch("attn_zero_kernel"));
   }
-  const dim3 grid((unsigned)a.nsplit, (unsigned)attn_tickets_per_request(cfg), (unsigned)batch);
+  const dim3 grid((unsigned)a.nsplit, (unsigned)cfg->num_kv_heads, (unsigned)batch);
   const bool rope = cfg->rope_mode == TS_ROPE_LLAMA, cap = cfg->logit_cap > 0.f;
-#define TS_ATTN_LAUNCH(G_, R_, C_) hipLaunchKernelGGL((attn_kernel<G_, R_, C_>), grid, dim3(256), 0, st, a)
+#define TS_ATTN_LAUNCH(G_, R_, C_)                                                                    \
+  do {                                                                                                \
+    if (dense) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, true>), grid, dim3(256), 0, st, a);        \
+    else hipLaunchKernelGGL((attn_kernel<G_, R_, C_, false>), grid, dim3(256), 0, st, a);             \
+  } while (0)
 #define TS_ATTN_CASE(G_)                              \
   case G_:                                            \
     if (rope && cap) TS_ATTN_LAUNCH(G_, true, true);  \

@@ -172,6 +172,11 @@ struct DenseList {
   int max_seq_len;
 };
 
+// What ts_kv_store requires of its arguments.
+int check_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride, const int32_t* out_cache_loc,
+                   const ts_page_pool* pages, const void* k_pool, const void* v_pool, int64_t pool_rows,
+                   const int32_t* table, int64_t table_stride, const int32_t* seq_lens, int32_t batch,
+                   int32_t max_tokens);
 // ts_kv_store and ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
 int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                     const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
@@ -195,16 +200,34 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
 // (request, KV head) tickets inside the workspace, which must be zero at launch:
 // tickets_clear = false makes the launcher clear them first, true says an earlier
 // kernel of the stream already did (attn_tickets() tells it where they are).
-uint32_t* attn_tickets(const ts_config* cfg, int batch, int max_sel_len, void* workspace);
+uint32_t* attn_tickets(void* workspace);
 size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len);
-// Tickets per request (the words to clear): one per KV head.
+// Tickets per request (the words to clear).
 int attn_tickets_per_request(const ts_config* cfg);
 // clear_after: regions that the kernel clears on the side (the counters of the stream's
 // next selection), or NULL.
+// dense: a decode step whose requests attend to all their tokens, in this launch alone; `sel` is
+// then the table in pages of cfg's size and sel_len the lengths before the step's append.
+struct AttnDense {
+  int32_t* sel;      // the selection that is left behind: every position, the new one included
+  int32_t* sel_pos;
+  int64_t sel_stride;
+  int32_t* sel_len;
+  int list_bound;    // entries that are there to be read, whatever the length
+  // The new tokens (loc == NULL: none, the lengths count them already), one per request.
+  const int32_t* loc;
+  const uint16_t* k;  // [B, Hkv*128] bf16, rows kv_stride elements apart
+  const uint16_t* v;
+  int64_t k_from_pool, v_from_pool;  // elements from the pools to them
+  int kv_stride;
+  int32_t* table;    // sel and sel_len of the launch, to be written
+  int32_t* seq_lens;
+  int max_tokens;
+};
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
-                hipStream_t stream, const ZeroSet* clear_after = nullptr);
+                hipStream_t stream, const ZeroSet* clear_after = nullptr, const AttnDense* dense = nullptr);
 
 constexpr int kHeadDim = 128;
 constexpr float kNegBig = -3.0e38f;  // finite stand-in for -inf in running maxima

@@ -15,7 +15,8 @@ namespace ts {
 // first.  A dense step then has two launches, this (2.2 us) and the attention, where it had
 // a store (1.7), a selection kernel or a rotation and a list (3.3 to 4.6) and the attention:
 // 8 layers of a 2003-token request, two steps, 320 -> 261 us; 2 layers of a 300-token prompt
-// with 8 tokens 430 -> 368 us.
+// with 8 tokens 430 -> 368 us.  (Once the caller can say that the attention's tickets are zero, the
+// attention stores the row and writes the list itself, and this form serves the calls before.)
 constexpr int kListThreads = 1024;  // one request's few thousand entries in a handful of steps
 constexpr int kListAhead = 4;       // table entries a thread asks for before it knows the length
 
@@ -235,10 +236,10 @@ static int check_pool_arg(const ts_config* cfg, const int32_t* out_cache_loc, co
   return TS_OK;
 }
 
-int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
-                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
-                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
-                    int32_t max_tokens, hipStream_t stream, const DenseList* list) {
+int check_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride, const int32_t* out_cache_loc,
+                   const ts_page_pool* pages, const void* k_pool, const void* v_pool, int64_t pool_rows,
+                   const int32_t* table, int64_t table_stride, const int32_t* seq_lens, int32_t batch,
+                   int32_t max_tokens) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_lens, TS_EINVAL,
              "ts_kv_store: NULL tensor argument");
@@ -253,8 +254,16 @@ int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t 
   TS_REQUIRE(batch == 1 || table_stride * (int64_t)cfg->page_size >= max_tokens, TS_EINVAL,
              "ts_kv_store: table_stride %lld x page_size %d < max_tokens %d", (long long)table_stride,
              cfg->page_size, max_tokens);
+  return check_row_stride(row_stride, (int64_t)cfg->num_kv_heads * cfg->head_dim, "ts_kv_store");
+}
+
+int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
+                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
+                    int32_t max_tokens, hipStream_t stream, const DenseList* list) {
+  TS_TRY(check_kv_store(cfg, k, v, row_stride, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride,
+                        seq_lens, batch, max_tokens));
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store"));
   const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
   TS_REQUIRE(list == nullptr || pages == nullptr, TS_EINVAL, "internal: a list needs a per-token table");
   if (pages) {
