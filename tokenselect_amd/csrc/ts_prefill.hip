@@ -206,20 +206,34 @@ constexpr float kPfRaise = 8.0f;       // a row's maximum is raised when a logit
 // and the next one wants those 8 as one 16-byte operand, in the order 4 kb + r.
 __device__ __forceinline__ int kv_pos(int kk) { return 8 * ((kk >> 2) & 3) + 4 * (kk >> 4) + (kk & 3); }
 
-// Grid (32-key tiles, KV heads).  Thread (key kk, chunk c) moves dims [8c, 8c+8) and
+// 16 bytes of the staging area.  With eight KV heads the workgroup that gathers a head's keys runs
+// on the XCD whose workgroups attend to them (the KV head is the fastest index of both grids), and
+// what it leaves in that XCD's L2 is read from there.  With fewer, several XCDs read a head, most of
+// what is written waits in the wrong L2, and the writes go past it.  Gather + attention, us: 28 heads
+// on 4 7.75 + 24.8 with the tile as the fastest index, 6.6 + 24.6 with the head, 5.6 + 24.8 past the
+// L2 as well; 32 on 8 7.4 + 27.4, 6.5 + 27.6, 6.7 + 28.3.
+typedef __attribute__((ext_vector_type(4))) unsigned int pf_u32x4;
+__device__ __forceinline__ void stage(const PrefillArgs& a, void* to, const uint4& w) {
+  if (a.num_kv_heads < 8)
+    __builtin_nontemporal_store(__builtin_bit_cast(pf_u32x4, w), (pf_u32x4*)to);
+  else
+    *(uint4*)to = w;
+}
+
+// Grid (KV heads, 32-key tiles).  Thread (key kk, chunk c) moves dims [8c, 8c+8) and
 // [64+8c, +8) of key j = tile + kk.  Keys past S are written as zeros.
 __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t vt_lds[kHeadDim * kPfVRow];
   const int tid = threadIdx.x;
   const int kk = tid >> 3, c8 = tid & 7;
-  const int kvh = blockIdx.y;
-  const int j = blockIdx.x * kPfKeys + kk;
+  const int kvh = blockIdx.x;
+  const int j = blockIdx.y * kPfKeys + kk;
   // (the slot is asked for together with the length, not after it)
   uint32_t slot = (uint32_t)a.sel[min(j, a.max_sel_len - 1)];
   const int S = min(max(*a.sel_len, 0), a.max_sel_len);
   // Whole blocks of kPfPadKeys: the keys between S and the next multiple are written as
   // zeros too (their weights are zero, but 0 x garbage is not).
-  if (blockIdx.x * kPfKeys >= (S + kPfPadKeys - 1) / kPfPadKeys * kPfPadKeys) return;
+  if (blockIdx.y * kPfKeys >= (S + kPfPadKeys - 1) / kPfPadKeys * kPfPadKeys) return;
   const bool live = j < S;
   uint4 kraw[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
   uint4 vraw[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
@@ -254,12 +268,12 @@ __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
     }
   }
   // key kk = 16 kb + qc, dims 32 ks + 8 g4: operand 4 kb + ks, lane 16 g4 + qc
-  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)blockIdx.x * kPfKeys) * kHeadDim;
+  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)blockIdx.y * kPfKeys) * kHeadDim;
   uint16_t* kout = a.kr + tile_at + ((4 * (kk >> 4) + (c8 >> 2)) * 64 + 16 * (c8 & 3) + (kk & 15)) * 8;
-  *(uint4*)kout = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]),
-                                        pack_bf16(lo[4], lo[5]), pack_bf16(lo[6], lo[7]));
-  *(uint4*)(kout + 2 * 64 * 8) = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
-                                             pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
+  stage(a, kout, make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
+                            pack_bf16(lo[6], lo[7])));
+  stage(a, kout + 2 * 64 * 8, make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
+                                         pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7])));
   // transpose the 32 x 128 V tile through LDS (key kk to column kv_pos(kk)), then write its
   // eight operands: piece p is lane p % 64 of operand p / 64, dim 16 (p / 64) + p % 16,
   // columns [8 g4, +8) with g4 = p % 64 / 16
@@ -278,7 +292,7 @@ __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int p = tid + 256 * i;
-    vout[p] = *(const uint4*)(vt_lds + (16 * (p >> 6) + (p & 15)) * kPfVRow + 8 * ((p >> 4) & 3));
+    stage(a, vout + p, *(const uint4*)(vt_lds + (16 * (p >> 6) + (p & 15)) * kPfVRow + 8 * ((p >> 4) & 3)));
   }
 }
 
@@ -774,7 +788,7 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
   a.vt = (uint16_t*)((char*)workspace + need / 2);
   a.out = (uint16_t*)out;
   hipStream_t st = stream;
-  hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)(a.s_pad / kPfKeys), (unsigned)cfg->num_kv_heads),
+  hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)cfg->num_kv_heads, (unsigned)(a.s_pad / kPfKeys)),
                      dim3(256), 0, st, a);
   TS_TRY(check_launch("prefill_gather_kernel"));
   const int group = cfg->num_heads / cfg->num_kv_heads;
