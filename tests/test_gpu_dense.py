@@ -159,3 +159,90 @@ def test_steps_on_one_workspace(dev, first, steps, page):
         _same(*got)
         assert torch.equal(sides[0]["pages"].free_count, sides[1]["pages"].free_count)
     assert sides[0]["lens"].tolist() == [last, min(lengths[1] + steps, room)]
+
+
+@pytest.mark.parametrize("case", ["one", "page begins", "page goes on", "batch", "batch of pages", "70 requests",
+                                  "no window", "foreign slot", "bad page", "no page left", "table full",
+                                  "own k", "separate kernels", "votes form", "pooled"])
+def test_a_step_stores_as_the_store_does(dev, case):
+    """A step whose launches score or rotate and store on the side, against ts_kv_store and the
+    layer on a fresh object: lengths, tables, pools, free pages, selections and outputs bit for bit,
+    over the first call (which rotates) and those that start with the selection."""
+    say(f"step that stores on the side: {case}")
+    page = 16 if "page" in case else 1
+    B = {"batch": 4, "batch of pages": 5, "70 requests": 70, "no page left": 3, "own k": 2}.get(case, 1)
+    if case in ("foreign slot", "bad page", "table full"):
+        B = 2
+    lengths = [3200 - 7 * b for b in range(B)]
+    if case == "page begins":
+        lengths = [3200]
+    if case == "page goes on":
+        lengths = [3205]
+    if case in ("batch", "own k"):
+        lengths[1] = 300  # dense among others
+    if case in ("batch of pages", "bad page", "no page left"):
+        lengths = [3200 + 16 * b for b in range(B)]
+        lengths[-1] += 3
+    top_k = 256 if case == "70 requests" else 1024
+    if case == "votes form":
+        lengths, B = [40000] * 9, 9
+    cfg = ops.LayerConfig(num_heads=32 if case == "votes form" else 8, num_kv_heads=8 if case == "votes form" else 2,
+                          n_init=16, n_local=0 if case == "no window" else 64, top_k=top_k, rope_theta=5e5,
+                          page_size=page, pool_kernel=5 if case == "pooled" else -1)
+    steps, H, row = 3, cfg.num_heads, cfg.num_kv_heads * 128
+    g = torch.Generator(device=dev).manual_seed(12)
+    width = (max(lengths) + steps) // page + 1
+    if case == "table full":
+        width = max(lengths) + 1  # (one more token of request 0; request 1 goes on)
+    held = [-(-n // page) for n in lengths]
+    pages = sum(held) + B * steps
+    order = torch.randperm(pages, generator=g, device=dev).to(torch.int32)
+    table, at = torch.zeros((B, width), dtype=torch.int32, device=dev), 0
+    for b, n in enumerate(held):
+        table[b, :n] = order[at:at + n]
+        at += n
+    free = order[at:].contiguous()
+    if case == "bad page":
+        free[-1] = pages + 5
+    count = 1 if case == "no page left" else free.shape[0]
+    start = [torch.randn((pages * page, cfg.num_kv_heads, 128), generator=g, device=dev).bfloat16() for _ in range(2)]
+    sides = [dict(k=start[0].clone(), v=start[1].clone(), table=table.clone(),
+                  lens=torch.tensor(lengths, dtype=torch.int32, device=dev),
+                  hint=torch.zeros(B, dtype=torch.int32, device=dev),
+                  pages=ops.PagePool(free.clone(), torch.tensor([count], dtype=torch.int32, device=dev),
+                                     torch.zeros(1, dtype=torch.int32, device=dev))) for _ in range(2)]
+    longest = min(max(lengths) + steps, width * page)
+    one = ops.DecodeLayer(cfg, B, longest, dev)
+    one.workspace.fill_(0xa5)
+    kpr = torch.tensor([700, 256][:B], dtype=torch.int32, device=dev) if case == "own k" else None
+    for t in range(steps):
+        q = torch.randn((B, H * 128), generator=g, device=dev).bfloat16()
+        kv = torch.randn((2, B, row), generator=g, device=dev).bfloat16()
+        loc = None
+        if page == 1:
+            loc = free[t * B:t * B + B].clone()
+            if case == "foreign slot":
+                loc[1 - t % 2] = start[0].shape[0] if t else -1
+        got = []
+        for s, whole in zip(sides, (True, False)):
+            most = min(max(lengths) + t + 1, width * page)
+            bt = ops.Batch(s["lens"], s["table"], most, k_per_req=kpr, hint=s["hint"],
+                           separate_kernels=case == "separate kernels")
+            if whole:
+                out, sel, sel_pos, sel_len = one.step(q, kv[0], kv[1], loc, s["k"], s["v"], bt,
+                                                      pages=None if page == 1 else s["pages"])
+            else:
+                ops.kv_store(cfg, kv[0], kv[1], loc, s["k"], s["v"], s["table"], s["lens"],
+                             pages=None if page == 1 else s["pages"])
+                layer = ops.DecodeLayer(cfg, B, longest, dev)
+                out, sel, sel_pos, sel_len = layer(q, s["k"], s["v"], bt)
+            got.append(dict(out=out.clone(), sel=sel, sel_pos=sel_pos, sel_len=sel_len, lens=s["lens"],
+                            table=s["table"], k=s["k"], v=s["v"]))
+        torch.cuda.synchronize()
+        assert not one.gave_up()
+        _same(*got)
+        assert torch.equal(got[0]["out"], got[1]["out"])
+        assert torch.equal(sides[0]["pages"].free_count, sides[1]["pages"].free_count)
+        assert int(sides[0]["pages"].ticket) == 0
+    if case in ("one", "page begins", "70 requests", "votes form"):
+        assert sides[0]["lens"].tolist() == [n + steps for n in lengths]

@@ -120,7 +120,7 @@ int64_t ts_score_stride(int32_t max_seq_len) {
 
 // Workspace of ts_decode_layer, carved in this order (256-byte aligned pieces).
 struct LayerWorkspace {
-  size_t qf, hit, scores, stats, votes, pooled, partials, topk_ws, select_ws, attn_ws, total;
+  size_t qf, hit, notes, scores, stats, votes, pooled, partials, topk_ws, select_ws, attn_ws, total;
   size_t partials_bytes;
   int64_t score_stride;
   int32_t max_sel;
@@ -140,6 +140,7 @@ static LayerWorkspace layer_workspace(const ts_config* cfg, int32_t batch, int32
   w.max_sel = cfg->n_init + cfg->top_k + cfg->n_local;
   w.qf = take(B * H * kHeadDim * 2);
   w.hit = take(B * 4);
+  w.notes = take(B * sizeof(int4));
   w.scores = take(B * H * (size_t)w.score_stride * 4);
   w.stats = take(B * H * 2 * 4);
   w.votes = take(B * (size_t)w.score_stride * 4);
@@ -277,8 +278,8 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   SeparateKernelsScope separate(bt->separate_kernels != 0);
   TS_REQUIRE(q && q_cos && q_sin && k_pool && v_pool && out && sel && sel_pos && sel_len, TS_EINVAL,
              "layer: NULL tensor argument");
-  TS_REQUIRE(store == nullptr || (cache != nullptr && chunk_rows == 0), TS_EINVAL,
-             "internal: a store rides in the rotation + cache decision launch only");
+  TS_REQUIRE(store == nullptr || (chunk_rows == 0 && !known_dense(cfg, bt, cache)), TS_EINVAL,
+             "internal: no launch for this step's store to ride in");
   TS_REQUIRE(chunk_store == nullptr || chunk_rows > 0, TS_EINVAL,
              "internal: a chunk's store rides in the fingerprint launch only");
   TS_REQUIRE(pool_rows >= 1 && pool_rows <= 0x7fffffffLL, TS_EINVAL, "pool_rows %lld out of range",
@@ -339,6 +340,18 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   // the query itself; this call's attention kernel clears the counters again.
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;
+  // That selection also stores the step's new tokens, and the attention after it writes the lengths
+  // (a layer of one request of 32K 38.0 -> 37.1 us, of 128K 71.8 -> 69.2).  Where a new token may be a
+  // candidate the store stays ahead.
+  StepCommit commit{};
+  if (starts_with_selection && store) {
+    if (cfg->n_local >= 1 && bt->batch <= kCommitBatch) {
+      commit = StepCommit{(int4*)(ws + w.notes), bt->batch, store->table, store->table_stride, store->seq_lens,
+                          store->free_count};
+    } else {
+      TS_TRY(launch_kv_store(*store, bt->batch, (hipStream_t)stream));
+    }
+  }
   if (dense) {
     if (dense_step)  // the attention reads the table, and leaves the list (and the new tokens) itself
       return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, bt->table, bt->table_stride, bt->seq_lens,
@@ -365,7 +378,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                                 zero, (hipStream_t)stream, store));
   } else {
     TS_TRY(launch_rope(q, q_stride, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
-                       zero, (hipStream_t)stream));
+                       zero, (hipStream_t)stream, store, bt->batch));
   }
   if (cache && chunk_rows > 0)
     TS_TRY(launch_selcache(cfg, bt, qf, cache, hit, bt->rerun ? sel_len : nullptr, (hipStream_t)stream));
@@ -375,7 +388,8 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                          nullptr, 0, ws + w.select_ws, tickets, attn_tickets_per_request(cfg),
                          (hipStream_t)stream, select_wait_ticks(bt),
                          (uint32_t)(bt->absent_workgroups > 0 ? bt->absent_workgroups : 0),
-                         starts_with_selection ? &unrotated : nullptr));
+                         starts_with_selection ? &unrotated : nullptr, commit.batch ? store : nullptr,
+                         commit.notes));
   } else if (vote_group > 0) {
     // With max-pooling the kernel writes the pooled votes (there is no un-pooled copy).
     TS_TRY(launch_score_votes(cfg, bt, qf, k_pool, pool_rows, hit, votes, w.score_stride, topk.ws,
@@ -401,7 +415,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                                w.max_sel, out, ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream);
   return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch,
                      w.max_sel, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream,
-                     plain_decode ? &zero : nullptr);
+                     plain_decode ? &zero : nullptr, nullptr, commit.batch ? &commit : nullptr);
 }
 
 int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, const float* q_cos,
@@ -414,10 +428,9 @@ int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, con
 }
 
 // The reference's decode forward in one call (tr.py:777-825): store_kv_cache + add_k_cache,
-// then selection and attention.  With a selection cache and slots chosen by the caller the
-// store rides in the layer's first launch (the rotation and the cache decision, whose
-// workgroup of a request stores that request's rows first); otherwise the two calls follow
-// each other.
+// then selection and attention.  The store rides in the layer's first launch: the rotation and
+// the cache decision, whose workgroup of a request stores that request's rows, the rotation alone,
+// the selection where that is the first, or the attention of a step known to be dense.
 int ts_decode_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
                            int32_t q_row_stride, int32_t kv_row_stride, const float* q_cos,
                            const float* q_sin, void* k_pool, void* v_pool, int64_t pool_rows,
@@ -430,93 +443,50 @@ int ts_decode_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_ne
   int32_t* table = const_cast<int32_t*>(bt->table);
   int32_t* seq_lens = const_cast<int32_t*>(bt->seq_lens);
   // (a call that repeats a step after a give-up does not append again: it is the layer alone)
-  const bool rides = cache != nullptr && bt->rerun == 0;
-  if (!rides) {
-    DenseList list{};
-    if (bt->rerun == 0) {
-      list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
-                       workspace_bytes);
-      if (list.sel && bt->workspace_clean != 0) {
-        // The attention alone (its tickets are zero, as any such call leaves them): the list of a
-        // dense request is its table, and the new row can be read where the caller has it.  With a
-        // page pool the store goes first, since a page is taken in the order of the requests.
-        // 8 layers of a 2003-token request, two steps: 273 -> 215-224 us; 2 layers of a 300-token
-        // prompt with 8 tokens 380 -> 320-350.
-        TS_TRY(check_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool, pool_rows,
-                              table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens));
-        AttnDense step{};
-        step.sel = sel;
-        step.sel_pos = sel_pos;
-        step.sel_stride = sel_stride;
-        step.sel_len = sel_len;
-        step.list_bound = bt->max_seq_len < kv->max_tokens ? bt->max_seq_len : kv->max_tokens;
-        if (kv->pages) {
-          TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
-                                 pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
-                                 (hipStream_t)stream));
-        } else {
-          step.loc = kv->out_cache_loc;
-          step.k = (const uint16_t*)kv->k;
-          step.v = (const uint16_t*)kv->v;
-          step.k_from_pool = ((intptr_t)kv->k - (intptr_t)k_pool) / 2;  // (both aligned to 16 bytes)
-          step.v_from_pool = ((intptr_t)kv->v - (intptr_t)v_pool) / 2;
-          step.kv_stride = kv_row_stride ? kv_row_stride : cfg->num_kv_heads * cfg->head_dim;
-          step.table = table;
-          step.seq_lens = seq_lens;
-          step.max_tokens = kv->max_tokens;
-        }
-        return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
-                         sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, true, &step);
-      }
-      if (kv->pages) list = DenseList{};  // (a paged store writes no list)
-      TS_TRY(launch_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
-                             pool_rows, table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens,
-                             (hipStream_t)stream, list.sel ? &list : nullptr));
+  if (bt->rerun != 0)
+    return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
+                     sel_stride, sel_len, workspace, workspace_bytes, stream);
+  TS_TRY(check_kv_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool, pool_rows,
+                        table, bt->table_stride, seq_lens, bt->batch, kv->max_tokens));
+  const StepStore st = step_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, k_pool, v_pool,
+                                  pool_rows, table, bt->table_stride, seq_lens, kv->max_tokens);
+  if (!known_dense(cfg, bt, cache))  // the store rides in the first launch of the layer
+    return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
+                     sel_stride, sel_len, workspace, workspace_bytes, stream, &st);
+  DenseList list = step_list(cfg, bt, cache, q, q_cos, q_sin, out, sel, sel_pos, sel_stride, sel_len, workspace,
+                             workspace_bytes);
+  if (list.sel && bt->workspace_clean != 0) {
+    // The attention alone (its tickets are zero, as any such call leaves them): the list of a
+    // dense request is its table, and the new row can be read where the caller has it.  With a
+    // page pool the store goes first, since a page is taken in the order of the requests.
+    // 8 layers of a 2003-token request, two steps: 273 -> 215-224 us; 2 layers of a 300-token
+    // prompt with 8 tokens 380 -> 320-350.
+    AttnDense step{};
+    step.sel = sel;
+    step.sel_pos = sel_pos;
+    step.sel_stride = sel_stride;
+    step.sel_len = sel_len;
+    step.list_bound = bt->max_seq_len < kv->max_tokens ? bt->max_seq_len : kv->max_tokens;
+    if (kv->pages) {
+      TS_TRY(launch_kv_store(st, bt->batch, (hipStream_t)stream));
+    } else {
+      step.loc = kv->out_cache_loc;
+      step.k = (const uint16_t*)kv->k;
+      step.v = (const uint16_t*)kv->v;
+      step.k_from_pool = ((intptr_t)kv->k - (intptr_t)k_pool) / 2;  // (both aligned to 16 bytes)
+      step.v_from_pool = ((intptr_t)kv->v - (intptr_t)v_pool) / 2;
+      step.kv_stride = kv_row_stride ? kv_row_stride : cfg->num_kv_heads * cfg->head_dim;
+      step.table = table;
+      step.seq_lens = seq_lens;
+      step.max_tokens = kv->max_tokens;
     }
     return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
-                     sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, list.sel != nullptr);
+                     sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, true, &step);
   }
-  // The checks ts_kv_store makes.
-  TS_REQUIRE(kv->k && kv->v && k_pool && v_pool, TS_EINVAL, "ts_decode_step: NULL tensor argument");
-  TS_REQUIRE_ALIGNED(kv->k, 16, "k");
-  TS_REQUIRE_ALIGNED(kv->v, 16, "v");
-  TS_REQUIRE_ALIGNED(k_pool, 16, "k_pool");
-  TS_REQUIRE_ALIGNED(v_pool, 16, "v_pool");
-  if (kv->pages) {
-    TS_REQUIRE(kv->pages->free_pages && kv->pages->free_count && kv->pages->ticket, TS_EINVAL,
-               "ts_decode_step: page pool has a NULL array");
-  } else {
-    TS_REQUIRE(cfg->page_size == 1, TS_EINVAL, "ts_decode_step: pages of %d tokens need a page pool",
-               cfg->page_size);
-    TS_REQUIRE(kv->out_cache_loc != nullptr, TS_EINVAL, "ts_decode_step: NULL out_cache_loc and no page pool");
-  }
-  TS_REQUIRE(bt->batch >= 1 && pool_rows >= 1 && pool_rows <= 0x7fffffffLL && kv->max_tokens >= 1, TS_EINVAL,
-             "ts_decode_step: batch=%d pool_rows=%lld max_tokens=%d out of range", bt->batch,
-             (long long)pool_rows, kv->max_tokens);
-  TS_REQUIRE(bt->batch == 1 || bt->table_stride * (int64_t)cfg->page_size >= kv->max_tokens, TS_EINVAL,
-             "ts_decode_step: table_stride %lld x page_size %d < max_tokens %d", (long long)bt->table_stride,
-             cfg->page_size, kv->max_tokens);
-  StepStore st{};
-  st.k = (const uint4*)kv->k;
-  st.v = (const uint4*)kv->v;
-  st.loc = kv->out_cache_loc;
-  st.k_pool = (uint4*)k_pool;
-  st.v_pool = (uint4*)v_pool;
-  st.pool_rows = pool_rows;
-  st.table = table;
-  st.table_stride = bt->table_stride;
-  st.seq_lens = seq_lens;
-  st.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  st.kv_stride = kv_row_stride ? kv_row_stride / 8 : st.row_vec;
-  st.max_tokens = kv->max_tokens;
-  if (kv->pages) {
-    st.free_pages = kv->pages->free_pages;
-    st.free_count = kv->pages->free_count;
-    st.ticket = kv->pages->ticket;
-    st.page_shift = page_shift_of(cfg->page_size);
-  }
+  if (kv->pages) list = DenseList{};  // (a paged store writes no list)
+  TS_TRY(launch_kv_store(st, bt->batch, (hipStream_t)stream, list.sel ? &list : nullptr));
   return run_layer(cfg, bt, q, q_row_stride, 0, q_cos, q_sin, 1, k_pool, v_pool, pool_rows, cache, out, sel, sel_pos,
-                   sel_stride, sel_len, workspace, workspace_bytes, stream, &st);
+                   sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr, list.sel != nullptr);
 }
 
 int ts_decode_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,

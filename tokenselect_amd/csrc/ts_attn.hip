@@ -41,6 +41,7 @@ struct AttnArgs {
   // list_bound: positions whose entries are there to be read.
   int list_shift, list_bound;
   AttnDense step;
+  StepCommit commit;  // what the step's store left to be written (batch 0: nothing)
 };
 
 // The last three wavefronts' share of the regions to clear.
@@ -62,6 +63,19 @@ __device__ __forceinline__ float2 load_coherent2(const float* p) {
 __device__ __forceinline__ void store_coherent2(float* p, float x, float y) {
   const uint64_t v = (uint64_t)__float_as_uint(x) | ((uint64_t)__float_as_uint(y) << 32);
   __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The lengths, table entries and page count that a store within the selection left to be written
+// (StepCommit), by one wavefront.  Nothing of this launch reads them.
+__device__ __forceinline__ void attn_commit(const StepCommit& c) {
+  const int b = threadIdx.x & 63;
+  if (b >= c.batch) return;
+  const int4 note = c.notes[b];
+  if (note.x >= 0) {
+    if (note.z >= 0) c.table[(int64_t)b * c.table_stride + note.y] = note.z;
+    c.seq_lens[b] = note.x;
+  }
+  if (b == 0 && c.free_count) *c.free_count = max(*c.free_count, 0) - note.w;
 }
 
 // Whether a request's new token is stored: what the store kernels ask (ts_store.hip).
@@ -153,6 +167,7 @@ __device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, i
     // (While the ticket is drawn, not ahead of the first loads: 0.6 us of the 38 that a layer of a
     // 32K request takes, 2.0 of 98 with eight of 8K.)
     attn_clear_on_the_side(a);
+    if (tid >= 192 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) attn_commit(a.commit);
   }
   __syncthreads();
   if (!s_last) return false;
@@ -670,10 +685,11 @@ size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
-                hipStream_t st, const ZeroSet* clear_after, const AttnDense* dense) {
+                hipStream_t st, const ZeroSet* clear_after, const AttnDense* dense, const StepCommit* commit) {
   const AttnWorkspace w = attn_workspace(cfg, batch, max_sel_len);
   AttnArgs a;
   a.step = AttnDense{};
+  a.commit = commit ? *commit : StepCommit{};
   a.list_shift = a.list_bound = 0;
   if (dense) {
     a.step = *dense;

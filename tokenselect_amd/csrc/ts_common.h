@@ -119,21 +119,8 @@ struct ChunkStore {
 int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const float* cos_table,
                        const float* sin_table, int64_t table_rows, void* qf, const ZeroSet& zero,
                        hipStream_t stream, const ChunkStore* store = nullptr);
-// x_stride: elements between the rows of x (out is contiguous).
-int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
-                const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
-                const ZeroSet& zero, hipStream_t stream);
-
-// Selection-cache decision (ts_selcache.hip); gave_up_len: see ts_batch.rerun (NULL: an
-// ordinary step).
-int launch_selcache(const ts_config* cfg, const ts_batch* bt, const void* qf, const ts_selcache* cache,
-                    int32_t* hit, const int32_t* gave_up_len, hipStream_t stream);
-
-// The fingerprint rotation of a decode step (one query row per request, q_cos / q_sin the
-// [D] table rows of its position) and the cache decision in one launch, which also clears
-// the regions of `zero`.
-// The new token's K/V rows of a decode step, stored by the first launch of the layer (as
-// kv_store_kernel stores them): slots chosen by the caller, one per request.
+// The new token's K/V rows of a decode step, for whatever launch stores them (store_step): slots
+// chosen by the caller, one per request.
 struct StepStore {
   const uint4* k;  // [B, Hkv*D] bf16 as 16-byte pieces
   const uint4* v;
@@ -154,6 +141,32 @@ struct StepStore {
   uint32_t* ticket;
   int page_shift;
 };
+// What a step's store leaves to be written when nobody reads the lengths any more: one per request,
+// noted by the selection that stored the rows and knows the length (ts_score.hip), written by
+// the attention after it.
+struct StepCommit {
+  int4* notes;  // [B] (length or -1: nothing, table index, table entry or -1: none, pages taken by the launch)
+  int batch;    // 0: nothing to write
+  int32_t* table;
+  int64_t table_stride;
+  int32_t* seq_lens;
+  int32_t* free_count;  // NULL: no page pool
+};
+constexpr int kCommitBatch = 64;  // requests that one wavefront writes for
+
+// x_stride: elements between the rows of x (out is contiguous).  store: rides in the launch.
+int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
+                const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
+                const ZeroSet& zero, hipStream_t stream, const StepStore* store = nullptr, int store_batch = 0);
+
+// Selection-cache decision (ts_selcache.hip); gave_up_len: see ts_batch.rerun (NULL: an
+// ordinary step).
+int launch_selcache(const ts_config* cfg, const ts_batch* bt, const void* qf, const ts_selcache* cache,
+                    int32_t* hit, const int32_t* gave_up_len, hipStream_t stream);
+
+// The fingerprint rotation of a decode step (one query row per request, q_cos / q_sin the
+// [D] table rows of its position) and the cache decision in one launch, which also clears
+// the regions of `zero`.
 int launch_rope_selcache(const ts_config* cfg, const ts_batch* bt, const void* q, int q_stride, void* qf,
                          const float* q_cos, const float* q_sin, const ts_selcache* cache, int32_t* hit,
                          const int32_t* gave_up_len, const ZeroSet& zero, hipStream_t stream,
@@ -177,11 +190,11 @@ int check_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t r
                    const ts_page_pool* pages, const void* k_pool, const void* v_pool, int64_t pool_rows,
                    const int32_t* table, int64_t table_stride, const int32_t* seq_lens, int32_t batch,
                    int32_t max_tokens);
-// ts_kv_store and ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
-int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
-                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
-                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
-                    int32_t max_tokens, hipStream_t stream, const DenseList* list = nullptr);
+StepStore step_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                     const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
+                     int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t max_tokens);
+int launch_kv_store(const StepStore& st, int32_t batch, hipStream_t stream, const DenseList* list = nullptr);
+// ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
 // (list: only where chunk_store_takes_list says so)
 bool chunk_store_takes_list(int32_t rows, int32_t max_tokens, int32_t max_seq_len);
 int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
@@ -227,7 +240,8 @@ struct AttnDense {
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
-                hipStream_t stream, const ZeroSet* clear_after = nullptr, const AttnDense* dense = nullptr);
+                hipStream_t stream, const ZeroSet* clear_after = nullptr, const AttnDense* dense = nullptr,
+                const StepCommit* commit = nullptr);
 
 constexpr int kHeadDim = 128;
 constexpr float kNegBig = -3.0e38f;  // finite stand-in for -inf in running maxima
@@ -315,16 +329,21 @@ struct ReqGeom {
 
 // seq_lens[b] is clamped to the host's max_seq_len, the bound every buffer and
 // grid was sized for.
-__device__ __forceinline__ ReqGeom request_geometry(const int32_t* seq_lens, const int32_t* k_per_req,
-                                                    int b, int n_init, int n_local, int top_k,
-                                                    int max_seq_len) {
+__device__ __forceinline__ ReqGeom geometry_of_length(int length, const int32_t* k_per_req, int b, int n_init,
+                                                      int n_local, int top_k, int max_seq_len) {
   ReqGeom g;
-  g.seq_len = min(max(seq_lens[b], 0), max_seq_len);
+  g.seq_len = min(max(length, 0), max_seq_len);
   int k = k_per_req ? k_per_req[b] : top_k;
   g.k = k < 0 ? 0 : (k > top_k ? top_k : k);
   g.dense = (n_init + g.k + n_local >= g.seq_len);
   g.n = g.dense ? 0 : g.seq_len - n_init - n_local;
   return g;
+}
+
+__device__ __forceinline__ ReqGeom request_geometry(const int32_t* seq_lens, const int32_t* k_per_req,
+                                                    int b, int n_init, int n_local, int top_k,
+                                                    int max_seq_len) {
+  return geometry_of_length(seq_lens[b], k_per_req, b, n_init, n_local, top_k, max_seq_len);
 }
 
 // Logical position -> physical KV slot through the (paged) table; page sizes are

@@ -118,4 +118,56 @@ __device__ __forceinline__ void commit_appends(int32_t* seq_lens, int32_t* table
   }
 }
 
+// The rows of request b stored and appended, by one workgroup of a launch in which `batch` of them
+// do this: at the slot that the caller chose, or (with a page pool) where the plan of the batch
+// says, which the last of them commits.  A full table (tr.py:334 asserts) or a slot outside the pool
+// leaves the request untouched.  Bound by its memory round trips; the new rows are asked for
+// together with the slot and the length, not after them.
+__device__ __forceinline__ void store_step(const StepStore& st, int b, int batch) {
+  const int first = threadIdx.x, threads = blockDim.x;
+  uint4 k0 = make_uint4(0u, 0u, 0u, 0u), v0 = k0;
+  if (first < st.row_vec) {
+    k0 = st.k[(size_t)b * st.kv_stride + first];
+    v0 = st.v[(size_t)b * st.kv_stride + first];
+  }
+  int64_t slot = -1;
+  int len = 0;
+  const PagePool pool{st.free_pages, st.free_count, st.ticket};
+  if (st.free_pages != nullptr) {
+    __shared__ int plan_slot;
+    if (threadIdx.x == 0) plan_slot = -1;
+    __syncthreads();
+    if (threadIdx.x < 64)
+      for_each_append(st.seq_lens, st.table, st.table_stride, batch, pool, st.page_shift, st.max_tokens,
+                      (uint32_t)st.pool_rows, (int)threadIdx.x, [&](int req, const AppendPlan& p) {
+                        if (req == b && p.ok) plan_slot = (int)p.slot;
+                      });
+    __syncthreads();
+    slot = plan_slot;
+  } else {
+    slot = st.loc[b];
+    len = st.seq_lens[b];
+    if (slot >= st.pool_rows || len >= st.max_tokens) slot = -1;
+  }
+  if (slot >= 0) {
+    if (first < st.row_vec) {
+      st.k_pool[(size_t)slot * st.row_vec + first] = k0;
+      st.v_pool[(size_t)slot * st.row_vec + first] = v0;
+    }
+    for (int i = first + threads; i < st.row_vec; i += threads) {
+      st.k_pool[(size_t)slot * st.row_vec + i] = st.k[(size_t)b * st.kv_stride + i];
+      st.v_pool[(size_t)slot * st.row_vec + i] = st.v[(size_t)b * st.kv_stride + i];
+    }
+  }
+  __syncthreads();
+  if (st.free_pages != nullptr) {
+    if (threadIdx.x < 64)
+      commit_appends(st.seq_lens, st.table, st.table_stride, batch, pool, st.page_shift, st.max_tokens,
+                     (uint32_t)st.pool_rows, (int)threadIdx.x, (uint32_t)batch);
+  } else if (threadIdx.x == 0 && slot >= 0) {
+    st.table[(int64_t)b * st.table_stride + len] = (int32_t)slot;
+    st.seq_lens[b] = len + 1;
+  }
+}
+
 }  // namespace ts

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "ts_grid.h"
+#include "ts_pages.h"
 #include "ts_topk.h"
 
 namespace ts {
@@ -34,6 +35,7 @@ struct ScoreArgs {
   int64_t table_stride;
   const int32_t* k_per_req;
   const int32_t* skip;  // per request: 1 = selection-cache hit, nothing to score
+  int appends;          // single-launch selection only: the launch stores the step's new tokens (append)
   int n_init, n_local, top_k, page_size, page_shift, max_seq_len;
   int64_t direct_n;  // >= 0: paged_matmul mode, candidates are table[0..direct_n)
   void* scores;
@@ -74,7 +76,6 @@ struct ScoreArgs {
   // rendezvous area is sync + p * kSyncWords.
   int nphases;
   int resident;           // workgroups of the launch that the device holds at once
-  VotePhase phases[kMaxPhases];
   uint32_t* hist_ws;      // per-request top-k workspace (ts_topk.h) whose hist0 is counted into, or NULL
   size_t hist_ws_stride;
   uint32_t* fault_word;   // votes-only: the word the kernels after this one consult
@@ -86,6 +87,16 @@ struct ScoreArgs {
   int pool_kernel;        // max-pool window over the votes (tr.py:366-369), <= 0: off
   float* pool_votes;      // [B,pool_stride] un-pooled votes exchanged between workgroups
   int64_t pool_stride;
+  // The step's new tokens (appends; at most kCommitBatch requests), which the launch stores on the
+  // side.  A new token is the newest of the local window and no
+  // candidate; seq_lens does not count it yet and is read by every workgroup, so what the append
+  // changes there, in the table and in the pool's count goes to `notes`, for the attention after
+  // this launch to write.
+  StepStore append;
+  int4* notes;
+  // Last: a workgroup's first look at a line of the arguments is a round trip of its own, and these
+  // 1.2 KB in the middle put what every launch needs at its start into as many lines more.
+  VotePhase phases[kMaxPhases];
 };
 
 // Selection counters of one request, in 32-bit words.  The first histogram is kept
@@ -213,6 +224,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
                   int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, float* votes,
                   int64_t vote_stride, void* workspace, uint32_t* clear, int clear_per_req,
                   hipStream_t stream, uint64_t wait_ticks, uint32_t absent,
-                  const UnrotatedQuery* unrotated = nullptr);
+                  const UnrotatedQuery* unrotated = nullptr, const StepStore* append = nullptr,
+                  int4* notes = nullptr);
 
 }  // namespace ts

@@ -108,6 +108,40 @@ __device__ __forceinline__ int packed_chunks(const LaunchPart& lp, int r, int n)
   return min(chunks, lp.pack_first[r + 1] - lp.pack_first[r]);
 }
 
+// A request's length, the new token counted where this launch appends it, and that token's slot
+// (kNoSlot: none).  With one request every thread knows them (`own`), else they are in LDS.
+constexpr uint32_t kNoSlot = 0xffffffffu;
+struct Appended {
+  int len;
+  uint32_t slot;
+};
+// (Chosen word by word: a choice between two structs puts both in memory.)
+__device__ __forceinline__ Appended append_at(bool ok, int len, uint32_t slot) {
+  return Appended{ok ? len + 1 : len, ok ? slot : kNoSlot};
+}
+struct Lengths {
+  int own_len;
+  uint32_t own_slot;
+  int taken;  // pages that the launch takes from the pool
+};
+__device__ __forceinline__ Appended appended(const ScoreArgs& a, const Lengths lens, const Appended* plans, int b) {
+  if (!a.appends) return Appended{a.seq_lens[b], kNoSlot};
+  if (a.batch == 1) return Appended{lens.own_len, lens.own_slot};
+  Appended noted = plans[b];
+  // (loaded here: one load for this and the case above it would be from either of two memories)
+  asm("" : "+v"(noted.len), "+v"(noted.slot));
+  return noted;
+}
+// The kernel's arguments, read again from here on.  What the compiler can see at the start of a
+// kernel it loads there and holds to the end: the scalar registers did not suffice, the first load
+// waited behind 50 moves of them to vector lanes and a second round of arguments, and the phases
+// after the stream began by fetching them back.
+__device__ __forceinline__ const ScoreArgs& late_args() {
+  auto args = (const __attribute__((address_space(4))) ScoreArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return *(const ScoreArgs*)args;
+}
+
 // The softmax statistics of the fused kernel, without a rendezvous: every workgroup
 // publishes its per-head (max, sum exp) into a table that was zero at launch; the
 // (request, head) pairs are dealt out over all wavefronts of the team; a wavefront polls
@@ -118,7 +152,8 @@ __device__ __forceinline__ int packed_chunks(const LaunchPart& lp, int r, int n)
 // of the rendezvous: on giving up it sets the fault word and merges what is there.
 template <bool PACKED>
 __device__ __forceinline__ void merge_request_stats(const ScoreArgs& a, const LaunchPart& lp,
-                                                    const GridTeam& team, int lane, int wave) {
+                                                    const GridTeam& team, const Lengths lens, const Appended* plans,
+                                                    int lane, int wave) {
   const int H = a.num_heads;
   const int items = (PACKED ? lp.packed : a.batch) * H;
   const int first = (int)team.index * 4 + wave;
@@ -126,8 +161,8 @@ __device__ __forceinline__ void merge_request_stats(const ScoreArgs& a, const La
   for (int item = first; item < items; item += step) {
     const int b = lp.batch_offset + item / H, h = item % H;
     if (a.skip && a.skip[b]) continue;
-    const ReqGeom geo =
-        request_geometry(a.seq_lens, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len);
+    const ReqGeom geo = geometry_of_length(PACKED ? a.seq_lens[b] : appended(a, lens, plans, b).len, a.k_per_req, b, a.n_init,
+                                           a.n_local, a.top_k, a.max_seq_len);
     if (geo.n <= 0) continue;
     const int chunks = PACKED ? packed_chunks(lp, item / H, geo.n)
                               : (geo.n + lp.tokens_per_block - 1) / lp.tokens_per_block;
@@ -238,8 +273,48 @@ struct Deal {
   int chunk, chunks;     // its chunk of that request, and the request's chunks
   int n;                 // the request's candidates
   uint32_t team_size, team_index;
+  int own_len;           // of the only request, with the new token that this launch appends,
+  uint32_t own_slot;     // and that token's slot (kNoSlot: none)
+  int taken;             // pages that the launch takes from the pool
 };
-constexpr int kDealPerLane = 8;  // requests per lane of the dealing wavefront: batches of up to 512
+constexpr int kDealRequests = 512;  // of a launch at most: every request has a workgroup of the grid
+
+// Where the new tokens go, as the store kernels place them (store_step): with one request by every
+// thread for itself, else by the dealing wavefront for all, a lane each (at most kCommitBatch of them).
+// Pages: the rank of the only request that may need one is zero.
+__device__ __forceinline__ void plan_append_one(const ScoreArgs& a, int len, Deal& d) {
+  const StepStore& st = late_args().append;
+  if (st.free_pages == nullptr) {
+    const int slot = st.loc[0];
+    const bool ok = slot >= 0 && slot < st.pool_rows && len >= 0 && len < st.max_tokens;
+    d.own_len = ok ? len + 1 : len;
+    d.own_slot = ok ? (uint32_t)slot : kNoSlot;
+    return;
+  }
+  const int page_mask = (1 << st.page_shift) - 1, count = max(*st.free_count, 0);
+  const bool room = len >= 0 && len < st.max_tokens, need = room && (len & page_mask) == 0;
+  const AppendPlan p = make_append_plan(st.table, len, room, need, 0u, count, st.free_pages, st.page_shift, page_mask,
+                                        (uint32_t)st.pool_rows);
+  d.taken = need ? min(1, count) : 0;
+  d.own_len = p.ok ? len + 1 : len;
+  d.own_slot = p.ok ? p.slot : kNoSlot;
+}
+__device__ __forceinline__ int plan_appends(const ScoreArgs& a, int lane, Appended* plans) {
+  const StepStore& st = late_args().append;
+  if (st.free_pages == nullptr) {
+    if (lane < a.batch) {
+      const int len = st.seq_lens[lane], slot = st.loc[lane];
+      const bool ok = slot >= 0 && slot < st.pool_rows && len >= 0 && len < st.max_tokens;
+      plans[lane] = append_at(ok, len, (uint32_t)slot);
+    }
+    return 0;
+  }
+  const PagePool pool{st.free_pages, st.free_count, st.ticket};
+  return for_each_append(st.seq_lens, st.table, st.table_stride, a.batch, pool, st.page_shift, st.max_tokens,
+                         (uint32_t)st.pool_rows, lane, [&](int b, const AppendPlan& p) {
+                           plans[b] = append_at(p.ok, p.len, p.slot);
+                         });
+}
 
 __device__ __forceinline__ int wave_sum(int x) {
 #pragma unroll
@@ -247,15 +322,20 @@ __device__ __forceinline__ int wave_sum(int x) {
   return x;
 }
 
-__device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
+// (cand: LDS of kDealRequests words, free again when this returns.  The loops over the requests are
+// rolled up and hold them there: unrolled over registers they were 2000 instructions at the head of
+// the kernel that one request skips, and a selection's start is bound by what it fetches of them.)
+__device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds, int* cand, Appended* plans) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int B = a.batch, T = (int)gridDim.x, w = (int)blockIdx.x;
-  if (B == 1) {  // one request: every thread works it out for itself, no exchange
-    Deal d{a.tokens_per_block, -1, 0, 0, 0, a.absent, (uint32_t)w};
+  if (__builtin_expect(B == 1, 1)) {  // one request: every thread works it out for itself, no exchange
+    Deal d{a.tokens_per_block, -1, 0, 0, 0, a.absent, (uint32_t)w, 0, kNoSlot, 0};
     int n = 0;
+    d.own_len = a.seq_lens[a.batch_offset];
+    if (__builtin_expect(a.appends != 0, 0)) plan_append_one(a, d.own_len, d);
     if (!(a.skip && a.skip[a.batch_offset]))
-      n = request_geometry(a.seq_lens, a.k_per_req, a.batch_offset, a.n_init, a.n_local, a.top_k,
-                           a.max_seq_len).n;
+      n = geometry_of_length(d.own_len, a.k_per_req, a.batch_offset, a.n_init, a.n_local, a.top_k,
+                             a.max_seq_len).n;
     if (n <= 0) return d;
     d.n = n;
     int tpb = max((n + T * 64 - 1) / (T * 64) * 64, 64);
@@ -270,18 +350,19 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
     return d;
   }
   if (tid < 64) {
-    // Request lane + 64 j: its candidates if it selects, else 0.
-    int n[kDealPerLane];
+    const int taken = a.appends ? plan_appends(a, lane, plans) : 0;
+    // Every request's candidates if it selects, else 0.
     int all = 0;  // (what one launch holds fits the LDS of the device: far below 2^31)
-#pragma unroll
-    for (int j = 0; j < kDealPerLane; ++j) {
-      const int b = lane + 64 * j;
-      n[j] = 0;
-      if (64 * j >= B) continue;
-      if (b < B && !(a.skip && a.skip[a.batch_offset + b]))
-        n[j] = request_geometry(a.seq_lens, a.k_per_req, a.batch_offset + b, a.n_init, a.n_local, a.top_k,
-                                a.max_seq_len).n;
-      all += n[j];
+#pragma unroll 1
+    for (int b = lane; b < B; b += 64) {
+      int len = 0, n = 0;
+      if (a.appends) len = plans[b].len;
+      asm("" : "+v"(len));  // (or the two loads become one, from either of two memories)
+      if (!a.appends) len = a.seq_lens[a.batch_offset + b];
+      if (!(a.skip && a.skip[a.batch_offset + b]))
+        n = geometry_of_length(len, a.k_per_req, a.batch_offset + b, a.n_init, a.n_local, a.top_k, a.max_seq_len).n;
+      cand[b] = n;
+      all += n;
     }
     const long long total_n = wave_sum(all);
     // Fewest tokens per workgroup that could do, then upwards until the chunks fit (a step
@@ -289,38 +370,32 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
     // fits: the host sized the grid for every request at the longest length.
     int tpb = (int)((total_n + (long long)T * 64 - 1) / ((long long)T * 64)) * 64;
     tpb = max(tpb, 64);
-    int chunks[kDealPerLane];
     for (;; tpb += 64) {
       int mine = 0;
-#pragma unroll
-      for (int j = 0; j < kDealPerLane; ++j) {
-        chunks[j] = 0;
-        if (64 * j >= B) continue;
-        chunks[j] = (n[j] + tpb - 1) / tpb;
-        mine += chunks[j];
-      }
+#pragma unroll 1
+      for (int b = lane; b < B; b += 64) mine += (cand[b] + tpb - 1) / tpb;
       if (wave_sum(mine) <= T || tpb >= a.tokens_per_block) break;
     }
-    // First workgroup of every request, in request order (lane + 64 j: j by j).
+    // First workgroup of every request, in request order, 64 of them at a time.
     int base = 0, req = -1, chunk = 0, req_chunks = 0, req_n = 0;
-#pragma unroll
-    for (int j = 0; j < kDealPerLane; ++j) {
-      if (64 * j >= B) break;
-      int incl = chunks[j];
+#pragma unroll 1
+    for (int b0 = 0; b0 < B; b0 += 64) {
+      const int n = b0 + lane < B ? cand[b0 + lane] : 0;
+      const int chunks = (n + tpb - 1) / tpb;
+      int incl = chunks;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
         const int up = __shfl_up(incl, off);
         if (lane >= off) incl += up;
       }
-      const int first = base + incl - chunks[j];
-      const bool here = w >= first && w < first + chunks[j];
-      const uint64_t who = __ballot(here);
+      const int first = base + incl - chunks;
+      const uint64_t who = __ballot(w >= first && w < first + chunks);
       if (who) {
         const int src = __ffsll((unsigned long long)who) - 1;
-        req = 64 * j + src;
+        req = b0 + src;
         chunk = w - __shfl(first, src);
-        req_chunks = __shfl(chunks[j], src);
-        req_n = __shfl(n[j], src);
+        req_chunks = __shfl(chunks, src);
+        req_n = __shfl(n, src);
       }
       base += __shfl(incl, 63);
     }
@@ -331,6 +406,7 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
       lds[3] = req_chunks;
       lds[4] = base;  // workgroups with tokens: the team
       lds[5] = req_n;
+      lds[6] = taken;
     }
   }
   __syncthreads();
@@ -340,10 +416,31 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
   d.chunk = lds[2];
   d.chunks = lds[3];
   d.n = lds[5];
+  d.own_len = 0;
+  d.own_slot = kNoSlot;
+  d.taken = lds[6];
   d.team_size = (uint32_t)lds[4] + a.absent;
   d.team_index = (uint32_t)w;
   __syncthreads();
   return d;
+}
+
+// The new token of request b, by one workgroup: its rows to the pool, and the note of what the
+// attention kernel is to write.
+__device__ __forceinline__ void append_token(const ScoreArgs& a, int b, const Appended& now, int taken) {
+  const StepStore& st = late_args().append;
+  const bool ok = now.slot != kNoSlot;
+  if (ok)
+    for (int i = threadIdx.x; i < st.row_vec; i += 256) {
+      const uint4 k = st.k[(size_t)b * st.kv_stride + i], v = st.v[(size_t)b * st.kv_stride + i];
+      st.k_pool[(size_t)now.slot * st.row_vec + i] = k;
+      st.v_pool[(size_t)now.slot * st.row_vec + i] = v;
+    }
+  if (threadIdx.x == 0) {
+    const int at = now.len - 1;
+    const bool entry = ok && (at & ((1 << st.page_shift) - 1)) == 0;
+    a.notes[b] = make_int4(ok ? now.len : -1, at >> st.page_shift, entry ? (int)(now.slot >> st.page_shift) : -1, taken);
+  }
 }
 
 // The parts of the output that need no votes, written while the statistics are on their way: a
@@ -352,9 +449,13 @@ __device__ __forceinline__ Deal deal_workgroups(const ScoreArgs& a, int* lds) {
 // length, the sink and the local window, and clears the words the next kernel of
 // the stream wants cleared.
 // (x of nx: this workgroup among those that write the request's fixed parts.)
-__device__ __forceinline__ void fixed_segments(const ScoreArgs& a, int b, int x, int nx) {
+__device__ __forceinline__ void fixed_segments(const ScoreArgs& a, const Lengths lens, const Appended* plans, int b, int x,
+                                               int nx) {
+  const Appended now = appended(a, lens, plans, b);
   const ReqGeom geo =
-      request_geometry(a.seq_lens, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len);
+      geometry_of_length(now.len, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len);
+  if (x == 0 && a.appends) append_token(a, b, now, b == 0 ? lens.taken : 0);
+  const int new_pos = now.slot == kNoSlot ? -1 : now.len - 1;  // (the table does not know its slot yet)
   const int32_t* tab = a.table + (int64_t)b * a.table_stride;
   int32_t* sel = a.sel + (int64_t)b * a.sel_stride;
   int32_t* sel_pos = a.sel_pos + (int64_t)b * a.sel_stride;
@@ -362,7 +463,7 @@ __device__ __forceinline__ void fixed_segments(const ScoreArgs& a, int b, int x,
   const int first = x * 256 + threadIdx.x, step = nx * 256;
   auto emit = [&](int out_idx, int pos) {
     sel_pos[out_idx] = pos;
-    sel[out_idx] = (int32_t)lookup_slot(tab, pos, a.page_size, a.page_shift, a.pool_rows);
+    sel[out_idx] = (int32_t)(pos == new_pos ? now.slot : lookup_slot(tab, pos, a.page_size, a.page_shift, a.pool_rows));
   };
   if (x == 0 && a.clear)
     for (int i = threadIdx.x; i < a.clear_per_req; i += 256)
@@ -419,9 +520,9 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t x) {
 // workgroup down, those of request w % B, as one of the workgroups w % B, w % B + B, ...
 // (The first workgroups of the team merge the statistics, and everybody waits for those; the
 // last ones often have no candidates.)
-__device__ __forceinline__ void fixed_parts(const ScoreArgs& a) {
+__device__ __forceinline__ void fixed_parts(const ScoreArgs& a, const Lengths lens, const Appended* plans) {
   const int B = a.batch, T = (int)gridDim.x, w = T - 1 - (int)blockIdx.x;
-  fixed_segments(a, a.batch_offset + w % B, w / B, (T - w % B + B - 1) / B);
+  fixed_segments(a, lens, plans, a.batch_offset + w % B, w / B, (T - w % B + B - 1) / B);
 }
 
 // Adds the wavefront's candidates to a histogram in memory with one fetch-add per
@@ -550,11 +651,22 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   constexpr int ITER = 16 * TG;    // tokens per iteration
   constexpr uint32_t ROW_BYTES = HKV * kHeadDim * 2;
 
+  constexpr bool SHARED_QUERY = FUSED && !PACKED;  // the query operands are shared in LDS (below)
+  constexpr bool RAW = SHARED_QUERY;               // and the query may be un-rotated (a.q_raw)
+  constexpr int OPS = HKV * NA, MINE = (OPS + 3) / 4;
+  // One after the other: the requests while they are dealt, the query operands, the histogram.
+  constexpr int LH = SHARED_QUERY && OPS * 256 > kTopkBins ? OPS * 256 : kTopkBins;
+  static_assert(LH >= kDealRequests, "a word per request");
+  __shared__ __attribute__((aligned(16))) uint32_t lh[FUSED ? LH : 4];
+
   // This workgroup's request within the launch, and its chunk of that request.
   LaunchPart lp{a.tokens_per_block, a.batch_offset, 0, nullptr, (int)blockIdx.x, a.sync};
   int req = blockIdx.y, chunk = blockIdx.x;
   int req_chunks = (int)gridDim.x;  // chunks of this workgroup's request (the single launch: dealt)
   int dealt_n = 0;
+  int own_len = 0, taken = 0;
+  uint32_t own_slot = kNoSlot;
+  __shared__ Appended plans[FUSED && !PACKED ? kCommitBatch : 1];
   GridTeam team{0u, 0u};
   if (PACKED) {
     TS_MARK(0);
@@ -571,9 +683,12 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   if constexpr (FUSED && !PACKED) {
     __shared__ int deal_lds[8];
     TS_MARK(0);
-    const Deal deal = deal_workgroups(a, deal_lds);
-    if (deal.req < 0) {  // no chunk left for this workgroup
-      fixed_parts(a);
+    const Deal deal = deal_workgroups(a, deal_lds, (int*)lh, plans);
+    own_len = deal.own_len;
+    own_slot = deal.own_slot;
+    taken = deal.taken;
+    if (__builtin_expect(deal.req < 0, 0)) {  // no chunk left for this workgroup
+      fixed_parts(late_args(), Lengths{own_len, own_slot, taken}, plans);
       return;
     }
     lp.tokens_per_block = deal.tokens_per_block;
@@ -637,12 +752,6 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   // 159.4 us shared, 155.4 without the barrier, 149.1 without those keys either; 18 x 20K 97.3,
   // 95.8 and 93.4; scores alone of 8 x 20K 54.0, 52.9 and 50.5; with four heads per KV head (16 x
   // 68K, 4 x 256K) all within the spread.
-  constexpr bool SHARED_QUERY = FUSED && !PACKED;
-  constexpr bool RAW = SHARED_QUERY;  // the query may be un-rotated (a.q_raw)
-  constexpr int OPS = HKV * NA, MINE = (OPS + 3) / 4;
-  // The histogram of the selection below takes the same place.
-  constexpr int LH = SHARED_QUERY && OPS * 256 > kTopkBins ? OPS * 256 : kTopkBins;
-  __shared__ __attribute__((aligned(16))) uint32_t lh[FUSED ? LH : 4];
   const bool raw = RAW && a.q_raw != nullptr;
   const bool lower = rg < 2;
   uint4 q_own[MINE], q_other[MINE];
@@ -918,6 +1027,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   }
 
   if constexpr (FUSED) {
+    const ScoreArgs& a = late_args();
+    const int32_t* tab = a.table + (int64_t)b * a.table_stride;
     __shared__ float s_rz[kMaxHeads];
     __shared__ uint32_t scratch[16];
     const int tid = threadIdx.x;
@@ -937,10 +1048,10 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // stream to the phase's end, and the next phase waits for them (4 x 256K: 420 us, 425 with
     // the exponentials first).
     if constexpr (PACKED) {
-      merge_request_stats<PACKED>(a, lp, team, lane, wave);
+      merge_request_stats<PACKED>(a, lp, team, Lengths{own_len, own_slot, taken}, plans, lane, wave);
       TS_MARK(3);
     } else {
-      fixed_parts(a);
+      fixed_parts(a, Lengths{own_len, own_slot, taken}, plans);
     }
     uint32_t ahead[kAheadLoads];
 #pragma unroll
@@ -950,9 +1061,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     }
     // While the statistics are on their way: the exponentials, relative to this
     // workgroup's own maxima; exp(s - max) / sum = exp(s - own max) * exp(own max - max) / sum.
-    const ReqGeom geo =
-        request_geometry(a.seq_lens, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len);
-    const uint32_t k = (uint32_t)geo.k;
+    // (only k: whatever the length)
+    const uint32_t k = (uint32_t)geometry_of_length(0, a.k_per_req, b, a.n_init, a.n_local, a.top_k, a.max_seq_len).k;
     const int count = min(lp.tokens_per_block, n - block_lo);
     uint32_t* ctr = a.counters + (size_t)b * kSelCounterWords;
     auto column = [&](int i) -> float* { return stage + (i >> 4) * tile_stride + (i & 15); };
@@ -971,7 +1081,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     }
     // (after the exponentials: the workgroups that merge are among those that wait for the last one's)
     if constexpr (!PACKED) {
-      merge_request_stats<PACKED>(a, lp, team, lane, wave);
+      merge_request_stats<PACKED>(a, lp, team, Lengths{own_len, own_slot, taken}, plans, lane, wave);
       TS_MARK(3);
     }
     if (tid < H) {  // H <= kMaxHeads < 256
@@ -2009,7 +2119,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
                   int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, float* votes,
                   int64_t vote_stride, void* workspace, uint32_t* clear, int clear_per_req,
                   hipStream_t stream, uint64_t wait_ticks, uint32_t absent,
-                  const UnrotatedQuery* unrotated) {
+                  const UnrotatedQuery* unrotated, const StepStore* append, int4* notes) {
   // (requests may be skipped when the caller brings hit flags: the selection cache)
   const SelectWorkspace w = select_workspace(cfg, bt->batch, bt->max_seq_len, false, hit != nullptr);
   TS_REQUIRE(w.tokens_per_block > 0, TS_ESHAPE, "fused selection: unsupported shape");
@@ -2023,6 +2133,13 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
     a.q_stride = unrotated->stride;
     a.q_cos = unrotated->cos;
     a.q_sin = unrotated->sin;
+  }
+  if (append) {
+    TS_REQUIRE(bt->batch <= kCommitBatch && cfg->n_local >= 1 && notes, TS_EINVAL,
+               "internal: this step's store does not ride in the selection");
+    a.appends = 1;
+    a.append = *append;
+    a.notes = notes;
   }
   a.sync = (uint32_t*)(ws + w.sync);
   a.stats = (float*)(ws + w.stats);

@@ -5,14 +5,12 @@
 
 namespace ts {
 
-// One workgroup per request: copies the new K and V rows (Hkv*128 bf16 each) to
-// pool slot out_cache_loc[b], appends the slot to the request's table and bumps
-// its length.  A full table (tr.py:334 asserts) or a slot outside the pool
-// leaves the request untouched.
-// LIST: every request of the step attends to all its tokens, and the workgroup also writes
-// the request's selection (list), the table itself.  Bound by three dependent memory round
-// trips (length and slot, stores, the length's store); the table entries are asked for with the
-// first.  A dense step then has two launches, this (2.2 us) and the attention, where it had
+__global__ __launch_bounds__(256) void kv_store_kernel(StepStore st) { store_step(st, blockIdx.x, gridDim.x); }
+
+// One workgroup per request: the same, at a slot that the caller chose, and (where every request of
+// the step attends to all its tokens) the request's selection (list), the table itself.  Bound by
+// three dependent memory round trips (length and slot, stores, the length's store); the table
+// entries are asked for with the first.  A dense step then has two launches, this (2.2 us) and the attention, where it had
 // a store (1.7), a selection kernel or a rotation and a list (3.3 to 4.6) and the attention:
 // 8 layers of a 2003-token request, two steps, 320 -> 261 us; 2 layers of a 300-token prompt
 // with 8 tokens 430 -> 368 us.  (Once the caller can say that the attention's tickets are zero, the
@@ -20,11 +18,11 @@ namespace ts {
 constexpr int kListThreads = 1024;  // one request's few thousand entries in a handful of steps
 constexpr int kListAhead = 4;       // table entries a thread asks for before it knows the length
 
-template <bool LIST>
-__global__ __launch_bounds__(LIST ? kListThreads : 256) void kv_store_kernel(
-    const uint4* __restrict__ k, const uint4* __restrict__ v, const int32_t* __restrict__ loc,
-    uint4* __restrict__ k_pool, uint4* __restrict__ v_pool, int64_t pool_rows, int32_t* table,
-    int64_t table_stride, int32_t* seq_lens, int row_vec, int kv_stride, int max_tokens, DenseList list) {
+__global__ __launch_bounds__(kListThreads) void kv_store_list_kernel(StepStore st, DenseList list) {
+  const uint4 *k = st.k, *v = st.v;
+  uint4 *k_pool = st.k_pool, *v_pool = st.v_pool;
+  const int64_t pool_rows = st.pool_rows;
+  const int row_vec = st.row_vec, kv_stride = st.kv_stride, max_tokens = st.max_tokens;
   const int b = blockIdx.x;
   // The new rows are asked for together with the slot and the length, not after them: the
   // kernel is two memory round trips long instead of three.
@@ -34,21 +32,17 @@ __global__ __launch_bounds__(LIST ? kListThreads : 256) void kv_store_kernel(
     k0 = k[(size_t)b * kv_stride + first];
     v0 = v[(size_t)b * kv_stride + first];
   }
-  const int slot = loc[b];
-  const int len = seq_lens[b];
-  int32_t* const tab = table + (int64_t)b * table_stride;
+  const int slot = st.loc[b];
+  const int len = st.seq_lens[b];
+  int32_t* const tab = st.table + (int64_t)b * st.table_stride;
   int32_t ahead[kListAhead];
-  int known = 0;  // entries that are there to be read, whatever the length: a table holds max_tokens
-  if (LIST) {
-    known = min(list.max_seq_len, max_tokens);
+  const int known = min(list.max_seq_len, max_tokens);  // entries there to be read: a table holds max_tokens
 #pragma unroll
-    for (int i = 0; i < kListAhead; ++i) {
-      const int pos = first + i * kListThreads;
-      ahead[i] = pos < known ? tab[pos] : 0;
-    }
+  for (int i = 0; i < kListAhead; ++i) {
+    const int pos = first + i * kListThreads;
+    ahead[i] = pos < known ? tab[pos] : 0;
   }
   const bool ok = slot >= 0 && slot < pool_rows && len < max_tokens;
-  if (!LIST && !ok) return;
   if (ok) {
     if (first < row_vec) {
       k_pool[(size_t)slot * row_vec + first] = k0;
@@ -59,30 +53,28 @@ __global__ __launch_bounds__(LIST ? kListThreads : 256) void kv_store_kernel(
       v_pool[(size_t)slot * row_vec + i] = v[(size_t)b * kv_stride + i];
     }
   }
-  if (LIST) {
-    const int L = min(max(ok ? len + 1 : len, 0), list.max_seq_len);
-    int32_t* const sel = list.sel + (int64_t)b * list.sel_stride;
-    int32_t* const sel_pos = list.sel_pos + (int64_t)b * list.sel_stride;
-    auto emit = [&](int pos, int32_t entry) {
-      const uint32_t s = (uint32_t)(ok && pos == len ? slot : entry);
-      sel_pos[pos] = pos;
-      sel[pos] = (int32_t)(s < (uint32_t)pool_rows ? s : (uint32_t)pool_rows - 1);
-    };
+  const int L = min(max(ok ? len + 1 : len, 0), list.max_seq_len);
+  int32_t* const sel = list.sel + (int64_t)b * list.sel_stride;
+  int32_t* const sel_pos = list.sel_pos + (int64_t)b * list.sel_stride;
+  auto emit = [&](int pos, int32_t entry) {
+    const uint32_t s = (uint32_t)(ok && pos == len ? slot : entry);
+    sel_pos[pos] = pos;
+    sel[pos] = (int32_t)(s < (uint32_t)pool_rows ? s : (uint32_t)pool_rows - 1);
+  };
 #pragma unroll
-    for (int i = 0; i < kListAhead; ++i) {
-      const int pos = first + i * kListThreads;
-      if (pos < L) emit(pos, pos < known ? ahead[i] : (ok && pos == len ? slot : tab[pos]));
-    }
-    for (int pos = first + kListAhead * kListThreads; pos < L; pos += kListThreads)
-      emit(pos, ok && pos == len ? slot : tab[pos]);
-    for (int i = first; i < list.clear_per_req; i += kListThreads)
-      list.clear[(size_t)b * list.clear_per_req + i] = 0u;
-    if (first == 0) list.sel_len[b] = L;
+  for (int i = 0; i < kListAhead; ++i) {
+    const int pos = first + i * kListThreads;
+    if (pos < L) emit(pos, pos < known ? ahead[i] : (ok && pos == len ? slot : tab[pos]));
   }
+  for (int pos = first + kListAhead * kListThreads; pos < L; pos += kListThreads)
+    emit(pos, ok && pos == len ? slot : tab[pos]);
+  for (int i = first; i < list.clear_per_req; i += kListThreads)
+    list.clear[(size_t)b * list.clear_per_req + i] = 0u;
+  if (first == 0) list.sel_len[b] = L;
   __syncthreads();
   if (threadIdx.x == 0 && ok) {
     tab[len] = slot;
-    seq_lens[b] = len + 1;
+    st.seq_lens[b] = len + 1;
   }
 }
 
@@ -123,49 +115,6 @@ __global__ void seq_len_add_kernel(int32_t* seq_len, int rows, int max_tokens) {
   *seq_len = len > max_tokens ? max_tokens : len;
 }
 
-
-// Paged form of kv_store_kernel: the slot comes from the request's table, or from a
-// fresh page of the caller's free list when the length is a multiple of the page size
-// (ts_pages.h).  One workgroup per request; nothing of the plan is written before the
-// launch's last workgroup commits it.
-__global__ __launch_bounds__(256) void kv_store_paged_kernel(
-    const uint4* __restrict__ k, const uint4* __restrict__ v, uint4* __restrict__ k_pool,
-    uint4* __restrict__ v_pool, uint32_t pool_rows, int32_t* table, int64_t table_stride,
-    int32_t* seq_lens, int batch, int row_vec, int kv_stride, int max_tokens, int page_shift, PagePool pool) {
-  __shared__ uint32_t plan_slot, plan_ok;
-  const int b = blockIdx.x, lane = threadIdx.x & 63;
-  // (the new rows are asked for before the plan is made, not after)
-  const int first = threadIdx.x;
-  uint4 k0 = make_uint4(0u, 0u, 0u, 0u), v0 = k0;
-  if (first < row_vec) {
-    k0 = k[(size_t)b * kv_stride + first];
-    v0 = v[(size_t)b * kv_stride + first];
-  }
-  if (threadIdx.x < 64)
-    for_each_append(seq_lens, table, table_stride, batch, pool, page_shift, max_tokens, pool_rows,
-                    lane, [&](int req, const AppendPlan& p) {
-                      if (req == b) {
-                        plan_slot = p.slot;
-                        plan_ok = p.ok ? 1u : 0u;
-                      }
-                    });
-  __syncthreads();
-  if (plan_ok) {
-    const size_t slot = plan_slot;
-    if (first < row_vec) {
-      k_pool[slot * row_vec + first] = k0;
-      v_pool[slot * row_vec + first] = v0;
-    }
-    for (int i = first + blockDim.x; i < row_vec; i += blockDim.x) {
-      k_pool[slot * row_vec + i] = k[(size_t)b * kv_stride + i];
-      v_pool[slot * row_vec + i] = v[(size_t)b * kv_stride + i];
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < 64)
-    commit_appends(seq_lens, table, table_stride, batch, pool, page_shift, max_tokens, pool_rows,
-                   lane, gridDim.x);
-}
 
 // Where row r of a chunk goes when the request's table is paged: positions
 // len .. len + rows - 1 fill the request's last page and then fresh pages from the
@@ -257,30 +206,37 @@ int check_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t r
   return check_row_stride(row_stride, (int64_t)cfg->num_kv_heads * cfg->head_dim, "ts_kv_store");
 }
 
-int launch_kv_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
-                    const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
-                    int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t batch,
-                    int32_t max_tokens, hipStream_t stream, const DenseList* list) {
-  TS_TRY(check_kv_store(cfg, k, v, row_stride, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride,
-                        seq_lens, batch, max_tokens));
-  const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
-  TS_REQUIRE(list == nullptr || pages == nullptr, TS_EINVAL, "internal: a list needs a per-token table");
+StepStore step_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                     const int32_t* out_cache_loc, const ts_page_pool* pages, void* k_pool, void* v_pool,
+                     int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t max_tokens) {
+  StepStore st{};
+  st.k = (const uint4*)k;
+  st.v = (const uint4*)v;
+  st.loc = out_cache_loc;
+  st.k_pool = (uint4*)k_pool;
+  st.v_pool = (uint4*)v_pool;
+  st.pool_rows = pool_rows;
+  st.table = table;
+  st.table_stride = table_stride;
+  st.seq_lens = seq_lens;
+  st.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  st.kv_stride = row_stride ? (int)(row_stride / 8) : st.row_vec;
+  st.max_tokens = max_tokens;
   if (pages) {
-    hipLaunchKernelGGL(kv_store_paged_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
-                       (const uint4*)k, (const uint4*)v, (uint4*)k_pool, (uint4*)v_pool,
-                       (uint32_t)pool_rows, table, table_stride, seq_lens, batch, row_vec, kv_stride, max_tokens,
-                       page_shift_of(cfg->page_size), page_pool_of(pages));
-    return check_launch("kv_store_paged_kernel");
+    st.free_pages = pages->free_pages;
+    st.free_count = pages->free_count;
+    st.ticket = pages->ticket;
+    st.page_shift = page_shift_of(cfg->page_size);
   }
+  return st;
+}
+
+int launch_kv_store(const StepStore& st, int32_t batch, hipStream_t stream, const DenseList* list) {
+  TS_REQUIRE(list == nullptr || st.free_pages == nullptr, TS_EINVAL, "internal: a list needs a per-token table");
   if (list)
-    hipLaunchKernelGGL(kv_store_kernel<true>, dim3((unsigned)batch), dim3(kListThreads), 0, stream,
-                       (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                       pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens, *list);
+    hipLaunchKernelGGL(kv_store_list_kernel, dim3((unsigned)batch), dim3(kListThreads), 0, stream, st, *list);
   else
-    hipLaunchKernelGGL(kv_store_kernel<false>, dim3((unsigned)batch), dim3(256), 0, stream,
-                       (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                       pool_rows, table, table_stride, seq_lens, row_vec, kv_stride, max_tokens, DenseList{});
+    hipLaunchKernelGGL(kv_store_kernel, dim3((unsigned)batch), dim3(256), 0, stream, st);
   return check_launch("kv_store_kernel");
 }
 
@@ -346,8 +302,11 @@ extern "C" {
 int ts_kv_store(const ts_config* cfg, const void* k, const void* v, const int32_t* out_cache_loc,
                 const ts_page_pool* pages, void* k_pool, void* v_pool, int64_t pool_rows, int32_t* table,
                 int64_t table_stride, int32_t* seq_lens, int32_t batch, int32_t max_tokens, ts_stream_t stream) {
-  return launch_kv_store(cfg, k, v, 0, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride,
-                         seq_lens, batch, max_tokens, (hipStream_t)stream);
+  TS_TRY(check_kv_store(cfg, k, v, 0, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride, seq_lens,
+                        batch, max_tokens));
+  return launch_kv_store(step_store(cfg, k, v, 0, out_cache_loc, pages, k_pool, v_pool, pool_rows, table, table_stride,
+                                    seq_lens, max_tokens),
+                         batch, (hipStream_t)stream);
 }
 
 int ts_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, const int32_t* out_cache_loc,
