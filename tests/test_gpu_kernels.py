@@ -1612,3 +1612,21 @@ def test_fused_select_hint_with_ties_and_a_batch(dev):
         order = sorted(range(n), key=lambda t: (-v[t].item(), t))[:ks[b]]
         S = int(got[2][b])
         assert sorted(order) == (got[1][b, c.n_init:S - c.n_local] - c.n_init).tolist(), b
+
+
+@pytest.mark.parametrize("splits", [1, 4, 5, 8, 9, 16, 17, 24, 25, 49])
+def test_attention_merges_any_number_of_splits(dev, splits):
+    """A list of 128 entries per workgroup, the last of them short: the merge reads the splits 4, 8, 16 or
+    24 at a time.  Against the oracle (the tolerance of every attention test)."""
+    say(f"attention merge: splits={splits}")
+    for heads, kv_heads in ((14, 2), (2, 2)):
+        g = torch.Generator(device=dev).manual_seed(splits)
+        S = 128 * splits - 37
+        q, k_pool, v_pool = (torch.randn((n, h, 128), generator=g, device=dev).bfloat16()
+                             for n, h in ((1, heads), (S + 9, kv_heads), (S + 9, kv_heads)))
+        cfg = ops.LayerConfig(num_heads=heads, num_kv_heads=kv_heads, rope_theta=5e5)
+        sel = torch.randperm(S + 9, generator=g, device=dev)[:S].to(torch.int32).view(1, S)
+        out = ops.sparse_decode_attention(cfg, q, k_pool, v_pool, sel, torch.tensor([S], dtype=torch.int32, device=dev))
+        ref = oracle.attend.sparse_decode_attention(q[0].cpu(), k_pool.cpu(), v_pool.cpu(), sel[0].cpu(), 128 ** -0.5, 5e5)
+        err = (out.cpu().float().view(heads, 128) - ref.float()).abs().max().item()
+        assert err <= 2e-2, f"{splits} splits, {heads}/{kv_heads}: {err}"

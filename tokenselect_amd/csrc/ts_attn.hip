@@ -18,6 +18,9 @@
 
 namespace ts {
 
+constexpr int kAttnWaves = 4;  // wavefronts of a workgroup
+constexpr int kAttnThreads = 64 * kAttnWaves;
+
 struct AttnArgs {
   const uint16_t* q;  // [B,H,128] bf16, un-rotated, rows q_stride elements apart
   int q_stride;
@@ -49,7 +52,7 @@ __device__ __forceinline__ void attn_clear_on_the_side(const AttnArgs& a) {
   if (a.zero.used == 0) return;
   const uint32_t wg = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  clear_regions(a.zero, wg * 3 + wave - 1, gridDim.x * gridDim.y * gridDim.z * 3);
+  clear_regions(a.zero, wg * (kAttnWaves - 1) + wave - 1, gridDim.x * gridDim.y * gridDim.z * (kAttnWaves - 1));
 }
 
 __device__ __forceinline__ float2 load_coherent2(const float* p) {
@@ -102,7 +105,7 @@ __device__ __forceinline__ void attn_dense_epilogue(const AttnArgs& a, int b, in
     const int32_t* tab = a.sel + (int64_t)b * a.sel_stride;
     int32_t* const sel = a.step.sel + (int64_t)b * a.step.sel_stride;
     int32_t* const sel_pos = a.step.sel_pos + (int64_t)b * a.step.sel_stride;
-    for (int pos = lo + tid; pos < min(hi, S); pos += 256) {
+    for (int pos = lo + tid; pos < min(hi, S); pos += kAttnThreads) {
       const uint32_t entry = ((uint32_t)tab[min(pos, a.list_bound - 1) >> a.list_shift] << a.list_shift) +
                              (uint32_t)(pos & ((1 << a.list_shift) - 1));
       sel_pos[pos] = pos;
@@ -137,14 +140,14 @@ __device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, i
   uint32_t& s_last = *s_last_ptr;
   __syncthreads();
   // A thread owns two adjacent dims of one head: one 64-bit coherent store.
-  for (int idx = tid; idx < G * (kHeadDim / 2); idx += 256) {
+  for (int idx = tid; idx < G * (kHeadDim / 2); idx += kAttnThreads) {
     const int g = idx / (kHeadDim / 2), d = (idx % (kHeadDim / 2)) * 2;
     float mm = kNegBig;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sm_m[w][g]);
+    for (int w = 0; w < kAttnWaves; ++w) mm = fmaxf(mm, sm_m[w][g]);
     float o0 = 0.f, o1 = 0.f, ll = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < kAttnWaves; ++w) {
       const float sc = __expf(sm_m[w][g] - mm);
       o0 += sm_acc[w][g][d] * sc;
       o1 += sm_acc[w][g][d + 1] * sc;
@@ -167,42 +170,46 @@ __device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, i
     // (While the ticket is drawn, not ahead of the first loads: 0.6 us of the 38 that a layer of a
     // 32K request takes, 2.0 of 98 with eight of 8K.)
     attn_clear_on_the_side(a);
-    if (tid >= 192 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) attn_commit(a.commit);
+    if (tid >= kAttnThreads - 64 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) attn_commit(a.commit);
   }
   __syncthreads();
   if (!s_last) return false;
 
   // out[b,h,:] = sum_s exp(m_s - M) acc_s / sum_s exp(m_s - M) l_s, rounded to bf16.
   // A wavefront per head slot (a thread owns two adjacent dims, and a head has 64 such
-  // pairs): lane s fetches the (max, sum) of split s, the wave takes the maximum and
-  // lane s the weight of its split, so that the accumulators, all requested at once, are
-  // added up with weights that are ready (read lane by lane): no chain of dependent
-  // exponentials, and one statistics load per wave instead of one per split and thread.
+  // pairs): lane s fetches the (max, sum) of split s, so that the wave takes the maximum and
+  // lane s the weight of its split while the accumulators, all requested at once, are on their
+  // way, and they are added up with weights that are ready (read lane by lane): no chain of
+  // dependent exponentials, and one statistics load per wave instead of one per split and thread.
   // With more than four head slots a wavefront has two of them, and works on both at once:
-  // one after the other they would be two chains of loads.
+  // one after the other they would be two chains of loads (as they are behind a branch).
   static_assert(kHeadDim / 2 == 64, "one wavefront per head slot");
-  constexpr int SLOTS = (G + 3) / 4;  // head slots per wavefront: wave, wave + 4
+  constexpr int SLOTS = (G + kAttnWaves - 1) / kAttnWaves;  // head slots per wavefront
   const int wave_id = tid >> 6, d = lane * 2;
   size_t ph[SLOTS];
   float mm[SLOTS], ll[SLOTS], o0[SLOTS], o1[SLOTS];
 #pragma unroll
   for (int it = 0; it < SLOTS; ++it) {
     // (a slot past the last head repeats the last one and is not written)
-    ph[it] = ((size_t)b * H + head_of_slot(min(wave_id + 4 * it, G - 1))) * a.nsplit;
+    ph[it] = ((size_t)b * H + head_of_slot(min(wave_id + kAttnWaves * it, G - 1))) * a.nsplit;
     mm[it] = kNegBig;
     ll[it] = o0[it] = o1[it] = 0.f;
   }
-  for (int s0 = 0; s0 < a.nsplit; s0 += 32) {
-    // 32 splits at a time, branch-free: loads past the last split repeat it and get
-    // the weight zero.
-    float2 ac[SLOTS][32], ml[SLOTS];
+  // COUNT splits from s0 on, branch-free: loads past the last split repeat it and get the weight
+  // zero.  As few as hold the launch's splits: this step takes what one CU needs to fetch their
+  // accumulators, some 10 ns per load of 512 bytes.  With 32 loads for any number of splits it was 3
+  // to 3.7 us of an attention of 10 to 11; now 0.8 us for 3 splits, 2.4 for 21.  (Wavefronts that share
+  // a workgroup of eight, for half as many splits, share a SIMD: 2.5 us more for the tiles.)
+  auto add_splits = [&](int s0, auto count_c) __attribute__((always_inline)) {
+    constexpr int COUNT = decltype(count_c)::value;
+    float2 ac[SLOTS][COUNT], ml[SLOTS];
 #pragma unroll
     for (int it = 0; it < SLOTS; ++it) {
 #pragma unroll
-      for (int i = 0; i < 32; ++i)
+      for (int i = 0; i < COUNT; ++i)
         ac[it][i] = load_coherent2(a.part_acc + (ph[it] + min(s0 + i, a.nsplit - 1)) * kHeadDim + d);
-      ml[it] = (lane < 32 && s0 + lane < a.nsplit) ? load_coherent2(a.part_ml + (ph[it] + s0 + lane) * 2)
-                                                   : make_float2(kNegBig, 0.f);
+      ml[it] = (lane < COUNT && s0 + lane < a.nsplit) ? load_coherent2(a.part_ml + (ph[it] + s0 + lane) * 2)
+                                                      : make_float2(kNegBig, 0.f);
     }
 #pragma unroll
     for (int it = 0; it < SLOTS; ++it) {
@@ -211,27 +218,35 @@ __device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, i
       mx = fmaxf(mx, dpp_move<kRowRor4>(mx));
       mx = fmaxf(mx, dpp_move<kRowRor2>(mx));
       mx = fmaxf(mx, dpp_move<kRowRor1>(mx));
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      if (COUNT > 16) mx = fmaxf(mx, __shfl_xor(mx, 16));
       const float mn = fmaxf(mm[it], __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mx))));
       const float keep = __expf(mm[it] - mn);  // what earlier batches hold
-      const float w = (lane < 32 && s0 + lane < a.nsplit) ? __expf(ml[it].x - mn) : 0.f;
+      const float w = (lane < COUNT && s0 + lane < a.nsplit) ? __expf(ml[it].x - mn) : 0.f;
       const float wl = ml[it].y * w;
       o0[it] *= keep;
       o1[it] *= keep;
       ll[it] *= keep;
       mm[it] = mn;
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
+      for (int i = 0; i < COUNT; ++i) {
         const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), i));
         ll[it] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), i));
         o0[it] += ac[it][i].x * wi;
         o1[it] += ac[it][i].y * wi;
       }
     }
-  }
+  };
+  if (a.nsplit <= 4)
+    add_splits(0, std::integral_constant<int, 4>{});
+  else if (a.nsplit <= 8)
+    add_splits(0, std::integral_constant<int, 8>{});
+  else if (a.nsplit <= 16)
+    add_splits(0, std::integral_constant<int, 16>{});
+  else
+    for (int s0 = 0; s0 < a.nsplit; s0 += 24) add_splits(s0, std::integral_constant<int, 24>{});
 #pragma unroll
   for (int it = 0; it < SLOTS; ++it) {
-    const int g = wave_id + 4 * it;
+    const int g = wave_id + kAttnWaves * it;
     if (g < G) {
       const uint32_t packed = (uint32_t)f32_to_bf16(ll[it] > 0.f ? o0[it] / ll[it] : 0.f) |
                               ((uint32_t)f32_to_bf16(ll[it] > 0.f ? o1[it] / ll[it] : 0.f) << 16);
@@ -274,7 +289,7 @@ typedef __attribute__((ext_vector_type(4))) float at_f32x4;
 constexpr float kAttnLog2e = 1.4426950408889634f, kAttnLn2 = 0.6931471805599453f;
 constexpr uint32_t kNewRow = 0xffffffffu;  // the slot of a row that is not in the pool (no pool has as many)
 constexpr int kAttnTile = 32;        // tokens per step of a wavefront
-constexpr int kAttnChunkUnit = 64;   // a workgroup's range is a multiple of this (16 per wavefront)
+constexpr int kAttnChunkUnit = 16 * kAttnWaves;  // a workgroup's range is a multiple of this
 
 __device__ __forceinline__ at_bf16x8 pack8(const float* x) {
   const uint4 w = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]),
@@ -321,14 +336,14 @@ __device__ __forceinline__ int opaque_zero(uint32_t after) {
 // DENSE (AttnDense) is an instantiation of its own: with its few instructions in the one kernel the
 // attention over a list took 1 us more.
 template <int G, bool ROPE, bool CAP, bool DENSE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_kernel(AttnArgs a) {
+__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_kernel(AttnArgs a) {
   static_assert(G >= 1 && G <= 8, "the query heads of a KV head are columns of one tile");
   const int split = blockIdx.x, b = blockIdx.z, kvh = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, qd = lane >> 4;
   const int chunk = attn_chunk(a.max_sel_len, a.nsplit);
-  const int wlen = chunk / 4;
+  const int wlen = chunk / kAttnWaves;
   const int32_t* sel = a.sel + (int64_t)b * a.sel_stride;
   const size_t row_elems = (size_t)a.num_kv_heads * kHeadDim;
 
@@ -338,8 +353,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __shared__ __attribute__((aligned(16))) uint4 sm_q_lo[4][64];  // its low halves
   __shared__ __attribute__((aligned(16))) uint4 sm_pick[2][64];  // B operand per half, per lane
   __shared__ __attribute__((aligned(16))) float2 sm_step[kHeadDim / 2];  // (cos, sin) of 16 tokens
-  __shared__ float sm_acc[4][G][kHeadDim];
-  __shared__ float sm_m[4][G], sm_l[4][G];
+  __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
+  __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ uint32_t s_last;
 
   // Column n of the logits: query head n of the KV head (zeros beyond its heads).  Wavefront
@@ -647,13 +662,13 @@ __global__ __launch_bounds__(256) void attn_zero_kernel(uint32_t* tickets, int c
 // Tickets per request (the words to clear): one per KV head, and one for the heads of a dense step.
 int attn_tickets_per_request(const ts_config* cfg) { return cfg->num_kv_heads + 1; }
 
-constexpr int kAttnRange = 128;  // list entries per workgroup as long as the device has room
+constexpr int kAttnRange = kAttnTile * kAttnWaves;  // list entries per workgroup as long as the device has room
 static int attn_splits(int batch, int num_kv_heads, int max_sel_len) {
   // One tile per wavefront (128 entries per workgroup) as long as the grid stays within the
   // 512 workgroups that are resident at once (two per CU): a second round of workgroups pays
   // the start-up and merge latencies again, which costs more than longer ranges do.
   int64_t want = ceil_div(max_sel_len, kAttnRange);
-  const int64_t cap = ceil_div(512, (int64_t)batch * num_kv_heads);
+  const int64_t cap = ceil_div(2048 / kAttnWaves, (int64_t)batch * num_kv_heads);
   if (want > cap) want = cap;
   if (want < 1) want = 1;
   // (ranges are whole multiples of 64 entries: the last splits may have nothing left)
@@ -735,8 +750,8 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
   const bool rope = cfg->rope_mode == TS_ROPE_LLAMA, cap = cfg->logit_cap > 0.f;
 #define TS_ATTN_LAUNCH(G_, R_, C_)                                                                    \
   do {                                                                                                \
-    if (dense) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, true>), grid, dim3(256), 0, st, a);        \
-    else hipLaunchKernelGGL((attn_kernel<G_, R_, C_, false>), grid, dim3(256), 0, st, a);             \
+    if (dense) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, true>), grid, dim3(kAttnThreads), 0, st, a);        \
+    else hipLaunchKernelGGL((attn_kernel<G_, R_, C_, false>), grid, dim3(kAttnThreads), 0, st, a);             \
   } while (0)
 #define TS_ATTN_CASE(G_)                              \
   case G_:                                            \
