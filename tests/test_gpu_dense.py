@@ -246,3 +246,46 @@ def test_a_step_stores_as_the_store_does(dev, case):
         assert int(sides[0]["pages"].ticket) == 0
     if case in ("one", "page begins", "70 requests", "votes form"):
         assert sides[0]["lens"].tolist() == [n + steps for n in lengths]
+
+
+@pytest.mark.parametrize("length,rows,room,page", [(0, 40, 64, 1), (600, 512, 1200, 1), (1000, 100, 1050, 1), (31, 33, 64, 16),
+                                                   (640, 512, 1200, 16), (1000, 100, 1040, 16), (2400, 288, 2688, 1)])
+def test_a_dense_chunk_stores_as_the_store_does(dev, length, rows, room, page):
+    """A dense chunk, whose gather stores its rows, against ts_kv_store_chunk and the chunk on a fresh
+    object: length, table, pools, free pages, list and output bit for bit; tables that end within the
+    chunk, slots that are none of the pool's (clamped, each to a row of its own)."""
+    say(f"dense chunk that stores on the side: {length}+{rows} room {room} pages of {page}")
+    cfg = ops.LayerConfig(num_heads=14, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5, page_size=page)
+    g = torch.Generator(device=dev).manual_seed(14)
+    pages = room // page + 4
+    order = torch.randperm(pages - 2, generator=g, device=dev).to(torch.int32) + 1  # (the first and the last row stay free)
+    held = -(-length // page)
+    table = torch.zeros((1, room // page), dtype=torch.int32, device=dev)
+    table[0, :held] = order[:held]
+    start = [torch.randn((pages * page, 2, 128), generator=g, device=dev).bfloat16() for _ in range(2)]
+    q, k, v = (torch.randn((rows, n * 128), generator=g, device=dev).bfloat16() for n in (14, 2, 2))
+    loc = None
+    if page == 1:
+        loc = torch.cat([order[held:], order[:0]])[:rows].clone()
+        loc = torch.nn.functional.pad(loc, (0, rows - loc.shape[0]), value=int(order[-1]))  # (past the table: not stored)
+        loc[3], loc[5] = -7, pages + 11
+    got = []
+    for whole in (True, False):
+        s = dict(k=start[0].clone(), v=start[1].clone(), table=table.clone(),
+                 lens=torch.tensor([length], dtype=torch.int32, device=dev))
+        pool = None if page == 1 else ops.PagePool(order[held:].contiguous(), torch.tensor([pages - 2 - held], dtype=torch.int32, device=dev),
+                                                   torch.zeros(1, dtype=torch.int32, device=dev))
+        chunk = ops.PrefillChunk(cfg, min(length + rows, room), dev, max_rows=512)
+        chunk.workspace.fill_(0xff)
+        bt = ops.Batch(s["lens"], s["table"], min(length + rows, room))
+        if whole:
+            out, sel, sel_pos, sel_len = chunk.step(q, k, v, loc, s["k"], s["v"], bt, pages=pool)
+        else:
+            ops.kv_store_chunk(cfg, k, v, loc, s["k"], s["v"], s["table"][0], s["lens"], pages=pool)
+            out, sel, sel_pos, sel_len = chunk(q, s["k"], s["v"], bt)
+        got.append(dict(out=out.clone(), sel=sel.view(1, -1).clone(), sel_pos=sel_pos.view(1, -1).clone(),
+                        sel_len=sel_len.view(-1).clone(), lens=s["lens"], table=s["table"], k=s["k"], v=s["v"]))
+    torch.cuda.synchronize()
+    _same(*got)
+    assert torch.equal(got[0]["out"], got[1]["out"])
+    assert int(got[0]["lens"]) == min(length + rows, room)

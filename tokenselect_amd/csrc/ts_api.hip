@@ -272,7 +272,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                      int64_t sel_stride, int32_t* sel_len, void* workspace, size_t workspace_bytes,
                      ts_stream_t stream, const StepStore* store = nullptr,
                      const ChunkStore* chunk_store = nullptr, bool listed = false,
-                     const AttnDense* dense_step = nullptr) {
+                     const AttnDense* dense_step = nullptr, const PrefillDense* dense_chunk = nullptr) {
   TS_TRY(validate_config(cfg));
   TS_TRY(validate_batch(cfg, bt));
   SeparateKernelsScope separate(bt->separate_kernels != 0);
@@ -353,13 +353,16 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
     }
   }
   if (dense) {
+    if (chunk_rows > 0) TS_TRY(check_fingerprint(q, chunk_rows, q_cos, q_sin, table_rows, qf, cfg->n_local));
     if (dense_step)  // the attention reads the table, and leaves the list (and the new tokens) itself
       return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, bt->table, bt->table_stride, bt->seq_lens,
                          bt->batch, longest, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream, nullptr,
                          dense_step);
+    if (dense_chunk)
+      return launch_prefill_attn(cfg, q, q_stride, chunk_rows, k_pool, v_pool, pool_rows, sel, sel_len, longest, out,
+                                 ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream, dense_chunk);
     // (listed: the store has written the selection; otherwise the last of the top-k kernels,
     // which writes a dense request's list, is all that is left of the selection)
-    if (chunk_rows > 0) TS_TRY(check_fingerprint(q, chunk_rows, q_cos, q_sin, table_rows, qf, cfg->n_local));
     if (!listed) TS_TRY(launch_topk(topk, bt->batch, 0, (hipStream_t)stream));
     if (chunk_rows > 0)
       return launch_prefill_attn(cfg, q, q_stride, chunk_rows, k_pool, v_pool, pool_rows, sel, sel_len, longest, out,
@@ -628,21 +631,32 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
   TS_REQUIRE(bt->table != nullptr && bt->seq_lens != nullptr, TS_EINVAL, "ts_prefill_step: NULL table / seq_lens");
   int32_t* table = const_cast<int32_t*>(bt->table);
   int32_t* seq_len = const_cast<int32_t*>(bt->seq_lens);
-  // A chunk that is known to be dense has no fingerprint to ride in: its store writes the
-  // selection instead.
-  DenseList list{};
-  if (kv->pages == nullptr && bt->rerun == 0 &&
-      chunk_store_takes_list(rows, kv->max_tokens, bt->max_seq_len) &&
-      cfg->page_size == 1 && table_rows >= (int64_t)cfg->n_local + rows && (uintptr_t)cos_table % 16 == 0 &&
-      (uintptr_t)sin_table % 16 == 0)
-    list = step_list(cfg, bt, nullptr, q, cos_table, sin_table, out, sel, sel_pos, sel_stride, sel_len, workspace,
-                     workspace_bytes);
-  if (list.sel) {
-    TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
-                                 v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream, &list));
-    return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr, out,
-                     sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr,
-                     /*listed=*/true);
+  // A chunk that is known to be dense has no fingerprint for its store to ride in, and no selection:
+  // the gather reads the table and stores the rows (with a page pool, whose pages are taken in order,
+  // it finds them stored).
+  if (bt->rerun == 0 && table_rows >= (int64_t)cfg->n_local + rows && (uintptr_t)cos_table % 16 == 0 &&
+      (uintptr_t)sin_table % 16 == 0 &&
+      step_list(cfg, bt, nullptr, q, cos_table, sin_table, out, sel, sel_pos, sel_stride, sel_len, workspace,
+                workspace_bytes).sel) {
+    TS_TRY(check_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool, v_pool,
+                                pool_rows, table, seq_len, kv->max_tokens));
+    PrefillDense dense{};
+    dense.table = table;
+    dense.page_shift = page_shift_of(cfg->page_size);
+    dense.seq_len = seq_len;
+    dense.sel = sel;
+    dense.sel_pos = sel_pos;
+    dense.sel_len = sel_len;
+    dense.list_bound = bt->max_seq_len < kv->max_tokens ? bt->max_seq_len : kv->max_tokens;
+    if (kv->pages)
+      TS_TRY(launch_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool,
+                                   v_pool, pool_rows, table, seq_len, kv->max_tokens, (hipStream_t)stream));
+    else
+      dense.store = chunk_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, rows, k_pool, v_pool, pool_rows,
+                                table, seq_len, kv->max_tokens);
+    return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
+                     out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, nullptr,
+                     /*listed=*/true, nullptr, &dense);
   }
   const bool rides = kv->pages == nullptr && bt->rerun == 0 && kv->max_tokens <= 0x1fffff &&
                      rows <= 1023 * 16;
@@ -653,29 +667,10 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
     return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                      out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream);
   }
-  // The checks ts_kv_store_chunk makes.
-  TS_REQUIRE(kv->k && kv->v && kv->out_cache_loc && k_pool && v_pool, TS_EINVAL,
-             "ts_prefill_step: NULL tensor argument");
-  TS_REQUIRE_ALIGNED(kv->k, 16, "k");
-  TS_REQUIRE_ALIGNED(kv->v, 16, "v");
-  TS_REQUIRE_ALIGNED(k_pool, 16, "k_pool");
-  TS_REQUIRE_ALIGNED(v_pool, 16, "v_pool");
-  TS_REQUIRE(cfg->page_size == 1, TS_EINVAL, "ts_prefill_step: pages of %d tokens need a page pool", cfg->page_size);
-  TS_REQUIRE(pool_rows >= 1 && pool_rows <= 0x7fffffffLL && kv->max_tokens >= 1, TS_EINVAL,
-             "ts_prefill_step: pool_rows=%lld max_tokens=%d out of range", (long long)pool_rows, kv->max_tokens);
-  ChunkStore cs{};
-  cs.k = (const uint4*)kv->k;
-  cs.v = (const uint4*)kv->v;
-  cs.loc = kv->out_cache_loc;
-  cs.k_pool = (uint4*)k_pool;
-  cs.v_pool = (uint4*)v_pool;
-  cs.pool_rows = pool_rows;
-  cs.table = table;
-  cs.seq_len = seq_len;
-  cs.rows = rows;
-  cs.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  cs.kv_stride = kv_row_stride ? kv_row_stride / 8 : cs.row_vec;
-  cs.max_tokens = kv->max_tokens;
+  TS_TRY(check_kv_store_chunk(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, kv->pages, rows, k_pool, v_pool,
+                              pool_rows, table, seq_len, kv->max_tokens));
+  const ChunkStore cs = chunk_store(cfg, kv->k, kv->v, kv_row_stride, kv->out_cache_loc, rows, k_pool, v_pool, pool_rows,
+                                    table, seq_len, kv->max_tokens);
   return run_layer(cfg, bt, q, q_row_stride, rows, cos_table, sin_table, table_rows, k_pool, v_pool, pool_rows, nullptr,
                    out, sel, sel_pos, sel_stride, sel_len, workspace, workspace_bytes, stream, nullptr, &cs);
 }

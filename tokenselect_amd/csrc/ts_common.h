@@ -195,19 +195,38 @@ StepStore step_store(const ts_config* cfg, const void* k, const void* v, int64_t
                      int64_t pool_rows, int32_t* table, int64_t table_stride, int32_t* seq_lens, int32_t max_tokens);
 int launch_kv_store(const StepStore& st, int32_t batch, hipStream_t stream, const DenseList* list = nullptr);
 // ts_kv_store_chunk for rows of k and v that lie row_stride elements apart.
-// (list: only where chunk_store_takes_list says so)
-bool chunk_store_takes_list(int32_t rows, int32_t max_tokens, int32_t max_seq_len);
 int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
                           const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
                           void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
-                          hipStream_t stream, const DenseList* list = nullptr);
+                          hipStream_t stream);
+// What it requires of its arguments, and the rows for whatever launch stores them.
+int check_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                         const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, const void* k_pool,
+                         const void* v_pool, int64_t pool_rows, const int32_t* table, const int32_t* seq_len,
+                         int32_t max_tokens);
+ChunkStore chunk_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                       const int32_t* out_cache_loc, int32_t rows, void* k_pool, void* v_pool, int64_t pool_rows,
+                       int32_t* table, int32_t* seq_len, int32_t max_tokens);
 // What launch_fingerprint requires of its arguments.
 int check_fingerprint(const void* q, int32_t rows, const float* cos_table, const float* sin_table,
                       int64_t table_rows, const void* qf, int32_t n_local);
+// A chunk that attends to all tokens: its gather reads the table, and stores the chunk's rows and
+// writes the list itself; the attention after it, which reads neither, writes the length.
+struct PrefillDense {
+  const int32_t* table;  // in pages of 1 << page_shift
+  int page_shift;
+  int32_t* seq_len;      // before the append, where there is one
+  int32_t* sel;          // the selection that is left behind
+  int32_t* sel_pos;
+  int32_t* sel_len;
+  int list_bound;        // entries that are there to be read, and the most that are listed
+  ChunkStore store;      // k == NULL: no append, the length counts the chunk already
+};
 // ts_sparse_prefill_attn for query rows that lie q_stride elements apart.
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
-                        int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes, hipStream_t stream);
+                        int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                        const PrefillDense* dense = nullptr);
 
 // Sparse decode attention (ts_attn.hip).  The kernel counts its workgroups in per
 // (request, KV head) tickets inside the workspace, which must be zero at launch:

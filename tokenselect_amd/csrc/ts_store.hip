@@ -82,32 +82,9 @@ __global__ __launch_bounds__(kListThreads) void kv_store_list_kernel(StepStore s
 // fingerprint launch of a chunk can also run on the side.
 constexpr int kChunkRowsPerWg = 256 / kChunkThreadsPerRow;  // few workgroups, few counts on one word
 
-// The workgroups past the first cs_wgs write the chunk's dense selection (list): entries
-// before the chunk from the table, those of the chunk from the caller's slots.
 template <bool COUNTED>
-__global__ __launch_bounds__(256) void kv_store_chunk_kernel(
-    const uint4* __restrict__ k, const uint4* __restrict__ v, const int32_t* __restrict__ loc,
-    uint4* __restrict__ k_pool, uint4* __restrict__ v_pool, int64_t pool_rows,
-    int32_t* table, int32_t* seq_len, int rows, int row_vec, int kv_stride, int max_tokens, int cs_wgs,
-    DenseList list) {
-  ChunkStore cs{k, v, loc, k_pool, v_pool, pool_rows, table, seq_len, rows, row_vec, max_tokens, kv_stride, (int)gridDim.x};
-  if (!COUNTED || (int)blockIdx.x < cs_wgs) {
-    store_chunk_rows<COUNTED>(cs, (int)blockIdx.x, 256);
-    return;
-  }
-  const int len = counted_length(cs);
-  const int L = min(max(min(len + rows, max_tokens), 0), list.max_seq_len);
-  const int pos = ((int)blockIdx.x - cs_wgs) * 256 + (int)threadIdx.x;
-  if (pos < L) {
-    // (a slot of the chunk is clamped to the pool as it is stored, an entry as it is looked up)
-    const int32_t at = pos < len ? table[pos] : loc[pos - len];
-    const uint32_t s = pos >= len && at < 0 ? 0u : (uint32_t)at;
-    list.sel_pos[pos] = pos;
-    list.sel[pos] = (int32_t)(s < (uint32_t)pool_rows ? s : (uint32_t)pool_rows - 1);
-  }
-  if (pos == 0) *list.sel_len = L;
-  if (pos < list.clear_per_req) list.clear[pos] = 0u;
-  count_chunk_workgroup(cs, len);
+__global__ __launch_bounds__(256) void kv_store_chunk_kernel(ChunkStore cs) {
+  store_chunk_rows<COUNTED>(cs, (int)blockIdx.x, 256);
 }
 
 __global__ void seq_len_add_kernel(int32_t* seq_len, int rows, int max_tokens) {
@@ -240,17 +217,10 @@ int launch_kv_store(const StepStore& st, int32_t batch, hipStream_t stream, cons
   return check_launch("kv_store_kernel");
 }
 
-static int chunk_list_workgroups(int32_t max_seq_len) { return (int)ceil_div(max_seq_len, 256); }
-
-bool chunk_store_takes_list(int32_t rows, int32_t max_tokens, int32_t max_seq_len) {
-  return max_tokens <= kLenMask &&
-         ceil_div(rows, kChunkRowsPerWg) + chunk_list_workgroups(max_seq_len) <= kChunkCountedWgs;
-}
-
-int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
-                          const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
-                          void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
-                          hipStream_t stream, const DenseList* list) {
+int check_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                         const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, const void* k_pool,
+                         const void* v_pool, int64_t pool_rows, const int32_t* table, const int32_t* seq_len,
+                         int32_t max_tokens) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(k && v && k_pool && v_pool && table && seq_len, TS_EINVAL,
              "ts_kv_store_chunk: NULL tensor argument");
@@ -262,12 +232,37 @@ int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, in
   TS_REQUIRE(rows >= 0 && pool_rows >= 1 && pool_rows <= 0x7fffffffLL && max_tokens >= 1, TS_EINVAL,
              "ts_kv_store_chunk: rows=%d pool_rows=%lld max_tokens=%d out of range", rows,
              (long long)pool_rows, max_tokens);
+  return check_row_stride(row_stride, (int64_t)cfg->num_kv_heads * cfg->head_dim, "ts_kv_store_chunk");
+}
+
+ChunkStore chunk_store(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                       const int32_t* out_cache_loc, int32_t rows, void* k_pool, void* v_pool, int64_t pool_rows,
+                       int32_t* table, int32_t* seq_len, int32_t max_tokens) {
+  ChunkStore cs{};
+  cs.k = (const uint4*)k;
+  cs.v = (const uint4*)v;
+  cs.loc = out_cache_loc;
+  cs.k_pool = (uint4*)k_pool;
+  cs.v_pool = (uint4*)v_pool;
+  cs.pool_rows = pool_rows;
+  cs.table = table;
+  cs.seq_len = seq_len;
+  cs.rows = rows;
+  cs.row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
+  cs.kv_stride = row_stride ? (int)(row_stride / 8) : cs.row_vec;
+  cs.max_tokens = max_tokens;
+  return cs;
+}
+
+int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, int64_t row_stride,
+                          const int32_t* out_cache_loc, const ts_page_pool* pages, int32_t rows, void* k_pool,
+                          void* v_pool, int64_t pool_rows, int32_t* table, int32_t* seq_len, int32_t max_tokens,
+                          hipStream_t stream) {
+  TS_TRY(check_kv_store_chunk(cfg, k, v, row_stride, out_cache_loc, pages, rows, k_pool, v_pool, pool_rows, table,
+                              seq_len, max_tokens));
   if (rows == 0) return TS_OK;
   const int row_vec = cfg->num_kv_heads * cfg->head_dim * 2 / 16;
-  TS_TRY(check_row_stride(row_stride, row_vec * 8, "ts_kv_store_chunk"));
   const int kv_stride = row_stride ? (int)(row_stride / 8) : row_vec;
-  TS_REQUIRE(list == nullptr || (pages == nullptr && chunk_store_takes_list(rows, max_tokens, list->max_seq_len)),
-             TS_EINVAL, "internal: a list of %d rows does not ride in the chunk's store", rows);
   if (pages) {
     hipLaunchKernelGGL(kv_store_chunk_paged_kernel, dim3((unsigned)rows), dim3(256), 0,
                        stream, (const uint4*)k, (const uint4*)v, (uint4*)k_pool,
@@ -276,17 +271,14 @@ int launch_kv_store_chunk(const ts_config* cfg, const void* k, const void* v, in
     return check_launch("kv_store_chunk_paged_kernel");
   }
   const unsigned wgs = (unsigned)ceil_div(rows, kChunkRowsPerWg);
+  ChunkStore cs = chunk_store(cfg, k, v, row_stride, out_cache_loc, rows, k_pool, v_pool, pool_rows, table, seq_len,
+                              max_tokens);
+  cs.workgroups = (int)wgs;
   if (wgs <= (unsigned)kChunkCountedWgs && max_tokens <= kLenMask) {
-    const unsigned list_wgs = list ? (unsigned)chunk_list_workgroups(list->max_seq_len) : 0u;
-    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs + list_wgs), dim3(256), 0, stream,
-                       (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                       pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens, (int)wgs,
-                       list ? *list : DenseList{});
+    hipLaunchKernelGGL(kv_store_chunk_kernel<true>, dim3(wgs), dim3(256), 0, stream, cs);
     return check_launch("kv_store_chunk_kernel");
   }
-  hipLaunchKernelGGL(kv_store_chunk_kernel<false>, dim3(wgs), dim3(256), 0, stream,
-                     (const uint4*)k, (const uint4*)v, out_cache_loc, (uint4*)k_pool, (uint4*)v_pool,
-                     pool_rows, table, seq_len, rows, row_vec, kv_stride, max_tokens, (int)wgs, DenseList{});
+  hipLaunchKernelGGL(kv_store_chunk_kernel<false>, dim3(wgs), dim3(256), 0, stream, cs);
   TS_TRY(check_launch("kv_store_chunk_kernel"));
   hipLaunchKernelGGL(seq_len_add_kernel, dim3(1), dim3(1), 0, stream, seq_len, rows,
                      max_tokens);
