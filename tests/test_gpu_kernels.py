@@ -3,7 +3,9 @@ the C ABI.  Tolerances: fp32 scores 1e-3 relative (to the score RMS); selected
 positions identical up to ties at the k-th vote; bf16 attention output 2e-2
 absolute."""
 
+import ctypes
 import random
+import threading
 
 import pytest
 import torch
@@ -1630,3 +1632,35 @@ def test_attention_merges_any_number_of_splits(dev, splits):
         ref = oracle.attend.sparse_decode_attention(q[0].cpu(), k_pool.cpu(), v_pool.cpu(), sel[0].cpu(), 128 ** -0.5, 5e5)
         err = (out.cpu().float().view(heads, 128) - ref.float()).abs().max().item()
         assert err <= 2e-2, f"{splits} splits, {heads}/{kv_heads}: {err}"
+
+
+def test_a_threads_plans_are_those_of_a_fresh_thread(dev):
+    """A thread keeps the last few plans of the selection: whatever was asked before, and by whichever
+    switch, the layout, the form and the sizes are those that a thread without any plan reports."""
+    lib = _lib.load()
+    shapes = [dict(num_heads=H, num_kv_heads=8 if H == 32 else 4, n_init=n_init, n_local=512, pool_kernel=pool)
+              for H in (32, 28) for n_init in (128, 64) for pool in (0, 5)]
+    asked = [(ops.LayerConfig(top_k=2048, **shape).to_c(), batch, length)
+             for shape in shapes for batch in (1, 2) for length in (600, 641, 2003, 32768)]
+
+    def answer(c, batch, length):
+        r = ctypes.byref(c)
+        return (lib.ts_decode_layer_layout(r, batch, length), lib.ts_decode_layer_selection(r, batch, length),
+                lib.ts_decode_layer_workspace_bytes(r, batch, length), lib.ts_select_workspace_bytes(r, batch, length))
+
+    def fresh(*one):
+        got = []
+        thread = threading.Thread(target=lambda: got.append(answer(*one)))
+        thread.start()
+        thread.join()
+        return got[0]
+
+    for fused in (1, 0, 1):
+        was = lib.ts_set_fused_select(fused)
+        try:
+            want = [fresh(*one) for one in asked]
+            for order in (range(len(asked)), reversed(range(len(asked)))):
+                for i in order:
+                    assert answer(*asked[i]) == want[i] and answer(*asked[i]) == want[i]
+        finally:
+            lib.ts_set_fused_select(was)
