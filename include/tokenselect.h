@@ -108,10 +108,10 @@ typedef struct ts_batch {
                                coarse code of where the k-th vote lay there and uses
                                the previous step's as a guess: while the votes of a
                                layer drift slowly from step to step, as the queries
-                               do, the selection is then through after one meeting of
-                               its workgroups instead of two (C2: 5 us of 60).  Only
-                               ever a guess: a wrong or stale value costs the saving
-                               and some 4 us, never the result, which is exact          */
+                               do, the selection is then through without a meeting of
+                               its workgroups instead of after two (C2: 6 us of 60).
+                               Only ever a guess: a wrong or stale value costs the
+                               saving and some 3 us, never the result, which is exact   */
   /* Per-call options; all zero = the defaults. */
   int32_t separate_kernels; /* 1: this call selects with ts_score + ts_vote +
                                ts_topk_ragged's kernels, whose workgroups never wait
@@ -276,8 +276,9 @@ int ts_topk_ragged(const ts_config* cfg, const ts_batch* bt, const float* votes,
  * candidates are left around the k-th vote, which are listed and ranked by every
  * workgroup in a last round together with the per-workgroup counts that place its
  * selected positions in the output (masses of exact ties take all three histogram
- * rounds and a count round).  With bt->threshold_hint they meet once when the k-th
- * vote lies near the hint, and once more than without when it does not; with
+ * rounds and a count round).  With bt->threshold_hint they need not meet when the k-th
+ * vote lies near the hint (what they hand over is its own flag again), and meet as often
+ * as without when it does not; with
  * cfg->pool_kernel > 0 once more in any case: the max-pool of tr.py:366-369 needs
  * the votes of the neighbouring workgroups.  Outputs and the hit / cache arguments are those of
  * ts_topk_ragged (same tie rule: lowest position first); votes, when not NULL,

@@ -1664,3 +1664,31 @@ def test_a_threads_plans_are_those_of_a_fresh_thread(dev):
                     assert answer(*asked[i]) == want[i] and answer(*asked[i]) == want[i]
         finally:
             lib.ts_set_fused_select(was)
+
+
+@pytest.mark.parametrize("length,k,rows", [(140000, 2048, 0), (6000, 256, 5), (6000, 256, 40), (3000, 64, 300)])
+def test_fused_select_hint_where_the_band_is_crowded(dev, length, k, rows):
+    """The counts that the workgroups send: of more than 256 workgroups (two of them to a thread), and of
+    bins with more tokens than a count's field or a bin's slots hold (`rows` distinct keys, so that hundreds
+    of tokens share each vote).  Bit for bit the launch without a hint, with the right hint and with hints
+    that put the crowded bins at every place of the band."""
+    import dataclasses
+    say(f"fused select, crowded band: L={length} k={k} rows={rows}")
+    wl = small(dev, SHAPES[0], seed=107, lens=[length], ks=[k], page=16, top_k=k)
+    c = wl.cfg
+    if rows:
+        wl.k_pool.copy_(wl.k_pool[torch.arange(wl.k_pool.shape[0], device=dev) % rows])
+    qf = fingerprint(wl, dev) * (0.02 if rows == 300 else 1.0)   # (votes close together, or far apart)
+    space = ops.select_workspace(c, wl.batch, dev)
+    want = ops.select(c, wl.batch, qf, wl.k_pool, workspace=space)[:3]
+    hint = torch.zeros(1, dtype=torch.int32, device=dev)
+    hinted = dataclasses.replace(wl.batch, hint=hint)
+    ops.select(c, hinted, qf, wl.k_pool, workspace=space)
+    code = int(hint[0])
+    for off in range(-5, 7):
+        hint.fill_(code + off)
+        got = ops.select(c, hinted, qf, wl.k_pool, workspace=space)[:3]
+        torch.cuda.synchronize()
+        assert not ops.select_fault(c, hinted, space), off
+        assert all(torch.equal(x, y) for x, y in zip(got, want)), off
+        assert int(hint[0]) == code, off

@@ -82,8 +82,7 @@ struct ScoreArgs {
   uint32_t absent;        // team members that never arrive (tests of the give-up path)
   uint32_t* fault_out;    // caller's word, set to 1 when a wait gave up, or NULL
   int32_t* hint;          // [B] threshold bin + 1 of the last selection (0: none), or NULL
-  uint32_t* band_above;   // [B][kBandBins][kSelMaxChunks]: tokens of a workgroup above a band bin << 16 | in it
-  uint4* band_slots;      // [B][kBandBins][kSelMaxChunks]: kBandSlots packed candidates
+  uint64_t* band;         // [B][kBandRows][kSelMaxChunks], zero at launch
   int pool_kernel;        // max-pool window over the votes (tr.py:366-369), <= 0: off
   float* pool_votes;      // [B,pool_stride] un-pooled votes exchanged between workgroups
   int64_t pool_stride;
@@ -121,27 +120,35 @@ constexpr int kSelListCap = 256;
 constexpr int kSelListParts = 8;
 constexpr int kSelListCount = kSelMaxBin + kSelHistCopies * 32;
 // With a hint of where the threshold bin is going to be (ts_batch.threshold_hint: the bin of
-// the request's previous selection on the same layer), every workgroup publishes, together
-// with its histogram and before the first rendezvous, what the last round would otherwise
-// need a rendezvous of its own for, for each of the kBandBins bins around the hint: one word
-// with the number of its tokens above that bin and of its candidates in it; those
-// candidates (up to kBandSlots, packed into 32 bits each: the low 21 key bits and the
-// token's index in the workgroup, which is why the band needs workgroups of at most 1024
-// tokens; into a 16-byte piece of its own, no counter to reserve from, and only the entries
-// the word counts are ever read, so nothing is cleared); and its counts of the band's bins
-// added to a small histogram of the band (kBandHistCopies copies a line apart, slot
-// kBandBins of each: the tokens above the band).  After the rendezvous the small histogram
-// says whether the threshold bin lies in the band, and if no workgroup had more candidates
-// in it than slots, the selection is through: one rendezvous, and a fraction of the
-// histogram to read.  Every memory-side atomic counts here (a few thousand of them in a
-// microsecond are what the device serves): a narrow band, and nothing written that is empty.
+// the request's previous selection on the same layer), every workgroup sends, in place of its
+// histogram, what the last round would otherwise need a rendezvous of its own for, for the
+// kBandBins bins around the hint: how many of its tokens lie in each of them and above them all
+// (two words of 64 bits), and those candidates (up to kBandSlots a bin, packed into 32 bits each:
+// the low 21 key bits and the token's index in the workgroup, which is why the band needs
+// workgroups of at most 1024 tokens; two to a word).  No word that is sent is zero and all are zero
+// before a launch, so each is its own flag: a thread per workgroup asks for them until they have
+// come, adds the counts up, and if the threshold bin lies in the band and no workgroup had more
+// candidates in it than fit, the selection is through without any rendezvous.  (With a rendezvous
+// and a histogram of the band in memory between the sending and the reading a layer of one request
+// of 32K tokens took 0.4 us more, one of eight requests of 3-16K 1.5 us.)
 constexpr int kBandBins = 8;
 constexpr int kBandBelow = 4;   // the band is [hint - kBandBelow, hint - kBandBelow + kBandBins)
-constexpr int kBandSlots = 4;   // candidates a workgroup can publish per bin (one 16-byte piece)
+constexpr int kBandSlots = 4;   // candidates a workgroup can send per bin (two words)
 constexpr int kBandMaxTokens = 1024;  // tokens per workgroup the packed index can address
-constexpr int kBandHistCopies = 32;   // one 128-byte line each: adds to one line are served one by one
-constexpr int kSelBandHist = kSelListCount + kSelListParts * 32;  // copies x 32 words (kBandBins + 1 live)
-constexpr int kSelCounterWords = kSelBandHist + kBandHistCopies * 32;
+// The word of counts: a field of six bits per bin (31: that many or more), the count above the band,
+// whether a field is 31, the flag.  Two such words can be added field by field.
+constexpr int kBandCountBits = 6, kBandOverAt = kBandBins * kBandCountBits;
+constexpr uint32_t kBandCountMost = 31u, kBandCountMask = 63u, kBandOverMask = 4095u;
+constexpr uint64_t kBandFields = (1ull << kBandOverAt) - 1ull;
+constexpr uint64_t kBandEven = 0x03f03f03f03full;    // every other field
+constexpr uint64_t kBandLowest = 0x041041041041ull;  // the lowest bit of every field
+constexpr uint64_t kBandFull = 1ull << 60, kBandSent = 1ull << 62;
+// The word goes to as many rows, of which a workgroup reads one: all reading the same keep its
+// lines from those who write (and 32 bytes of each asked for by everyone took 5 us).
+constexpr int kBandReplicas = 8;
+constexpr int kBandRows = kBandReplicas + 2 * kBandBins;  // the counts, then two words of candidates per bin
+__device__ __forceinline__ int band_piece_row(int bin, int half) { return kBandReplicas + 2 * bin + half; }
+constexpr int kSelCounterWords = kSelListCount + kSelListParts * 32;
 
 // Workgroups of one request the workspace of ts_select is laid out for (the device keeps
 // at most 512 resident at once).
@@ -149,7 +156,7 @@ constexpr int kSelMaxChunks = 1024;
 
 // Workspace of ts_select, carved in this order (256-byte aligned pieces).
 struct SelectWorkspace {
-  size_t partials, counters, stats, block_counts, short_list, band_above, band_slots, pool_votes, sync,
+  size_t partials, counters, stats, block_counts, short_list, pool_votes, sync,
       total;  // sync stays last
   int64_t stats_stride;
   int64_t pool_stride;

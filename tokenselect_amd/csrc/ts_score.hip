@@ -491,8 +491,8 @@ __device__ __forceinline__ void fixed_segments(const ScoreArgs& a, const Lengths
   for (int i = threadIdx.x; i < a.n_local; i += 256) emit(a.n_init + k + i, L - a.n_local + i);
 }
 
-// Sum over the wavefront, in every lane.
-__device__ __forceinline__ uint32_t wave_total(uint32_t x) {
+// Sum over the 16 lanes of a DPP row, in every lane of it.
+__device__ __forceinline__ uint32_t row16_total(uint32_t x) {
   auto ror = [](uint32_t v, auto ctrl) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
   };
@@ -500,6 +500,11 @@ __device__ __forceinline__ uint32_t wave_total(uint32_t x) {
   x += ror(x, std::integral_constant<int, kRowRor4>{});
   x += ror(x, std::integral_constant<int, kRowRor2>{});
   x += ror(x, std::integral_constant<int, kRowRor1>{});
+  return x;
+}
+// Sum over the wavefront, in every lane.
+__device__ __forceinline__ uint32_t wave_total(uint32_t x) {
+  x = row16_total(x);
   return (uint32_t)(__builtin_amdgcn_readlane((int)x, 0) + __builtin_amdgcn_readlane((int)x, 16) +
                     __builtin_amdgcn_readlane((int)x, 32) + __builtin_amdgcn_readlane((int)x, 48));
 }
@@ -1045,7 +1050,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     static_assert(kBandSlots == 4, "a workgroup's candidates of a bin are one 16-byte piece");
     __shared__ uint32_t band_lds[kBandBins][kBandSlots];
     __shared__ uint32_t band_count[kBandBins + 1];  // per bin; [kBandBins]: tokens above the band
-    __shared__ uint32_t band_sum[kBandBins + 2];    // the same over all workgroups; a bin's candidates do not fit
+    // Over all workgroups: [0..3] the counts of two bins each, [4] the tokens above the band, [8] how many
+    // bins from the lowest on hold one without room for its count, [9] a bin's candidates do not fit.
+    __shared__ uint32_t band_sum[kBandBins + 2];
     for (int i = tid; i < kTopkBins; i += 256) lh[i] = 0u;
     if (tid < 16) scratch[tid] = 0u;
     if (tid < kBandBins * kBandSlots) band_lds[tid / kBandSlots][tid % kBandSlots] = 0u;
@@ -1199,7 +1206,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // performed one after the other, which for 256 candidates is a few hundred cycles).
     const int hint_bin = hint_word - 1;
     const bool banded = hint_bin >= 0 && hint_bin < kTopkBins && lp.tokens_per_block <= kBandMaxTokens &&
-                        req_chunks <= kSelMaxChunks / 2;
+                        req_chunks <= kSelMaxChunks / 2 && a.absent == 0u;
     const int band_lo = hint_bin - kBandBelow;  // (bins outside [0, kTopkBins) hold nothing)
     if (banded) {
       uint32_t over_band = 0;  // this thread's tokens above the band
@@ -1235,9 +1242,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // of the copies and note the highest occupied bin; afterwards each searches
     // downwards from that bin, 256 bins at a time (one is enough unless the votes
     // span more than 64 binades).  With a hint the band's counts go out instead, and the
-    // histogram only follows, a rendezvous later, when the threshold turns out to lie outside
-    // the band: some 40 of a workgroup's 70 read-modify-writes, which the device serves at
-    // 10-15 thousand a microsecond.
+    // histogram only follows when the threshold turns out to lie outside the band.
     uint32_t* hist0 = ctr + kSelHist0 + (chunk % kSelHistCopies) * kTopkBins;
     auto publish_histogram = [&]() {
       // Two adjacent bins per 64-bit add (their counts cannot carry into each other):
@@ -1255,67 +1260,88 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         done += fetch_max_coherent(&ctr[kSelMaxBin + (chunk % kSelHistCopies) * 32], scratch[8]);
       await(done);
     };
+    uint64_t* const band = a.band + (size_t)b * kBandRows * kSelMaxChunks;  // [kBandRows][workgroup]
     if (!banded) {
       publish_histogram();
-    } else if (wave < 2) {
-      // The band, its words by one wavefront and its histogram by another.  Lane l holds the count of band bin l (lane kBandBins: of the bins above
-      // the band); the tokens above bin l are the sum over the lanes after it.
-      uint64_t done = 0;
-      uint4* slots = a.band_slots + (size_t)b * kBandBins * kSelMaxChunks;
-      uint32_t* above = a.band_above + (size_t)b * kBandBins * kSelMaxChunks;
-      const uint32_t here = lane <= kBandBins ? band_count[lane] : 0u;
-      if (wave == 1) {
-        if (here) done += fetch_add_coherent(&ctr[kSelBandHist + (chunk % kBandHistCopies) * 32 + lane], here);
-      } else {
-      uint32_t run = here;  // becomes the sum over lanes l .. l + 15
+    } else if (wave == 0) {
+      // The candidates of bin l by lane l (none when they do not fit, since the bin is then not
+      // ranked from the band), then the counts.  Nothing waits for these stores: no word of them
+      // is zero, and whoever needs one asks until it has come.
+      const uint32_t here = lane < kBandBins ? band_count[lane] : 0u;
+      if (here >= 1 && here <= (uint32_t)kBandSlots) {
+        store_coherent(&band[(size_t)band_piece_row(lane, 0) * kSelMaxChunks + chunk],
+                       (uint64_t)band_lds[lane][0] | ((uint64_t)band_lds[lane][1] << 32));
+        if (here >= 3)
+          store_coherent(&band[(size_t)band_piece_row(lane, 1) * kSelMaxChunks + chunk],
+                         (uint64_t)band_lds[lane][2] | ((uint64_t)band_lds[lane][3] << 32));
+      }
+      const bool full = __any(here >= kBandCountMost);
+      uint32_t low = 0, high = 0;  // four counts each
 #pragma unroll
-      for (int off = 1; off < 16; off <<= 1) {
-        const uint32_t up = (uint32_t)__shfl_down((int)run, off);
-        run += lane + off < 64 ? up : 0u;
+      for (int d = 0; d < 4; ++d) {
+        low |= min(band_count[d], kBandCountMost) << (d * kBandCountBits);
+        high |= min(band_count[4 + d], kBandCountMost) << (d * kBandCountBits);
       }
-      static_assert(kBandBins + 1 <= 16, "the sum spans the band");
-      if (lane < kBandBins) {
-        done += __hip_atomic_exchange(&above[(size_t)lane * kSelMaxChunks + chunk], ((run - here) << 16) | here,
-                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // (the candidates: the first 8-byte half of the piece, the second only if used; none
-        // when they do not fit, since the bin is then not ranked from the band)
-        uint64_t* piece = (uint64_t*)&slots[(size_t)lane * kSelMaxChunks + chunk];
-        if (here >= 1 && here <= (uint32_t)kBandSlots)
-          done += __hip_atomic_exchange(piece, (uint64_t)band_lds[lane][0] | ((uint64_t)band_lds[lane][1] << 32),
-                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (here >= 3 && here <= (uint32_t)kBandSlots)
-          done += __hip_atomic_exchange(piece + 1, (uint64_t)band_lds[lane][2] | ((uint64_t)band_lds[lane][3] << 32),
-                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      }
-      await(done);
+      if (lane < kBandReplicas)
+        store_coherent(&band[(size_t)lane * kSelMaxChunks + chunk],
+                       (uint64_t)low | ((uint64_t)high << (4 * kBandCountBits)) |
+                           ((uint64_t)band_count[kBandBins] << kBandOverAt) |
+                           (full ? kBandFull : 0ull) | kBandSent);
     }
     TS_MARK(7);
-    grid_arrive(lp.sync, ++round, a.spin_ticks, team.size, team.index);
+    if (!banded) grid_arrive(lp.sync, ++round, a.spin_ticks, team.size, team.index);
     TS_MARK(8);
     uint32_t t0 = 0, above0 = 0, in_bin0 = 0;
-    // With a hint: the band's small histogram, the flags, the counts of the workgroups before
-    // this one and every workgroup's slots for the bin the hint names are requested
-    // together (the bin is a guess: the threshold bin is known after the search, and
-    // another bin of the band costs one more round of loads).
+    // With a hint: every workgroup's counts and its candidates of the bin the hint names, a thread
+    // per workgroup, asked for until they have come (the bin is a guess: the threshold bin is
+    // known after the search, and another bin of the band costs one more round of loads).
     constexpr int kBandLoads = kSelMaxChunks / 2 / 256;  // (512 chunks at most)
-    uint32_t band_word[kBandLoads];
-    uint4 band_piece[kBandLoads];
-    auto load_band = [&](int d) {
-      const uint32_t* above = a.band_above + ((size_t)b * kBandBins + d) * kSelMaxChunks;
-      const uint4* slots = a.band_slots + ((size_t)b * kBandBins + d) * kSelMaxChunks;
-#pragma unroll
-      for (int r = 0; r < kBandLoads; ++r) {
-        const int at = tid + 256 * r;
-        band_word[r] = 0u;
-        band_piece[r] = make_uint4(0u, 0u, 0u, 0u);
-        if (at < req_chunks) {
-          band_word[r] = load_coherent(&above[at]);
-          const uint64_t lo = __hip_atomic_load((const uint64_t*)&slots[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          const uint64_t hi = __hip_atomic_load((const uint64_t*)&slots[at] + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          band_piece[r] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    uint64_t band_counts[kBandLoads];
+    uint64_t band_piece[kBandLoads][2];
+    auto band_here = [&](int r, int d) {  // candidates in bin d
+      return (uint32_t)(band_counts[r] >> (d * kBandCountBits)) & kBandCountMask;
+    };
+    // Asks with `ask` until that says that all has come; bounded, as every wait is.
+    auto until_come = [&](auto&& ask) {
+      const uint64_t t_start = wall_clock64();
+      for (uint32_t polls = 1; !__all(ask()); ++polls) {
+        if ((polls & 15u) == 0) {
+          if (load_coherent(&lp.sync[0]) != 0u) break;
+          if (wall_clock64() - t_start > a.spin_ticks) {
+            __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+          }
         }
+        __builtin_amdgcn_s_sleep(1);
       }
+    };
+    auto load_counts = [&]() {
+      const uint64_t* from = &band[(size_t)(team.index % kBandReplicas) * kSelMaxChunks];
+      until_come([&]() {
+        bool come = true;
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r) {
+          const int at = tid + 256 * r;
+          band_counts[r] = at < req_chunks ? load_coherent(&from[at]) : 0ull;
+          come = come && (at >= req_chunks || band_counts[r] != 0ull);
+        }
+        return come;
+      });
+    };
+    auto load_pieces = [&](int d) {
+      until_come([&]() {
+        bool come = true;
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r) {
+          const int at = tid + 256 * r;
+          const uint32_t here = band_here(r, d);
+          const bool fits = here >= 1 && here <= (uint32_t)kBandSlots;
+          band_piece[r][0] = fits ? load_coherent(&band[(size_t)band_piece_row(d, 0) * kSelMaxChunks + at]) : 0ull;
+          band_piece[r][1] = fits && here >= 3 ? load_coherent(&band[(size_t)band_piece_row(d, 1) * kSelMaxChunks + at]) : 0ull;
+          come = come && (!fits || (band_piece[r][0] != 0ull && (here < 3 || band_piece[r][1] != 0ull)));
+        }
+        return come;
+      });
     };
     bool found = false;     // the threshold bin is known
     bool from_band = false; // and its candidates are in `entries`
@@ -1325,13 +1351,23 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // Appends the band's candidates of the loaded bin and counts the tokens above it in the
     // workgroups before this one; a workgroup with more candidates than slots is noted.
     auto gather_band = [&](uint32_t bin) {
-      uint32_t before = 0;
+      const int bin_at = (int)bin - band_lo;
+      // What the workgroups before this one hold above the bin: their fields of six bits, added
+      // in pairs, then the pairs.
+      uint64_t lower = 0;
+#pragma unroll
+      for (int r = 0; r < kBandLoads; ++r) lower += tid + 256 * r < chunk ? band_counts[r] : 0ull;
+      uint32_t before = (uint32_t)(lower >> kBandOverAt) & kBandOverMask;
+      lower = (lower & kBandFields) >> (kBandCountBits * bin_at);
+      lower = ((lower >> 6) & kBandEven) + ((lower >> 12) & kBandEven);
+      lower += lower >> 24;
+      before += ((uint32_t)lower & 0xfffu) + ((uint32_t)(lower >> 12) & 0xfffu);
 #pragma unroll
       for (int r = 0; r < kBandLoads; ++r) {
-        const uint32_t packed[4] = {band_piece[r].x, band_piece[r].y, band_piece[r].z, band_piece[r].w};
+        const uint32_t packed[4] = {(uint32_t)band_piece[r][0], (uint32_t)(band_piece[r][0] >> 32),
+                                    (uint32_t)band_piece[r][1], (uint32_t)(band_piece[r][1] >> 32)};
         const uint32_t from = (uint32_t)(tid + 256 * r) * (uint32_t)lp.tokens_per_block;  // that workgroup's first token
-        uint32_t have = band_word[r] & 0xffffu;  // (zero where the load was skipped)
-        if (tid + 256 * r < chunk) before += band_word[r] >> 16;
+        uint32_t have = band_here(r, bin_at);  // (zero where the load was skipped)
         if (have > (uint32_t)kBandSlots) {
           band_sum[kBandBins + 1] = 1u;
           have = 0u;
@@ -1355,27 +1391,46 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       if (lane == 0 && before) atomicAdd(&scratch[10], before);
     };
     if (banded) {
-      constexpr int kWords = kBandHistCopies * (kBandBins + 1);
-      constexpr int kPerThread = (kWords + 255) / 256;
-      uint32_t part[kPerThread];
+      load_counts();
+      TS_MARK(16);
+      load_pieces(kBandBelow);
+      TS_MARK(17);
+      // The counts of all workgroups: two fields to a register, 16 lanes each, then in LDS; and the
+      // highest bin that some workgroup's field has no room for.
+      {
+        uint64_t both = 0;
 #pragma unroll
-      for (int r = 0; r < kPerThread; ++r) {
-        const int word = tid + 256 * r;
-        part[r] = word < kWords
-                      ? load_coherent(&ctr[kSelBandHist + (word / (kBandBins + 1)) * 32 + word % (kBandBins + 1)])
-                      : 0u;
+        for (int r = 0; r < kBandLoads; ++r) {
+          both += band_counts[r];
+          if (__builtin_expect((band_counts[r] & kBandFull) != 0ull, 0)) {
+            uint64_t ones = band_counts[r] & kBandFields;  // becomes: the lowest bit of a field of ones
+            ones &= ones >> 1;
+            ones &= (ones >> 2) & (ones >> 3);
+            ones &= kBandLowest;
+            if (ones) atomicMax(&band_sum[kBandBins], (63u - (uint32_t)__builtin_clzll(ones)) / kBandCountBits + 1u);
+          }
+        }
+        uint32_t sums[kBandBins / 2 + 1];
+#pragma unroll
+        for (int j = 0; j < kBandBins / 2; ++j) {
+          const uint32_t two = (uint32_t)(both >> (2 * j * kBandCountBits));
+          sums[j] = (two & kBandCountMask) | ((two >> kBandCountBits & kBandCountMask) << 16);
+        }
+        sums[kBandBins / 2] = (uint32_t)(both >> kBandOverAt) & kBandOverMask;
+#pragma unroll
+        for (int j = 0; j <= kBandBins / 2; ++j) sums[j] = row16_total(sums[j]);
+        if ((lane & 15) == 0) {
+#pragma unroll
+          for (int j = 0; j <= kBandBins / 2; ++j) atomicAdd(&band_sum[j], sums[j]);
+        }
       }
-      load_band(kBandBelow);
-#pragma unroll
-      for (int r = 0; r < kPerThread; ++r)
-        if (part[r]) atomicAdd(&band_sum[(tid + 256 * r) % (kBandBins + 1)], part[r]);
       gather_band((uint32_t)hint_bin);
       __syncthreads();
       // Downwards from the bins above the band: the bin in which the count reaches k.
-      uint32_t sums[kBandBins + 1];
+      uint32_t sums[kBandBins];
 #pragma unroll
-      for (int d = 0; d <= kBandBins; ++d) sums[d] = band_sum[d];
-      uint32_t run = sums[kBandBins];
+      for (int d = 0; d < kBandBins; ++d) sums[d] = band_sum[d / 2] >> (16 * (d & 1)) & 0xffffu;
+      uint32_t run = band_sum[kBandBins / 2];
       int d0 = -1;
 #pragma unroll
       for (int d = kBandBins - 1; d >= 0; --d) {
@@ -1386,7 +1441,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         }
         if (d0 < 0) run += sums[d];
       }
-      if (d0 >= 0 && band_lo + d0 >= 0) {
+      // (the sums above the highest bin without room are exact, and the threshold has to lie there)
+      if (d0 >= (int)band_sum[kBandBins] && band_lo + d0 >= 0) {
         found = true;
         t0 = (uint32_t)(band_lo + d0);
         above0 = run;
@@ -1394,7 +1450,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
           if (d0 != kBandBelow) {  // another bin of the band: once more, with its words
             __syncthreads();
             if (tid == 0) scratch[10] = scratch[15] = band_sum[kBandBins + 1] = 0u;
-            load_band(d0);
+            load_pieces(d0);
             __syncthreads();
             gather_band(t0);
             __syncthreads();
@@ -1988,7 +2044,8 @@ static SelectWorkspace plan_select_workspace(const ts_config* cfg, int batch, in
     off += align_up(bytes, 256);
     return at;
   };
-  w.partials = take(B * H * (size_t)kSelMaxChunks * 2 * sizeof(float));
+  w.partials = take(B * H * (size_t)kSelMaxChunks * 2 * sizeof(float) +
+                    B * kBandRows * (size_t)kSelMaxChunks * sizeof(uint64_t));  // (rows of the same size)
   // The counters and, right behind them, the replicas of the statistics are cleared
   // together before every launch.
   w.counters = take(B * kSelCounterWords * 4);
@@ -1996,8 +2053,6 @@ static SelectWorkspace plan_select_workspace(const ts_config* cfg, int batch, in
   w.stats = take((size_t)kSyncSlots * w.stats_stride * sizeof(float));
   w.block_counts = take(B * (size_t)kSelMaxChunks * sizeof(uint2));
   w.short_list = take(B * kSelListParts * kSelListCap * sizeof(uint2));
-  w.band_above = take(B * kBandBins * (size_t)kSelMaxChunks * sizeof(uint32_t));
-  w.band_slots = take(B * kBandBins * (size_t)kSelMaxChunks * sizeof(uint4));
   w.pool_stride = (int64_t)align_up((size_t)std::max(max_n, 1), 64);
   w.pool_votes = take(cfg->pool_kernel > 0 ? B * (size_t)w.pool_stride * sizeof(float) : 0);
   w.sync = take(B * kSyncWords * 4);  // one rendezvous area per launch of a batch served in groups
@@ -2053,14 +2108,14 @@ bool plan_vote_launches(const ts_config* cfg, const ts_batch* bt, VotePlan* plan
 
 // The per-workgroup statistics are their own flags (a sum of exponentials is never
 // zero): the chunks a launch may fill have to be zero before it, `chunks` of every
-// (request, head) row.
-static ZeroRegion partials_zero_region(const SelectWorkspace& w, void* workspace, int batch, int heads,
+// (request, head) row, and of every row of the bands behind them.
+static ZeroRegion partials_zero_region(const SelectWorkspace& w, void* workspace, int batch, int rows,
                                        int chunks) {
   ZeroRegion z;
   z.base = (uint32_t*)((char*)workspace + w.partials);
   z.stride = (int64_t)kSelMaxChunks * 2;
   z.words = std::min(chunks, kSelMaxChunks) * 2;
-  z.count = batch * heads;
+  z.count = batch * rows;
   return z;
 }
 static ZeroRegion stats_zero_region(const SelectWorkspace& w, void* workspace, int batch, int heads) {
@@ -2090,7 +2145,7 @@ void select_zero_regions(const ts_config* cfg, const SelectWorkspace& w, void* w
   zero->add(counters);
   zero->add(stats_zero_region(w, workspace, batch, cfg->num_heads));
   zero->add(sync_zero_region(w, workspace, 1));
-  zero->add(partials_zero_region(w, workspace, batch, cfg->num_heads, w.clear_chunks));
+  zero->add(partials_zero_region(w, workspace, batch, cfg->num_heads + kBandRows, w.clear_chunks));
 }
 
 void score_votes_zero_regions(const ts_config* cfg, const ts_batch* bt, const SelectWorkspace& w,
@@ -2194,8 +2249,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
   a.block_counts = (uint2*)(ws + w.block_counts);
   a.short_list = (uint2*)(ws + w.short_list);
   a.hint = bt->threshold_hint;
-  a.band_above = (uint32_t*)(ws + w.band_above);
-  a.band_slots = (uint4*)(ws + w.band_slots);
+  a.band = (uint64_t*)(ws + w.partials) + (size_t)bt->batch * cfg->num_heads * kSelMaxChunks;
   a.sel = sel;
   a.sel_pos = sel_pos;
   a.sel_stride = sel_stride;
