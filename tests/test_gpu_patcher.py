@@ -418,3 +418,42 @@ def test_rows_of_k_and_v_match_the_step(dev):
     assert retriever.num_tokens == [0] and not pool.k_buffer[0].any() and not pool.v_buffer[0].any()
     attn.forward(q, rows[1], rows[1], meta)
     assert retriever.num_tokens == [1] and bool((pool.k_buffer[0][3] == 1).all())
+
+
+@pytest.mark.parametrize("chunk,prompt", [(64, 192), (32, 339), (32, 900), (64, 1000)])
+def test_a_prompts_chunks_hand_on_where_the_threshold_lay(dev, monkeypatch, chunk, prompt):
+    """A chunk that adds at most a tenth to its context gets the threshold of the chunk before as a guess:
+    bit for bit the outputs of chunks without one, of the right guess and of nonsense; shorter contexts
+    neither read nor leave one."""
+    H, Hkv, D = 8, 2, 128
+    say(f"chunks with hints: chunk {chunk}, prompt {prompt}")
+    monkeypatch.setattr(tr, "PREFILL_CHUNK_SIZE", 512)
+    tr.patch(rope_base=1e4, rope_scale=1, rope_model="ROPE_LLAMA", max_n_tokens=1024, top_k=24, n_init=4, n_local=32)
+    tr.PREFILL_CHUNK_SIZE = chunk
+    g = torch.Generator(device=dev).manual_seed(23)
+    q, k, v = (torch.randn(prompt, n * D, generator=g, device=dev).bfloat16() for n in (H, Hkv, Hkv))
+    slots = torch.randperm(1024, generator=g, device=dev).to(torch.int32)[:prompt].contiguous()
+    plain = tr.TokenRetriever._chunk_hint
+
+    def run(hint):
+        monkeypatch.setattr(tr.TokenRetriever, "_chunk_hint", hint)
+        pool = sg.TokenToKVPool(1024, torch.bfloat16, Hkv, D, 1, dev)
+        runner = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool,
+                                dtype=torch.bfloat16)
+        retriever = runner.req_to_token_retriever.get_token_retriever("req-hints")
+        attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
+        out = attn.forward(q, k, v, sg.InputMetadata(sg.ForwardMode.EXTEND, retriever, pool, slots))
+        torch.cuda.synchronize()
+        return out, int(retriever._chunk_hints[0])
+
+    want, left = run(lambda self, layer, before, rows: None)
+    assert left == 0
+    got, left = run(plain)
+    assert torch.equal(got, want)
+    assert (left != 0) == any(s >= 10 * min(chunk, prompt - s) for s in range(0, prompt, chunk))
+    nonsense = torch.empty(1, dtype=torch.int32, device=dev)
+
+    def wild(self, layer, before, rows):
+        return nonsense.fill_((before * 37) % 4096 - 1000)
+
+    assert torch.equal(run(wild)[0], want)
