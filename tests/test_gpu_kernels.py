@@ -1692,3 +1692,26 @@ def test_fused_select_hint_where_the_band_is_crowded(dev, length, k, rows):
         assert not ops.select_fault(c, hinted, space), off
         assert all(torch.equal(x, y) for x, y in zip(got, want)), off
         assert int(hint[0]) == code, off
+
+
+@pytest.mark.parametrize("page", [1, 16])
+@pytest.mark.parametrize("n,k", [(16383, 16382), (16384, 16383), (16385, 16384), (40000, 39999), (40000, 700), (33, 32)])
+def test_topk_slices_full_of_selected_positions(dev, n, k, page):
+    """The last top-k kernel lists a slice of 16384 positions in LDS before it looks their slots up: slices
+    with all positions selected, with one left out, of one position, and a request without candidates beside
+    it.  Positions and slots exactly, sinks and local window included."""
+    say(f"topk slices: n={n} k={k} page={page}")
+    lens = [n + 24, 20]
+    wl = small(dev, SHAPES[0], seed=9, lens=lens, ks=[k, k], page=page, top_k=k)
+    votes = torch.zeros((2, ops.score_stride_for(lens[0])), dtype=torch.float32, device=dev)
+    v = torch.randperm(n, generator=torch.Generator().manual_seed(n)).float()   # (no ties)
+    votes[0, :n] = v.to(dev)
+    sel, pos, slen = ops.topk_ragged(wl.cfg, wl.batch, votes)
+    torch.cuda.synchronize()
+    picked = torch.sort(torch.argsort(v, descending=True)[:k]).values + 8
+    want = torch.cat([torch.arange(8), picked, torch.arange(lens[0] - 16, lens[0])])
+    assert slen.tolist() == [k + 24, 20]
+    for b, w in enumerate((want, torch.arange(20))):
+        assert torch.equal(pos[b, :len(w)].cpu().long(), w)
+        table = wl.batch.table[b].cpu().long()
+        assert torch.equal(sel[b, :len(w)].cpu().long(), table[w // page] * page + w % page)
