@@ -3,6 +3,9 @@ and nothing is scored.  Compared with the general path, which a call takes when 
 a k of their own (the same k here).  And steps of a growing context, which start with the selection
 as long as the workspace's layout stays what the step before left clean."""
 
+import os
+
+import numpy as np
 import pytest
 import torch
 
@@ -289,3 +292,44 @@ def test_a_dense_chunk_stores_as_the_store_does(dev, length, rows, room, page):
     _same(*got)
     assert torch.equal(got[0]["out"], got[1]["out"])
     assert int(got[0]["lens"]) == min(length + rows, room)
+
+
+ROUNDING = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "attn_rounding.npz")
+
+
+def rounding_outputs(dev, heads, kv_heads):
+    """Attention outputs (int16 bit patterns) of seeded inputs: the first step of an object, whose
+    attention reads a list, and five more, whose attention reads the table."""
+    cfg = ops.LayerConfig(num_heads=heads, num_kv_heads=kv_heads, n_init=128, n_local=512, top_k=2048, rope_theta=5e5)
+    g = torch.Generator().manual_seed(heads)
+    lengths = [2003, 1500, 517, 2600, 64, 1999, 1024, 300]
+    B, total = len(lengths), 12000
+    randn = lambda *shape: torch.randn(shape, generator=g).bfloat16().to(dev)
+    order = torch.randperm(total, generator=g).to(torch.int32).to(dev)
+    table, at = torch.zeros((B, 2700), dtype=torch.int32, device=dev), 0
+    for b, n in enumerate(lengths):
+        table[b, :n] = order[at:at + n]
+        at += n
+    k_pool, v_pool = randn(total, kv_heads, 128), randn(total, kv_heads, 128)
+    lens = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    layer, outs = ops.DecodeLayer(cfg, B, 2688, dev), []
+    for t in range(6):
+        q, k, v = randn(B, heads * 128), randn(B, kv_heads * 128), randn(B, kv_heads * 128)
+        loc = order[at + B * t:at + B * (t + 1)].clone()
+        bt = ops.Batch(lens, table, max(lengths) + t + 1)
+        outs.append(layer.step(q, k, v, loc, k_pool, v_pool, bt)[0].clone())
+    torch.cuda.synchronize()
+    return torch.stack(outs).cpu().contiguous().view(torch.int16).numpy()
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(8, 2), (7, 1), (4, 4)])
+def test_attention_rounds_as_it_did(dev, heads, kv_heads):
+    """The rotations of queries and keys say which of their products is rounded: the outputs keep their
+    bits whatever else changes in the kernel.  The fixture holds rounding_outputs() of the kernel
+    before its attention read tables (a compiler that contracts on its own gave others since)."""
+    say(f"rounding of the attention: {heads} heads on {kv_heads}")
+    want = np.load(ROUNDING)[f"{heads}_{kv_heads}"]
+    got = rounding_outputs(dev, heads, kv_heads)
+    assert got.shape == want.shape
+    differ = np.argwhere(got != want)
+    assert differ.shape[0] == 0, f"{differ.shape[0]} of {want.size} outputs: {differ[:8].tolist()}"

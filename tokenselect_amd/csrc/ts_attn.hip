@@ -449,8 +449,10 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
             a.rope_rcp_scale * __builtin_amdgcn_exp2f(-(float)pair * (2.0f / kHeadDim) * a.log2_theta);
         float sn, cs;
         sincos_reduced((float)(S - 1) * freq, sn, cs);
-        const float xr = x[e] * cs - y[e] * sn;
-        y[e] = y[e] * cs + x[e] * sn;
+        // (which product is rounded is said here and for the keys below: left to the compiler it
+        // changed with code elsewhere in the kernel, and one output in some 3000 by an ulp)
+        const float xr = fmaf(x[e], cs, -(y[e] * sn));
+        y[e] = fmaf(y[e], cs, x[e] * sn);
         x[e] = xr;
       }
     }
@@ -518,8 +520,8 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
               const float c = kc[8 * kb2 + e], sn = ks[8 * kb2 + e];
-              const float xr = x[e] * c - y[e] * sn;
-              y[e] = y[e] * c + x[e] * sn;
+              const float xr = fmaf(x[e], c, -(y[e] * sn));
+              y[e] = fmaf(y[e], c, x[e] * sn);
               x[e] = xr;
             }
           }
@@ -553,8 +555,8 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
               for (int o = 0; o < 2; ++o) {
                 const int i = 8 * kb2 + 2 * e2 + o;
-                const float c2 = kc[i] * dcs[o] - ks[i] * dsn[o];
-                ks[i] = ks[i] * dcs[o] + kc[i] * dsn[o];
+                const float c2 = fmaf(kc[i], dcs[o], -(ks[i] * dsn[o]));
+                ks[i] = fmaf(kc[i], dsn[o], ks[i] * dcs[o]);
                 kc[i] = c2;
               }
             }
