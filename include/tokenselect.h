@@ -128,7 +128,9 @@ typedef struct ts_batch {
   int32_t absent_workgroups; /* tests of the give-up path only (0 in production):
                                workgroups counted as members of every rendezvous
                                that never arrive, so that every wait gives up
-                               after wait_us while all kernels still exit        */
+                               after wait_us while all kernels still exit (with a
+                               threshold_hint, where there is no rendezvous: the
+                               waits of all but a request's first workgroup)     */
   int32_t workspace_clean;  /* ts_decode_layer and ts_decode_step.  1: the caller states that
                                this workspace was last used by one of these calls with
                                the same cfg, batch, max_seq_len (or one of the same

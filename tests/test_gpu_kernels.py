@@ -1576,6 +1576,60 @@ def test_fused_select_with_a_threshold_hint(dev, shape):
     run(q2, want2)
 
 
+@pytest.mark.parametrize("lens,ks", [([40000], [512]), ([3000, 40, 1531], [64, 64, 100])])
+def test_hinted_select_reports_a_wait_that_gave_up(dev, lens, ks):
+    """A selection whose hint holds meets nobody, and its waits for the other workgroups' words are
+    bounded like any other: forced (a member that all but a request's first workgroup wait for in vain,
+    a bound of 1 ms, which the statistics before keep), the request is reported though its first workgroup was through long before, and
+    the next launch is that of a fresh one."""
+    import dataclasses
+    say(f"fused select with hints, forced give-up lens={lens}")
+    wl = small(dev, SHAPES[0], seed=111, lens=lens, ks=ks, page=16, top_k=max(ks))
+    c, B = wl.cfg, len(lens)
+    qf = fingerprint(wl, dev)
+    word = ops.fault_word()
+    hint = torch.zeros(B, dtype=torch.int32, device=dev)
+    bt = dataclasses.replace(wl.batch, hint=hint, fault=word)
+    space = ops.select_workspace(c, bt, dev)
+    want = [t.clone() for t in ops.select(c, bt, qf, wl.k_pool, workspace=space)[:3]]
+    codes = hint.clone()
+    for launch in range(3):
+        hint.copy_(torch.where(codes > 0, codes + 1, 0))   # (still in the band)
+        sel_len = ops.select(c, bt, qf, wl.k_pool, workspace=space, wait_ticks=100_000, absent_workgroups=1)[2]
+        torch.cuda.synchronize()
+        assert torch.equal(hint, codes), "the first workgroup was through"
+        assert sel_len.tolist() == [-1 if n > 200 else n for n in lens], launch
+        assert int(word[0]) == 1 and ops.select_fault(c, bt, space)
+        word.zero_()
+    got = ops.select(c, bt, qf, wl.k_pool, workspace=space)[:3]
+    torch.cuda.synchronize()
+    assert int(word[0]) == 0 and not ops.select_fault(c, bt, space)
+    assert torch.equal(got[2], want[2])
+    for b, S in enumerate(want[2].tolist()):
+        assert torch.equal(got[0][b, :S], want[0][b, :S]) and torch.equal(got[1][b, :S], want[1][b, :S])
+
+
+def test_layer_object_recovers_a_hinted_step_that_gave_up(dev):
+    """The same through a decode layer: steps with hints, one that gives up, recover()."""
+    import dataclasses
+    lens, ks = [3000, 40, 1531], [64, 64, 100]
+    say(f"decode layer with hints, forced give-up and recovery lens={lens}")
+    wl = small(dev, SHAPES[0], seed=112, lens=lens, ks=ks, page=16, top_k=100)
+    bt = dataclasses.replace(wl.batch, hint=torch.zeros(3, dtype=torch.int32, device=dev))
+    layer = ops.DecodeLayer(wl.cfg, 3, max(lens), dev)
+    for _ in range(2):
+        got = layer(wl.q, wl.k_pool, wl.v_pool, bt)
+        torch.cuda.synchronize()
+        assert not layer.gave_up()
+    forced = dataclasses.replace(bt, wait_us=20, absent_workgroups=1)
+    sel_len = layer(wl.q, wl.k_pool, wl.v_pool, forced)[3]
+    torch.cuda.synchronize()
+    assert layer.gave_up() and sel_len.tolist() == [-1, 40, -1]
+    got = layer.recover(wl.q, wl.k_pool, wl.v_pool, forced)
+    torch.cuda.synchronize()
+    layer_matches_oracle(wl, *got, "recovered step")
+
+
 def test_fused_select_hint_with_ties_and_a_batch(dev):
     """The band path where it is hardest: exact ties at the k-th vote inside and across
     workgroups (duplicated key rows), and a batch whose requests differ in length, one of them

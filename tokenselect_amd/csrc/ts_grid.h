@@ -39,11 +39,17 @@ __device__ __forceinline__ void store_coherent(uint2* p, uint32_t x, uint32_t y)
 __device__ __forceinline__ uint32_t fetch_add_coherent(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ uint32_t fetch_or_coherent(uint32_t* p, uint32_t v) {
+  return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ uint32_t fetch_max_coherent(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ uint64_t load_coherent(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_coherent(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void store_coherent(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -84,6 +90,13 @@ __device__ __forceinline__ bool grid_count(uint32_t* sync, uint32_t round, uint3
                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == members;
 }
 
+// Says for the launch that a wait gave up.  Performed when this returns: whatever the workgroup
+// publishes next is seen by others only after the word is.
+__device__ __forceinline__ void raise_fault(uint32_t* sync) {
+  __hip_atomic_store(&sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // A whole wavefront polls the replica of its workgroup, lane g the word of group g, until
 // every group has completed `round`.
 __device__ __forceinline__ void grid_poll(uint32_t* sync, uint32_t round, uint64_t ticks,
@@ -97,7 +110,7 @@ __device__ __forceinline__ void grid_poll(uint32_t* sync, uint32_t round, uint64
       // Some workgroup has given up already: the launch is lost, do not wait again.
       if (load_coherent(&sync[0]) != 0u) break;
       if (wall_clock64() - t0 > ticks) {
-        __hip_atomic_store(&sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_fault(sync);
         break;
       }
     }
@@ -182,7 +195,7 @@ __device__ __forceinline__ uint64_t poll_nonzero(const uint64_t* p, uint32_t* sy
     if ((polls & 15u) == 0) {
       if (load_coherent(&sync[0]) != 0u) return 0ull;
       if (wall_clock64() - t0 > ticks) {
-        __hip_atomic_store(&sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        raise_fault(sync);
         return 0ull;
       }
     }

@@ -113,6 +113,12 @@ constexpr int kSelHist2 = kSelHist1 + kSelHist1Copies * kTopkBins;  // 1024, las
 // Highest occupied bin of hist0, one word per copy, 128 bytes apart (hundreds of
 // read-modify-writes of one address, or one line, take microseconds).
 constexpr int kSelMaxBin = kSelHist2 + 1024;
+// Whether the length that workgroup 0 of the request has written stands, two bits in one word:
+// kSelDecided by that workgroup when it is through, kSelLost by one that gave up waiting for the
+// band.  A wait for the band has no rendezvous after it, so workgroup 0 can be through while
+// another is still waiting: whichever of the two comes second knows of both, and reports it.
+constexpr int kSelVerdict = kSelMaxBin + 1;
+constexpr uint32_t kSelDecided = 1u, kSelLost = 2u;
 // Once at most kSelListCap candidates are left in the threshold bin they are listed
 // instead of being resolved by further histogram levels; the list is kept in parts
 // with a fill counter each (128 bytes apart), workgroup x appending to part x % parts.

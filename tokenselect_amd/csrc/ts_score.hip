@@ -186,7 +186,7 @@ __device__ __forceinline__ void merge_request_stats(const ScoreArgs& a, const La
           if (load_coherent(&lp.sync[0]) != 0u) {
             lost = true;
           } else if (wall_clock64() - t0 > a.spin_ticks) {
-            __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            raise_fault(lp.sync);
             lost = true;
           }
         }
@@ -1206,7 +1206,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // performed one after the other, which for 256 candidates is a few hundred cycles).
     const int hint_bin = hint_word - 1;
     const bool banded = hint_bin >= 0 && hint_bin < kTopkBins && lp.tokens_per_block <= kBandMaxTokens &&
-                        req_chunks <= kSelMaxChunks / 2 && a.absent == 0u;
+                        req_chunks <= kSelMaxChunks / 2;
     const int band_lo = hint_bin - kBandBelow;  // (bins outside [0, kTopkBins) hold nothing)
     if (banded) {
       uint32_t over_band = 0;  // this thread's tokens above the band
@@ -1288,6 +1288,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
                            ((uint64_t)band_count[kBandBins] << kBandOverAt) |
                            (full ? kBandFull : 0ull) | kBandSent);
     }
+    // (Ahead of the waits that follow: in memory before this workgroup decides that it stands.)
+    if (chunk == 0 && tid == 0) store_coherent((uint32_t*)&a.sel_len[b], (uint32_t)(a.n_init + (int)k + a.n_local));
     TS_MARK(7);
     if (!banded) grid_arrive(lp.sync, ++round, a.spin_ticks, team.size, team.index);
     TS_MARK(8);
@@ -1301,16 +1303,21 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     auto band_here = [&](int r, int d) {  // candidates in bin d
       return (uint32_t)(band_counts[r] >> (d * kBandCountBits)) & kBandCountMask;
     };
-    // Asks with `ask` until that says that all has come; bounded, as every wait is.
+    // Asks with `ask` until that says that all has come; bounded, as every wait is.  On giving up
+    // (or when another wait did) the request is lost: what this workgroup is going to write is
+    // wrong, and if the length stands already it is taken back here.
     auto until_come = [&](auto&& ask) {
       const uint64_t t_start = wall_clock64();
       for (uint32_t polls = 1; !__all(ask()); ++polls) {
-        if ((polls & 15u) == 0) {
-          if (load_coherent(&lp.sync[0]) != 0u) break;
-          if (wall_clock64() - t_start > a.spin_ticks) {
-            __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
+        if ((polls & 15u) == 0 &&
+            (load_coherent(&lp.sync[0]) != 0u || wall_clock64() - t_start > a.spin_ticks)) {
+          raise_fault(lp.sync);
+          if (lane == 0 && (fetch_or_coherent(&ctr[kSelVerdict], kSelLost) & kSelDecided) != 0u) {
+            store_coherent((uint32_t*)&a.sel_len[b], 0xffffffffu);
+            if (a.fault_out)
+              __hip_atomic_store(a.fault_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           }
+          break;
         }
         __builtin_amdgcn_s_sleep(1);
       }
@@ -1318,7 +1325,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     auto load_counts = [&]() {
       const uint64_t* from = &band[(size_t)(team.index % kBandReplicas) * kSelMaxChunks];
       until_come([&]() {
-        bool come = true;
+        // (An absent member, in tests, is missed by all but the request's first workgroup: the harder
+        // order, in which the length stands before a wait gives up.)
+        bool come = a.absent == 0u || chunk == 0;
 #pragma unroll
         for (int r = 0; r < kBandLoads; ++r) {
           const int at = tid + 256 * r;
@@ -1394,6 +1403,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       load_counts();
       TS_MARK(16);
       load_pieces(kBandBelow);
+      if (chunk == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the length's store among others
       TS_MARK(17);
       // The counts of all workgroups: two fields to a register, 16 lanes each, then in LDS; and the
       // highest bin that some workgroup's field has no room for.
@@ -1457,8 +1467,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
           }
           from_band = band_sum[kBandBins + 1] == 0u;
           // (every candidate of the bin is in a slot: the count is that of the histogram)
-          if (from_band && scratch[15] != in_bin0 && tid == 0)
-            __hip_atomic_store(&lp.sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (from_band && scratch[15] != in_bin0 && tid == 0) raise_fault(lp.sync);
         }
       }
     }
@@ -1860,13 +1869,19 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     TS_MARK(14);
     // A grid-wide wait of this launch gave up (the workgroups were not all resident
     // within the bound): what was selected is not valid.  The first workgroup of every
-    // selecting request says so in place of the length, and in the caller's word.
+    // selecting request says so in place of the length, and in the caller's word.  A wait before a
+    // rendezvous, or before this workgroup's words of the band were sent, raised the fault word
+    // ahead of those; one for the band itself answers for itself (kSelVerdict).
     if (chunk == 0 && tid == 0) {
-      const bool gave_up = load_coherent(&lp.sync[0]) != 0u;
-      a.sel_len[b] = gave_up ? -1 : a.n_init + (int)k + a.n_local;
-      if (a.hint && !gave_up) a.hint[b] = (int)t0 + 1;  // where the next step's band is going to lie
-      if (gave_up && a.fault_out)
-        __hip_atomic_store(a.fault_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      const uint32_t verdict = fetch_or_coherent(&ctr[kSelVerdict], kSelDecided);
+      const bool gave_up = load_coherent(&lp.sync[0]) != 0u || (verdict & kSelLost) != 0u;
+      if (gave_up) {
+        store_coherent((uint32_t*)&a.sel_len[b], 0xffffffffu);
+        if (a.fault_out)
+          __hip_atomic_store(a.fault_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      } else if (a.hint) {
+        a.hint[b] = (int)t0 + 1;  // where the next step's band is going to lie
+      }
     }
   }
 }
