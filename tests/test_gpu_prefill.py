@@ -145,6 +145,24 @@ def test_sparse_prefill_attention_short_selections(dev, m, S):
     assert err <= 2e-2, err
 
 
+@pytest.mark.parametrize("shape", [SHAPES[2], SHAPES[3]], ids=[IDS[2], IDS[3]])
+def test_sparse_prefill_attention_room_for_millions(dev, shape):
+    """A list with room for more entries than the second dimension of a grid may have tiles of 32 (65536):
+    the same bits as with as much room as it needs."""
+    m, S, room = 20, 700, 65536 * 32 + 1
+    say(f"prefill attention, room for {room} entries")
+    wl = workloads.build("pf", shape, [S + 8], [8], 1, dev, seed=23, n_init=1, n_local=m)
+    g = torch.Generator(device=dev).manual_seed(24)
+    q = torch.randn((m, wl.cfg.num_heads * 128), generator=g, device=dev).bfloat16()
+    sel = torch.zeros(room, dtype=torch.int32, device=dev)
+    sel[:S] = wl.table[0, :S]
+    sel_len = torch.tensor([S], dtype=torch.int32, device=dev)
+    out = ops.sparse_prefill_attention(wl.cfg, q, wl.k_pool, wl.v_pool, sel, sel_len)
+    want = ops.sparse_prefill_attention(wl.cfg, q, wl.k_pool, wl.v_pool, sel[:S].contiguous(), sel_len)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[3], SHAPES[4], SHAPES[7]],
                          ids=[IDS[0], IDS[3], IDS[4], IDS[7]])
 @pytest.mark.parametrize("m,S", [(15, 140), (16, 128), (63, 190), (64, 64), (65, 257)])

@@ -222,7 +222,8 @@ __device__ __forceinline__ void stage(const PrefillArgs& a, void* to, const uint
     *(uint4*)to = w;
 }
 
-// Grid (KV heads, 32-key tiles).  Thread (key kk, chunk c) moves dims [8c, 8c+8) and
+// Grid (32-key tiles x KV heads, the head fastest; all on x: the device reports 65536 as the end of y, 2.1 M keys).
+// Thread (key kk, chunk c) moves dims [8c, 8c+8) and
 // [64+8c, +8) of key j = tile + kk.  Keys past S are written as zeros.
 // DENSE (PrefillDense): key j is position j, its slot the table's or, from the length on, one of the
 // chunk's new rows, which is read where the caller has it and stored on the way.  A dense chunk was
@@ -233,8 +234,10 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
   __shared__ __attribute__((aligned(16))) uint16_t vt_lds[kHeadDim * kPfVRow];
   const int tid = threadIdx.x;
   const int kk = tid >> 3, c8 = tid & 7;
-  const int kvh = blockIdx.x;
-  const int j = blockIdx.y * kPfKeys + kk;
+  const int head_bits = __builtin_ctz((unsigned)a.num_kv_heads);  // (1, 2, 4 or 8 of them)
+  const int kvh = blockIdx.x & (a.num_kv_heads - 1);
+  const uint32_t tile = blockIdx.x >> head_bits, tiles = gridDim.x >> head_bits;
+  const int j = tile * kPfKeys + kk;
   // (the slot is asked for together with the length, not after it)
   uint32_t slot;
   if (DENSE) {
@@ -265,8 +268,8 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
   };
   if (DENSE) {
     // Rows past the tiles (a bound below the length is the caller's error, but they are stored).
-    if (appends && len >= 0 && blockIdx.y + 1 == gridDim.y)
-      for (int at = max((int)gridDim.y * kPfKeys, len) + kk; at < end; at += kPfKeys) {
+    if (appends && len >= 0 && tile + 1 == tiles)
+      for (int at = max((int)tiles * kPfKeys, len) + kk; at < end; at += kPfKeys) {
         const uint32_t to = chunk_slot(at - len);
         for (int half = 0; half < 2; ++half)
           store_piece(to, half, chunk_piece(dense.store.k, at - len, half), chunk_piece(dense.store.v, at - len, half));
@@ -284,7 +287,7 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
   }
   // Whole blocks of kPfPadKeys: the keys between S and the next multiple are written as
   // zeros too (their weights are zero, but 0 x garbage is not).
-  if (blockIdx.y * kPfKeys >= (S + kPfPadKeys - 1) / kPfPadKeys * kPfPadKeys && !(DENSE && blockIdx.y * kPfKeys < (unsigned)max(end, 0)))
+  if (tile * kPfKeys >= (S + kPfPadKeys - 1) / kPfPadKeys * kPfPadKeys && !(DENSE && tile * kPfKeys < (unsigned)max(end, 0)))
     return;
   const bool live = j < S;
   uint4 kraw[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
@@ -332,7 +335,7 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
     }
   }
   // key kk = 16 kb + qc, dims 32 ks + 8 g4: operand 4 kb + ks, lane 16 g4 + qc
-  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)blockIdx.y * kPfKeys) * kHeadDim;
+  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)tile * kPfKeys) * kHeadDim;
   uint16_t* kout = a.kr + tile_at + ((4 * (kk >> 4) + (c8 >> 2)) * 64 + 16 * (c8 & 3) + (kk & 15)) * 8;
   stage(a, kout, make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
                             pack_bf16(lo[6], lo[7])));
@@ -866,7 +869,7 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
   a.new_len = dense && dense->store.k ? dense->seq_len : nullptr;
   a.len_cap = dense ? dense->store.max_tokens : 0;
   hipStream_t st = stream;
-  const dim3 gather_grid((unsigned)cfg->num_kv_heads, (unsigned)(a.s_pad / kPfKeys));
+  const dim3 gather_grid((unsigned)cfg->num_kv_heads * (unsigned)(a.s_pad / kPfKeys));
   if (dense)
     hipLaunchKernelGGL(prefill_gather_dense_kernel, gather_grid, dim3(256), 0, st, a, *dense);
   else
