@@ -251,6 +251,46 @@ def test_a_step_stores_as_the_store_does(dev, case):
         assert sides[0]["lens"].tolist() == [n + steps for n in lengths]
 
 
+@pytest.mark.parametrize("page", [1, 16], ids=["tokens", "pages"])
+@pytest.mark.parametrize("longest,cached", [(700, False), (3000, False), (3000, True)],
+                         ids=["dense", "selected", "selection cache"])
+def test_a_request_without_a_length_is_left_alone(dev, longest, cached, page):
+    """A negative length is refused as a full table is, by whatever launch places the new token: the
+    store alone, the first launch of a first call and that of the calls after it.  (Request 1's: an
+    entry of its table written all the same would be one of request 0's last.)"""
+    say(f"request without a length: longest={longest} cached={cached} pages of {page}")
+    cfg = ops.LayerConfig(num_heads=8, num_kv_heads=2, n_init=128, n_local=512, top_k=1024, rope_theta=5e5,
+                          page_size=page)
+    g = torch.Generator(device=dev).manual_seed(15)
+    pages = longest // page + 8
+    order = torch.randperm(pages, generator=g, device=dev).to(torch.int32)
+    held = -(-longest // page)
+    table = torch.full((2, pages), -1, dtype=torch.int32, device=dev)
+    table[0, :held] = order[:held]
+    k_pool, v_pool = (torch.randn((pages * page, 2, 128), generator=g, device=dev).bfloat16() for _ in range(2))
+    lens = torch.tensor([longest, -5 * page], dtype=torch.int32, device=dev)
+    pool = None if page == 1 else ops.PagePool(order[held:].contiguous(),
+                                               torch.tensor([pages - held], dtype=torch.int32, device=dev),
+                                               torch.zeros(1, dtype=torch.int32, device=dev))
+    cache = ops.SelectionCache.allocate(cfg, 2, dev) if cached else None
+    layer = ops.DecodeLayer(cfg, 2, longest + 8, dev)
+    now = longest
+    for t in range(4):
+        q, k, v = (torch.randn((2, n * 128), generator=g, device=dev).bfloat16() for n in (8, 2, 2))
+        loc = None if pool else torch.stack([order[held + t], order[held + 4]])
+        want_k = k_pool.clone()
+        if t == 0:
+            ops.kv_store(cfg, k, v, loc, k_pool, v_pool, table, lens, pages=pool)
+        else:
+            layer.step(q, k, v, loc, k_pool, v_pool, ops.Batch(lens, table, now + 1), cache, pages=pool)
+        torch.cuda.synchronize()
+        want_k[int(table[0, now // page]) * page + now % page] = k[0].view(2, 128)
+        now += 1
+        assert not layer.gave_up()
+        assert lens.tolist() == [now, -5 * page] and torch.equal(k_pool, want_k), t
+        assert bool((table[1] == -1).all()) and bool((table[0, -(-now // page):] == -1).all()), t
+
+
 @pytest.mark.parametrize("length,rows,room,page", [(0, 40, 64, 1), (600, 512, 1200, 1), (1000, 100, 1050, 1), (31, 33, 64, 16),
                                                    (640, 512, 1200, 16), (1000, 100, 1040, 16), (2400, 288, 2688, 1)])
 def test_a_dense_chunk_stores_as_the_store_does(dev, length, rows, room, page):

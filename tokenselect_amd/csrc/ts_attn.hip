@@ -81,9 +81,8 @@ __device__ __forceinline__ void attn_commit(const StepCommit& c) {
   if (b == 0 && c.free_count) *c.free_count = max(*c.free_count, 0) - note.w;
 }
 
-// Whether a request's new token is stored: what the store kernels ask (ts_store.hip).
 __device__ __forceinline__ bool attn_appends(const AttnArgs& a, int slot, int len) {
-  return a.step.loc != nullptr && (uint32_t)slot < a.pool_rows && len >= 0 && len < a.step.max_tokens;
+  return a.step.loc != nullptr && append_fits(slot, len, a.pool_rows, a.step.max_tokens);
 }
 
 // What a dense step leaves behind besides the output, after a workgroup's share of the attention:

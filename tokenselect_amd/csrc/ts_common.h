@@ -141,6 +141,11 @@ struct StepStore {
   uint32_t* ticket;
   int page_shift;
 };
+// Whether a request's new token is stored: a slot of the pool, and a table with room at that length.
+// (Asked by everyone who places one: what a call does must not depend on which launch that is.)
+__device__ __forceinline__ bool append_fits(int slot, int len, int64_t pool_rows, int max_tokens) {
+  return slot >= 0 && slot < pool_rows && len >= 0 && len < max_tokens;
+}
 // What a step's store leaves to be written when nobody reads the lengths any more: one per request,
 // noted by the selection that stored the rows and knows the length (ts_score.hip), written by
 // the attention after it.

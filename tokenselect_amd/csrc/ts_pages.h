@@ -120,8 +120,8 @@ __device__ __forceinline__ void commit_appends(int32_t* seq_lens, int32_t* table
 
 // The rows of request b stored and appended, by one workgroup of a launch in which `batch` of them
 // do this: at the slot that the caller chose, or (with a page pool) where the plan of the batch
-// says, which the last of them commits.  A full table (tr.py:334 asserts) or a slot outside the pool
-// leaves the request untouched.  Bound by its memory round trips; the new rows are asked for
+// says, which the last of them commits.  A full table (tr.py:334 asserts), a slot outside the pool or
+// a length that is none leaves the request untouched.  Bound by its memory round trips; the new rows are asked for
 // together with the slot and the length, not after them.
 __device__ __forceinline__ void store_step(const StepStore& st, int b, int batch) {
   const int first = threadIdx.x, threads = blockDim.x;
@@ -145,9 +145,9 @@ __device__ __forceinline__ void store_step(const StepStore& st, int b, int batch
     __syncthreads();
     slot = plan_slot;
   } else {
-    slot = st.loc[b];
+    const int asked = st.loc[b];
     len = st.seq_lens[b];
-    if (slot >= st.pool_rows || len >= st.max_tokens) slot = -1;
+    if (append_fits(asked, len, st.pool_rows, st.max_tokens)) slot = asked;
   }
   if (slot >= 0) {
     if (first < st.row_vec) {

@@ -287,7 +287,7 @@ __device__ __forceinline__ void plan_append_one(const ScoreArgs& a, int len, Dea
   const StepStore& st = late_args().append;
   if (st.free_pages == nullptr) {
     const int slot = st.loc[0];
-    const bool ok = slot >= 0 && slot < st.pool_rows && len >= 0 && len < st.max_tokens;
+    const bool ok = append_fits(slot, len, st.pool_rows, st.max_tokens);
     d.own_len = ok ? len + 1 : len;
     d.own_slot = ok ? (uint32_t)slot : kNoSlot;
     return;
@@ -305,7 +305,7 @@ __device__ __forceinline__ int plan_appends(const ScoreArgs& a, int lane, Append
   if (st.free_pages == nullptr) {
     if (lane < a.batch) {
       const int len = st.seq_lens[lane], slot = st.loc[lane];
-      const bool ok = slot >= 0 && slot < st.pool_rows && len >= 0 && len < st.max_tokens;
+      const bool ok = append_fits(slot, len, st.pool_rows, st.max_tokens);
       plans[lane] = append_at(ok, len, (uint32_t)slot);
     }
     return 0;

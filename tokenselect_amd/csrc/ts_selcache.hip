@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
       if (store_slot >= 0) len_now += 1;
     } else {
       const int slot = st.loc[b];
-      if (slot >= 0 && slot < st.pool_rows && len_now < st.max_tokens) {
+      if (append_fits(slot, len_now, st.pool_rows, st.max_tokens)) {
         store_slot = slot;
         if (threadIdx.x == 0) {
           st.table[(int64_t)b * st.table_stride + len_now] = slot;

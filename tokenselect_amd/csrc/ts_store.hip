@@ -42,7 +42,7 @@ __global__ __launch_bounds__(kListThreads) void kv_store_list_kernel(StepStore s
     const int pos = first + i * kListThreads;
     ahead[i] = pos < known ? tab[pos] : 0;
   }
-  const bool ok = slot >= 0 && slot < pool_rows && len < max_tokens;
+  const bool ok = append_fits(slot, len, pool_rows, max_tokens);
   if (ok) {
     if (first < row_vec) {
       k_pool[(size_t)slot * row_vec + first] = k0;
