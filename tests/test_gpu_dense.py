@@ -251,6 +251,27 @@ def test_a_step_stores_as_the_store_does(dev, case):
         assert sides[0]["lens"].tolist() == [n + steps for n in lengths]
 
 
+@pytest.mark.parametrize("bound", [300, 511, 512, 700])
+def test_a_dense_step_beyond_the_bound_is_stored(dev, bound):
+    """max_seq_len below the length: attended to are the positions below it, as before, but the new
+    token's row is stored and listed in the table by a first call and by those after it."""
+    say(f"dense step beyond a bound of {bound}")
+    cfg = ops.LayerConfig(num_heads=14, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5)
+    length = 700
+    g, (k_pool, v_pool), table, lens, free = _state(cfg, [length, 40], 8, dev, 16)
+    layer = ops.DecodeLayer(cfg, 2, 800, dev)
+    for t in range(3):
+        q, k, v = (torch.randn((2, n * 128), generator=g, device=dev).bfloat16() for n in (14, 2, 2))
+        want_k, want_v, loc = k_pool.clone(), v_pool.clone(), free[2 * t:2 * t + 2].clone()
+        want_k[loc.long()], want_v[loc.long()] = k.view(2, 2, 128), v.view(2, 2, 128)
+        _, sel, _, sel_len = layer.step(q, k, v, loc, k_pool, v_pool, ops.Batch(lens, table, bound))
+        torch.cuda.synchronize()
+        assert lens.tolist() == [length + t + 1, 41 + t] and table[0, length + t] == loc[0]
+        assert torch.equal(k_pool, want_k) and torch.equal(v_pool, want_v), t
+        assert sel_len.tolist() == [min(bound, length + t + 1), 41 + t]
+        assert torch.equal(sel[0, :sel_len[0]], table[0, :sel_len[0]])
+
+
 @pytest.mark.parametrize("page", [1, 16], ids=["tokens", "pages"])
 @pytest.mark.parametrize("longest,cached", [(700, False), (3000, False), (3000, True)],
                          ids=["dense", "selected", "selection cache"])

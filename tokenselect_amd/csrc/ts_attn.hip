@@ -93,7 +93,8 @@ __device__ __forceinline__ bool attn_appends(const AttnArgs& a, int slot, int le
 __device__ __forceinline__ void attn_dense_epilogue(const AttnArgs& a, int b, int kvh, int lo, int hi, int S,
                                                     int slot, int len, bool ok, bool last) {
   const int tid = threadIdx.x;
-  if (ok && lo <= len && len < hi && tid < 2 * (kHeadDim / 8)) {
+  // (a host bound below the length is the caller's error, but the row is stored: the table lists it)
+  if (ok && lo <= len && (len < hi || (int)blockIdx.x + 1 == a.nsplit) && tid < 2 * (kHeadDim / 8)) {
     const bool is_v = tid >= kHeadDim / 8;
     const int at = 8 * (tid % (kHeadDim / 8));
     const uint16_t* row = (is_v ? a.step.v : a.step.k) + (size_t)b * a.step.kv_stride + kvh * kHeadDim + at;
