@@ -402,10 +402,13 @@ int ts_kv_store(const ts_config* cfg, const void* k, const void* v, const int32_
  * K/V stored and appended as ts_kv_store does it (kv: its k, v, out_cache_loc, pages
  * and max_tokens; the table and the lengths are bt's, which the call therefore
  * writes), then ts_decode_layer on the lengths after the append (bt->max_seq_len and
- * host_seq_lens bound those).  Results are those of the two calls.  With a selection
- * cache the store rides in the layer's first launch, the rotation and cache decision
- * (slots chosen by the caller or taken from a page pool alike), and a step is three
- * kernels instead of four; otherwise the two calls follow each other.  With
+ * host_seq_lens bound those).  Results are those of the two calls, as long as no slot
+ * that the step stores to is one of another request's context or of a context's
+ * candidates: the store rides in the layer's first launch (the rotation, with or without
+ * the cache decision, the selection, or the attention of a step known to be dense),
+ * whose other workgroups may read such a row before or after it is written.  (Padded
+ * requests may share a slot and list it: a short request's own entries of it are the new
+ * row.)  With
  * bt->rerun the step's token has been appended by the call that gave up, and only
  * the layer runs. */
 typedef struct ts_new_kv {
@@ -513,9 +516,12 @@ int ts_prefill_chunk(const ts_config* cfg, const ts_batch* bt, const void* q, in
  * chunk's K/V (kv: k, v [rows, Hkv, D], out_cache_loc [rows], pages, max_tokens; the
  * table row and the length word are bt's, which the call therefore writes), then
  * ts_prefill_chunk on the length after the append (which bt->max_seq_len bounds).
- * Results are those of the two calls.  With slots chosen by the caller (pages == NULL,
- * page_size 1) the store rides in the chunk's first launch, the fingerprint, as spare
- * workgroups; otherwise the two calls follow each other.  With bt->rerun the chunk has been
+ * Results are those of the two calls, where the chunk's slots are all different and none of
+ * them is listed in the context before it.  With slots chosen by the caller (pages == NULL,
+ * page_size 1) the store rides in the chunk's first launch: spare workgroups of the
+ * fingerprint, or, where the chunk is known to be dense, the gather of the keys, which takes
+ * the chunk's own from k and v while their rows are written.  Otherwise the two calls follow
+ * each other.  With bt->rerun the chunk has been
  * appended by the call that gave up, and only ts_prefill_chunk runs. */
 int ts_prefill_step(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
                     int32_t rows, const float* cos_table, const float* sin_table, int64_t table_rows,

@@ -251,6 +251,37 @@ def test_a_step_stores_as_the_store_does(dev, case):
         assert sides[0]["lens"].tolist() == [n + steps for n in lengths]
 
 
+@pytest.mark.parametrize("padded", [[1], [0], [5, 1], [300, 40]])
+def test_padded_requests_on_one_slot(dev, padded):
+    """Requests that pad a batch list one slot over and over and store to it.  One of them: the step's
+    output is that of the store and the layer, whose context holds the new row wherever the slot is
+    listed.  Several: each attends to its own new row.  The request beside them as if alone."""
+    say(f"padded requests of {padded} tokens")
+    cfg = ops.LayerConfig(num_heads=14, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5)
+    B, steps = 1 + len(padded), 3
+    g, (k_pool, v_pool), table, lens, free = _state(cfg, [900], 8, dev, 17)
+    slot = int(free[-1])
+    table = torch.cat([table, torch.full((len(padded), MAX_TOKENS), slot, dtype=torch.int32, device=dev)])
+    layer = ops.DecodeLayer(cfg, B, 1000, dev)
+    now = torch.tensor([900] + padded, dtype=torch.int32, device=dev)
+    for t in range(steps):
+        q, k, v = (torch.randn((B, n * 128), generator=g, device=dev).bfloat16() for n in (14, 2, 2))
+        loc = torch.cat([free[t:t + 1], torch.full((len(padded),), slot, dtype=torch.int32, device=dev)])
+        want = []
+        for b in range(B):   # each by itself
+            pools, one, row = (k_pool.clone(), v_pool.clone()), now[b:b + 1].clone(), table[b:b + 1].clone()
+            ops.kv_store(cfg, k[b:b + 1], v[b:b + 1], loc[b:b + 1], *pools, row, one)
+            alone = ops.DecodeLayer(cfg, 1, 1000, dev)
+            want.append(alone(q[b:b + 1], *pools, ops.Batch(one, row, 900 + t + 1))[0].clone())
+        lens = now.clone()
+        out = layer.step(q, k, v, loc, k_pool, v_pool, ops.Batch(lens, table, 900 + t + 1))[0]
+        torch.cuda.synchronize()
+        if t > 0 or len(padded) == 1:   # (a first call stores in a launch of its own: one row for all)
+            ref = torch.cat(want).float()
+            assert bool(((out.float() - ref).abs() <= ref.abs() * 2.0 ** -7 + 1e-6).all()), t   # (other splits: an ulp)
+        now[0] += 1
+
+
 @pytest.mark.parametrize("bound", [300, 511, 512, 700])
 def test_a_dense_step_beyond_the_bound_is_stored(dev, bound):
     """max_seq_len below the length: attended to are the positions below it, as before, but the new

@@ -394,7 +394,8 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   if (DENSE && wlo == new_pos) first_slot = kNewRow;
   auto checked = [&](uint32_t slot, int j) {
     if (!DENSE) return j < whi && slot < a.pool_rows ? slot : first_slot;
-    if (j == new_pos) return kNewRow;
+    // (a slot that the table lists already, as a padded request's is: the row that is about to be there)
+    if (j == new_pos || (appends && j < whi && slot == (uint32_t)new_slot)) return kNewRow;
     return j < whi ? min(slot, a.pool_rows - 1) : first_slot;  // (an entry that is no slot: as it is listed)
   };
   slot_cur[0] = checked(slot_cur[0], wlo + n);
