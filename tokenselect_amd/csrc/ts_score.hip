@@ -1886,6 +1886,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
   }
 }
 
+static_assert(std::is_same<decltype(&score_kernel<8, 4, false, kScoreFused>), void (*)(ScoreArgs)>::value,
+              "late_args() reads ScoreArgs from the start of the arguments");
+
 template <bool OUT_BF16, int MODE>
 static int launch_score(int hkv, int group, const ScoreArgs& a, dim3 grid, hipStream_t stream) {
   const size_t lds =
