@@ -118,9 +118,9 @@ def test_growing_context_on_one_workspace(dev, first, steps, B, pool):
 def test_steps_on_one_workspace(dev, first, steps, page):
     """Steps that store their own tokens, over the ends of the sinks, of sinks and window (where a
     selection's counters begin) and of dense, one object for all against a fresh one at each, whose
-    first call clears everything and stores in a launch of its own: the same bit for bit, the
-    attention apart (other splits: one ulp of the output's rounding).  Request 1 is shorter, and its
-    table is full for the last steps."""
+    first call clears everything and stores in a launch of its own: the same bit for bit, outputs
+    included (the same splits, the same roundings).  Request 1 is shorter, and its table is full for
+    the last steps."""
     say(f"steps from {first}, pages of {page}")
     cfg = ops.LayerConfig(num_heads=14, num_kv_heads=2, n_init=128, n_local=512, top_k=2048, rope_theta=5e5,
                           page_size=page)
@@ -160,6 +160,7 @@ def test_steps_on_one_workspace(dev, first, steps, page):
         torch.cuda.synchronize()
         assert not one.gave_up()
         _same(*got)
+        assert torch.equal(got[0]["out"], got[1]["out"]), t
         assert torch.equal(sides[0]["pages"].free_count, sides[1]["pages"].free_count)
     assert sides[0]["lens"].tolist() == [last, min(lengths[1] + steps, room)]
 

@@ -1528,10 +1528,10 @@ def test_selection_form_agrees_with_what_the_launchers_serve(dev):
                          ids=lambda s: f"H{s['num_heads']}kv{s['num_kv_heads']}")
 def test_fused_select_with_a_threshold_hint(dev, shape):
     """ts_batch.threshold_hint: the selection notes the bin of the k-th vote and, given it
-    back, publishes what its last round needs before the first rendezvous, so that one
-    rendezvous is enough.  The result is that of a launch without a hint, bit for bit: with
-    the right hint (one round met for), with hints off by a few bins inside the band, with
-    hints outside it and with nonsense (two rounds again), and for another query whose
+    back, its workgroups hand each other what they need as words that are their own flags: no
+    rendezvous.  The result is that of a launch without a hint, bit for bit: with the right
+    hint and with hints off by a few bins inside the band (no round met for), with hints
+    outside it and with nonsense (two rounds, as without one), and for another query whose
     threshold has moved."""
     import dataclasses
     L, k = 40000, 512
@@ -1542,7 +1542,7 @@ def test_fused_select_with_a_threshold_hint(dev, shape):
     space = ops.select_workspace(c, wl.batch, dev)
     want = ops.select(c, wl.batch, qf, wl.k_pool, workspace=space)[:3]
     torch.cuda.synchronize()
-    assert ops.select_rounds(c, wl.batch, space)[:2][1] > 0, "without a hint: a second round"
+    assert all(r > 0 for r in ops.select_rounds(c, wl.batch, space)[:2]), "without a hint: two rounds"
     hint = torch.zeros(1, dtype=torch.int32, device=dev)
     hinted = dataclasses.replace(wl.batch, hint=hint)
 
@@ -1554,20 +1554,24 @@ def test_fused_select_with_a_threshold_hint(dev, shape):
             assert torch.equal(x, y), name
         return ops.select_rounds(c, hinted, space)
 
-    assert run()[1] > 0                 # no hint yet: the usual two rounds, and the hint is left
+    def met():
+        return [r > 0 for r in run()]
+
+    both, none = [True, True, False, False], [False] * 4
+    assert met() == both                # no hint yet: the usual two rounds, and the hint is left
     code = int(hint[0])
     assert 1 <= code <= 2048
-    assert run()[1] == 0                # the right hint: one round
+    assert met() == none                # the right hint: nobody is met
     for off in (-3, -1, 1, 4):          # the band [hint - 4, hint + 3] still holds the bin
         hint.fill_(code + off)
-        assert run()[1] == 0, off
+        assert met() == none, off
         assert int(hint[0]) == code
-    for off in (-4, 5, 300, -code):     # it does not, or there is no hint at all: the list round is back
+    for off in (-4, 5, 300, -code):     # it does not, or there is no hint at all: both rounds are back
         hint.fill_(code + off)
-        assert run()[1] > 0, off
+        assert met() == both, off
         assert int(hint[0]) == code
     hint.fill_(5000)                    # nonsense
-    assert run()[1] > 0
+    assert met() == both
     # another query: its own selection, whatever the old hint says
     g = torch.Generator(device=dev).manual_seed(102)
     q2 = (qf.float() + 0.3 * torch.randn(qf.shape, generator=g, device=dev)).bfloat16()
