@@ -37,7 +37,7 @@ CXXFLAGS = [
 # The selection's additions to one word of LDS come from one lane of a wavefront each, or are combined
 # by the code itself: left alone they are one instruction, while the compiler otherwise turns each
 # into a loop over the active lanes (0.15 us apiece where a workgroup runs it once; one request of
-# 32K tokens 36.9 -> 36.5 us a layer).
+# 32K tokens 36.8 -> 35.9 us a layer).
 SOURCE_FLAGS = {"ts_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 "ts_score.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]}
 

@@ -135,7 +135,7 @@ struct StepStore {
   int kv_stride;   // 16-byte pieces between rows of k, and of v
   int max_tokens;
   // With a page pool (free_pages != NULL; loc is not read): the slots come from the table and
-  // the pool as kv_store_paged_kernel takes them.
+  // the pool by the plan of the batch (ts_pages.h).
   const int32_t* free_pages;
   int32_t* free_count;
   uint32_t* ticket;

@@ -213,7 +213,9 @@ __device__ __forceinline__ int kv_pos(int kk) { return 8 * ((kk >> 2) & 3) + 4 *
 // what it leaves in that XCD's L2 is read from there.  With fewer, several XCDs read a head, most of
 // what is written waits in the wrong L2, and the writes go past it.  Gather + attention, us: 28 heads
 // on 4 7.75 + 24.8 with the tile as the fastest index, 6.6 + 24.6 with the head, 5.6 + 24.8 past the
-// L2 as well; 32 on 8 7.4 + 27.4, 6.5 + 27.6, 6.7 + 28.3.
+// L2 as well; 32 on 8 7.4 + 27.4, 6.5 + 27.6, 6.7 + 28.3.  A prompt of 31600 tokens, 28 heads on 4:
+// 3675 us kept, 3651 past the L2.  On two heads and on one (whose keys are a quarter and an eighth) it is the
+// same either way: 28.6 and 27.0 us for both launches, prompts of 12000 tokens 1250 and 1198.
 typedef __attribute__((ext_vector_type(4))) unsigned int pf_u32x4;
 __device__ __forceinline__ void stage(const PrefillArgs& a, void* to, const uint4& w) {
   if (a.num_kv_heads < 8)

@@ -75,7 +75,7 @@ constexpr int kQuadSwap2 = 0x4E;  // quad_perm [2,3,0,1]
 //     the keys stream in costs a quarter of the read bandwidth (DRAM read/write
 //     turnarounds).
 //   kScoreFused (the whole selection in one launch whose workgroups are all
-//     resident at once and meet two to four times): the scores never leave LDS.
+//     resident at once and wait for each other): the scores never leave LDS.
 //     Every workgroup publishes its per-head (max, sum exp); the (request, head)
 //     pairs are dealt out over the grid, merged and written to replicas that the
 //     workgroups poll; every workgroup turns its own
@@ -84,6 +84,8 @@ constexpr int kQuadSwap2 = 0x4E;  // quad_perm [2,3,0,1]
 //     listed and ranked by every workgroup together with the counts that tell it
 //     where its selected positions, in ascending order, belong (tr.py:371-373,
 //     433-449); masses of exact ties go through all three levels and a count round.
+//     That is two to four rendezvous, and one more for the max-pool's neighbours; none
+//     where a hint says near which bin the threshold lies and it does.
 constexpr int kScoreDirect = 0, kScoreTiled = 1, kScoreFused = 2;
 // The fused kernel's votes-only form (phases of requests in one launch): a kernel of its
 // own, so that the single-launch selection does not carry the bookkeeping.
@@ -1573,9 +1575,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     uint2* counts = a.block_counts + (size_t)b * kSelMaxChunks;
     const bool listed = in_bin <= (uint32_t)kSelListCap;
     uint32_t kth, need_eq = 0, pos_thr = 0, lower_taken = 0;
-    // With a hint whose band holds the threshold bin, everything the ranking needs was
-    // published before the first rendezvous: no list round.  The test was the same for every
-    // workgroup of the request (the band's histogram, the flags), so all take the same way.
+    // With a hint whose band holds the threshold bin and its candidates, everything the ranking
+    // needs has come in the words of the band: no list round.  The test was the same for every
+    // workgroup of the request (the same words, whole unless a wait gave up), so all take the same way.
     if (!from_band) {
       __syncthreads();
       if (tid < 8) scratch[8 + tid] = 0u;

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void rope_selcache_kernel(const uint16_t* __re
   constexpr int kMaxUnits = kSelCacheMaxVec / 2;
   const int units = a.dim >> 4;  // (heads x 8)
   // With a token to store (st.k): this workgroup stores request b's rows and appends the slot
-  // exactly as kv_store_kernel does, and decides with the length after the append, which it
+  // exactly as store_step does, and decides with the length after the append, which it
   // knows without reading it back.
   // (One thread reads the length and hands it round: the append below rewrites the word.)
   __shared__ int len_before;
