@@ -129,7 +129,7 @@ constexpr int kSelListCount = kSelMaxBin + kSelHistCopies * 32;
 // the request's previous selection on the same layer), every workgroup sends, in place of its
 // histogram, what the last round would otherwise need a rendezvous of its own for, for the
 // kBandBins bins around the hint: how many of its tokens lie in each of them and above them all
-// (two words of 64 bits), and those candidates (up to kBandSlots a bin, packed into 32 bits each:
+// (one word of 64 bits), and those candidates (up to kBandSlots a bin, packed into 32 bits each:
 // the low 21 key bits and the token's index in the workgroup, which is why the band needs
 // workgroups of at most 1024 tokens; two to a word).  No word that is sent is zero and all are zero
 // before a launch, so each is its own flag: a thread per workgroup asks for them until they have

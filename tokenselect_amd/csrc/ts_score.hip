@@ -1049,7 +1049,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     __shared__ float s_rz[kMaxHeads];
     __shared__ uint32_t scratch[16];
     const int tid = threadIdx.x;
-    static_assert(kBandSlots == 4, "a workgroup's candidates of a bin are one 16-byte piece");
+    static_assert(kBandSlots == 4, "a workgroup's candidates of a bin are two words");
     __shared__ uint32_t band_lds[kBandBins][kBandSlots];
     __shared__ uint32_t band_count[kBandBins + 1];  // per bin; [kBandBins]: tokens above the band
     // Over all workgroups: [0..3] the counts of two bins each, [4] the tokens above the band, [8] how many
