@@ -387,6 +387,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   const int new_slot = DENSE ? (a.step.loc ? a.step.loc : a.sel_len)[b] : -1;
   const bool appends = DENSE && attn_appends(a, new_slot, length);
   const int new_pos = appends ? length : -1;
+  const uint32_t own_slot = appends ? (uint32_t)new_slot : kNewRow;
   const int S = min(max(length + (appends ? 1 : 0), 0), DENSE ? a.list_bound : a.max_sel_len);
   const int whi = min(S, wlo + wlen);
   uint32_t first_slot =
@@ -394,9 +395,10 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   if (DENSE && wlo == new_pos) first_slot = kNewRow;
   auto checked = [&](uint32_t slot, int j) {
     if (!DENSE) return j < whi && slot < a.pool_rows ? slot : first_slot;
-    // (a slot that the table lists already, as a padded request's is: the row that is about to be there)
-    if (j == new_pos || (appends && j < whi && slot == (uint32_t)new_slot)) return kNewRow;
-    return j < whi ? min(slot, a.pool_rows - 1) : first_slot;  // (an entry that is no slot: as it is listed)
+    // (an entry that is no slot: as it is listed; one that the table lists already, as a padded
+    // request's does: the row that is about to be there)
+    const uint32_t entry = j < whi ? min(slot, a.pool_rows - 1) : first_slot;
+    return (j == new_pos) | (entry == own_slot) ? kNewRow : entry;
   };
   slot_cur[0] = checked(slot_cur[0], wlo + n);
   slot_cur[1] = checked(slot_cur[1], wlo + 16 + n);

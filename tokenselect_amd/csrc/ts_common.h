@@ -143,8 +143,9 @@ struct StepStore {
 };
 // Whether a request's new token is stored: a slot of the pool, and a table with room at that length.
 // (Asked by everyone who places one: what a call does must not depend on which launch that is.)
+// (Both bounds are below 2^31: a negative one of the two is beyond them.)
 __device__ __forceinline__ bool append_fits(int slot, int len, int64_t pool_rows, int max_tokens) {
-  return slot >= 0 && slot < pool_rows && len >= 0 && len < max_tokens;
+  return (uint32_t)slot < (uint32_t)pool_rows && (uint32_t)len < (uint32_t)max_tokens;
 }
 // What a step's store leaves to be written when nobody reads the lengths any more: one per request,
 // noted by the selection that stored the rows and knows the length (ts_score.hip), written by
