@@ -47,13 +47,13 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 # Each figure carries the commit of the kernels it was measured on: a later change to the
 # kernel makes it stale until the two counter runs are repeated.
 MEASURED_TRAFFIC = {  # workload -> (bytes per launch of its dominant kernel, commit); profiles/decode_layer_hbm_traffic.txt
-    "C2": (269557041, "6de2775"),        # ts_select, score_kernel<8,4,false,2>
-    "C3": (2230060989, "6de2775"),       # the votes-only launch, score_kernel<8,4,false,3>
-    "C5-layer": (2154460696, "6de2775"),  # likewise
-    "MODEL": (2158911492, "6de2775"),     # likewise, inside the 32-layer decoder (page 1)
+    "C2": (269404338, "1f23e95"),        # ts_select, score_kernel<8,4,false,2>
+    "C3": (2229759047, "1f23e95"),       # the votes-only launch, score_kernel<8,4,false,3>
+    "C5-layer": (2154451912, "1f23e95"),  # likewise
+    "MODEL": (2158924619, "1f23e95"),     # likewise, inside the 32-layer decoder (page 1)
 }
 # attn_kernel<4>, same runs
-MEASURED_ATTN_TRAFFIC = {"C2": 12265601, "C3": 180816643, "C5-layer": 82170062}
+MEASURED_ATTN_TRAFFIC = {"C2": 12288543, "C3": 180834151, "C5-layer": 82201640}
 
 
 def event_time_us(fn, launches: int, warmup: int, before=None, burst: int = 1):
