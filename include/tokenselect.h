@@ -536,6 +536,21 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
                             int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, void* workspace,
                             size_t workspace_bytes, ts_stream_t stream);
 
+/* The chunks of a prompt part together: what ts_prefill_step_strided does for chunk after chunk of
+ * chunk_rows rows (the last one of what is left), in rounds of up to 16 chunks: all rows of a round
+ * are stored first, then its chunks select, each from the context up to its own last row, and attend.
+ * Results are those of the chunks one by one (their votes are added up in another order), where the
+ * slots of the whole part are all different and none of them is listed in the context before it.
+ * With slots chosen by the caller and a per-token table only (pages == NULL, page_size 1);
+ * bt->max_seq_len bounds the length after the last row; no k_per_req.  No workgroup waits for another.
+ * bt->threshold_hint, where given, is not read; it receives what the last chunk's selection
+ * leaves there.  q, out: [rows, H*D]; kv: k, v [rows, Hkv, D], out_cache_loc [rows]. */
+size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len);
+int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
+                      int32_t q_row_stride, int32_t kv_row_stride, int32_t rows, int32_t chunk_rows,
+                      const float* cos_table, const float* sin_table, int64_t table_rows, void* k_pool, void* v_pool,
+                      int64_t pool_rows, void* out, void* workspace, size_t workspace_bytes, ts_stream_t stream);
+
 /* One layer of patched_radix_attention_decode_forward_flashinfer after the KV
  * store (tr.py:791-825): fingerprint (q rotated with q_cos/q_sin, the [D] table
  * rows of position n_local, tr.py:380-388) -> [selection cache] -> score ->

@@ -3,6 +3,8 @@ chunk fingerprint within one bf16 ulp (fp32 summation order), selection identica
 for the same fingerprint up to ties at the k-th vote, causal sparse attention
 within 2e-2 absolute in bf16."""
 
+import dataclasses
+
 import pytest
 import torch
 
@@ -412,6 +414,53 @@ def test_prefill_step_is_store_then_chunk(dev, shape, chunk):
         S = int(x[3][0])
         assert torch.equal(x[1][0, :S], y[1][0, :S]) and torch.equal(x[2][0, :S], y[2][0, :S]), f"chunk {t}"
         assert torch.equal(x[0].view(torch.int16), y[0].view(torch.int16)), f"chunk {t}: output"
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"H{s['num_heads']}kv{s['num_kv_heads']}")
+@pytest.mark.parametrize("case", [dict(L0=3000, T=175, chunk=64), dict(L0=2600, T=1400, chunk=512),
+                                  dict(L0=0, T=37 * 16 - 3, chunk=16), dict(L0=90, T=400, chunk=64, pool=5),
+                                  dict(L0=5, T=333, chunk=1, pool=4, head_map="div"),
+                                  dict(L0=70000, T=130, chunk=65)],
+                         ids=lambda c: "-".join(f"{k}{v}" for k, v in c.items()))
+def test_chunks_of_a_prompt_together(dev, shape, case):
+    """ts_prefill_prompt against the chunks one by one: pools, table and length the same, and with the
+    same selections the outputs bit for bit.  Contexts on both sides of what is attended to densely, more chunks
+    than a round takes, ragged last chunks, a block of more than one step of tokens, pooled votes."""
+    case = dict(case)
+    L0, T, chunk, top_k = case.pop("L0"), case.pop("T"), case.pop("chunk"), 96
+    say(f"prompt H={shape['num_heads']} L0={L0} T={T} chunk={chunk} {case}")
+    wl = workloads.build("pr", shape, [max(L0, 1)], [top_k], 1, dev, seed=21, n_init=8, n_local=64, top_k=top_k,
+                         extra_pages=T)
+    c = dataclasses.replace(wl.cfg, pool_kernel=case.get("pool", -1), head_map=case.get("head_map", "mod"))
+    g = torch.Generator(device=dev).manual_seed(22)
+    common = torch.randn((1, c.num_heads * 128), generator=g, device=dev)
+    q = (common + torch.randn((T, c.num_heads * 128), generator=g, device=dev)).bfloat16()
+    k_new = torch.randn((T, c.num_kv_heads, 128), generator=g, device=dev).bfloat16()
+    v_new = torch.randn((T, c.num_kv_heads, 128), generator=g, device=dev).bfloat16()
+    new_slots = wl.free_pages[:T].contiguous()
+    results = []
+    for together in (True, False):
+        k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
+        table = torch.zeros((1, L0 + T + 3), dtype=torch.int32, device=dev)
+        table[0, :L0] = wl.table[0, :L0]
+        seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
+        hint = torch.zeros(1, dtype=torch.int32, device=dev)
+        out = torch.empty_like(q)
+        layer = ops.PrefillChunk(c, L0 + T + 3, dev, max_rows=chunk)
+        if together:
+            layer._prompt(q, k_new, v_new, new_slots, k_pool, v_pool, ops.Batch(seq, table, L0 + T, hint=hint), out, 0,
+                          T, chunk)
+        else:
+            for start in range(0, T, chunk):
+                end = min(start + chunk, T)
+                layer._serve(q, k_new, v_new, new_slots, k_pool, v_pool, ops.Batch(seq, table, L0 + end), None, out,
+                             start, end - start)
+        torch.cuda.synchronize()
+        assert not layer.gave_up()
+        results.append((k_pool, v_pool, table[:, :L0 + T], seq, out.view(torch.int16)))
+        assert (int(hint) != 0) == (together and L0 + T > c.max_sel)
+    for name, x, y in zip(("k", "v", "table", "length", "out"), *results):
+        assert torch.equal(x, y), f"{name}: {int((x != y).sum())} of {x.numel()} differ"
 
 
 def test_prefill_short_context_attends_densely(dev):

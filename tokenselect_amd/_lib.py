@@ -109,6 +109,9 @@ SIGNATURES = {
                                _ptr, _i64, _ptr, _ptr, _size, _ptr]),
     "ts_prefill_step_strided": (_i32, [_CFG, _BT, _KV, _ptr, _i32, _i32, _i32, _ptr, _ptr, _i64, _ptr, _ptr,
                                        _i64, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _size, _ptr]),
+    "ts_prefill_prompt_workspace_bytes": (_size, [_CFG, _i32, _i32, _i32]),
+    "ts_prefill_prompt": (_i32, [_CFG, _BT, _KV, _ptr, _i32, _i32, _i32, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _i64,
+                                 _ptr, _ptr, _size, _ptr]),
     "ts_set_fused_select": (_i32, [_i32]),
     "ts_decode_layer_selection": (_i32, [_CFG, _i32, _i32]),
     "ts_decode_layer_selection_of": (_i32, [_CFG, _BT]),
@@ -170,7 +173,7 @@ def binding():
                               "build it with `python -m tokenselect_amd.build`") from e
         _ts_bind.connect(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in
                            ("ts_decode_layer", "ts_decode_step_strided", "ts_prefill_chunk", "ts_prefill_step_strided",
-                            "ts_decode_layer_layout")))
+                            "ts_decode_layer_layout", "ts_prefill_prompt", "ts_prefill_prompt_workspace_bytes")))
         _bind = _ts_bind
     return _bind
 

@@ -133,12 +133,18 @@ using ChunkStepFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*,
 using ChunkFn = int (*)(const ts_config*, const ts_batch*, const void*, int32_t, const float*, const float*, int64_t,
                         const void*, const void*, int64_t, void*, int32_t*, int32_t*, int64_t, int32_t*, void*,
                         size_t, ts_stream_t);
+using PromptFn = int (*)(const ts_config*, const ts_batch*, const ts_new_kv*, const void*, int32_t, int32_t, int32_t,
+                         int32_t, const float*, const float*, int64_t, void*, void*, int64_t, void*, void*, size_t,
+                         ts_stream_t);
+using PromptBytesFn = size_t (*)(const ts_config*, int32_t, int32_t, int32_t);
 using LayoutFn = int64_t (*)(const ts_config*, int32_t, int32_t);
 LayoutFn decode_layer_layout;
 StepFn decode_step;
 LayerFn decode_layer;
 ChunkStepFn prefill_step;
 ChunkFn prefill_chunk;
+PromptFn prefill_prompt;
+PromptBytesFn prefill_prompt_bytes;
 
 // What a DecodeLayer (max_rows == 0) or a PrefillChunk owns.
 struct Owned {
@@ -509,6 +515,52 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   return THPVariable_Wrap(std::move(out));
 }
 
+// prompt(q, k, v, out_cache_loc, k_pool, v_pool, bt, out, from, rows, chunk_rows): `rows` rows of a prompt
+// part from `from` on, in chunks of chunk_rows, as serve() does them one by one.  The workspace is
+// the call's own, in the order of the stream: a prompt's is larger than what a request would keep.
+PyObject* prompt(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 11) raise(PyExc_TypeError, "prompt() takes 11 arguments");
+  Owned& o = *self->own;
+  if (fault_of(o) != 0) Py_RETURN_NONE;
+  const ts_config& cfg = o.cfg;
+  const int64_t width = (int64_t)cfg.num_heads * cfg.head_dim, row = (int64_t)cfg.num_kv_heads * cfg.head_dim;
+  Call call;
+  fill_batch(o, args[6], false, false, &call);
+  ts_batch& bt = call.bt;
+  const int64_t from = as_long(args[8]), rows = as_long(args[9]), chunk_rows = as_long(args[10]);
+  if (o.max_rows < 1 || bt.batch != 1 || chunk_rows > o.max_rows)
+    bad_value("one request, within the sizes this PrefillChunk was built for");
+  if (from < 0 || rows < 1 || rows > INT32_MAX || chunk_rows < 1) bad_value("a chunk has at least one row");
+  const Rows q = rows_of(args[0], "q", from, rows, width, false);
+  Rows k = rows_of(args[1], "k", from, rows, row, false), v = rows_of(args[2], "v", from, rows, row, false);
+  if (k.stride != v.stride) {
+    if (k.stride != row) k = rows_of(args[1], "k", from, rows, row, true);
+    if (v.stride != row) v = rows_of(args[2], "v", from, rows, row, true);
+  }
+  const at::Tensor& k_pool = check_pool(cfg, args[4], "k_pool");
+  const at::Tensor& v_pool = check_pool(cfg, args[5], "v_pool");
+  if (k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
+  if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
+  const Rows loc = slots_of(args[3], from, rows);
+  const ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.ptr, nullptr, (int32_t)call.table_tokens};
+  const at::Tensor& out = need(args[7], "out", at::kBFloat16);
+  if (out.dim() < 1 || out.numel() != out.size(0) * width || out.size(0) < from + rows)
+    bad_value("out must hold the rows of q");
+  const size_t bytes = prefill_prompt_bytes(&cfg, (int32_t)rows, (int32_t)chunk_rows, bt.max_seq_len);
+  const at::Tensor workspace = at::empty({(int64_t)bytes}, o.workspace.options());
+  const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
+  int code;
+  Py_BEGIN_ALLOW_THREADS
+  code = prefill_prompt(&cfg, &bt, &kv, q.ptr, (int32_t)q.stride, (int32_t)k.stride, (int32_t)rows, (int32_t)chunk_rows,
+                        (const float*)o.cos.data_ptr(), (const float*)o.sin.data_ptr(), o.cos.size(0),
+                        k_pool.data_ptr(), v_pool.data_ptr(), k_pool.size(0),
+                        (char*)out.data_ptr() + 2 * from * width, workspace.data_ptr(), bytes, stream);
+  Py_END_ALLOW_THREADS
+  if (code != TS_OK) return PyLong_FromLong(code);
+  Py_INCREF(args[7]);
+  return args[7];
+}
+
 // Runs `f`, with C++ exceptions turned into Python's.
 template <typename F>
 PyObject* guarded(F&& f) {
@@ -527,6 +579,10 @@ PyObject* runner_run(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
 
 PyObject* runner_serve(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&] { return serve((Runner*)self, args, nargs); });
+}
+
+PyObject* runner_prompt(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&] { return prompt((Runner*)self, args, nargs); });
 }
 
 PyObject* runner_new(PyTypeObject* type, PyObject* args, PyObject*) {
@@ -611,6 +667,7 @@ int set_shared(PyObject* self, PyObject* value, void*) {
 PyMethodDef runner_methods[] = {
     {"run", (PyCFunction)(void (*)(void))runner_run, METH_FASTCALL, nullptr},
     {"serve", (PyCFunction)(void (*)(void))runner_serve, METH_FASTCALL, nullptr},
+    {"prompt", (PyCFunction)(void (*)(void))runner_prompt, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyGetSetDef runner_getset[] = {{"clean", get_clean, set_clean, nullptr, nullptr},
                                {"shared", get_shared, set_shared, nullptr, nullptr},
@@ -619,10 +676,13 @@ PyType_Slot runner_slots[] = {{Py_tp_new, (void*)runner_new}, {Py_tp_dealloc, (v
                               {Py_tp_methods, runner_methods}, {Py_tp_getset, runner_getset}, {0, nullptr}};
 PyType_Spec runner_spec = {"_ts_bind.Runner", sizeof(Runner), 0, Py_TPFLAGS_DEFAULT, runner_slots};
 
-// connect(addresses): the library's entry points, in this order.
+// connect(addresses): the library's entry points, in this order (the last two stay where they are
+// not given).
 PyObject* connect(PyObject*, PyObject* args) {
-  unsigned long long a, b, c, d, e;
-  if (!PyArg_ParseTuple(args, "KKKKK", &a, &b, &c, &d, &e)) return nullptr;
+  unsigned long long a, b, c, d, e, f = (uintptr_t)prefill_prompt, g = (uintptr_t)prefill_prompt_bytes;
+  if (!PyArg_ParseTuple(args, "KKKKK|KK", &a, &b, &c, &d, &e, &f, &g)) return nullptr;
+  prefill_prompt = (PromptFn)(uintptr_t)f;
+  prefill_prompt_bytes = (PromptBytesFn)(uintptr_t)g;
   decode_layer = (LayerFn)(uintptr_t)a;
   decode_step = (StepFn)(uintptr_t)b;
   prefill_chunk = (ChunkFn)(uintptr_t)c;

@@ -228,6 +228,24 @@ struct PrefillDense {
   int list_bound;        // entries that are there to be read, and the most that are listed
   ChunkStore store;      // k == NULL: no append, the length counts the chunk already
 };
+// Several chunks of a prompt: of chunk_rows rows each, the last one of what is left.
+struct PromptChunks {
+  int rows, chunk_rows, chunks;
+  int32_t* lens;         // [chunks] the length after each, written by the fingerprints' launch
+  uint32_t* counters;    // what their selections count into, cleared by it
+  size_t counters_stride;
+  int counter_words;
+};
+// Their fingerprints [chunks, H, D], and the store of all their rows (lengths left alone).
+int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride, const float* cos_table,
+                              const float* sin_table, int64_t table_rows, void* qf, const PromptChunks& pc,
+                              const ChunkStore& store, hipStream_t stream);
+// ts_sparse_prefill_attn for several chunks, each over its list; workspace: a chunk's after the other.
+int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride, int32_t rows, int32_t chunk_rows,
+                               const void* k_pool, const void* v_pool, int64_t pool_rows, const int32_t* sel,
+                               int64_t sel_stride, const int32_t* sel_len, int32_t max_sel_len, void* out,
+                               void* workspace, size_t workspace_bytes, hipStream_t stream,
+                               const PrefillDense* dense = nullptr);
 // ts_sparse_prefill_attn for query rows that lie q_stride elements apart.
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,

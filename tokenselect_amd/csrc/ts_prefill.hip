@@ -26,33 +26,18 @@ constexpr int kFpSplit = 4;     // workgroups per head
 constexpr int kFpClear = 16;    // workgroups that clear
 constexpr int kFpThreads = kHeadDim / 2 / kFpSplit / kFpVec * kFpRowGroups;
 
-__global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
+// Workgroup (h, quarter): head h, the quarter's rotation pairs, of one chunk of `rows` rows.
+__device__ __forceinline__ void fingerprint_quarter(
     const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
-    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int heads,
-    ZeroSet zero, ChunkStore cs) {
+    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int h, int quarter) {
 #pragma clang fp contract(off)
   constexpr int half = kHeadDim / 2;
   constexpr int kPairs = half / kFpSplit;   // rotation pairs of this workgroup
   constexpr int kLanes = kPairs / kFpVec;   // threads per row
   static_assert(kFpThreads == kLanes * kFpRowGroups && kFpThreads == 2 * kPairs * kFpRowGroups / 8,
                 "a thread per row group and four pairs, and per eight row groups and column");
-  const int h = blockIdx.x;
-  const int first_pair = blockIdx.y * kPairs;
+  const int first_pair = quarter * kPairs;
   const int i = first_pair + (threadIdx.x % kLanes) * kFpVec, rg = threadIdx.x / kLanes;
-  // On the side: the workgroups past the fingerprint's own store the chunk's K/V rows (the
-  // caller's store of the chunk, which the selection after this launch must find done, riding here
-  // instead of in a launch of its own), and the last kFpClear of them clear the words that the
-  // selection counts into.
-  if ((int)blockIdx.y >= kFpSplit) {
-    const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
-    const int stores = cs.k != nullptr ? cs.workgroups : 0;
-    if (wg < stores)
-      store_chunk_rows<true>(cs, wg, kFpThreads);
-    else if (wg < stores + kFpClear)
-      clear_regions(zero, (uint32_t)(wg - stores) * (kFpThreads / 64) + (threadIdx.x >> 6),
-                    kFpClear * (kFpThreads / 64));
-    return;
-  }
   float lo_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f}, hi_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f};
   // Four rows per step: their loads are independent and go out together; the sums
   // are still taken in row order.
@@ -123,6 +108,53 @@ __global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
   }
 }
 
+__global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
+    const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
+    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int heads,
+    ZeroSet zero, ChunkStore cs) {
+  // On the side: the workgroups past the fingerprint's own store the chunk's K/V rows (the
+  // caller's store of the chunk, which the selection after this launch must find done, riding here
+  // instead of in a launch of its own), and the last kFpClear of them clear the words that the
+  // selection counts into.
+  if ((int)blockIdx.y >= kFpSplit) {
+    const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
+    const int stores = cs.k != nullptr ? cs.workgroups : 0;
+    if (wg < stores)
+      store_chunk_rows<true>(cs, wg, kFpThreads);
+    else if (wg < stores + kFpClear)
+      clear_regions(zero, (uint32_t)(wg - stores) * (kFpThreads / 64) + (threadIdx.x >> 6),
+                    kFpClear * (kFpThreads / 64));
+    return;
+  }
+  fingerprint_quarter(q, q_stride, qf, cos_table, sin_table, table_rows, first_pos, rows, (int)blockIdx.x,
+                      (int)blockIdx.y);
+}
+
+// The same for several chunks of a prompt, chunk blockIdx.z: its fingerprint, the store of its rows
+// (whose positions follow from the length before the first chunk, which the launch after this one
+// advances), the words its selection counts into, and its length.
+__global__ __launch_bounds__(kFpThreads) void prompt_fingerprint_kernel(
+    const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
+    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int heads, PromptChunks pc, ChunkStore cs) {
+  const int chunk = blockIdx.z;
+  const int first = chunk * pc.chunk_rows, rows = min(pc.chunk_rows, pc.rows - first);
+  if ((int)blockIdx.y >= kFpSplit) {
+    const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
+    const int len = *cs.seq_len;
+    if (wg < cs.workgroups) {
+      store_rows_at(cs, len, first + wg * (kFpThreads / kChunkThreadsPerRow) + (int)threadIdx.x / kChunkThreadsPerRow,
+                    first + rows);
+    } else if (wg == cs.workgroups) {
+      uint32_t* const counters = pc.counters + (size_t)chunk * pc.counters_stride;
+      for (int w = threadIdx.x; w < pc.counter_words; w += kFpThreads) counters[w] = 0u;
+      if (threadIdx.x == 0) pc.lens[chunk] = min(len + first + rows, cs.max_tokens);
+    }
+    return;
+  }
+  fingerprint_quarter(q + (size_t)first * q_stride, q_stride, qf + (size_t)chunk * heads * kHeadDim, cos_table,
+                      sin_table, table_rows, first_pos, rows, (int)blockIdx.x, (int)blockIdx.y);
+}
+
 // ------------------------------------------------------------ prefill attention
 // Two launches.
 //
@@ -134,7 +166,7 @@ __global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
 // of the tile one after the other, 1 KB each, 16 bytes per lane in lane order.  The keys of
 // a V^T operand are in the order in which the logits' product leaves them (kv_pos below).
 //
-// prefill_attn_kernel<G>: grid (KV heads, query tiles, head blocks); 256 threads = four
+// prefill_attn_kernel<G>: grid (KV heads, query tiles, head blocks x chunks); 256 threads = four
 // wavefronts, one per SIMD, each a key group of its own: group g takes the 32-key tiles
 // g, g + 4, g + 8, ... for all 64 query columns of the workgroup (kPfBlocks column blocks of
 // 16 query rows of one head: four heads x 16 rows, two x 32 or one x 64, whatever divides G
@@ -172,11 +204,14 @@ struct PrefillArgs {
   const uint16_t* k_pool;
   const uint16_t* v_pool;
   uint32_t pool_rows;
-  const int32_t* sel;      // [S] selected slots in attention order
-  const int32_t* sel_len;  // device scalar S
+  const int32_t* sel;      // [chunk][S] selected slots in attention order
+  const int32_t* sel_len;  // [chunk] S
   int max_sel_len;
   int s_pad;               // keys in kr and vt per KV head: max_sel_len rounded up to kPfPadKeys
-  int rows;
+  int rows;                // of all chunks
+  int chunk_rows;          // of a chunk (the last one may have fewer): a selection for each of them
+  int64_t sel_stride;      // entries between the chunks' lists
+  size_t stage_stride;     // elements between their parts of kr, and of vt
   int32_t* new_len;        // the length that the attention advances by `rows`, up to len_cap, or NULL
   int len_cap;
   int num_heads, num_kv_heads, rope_mode;
@@ -224,7 +259,8 @@ __device__ __forceinline__ void stage(const PrefillArgs& a, void* to, const uint
     *(uint4*)to = w;
 }
 
-// Grid (32-key tiles x KV heads, the head fastest; all on x: the device reports 65536 as the end of y, 2.1 M keys).
+// Grid (32-key tiles x KV heads, the head fastest; all on x: the device reports 65536 as the end of y, 2.1 M keys),
+// by chunks.
 // Thread (key kk, chunk c) moves dims [8c, 8c+8) and
 // [64+8c, +8) of key j = tile + kk.  Keys past S are written as zeros.
 // DENSE (PrefillDense): key j is position j, its slot the table's or, from the length on, one of the
@@ -240,6 +276,7 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
   const int kvh = blockIdx.x & (a.num_kv_heads - 1);
   const uint32_t tile = blockIdx.x >> head_bits, tiles = gridDim.x >> head_bits;
   const int j = tile * kPfKeys + kk;
+  const int chunk = DENSE ? 0 : (int)blockIdx.y;
   // (the slot is asked for together with the length, not after it)
   uint32_t slot;
   if (DENSE) {
@@ -247,12 +284,12 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
     slot = ((uint32_t)d.table[min(j, d.list_bound - 1) >> d.page_shift] << d.page_shift) +
            (uint32_t)(j & ((1 << d.page_shift) - 1));
   } else {
-    slot = (uint32_t)a.sel[min(j, a.max_sel_len - 1)];
+    slot = (uint32_t)a.sel[chunk * a.sel_stride + min(j, a.max_sel_len - 1)];
   }
   const int len = DENSE ? *dense.seq_len : 0;
   const bool appends = DENSE && dense.store.k != nullptr;
   const int end = appends ? min(len + dense.store.rows, dense.store.max_tokens) : len;  // of what is stored
-  const int S = DENSE ? min(max(end, 0), dense.list_bound) : min(max(*a.sel_len, 0), a.max_sel_len);
+  const int S = DENSE ? min(max(end, 0), dense.list_bound) : min(max(a.sel_len[chunk], 0), a.max_sel_len);
   const int row = j - len;  // of the chunk
   const bool fresh = appends && len >= 0 && row >= 0 && j < end;
   // A row of the chunk to its slot (clamped to the pool, as ts_kv_store_chunk does).
@@ -337,7 +374,7 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
     }
   }
   // key kk = 16 kb + qc, dims 32 ks + 8 g4: operand 4 kb + ks, lane 16 g4 + qc
-  const size_t tile_at = ((size_t)kvh * a.s_pad + (size_t)tile * kPfKeys) * kHeadDim;
+  const size_t tile_at = chunk * a.stage_stride + ((size_t)kvh * a.s_pad + (size_t)tile * kPfKeys) * kHeadDim;
   uint16_t* kout = a.kr + tile_at + ((4 * (kk >> 4) + (c8 >> 2)) * 64 + 16 * (c8 & 3) + (kk & 15)) * 8;
   stage(a, kout, make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
                             pack_bf16(lo[6], lo[7])));
@@ -427,6 +464,7 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   constexpr int NH = prefill_heads(G);   // heads of the workgroup
   constexpr int RT = CB / NH;            // query tiles of 16 rows
   constexpr int kRows = 16 * RT;
+  constexpr int kHeadBlocks = (G + NH - 1) / NH;
   // Column block cb: head cb % NH of the workgroup's, query tile cb / NH.
   extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];
   const int group = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // wavefront = key group
@@ -439,15 +477,18 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   const int kvh = blockIdx.x;
   const int q_row0 = (int)(gridDim.y - 1 - blockIdx.y) * kRows;
   const int H = a.num_heads;
-  const int m = a.rows;
-  auto head_in_group = [&](int cb) { return (int)blockIdx.z * NH + cb % NH; };
+  const int chunk = (int)blockIdx.z / kHeadBlocks;
+  const int first_row = chunk * a.chunk_rows;
+  const int m = min(a.chunk_rows, a.rows - first_row);
+  if (q_row0 >= m) return;  // (the last chunk of several may be shorter)
+  auto head_in_group = [&](int cb) { return (int)blockIdx.z % kHeadBlocks * NH + cb % NH; };
   auto head_of = [&](int cb) { return kvh * G + min(head_in_group(cb), G - 1); };
   auto row_of = [&](int cb) { return q_row0 + 16 * (cb / NH) + qc; };
 
   // Tile t of this group holds the keys [(t kPfGroups + group) kPfKeys, + kPfKeys).  A tile
   // past the staging area (asked for ahead, never used) is replaced by the last one.
-  const uint16_t* const k_base = a.kr + (size_t)kvh * a.s_pad * kHeadDim;
-  const uint16_t* const v_base = a.vt + (size_t)kvh * a.s_pad * kHeadDim;
+  const uint16_t* const k_base = a.kr + chunk * a.stage_stride + (size_t)kvh * a.s_pad * kHeadDim;
+  const uint16_t* const v_base = a.vt + chunk * a.stage_stride + (size_t)kvh * a.s_pad * kHeadDim;
   const int last_tile = a.s_pad / kPfKeys - 1;
   auto tile_at = [&](const uint16_t* base, int t) __attribute__((always_inline)) {
     return (const uint4*)(base + (size_t)min(t * kPfGroups + group, last_tile) * kPfTileElems);
@@ -468,12 +509,12 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   uint2 q_raw[CB][2];
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
-    const uint16_t* qrow = a.q + (size_t)min(row_of(cb), m - 1) * a.q_stride + head_of(cb) * kHeadDim +
+    const uint16_t* qrow = a.q + (size_t)(first_row + min(row_of(cb), m - 1)) * a.q_stride + head_of(cb) * kHeadDim +
                            32 * my_ks + 8 * g4 + my_half;
     q_raw[cb][0] = *(const uint2*)qrow;
     q_raw[cb][1] = *(const uint2*)(qrow + 64);
   }
-  const int S = min(max(*a.sel_len, 0), a.max_sel_len);
+  const int S = min(max(a.sel_len[chunk], 0), a.max_sel_len);
   // The length of a dense chunk, whose gather is through (nothing here reads it), by one of the
   // workgroups of the first rows, which see the fewest keys.
   auto commit_length = [&]() {
@@ -491,7 +532,7 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
       for (int i = lane; i < 16 * (kHeadDim / 8); i += 64) {
         const int row = q_row0 + 16 * (cb / NH) + i / (kHeadDim / 8);
         if (row < m)
-          *(uint4*)(a.out + ((size_t)row * H + head_of(cb)) * kHeadDim + 8 * (i % (kHeadDim / 8))) =
+          *(uint4*)(a.out + ((size_t)(first_row + row) * H + head_of(cb)) * kHeadDim + 8 * (i % (kHeadDim / 8))) =
               make_uint4(0u, 0u, 0u, 0u);
       }
     commit_length();
@@ -786,7 +827,7 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   const int row = row_of(cb);
   if (row >= m || head_in_group(cb) >= G) return;
   const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
-  uint16_t* orow = a.out + ((size_t)row * H + head_of(cb)) * kHeadDim;
+  uint16_t* orow = a.out + ((size_t)(first_row + row) * H + head_of(cb)) * kHeadDim;
 #pragma unroll
   for (int db = 0; db < 8; ++db)
     *(uint2*)(orow + 16 * db + 4 * g4) = make_uint2(pack_bf16(sum[db][0] * inv, sum[db][1] * inv),
@@ -827,19 +868,42 @@ int launch_fingerprint(const ts_config* cfg, const void* q, int q_stride, int32_
   return check_launch("fingerprint_kernel");
 }
 
+int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride, const float* cos_table,
+                              const float* sin_table, int64_t table_rows, void* qf, const PromptChunks& pc,
+                              const ChunkStore& store, hipStream_t stream) {
+  TS_TRY(check_fingerprint(q, pc.chunk_rows, cos_table, sin_table, table_rows, qf, cfg->n_local));
+  ChunkStore cs = store;
+  cs.workgroups = (int)ceil_div(pc.chunk_rows, kFpThreads / kChunkThreadsPerRow);
+  const unsigned grid_y = kFpSplit + (unsigned)ceil_div(cs.workgroups + 1, cfg->num_heads);
+  hipLaunchKernelGGL(prompt_fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y, (unsigned)pc.chunks),
+                     dim3(kFpThreads), 0, stream, (const uint16_t*)q, q_stride, (uint16_t*)qf, cos_table, sin_table,
+                     table_rows, cfg->n_local, cfg->num_heads, pc, cs);
+  return check_launch("prompt_fingerprint_kernel");
+}
+
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }
 
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
                         int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes,
                         hipStream_t stream, const PrefillDense* dense) {
+  return launch_prefill_attn_chunks(cfg, q, q_stride, rows, rows, k_pool, v_pool, pool_rows, sel, 0, sel_len,
+                                    max_sel_len, out, workspace, workspace_bytes, stream, dense);
+}
+
+int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride, int32_t rows, int32_t chunk_rows,
+                               const void* k_pool, const void* v_pool, int64_t pool_rows, const int32_t* sel,
+                               int64_t sel_stride, const int32_t* sel_len, int32_t max_sel_len, void* out,
+                               void* workspace, size_t workspace_bytes, hipStream_t stream,
+                               const PrefillDense* dense) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(q && k_pool && v_pool && sel && sel_len && out, TS_EINVAL,
              "ts_sparse_prefill_attn: NULL tensor argument");
   TS_REQUIRE(rows >= 1 && rows <= 65535 * 16, TS_EINVAL, "rows %d out of range", rows);
   TS_REQUIRE(pool_rows >= 1 && pool_rows <= 0x7fffffffLL, TS_EINVAL, "pool_rows %lld out of range",
              (long long)pool_rows);
-  const size_t need = ts_prefill_attn_workspace_bytes(cfg, max_sel_len);
+  const unsigned chunks = (unsigned)ceil_div(rows, chunk_rows);
+  const size_t per_chunk = ts_prefill_attn_workspace_bytes(cfg, max_sel_len), need = chunks * per_chunk;
   TS_REQUIRE(workspace != nullptr && workspace_bytes >= need, TS_EWORKSPACE,
              "ts_sparse_prefill_attn: workspace %zu bytes < required %zu", workspace_bytes, need);
   TS_REQUIRE_ALIGNED(workspace, 256, "workspace");
@@ -858,6 +922,9 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
   a.max_sel_len = max_sel_len;
   a.s_pad = prefill_s_pad(max_sel_len);
   a.rows = rows;
+  a.chunk_rows = chunk_rows;
+  a.sel_stride = sel_stride;
+  a.stage_stride = per_chunk / 2;  // (a chunk's kr, then its vt: bytes to elements, twice as far apart)
   a.num_heads = cfg->num_heads;
   a.num_kv_heads = cfg->num_kv_heads;
   a.rope_mode = cfg->rope_mode;
@@ -866,12 +933,12 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
   a.sm_scale = cfg->sm_scale;
   a.logit_cap = cfg->logit_cap;
   a.kr = (uint16_t*)workspace;
-  a.vt = (uint16_t*)((char*)workspace + need / 2);
+  a.vt = (uint16_t*)((char*)workspace + per_chunk / 2);
   a.out = (uint16_t*)out;
   a.new_len = dense && dense->store.k ? dense->seq_len : nullptr;
   a.len_cap = dense ? dense->store.max_tokens : 0;
   hipStream_t st = stream;
-  const dim3 gather_grid((unsigned)cfg->num_kv_heads * (unsigned)(a.s_pad / kPfKeys));
+  const dim3 gather_grid((unsigned)cfg->num_kv_heads * (unsigned)(a.s_pad / kPfKeys), chunks);
   if (dense)
     hipLaunchKernelGGL(prefill_gather_dense_kernel, gather_grid, dim3(256), 0, st, a, *dense);
   else
@@ -879,8 +946,8 @@ int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32
   TS_TRY(check_launch("prefill_gather_kernel"));
   const int group = cfg->num_heads / cfg->num_kv_heads;
   const int heads = prefill_heads(group);
-  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(rows, 16 * (kPfBlocks / heads)),
-                  (unsigned)ceil_div(group, heads));
+  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(chunk_rows, 16 * (kPfBlocks / heads)),
+                  (unsigned)ceil_div(group, heads) * chunks);
   const bool cap = cfg->logit_cap > 0.f;
 #define TS_PF_LAUNCH(G_, C_)                                                                  \
   {                                                                                           \

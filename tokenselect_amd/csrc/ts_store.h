@@ -37,14 +37,11 @@ __device__ __forceinline__ int counted_length(const ChunkStore& cs) {
   return __hip_atomic_load(cs.seq_len, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kLenMask;
 }
 
-// wg: this workgroup among the cs.workgroups that store; threads: its size.
-template <bool COUNTED>
-__device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, int threads) {
-  const int len = COUNTED ? counted_length(cs) : *cs.seq_len;
-  const int r = wg * (threads / kChunkThreadsPerRow) + (int)threadIdx.x / kChunkThreadsPerRow;
+// Row r (below `end`) of those that follow the length `len`, by kChunkThreadsPerRow threads.
+__device__ __forceinline__ void store_rows_at(const ChunkStore& cs, int len, int r, int end) {
   const int t = threadIdx.x % kChunkThreadsPerRow;
   const int at = len + r;
-  if (r < cs.rows && at >= 0 && at < cs.max_tokens) {
+  if (r < end && at >= 0 && at < cs.max_tokens) {
     int64_t slot = cs.loc[r];
     slot = slot < 0 ? 0 : (slot >= cs.pool_rows ? cs.pool_rows - 1 : slot);
     for (int i = t; i < cs.row_vec; i += kChunkThreadsPerRow) {
@@ -53,6 +50,13 @@ __device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, i
     }
     if (t == 0) cs.table[at] = (int32_t)slot;
   }
+}
+
+// wg: this workgroup among the cs.workgroups that store; threads: its size.
+template <bool COUNTED>
+__device__ __forceinline__ void store_chunk_rows(const ChunkStore& cs, int wg, int threads) {
+  const int len = COUNTED ? counted_length(cs) : *cs.seq_len;
+  store_rows_at(cs, len, wg * (threads / kChunkThreadsPerRow) + (int)threadIdx.x / kChunkThreadsPerRow, cs.rows);
   if (COUNTED) count_chunk_workgroup(cs, len);
 }
 

@@ -48,6 +48,9 @@ struct TopkArgs {
   // A word an earlier kernel of the stream leaves non-zero when the votes are not
   // valid (a wait of the fused scoring gave up): sel_len then reports -1.  Or NULL.
   const uint32_t* fault;
+  // Where the last request's k-th vote is left for a later selection's guess (ts_batch.threshold_hint,
+  // as ts_select leaves it), or NULL.
+  int32_t* hint;
 };
 
 __device__ __host__ __forceinline__ uint32_t* topk_ws(uint32_t* ws, size_t stride, int b) {

@@ -216,6 +216,7 @@ __global__ __launch_bounds__(kTopkFinalThreads) void topk_final_kernel(TopkArgs 
 
   uint32_t t0, above0, t1, above1, t2, above2;
   search_threshold_bins<kTopkBins, kTopkFinalThreads>(bins0, (uint32_t)k, scratch, t0, above0);
+  if (a.hint && b + 1 == (int)gridDim.y && part == 0 && tid == 0) *a.hint = (int)t0 + 1;
   const uint32_t need1 = (uint32_t)k - above0;  // still to take inside bin t0
   search_threshold_bins<kTopkBins, kTopkFinalThreads>(bins1, need1, scratch, t1, above1);
   const uint32_t need2 = need1 - above1;  // still to take inside (t0, t1)
@@ -355,6 +356,7 @@ TopkArgs make_topk_args(const ts_config* cfg, const ts_batch* bt, const float* v
   a.clear = nullptr;
   a.clear_per_req = 0;
   a.fault = nullptr;
+  a.hint = nullptr;
   a.slice = kTopkSlice;
   return a;
 }

@@ -998,6 +998,17 @@ class PrefillChunk(_GiveUpLatch):
     def _shapes(self):
         return self.cos, self.sin, None, 1, self.max_rows
 
+    def _prompt(self, q, k, v, loc, k_pool, v_pool, bt, out, start: int, rows: int, chunk_rows: int) -> torch.Tensor:
+        """``rows`` rows of a prompt part from row ``start`` on as chunks of ``chunk_rows`` that are taken
+        together (``ts_prefill_prompt``), where :meth:`_serve` takes one; ``bt.max_seq_len`` bounds the
+        length after the last of them."""
+        got = self._native.prompt(q, k, v, loc, k_pool, v_pool, bt, out, start, rows, chunk_rows)
+        if got is None:   # an earlier call gave up
+            self.check()
+        if type(got) is int:
+            _lib.check(got)
+        return got
+
     def recover(self, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, bt: Batch,
                 out: Optional[torch.Tensor] = None):
         """As :meth:`DecodeLayer.recover`: after a synchronisation, repeats a chunk whose

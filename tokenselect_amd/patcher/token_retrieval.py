@@ -563,14 +563,32 @@ class TokenRetriever:
         out, _, _, _ = self._prefill_chunk(attn)(q, k_buffer, v_buffer, bt)
         return out
 
+    def _together(self, layer_id, rows) -> bool:
+        """Whether the chunks of ``rows`` more tokens all select, and fit the table and what the library
+        ranks (2^20 candidates)."""
+        held = self.num_tokens[layer_id]
+        fixed = max(N_INIT, 0) + max(N_Local, 0)
+        return held + PREFILL_CHUNK_SIZE > fixed + TOP_K and held + rows <= self.max_num_tokens \
+            and held + rows - fixed <= 1 << 20
+
     def prefill_step(self, attn, q, k, v, loc, k_buffer, v_buffer, out):
-        """The whole prompt part in chunks (tr.py:716-773), each one library call: its store,
-        then :meth:`prefill_attention`, the rows of ``out`` written in place."""
+        """The whole prompt part in chunks (tr.py:716-773): each its store, then
+        :meth:`prefill_attention`, the rows of ``out`` written in place.  From the first chunk on that
+        selects they are taken together, if there are several (a part that does not fit the
+        table goes up to where it does not, chunk by chunk)."""
         layer_id, rows = attn.layer_id, q.shape[0]
         runner = self._prefill_chunk(attn)
         bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
                        self.token_indices[layer_id:layer_id + 1], 0)
         for start in range(0, rows, PREFILL_CHUNK_SIZE):
+            if PREFILL_CHUNK_SIZE < rows - start and self._together(layer_id, rows - start):
+                length = self.num_tokens[layer_id] + rows - start
+                last = (rows - start - 1) % PREFILL_CHUNK_SIZE + 1
+                bt.max_seq_len = length
+                bt.hint = self._chunk_hint(layer_id, length - last, last)
+                runner._prompt(q, k, v, loc, k_buffer, v_buffer, bt, out, start, rows - start, PREFILL_CHUNK_SIZE)
+                self.num_tokens[layer_id] = length
+                break
             here = min(PREFILL_CHUNK_SIZE, rows - start)
             length = self.num_tokens[layer_id] + here
             assert length <= self.max_num_tokens   # tr.py:334
