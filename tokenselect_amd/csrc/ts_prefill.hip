@@ -4,9 +4,10 @@
 // prefill, tr.py:759-771, page size 1, in-kernel Llama RoPE).
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
-#include "ts_common.h"
+#include "ts_prefill.h"
 #include "ts_store.h"
 
 namespace ts {
@@ -198,45 +199,10 @@ __global__ __launch_bounds__(kFpThreads) void prompt_fingerprint_kernel(
 // CU at the 110 GB/s that L2 delivers to one: 13 us).  What is left over is mostly the
 // loads' latency: 64 KB per CU in flight, 0.6 to 0.85 us from L2 under this load.
 // Alternating products and exp2 in the source order of the logits' steps changed nothing.
-struct PrefillArgs {
-  const uint16_t* q;  // [rows, H, 128] bf16, un-rotated, rows q_stride elements apart
-  int q_stride;
-  const uint16_t* k_pool;
-  const uint16_t* v_pool;
-  uint32_t pool_rows;
-  const int32_t* sel;      // [chunk][S] selected slots in attention order
-  const int32_t* sel_len;  // [chunk] S
-  int max_sel_len;
-  int s_pad;               // keys in kr and vt per KV head: max_sel_len rounded up to kPfPadKeys
-  int rows;                // of all chunks
-  int chunk_rows;          // of a chunk (the last one may have fewer): a selection for each of them
-  int64_t sel_stride;      // entries between the chunks' lists
-  size_t stage_stride;     // elements between their parts of kr, and of vt
-  int32_t* new_len;        // the length that the attention advances by `rows`, up to len_cap, or NULL
-  int len_cap;
-  int num_heads, num_kv_heads, rope_mode;
-  float log2_theta, rope_rcp_scale, sm_scale, logit_cap;
-  uint16_t* kr;   // [Hkv, s_pad / 32, operand 4 kb + ks, lane, 8] bf16 rotated keys
-  uint16_t* vt;   // [Hkv, s_pad / 32, operand db, lane, 8] bf16 transposed values
-  uint16_t* out;  // [rows, H, 128] bf16
-};
-
-typedef __attribute__((ext_vector_type(8))) __bf16 pf_bf16x8;
-typedef __attribute__((ext_vector_type(4))) float pf_f32x4;
-constexpr float kLog2e = 1.4426950408889634f;
-
-constexpr int kPfKeys = 32;            // keys per tile: of the gather kernel and of the attention kernel
 constexpr int kPfVRow = kPfKeys + 8;   // halfwords per V^T row in the gather kernel's LDS (80 B)
-constexpr int kPfPadKeys = 64;         // the staging area holds whole multiples of this many keys
-constexpr int kPfGroups = 4;           // key groups of an attention workgroup: its wavefronts
-constexpr int kPfBlocks = 4;           // column blocks (16 query rows of one head) of a wavefront
-constexpr int kPfTileElems = kPfKeys * kHeadDim;      // a K tile; a V^T tile is as large
-constexpr int kPfOperands = kPfTileElems / (64 * 8);  // operands of a tile: 16 bytes per lane each
 // The merge area: per group and column block eight vectors of accumulators and (max, sum),
 // four floats per lane each.  (The rotated queries pass through the same space at the start.)
 constexpr size_t kPfLdsBytes = (size_t)kPfGroups * kPfBlocks * 9 * 64 * 16;  // 144 KB
-static_assert(kPfOperands == 8, "a tile has eight operands");
-constexpr float kPfRaise = 8.0f;       // a row's maximum is raised when a logit exceeds it by this much
 
 // Position of key kk (0..31 within its block) in a V^T row: the matrix instruction
 // that made the logits left lane group g4 with keys 16 kb + 4 g4 + r (kb < 2, r < 4),
@@ -404,50 +370,6 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
 __global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) { gather_tile<false>(a, PrefillDense{}); }
 __global__ __launch_bounds__(256) void prefill_gather_dense_kernel(PrefillArgs a, PrefillDense dense) {
   gather_tile<true>(a, dense);
-}
-
-// Largest of three, without the NaN-quieting copies fmaxf brings along.
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float d;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-  return d;
-}
-
-// The products, with their registers in the half of the register file that suits them: the
-// accumulators of the output and the queries in the accumulation registers, the logits,
-// which vector instructions read, in the others.  Written as assembly because the compiler,
-// left to choose, moves accumulators to and fro around every product (480 moves per tile).
-// What it does not see it does not keep apart: between a product and any use of its result other
-// than as the same product's next accumulator there must be eight instructions' issue, and two
-// between a vector instruction and a product that reads its result.  The two fences below make
-// that order a dependency of the values themselves; tests/test_prefill_hazards_cpu.py looks
-// through the compiler's listing for what register copies could still have put in between.
-__device__ __forceinline__ void mfma_acc(pf_f32x4& acc, const pf_bf16x8& a, const pf_bf16x8& b) {
-  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ pf_f32x4 mfma_logits(const pf_f32x4& s, const uint4& k, const pf_bf16x8& q) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, k), q, s, 0, 0, 0);
-}
-// Says that acc lives in the accumulation registers here, so that where paths join it stays there.
-template <typename V>
-__device__ __forceinline__ void keep_acc(V& acc) { asm("" : "+a"(acc)); }
-// The accumulators behind this are those before it, sixteen idle instructions later: no use of
-// one can come before the idling, and no product that makes one after it.
-template <int CB>
-__device__ __forceinline__ void mfma_settled(pf_f32x4 (&o)[CB][8]) {
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-    for (int db = 0; db < 8; ++db) asm volatile("" : "+a"(o[cb][db]));
-  asm volatile("s_nop 15" ::: "memory");
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-    for (int db = 0; db < 8; ++db) asm volatile("" : "+a"(o[cb][db]));
-}
-// The weights behind this are those before it, two idle instructions later.
-__device__ __forceinline__ void packed_settled(pf_bf16x8 (&pb)[4]) {
-  asm("s_nop 1" : "+v"(pb[0]), "+v"(pb[1]), "+v"(pb[2]), "+v"(pb[3]));
 }
 
 // Heads of a workgroup's column blocks; the kPfBlocks / heads blocks of a head are
@@ -881,6 +803,23 @@ int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride,
   return check_launch("prompt_fingerprint_kernel");
 }
 
+// Chunks, from the first on, whose attention takes the workgroups of 256 columns.  A wave of those over the
+// device, a workgroup per CU, takes 75 us for 2688 keys, and one of the workgroups of 64 columns 20 where all
+// of them read the same 1.4 MB per head, 26 where each chunk has its own: so they get all chunks where
+// their last wave is at least 0.8 full, else as many as fill whole waves (20 chunks of 512 rows, 28 heads on 4,
+// are 1120: 18 of them four waves less 16, 300 us, and two chunks 52).  The rows of a long dense chunk
+// see fewer keys the earlier they are, and the early ones fill the last wave up: 115 us instead of 161 with
+// 1.5 waves, 159 instead of 192 with two, 107 instead of 77 with 0.75.
+static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_rows) {
+  const int64_t each = prefill_shared_workgroups(num_heads, num_kv_heads, chunk_rows), chunks = ceil_div(rows, chunk_rows);
+  // (small chunks would leave most of a workgroup without columns)
+  if (4 * chunk_rows * (int64_t)num_heads < 3 * each * 256) return 0;
+  const int64_t full = each * chunks / 256, rest = each * chunks - full * 256;
+  if (rest >= 205 || rest == 0 || (chunks == 1 && each >= 320)) return (int)chunks;
+  return (int)(full * 256 / each);
+}
+
+
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }
 
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
@@ -944,10 +883,23 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
   else
     hipLaunchKernelGGL(prefill_gather_kernel, gather_grid, dim3(256), 0, st, a);
   TS_TRY(check_launch("prefill_gather_kernel"));
+  const int together = shared_chunks(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows);
+  if (together > 0) {
+    PrefillArgs first = a;
+    first.rows = (int)std::min<int64_t>(rows, (int64_t)together * chunk_rows);
+    TS_TRY(launch_prefill_shared(first, together, st));
+    if (together == (int)chunks) return TS_OK;
+    a.q += (size_t)first.rows * q_stride;
+    a.out += (size_t)first.rows * cfg->num_heads * kHeadDim;
+    a.sel_len += together;
+    a.kr += together * a.stage_stride;
+    a.vt += together * a.stage_stride;
+    a.rows -= first.rows;
+  }
   const int group = cfg->num_heads / cfg->num_kv_heads;
   const int heads = prefill_heads(group);
   const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(chunk_rows, 16 * (kPfBlocks / heads)),
-                  (unsigned)ceil_div(group, heads) * chunks);
+                  (unsigned)ceil_div(group, heads) * (chunks - (unsigned)together));
   const bool cap = cfg->logit_cap > 0.f;
 #define TS_PF_LAUNCH(G_, C_)                                                                  \
   {                                                                                           \

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(kPrThreads, 2) void prompt_votes_kernel(PromptScore
 // --------------------------------------------------------------------------------- host
 // Chunks that one round of launches takes, at most: the launches' fixed cost is shared by then, and the
 // staged keys and values of a round (11 MB a chunk at 8 KV heads) stay below the last-level cache.
-constexpr int kPrGroup = 16;
+constexpr int kPrGroup = 20;
 // Blocks of tokens: enough for two workgroups per CU, few enough for their statistics to be merged by
 // every workgroup of the votes on its own (128 of four chunks' 28 heads: 110 KB from L2, 1 us).
 constexpr int kPrBlocks = 128;
