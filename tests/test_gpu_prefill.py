@@ -463,6 +463,47 @@ def test_chunks_of_a_prompt_together(dev, shape, case):
         assert torch.equal(x, y), f"{name}: {int((x != y).sum())} of {x.numel()} differ"
 
 
+# A wavefront of the prompt's scores takes 64 tokens a step of one KV head or of two, and a workgroup 64, 128
+# or 256 of all of them; five sets of chunks get 103 blocks of whole steps each.
+@pytest.mark.parametrize("heads,kv_heads", [(4, 1), (8, 1), (6, 2), (14, 2), (4, 4), (28, 4), (8, 8), (64, 8)])
+@pytest.mark.parametrize("steps,odd", [(0, 1), (1, 0), (1, 1), (2, -1), (3, 0), (3, 1), (4, -17)])
+def test_scores_of_a_prompts_chunks_by_steps(dev, heads, kv_heads, steps, odd):
+    """Chunks together against one by one where the last chunk's candidates are around whole steps of a
+    block (of one to four of them, some chunks of a set with fewer): the same selections, so the same outputs."""
+    per_step = 64 * max(1, 4 // kv_heads)
+    T, top_k, n_init, n_local = 18, 64, 8, 32
+    n = (per_step * (steps if steps < 2 else 103 * (steps - 1) + 5)) + odd
+    L0 = max(n + n_init + n_local - T, 1)
+    say(f"prompt steps H={heads} kv={kv_heads} candidates={n} L0={L0}")
+    shape = dict(SHAPES[0], num_heads=heads, num_kv_heads=kv_heads)
+    wl = workloads.build("ps", shape, [L0], [top_k], 1, dev, seed=31, n_init=n_init, n_local=n_local, top_k=top_k,
+                         extra_pages=T)
+    c = wl.cfg
+    g = torch.Generator(device=dev).manual_seed(32)
+    common = torch.randn((1, c.num_heads * 128), generator=g, device=dev)
+    q = (common + torch.randn((T, c.num_heads * 128), generator=g, device=dev)).bfloat16()
+    k_new, v_new = torch.randn((2, T, c.num_kv_heads, 128), generator=g, device=dev).bfloat16()
+    slots = wl.free_pages[:T].contiguous()
+    results = []
+    for together in (True, False):
+        k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
+        table = torch.zeros((1, L0 + T), dtype=torch.int32, device=dev)
+        table[0, :L0] = wl.table[0, :L0]
+        seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
+        out = torch.empty_like(q)
+        layer = ops.PrefillChunk(c, L0 + T, dev, max_rows=1)
+        if together:
+            layer._prompt(q, k_new, v_new, slots, k_pool, v_pool, ops.Batch(seq, table, L0 + T), out, 0, T, 1)
+        else:
+            for i in range(T):
+                layer._serve(q, k_new, v_new, slots, k_pool, v_pool, ops.Batch(seq, table, L0 + i + 1), None, out, i, 1)
+        torch.cuda.synchronize()
+        assert not layer.gave_up()
+        results.append((k_pool, v_pool, table, seq, out.view(torch.int16)))
+    for name, x, y in zip(("k", "v", "table", "length", "out"), *results):
+        assert torch.equal(x, y), f"{name}: {int((x != y).sum())} of {x.numel()} differ"
+
+
 def test_prefill_short_context_attends_densely(dev):
     """n_init + k + n_local >= L: the chunk attends over every token so far (tr.py:741-744)."""
     say("prefill chunk, dense context")

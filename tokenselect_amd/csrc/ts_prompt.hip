@@ -4,11 +4,12 @@
 // What a chunk selects from is the context before it and its own rows, and what it attends to are
 // rows of that: once all rows are stored no chunk needs another one's result.  A chunk on its own
 // is four launches that are chains of round trips (fingerprint 7 us, selection 23 to 60 with its
-// workgroups waiting for each other, gather 6.5, attention 25); together they are seven launches
+// workgroups waiting for each other, gather 6.5, attention 25); together they are eight launches
 // for all of them, of which only the attention is long:
 //
 //   fingerprints    of all chunks, the store of all their rows, every chunk's length
 //   statistics      per (chunk, head) maximum and sum of exponentials of the scores, by blocks of tokens
+//   merge           of the blocks' statistics
 //   votes           the scores once more, as votes (tr.py:361), and the first histogram of the top-k
 //   [max-pool]      tr.py:366-369
 //   mark, final     the ragged top-k, a chunk as a request
@@ -17,9 +18,10 @@
 // Nobody waits for anybody.  The scores are computed twice instead of kept: for one chunk the keys
 // are the cost (the single launch streams them once and holds the scores in LDS), for four chunks
 // that a workgroup serves together they are read for all of them, and 16 query rows fill the
-// matrix instruction's tile.  A prompt of 31599 tokens with 16 more, 28 heads on 4: 4112 -> 2584 us;
-// three of 700 to 5200 tokens, 32 heads on 8, two layers: 2343 -> 2126.
+// matrix instruction's tile.  A prompt of 31599 tokens with 16 more, 28 heads on 4, its chunks one after
+// the other and together: 4140 and 2075 us; three of 700 to 5200 tokens, 32 heads on 8, two layers: 2340 and 1920.
 #include <algorithm>
+#include <type_traits>
 
 #include "ts_topk.h"
 
@@ -28,23 +30,38 @@ namespace ts {
 typedef __attribute__((ext_vector_type(8))) __bf16 pr_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float pr_f32x4;
 
-constexpr int kPrThreads = 256;
+constexpr int kPrWaves = 4;
+constexpr int kPrThreads = 64 * kPrWaves;
 constexpr int kPrChunks = 4;    // chunks of a workgroup: lane group l / 16 of a product's result has chunk l / 16
 constexpr int kPrTiles = 4;     // tiles of 16 tokens of a wavefront's step
-constexpr int kPrTokens = kPrThreads / 64 * kPrTiles * 16;  // tokens of a workgroup's step
+
+// A workgroup's four wavefronts take KV heads of their own: 64 tokens a step with four of them or more, and
+// more tokens where the heads are fewer.  A wavefront then has its query rows in registers for all its tokens,
+// and a workgroup of few tokens is a short chain: with all heads one after the other in every wavefront, the
+// queries in LDS and each workgroup merging the statistics for itself, a workgroup of 256 tokens took 23 us
+// (statistics) and 46 us (votes) whatever the length.  Statistics, merge and votes of 19 chunks up to 31K tokens,
+// 28 heads on 4: 43 + 95 -> 26 + 5 + 31 us; of 6 up to 5K, 32 on 8: 23 + 51 -> 9 + 5 + 12.
+template <int HKV>
+struct PromptSplit {
+  static constexpr int kHeadGroups = HKV < kPrWaves ? HKV : kPrWaves;
+  static constexpr int kHeads = HKV / kHeadGroups;          // of a wavefront
+  static constexpr int kTokenGroups = kPrWaves / kHeadGroups;
+  static constexpr int kTokens = kTokenGroups * kPrTiles * 16;  // of a step
+};
+constexpr int prompt_token_groups(int kv_heads) { return kv_heads < kPrWaves ? kPrWaves / kv_heads : 1; }
 
 struct PromptScoreArgs {
   const uint16_t* qf;  // [chunks, H, 128] bf16 fingerprints
   const uint4* k_pool;
   uint32_t pool_rows;
-  const int32_t* table;
-  int page_size, page_shift;
+  const int32_t* table; // per token
   const int32_t* lens;  // [chunks]
   int chunks, sets;     // sets of kPrChunks
   int n_init, n_local, top_k, max_seq_len, num_heads, head_map;
   int blocks, tokens_per_block;
-  float2* partials;     // [chunk][head slot][block] (max, sum exp); head slot: KV head x G + g
-  int32_t* seq_len;     // the request's length, advanced by the first of the two
+  float2* partials;     // [chunk][head slot][block, token group] (max, sum exp); head slot: KV head x G + g
+  float2* stats;        // [chunk][head slot] (max, 1 / sum exp)
+  int32_t* seq_len;     // the request's length, advanced by the first of the launches
   float* votes;
   int64_t vote_stride;
   uint32_t* hist_ws;    // top-k workspace, or NULL: no histogram
@@ -59,74 +76,87 @@ __device__ __forceinline__ void prompt_workgroup(const PromptScoreArgs& a, int& 
   block = q * 8 + r % 8;
 }
 
-// The query rows of a set as A operands in LDS: operand (KV head, block of four heads, k-step), lane l
-// row l % 16, dims 32 ks + 8 (l / 16) + [0, 8).  Row 4 c + i is chunk c's head 4 nb + i of the KV
-// head's G (zeros where there is none), so that a lane of the result holds heads of one chunk.
-template <int HKV, int NB>
-__device__ __forceinline__ void stage_queries(const PromptScoreArgs& a, int set, uint4* to) {
-  const int G = a.num_heads / HKV;
-  for (int i = threadIdx.x; i < HKV * NB * 4 * 64; i += kPrThreads) {
-    const int lane = i & 63, ks = (i >> 6) & 3, nb = (i >> 8) % NB, kvh = (i >> 8) / NB;
-    const int chunk = set * kPrChunks + ((lane & 15) >> 2), g = 4 * nb + (lane & 3);
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (chunk < a.chunks && g < G) {
-      const int h = a.head_map == TS_HEADMAP_MOD ? kvh + HKV * g : kvh * G + g;
-      v = *(const uint4*)(a.qf + ((size_t)chunk * a.num_heads + h) * kHeadDim + 32 * ks + 8 * (lane >> 4));
-    }
-    to[i] = v;
-  }
-}
-
-// What a workgroup's set and block are: candidates of each chunk, rows of the pool per token.
+// What a workgroup's set and block are, and a wavefront's share of them.
 struct PromptBlock {
-  int set, base, steps;  // steps of kPrTokens tokens that hold candidates of the last chunk
-  int n;                 // candidates of this lane's chunk (0: attends to everything, or no chunk)
+  int set, block, base, steps;  // steps that hold candidates of the last chunk
+  int most;                     // candidates of that
+  int chunk, n;                 // this lane's chunk, and its candidates (0: attends to everything, or no chunk)
+  int token0;                   // the lane's first token
+  int kvh0, token_group;        // the wavefront's first KV head
 };
 __device__ __forceinline__ int candidates(const PromptScoreArgs& a, int chunk) {
   if (chunk >= a.chunks) return 0;
   return request_geometry(a.lens, nullptr, chunk, a.n_init, a.n_local, a.top_k, a.max_seq_len).n;
 }
-// false: nothing to do.  rows: tokens_per_block words of LDS.
-__device__ __forceinline__ bool prompt_block(const PromptScoreArgs& a, PromptBlock& pb, uint32_t* rows) {
-  int block;
-  prompt_workgroup(a, block, pb.set);
-  if (block >= a.blocks) return false;
-  pb.base = block * a.tokens_per_block;
+// false: nothing to do.
+template <int HKV>
+__device__ __forceinline__ bool prompt_block(const PromptScoreArgs& a, PromptBlock& pb) {
+  using Split = PromptSplit<HKV>;
+  prompt_workgroup(a, pb.block, pb.set);
+  if (pb.block >= a.blocks) return false;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  pb.base = pb.block * a.tokens_per_block;
+  pb.chunk = pb.set * kPrChunks + (lane >> 4);
   // (lengths do not fall from chunk to chunk)
-  const int most = candidates(a, min(pb.set * kPrChunks + kPrChunks, a.chunks) - 1);
-  if (pb.base >= most) return false;
-  pb.n = candidates(a, pb.set * kPrChunks + ((int)(threadIdx.x & 63) >> 4));
-  const int end = min(a.tokens_per_block, most - pb.base);
-  pb.steps = (end + kPrTokens - 1) / kPrTokens;
-  for (int i = threadIdx.x; i < pb.steps * kPrTokens; i += kPrThreads)
-    rows[i] = lookup_slot(a.table, a.n_init + pb.base + min(i, end - 1), a.page_size, a.page_shift, a.pool_rows);
+  pb.most = candidates(a, min(pb.set * kPrChunks + kPrChunks, a.chunks) - 1);
+  pb.n = candidates(a, pb.chunk);
+  if (pb.base >= pb.most) return false;
+  pb.steps = (min(a.tokens_per_block, pb.most - pb.base) + Split::kTokens - 1) / Split::kTokens;
+  pb.token_group = wave / Split::kHeadGroups;
+  pb.kvh0 = wave % Split::kHeadGroups * Split::kHeads;
+  pb.token0 = pb.base + pb.token_group * (16 * kPrTiles) + (lane & 15);
   return true;
+}
+
+// The query rows of a set for a wavefront's KV heads as A operands: lane l row l % 16, dims
+// 32 ks + 8 (l / 16) + [0, 8).  Row 4 c + i is chunk c's head 4 nb + i of the KV head's G (zeros where
+// there is none), so that a lane of the result holds heads of one chunk.
+template <int HKV, int NB>
+struct PromptQueries {
+  uint4 q[PromptSplit<HKV>::kHeads][NB][4];
+};
+template <int HKV, int NB>
+__device__ __forceinline__ void load_queries(const PromptScoreArgs& a, const PromptBlock& pb, PromptQueries<HKV, NB>& to) {
+  const int lane = threadIdx.x & 63, G = a.num_heads / HKV, chunk = pb.set * kPrChunks + ((lane & 15) >> 2);
+#pragma unroll
+  for (int x = 0; x < PromptSplit<HKV>::kHeads; ++x)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int g = 4 * nb + (lane & 3), kvh = pb.kvh0 + x;
+      const bool there = chunk < a.chunks && g < G;
+      const int h = a.head_map == TS_HEADMAP_MOD ? kvh + HKV * g : kvh * G + g;
+      const uint16_t* const row = a.qf + ((size_t)chunk * a.num_heads + h) * kHeadDim + 8 * (lane >> 4);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) to.q[x][nb][ks] = there ? *(const uint4*)(row + 32 * ks) : make_uint4(0u, 0u, 0u, 0u);
+    }
 }
 
 // A wavefront's 64 tokens of a step: lane (token l % 16, l / 16) has dims 32 ks + 8 (l / 16) + [0, 8).
 struct KeyTiles {
   uint4 k[kPrTiles][4];
 };
+// (rows as the table has them: they are checked here, where they are used, and not where they are asked for)
 template <int HKV>
 __device__ __forceinline__ void load_keys(const PromptScoreArgs& a, const uint32_t (&row)[kPrTiles], int kvh, KeyTiles& t) {
   const int g4 = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int j = 0; j < kPrTiles; ++j) {
-    const uint4* const at = a.k_pool + ((size_t)row[j] * HKV + kvh) * (kHeadDim / 8) + g4;
+    const uint4* const at = a.k_pool + ((size_t)min(row[j], a.pool_rows - 1) * HKV + kvh) * (kHeadDim / 8) + g4;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) t.k[j][ks] = at[4 * ks];
   }
 }
-__device__ __forceinline__ void step_rows(const uint32_t* rows, int step, uint32_t (&row)[kPrTiles]) {
-  const int first = step * kPrTokens + ((int)threadIdx.x >> 6) * (16 * kPrTiles) + (int)(threadIdx.x & 15);
+template <int HKV>
+__device__ __forceinline__ void step_rows(const PromptScoreArgs& a, const PromptBlock& pb, int step, uint32_t (&row)[kPrTiles]) {
 #pragma unroll
-  for (int j = 0; j < kPrTiles; ++j) row[j] = rows[first + 16 * j];
+  for (int j = 0; j < kPrTiles; ++j)
+    row[j] = (uint32_t)a.table[a.n_init + min(pb.token0 + step * PromptSplit<HKV>::kTokens + 16 * j, pb.most - 1)];
 }
 // s[j][r]: the score of token 16 j + l % 16 and head 4 nb + r of chunk l / 16.
-__device__ __forceinline__ void score_tiles(const uint4* queries, int at, const KeyTiles& t, pr_f32x4 (&s)[kPrTiles]) {
+__device__ __forceinline__ void score_tiles(const uint4 (&queries)[4], const KeyTiles& t, pr_f32x4 (&s)[kPrTiles]) {
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
-    const pr_bf16x8 q = __builtin_bit_cast(pr_bf16x8, queries[(at * 4 + ks) * 64 + (threadIdx.x & 63)]);
+    const pr_bf16x8 q = __builtin_bit_cast(pr_bf16x8, queries[ks]);
 #pragma unroll
     for (int j = 0; j < kPrTiles; ++j) {
       const pr_f32x4 c = ks == 0 ? pr_f32x4{0.f, 0.f, 0.f, 0.f} : s[j];
@@ -135,189 +165,219 @@ __device__ __forceinline__ void score_tiles(const uint4* queries, int at, const 
   }
 }
 
-template <int HKV, int NB>
-constexpr size_t prompt_query_bytes() { return (size_t)HKV * NB * 4 * 64 * 16; }
+// body(step, x, keys) for every step and every KV head x of the wavefront's, the next turn's keys and
+// the table's entries for those of the step after under way.  The entries are asked for before the
+// keys: they are waited for first.  No load is behind a branch within the loops, or the compiler would wait
+// for all loads where the paths meet.
+template <int HKV, typename Body>
+__device__ __forceinline__ void walk_keys(const PromptScoreArgs& a, const PromptBlock& pb, Body body) {
+  constexpr int kHeads = PromptSplit<HKV>::kHeads;
+  static_assert(kHeads == 1 || kHeads == 2, "the turns alternate between two sets of registers");
+  constexpr std::integral_constant<int, 0> head0{};
+  uint32_t row[kPrTiles], ahead[kPrTiles];
+  KeyTiles even, odd;
+  step_rows<HKV>(a, pb, 0, row);
+  step_rows<HKV>(a, pb, 1, ahead);
+  load_keys<HKV>(a, row, pb.kvh0, even);
+  auto next_step = [&](int step, KeyTiles& keys) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kPrTiles; ++j) row[j] = ahead[j];
+    step_rows<HKV>(a, pb, step + 1, ahead);
+    load_keys<HKV>(a, row, pb.kvh0, keys);
+  };
+  int step = 0;
+  if constexpr (kHeads == 2) {
+    constexpr std::integral_constant<int, 1> head1{};
+    for (; step + 1 < pb.steps; ++step) {
+      load_keys<HKV>(a, row, pb.kvh0 + 1, odd);
+      body(step, head0, even);
+      next_step(step + 1, even);
+      body(step, head1, odd);
+    }
+    load_keys<HKV>(a, row, pb.kvh0 + 1, odd);
+    body(step, head0, even);
+    body(step, head1, odd);
+  } else {
+    for (; step + 2 < pb.steps; step += 2) {
+      next_step(step + 1, odd);
+      body(step, head0, even);
+      next_step(step + 2, even);
+      body(step + 1, head0, odd);
+    }
+    if (step + 1 < pb.steps) {
+      next_step(step + 1, odd);
+      body(step, head0, even);
+      body(step + 1, head0, odd);
+    } else {
+      body(step, head0, even);
+    }
+  }
+}
 
-// Per (chunk, head) and block of tokens: the largest score and the sum of the exponentials.
+// Per (chunk, head), block of tokens and token group: the largest score and the sum of the exponentials.
 template <int HKV, int NB>
-__global__ __launch_bounds__(kPrThreads, 2) void prompt_stats_kernel(PromptScoreArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char pr_lds[];
-  uint4* const queries = (uint4*)pr_lds;
-  float2* const stats = (float2*)(pr_lds + prompt_query_bytes<HKV, NB>());  // [wavefront][KV head, nb][16]
-  uint32_t* const rows = (uint32_t*)(stats + 4 * HKV * NB * 16);
+__global__ __launch_bounds__(kPrThreads, HKV * NB > 8 ? 1 : 2) void prompt_stats_kernel(PromptScoreArgs a) {
+  using Split = PromptSplit<HKV>;
   // (the launch before this one has stored the rows; nobody reads the length from here on)
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.seq_len = a.lens[a.chunks - 1];
   PromptBlock pb;
-  if (!prompt_block(a, pb, rows)) return;
-  stage_queries<HKV, NB>(a, pb.set, queries);
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = a.num_heads / HKV;
-  const int token0 = pb.base + wave * (16 * kPrTiles) + (lane & 15);
-  uint32_t row[kPrTiles];
-  KeyTiles now, next;
-  step_rows(rows, 0, row);
-  load_keys<HKV>(a, row, 0, now);
-  for (int kvh = 0; kvh < HKV; ++kvh) {
-    float m[NB][4], l[NB][4];
+  if (!prompt_block<HKV>(a, pb)) return;
+  PromptQueries<HKV, NB> queries;
+  load_queries<HKV, NB>(a, pb, queries);
+  float m[Split::kHeads][NB][4], l[Split::kHeads][NB][4];
+#pragma unroll
+  for (int x = 0; x < Split::kHeads; ++x)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        m[nb][r] = kNegBig;
-        l[nb][r] = 0.f;
+        m[x][nb][r] = kNegBig;
+        l[x][nb][r] = 0.f;
       }
-    for (int step = 0; step < pb.steps; ++step) {
-      const bool last = step + 1 == pb.steps;
-      if (!last || kvh + 1 < HKV) {
-        step_rows(rows, last ? 0 : step + 1, row);
-        load_keys<HKV>(a, row, last ? kvh + 1 : kvh, next);
-      }
+  walk_keys<HKV>(a, pb, [&](int step, auto which, const KeyTiles& keys) __attribute__((always_inline)) {
+    constexpr int x = decltype(which)::value;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        pr_f32x4 s[kPrTiles];
-        score_tiles(queries, kvh * NB + nb, now, s);
+    for (int nb = 0; nb < NB; ++nb) {
+      pr_f32x4 s[kPrTiles];
+      score_tiles(queries.q[x][nb], keys, s);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float top = m[nb][r];
+      for (int r = 0; r < 4; ++r) {
+        float top = m[x][nb][r];
 #pragma unroll
-          for (int j = 0; j < kPrTiles; ++j) {
-            s[j][r] = token0 + step * kPrTokens + 16 * j < pb.n ? s[j][r] : -INFINITY;
-            top = fmaxf(top, s[j][r]);
-          }
-          float sum = l[nb][r] * __expf(m[nb][r] - top);
-#pragma unroll
-          for (int j = 0; j < kPrTiles; ++j) sum += __expf(s[j][r] - top);
-          m[nb][r] = top;
-          l[nb][r] = sum;
+        for (int j = 0; j < kPrTiles; ++j) {
+          s[j][r] = pb.token0 + step * Split::kTokens + 16 * j < pb.n ? s[j][r] : -INFINITY;
+          top = fmaxf(top, s[j][r]);
         }
+        float sum = l[x][nb][r] * __expf(m[x][nb][r] - top);
+#pragma unroll
+        for (int j = 0; j < kPrTiles; ++j) sum += __expf(s[j][r] - top);
+        m[x][nb][r] = top;
+        l[x][nb][r] = sum;
       }
-      now = next;
     }
+  });
+  const int lane = threadIdx.x & 63, G = a.num_heads / HKV;
+#pragma unroll
+  for (int x = 0; x < Split::kHeads; ++x)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        row16_softmax_merge(m[nb][r], l[nb][r]);
-        if ((lane & 15) == 0) stats[(wave * HKV * NB + kvh * NB + nb) * 16 + 4 * (lane >> 4) + r] = make_float2(m[nb][r], l[nb][r]);
+        row16_softmax_merge(m[x][nb][r], l[x][nb][r]);
+        const int g = 4 * nb + r;
+        if ((lane & 15) == 0 && pb.chunk < a.chunks && g < G)
+          a.partials[(((size_t)pb.chunk * a.num_heads + (pb.kvh0 + x) * G + g) * a.blocks + pb.block) * Split::kTokenGroups +
+                     pb.token_group] = make_float2(m[x][nb][r], l[x][nb][r]);
       }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < HKV * NB * 16; i += kPrThreads) {
-    const int chunk = pb.set * kPrChunks + ((i & 15) >> 2), nb = (i >> 4) % NB, kvh = (i >> 4) / NB, g = 4 * nb + (i & 3);
-    if (chunk >= a.chunks || g >= G) continue;
-    float mm = kNegBig, ll = 0.f;
+}
+
+// The blocks' statistics merged, a wavefront a (chunk, head).
+__global__ __launch_bounds__(kPrThreads) void prompt_merge_kernel(PromptScoreArgs a, int token_groups) {
+  const int i = (int)blockIdx.x * kPrWaves + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= a.chunks * a.num_heads) return;
+  const int n = candidates(a, i / a.num_heads);
+  const int entries = (n + a.tokens_per_block - 1) / a.tokens_per_block * token_groups;
+  const float2* const from = a.partials + (size_t)i * a.blocks * token_groups;
+  float m = kNegBig, l = 0.f;
+  for (int at = lane; at < entries; at += 4 * 64) {
+    float2 p[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float2 p = stats[w * HKV * NB * 16 + i];
-      softmax_merge(mm, ll, p.x, p.y);
-    }
-    a.partials[((size_t)chunk * a.num_heads + kvh * G + g) * a.blocks + pb.base / a.tokens_per_block] = make_float2(mm, ll);
+    for (int x = 0; x < 4; ++x) p[x] = at + 64 * x < entries ? from[at + 64 * x] : make_float2(kNegBig, 0.f);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) softmax_merge(m, l, p[x].x, p[x].y);
   }
+  row16_softmax_merge(m, l);
+  softmax_merge(m, l, __shfl_xor(m, 16), __shfl_xor(l, 16));
+  softmax_merge(m, l, __shfl_xor(m, 32), __shfl_xor(l, 32));
+  if (lane == 0) a.stats[i] = n > 0 ? make_float2(m, 1.0f / l) : make_float2(0.f, 0.f);
 }
 
 // The votes of a block of tokens for a set of chunks, and their share of the top-k's first histogram.
 template <int HKV, int NB>
-__global__ __launch_bounds__(kPrThreads, 2) void prompt_votes_kernel(PromptScoreArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char pr_lds[];
-  uint4* const queries = (uint4*)pr_lds;
-  float2* const stats = (float2*)(pr_lds + prompt_query_bytes<HKV, NB>());  // [KV head, nb][16]: maximum, 1 / sum
-  uint32_t* const hist = (uint32_t*)(stats + HKV * NB * 16);                // [chunk][bin]
-  uint32_t* const rows = hist + (a.hist_ws ? kPrChunks * kTopkBins : 0);
+__global__ __launch_bounds__(kPrThreads, HKV * NB > 8 ? 1 : 2) void prompt_votes_kernel(PromptScoreArgs a) {
+  using Split = PromptSplit<HKV>;
+  constexpr int kTileWords = 80;  // (64, and 16 more: the readers' tiles start in different banks)
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kPrChunks * kTopkBins];
+  __shared__ float shares[2][kPrWaves][kPrTiles * kTileWords];  // of a step's votes: [wavefront][tile][lane]
   PromptBlock pb;
-  if (!prompt_block(a, pb, rows)) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = a.num_heads / HKV;
-  stage_queries<HKV, NB>(a, pb.set, queries);
+  if (!prompt_block<HKV>(a, pb)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = a.num_heads / HKV;
+  PromptQueries<HKV, NB> queries;
+  load_queries<HKV, NB>(a, pb, queries);
+  float2 st[Split::kHeads][NB][4];
+#pragma unroll
+  for (int x = 0; x < Split::kHeads; ++x)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int g = 4 * nb + r;
+        // (a row without a head: its scores are zero, and so is its share of the vote)
+        st[x][nb][r] = pb.chunk < a.chunks && g < G
+                           ? a.stats[(size_t)pb.chunk * a.num_heads + (pb.kvh0 + x) * G + g] : make_float2(0.f, 0.f);
+      }
   if (a.hist_ws)
-    for (int i = threadIdx.x; i < kPrChunks * kTopkBins; i += kPrThreads) hist[i] = 0u;
-  __syncthreads();
-  uint32_t row[kPrTiles];
-  KeyTiles now, next;
-  step_rows(rows, 0, row);
-  load_keys<HKV>(a, row, 0, now);
-  // The statistics of the set's chunks and heads, a wavefront a row at a time, a lane a block.
-  for (int i0 = wave; i0 < HKV * NB * 16; i0 += 4 * 4) {
-    float2 p[4][2];
-    int blocks[4];
-    size_t at[4];
+    for (int i = tid; i < kPrChunks * kTopkBins / 4; i += kPrThreads) ((uint4*)hist)[i] = make_uint4(0u, 0u, 0u, 0u);
+  // Of the step's sums this wavefront adds up those of its chunk of the set, a lane a token.
+  const int mine = pb.set * kPrChunks + wave, n_mine = candidates(a, mine);
+  float vote[kPrTiles];
+  walk_keys<HKV>(a, pb, [&](int step, auto which, const KeyTiles& keys) __attribute__((always_inline)) {
+    constexpr int x = decltype(which)::value;
+    if (x == 0)
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int i = i0 + 4 * x;
-      const int chunk = pb.set * kPrChunks + ((i & 15) >> 2), nb = (i >> 4) % NB, kvh = (i >> 4) / NB, g = 4 * nb + (i & 3);
-      const bool there = i < HKV * NB * 16 && chunk < a.chunks && g < G;
-      blocks[x] = there ? (candidates(a, chunk) + a.tokens_per_block - 1) / a.tokens_per_block : 0;
-      at[x] = there ? ((size_t)chunk * a.num_heads + kvh * G + g) * a.blocks : 0;
+      for (int j = 0; j < kPrTiles; ++j) vote[j] = 0.f;
 #pragma unroll
-      for (int y = 0; y < 2; ++y)
-        p[x][y] = lane + 64 * y < blocks[x] ? a.partials[at[x] + lane + 64 * y] : make_float2(kNegBig, 0.f);
+    for (int nb = 0; nb < NB; ++nb) {
+      pr_f32x4 s[kPrTiles];
+      score_tiles(queries.q[x][nb], keys, s);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < kPrTiles; ++j) vote[j] += __expf(s[j][r] - st[x][nb][r].x) * st[x][nb][r].y;
     }
+    if (x + 1 < Split::kHeads) return;
+    float* const to = shares[step & 1][wave];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      float m = p[x][0].x, l = p[x][0].y;
-      softmax_merge(m, l, p[x][1].x, p[x][1].y);
-      for (int y = lane + 128; y < blocks[x]; y += 64) {
-        const float2 more = a.partials[at[x] + y];
-        softmax_merge(m, l, more.x, more.y);
-      }
-      row16_softmax_merge(m, l);
-      softmax_merge(m, l, __shfl_xor(m, 16), __shfl_xor(l, 16));
-      softmax_merge(m, l, __shfl_xor(m, 32), __shfl_xor(l, 32));
-      const int i = i0 + 4 * x;
-      // (a row without a head: its scores are zero, and so is its share of the vote)
-      if (lane == 0 && i < HKV * NB * 16) stats[i] = blocks[x] > 0 ? make_float2(m, 1.0f / l) : make_float2(0.f, 0.f);
-    }
-  }
-  __syncthreads();
-  const int chunk = pb.set * kPrChunks + (lane >> 4);
-  for (int step = 0; step < pb.steps; ++step) {
-    float vote[kPrTiles];
+    for (int j = 0; j < kPrTiles; ++j) to[j * kTileWords + lane] = vote[j];
+    // One meeting a step: who writes these shares again, two steps on, has met those who read them one step on.
+    // (The histogram is cleared before the first.)
+    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kPrTiles; ++j) vote[j] = 0.f;
-    for (int kvh = 0; kvh < HKV; ++kvh) {
-      const bool last = kvh + 1 == HKV;
-      if (!last || step + 1 < pb.steps) {
-        if (last) step_rows(rows, step + 1, row);
-        load_keys<HKV>(a, row, last ? 0 : kvh + 1, next);
-      }
+    for (int tg = 0; tg < Split::kTokenGroups; ++tg) {
+      float sum = 0.f;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        pr_f32x4 s[kPrTiles];
-        score_tiles(queries, kvh * NB + nb, now, s);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float2 st = stats[(kvh * NB + nb) * 16 + 4 * (lane >> 4) + r];
-#pragma unroll
-          for (int j = 0; j < kPrTiles; ++j) vote[j] += __expf(s[j][r] - st.x) * st.y;
-        }
-      }
-      now = next;
-    }
-#pragma unroll
-    for (int j = 0; j < kPrTiles; ++j) {
-      const int t = pb.base + step * kPrTokens + wave * (16 * kPrTiles) + 16 * j + (lane & 15);
-      if (t < pb.n) {
-        a.votes[(size_t)chunk * a.vote_stride + t] = vote[j];
-        if (a.hist_ws) atomicAdd(&hist[(lane >> 4) * kTopkBins + key_bin0(vote_key(vote[j]))], 1u);
+      for (int hg = 0; hg < Split::kHeadGroups; ++hg)
+        sum += shares[step & 1][tg * Split::kHeadGroups + hg][(lane >> 4) * kTileWords + 16 * wave + (lane & 15)];
+      const int t = pb.base + step * Split::kTokens + 64 * tg + lane;
+      if (t < n_mine) {
+        a.votes[(size_t)mine * a.vote_stride + t] = sum;
+        if (a.hist_ws) atomicAdd(&hist[wave * kTopkBins + key_bin0(vote_key(sum))], 1u);
       }
     }
-  }
+  });
   if (!a.hist_ws) return;
-  __syncthreads();
-  for (int i = threadIdx.x; i < kPrChunks * kTopkBins; i += kPrThreads)
-    if (hist[i])  // (of a chunk that is there: others count nothing)
-      atomicAdd(&topk_ws(a.hist_ws, a.hist_ws_stride, pb.set * kPrChunks + i / kTopkBins)[kTopkHist0 + i % kTopkBins], hist[i]);
+  // (each wavefront has counted its chunk's on its own)
+  uint32_t* const counts = topk_ws(a.hist_ws, a.hist_ws_stride, mine) + kTopkHist0;
+  for (int i = 4 * lane; i < kTopkBins; i += 4 * 64) {
+    const uint4 c = *(const uint4*)(hist + wave * kTopkBins + i);
+    // (of a chunk that is there: others count nothing)
+    if (c.x) atomicAdd(&counts[i], c.x);
+    if (c.y) atomicAdd(&counts[i + 1], c.y);
+    if (c.z) atomicAdd(&counts[i + 2], c.z);
+    if (c.w) atomicAdd(&counts[i + 3], c.w);
+  }
 }
 
 // --------------------------------------------------------------------------------- host
 // Chunks that one round of launches takes, at most: the launches' fixed cost is shared by then, and the
 // staged keys and values of a round (11 MB a chunk at 8 KV heads) stay below the last-level cache.
 constexpr int kPrGroup = 20;
-// Blocks of tokens: enough for two workgroups per CU, few enough for their statistics to be merged by
-// every workgroup of the votes on its own (128 of four chunks' 28 heads: 110 KB from L2, 1 us).
-constexpr int kPrBlocks = 128;
+// Workgroups of the scores' launches: two per CU, as many as run at once.
+constexpr int kPrWorkgroups = 512;
 
 // Workspace of a round, carved in this order (256-byte aligned pieces).
 struct PromptWorkspace {
-  size_t qf, lens, sel, sel_pos, sel_len, votes, pooled, partials, topk, stage, total;
+  size_t qf, lens, sel, sel_pos, sel_len, votes, pooled, partials, stats, topk, stage, total;
   int64_t vote_stride;
   int max_sel, blocks, tokens_per_block;
 };
@@ -334,7 +394,9 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
   const int max_n = std::max(max_seq_len - cfg->n_init - cfg->n_local, 1);
   w.vote_stride = ts_score_stride(max_n);
   w.max_sel = cfg->n_init + cfg->top_k + cfg->n_local;
-  w.tokens_per_block = (int)ceil_div(max_n, (int64_t)kPrBlocks * kPrTokens) * kPrTokens;
+  const int token_groups = prompt_token_groups(cfg->num_kv_heads), step = token_groups * kPrTiles * 16;
+  const int64_t sets = ceil_div(chunks, kPrChunks);
+  w.tokens_per_block = (int)ceil_div(max_n, ceil_div(kPrWorkgroups, sets) * step) * step;
   w.blocks = (int)ceil_div(max_n, w.tokens_per_block);
   w.qf = take(C * H * kHeadDim * 2);
   w.lens = take(C * 4);
@@ -343,7 +405,9 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
   w.sel_len = take(C * 4);
   w.votes = take(C * w.vote_stride * 4);
   w.pooled = take(cfg->pool_kernel > 0 ? C * w.vote_stride * 4 : 0);
-  w.partials = take(C * H * kPrBlocks * sizeof(float2));  // (fewer tokens can be more blocks)
+  // (as much for any round: at most ceil(workgroups / sets) blocks of at most 4 sets chunks)
+  w.partials = take((size_t)(kPrWorkgroups + ceil_div(kPrGroup, kPrChunks)) * kPrChunks * H * token_groups * sizeof(float2));
+  w.stats = take(C * H * sizeof(float2));
   w.topk = take(ts_topk_workspace_bytes(cfg, chunks, max_seq_len));
   w.stage = take(C * ts_prefill_attn_workspace_bytes(cfg, w.max_sel));
   w.total = off;
@@ -352,21 +416,13 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
 
 template <int HKV, int NB>
 static int launch_prompt_scores(const PromptScoreArgs& a, hipStream_t stream) {
-  const size_t queries = prompt_query_bytes<HKV, NB>(), rows = (size_t)a.tokens_per_block * 4;
-  const size_t stats_lds = queries + 4 * HKV * NB * 16 * sizeof(float2) + rows;
-  const size_t votes_lds = queries + HKV * NB * 16 * sizeof(float2) + (a.hist_ws ? kPrChunks * kTopkBins * 4 : 0) + rows;
-  // (2^20 candidates in kPrBlocks blocks: 32 KB of rows, and at most 104 KB of the others)
-  constexpr int kMostLds = 160 * 1024;
-  static const hipError_t ok1 = hipFuncSetAttribute((const void*)prompt_stats_kernel<HKV, NB>,
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMostLds);
-  static const hipError_t ok2 = hipFuncSetAttribute((const void*)prompt_votes_kernel<HKV, NB>,
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMostLds);
-  if (ok1 != hipSuccess || ok2 != hipSuccess || stats_lds > kMostLds || votes_lds > kMostLds)
-    return fail(TS_EHIP, "prompt scores: %zu and %zu bytes of LDS refused", stats_lds, votes_lds);
   const dim3 grid((unsigned)(ceil_div(a.blocks, 8) * 8 * a.sets));
-  hipLaunchKernelGGL((prompt_stats_kernel<HKV, NB>), grid, dim3(kPrThreads), stats_lds, stream, a);
+  hipLaunchKernelGGL((prompt_stats_kernel<HKV, NB>), grid, dim3(kPrThreads), 0, stream, a);
   TS_TRY(check_launch("prompt_stats_kernel"));
-  hipLaunchKernelGGL((prompt_votes_kernel<HKV, NB>), grid, dim3(kPrThreads), votes_lds, stream, a);
+  hipLaunchKernelGGL(prompt_merge_kernel, dim3((unsigned)ceil_div(a.chunks * a.num_heads, kPrWaves)), dim3(kPrThreads), 0,
+                     stream, a, PromptSplit<HKV>::kTokenGroups);
+  TS_TRY(check_launch("prompt_merge_kernel"));
+  hipLaunchKernelGGL((prompt_votes_kernel<HKV, NB>), grid, dim3(kPrThreads), 0, stream, a);
   return check_launch("prompt_votes_kernel");
 }
 
@@ -466,7 +522,6 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     a.k_pool = (const uint4*)k_pool;
     a.pool_rows = (uint32_t)pool_rows;
     a.table = table;
-    a.page_size = 1;
     a.lens = lens;
     a.chunks = here;
     a.sets = (int)ceil_div(here, kPrChunks);
@@ -479,6 +534,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     a.blocks = w.blocks;
     a.tokens_per_block = w.tokens_per_block;
     a.partials = (float2*)(ws + w.partials);
+    a.stats = (float2*)(ws + w.stats);
     a.seq_len = seq_len;
     a.votes = votes;
     a.vote_stride = w.vote_stride;
