@@ -537,7 +537,8 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
                             size_t workspace_bytes, ts_stream_t stream);
 
 /* The chunks of a prompt part together: what ts_prefill_step_strided does for chunk after chunk of
- * chunk_rows rows (the last one of what is left), in rounds of up to 20 chunks: all rows of a round
+ * chunk_rows rows (the last one of what is left). The first chunks, as far as max_seq_len says that they attend
+ * to all tokens, are one; the others follow in rounds of up to 20: all rows of a round
  * are stored first, then its chunks select, each from the context up to its own last row, and attend.
  * Results are those of the chunks one by one (their votes are added up in another order), where the
  * slots of the whole part are all different and none of them is listed in the context before it.

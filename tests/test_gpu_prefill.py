@@ -504,6 +504,49 @@ def test_scores_of_a_prompts_chunks_by_steps(dev, heads, kv_heads, steps, odd):
         assert torch.equal(x, y), f"{name}: {int((x != y).sum())} of {x.numel()} differ"
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(8, 1), (28, 4), (64, 8)])
+@pytest.mark.parametrize("L0,T,chunk,bound", [(0, 168, 16, 0), (0, 169, 16, 0), (0, 168, 24, 0), (3, 170, 33, 0),
+                                              (150, 19, 18, 0), (150, 40, 19, 0), (167, 5, 1, 0), (0, 100, 32, 500),
+                                              (5, 1283, 96, 0)])
+def test_first_chunks_of_a_prompt_are_one(dev, heads, kv_heads, L0, T, chunk, bound):
+    """Dense chunks together against one by one: all of them, all but the last, exactly as many tokens as are
+    attended to and one more, none, a bound above the length, and enough columns for the wide workgroups.
+    Pools, table and length the same; outputs are sums in fp32 of weights rounded to bf16, by one kernel or
+    another: 2^-8 of a weighted mean of normal values, and a rounding of the result on each side."""
+    top_k = 1224 if T > 1000 else 96
+    say(f"dense prompt H={heads} kv={kv_heads} L0={L0} T={T} chunk={chunk} bound={bound}")
+    shape = dict(SHAPES[0], num_heads=heads, num_kv_heads=kv_heads)
+    wl = workloads.build("pd", shape, [max(L0, 1)], [top_k], 1, dev, seed=41, n_init=8, n_local=64, top_k=top_k,
+                         extra_pages=T)
+    c = wl.cfg
+    g = torch.Generator(device=dev).manual_seed(42)
+    q = torch.randn((T, c.num_heads * 128), generator=g, device=dev).bfloat16()
+    k_new, v_new = torch.randn((2, T, c.num_kv_heads, 128), generator=g, device=dev).bfloat16()
+    slots = wl.free_pages[:T].contiguous()
+    results = []
+    for together in (True, False):
+        k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
+        table = torch.zeros((1, max(L0 + T, bound)), dtype=torch.int32, device=dev)
+        table[0, :L0] = wl.table[0, :L0]
+        seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
+        out = torch.empty_like(q)
+        layer = ops.PrefillChunk(c, table.shape[1], dev, max_rows=chunk)
+        if together:
+            layer._prompt(q, k_new, v_new, slots, k_pool, v_pool, ops.Batch(seq, table, max(L0 + T, bound)), out, 0, T, chunk)
+        else:
+            for start in range(0, T, chunk):
+                end = min(start + chunk, T)
+                layer._serve(q, k_new, v_new, slots, k_pool, v_pool, ops.Batch(seq, table, L0 + end), None, out,
+                             start, end - start)
+        torch.cuda.synchronize()
+        assert not layer.gave_up()
+        results.append((k_pool, v_pool, table[:, :L0 + T], seq, out.float()))
+    for name, x, y in list(zip(("k", "v", "table", "length"), *results))[:4]:
+        assert torch.equal(x, y), f"{name}: {int((x != y).sum())} of {x.numel()} differ"
+    x, y = results[0][4], results[1][4]
+    assert (x - y).abs().max().item() <= 2 ** -7 * y.abs().max().item()
+
+
 def test_prefill_short_context_attends_densely(dev):
     """n_init + k + n_local >= L: the chunk attends over every token so far (tr.py:741-744)."""
     say("prefill chunk, dense context")

@@ -815,13 +815,13 @@ int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride,
 // their last wave is at least 0.8 full, else as many as fill whole waves (20 chunks of 512 rows, 28 heads on 4,
 // are 1120: 18 of them four waves less 16, 300 us, and two chunks 52).  The rows of a long dense chunk
 // see fewer keys the earlier they are, and the early ones fill the last wave up: 115 us instead of 161 with
-// 1.5 waves, 159 instead of 192 with two, 107 instead of 77 with 0.75.
+// 1.5 waves, 159 instead of 192 with two, 107 instead of 77 with 0.75; 2560 rows that are all there is, 79 instead of 88 with 1.1.
 static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_rows) {
   const int64_t each = prefill_shared_workgroups(num_heads, num_kv_heads, chunk_rows), chunks = ceil_div(rows, chunk_rows);
   // (small chunks would leave most of a workgroup without columns)
   if (4 * chunk_rows * (int64_t)num_heads < 3 * each * 256) return 0;
   const int64_t full = each * chunks / 256, rest = each * chunks - full * 256;
-  if (rest >= 205 || rest == 0 || (chunks == 1 && each >= 320)) return (int)chunks;
+  if (rest >= 205 || rest == 0 || (chunks == 1 && each >= 256)) return (int)chunks;
   return (int)(full * 256 / each);
 }
 

@@ -1,5 +1,6 @@
 // Several chunks of a prompt at once (patched_radix_attention_extend_forward_flashinfer,
-// tr.py:716-773, which takes them one after the other).
+// tr.py:716-773, which takes them one after the other).  The first of them, which attend to all tokens so far,
+// are one long chunk; what follows is about the others.
 //
 // What a chunk selects from is the context before it and its own rows, and what it attends to are
 // rows of that: once all rows are stored no chunk needs another one's result.  A chunk on its own
@@ -19,7 +20,7 @@
 // are the cost (the single launch streams them once and holds the scores in LDS), for four chunks
 // that a workgroup serves together they are read for all of them, and 16 query rows fill the
 // matrix instruction's tile.  A prompt of 31599 tokens with 16 more, 28 heads on 4, its chunks one after
-// the other and together: 4140 and 2075 us; three of 700 to 5200 tokens, 32 heads on 8, two layers: 2340 and 1920.
+// the other and together: 4271 and 2143 us; three of 700 to 5200 tokens, 32 heads on 8, two layers: 2423 and 1789.
 #include <algorithm>
 #include <type_traits>
 
@@ -484,17 +485,51 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   const hipStream_t st = (hipStream_t)stream;
   const int q_stride = q_row_stride ? q_row_stride : cfg->num_heads * cfg->head_dim;
   const int kv_stride = kv_row_stride ? kv_row_stride : cfg->num_kv_heads * cfg->head_dim;
-  const int group = (int)ceil_div(chunks, ceil_div(chunks, kPrGroup));  // (rounds of about the same size)
-  for (int first = 0; first < chunks; first += group) {
+  char* const ws = (char*)workspace;
+  const auto rows_at = [&](int64_t row0, int32_t n_rows) {
+    return chunk_store(cfg, (const uint16_t*)kv->k + row0 * kv_stride, (const uint16_t*)kv->v + row0 * kv_stride,
+                       kv_row_stride, kv->out_cache_loc + row0, n_rows, k_pool, v_pool, pool_rows, table, seq_len,
+                       kv->max_tokens);
+  };
+  // Bounds the length after the first `done` rows: what follows them is not there yet (unless the table
+  // gets full, and rows are dropped).
+  const auto bound_after = [&](int64_t done) {
+    const int64_t later = bt->max_seq_len < kv->max_tokens ? rows - done : 0;
+    return (int32_t)std::max<int64_t>(bt->max_seq_len - later, 1);
+  };
+
+  // The first chunks, which attend to everything before them, are one: a row's keys are the same wherever its
+  // chunk ends.  Five chunks of 512, 32 heads on 8: five times a gather (5 to 8 us) and an attention (12 to 23),
+  // each with the device half idle at its end, and together 9 and 79 us.  Three prompts of 700 to 5200
+  // tokens, two layers, in the same run as the code that takes every chunk on its own: 1915 of 2351 us, and 1789 of
+  // 2423 with this; a prompt of 31599, 28 heads on 4: 2108 of 4179, 2143 of 4271.
+  int dense = 0;
+  while (dense < chunks && bound_after(std::min<int64_t>((dense + 1LL) * chunk_rows, rows)) <=
+                               (int64_t)cfg->n_init + cfg->top_k + cfg->n_local)
+    ++dense;
+  if (dense > 0) {
+    const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)dense * chunk_rows, rows), bound = bound_after(n_rows);
+    const PromptWorkspace w = prompt_workspace(cfg, 1, bound);
+    PrefillDense all{};
+    all.table = table;
+    all.seq_len = seq_len;
+    all.sel = (int32_t*)(ws + w.sel);
+    all.sel_pos = (int32_t*)(ws + w.sel_pos);
+    all.sel_len = (int32_t*)(ws + w.sel_len);
+    all.list_bound = std::min(bound, kv->max_tokens);
+    all.store = rows_at(0, n_rows);
+    TS_TRY(launch_prefill_attn(cfg, q, q_stride, n_rows, k_pool, v_pool, pool_rows, all.sel, all.sel_len, bound, out,
+                               ws + w.stage, w.total - w.stage, st, &all));
+    if (dense == chunks) return TS_OK;
+  }
+
+  const int rest = chunks - dense, group = (int)ceil_div(rest, ceil_div(rest, kPrGroup));  // (rounds of about the same size)
+  for (int first = dense; first < chunks; first += group) {
     const int here = std::min(group, chunks - first);
     const int64_t row0 = (int64_t)first * chunk_rows;
     const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)here * chunk_rows, rows - row0);
-    // Bounds every length of the round: what follows it is not there yet (unless the table gets full,
-    // and rows are dropped).
-    const int64_t later = bt->max_seq_len < kv->max_tokens ? rows - row0 - n_rows : 0;
-    const int32_t bound = (int32_t)std::max<int64_t>(bt->max_seq_len - later, 1);
+    const int32_t bound = bound_after(row0 + n_rows);
     const PromptWorkspace w = prompt_workspace(cfg, here, bound);
-    char* const ws = (char*)workspace;
     int32_t *const lens = (int32_t*)(ws + w.lens), *const sel = (int32_t*)(ws + w.sel),
                    *const sel_len = (int32_t*)(ws + w.sel_len);
     float *const votes = (float*)(ws + w.votes), *const pooled = cfg->pool_kernel > 0 ? (float*)(ws + w.pooled) : nullptr;
@@ -511,11 +546,8 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     if (first + here == chunks) topk.hint = bt->threshold_hint;
     const ZeroRegion counters = topk_zero_region(topk, here);
     const PromptChunks pc{n_rows, chunk_rows, here, lens, counters.base, (size_t)counters.stride, counters.words};
-    const ChunkStore cs = chunk_store(cfg, (const uint16_t*)kv->k + row0 * kv_stride,
-                                      (const uint16_t*)kv->v + row0 * kv_stride, kv_row_stride,
-                                      kv->out_cache_loc + row0, n_rows, k_pool, v_pool, pool_rows, table, seq_len,
-                                      kv->max_tokens);
-    TS_TRY(launch_prompt_fingerprint(cfg, q0, q_stride, cos_table, sin_table, table_rows, ws + w.qf, pc, cs, st));
+    TS_TRY(launch_prompt_fingerprint(cfg, q0, q_stride, cos_table, sin_table, table_rows, ws + w.qf, pc,
+                                     rows_at(row0, n_rows), st));
 
     PromptScoreArgs a{};
     a.qf = (const uint16_t*)(ws + w.qf);

@@ -564,18 +564,16 @@ class TokenRetriever:
         return out
 
     def _together(self, layer_id, rows) -> bool:
-        """Whether the chunks of ``rows`` more tokens all select, and fit the table and what the library
-        ranks (2^20 candidates)."""
+        """Whether the chunks of ``rows`` more tokens fit the table and what the library ranks (2^20
+        candidates)."""
         held = self.num_tokens[layer_id]
-        fixed = max(N_INIT, 0) + max(N_Local, 0)
-        return held + PREFILL_CHUNK_SIZE > fixed + TOP_K and held + rows <= self.max_num_tokens \
-            and held + rows - fixed <= 1 << 20
+        return held + rows <= self.max_num_tokens \
+            and held + rows - max(N_INIT, 0) - max(N_Local, 0) <= 1 << 20
 
     def prefill_step(self, attn, q, k, v, loc, k_buffer, v_buffer, out):
         """The whole prompt part in chunks (tr.py:716-773): each its store, then
-        :meth:`prefill_attention`, the rows of ``out`` written in place.  From the first chunk on that
-        selects they are taken together, if there are several (a part that does not fit the
-        table goes up to where it does not, chunk by chunk)."""
+        :meth:`prefill_attention`, the rows of ``out`` written in place.  Several chunks are taken
+        together (a part that does not fit the table goes up to where it does not, chunk by chunk)."""
         layer_id, rows = attn.layer_id, q.shape[0]
         runner = self._prefill_chunk(attn)
         bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
