@@ -25,12 +25,15 @@ constexpr int kFpInFlight = 4;  // rows per step of a row group
 constexpr int kFpVec = 4;       // rotation pairs per thread
 constexpr int kFpSplit = 4;     // workgroups per head
 constexpr int kFpClear = 16;    // workgroups that clear
+constexpr int kFpHeads = 2;     // heads of a workgroup where chunks are taken together
 constexpr int kFpThreads = kHeadDim / 2 / kFpSplit / kFpVec * kFpRowGroups;
 
-// Workgroup (h, quarter): head h, the quarter's rotation pairs, of one chunk of `rows` rows.
+// Heads [h0, h0 + NH) below `heads`, the quarter's rotation pairs, of one chunk of `rows` rows: the tables' rows are
+// read once for all of them.
+template <int NH>
 __device__ __forceinline__ void fingerprint_quarter(
     const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
-    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int h, int quarter) {
+    const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int rows, int heads, int h0, int quarter) {
 #pragma clang fp contract(off)
   constexpr int half = kHeadDim / 2;
   constexpr int kPairs = half / kFpSplit;   // rotation pairs of this workgroup
@@ -39,11 +42,11 @@ __device__ __forceinline__ void fingerprint_quarter(
                 "a thread per row group and four pairs, and per eight row groups and column");
   const int first_pair = quarter * kPairs;
   const int i = first_pair + (threadIdx.x % kLanes) * kFpVec, rg = threadIdx.x / kLanes;
-  float lo_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f}, hi_sum[kFpVec] = {0.f, 0.f, 0.f, 0.f};
+  float lo_sum[NH][kFpVec] = {}, hi_sum[NH][kFpVec] = {};
   // Four rows per step: their loads are independent and go out together; the sums
   // are still taken in row order.
   for (int r0 = rg; r0 < rows; r0 += kFpInFlight * kFpRowGroups) {
-    uint2 x1[kFpInFlight], x2[kFpInFlight];
+    uint2 x1[NH][kFpInFlight], x2[NH][kFpInFlight];
     float4 c1[kFpInFlight], c2[kFpInFlight], s1[kFpInFlight], s2[kFpInFlight];
 #pragma unroll
     for (int j = 0; j < kFpInFlight; ++j) {
@@ -52,9 +55,12 @@ __device__ __forceinline__ void fingerprint_quarter(
       pos = pos < table_rows ? pos : table_rows - 1;
       const float* c = cos_table + pos * kHeadDim;
       const float* s = sin_table + pos * kHeadDim;
-      const size_t base = (size_t)r * q_stride + h * kHeadDim;
-      x1[j] = *(const uint2*)(q + base + i);
-      x2[j] = *(const uint2*)(q + base + i + half);
+#pragma unroll
+      for (int x = 0; x < NH; ++x) {
+        const size_t base = (size_t)r * q_stride + (NH == 1 ? h0 : min(h0 + x, heads - 1)) * kHeadDim;
+        x1[x][j] = *(const uint2*)(q + base + i);
+        x2[x][j] = *(const uint2*)(q + base + i + half);
+      }
       c1[j] = *(const float4*)(c + i);
       c2[j] = *(const float4*)(c + i + half);
       s1[j] = *(const float4*)(s + i);
@@ -63,49 +69,57 @@ __device__ __forceinline__ void fingerprint_quarter(
 #pragma unroll
     for (int j = 0; j < kFpInFlight; ++j) {
       if (r0 + j * kFpRowGroups < rows) {
-        const float a1[kFpVec] = {bf16_to_f32((uint16_t)x1[j].x), bf16_to_f32((uint16_t)(x1[j].x >> 16)),
-                                  bf16_to_f32((uint16_t)x1[j].y), bf16_to_f32((uint16_t)(x1[j].y >> 16))};
-        const float a2[kFpVec] = {bf16_to_f32((uint16_t)x2[j].x), bf16_to_f32((uint16_t)(x2[j].x >> 16)),
-                                  bf16_to_f32((uint16_t)x2[j].y), bf16_to_f32((uint16_t)(x2[j].y >> 16))};
         const float cc1[kFpVec] = {c1[j].x, c1[j].y, c1[j].z, c1[j].w};
         const float cc2[kFpVec] = {c2[j].x, c2[j].y, c2[j].z, c2[j].w};
         const float ss1[kFpVec] = {s1[j].x, s1[j].y, s1[j].z, s1[j].w};
         const float ss2[kFpVec] = {s2[j].x, s2[j].y, s2[j].z, s2[j].w};
 #pragma unroll
-        for (int e = 0; e < kFpVec; ++e) {
-          const float lo = a1[e] * cc1[e] + (-a2[e]) * ss1[e];
-          const float hi = a2[e] * cc2[e] + a1[e] * ss2[e];
-          lo_sum[e] += bf16_to_f32(f32_to_bf16(lo));
-          hi_sum[e] += bf16_to_f32(f32_to_bf16(hi));
+        for (int x = 0; x < NH; ++x) {
+          const uint2 y1 = x1[x][j], y2 = x2[x][j];
+          const float a1[kFpVec] = {bf16_to_f32((uint16_t)y1.x), bf16_to_f32((uint16_t)(y1.x >> 16)),
+                                    bf16_to_f32((uint16_t)y1.y), bf16_to_f32((uint16_t)(y1.y >> 16))};
+          const float a2[kFpVec] = {bf16_to_f32((uint16_t)y2.x), bf16_to_f32((uint16_t)(y2.x >> 16)),
+                                    bf16_to_f32((uint16_t)y2.y), bf16_to_f32((uint16_t)(y2.y >> 16))};
+#pragma unroll
+          for (int e = 0; e < kFpVec; ++e) {
+            const float lo = a1[e] * cc1[e] + (-a2[e]) * ss1[e];
+            const float hi = a2[e] * cc2[e] + a1[e] * ss2[e];
+            const uint32_t rounded = pack_bf16(lo, hi);  // (a NaN stays one, and is one in the mean)
+            lo_sum[x][e] += bf16_lo(rounded);
+            hi_sum[x][e] += bf16_hi(rounded);
+          }
         }
       }
     }
   }
   // Columns of this workgroup: its kPairs low halves, then its kPairs high halves.
   // The row groups are added in order, eight at a time and then the sixteen eights.
-  __shared__ float part[kFpRowGroups][2 * kPairs];
-  __shared__ float part8[kFpRowGroups / 8][2 * kPairs];
+  // (A head's sums are written again two heads on: by then everybody has read them.)
+  constexpr int kBuffers = NH > 1 ? 2 : 1;
+  __shared__ float part[kBuffers][kFpRowGroups][2 * kPairs];
+  __shared__ float part8[NH][kFpRowGroups / 8][2 * kPairs];
   const int col = i - first_pair;
 #pragma unroll
-  for (int e = 0; e < kFpVec; ++e) {
-    part[rg][col + e] = lo_sum[e];
-    part[rg][col + e + kPairs] = hi_sum[e];
-  }
-  __syncthreads();
-  {
+  for (int x = 0; x < NH; ++x) {
+#pragma unroll
+    for (int e = 0; e < kFpVec; ++e) {
+      part[x % kBuffers][rg][col + e] = lo_sum[x][e];
+      part[x % kBuffers][rg][col + e + kPairs] = hi_sum[x][e];
+    }
+    __syncthreads();
     const int c = threadIdx.x % (2 * kPairs), set = threadIdx.x / (2 * kPairs);
     float sum = 0.f;
 #pragma unroll
-    for (int g = 0; g < 8; ++g) sum += part[set * 8 + g][c];
-    part8[set][c] = sum;
+    for (int g = 0; g < 8; ++g) sum += part[x % kBuffers][set * 8 + g][c];
+    part8[x][set][c] = sum;
   }
   __syncthreads();
-  if (threadIdx.x < 2 * kPairs) {
+  if (threadIdx.x < NH * 2 * kPairs) {
+    const int x = threadIdx.x / (2 * kPairs), c = threadIdx.x % (2 * kPairs);
     float total = 0.f;
-    for (int g = 0; g < kFpRowGroups / 8; ++g) total += part8[g][threadIdx.x];
-    const int c = threadIdx.x;
+    for (int g = 0; g < kFpRowGroups / 8; ++g) total += part8[x][g][c];
     const int dim = c < kPairs ? first_pair + c : half + first_pair + (c - kPairs);
-    qf[(size_t)h * kHeadDim + dim] = f32_to_bf16(total / (float)rows);
+    if (NH == 1 || h0 + x < heads) qf[(size_t)(h0 + x) * kHeadDim + dim] = f32_to_bf16(total / (float)rows);
   }
 }
 
@@ -127,33 +141,43 @@ __global__ __launch_bounds__(kFpThreads) void fingerprint_kernel(
                     kFpClear * (kFpThreads / 64));
     return;
   }
-  fingerprint_quarter(q, q_stride, qf, cos_table, sin_table, table_rows, first_pos, rows, (int)blockIdx.x,
-                      (int)blockIdx.y);
+  fingerprint_quarter<1>(q, q_stride, qf, cos_table, sin_table, table_rows, first_pos, rows, heads, (int)blockIdx.x,
+                         (int)blockIdx.y);
 }
 
-// The same for several chunks of a prompt, chunk blockIdx.z: its fingerprint, the store of its rows
-// (whose positions follow from the length before the first chunk, which the launch after this one
-// advances), the words its selection counts into, and its length.
+// The same for several chunks of a prompt: the store of their rows (whose positions follow from the length before
+// the first chunk, which the launch after this one advances), the words their selections count into and their
+// lengths, by the first workgroups, cs.workgroups + 1 per chunk; then the fingerprints, two heads of a chunk to
+// a workgroup, their quarters eight workgroups apart: on one XCD, whose L2 has the lines of the queries
+// that they share.  With a workgroup per head and quarter the tables were four times the queries, and the two bf16
+// roundings of a pair eleven instructions instead of one: 19 chunks of 28 heads 46.8 -> 38.8 us, 6 of 32 20.8 ->
+// 19.1, 3 of 32 12.5 -> 11.6 (the rows alone, read and stored, are 110 MB of the first: 22 us).  Four heads, whose
+// registers leave one workgroup to a CU, 59.
 __global__ __launch_bounds__(kFpThreads) void prompt_fingerprint_kernel(
     const uint16_t* __restrict__ q, int q_stride, uint16_t* __restrict__ qf, const float* __restrict__ cos_table,
     const float* __restrict__ sin_table, int64_t table_rows, int first_pos, int heads, PromptChunks pc, ChunkStore cs) {
-  const int chunk = blockIdx.z;
-  const int first = chunk * pc.chunk_rows, rows = min(pc.chunk_rows, pc.rows - first);
-  if ((int)blockIdx.y >= kFpSplit) {
-    const int wg = ((int)blockIdx.y - kFpSplit) * (int)gridDim.x + (int)blockIdx.x;
+  const int on_the_side = pc.chunks * (cs.workgroups + 1);
+  if ((int)blockIdx.x < on_the_side) {
+    const int chunk = (int)blockIdx.x / (cs.workgroups + 1), wg = (int)blockIdx.x % (cs.workgroups + 1);
+    const int first = chunk * pc.chunk_rows, rows = min(pc.chunk_rows, pc.rows - first);
     const int len = *cs.seq_len;
     if (wg < cs.workgroups) {
       store_rows_at(cs, len, first + wg * (kFpThreads / kChunkThreadsPerRow) + (int)threadIdx.x / kChunkThreadsPerRow,
                     first + rows);
-    } else if (wg == cs.workgroups) {
+    } else {
       uint32_t* const counters = pc.counters + (size_t)chunk * pc.counters_stride;
       for (int w = threadIdx.x; w < pc.counter_words; w += kFpThreads) counters[w] = 0u;
       if (threadIdx.x == 0) pc.lens[chunk] = min(len + first + rows, cs.max_tokens);
     }
     return;
   }
-  fingerprint_quarter(q + (size_t)first * q_stride, q_stride, qf + (size_t)chunk * heads * kHeadDim, cos_table,
-                      sin_table, table_rows, first_pos, rows, (int)blockIdx.x, (int)blockIdx.y);
+  const int id = (int)blockIdx.x - on_the_side, per_chunk = (heads + kFpHeads - 1) / kFpHeads;
+  const int unit = id / (8 * kFpSplit) * 8 + id % 8, quarter = id / 8 % kFpSplit;
+  if (unit >= pc.chunks * per_chunk) return;
+  const int chunk = unit / per_chunk, first = chunk * pc.chunk_rows;
+  fingerprint_quarter<kFpHeads>(q + (size_t)first * q_stride, q_stride, qf + (size_t)chunk * heads * kHeadDim, cos_table,
+                          sin_table, table_rows, first_pos, min(pc.chunk_rows, pc.rows - first), heads,
+                          unit % per_chunk * kFpHeads, quarter);
 }
 
 // ------------------------------------------------------------ prefill attention
@@ -802,10 +826,10 @@ int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride,
   TS_TRY(check_fingerprint(q, pc.chunk_rows, cos_table, sin_table, table_rows, qf, cfg->n_local));
   ChunkStore cs = store;
   cs.workgroups = (int)ceil_div(pc.chunk_rows, kFpThreads / kChunkThreadsPerRow);
-  const unsigned grid_y = kFpSplit + (unsigned)ceil_div(cs.workgroups + 1, cfg->num_heads);
-  hipLaunchKernelGGL(prompt_fingerprint_kernel, dim3((unsigned)cfg->num_heads, grid_y, (unsigned)pc.chunks),
-                     dim3(kFpThreads), 0, stream, (const uint16_t*)q, q_stride, (uint16_t*)qf, cos_table, sin_table,
-                     table_rows, cfg->n_local, cfg->num_heads, pc, cs);
+  const int64_t units = ceil_div(cfg->num_heads, kFpHeads) * pc.chunks;
+  const dim3 grid((unsigned)(pc.chunks * (int64_t)(cs.workgroups + 1) + ceil_div(units, 8) * 8 * kFpSplit));
+  hipLaunchKernelGGL(prompt_fingerprint_kernel, grid, dim3(kFpThreads), 0, stream, (const uint16_t*)q, q_stride,
+                     (uint16_t*)qf, cos_table, sin_table, table_rows, cfg->n_local, cfg->num_heads, pc, cs);
   return check_launch("prompt_fingerprint_kernel");
 }
 
