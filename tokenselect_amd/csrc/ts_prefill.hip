@@ -257,8 +257,7 @@ __device__ __forceinline__ void stage(const PrefillArgs& a, void* to, const uint
 // chunk's new rows, which is read where the caller has it and stored on the way.  A dense chunk was
 // a store that also wrote the list (4.6 us and a gap), this (5.4) and the attention; this is 6.2 now: three
 // prompts of 700 to 5200 tokens and 8 tokens 2475 -> 2400 us a pass.
-// MANY: chunk blockIdx.y of several.  One chunk leaves out what finds its own, here and in the attention: 512 rows
-// behind 131072 tokens, 32 heads on 8, two layers, 200.7 -> 197.7 us.
+// MANY: chunk blockIdx.y of several.  One chunk leaves out what finds its own.
 template <bool DENSE, bool MANY>
 __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillDense& dense) {
   __shared__ __attribute__((aligned(16))) uint16_t vt_lds[kHeadDim * kPfVRow];
@@ -408,7 +407,7 @@ constexpr int prefill_heads(int group) { return group % 4 == 0 || group % 4 == 3
 
 // One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
 // LDS): saying so lets the compiler use all 512 registers.
-template <int G, bool CAP, bool MANY>
+template <int G, bool CAP>
 __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
     PrefillArgs a) {
   constexpr int CB = kPfBlocks;
@@ -428,11 +427,10 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   const int kvh = blockIdx.x;
   const int q_row0 = (int)(gridDim.y - 1 - blockIdx.y) * kRows;
   const int H = a.num_heads;
-  const int chunk = MANY ? (int)blockIdx.z / kHeadBlocks : 0;
-  const int head_block = MANY ? (int)blockIdx.z % kHeadBlocks : (int)blockIdx.z;
-  const int first_row = MANY ? chunk * a.chunk_rows : 0;
-  const int m = MANY ? min(a.chunk_rows, a.rows - first_row) : a.rows;
-  if (MANY && q_row0 >= m) return;  // (the last chunk of several may be shorter)
+  const int chunk = (int)blockIdx.z / kHeadBlocks, head_block = (int)blockIdx.z % kHeadBlocks;
+  const int first_row = chunk * a.chunk_rows;
+  const int m = min(a.chunk_rows, a.rows - first_row);
+  if (q_row0 >= m) return;  // (the last chunk of several may be shorter)
   auto head_in_group = [&](int cb) { return head_block * NH + cb % NH; };
   auto head_of = [&](int cb) { return kvh * G + min(head_in_group(cb), G - 1); };
   auto row_of = [&](int cb) { return q_row0 + 16 * (cb / NH) + qc; };
@@ -932,21 +930,18 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
   const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(chunk_rows, 16 * (kPfBlocks / heads)),
                   (unsigned)ceil_div(group, heads) * (chunks - (unsigned)together));
   const bool cap = cfg->logit_cap > 0.f;
-  const bool many = chunks - (unsigned)together > 1;
-#define TS_PF_LAUNCH(G_, C_, M_)                                                                  \
-  {                                                                                               \
-    static const hipError_t lds_ok = hipFuncSetAttribute(                                         \
-        (const void*)prefill_attn_kernel<G_, C_, M_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-        (int)kPfLdsBytes);                                                                        \
+#define TS_PF_LAUNCH(G_, C_)                                                                  \
+  {                                                                                           \
+    static const hipError_t lds_ok = hipFuncSetAttribute(                                     \
+        (const void*)prefill_attn_kernel<G_, C_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+        (int)kPfLdsBytes);                                                                    \
     if (lds_ok != hipSuccess) return fail(TS_EHIP, "prefill attention: %zu bytes of LDS refused", kPfLdsBytes); \
-    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_, M_>), grid, dim3(64 * kPfGroups), kPfLdsBytes, st, a); \
+    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_>), grid, dim3(64 * kPfGroups), kPfLdsBytes, st, a); \
   }
-#define TS_PF_CASE(G_)                        \
-  case G_:                                    \
-    if (cap && many) TS_PF_LAUNCH(G_, true, true)        \
-    else if (cap) TS_PF_LAUNCH(G_, true, false)          \
-    else if (many) TS_PF_LAUNCH(G_, false, true)         \
-    else TS_PF_LAUNCH(G_, false, false)       \
+#define TS_PF_CASE(G_)               \
+  case G_:                           \
+    if (cap) TS_PF_LAUNCH(G_, true)  \
+    else TS_PF_LAUNCH(G_, false)     \
     break;
   switch (group) {
     TS_PF_CASE(1)
