@@ -538,7 +538,8 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
 
 /* The chunks of a prompt part together: what ts_prefill_step_strided does for chunk after chunk of
  * chunk_rows rows (the last one of what is left). The first chunks, as far as max_seq_len says that they attend
- * to all tokens, are one; the others follow in rounds of up to 20: all rows of a round
+ * to all tokens, are one, or, where max_seq_len is the table's size and rows may be dropped at its
+ * end, each on its own; the others follow in rounds of up to 20: all rows of a round
  * are stored first, then its chunks select, each from the context up to its own last row, and attend.
  * Results are those of the chunks one by one (their votes are added up in another order), where the
  * slots of the whole part are all different and none of them is listed in the context before it.

@@ -526,7 +526,8 @@ def test_first_chunks_of_a_prompt_are_one(dev, heads, kv_heads, L0, T, chunk, bo
     results = []
     for together in (True, False):
         k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
-        table = torch.zeros((1, max(L0 + T, bound)), dtype=torch.int32, device=dev)
+        # (an entry to spare: of a table that may get full the chunks are taken one by one)
+        table = torch.zeros((1, max(L0 + T, bound) + 1), dtype=torch.int32, device=dev)
         table[0, :L0] = wl.table[0, :L0]
         seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
         out = torch.empty_like(q)

@@ -1,0 +1,63 @@
+"""A prompt's chunks taken together (``ts_prefill_prompt``) where the sizes are at their limits: tables that
+get full, more rows than one launch takes, too little memory for the workspace, values that are not finite.
+What is compared with is the chunks one by one (``ts_prefill_step_strided``)."""
+
+import dataclasses
+
+import pytest
+import torch
+
+from tokenselect_amd import ops, workloads
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _prompt(dev, heads, kv_heads, L0, T, top_k, seed=51, n_init=8, n_local=64, **config):
+    """A layer's configuration, its pools and table, and T rows more."""
+    shape = dict(num_heads=heads, num_kv_heads=kv_heads, rope_theta=5e5)
+    wl = workloads.build("pp", shape, [max(L0, 1)], [top_k], 1, dev, seed=seed, n_init=n_init, n_local=n_local,
+                         top_k=top_k, extra_pages=T)
+    g = torch.Generator(device=dev).manual_seed(seed + 1)
+    common = torch.randn((1, heads * 128), generator=g, device=dev)
+    q = (common + torch.randn((T, heads * 128), generator=g, device=dev)).bfloat16()
+    k, v = (torch.randn((T, kv_heads, 128), generator=g, device=dev).bfloat16() for _ in range(2))
+    return wl, dataclasses.replace(wl.cfg, **config), q, k, v, wl.free_pages[:T].contiguous()
+
+
+def _served(dev, wl, c, q, k, v, slots, L0, width, chunk, together, bound=None):
+    """(K pool, V pool, table, length, output) after the rows, with a table of `width` tokens."""
+    T = q.shape[0]
+    k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
+    table = torch.zeros((1, width), dtype=torch.int32, device=dev)
+    table[0, :L0] = wl.table[0, :L0]
+    seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
+    out = torch.full_like(q, 7.0)
+    layer = ops.PrefillChunk(c, width, dev, max_rows=chunk)
+    if together:
+        layer._prompt(q, k, v, slots, k_pool, v_pool, ops.Batch(seq, table, bound or min(L0 + T, width)), out, 0, T, chunk)
+    else:
+        for start in range(0, T, chunk):
+            end = min(start + chunk, T)
+            layer._serve(q, k, v, slots, k_pool, v_pool, ops.Batch(seq, table, min(L0 + end, width)), None, out, start,
+                         end - start)
+    torch.cuda.synchronize()
+    assert not layer.gave_up()
+    return k_pool, v_pool, table, seq, out
+
+
+def _same(x, y, names=("k", "v", "table", "length", "out")):
+    for name, a, b in zip(names, x, y):
+        a, b = (t.view(torch.int16) if t.dtype == torch.bfloat16 else t for t in (a, b))
+        assert torch.equal(a, b), f"{name}: {int((a != b).sum())} of {a.numel()} differ"
+
+
+@pytest.mark.parametrize("top_k", [2048, 96], ids=["dense", "selecting"])
+@pytest.mark.parametrize("L0,T,width", [(0, 1500, 1000), (0, 1500, 1500), (0, 1500, 1501), (700, 900, 1100),
+                                        (700, 300, 700), (3, 500, 130)])
+def test_a_table_that_gets_full(dev, top_k, L0, T, width):
+    """Rows beyond the table are not stored, and every chunk's rows lie where they lie if it is taken alone:
+    tables that end within a chunk, with the last chunk, and that are full from the start."""
+    say(f"prompt of {T} on {L0} in a table of {width}, top_k {top_k}")
+    case = _prompt(dev, 8, 2, L0, T, top_k)
+    _same(*(_served(dev, *case, L0, width, 128, together) for together in (True, False)))

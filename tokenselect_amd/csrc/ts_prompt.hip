@@ -507,8 +507,13 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   while (dense < chunks && bound_after(std::min<int64_t>((dense + 1LL) * chunk_rows, rows)) <=
                                (int64_t)cfg->n_init + cfg->top_k + cfg->n_local)
     ++dense;
-  if (dense > 0) {
-    const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)dense * chunk_rows, rows), bound = bound_after(n_rows);
+  // (A table that may get full: where a chunk's rows lie follows from the length after the chunk, which stops at
+  // the table's end, so that they are taken one by one.)
+  const int merged = bt->max_seq_len < kv->max_tokens ? dense : 1;
+  for (int first = 0; first < dense; first += merged) {
+    const int64_t row0 = (int64_t)first * chunk_rows;
+    const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)merged * chunk_rows, rows - row0);
+    const int32_t bound = bound_after(row0 + n_rows);
     const PromptWorkspace w = prompt_workspace(cfg, 1, bound);
     PrefillDense all{};
     all.table = table;
@@ -517,12 +522,13 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     all.sel_pos = (int32_t*)(ws + w.sel_pos);
     all.sel_len = (int32_t*)(ws + w.sel_len);
     all.list_bound = std::min(bound, kv->max_tokens);
-    all.store = rows_at(0, n_rows);
-    TS_TRY(launch_prefill_attn(cfg, q, q_stride, n_rows, k_pool, v_pool, pool_rows, all.sel, all.sel_len, bound, out,
+    all.store = rows_at(row0, n_rows);
+    TS_TRY(launch_prefill_attn(cfg, (const uint16_t*)q + row0 * q_stride, q_stride, n_rows, k_pool, v_pool, pool_rows,
+                               all.sel, all.sel_len, bound, (uint16_t*)out + row0 * cfg->num_heads * cfg->head_dim,
                                ws + w.stage, w.total - w.stage, st, &all));
-    if (dense == chunks) return TS_OK;
   }
 
+  if (dense == chunks) return TS_OK;
   const int rest = chunks - dense, group = (int)ceil_div(rest, ceil_div(rest, kPrGroup));  // (rounds of about the same size)
   for (int first = dense; first < chunks; first += group) {
     const int here = std::min(group, chunks - first);
