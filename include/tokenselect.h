@@ -544,7 +544,8 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
  * Results are those of the chunks one by one (their votes are added up in another order), where the
  * slots of the whole part are all different and none of them is listed in the context before it.
  * With slots chosen by the caller and a per-token table only (pages == NULL, page_size 1);
- * bt->max_seq_len bounds the length after the last row; no k_per_req.  No workgroup waits for another.
+ * bt->max_seq_len bounds the length after the last row; no k_per_req.  No workgroup waits for another, so that
+ * no call gives up: one that says it repeats another (bt->rerun) is refused.
  * bt->threshold_hint, where given, is not read; it receives what the last chunk's selection
  * leaves there.  q, out: [rows, H*D]; kv: k, v [rows, Hkv, D], out_cache_loc [rows]. */
 size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len);

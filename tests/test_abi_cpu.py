@@ -283,3 +283,23 @@ def test_header_is_plain_c_and_agrees_with_the_ctypes_mirror(tmp_path):
     want = [n for mirror in mirrors.values() for n in
             (ctypes.sizeof(mirror), *(getattr(mirror, field[0]).offset for field in mirror._fields_))]
     assert got == want
+
+
+def test_a_prompts_arguments_are_checked_before_anything_is_launched(lib):
+    """ts_prefill_prompt: what it does not take is refused on the host."""
+    c, one = cfg(), ctypes.c_void_p(0x1000)
+    pool = ctypes.pointer(_lib.TsPagePool(one, one, one))
+
+    def call(rows=4096, chunk=512, batch=1, config=c, q=one, pages=None, stride=0, nbytes=64, k_per_req=None, **options):
+        bt = _lib.TsBatch(batch, 4096, one, one, 4096, k_per_req)
+        for name, value in options.items():
+            setattr(bt, name, value)
+        kv = _lib.TsNewKv(one, one, one, pages, 4096)
+        return lib.ts_prefill_prompt(ctypes.byref(config), ctypes.byref(bt), ctypes.byref(kv), q, stride, 0, rows, chunk,
+                                     one, one, 4096, one, one, 10, one, one, nbytes, None)
+
+    assert call() == _lib.TS_EWORKSPACE, err(lib)
+    for bad in (dict(rows=0), dict(chunk=0), dict(batch=2), dict(q=None), dict(pages=pool), dict(stride=4088),
+                dict(config=cfg(page_size=16)), dict(k_per_req=one), dict(chunk=4000), dict(rerun=1)):
+        assert call(**bad) == _lib.TS_EINVAL, (bad, err(lib))
+    assert lib.ts_prefill_prompt_workspace_bytes(ctypes.byref(c), 0, 512, 4096) == 0

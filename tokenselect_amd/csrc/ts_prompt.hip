@@ -464,6 +464,8 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   TS_TRY(validate_batch(cfg, bt));
   TS_REQUIRE(rows >= 1 && chunk_rows >= 1 && chunk_rows <= 65535 * 16, TS_EINVAL,
              "ts_prefill_prompt: %d rows in chunks of %d", rows, chunk_rows);
+  // (nothing waits here, so that no call gives up and has to be repeated without its append)
+  TS_REQUIRE(bt->rerun == 0, TS_EINVAL, "ts_prefill_prompt has no call to repeat (rerun)");
   TS_REQUIRE(kv->pages == nullptr && cfg->page_size == 1, TS_EINVAL,
              "ts_prefill_prompt: slots chosen by the caller and a per-token table only");
   TS_REQUIRE(q && cos_table && sin_table && out, TS_EINVAL, "ts_prefill_prompt: NULL tensor argument");
