@@ -61,3 +61,14 @@ def test_a_table_that_gets_full(dev, top_k, L0, T, width):
     say(f"prompt of {T} on {L0} in a table of {width}, top_k {top_k}")
     case = _prompt(dev, 8, 2, L0, T, top_k)
     _same(*(_served(dev, *case, L0, width, 128, together) for together in (True, False)))
+
+
+def test_more_rows_than_one_attention_takes(dev):
+    """Ten chunks of 104900 rows: a launch of the attention takes 65535 x 16 = 1048560 rows.  Pools, table and
+    length the same; outputs as the two kernels' (2^-8 of a mean of normal values, and the result's rounding)."""
+    T, chunk = 1049000, 104900
+    say(f"prompt of {T} rows in chunks of {chunk}")
+    case = _prompt(dev, 1, 1, 0, T, 64, n_local=600)
+    x, y = (_served(dev, *case, 0, T, chunk, together) for together in (True, False))
+    _same(x[:4], y[:4])
+    assert (x[4].float() - y[4].float()).abs().max().item() <= 2 ** -7 * y[4].float().abs().max().item()

@@ -373,6 +373,8 @@ __global__ __launch_bounds__(kPrThreads, HKV * NB > 8 ? 1 : 2) void prompt_votes
 // Chunks that one round of launches takes, at most: the launches' fixed cost is shared by then, and the
 // staged keys and values of a round (11 MB a chunk at 8 KV heads) stay below the last-level cache.
 constexpr int kPrGroup = 20;
+// Rows that one launch of the attention takes (ts_sparse_prefill_attn's limit too).
+constexpr int kPrRows = 65535 * 16;
 // Workgroups of the scores' launches: two per CU, as many as run at once.
 constexpr int kPrWorkgroups = 512;
 
@@ -415,6 +417,11 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
   return w;
 }
 
+// The most chunks of a round.
+static int prompt_group(int32_t rows, int32_t chunk_rows) {
+  return (int)std::min<int64_t>({ceil_div(rows, chunk_rows), kPrGroup, kPrRows / chunk_rows});
+}
+
 template <int HKV, int NB>
 static int launch_prompt_scores(const PromptScoreArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)(ceil_div(a.blocks, 8) * 8 * a.sets));
@@ -448,8 +455,9 @@ using namespace ts;
 extern "C" {
 
 size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
-  if (validate_config(cfg) != TS_OK || rows < 1 || chunk_rows < 1 || max_seq_len < 1) return 0;
-  return prompt_workspace(cfg, (int)std::min<int64_t>(ceil_div(rows, chunk_rows), kPrGroup), max_seq_len).total;
+  if (validate_config(cfg) != TS_OK || rows < 1 || chunk_rows < 1 || chunk_rows > kPrRows || max_seq_len < 1)
+    return 0;
+  return prompt_workspace(cfg, prompt_group(rows, chunk_rows), max_seq_len).total;
 }
 
 int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
@@ -462,7 +470,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   TS_REQUIRE(bt != nullptr && bt->batch == 1 && bt->k_per_req == nullptr && kv != nullptr, TS_EINVAL,
              "ts_prefill_prompt serves one request at a time (batch must be 1) and needs the prompt's K/V");
   TS_TRY(validate_batch(cfg, bt));
-  TS_REQUIRE(rows >= 1 && chunk_rows >= 1 && chunk_rows <= 65535 * 16, TS_EINVAL,
+  TS_REQUIRE(rows >= 1 && chunk_rows >= 1 && chunk_rows <= kPrRows, TS_EINVAL,
              "ts_prefill_prompt: %d rows in chunks of %d", rows, chunk_rows);
   // (nothing waits here, so that no call gives up and has to be repeated without its append)
   TS_REQUIRE(bt->rerun == 0, TS_EINVAL, "ts_prefill_prompt has no call to repeat (rerun)");
@@ -479,10 +487,10 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   TS_TRY(check_fingerprint(q, std::min(rows, chunk_rows), cos_table, sin_table, table_rows, workspace, cfg->n_local));
   TS_REQUIRE(bt->max_seq_len - cfg->n_init - cfg->n_local <= (1 << 20), TS_ESHAPE,
              "ts_prefill_prompt: at most 2^20 candidates (max_seq_len %d)", bt->max_seq_len);
-  const int chunks = (int)ceil_div(rows, chunk_rows);
-  TS_REQUIRE(workspace_bytes >= prompt_workspace(cfg, std::min(chunks, kPrGroup), bt->max_seq_len).total, TS_EWORKSPACE,
-             "ts_prefill_prompt: workspace %zu bytes < required %zu", workspace_bytes,
-             prompt_workspace(cfg, std::min(chunks, kPrGroup), bt->max_seq_len).total);
+  const int chunks = (int)ceil_div(rows, chunk_rows), most = prompt_group(rows, chunk_rows);
+  const size_t need = prompt_workspace(cfg, most, bt->max_seq_len).total;
+  TS_REQUIRE(workspace_bytes >= need, TS_EWORKSPACE, "ts_prefill_prompt: workspace %zu bytes < required %zu",
+             workspace_bytes, need);
 
   const hipStream_t st = (hipStream_t)stream;
   const int q_stride = q_row_stride ? q_row_stride : cfg->num_heads * cfg->head_dim;
@@ -511,10 +519,10 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     ++dense;
   // (A table that may get full: where a chunk's rows lie follows from the length after the chunk, which stops at
   // the table's end, so that they are taken one by one.)
-  const int merged = bt->max_seq_len < kv->max_tokens ? dense : 1;
+  const int merged = bt->max_seq_len < kv->max_tokens ? std::min(dense, kPrRows / chunk_rows) : 1;
   for (int first = 0; first < dense; first += merged) {
     const int64_t row0 = (int64_t)first * chunk_rows;
-    const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)merged * chunk_rows, rows - row0);
+    const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)std::min(merged, dense - first) * chunk_rows, rows - row0);
     const int32_t bound = bound_after(row0 + n_rows);
     const PromptWorkspace w = prompt_workspace(cfg, 1, bound);
     PrefillDense all{};
@@ -531,7 +539,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   }
 
   if (dense == chunks) return TS_OK;
-  const int rest = chunks - dense, group = (int)ceil_div(rest, ceil_div(rest, kPrGroup));  // (rounds of about the same size)
+  const int rest = chunks - dense, group = (int)ceil_div(rest, ceil_div(rest, most));  // (rounds of about the same size)
   for (int first = dense; first < chunks; first += group) {
     const int here = std::min(group, chunks - first);
     const int64_t row0 = (int64_t)first * chunk_rows;
