@@ -2,12 +2,13 @@
 get full, more rows than one launch takes, too little memory for the workspace, values that are not finite.
 What is compared with is the chunks one by one (``ts_prefill_step_strided``)."""
 
+import ctypes
 import dataclasses
 
 import pytest
 import torch
 
-from tokenselect_amd import ops, workloads
+from tokenselect_amd import _lib, ops, workloads
 from helpers import say
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +73,29 @@ def test_more_rows_than_one_attention_takes(dev):
     x, y = (_served(dev, *case, 0, T, chunk, together) for together in (True, False))
     _same(x[:4], y[:4])
     assert (x[4].float() - y[4].float()).abs().max().item() <= 2 ** -7 * y[4].float().abs().max().item()
+
+
+def test_fewer_rows_than_a_chunk_need_no_longer_tables(dev):
+    """The rotation tables cover the rows that are there, whatever a chunk may have."""
+    L0, T = 1000, 20
+    say("prompt of fewer rows than a chunk, tables of as many")
+    wl, c, q, k, v, slots = _prompt(dev, 8, 2, L0, T, 96)
+    want = _served(dev, wl, c, q, k, v, slots, L0, L0 + T, T, False)
+    lib, cc = _lib.load(), c.to_c()
+    k_pool, v_pool = wl.k_pool.clone(), wl.v_pool.clone()
+    table = torch.zeros((1, L0 + T), dtype=torch.int32, device=dev)
+    table[0, :L0] = wl.table[0, :L0]
+    seq = torch.full((1,), L0, dtype=torch.int32, device=dev)
+    out = torch.empty_like(q)
+    cos, sin = ops.rope_tables(c.head_dim, c.rope_theta, c.rope_scale, c.n_local + T, dev)
+    nbytes = lib.ts_prefill_prompt_workspace_bytes(ctypes.byref(cc), T, 512, L0 + T)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    bt = _lib.TsBatch(1, L0 + T, seq.data_ptr(), table.data_ptr(), L0 + T, None)
+    kv = _lib.TsNewKv(k.data_ptr(), v.data_ptr(), slots.data_ptr(), None, L0 + T)
+    code = lib.ts_prefill_prompt(ctypes.byref(cc), ctypes.byref(bt), ctypes.byref(kv), q.data_ptr(), 0, 0, T, 512,
+                                 cos.data_ptr(), sin.data_ptr(), cos.shape[0], k_pool.data_ptr(), v_pool.data_ptr(),
+                                 k_pool.shape[0], out.data_ptr(), workspace.data_ptr(), nbytes,
+                                 torch.cuda.current_stream().cuda_stream)
+    assert code == _lib.TS_OK, lib.ts_last_error()
+    torch.cuda.synchronize()
+    _same((k_pool, v_pool, table, seq, out), want)

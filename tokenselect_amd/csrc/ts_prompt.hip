@@ -561,7 +561,8 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
                                    (int32_t*)(ws + w.sel_pos), w.max_sel, sel_len, (uint32_t*)(ws + w.topk));
     if (first + here == chunks) topk.hint = bt->threshold_hint;
     const ZeroRegion counters = topk_zero_region(topk, here);
-    const PromptChunks pc{n_rows, chunk_rows, here, lens, counters.base, (size_t)counters.stride, counters.words};
+    const PromptChunks pc{n_rows, std::min(chunk_rows, n_rows), here, lens, counters.base, (size_t)counters.stride,
+                          counters.words};
     TS_TRY(launch_prompt_fingerprint(cfg, q0, q_stride, cos_table, sin_table, table_rows, ws + w.qf, pc,
                                      rows_at(row0, n_rows), st));
 
