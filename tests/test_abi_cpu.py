@@ -303,3 +303,13 @@ def test_a_prompts_arguments_are_checked_before_anything_is_launched(lib):
                 dict(config=cfg(page_size=16)), dict(k_per_req=one), dict(chunk=4000), dict(rerun=1)):
         assert call(**bad) == _lib.TS_EINVAL, (bad, err(lib))
     assert lib.ts_prefill_prompt_workspace_bytes(ctypes.byref(c), 0, 512, 4096) == 0
+
+
+def test_a_prompts_workspace_is_bounded(lib):
+    """512 MiB, or what one chunk needs where that is more, however long the prompt."""
+    for c in (cfg(), cfg(top_k=4096, pool_kernel=15), cfg(num_heads=28, num_kv_heads=4), cfg(n_local=65536),
+              cfg(num_heads=4, num_kv_heads=1, top_k=64)):
+        for length in (700, 31615, 131072, 1 << 20):
+            one = lib.ts_prefill_prompt_workspace_bytes(ctypes.byref(c), 512, 512, length)
+            few, many = (lib.ts_prefill_prompt_workspace_bytes(ctypes.byref(c), n * 512, 512, length) for n in (2, 2000))
+            assert 0 < one <= few <= many <= max(512 << 20, one), (length, one, few, many)

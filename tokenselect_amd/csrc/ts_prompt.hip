@@ -370,9 +370,13 @@ __global__ __launch_bounds__(kPrThreads, HKV * NB > 8 ? 1 : 2) void prompt_votes
 }
 
 // --------------------------------------------------------------------------------- host
-// Chunks that one round of launches takes, at most: the launches' fixed cost is shared by then, and the
-// staged keys and values of a round (11 MB a chunk at 8 KV heads) stay below the last-level cache.
+// Chunks that one round of launches takes, at most: the launches' fixed cost is shared by then.
 constexpr int kPrGroup = 20;
+// And the most workspace of a round of several chunks, so that what a prompt needs beside the KV pool is bounded.
+// 20 chunks of 32 heads on 8 and top-k 2048 are 229 MB at 31.6K tokens, 253 at 131K and 476 at 1M; with top-k 4096
+// 397, 421 and, of 16 chunks, 515.  (Half of this cost 10240 rows behind 900K tokens 3.59 -> 4.36 ms, two sets of
+// chunks more to read the keys for, and 31599 rows with top-k 4096 2.57 -> 2.76.)
+constexpr size_t kPrBytes = (size_t)512 << 20;
 // Rows that one launch of the attention takes (ts_sparse_prefill_attn's limit too).
 constexpr int kPrRows = 65535 * 16;
 // Workgroups of the scores' launches: two per CU, as many as run at once.
@@ -418,8 +422,11 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
 }
 
 // The most chunks of a round.
-static int prompt_group(int32_t rows, int32_t chunk_rows) {
-  return (int)std::min<int64_t>({ceil_div(rows, chunk_rows), kPrGroup, kPrRows / chunk_rows});
+static int prompt_group(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
+  int group = (int)std::min<int64_t>({ceil_div(rows, chunk_rows), kPrGroup, kPrRows / chunk_rows});
+  while (group > 1 && prompt_workspace(cfg, group, max_seq_len).total > kPrBytes)  // (whole sets, while there are any)
+    group = group > kPrChunks ? (group - 1) / kPrChunks * kPrChunks : group - 1;
+  return group;
 }
 
 template <int HKV, int NB>
@@ -457,7 +464,7 @@ extern "C" {
 size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
   if (validate_config(cfg) != TS_OK || rows < 1 || chunk_rows < 1 || chunk_rows > kPrRows || max_seq_len < 1)
     return 0;
-  return prompt_workspace(cfg, prompt_group(rows, chunk_rows), max_seq_len).total;
+  return prompt_workspace(cfg, prompt_group(cfg, rows, chunk_rows, max_seq_len), max_seq_len).total;
 }
 
 int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
@@ -487,7 +494,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   TS_TRY(check_fingerprint(q, std::min(rows, chunk_rows), cos_table, sin_table, table_rows, workspace, cfg->n_local));
   TS_REQUIRE(bt->max_seq_len - cfg->n_init - cfg->n_local <= (1 << 20), TS_ESHAPE,
              "ts_prefill_prompt: at most 2^20 candidates (max_seq_len %d)", bt->max_seq_len);
-  const int chunks = (int)ceil_div(rows, chunk_rows), most = prompt_group(rows, chunk_rows);
+  const int chunks = (int)ceil_div(rows, chunk_rows), most = prompt_group(cfg, rows, chunk_rows, bt->max_seq_len);
   const size_t need = prompt_workspace(cfg, most, bt->max_seq_len).total;
   TS_REQUIRE(workspace_bytes >= need, TS_EWORKSPACE, "ts_prefill_prompt: workspace %zu bytes < required %zu",
              workspace_bytes, need);
