@@ -9,6 +9,8 @@ import pytest
 import torch
 
 from tokenselect_amd import _lib, ops, workloads
+from tokenselect_amd.patcher import sglang_standins as sg
+from tokenselect_amd.patcher import token_retrieval as tr
 from helpers import say
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +101,39 @@ def test_fewer_rows_than_a_chunk_need_no_longer_tables(dev):
     assert code == _lib.TS_OK, lib.ts_last_error()
     torch.cuda.synchronize()
     _same((k_pool, v_pool, table, seq, out), want)
+
+
+def test_a_prompt_without_memory_for_its_workspace(dev, monkeypatch):
+    """Where a round's workspace (some 230 MB here) cannot be had, the chunks go one by one, in the memory that
+    the request holds anyway: the results are those of the chunks together (kernels of either width: 2e-2)."""
+    monkeypatch.setattr(tr, "PREFILL_CHUNK_SIZE", 512)
+    H, Hkv, D, prompt = 8, 8, 128, 13000
+    say("prompt without memory for its workspace")
+    tr.patch(rope_base=5e5, rope_scale=1, rope_model="ROPE_LLAMA", max_n_tokens=16384, top_k=2048, n_init=128, n_local=512)
+    g = torch.Generator(device=dev).manual_seed(61)
+    common = torch.randn(1, H * D, generator=g, device=dev)
+    q = (common + torch.randn(prompt, H * D, generator=g, device=dev)).bfloat16()
+    k, v = (torch.randn(prompt, Hkv * D, generator=g, device=dev).bfloat16() for _ in range(2))
+    slots = torch.randperm(prompt, generator=g, device=dev).to(torch.int32)
+    pool = sg.TokenToKVPool(prompt, torch.bfloat16, Hkv, D, 1, dev)
+    runner = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool, dtype=torch.bfloat16)
+    attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
+
+    def serve(name):
+        retriever = runner.req_to_token_retriever.get_token_retriever(name)
+        out = attn.forward(q, k, v, sg.InputMetadata(sg.ForwardMode.EXTEND, retriever, pool, slots))
+        torch.cuda.synchronize()
+        return out.float(), retriever.num_tokens[0], int(retriever._num_tokens_dev[0])
+
+    want = serve("with")
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (150 << 20)) / total)
+    refused = torch.cuda.memory_stats(dev)["num_ooms"]
+    try:
+        got = serve("without")
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.cuda.memory_stats(dev)["num_ooms"] > refused
+    assert got[1:] == want[1:] == (prompt, prompt)
+    assert (got[0] - want[0]).abs().max().item() <= 2e-2

@@ -518,6 +518,7 @@ PyObject* serve(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
 // prompt(q, k, v, out_cache_loc, k_pool, v_pool, bt, out, from, rows, chunk_rows): `rows` rows of a prompt
 // part from `from` on, in chunks of chunk_rows, as serve() does them one by one.  The workspace is
 // the call's own, in the order of the stream: a prompt's is larger than what a request would keep.
+// False, and nothing done, where the memory for it (or for a copy of rows that lie otherwise) is not to be had.
 PyObject* prompt(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 11) raise(PyExc_TypeError, "prompt() takes 11 arguments");
   Owned& o = *self->own;
@@ -531,23 +532,29 @@ PyObject* prompt(Runner* self, PyObject* const* args, Py_ssize_t nargs) {
   if (o.max_rows < 1 || bt.batch != 1 || chunk_rows > o.max_rows)
     bad_value("one request, within the sizes this PrefillChunk was built for");
   if (from < 0 || rows < 1 || rows > INT32_MAX || chunk_rows < 1) bad_value("a chunk has at least one row");
-  const Rows q = rows_of(args[0], "q", from, rows, width, false);
-  Rows k = rows_of(args[1], "k", from, rows, row, false), v = rows_of(args[2], "v", from, rows, row, false);
-  if (k.stride != v.stride) {
-    if (k.stride != row) k = rows_of(args[1], "k", from, rows, row, true);
-    if (v.stride != row) v = rows_of(args[2], "v", from, rows, row, true);
-  }
   const at::Tensor& k_pool = check_pool(cfg, args[4], "k_pool");
   const at::Tensor& v_pool = check_pool(cfg, args[5], "v_pool");
   if (k_pool.size(0) != v_pool.size(0)) bad_value("k_pool and v_pool must have the same shape");
   if (cfg.page_size != 1) bad_value("page_size " + std::to_string(cfg.page_size) + " needs a PagePool");
-  const Rows loc = slots_of(args[3], from, rows);
-  const ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.ptr, nullptr, (int32_t)call.table_tokens};
   const at::Tensor& out = need(args[7], "out", at::kBFloat16);
   if (out.dim() < 1 || out.numel() != out.size(0) * width || out.size(0) < from + rows)
     bad_value("out must hold the rows of q");
+  Rows q, k, v, loc;
   const size_t bytes = prefill_prompt_bytes(&cfg, (int32_t)rows, (int32_t)chunk_rows, bt.max_seq_len);
-  const at::Tensor workspace = at::empty({(int64_t)bytes}, o.workspace.options());
+  at::Tensor workspace;
+  try {
+    q = rows_of(args[0], "q", from, rows, width, false);
+    k = rows_of(args[1], "k", from, rows, row, false), v = rows_of(args[2], "v", from, rows, row, false);
+    if (k.stride != v.stride) {
+      if (k.stride != row) k = rows_of(args[1], "k", from, rows, row, true);
+      if (v.stride != row) v = rows_of(args[2], "v", from, rows, row, true);
+    }
+    loc = slots_of(args[3], from, rows);
+    workspace = at::empty({(int64_t)bytes}, o.workspace.options());
+  } catch (const c10::OutOfMemoryError&) {
+    Py_RETURN_FALSE;
+  }
+  const ts_new_kv kv{k.ptr, v.ptr, (const int32_t*)loc.ptr, nullptr, (int32_t)call.table_tokens};
   const ts_stream_t stream = (ts_stream_t)c10::hip::getCurrentHIPStream().stream();
   int code;
   Py_BEGIN_ALLOW_THREADS

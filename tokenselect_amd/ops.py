@@ -998,10 +998,11 @@ class PrefillChunk(_GiveUpLatch):
     def _shapes(self):
         return self.cos, self.sin, None, 1, self.max_rows
 
-    def _prompt(self, q, k, v, loc, k_pool, v_pool, bt, out, start: int, rows: int, chunk_rows: int) -> torch.Tensor:
+    def _prompt(self, q, k, v, loc, k_pool, v_pool, bt, out, start: int, rows: int, chunk_rows: int):
         """``rows`` rows of a prompt part from row ``start`` on as chunks of ``chunk_rows`` that are taken
         together (``ts_prefill_prompt``), where :meth:`_serve` takes one; ``bt.max_seq_len`` bounds the
-        length after the last of them."""
+        length after the last of them.  ``False``, and nothing done, where there is no memory for the
+        workspace: some 12 MB a chunk, up to 512 MiB."""
         got = self._native.prompt(q, k, v, loc, k_pool, v_pool, bt, out, start, rows, chunk_rows)
         if got is None:   # an earlier call gave up
             self.check()

@@ -573,20 +573,24 @@ class TokenRetriever:
     def prefill_step(self, attn, q, k, v, loc, k_buffer, v_buffer, out):
         """The whole prompt part in chunks (tr.py:716-773): each its store, then
         :meth:`prefill_attention`, the rows of ``out`` written in place.  Several chunks are taken
-        together (a part that does not fit the table goes up to where it does not, chunk by chunk)."""
+        together (a part that does not fit the table goes up to where it does not, chunk by chunk, and so does
+        one for whose workspace there is no memory)."""
         layer_id, rows = attn.layer_id, q.shape[0]
         runner = self._prefill_chunk(attn)
         bt = ops.Batch(self._num_tokens_dev[layer_id:layer_id + 1],
                        self.token_indices[layer_id:layer_id + 1], 0)
+        memory = True
         for start in range(0, rows, PREFILL_CHUNK_SIZE):
-            if PREFILL_CHUNK_SIZE < rows - start and self._together(layer_id, rows - start):
+            if memory and PREFILL_CHUNK_SIZE < rows - start and self._together(layer_id, rows - start):
                 length = self.num_tokens[layer_id] + rows - start
                 last = (rows - start - 1) % PREFILL_CHUNK_SIZE + 1
                 bt.max_seq_len = length
                 bt.hint = self._chunk_hint(layer_id, length - last, last)
-                runner._prompt(q, k, v, loc, k_buffer, v_buffer, bt, out, start, rows - start, PREFILL_CHUNK_SIZE)
-                self.num_tokens[layer_id] = length
-                break
+                if runner._prompt(q, k, v, loc, k_buffer, v_buffer, bt, out, start, rows - start,
+                                  PREFILL_CHUNK_SIZE) is not False:
+                    self.num_tokens[layer_id] = length
+                    break
+                memory = False
             here = min(PREFILL_CHUNK_SIZE, rows - start)
             length = self.num_tokens[layer_id] + here
             assert length <= self.max_num_tokens   # tr.py:334
