@@ -405,11 +405,10 @@ __global__ __launch_bounds__(256) void prefill_gather_dense_kernel(PrefillArgs a
 // without a head, and of those the one with the most heads (which share a row's rotation).
 constexpr int prefill_heads(int group) { return group % 4 == 0 || group % 4 == 3 ? 4 : group % 2 == 0 ? 2 : 1; }
 
-// One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
-// LDS): saying so lets the compiler use all 512 registers.
-template <int G, bool CAP>
-__global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
-    PrefillArgs a) {
+// MANY: a chunk of several, which the workgroup finds first.  One chunk leaves that out: with it a chunk of 512 rows
+// behind 131072 tokens took 26.7 us, without 26.4, as before there were several.
+template <int G, bool CAP, bool MANY>
+__device__ __forceinline__ void prefill_attn(const PrefillArgs& a) {
   constexpr int CB = kPfBlocks;
   constexpr int NH = prefill_heads(G);   // heads of the workgroup
   constexpr int RT = CB / NH;            // query tiles of 16 rows
@@ -427,10 +426,11 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   const int kvh = blockIdx.x;
   const int q_row0 = (int)(gridDim.y - 1 - blockIdx.y) * kRows;
   const int H = a.num_heads;
-  const int chunk = (int)blockIdx.z / kHeadBlocks, head_block = (int)blockIdx.z % kHeadBlocks;
+  const int chunk = MANY ? (int)blockIdx.z / kHeadBlocks : 0;
+  const int head_block = (int)blockIdx.z - chunk * kHeadBlocks;
   const int first_row = chunk * a.chunk_rows;
-  const int m = min(a.chunk_rows, a.rows - first_row);
-  if (q_row0 >= m) return;  // (the last chunk of several may be shorter)
+  const int m = MANY ? min(a.chunk_rows, a.rows - first_row) : a.rows;
+  if (MANY && q_row0 >= m) return;  // (the last chunk of several may be shorter)
   auto head_in_group = [&](int cb) { return head_block * NH + cb % NH; };
   auto head_of = [&](int cb) { return kvh * G + min(head_in_group(cb), G - 1); };
   auto row_of = [&](int cb) { return q_row0 + 16 * (cb / NH) + qc; };
@@ -763,12 +763,13 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
     const float m_new = fmaxf(m_all, ml[0]);
     const float e0 = __builtin_amdgcn_exp2f(m_all - m_new), e1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
     m_all = m_new;
-    l_all = l_all * e0 + ml[1] * e1;
+    // (which product is rounded is said here: the compiler chooses by what is around, and a chunk's bits with it)
+    l_all = fmaf(l_all, e0, ml[1] * e1);
 #pragma unroll
     for (int db = 0; db < 8; ++db) {
       const pf_f32x4 od = other[db * 64];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sum[db][r] = sum[db][r] * e0 + od[r] * e1;
+      for (int r = 0; r < 4; ++r) sum[db][r] = fmaf(od[r], e1, sum[db][r] * e0);
     }
   }
 
@@ -782,6 +783,17 @@ __global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(
   for (int db = 0; db < 8; ++db)
     *(uint2*)(orow + 16 * db + 4 * g4) = make_uint2(pack_bf16(sum[db][0] * inv, sum[db][1] * inv),
                                                     pack_bf16(sum[db][2] * inv, sum[db][3] * inv));
+}
+// One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
+// LDS): saying so lets the compiler use all 512 registers.
+// (Both forms are one kernel: which it is is known from its arguments before the first load.)
+template <int G, bool CAP>
+__global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
+    PrefillArgs a) {
+  if (a.rows > a.chunk_rows)
+    prefill_attn<G, CAP, true>(a);
+  else
+    prefill_attn<G, CAP, false>(a);
 }
 
 int check_fingerprint(const void* q, int32_t rows, const float* cos_table, const float* sin_table,
@@ -846,7 +858,6 @@ static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_ro
   if (rest >= 205 || rest == 0 || (chunks == 1 && each >= 256)) return (int)chunks;
   return (int)(full * 256 / each);
 }
-
 
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }
 
@@ -927,7 +938,7 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
   }
   const int group = cfg->num_heads / cfg->num_kv_heads;
   const int heads = prefill_heads(group);
-  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(chunk_rows, 16 * (kPfBlocks / heads)),
+  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(std::min(chunk_rows, a.rows), 16 * (kPfBlocks / heads)),
                   (unsigned)ceil_div(group, heads) * (chunks - (unsigned)together));
   const bool cap = cfg->logit_cap > 0.f;
 #define TS_PF_LAUNCH(G_, C_)                                                                  \
