@@ -39,6 +39,7 @@ CXXFLAGS = [
 # into a loop over the active lanes (0.15 us apiece where a workgroup runs it once; one request of
 # 32K tokens 36.8 -> 35.9 us a layer).
 SOURCE_FLAGS = {"ts_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+                "ts_prefill_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 "ts_prefill_shared.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 "ts_score.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]}
 

@@ -91,5 +91,7 @@ __device__ __forceinline__ void packed_settled(pf_bf16x8 (&pb)[4]) {
 // them a chunk is (ts_prefill_shared.hip).
 int64_t prefill_shared_workgroups(int num_heads, int num_kv_heads, int chunk_rows);
 int launch_prefill_shared(const PrefillArgs& a, int chunks, hipStream_t stream);
+// The same in workgroups of 64 columns, for several chunks (ts_prefill_chunks.hip).
+int launch_prefill_several(const PrefillArgs& a, int chunks, hipStream_t stream);
 
 }  // namespace ts

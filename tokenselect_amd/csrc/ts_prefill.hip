@@ -10,8 +10,12 @@
 #include "ts_prefill.h"
 #include "ts_store.h"
 
+// ts_prefill_chunks.hip is this file's attention once more, for chunks that each have keys of their own, and nothing else
+// of it.
+
 namespace ts {
 
+#ifndef TS_PREFILL_CHUNKS
 // ------------------------------------------------------------------ fingerprint
 // Four workgroups per head (16 rotation pairs each), 512 threads = 4 quads of pairs
 // x 128 row groups, so that a chunk of 512 rows is one step of four independent rows
@@ -180,6 +184,8 @@ __global__ __launch_bounds__(kFpThreads) void prompt_fingerprint_kernel(
                           unit % per_chunk * kFpHeads, quarter);
 }
 
+#endif  // TS_PREFILL_CHUNKS
+
 // ------------------------------------------------------------ prefill attention
 // Two launches.
 //
@@ -223,10 +229,12 @@ __global__ __launch_bounds__(kFpThreads) void prompt_fingerprint_kernel(
 // CU at the 110 GB/s that L2 delivers to one: 13 us).  What is left over is mostly the
 // loads' latency: 64 KB per CU in flight, 0.6 to 0.85 us from L2 under this load.
 // Alternating products and exp2 in the source order of the logits' steps changed nothing.
-constexpr int kPfVRow = kPfKeys + 8;   // halfwords per V^T row in the gather kernel's LDS (80 B)
 // The merge area: per group and column block eight vectors of accumulators and (max, sum),
 // four floats per lane each.  (The rotated queries pass through the same space at the start.)
 constexpr size_t kPfLdsBytes = (size_t)kPfGroups * kPfBlocks * 9 * 64 * 16;  // 144 KB
+
+#ifndef TS_PREFILL_CHUNKS
+constexpr int kPfVRow = kPfKeys + 8;   // halfwords per V^T row in the gather kernel's LDS (80 B)
 
 // Position of key kk (0..31 within its block) in a V^T row: the matrix instruction
 // that made the logits left lane group g4 with keys 16 kb + 4 g4 + r (kb < 2, r < 4),
@@ -400,15 +408,21 @@ __global__ __launch_bounds__(256) void prefill_gather_dense_kernel(PrefillArgs a
   gather_tile<true, false>(a, dense);
 }
 
+#endif  // TS_PREFILL_CHUNKS
+
 // Heads of a workgroup's column blocks; the kPfBlocks / heads blocks of a head are
 // consecutive query tiles.  The choice that leaves the fewest columns of the last head block
 // without a head, and of those the one with the most heads (which share a row's rotation).
 constexpr int prefill_heads(int group) { return group % 4 == 0 || group % 4 == 3 ? 4 : group % 2 == 0 ? 2 : 1; }
 
-// MANY: a chunk of several, which the workgroup finds first.  One chunk leaves that out: with it a chunk of 512 rows
-// behind 131072 tokens took 26.7 us, without 26.4, as before there were several.
+// One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
+// LDS): saying so lets the compiler use all 512 registers.
+// MANY: a chunk of several, which the workgroup finds first.  One chunk leaves that out: 512 rows behind 131072
+// tokens 25.8 us with it, 25.3 without (with both in one kernel, chosen by its arguments, 25.5, and two or three
+// chunks of a prompt half a microsecond more).
 template <int G, bool CAP, bool MANY>
-__device__ __forceinline__ void prefill_attn(const PrefillArgs& a) {
+__global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
+    PrefillArgs a) {
   constexpr int CB = kPfBlocks;
   constexpr int NH = prefill_heads(G);   // heads of the workgroup
   constexpr int RT = CB / NH;            // query tiles of 16 rows
@@ -784,18 +798,47 @@ __device__ __forceinline__ void prefill_attn(const PrefillArgs& a) {
     *(uint2*)(orow + 16 * db + 4 * g4) = make_uint2(pack_bf16(sum[db][0] * inv, sum[db][1] * inv),
                                                     pack_bf16(sum[db][2] * inv, sum[db][3] * inv));
 }
-// One wavefront per SIMD by construction (four per workgroup, one workgroup per CU by its
-// LDS): saying so lets the compiler use all 512 registers.
-// (Both forms are one kernel: which it is is known from its arguments before the first load.)
-template <int G, bool CAP>
-__global__ __launch_bounds__(64 * kPfGroups) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_attn_kernel(
-    PrefillArgs a) {
-  if (a.rows > a.chunk_rows)
-    prefill_attn<G, CAP, true>(a);
-  else
-    prefill_attn<G, CAP, false>(a);
+
+template <bool MANY>
+static int launch_attention(const PrefillArgs& a, int chunks, hipStream_t stream) {
+  const int group = a.num_heads / a.num_kv_heads, heads = prefill_heads(group);
+  const dim3 grid((unsigned)a.num_kv_heads, (unsigned)ceil_div(std::min(a.chunk_rows, a.rows), 16 * (kPfBlocks / heads)),
+                  (unsigned)(ceil_div(group, heads) * chunks));
+  const bool cap = a.logit_cap > 0.f;
+#define TS_PF_LAUNCH(G_, C_)                                                                        \
+  {                                                                                                 \
+    static const hipError_t lds_ok = hipFuncSetAttribute(                                           \
+        (const void*)prefill_attn_kernel<G_, C_, MANY>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+        (int)kPfLdsBytes);                                                                          \
+    if (lds_ok != hipSuccess) return fail(TS_EHIP, "prefill attention: %zu bytes of LDS refused", kPfLdsBytes); \
+    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_, MANY>), grid, dim3(64 * kPfGroups), kPfLdsBytes, stream, a); \
+  }
+#define TS_PF_CASE(G_)               \
+  case G_:                           \
+    if (cap) TS_PF_LAUNCH(G_, true)  \
+    else TS_PF_LAUNCH(G_, false)     \
+    break;
+  switch (group) {
+    TS_PF_CASE(1)
+    TS_PF_CASE(2)
+    TS_PF_CASE(3)
+    TS_PF_CASE(4)
+    TS_PF_CASE(5)
+    TS_PF_CASE(6)
+    TS_PF_CASE(7)
+    TS_PF_CASE(8)
+    default: return fail(TS_ESHAPE, "unsupported head group %d", group);
+  }
+#undef TS_PF_CASE
+#undef TS_PF_LAUNCH
+  return check_launch("prefill_attn_kernel");
 }
 
+#ifdef TS_PREFILL_CHUNKS
+int launch_prefill_several(const PrefillArgs& a, int chunks, hipStream_t stream) {
+  return launch_attention<true>(a, chunks, stream);
+}
+#else
 int check_fingerprint(const void* q, int32_t rows, const float* cos_table, const float* sin_table,
                       int64_t table_rows, const void* qf, int32_t n_local) {
   TS_REQUIRE(q && cos_table && sin_table && qf, TS_EINVAL, "ts_fingerprint: NULL tensor argument");
@@ -936,42 +979,14 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
     a.vt += together * a.stage_stride;
     a.rows -= first.rows;
   }
-  const int group = cfg->num_heads / cfg->num_kv_heads;
-  const int heads = prefill_heads(group);
-  const dim3 grid((unsigned)cfg->num_kv_heads, (unsigned)ceil_div(std::min(chunk_rows, a.rows), 16 * (kPfBlocks / heads)),
-                  (unsigned)ceil_div(group, heads) * (chunks - (unsigned)together));
-  const bool cap = cfg->logit_cap > 0.f;
-#define TS_PF_LAUNCH(G_, C_)                                                                  \
-  {                                                                                           \
-    static const hipError_t lds_ok = hipFuncSetAttribute(                                     \
-        (const void*)prefill_attn_kernel<G_, C_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-        (int)kPfLdsBytes);                                                                    \
-    if (lds_ok != hipSuccess) return fail(TS_EHIP, "prefill attention: %zu bytes of LDS refused", kPfLdsBytes); \
-    hipLaunchKernelGGL((prefill_attn_kernel<G_, C_>), grid, dim3(64 * kPfGroups), kPfLdsBytes, st, a); \
-  }
-#define TS_PF_CASE(G_)               \
-  case G_:                           \
-    if (cap) TS_PF_LAUNCH(G_, true)  \
-    else TS_PF_LAUNCH(G_, false)     \
-    break;
-  switch (group) {
-    TS_PF_CASE(1)
-    TS_PF_CASE(2)
-    TS_PF_CASE(3)
-    TS_PF_CASE(4)
-    TS_PF_CASE(5)
-    TS_PF_CASE(6)
-    TS_PF_CASE(7)
-    TS_PF_CASE(8)
-    default: return fail(TS_ESHAPE, "unsupported head group %d", group);
-  }
-#undef TS_PF_CASE
-#undef TS_PF_LAUNCH
-  return check_launch("prefill_attn_kernel");
+  return together < (int)chunks - 1 ? launch_prefill_several(a, (int)chunks - together, st)
+                                    : launch_attention<false>(a, 1, st);
 }
+#endif  // TS_PREFILL_CHUNKS
 
 }  // namespace ts
 
+#ifndef TS_PREFILL_CHUNKS
 using namespace ts;
 
 extern "C" {
@@ -996,3 +1011,4 @@ int ts_sparse_prefill_attn(const ts_config* cfg, const void* q, int32_t rows, co
 }
 
 }  // extern "C"
+#endif  // TS_PREFILL_CHUNKS
