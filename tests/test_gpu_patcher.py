@@ -422,9 +422,9 @@ def test_rows_of_k_and_v_match_the_step(dev):
 
 @pytest.mark.parametrize("chunk,prompt", [(64, 192), (32, 339), (32, 900), (64, 1000)])
 def test_a_prompts_chunks_hand_on_where_the_threshold_lay(dev, monkeypatch, chunk, prompt):
-    """A chunk that adds at most a tenth to its context gets the threshold of the chunk before as a guess:
-    bit for bit the outputs of chunks without one, of the right guess and of nonsense; shorter contexts
-    neither read nor leave one."""
+    """A prompt that comes a chunk a call: one that adds at most a tenth to its context gets the threshold of the
+    one before as a guess.  Bit for bit the outputs of chunks without one, of the right guess and of nonsense;
+    shorter contexts neither read nor leave one.  Chunks that come together leave the last one's, the same."""
     H, Hkv, D = 8, 2, 128
     say(f"chunks with hints: chunk {chunk}, prompt {prompt}")
     monkeypatch.setattr(tr, "PREFILL_CHUNK_SIZE", 512)
@@ -434,26 +434,44 @@ def test_a_prompts_chunks_hand_on_where_the_threshold_lay(dev, monkeypatch, chun
     q, k, v = (torch.randn(prompt, n * D, generator=g, device=dev).bfloat16() for n in (H, Hkv, Hkv))
     slots = torch.randperm(1024, generator=g, device=dev).to(torch.int32)[:prompt].contiguous()
     plain = tr.TokenRetriever._chunk_hint
+    read = []
+    served = ops.PrefillChunk._serve
 
-    def run(hint):
+    def serve(self, q, k, v, loc, k_pool, v_pool, bt, *rest):
+        read.append(bt.hint is not None)
+        return served(self, q, k, v, loc, k_pool, v_pool, bt, *rest)
+
+    monkeypatch.setattr(ops.PrefillChunk, "_serve", serve)
+
+    def run(hint, rows=chunk):
         monkeypatch.setattr(tr.TokenRetriever, "_chunk_hint", hint)
         pool = sg.TokenToKVPool(1024, torch.bfloat16, Hkv, D, 1, dev)
         runner = sg.ModelRunner(model_config=sg.ModelConfig(1, D, H, Hkv), token_to_kv_pool=pool,
                                 dtype=torch.bfloat16)
         retriever = runner.req_to_token_retriever.get_token_retriever("req-hints")
         attn = sg.RadixAttention(H, D, D ** -0.5, Hkv, layer_id=0)
-        out = attn.forward(q, k, v, sg.InputMetadata(sg.ForwardMode.EXTEND, retriever, pool, slots))
+        read.clear()
+        out = torch.cat([attn.forward(q[s:s + rows], k[s:s + rows], v[s:s + rows], sg.InputMetadata(
+            sg.ForwardMode.EXTEND, retriever, pool, slots[s:s + rows])) for s in range(0, prompt, rows)])
         torch.cuda.synchronize()
         return out, int(retriever._chunk_hints[0])
 
+    long = [s >= 10 * min(chunk, prompt - s) for s in range(0, prompt, chunk)]
     want, left = run(lambda self, layer, before, rows: None)
-    assert left == 0
+    assert left == 0 and read == [False] * len(long)
     got, left = run(plain)
+    assert read == long
     assert torch.equal(got, want)
-    assert (left != 0) == any(s >= 10 * min(chunk, prompt - s) for s in range(0, prompt, chunk))
+    assert (left != 0) == any(long)
     nonsense = torch.empty(1, dtype=torch.int32, device=dev)
 
     def wild(self, layer, before, rows):
         return nonsense.fill_((before * 37) % 4096 - 1000)
 
-    assert torch.equal(run(wild)[0], want)
+    got, _ = run(wild)
+    assert all(read) and torch.equal(got, want)
+    got, together = run(plain, prompt)
+    assert read == []
+    # (dense chunks together are sums in another order: 2^-8 of a mean of normal values, and a rounding each)
+    assert (got.float() - want.float()).abs().max().item() <= 2 ** -7 * want.float().abs().max().item()
+    assert together == (left if long[-1] else 0)

@@ -103,6 +103,24 @@ def test_fewer_rows_than_a_chunk_need_no_longer_tables(dev):
     _same((k_pool, v_pool, table, seq, out), want)
 
 
+@pytest.mark.parametrize("where", ["key", "query"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("pool", [-1, 5], ids=["votes", "pooled"])
+def test_values_that_are_not_finite(dev, where, value, pool):
+    """A key of the context or a query row that is not finite: its head's scores, and with them the votes of the
+    chunks that see it, are what they are for the chunks one by one, and so is what is selected and attended to."""
+    L0, T, chunk = 900, 300, 64
+    say(f"prompt with {value} in a {where}, pool {pool}")
+    wl, c, q, k, v, slots = _prompt(dev, 8, 2, L0, T, 96, pool_kernel=pool)
+    if where == "key":
+        wl.k_pool[wl.table[0, 500].long(), 1, 7] = value
+    else:
+        q[chunk + 3, 2 * 128 + 9] = value
+    x, y = (_served(dev, wl, c, q, k, v, slots, L0, L0 + T, chunk, together) for together in (True, False))
+    _same([t.nan_to_num(nan=77.0) if t.dtype == torch.bfloat16 else t for t in x],
+          [t.nan_to_num(nan=77.0) if t.dtype == torch.bfloat16 else t for t in y])
+
+
 def test_a_prompt_without_memory_for_its_workspace(dev, monkeypatch):
     """Where a round's workspace (some 230 MB here) cannot be had, the chunks go one by one, in the memory that
     the request holds anyway: the results are those of the chunks together (kernels of either width: 2e-2)."""
@@ -128,9 +146,14 @@ def test_a_prompt_without_memory_for_its_workspace(dev, monkeypatch):
     want = serve("with")
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(dev).total_memory
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (150 << 20)) / total)
-    refused = torch.cuda.memory_stats(dev)["num_ooms"]
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (192 << 20)) / total)
     try:
+        held = []
+        with pytest.raises(torch.OutOfMemoryError):
+            while len(held) < 4096:
+                held.append(torch.empty(64 << 20, dtype=torch.uint8, device=dev))
+        del held[-2:]
+        refused = torch.cuda.memory_stats(dev)["num_ooms"]
         got = serve("without")
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
