@@ -539,13 +539,16 @@ int ts_prefill_step_strided(const ts_config* cfg, const ts_batch* bt, const ts_n
 /* The chunks of a prompt part together: what ts_prefill_step_strided does for chunk after chunk of
  * chunk_rows rows (the last one of what is left). The first chunks, as far as max_seq_len says that they attend
  * to all tokens, are one, or, where max_seq_len is the table's size and rows may be dropped at its
- * end, each on its own; the others follow in rounds of up to 20: all rows of a round
+ * end, each on its own; the others follow in rounds of up to 20 (fewer where more than one would need over
+ * 512 MiB of workspace): all rows of a round
  * are stored first, then its chunks select, each from the context up to its own last row, and attend.
  * Results are those of the chunks one by one (their votes are added up in another order), where the
- * slots of the whole part are all different and none of them is listed in the context before it.
+ * slots of the WHOLE part are all different and none of them is listed in the context before it: rows
+ * of two chunks that share a slot are written at the same time, and which of them stays, and which an
+ * earlier chunk attends to, is not defined (ts_prefill_step asks that of a chunk's own slots only).
  * With slots chosen by the caller and a per-token table only (pages == NULL, page_size 1);
- * bt->max_seq_len bounds the length after the last row; no k_per_req.  No workgroup waits for another, so that
- * no call gives up: one that says it repeats another (bt->rerun) is refused.
+ * bt->max_seq_len bounds the length after the last row, with at most 2^20 candidates; no k_per_req.  No workgroup
+ * waits for another, so that no call gives up: one that says it repeats another (bt->rerun) is refused.
  * bt->threshold_hint, where given, is not read; it receives what the last chunk's selection
  * leaves there.  q, out: [rows, H*D]; kv: k, v [rows, Hkv, D], out_cache_loc [rows]. */
 size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len);

@@ -8,7 +8,7 @@
 // beyond L2: 25.7 us a workgroup, and fifteen chunks of 28 heads on 4 (13.1 workgroups per CU) 337 us.
 // Here a wavefront has 64 columns of its own and all keys, so that a workgroup has 256 columns: a quarter of
 // the reads, nothing to merge, and 84 tiles instead of 21 for the rotation of the queries and the first loads
-// to be paid from.  75 us a workgroup, 0.75 of it the matrix unit's: 5712 products of 16 cycles, at the
+// to be paid from.  75 us a workgroup, 0.61 to 0.68 of it the matrix unit's: 5712 products of 16 cycles, at the
 // 1.8 to 2.0 GHz that the device keeps up under them.
 //
 // The tiles pass through LDS, past the registers.  From there the operands go to the registers as they do from

@@ -6,21 +6,23 @@
 // rows of that: once all rows are stored no chunk needs another one's result.  A chunk on its own
 // is four launches that are chains of round trips (fingerprint 7 us, selection 23 to 60 with its
 // workgroups waiting for each other, gather 6.5, attention 25); together they are eight launches
-// for all of them, of which only the attention is long:
+// for all of them, nine or ten where some chunks fill no wave of the wide attention or votes are
+// pooled (whose first histogram is then a launch too), and only the attention is long:
 //
 //   fingerprints    of all chunks, the store of all their rows, every chunk's length
 //   statistics      per (chunk, head) maximum and sum of exponentials of the scores, by blocks of tokens
 //   merge           of the blocks' statistics
 //   votes           the scores once more, as votes (tr.py:361), and the first histogram of the top-k
-//   [max-pool]      tr.py:366-369
+//   [max-pool, histogram]  tr.py:366-369
 //   mark, final     the ragged top-k, a chunk as a request
-//   gather, attention
+//   gather, attention [, attention of the chunks that are left]
 //
 // Nobody waits for anybody.  The scores are computed twice instead of kept: for one chunk the keys
 // are the cost (the single launch streams them once and holds the scores in LDS), for four chunks
 // that a workgroup serves together they are read for all of them, and 16 query rows fill the
 // matrix instruction's tile.  A prompt of 31599 tokens with 16 more, 28 heads on 4, its chunks one after
-// the other and together: 4271 and 2143 us; three of 700 to 5200 tokens, 32 heads on 8, two layers: 2423 and 1789.
+// the other and together: 4183 and 2040 us; three of 700 to 5200 tokens + 8, 32 heads on 8, two layers: 2352 and 1713
+// (both of a case in turn on one box).
 #include <algorithm>
 #include <type_traits>
 
@@ -518,8 +520,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   // The first chunks, which attend to everything before them, are one: a row's keys are the same wherever its
   // chunk ends.  Five chunks of 512, 32 heads on 8: five times a gather (5 to 8 us) and an attention (12 to 23),
   // each with the device half idle at its end, and together 9 and 79 us.  Three prompts of 700 to 5200
-  // tokens, two layers, in the same run as the code that takes every chunk on its own: 1915 of 2351 us, and 1789 of
-  // 2423 with this; a prompt of 31599, 28 heads on 4: 2108 of 4179, 2143 of 4271.
+  // tokens + 8, two layers, 32 heads on 8: 1915 -> 1729 us.
   int dense = 0;
   while (dense < chunks && bound_after(std::min<int64_t>((dense + 1LL) * chunk_rows, rows)) <=
                                (int64_t)cfg->n_init + cfg->top_k + cfg->n_local)

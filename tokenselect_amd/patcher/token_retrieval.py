@@ -547,8 +547,9 @@ class TokenRetriever:
 
     def _chunk_hint(self, layer_id, before, rows):
         """Where the threshold of the chunk before lay, for a chunk that adds at most a tenth to the context:
-        with more, the k-th of the candidates is another bin's too often (a prompt of 31600 tokens, 28 heads:
-        4302 -> 4146 us; of 12000 1305 -> 1266; three of 700 to 5200, each chunk with a hint, 2368 -> 2388)."""
+        with more, the k-th of the candidates is another bin's too often.  A chunk that comes alone reads it;
+        of chunks that are taken together the last one leaves it.  (Chunk by chunk, a prompt of 31600 tokens, 28
+        heads: 4302 -> 4146 us; of 12000 1305 -> 1266; three of 700 to 5200, each chunk with a hint, 2368 -> 2388.)"""
         return self._chunk_hints[layer_id:layer_id + 1] if before >= 10 * rows else None
 
     def prefill_attention(self, attn, q, k_buffer, v_buffer):
