@@ -1,4 +1,4 @@
-"""As test_prefill_hazards_cpu, for the attention's workgroups of 256 columns."""
+"""As test_prefill_hazards_cpu, for the attention in workgroups of 256 columns (ts_prefill_shared.hip)."""
 
 import os
 import re
@@ -25,5 +25,5 @@ def test_output_products_keep_their_distance(tmp_path, kind):
     kernels = _parse(out.read_text())
     assert len(kernels) == 2                                   # with and without a cap
     for name, kernel in kernels.items():
-        assert sum(i[3] and i[4] for i in kernel) >= 64, name
+        assert sum(i[3] and i[4] for i in kernel) >= 4 * 32, name
         assert _hazards(kernel) == [], name

@@ -86,6 +86,7 @@ __device__ __forceinline__ void mfma_settled(pf_f32x4 (&o)[CB][8]) {
 __device__ __forceinline__ void packed_settled(pf_bf16x8 (&pb)[4]) {
   asm("s_nop 1" : "+v"(pb[0]), "+v"(pb[1]), "+v"(pb[2]), "+v"(pb[3]));
 }
+__device__ __forceinline__ void weights_settled(pf_bf16x8& p) { asm("s_nop 1" : "+v"(p)); }
 
 // The attention over a staging area that has been filled, in workgroups of 256 columns, and how many of
 // them a chunk is (ts_prefill_shared.hip).
