@@ -245,12 +245,16 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
                                const void* k_pool, const void* v_pool, int64_t pool_rows, const int32_t* sel,
                                int64_t sel_stride, const int32_t* sel_len, int32_t max_sel_len, void* out,
                                void* workspace, size_t workspace_bytes, hipStream_t stream,
-                               const PrefillDense* dense = nullptr);
+                               const PrefillDense* dense = nullptr, void* cut_space = nullptr);
 // ts_sparse_prefill_attn for query rows that lie q_stride elements apart.
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
                         int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes, hipStream_t stream,
-                        const PrefillDense* dense = nullptr);
+                        const PrefillDense* dense = nullptr, void* cut_space = nullptr);
+// Space for the pieces of jobs that the attention's workgroups of 256 columns share (ts_prefill_shared.hip), and
+// whether so many rows over so many keys would use it.
+size_t prefill_cut_bytes();
+bool prefill_cuts_pay(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys);
 
 // Sparse decode attention (ts_attn.hip).  The kernel counts its workgroups in per
 // (request, KV head) tickets inside the workspace, which must be zero at launch:

@@ -91,7 +91,21 @@ __device__ __forceinline__ void weights_settled(pf_bf16x8& p) { asm("s_nop 1" : 
 // The attention over a staging area that has been filled, in workgroups of 256 columns, and how many of
 // them a chunk is (ts_prefill_shared.hip).
 int64_t prefill_shared_workgroups(int num_heads, int num_kv_heads, int chunk_rows);
-int launch_prefill_shared(const PrefillArgs& a, int chunks, hipStream_t stream);
+// Their jobs, per KV head: a workgroup each for the first `whole`, and the others shared out evenly between
+// `streams` workgroups, by what they cost, so that a share may begin and end within a job.
+struct PrefillCuts {
+  int chunks, per_chunk, jobs;  // chunks, jobs of a chunk (the last one may have fewer), of all
+  int whole, streams;
+  int keys;                     // that the last row of a chunk sees, by the host's knowledge
+  int quantum;                  // cost of a share
+  uint32_t* tickets;            // zero at launch: of the jobs that are cut
+  char* pieces;                 // and what there is of each
+};
+constexpr int kPsSlots = 256;   // workgroups that share jobs, of all KV heads: one per CU
+constexpr int kPsTicketBytes = kPsSlots * 4 * 4;
+// (without a workspace of prefill_cut_bytes() no job is cut)
+PrefillCuts prefill_cuts(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys, void* workspace);
+int launch_prefill_shared(const PrefillArgs& a, const PrefillCuts& cuts, hipStream_t stream);
 // The same in workgroups of 64 columns, for several chunks (ts_prefill_chunks.hip).
 int launch_prefill_several(const PrefillArgs& a, int chunks, hipStream_t stream);
 

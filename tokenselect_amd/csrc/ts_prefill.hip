@@ -400,11 +400,18 @@ __device__ __forceinline__ void gather_tile(const PrefillArgs& a, const PrefillD
     stage(a, vout + p, *(const uint4*)(vt_lds + (16 * (p >> 6) + (p & 15)) * kPfVRow + 8 * ((p >> 4) & 3)));
   }
 }
+// The tickets of the attention's jobs that are cut (PrefillCuts), if there are any.
+__device__ __forceinline__ void clear_tickets(uint32_t* tickets) {
+  if (tickets && blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < kPsTicketBytes / 4; i += 256) tickets[i] = 0u;
+}
 template <bool MANY>
-__global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256) void prefill_gather_kernel(PrefillArgs a, uint32_t* tickets) {
+  clear_tickets(tickets);
   gather_tile<false, MANY>(a, PrefillDense{});
 }
-__global__ __launch_bounds__(256) void prefill_gather_dense_kernel(PrefillArgs a, PrefillDense dense) {
+__global__ __launch_bounds__(256) void prefill_gather_dense_kernel(PrefillArgs a, PrefillDense dense, uint32_t* tickets) {
+  clear_tickets(tickets);
   gather_tile<true, false>(a, dense);
 }
 
@@ -902,21 +909,34 @@ static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_ro
   return (int)(full * 256 / each);
 }
 
+// Whether the workgroups of 256 columns take all rows, with jobs that are cut: one long dense chunk from 0.87 waves of
+// jobs on, several chunks from 0.59.  us for a whole call, in workgroups of 64 columns and so: 28 heads on 4, 1536
+// dense rows (0.66) 46 and 45, 2048 (0.87) 61 and 54; 32 on 8, 1536 (0.75) 46 and 48, 2048 (1) 62 and 60; two full chunks of
+// 28 heads (0.44) 95 and 96, of 32 (0.5) 99 and 103; 1436 rows in chunks of 512 of 28 heads (0.61) 117 and 110, of 32
+// (0.7) 124 and 122, 1948 of 24 on 8 (0.72) 149 and 125.  And from 1024 keys on: the start of a piece costs ten tiles of 32.
+bool prefill_cuts_pay(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys) {
+  if (keys < 1024) return false;
+  const PrefillCuts c = prefill_cuts(num_heads, num_kv_heads, rows, chunk_rows, 1, nullptr);
+  // (small chunks would leave most of a workgroup without columns)
+  if (4 * (int64_t)std::min(rows, chunk_rows) * num_heads < 3 * (int64_t)c.per_chunk * num_kv_heads * 256) return false;
+  return c.jobs * num_kv_heads >= (c.chunks == 1 ? 224 : 152);
+}
+
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }
 
 int launch_prefill_attn(const ts_config* cfg, const void* q, int q_stride, int32_t rows, const void* k_pool,
                         const void* v_pool, int64_t pool_rows, const int32_t* sel, const int32_t* sel_len,
                         int32_t max_sel_len, void* out, void* workspace, size_t workspace_bytes,
-                        hipStream_t stream, const PrefillDense* dense) {
+                        hipStream_t stream, const PrefillDense* dense, void* cut_space) {
   return launch_prefill_attn_chunks(cfg, q, q_stride, rows, rows, k_pool, v_pool, pool_rows, sel, 0, sel_len,
-                                    max_sel_len, out, workspace, workspace_bytes, stream, dense);
+                                    max_sel_len, out, workspace, workspace_bytes, stream, dense, cut_space);
 }
 
 int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride, int32_t rows, int32_t chunk_rows,
                                const void* k_pool, const void* v_pool, int64_t pool_rows, const int32_t* sel,
                                int64_t sel_stride, const int32_t* sel_len, int32_t max_sel_len, void* out,
                                void* workspace, size_t workspace_bytes, hipStream_t stream,
-                               const PrefillDense* dense) {
+                               const PrefillDense* dense, void* cut_space) {
   TS_TRY(validate_config(cfg));
   TS_REQUIRE(q && k_pool && v_pool && sel && sel_len && out, TS_EINVAL,
              "ts_sparse_prefill_attn: NULL tensor argument");
@@ -960,17 +980,21 @@ int launch_prefill_attn_chunks(const ts_config* cfg, const void* q, int q_stride
   a.len_cap = dense ? dense->store.max_tokens : 0;
   hipStream_t st = stream;
   const dim3 gather_grid((unsigned)cfg->num_kv_heads * (unsigned)(a.s_pad / kPfKeys), chunks);
+  const bool cut = cut_space != nullptr && prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows, max_sel_len);
+  const int together = cut ? (int)chunks : shared_chunks(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows);
+  PrefillArgs first = a;
+  first.rows = (int)std::min<int64_t>(rows, (int64_t)together * chunk_rows);
+  PrefillCuts cuts{};
+  if (together > 0)
+    cuts = prefill_cuts(cfg->num_heads, cfg->num_kv_heads, first.rows, chunk_rows, max_sel_len, cut ? cut_space : nullptr);
   if (dense)
-    hipLaunchKernelGGL(prefill_gather_dense_kernel, gather_grid, dim3(256), 0, st, a, *dense);
+    hipLaunchKernelGGL(prefill_gather_dense_kernel, gather_grid, dim3(256), 0, st, a, *dense, cuts.tickets);
   else
     hipLaunchKernelGGL(chunks > 1 ? prefill_gather_kernel<true> : prefill_gather_kernel<false>, gather_grid, dim3(256), 0,
-                       st, a);
+                       st, a, cuts.tickets);
   TS_TRY(check_launch("prefill_gather_kernel"));
-  const int together = shared_chunks(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows);
   if (together > 0) {
-    PrefillArgs first = a;
-    first.rows = (int)std::min<int64_t>(rows, (int64_t)together * chunk_rows);
-    TS_TRY(launch_prefill_shared(first, together, st));
+    TS_TRY(launch_prefill_shared(first, cuts, st));
     if (together == (int)chunks) return TS_OK;
     a.q += (size_t)first.rows * q_stride;
     a.out += (size_t)first.rows * cfg->num_heads * kHeadDim;

@@ -23,9 +23,21 @@
 // GHz: their accumulators' registers are read and written twice as often for the same sums), four products in a
 // row into one accumulator (3 % less in the probe, here all operands of K are refilled at the end of a pass: 1585).
 //
+// Jobs that are cut: 256 columns and their keys are a job, and where the jobs do not fill whole waves of a workgroup per
+// CU, or are of very different lengths (a long dense chunk, whose first rows see few keys), the workgroups of the last
+// wave and a bit take equal shares of what is left instead, in the order of the jobs, so that a share begins and ends within
+// a job; the pieces of a job meet in memory.  A piece costs 6.5 us before its first tile (1.5 until the queries are
+// asked for, 2 until all is, 2.2 for their rotation, 1 for the first logits), 2.5 to be left or 4.5 to be added up, 2.2 for
+// the output: some 10 tiles.  us for a whole call, without and with: eight chunks of 28 heads on 4 (1.75 waves) 229 ->
+// 198, six (1.3) 177 -> 162, six of 32 on 8 (1.5) 191 -> 183, three of 28 (0.6) 117 -> 110; 2048 dense rows of 28 heads
+// 61 -> 54, 2560 of 32 75 -> 73.  That the first operands pass through LDS as the others do (each wavefront for itself
+// asked for 96 KB a workgroup in place of 24: 2.7 us until all was), the scale is the rotation's, and the output is written in
+// pieces of 16 bytes (3.6 -> 2.0 us) made a workgroup 79 -> 77 us, which four waves of them give back to the clock.
+//
 // Which columns: the query rows of a chunk are cut into tiles of 16, the G heads of a KV head that see the same
 // tile are G column blocks, and these are numbered tile by tile.  A workgroup takes sixteen in a
 // row, so that no column is left without a head whatever G is.
+#include <algorithm>
 #include <utility>
 
 #include "ts_prefill.h"
@@ -37,6 +49,11 @@ constexpr int kPsThreads = 64 * kPsWaves;
 constexpr int kPsUnits = kPsWaves * kPfBlocks;             // column blocks of a workgroup
 constexpr int kPsPackage = 2 * kPfOperands * 64;           // a K tile and a V^T tile, in 16 bytes
 constexpr int kPsBuffers = 4;
+typedef __attribute__((ext_vector_type(4))) uint32_t ps_u32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t ps_u32x2;
+constexpr int kPsCoherent = 16;  // a buffer access past the XCD's L2 (sc1), as agent-scope atomics are
+constexpr int kPsCost = 10;       // what a piece of a job costs besides its tiles, in tiles
+constexpr int kPsLeast = 8;      // tiles of a piece of a job that is cut, at least
 constexpr size_t kPsLdsBytes = (size_t)kPsBuffers * kPsPackage * 16;  // 64 KB
 
 // Two kilobytes, 16 bytes per lane of each, from `at` bytes behind the start of `from` to `to` (a byte of LDS), past
@@ -71,22 +88,104 @@ constexpr int weighed(int n) { return n <= 0 ? 0 : n <= 32 ? 20 * n / 32 : n < 5
 constexpr int packed(int n) { return weighed(n - 1) / 2; }
 constexpr int kMaxAt = 8;  // the product of the second thirty-six behind which the search for the largest logit begins
 
+// ---- the jobs that are cut (PrefillCuts)
+// The tiles that the rows of workgroup i of a chunk of m rows see, of `keys` keys.
+__host__ __device__ __forceinline__ int job_tiles(int keys, int m, int i, int group) {
+  const int row_end = (i * kPsUnits + kPsUnits - 1) / group * 16 + 16;
+  const int last = keys - m + (row_end < m ? row_end : m) - 1;
+  return last < 0 ? 1 : last / kPfKeys + 1;
+}
+// Job j of a KV head, the chunks one after the other, the last rows of each first.
+struct PsJob {
+  int chunk, m, i, tiles;
+};
+__host__ __device__ __forceinline__ PsJob job_at(const PrefillCuts& c, int rows, int chunk_rows, int group, int j) {
+  PsJob job;
+  job.chunk = j / c.per_chunk < c.chunks ? j / c.per_chunk : c.chunks - 1;
+  const int begin = job.chunk * c.per_chunk;
+  job.m = rows - job.chunk * chunk_rows < chunk_rows ? rows - job.chunk * chunk_rows : chunk_rows;
+  job.i = (job.chunk + 1 < c.chunks ? c.per_chunk : c.jobs - begin) - 1 - (j - begin);
+  job.tiles = job_tiles(c.keys, job.m, job.i, group);
+  return job;
+}
+// Where a boundary that lies `at` tiles into a job cuts it: not so close to an end that a piece would be shorter than
+// kPsLeast; 0 and `tiles` are no cut.
+__host__ __device__ __forceinline__ int cut_at(int at, int tiles) {
+  return at >= tiles ? tiles : at < kPsLeast ? 0 : at > tiles - kPsLeast ? tiles : at;
+}
+
+constexpr int kPsPiece = 4 * 8 * 64 * 16 + 4 * 64 * 8;  // bytes that a wavefront leaves of a piece: sums; maxima and weights
+constexpr int kPsPieces = 2 * kPsSlots;                 // two of each workgroup: one cut at its start, one at its end
+static_assert(kPsTicketBytes == kPsSlots * kPsWaves * 4, "a ticket per wavefront of the workgroup that has a job's first piece");
+size_t prefill_cut_bytes() { return kPsTicketBytes + (size_t)kPsPieces * kPsWaves * kPsPiece; }
+
 template <bool CAP>
 __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_shared_kernel(
-    PrefillArgs a) {
+    PrefillArgs a, PrefillCuts cuts) {
   constexpr int CB = kPfBlocks;
   extern __shared__ __attribute__((aligned(16))) uint4 ps_lds[];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   const int qc = lane & 15, g4 = lane >> 4;  // query column / key group of the matrix layouts
   // The KV head fastest, as in the other kernel; the last rows, which see the most keys, start first.
-  const int kvh = blockIdx.x, chunk = blockIdx.z;
+  const int kvh = blockIdx.x;
   const int G = a.num_heads / a.num_kv_heads;
-  const int unit0 = (int)(gridDim.y - 1 - blockIdx.y) * kPsUnits;
+  // This workgroup's job; or, of those that share the last jobs, where it begins: `own` is its number among
+  // them, its share the costs [own, own + 1) x quantum, `job_cost` the costs before the job, `t_from` the tile.
+  int j = blockIdx.y, t_from = 0, job_cost = 0;
+  const int own = (int)blockIdx.y - cuts.whole;
+  if (own >= 0) {
+    const int target = own * cuts.quantum;
+    bool found = false;
+    for (int base = cuts.whole; base < cuts.jobs && !found; base += 64) {
+      const int at = base + lane;
+      const int cost = at < cuts.jobs ? kPsCost + job_at(cuts, a.rows, a.chunk_rows, G, at).tiles : 0;
+      int upto = cost;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int before = __shfl_up(upto, off);
+        upto += lane >= off ? before : 0;
+      }
+      const uint64_t behind = __ballot(job_cost + upto > target);
+      if (behind != 0) {
+        const int l = __builtin_ctzll(behind);
+        j = base + l;
+        const int tiles = __builtin_amdgcn_readlane(cost, l) - kPsCost;
+        job_cost += __builtin_amdgcn_readlane(upto, l) - tiles - kPsCost;
+        t_from = cut_at(target - job_cost - kPsCost, tiles);
+        if (t_from == tiles) {
+          job_cost += tiles + kPsCost;
+          t_from = 0;
+          ++j;
+        }
+        found = j < cuts.jobs;
+        break;
+      }
+      job_cost += __builtin_amdgcn_readlane(upto, 63);
+    }
+    if (!found) return;
+  }
+  for (;;) {  // over the jobs of a share
+  j = __builtin_amdgcn_readfirstlane(j);
+  t_from = __builtin_amdgcn_readfirstlane(t_from);
+  job_cost = __builtin_amdgcn_readfirstlane(job_cost);
+  const PsJob job = job_at(cuts, a.rows, a.chunk_rows, G, j);
+  // Its end: within the job, at its end, or further on.
+  int t_to = job.tiles;
+  bool more = false;
+  if (own >= 0) {
+    const int end = (own + 1) * cuts.quantum - kPsCost;  // in tiles of this job: less job_cost
+    t_to = cut_at(end - job_cost, job.tiles);
+    if (t_to == job.tiles && j + 1 < cuts.jobs) {
+      const int next_cost = job_cost + kPsCost + job.tiles;
+      more = cut_at(end - next_cost, job_at(cuts, a.rows, a.chunk_rows, G, j + 1).tiles) > 0;
+    }
+  }
+  const bool cut = t_from > 0 || t_to < job.tiles;
+  const int chunk = job.chunk, m = job.m;
+  const int unit0 = job.i * kPsUnits;
   const int first_row = chunk * a.chunk_rows;
-  const int m = min(a.chunk_rows, a.rows - first_row);
   const int row_begin = unit0 / G * 16;                     // of the workgroup
-  if (row_begin >= m) return;  // (the last chunk of several may be shorter)
   const int row_end = min((unit0 + kPsUnits - 1) / G * 16 + 16, m);
   int row0[CB], head[CB];      // of the column blocks: first row, head
 #pragma unroll
@@ -97,14 +196,9 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   }
 
   const size_t head_at = chunk * a.stage_stride + (size_t)kvh * a.s_pad * kHeadDim;
-  const int last_tile = a.s_pad / kPfKeys - 1;
-  // (a tile past the staging area, asked for ahead and never used, is replaced by the last one)
-  auto tile_at = [&](const uint16_t* base, int t) __attribute__((always_inline)) {
-    return (const pf_bf16x8*)(base + head_at + (size_t)min(t, last_tile) * kPfTileElems);
-  };
   // ---- queries: B operand, lane (qc, g4) holds dims [32 ks + 8 g4, +8) of its column block's row.
   // Their loads do not wait for the selection's length.
-  const int S = min(max(a.sel_len[chunk], 0), a.max_sel_len);
+  const int listed = a.sel_len[chunk];
   uint4 raw[CB][4];
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
@@ -113,17 +207,31 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) raw[cb][ks] = *(const uint4*)(row + 32 * ks);
   }
-  // (behind the queries, which are wanted first: loads return in order)
-  pf_bf16x8 kw[kPfOperands], vw[kPfOperands], k_second[kPfOperands];  // the operands of the next K tile and of the current V^T tile
+  // The tiles pass through LDS.  Package t, what the operands' registers are refilled with in iteration t of the loop
+  // below, is the K tile t + 2 and the V^T tile t + 1: sixteen kilobytes, of which a wavefront asks for four.  The
+  // first operands, the K tiles t_from and t_from + 1 and the V^T tile t_from, are the two packages before the loop's, as
+  // far as they are needed.  (A tile past the staging area, asked for ahead and never used, arrives as zeros.)
+  constexpr uint32_t kBytes = kPsPackage * 16, kPart = kBytes / 2 / kPsWaves;
+  const uint32_t lane16 = 16 * lane, part_at = kPart * wave;
+  const int64_t tiles_bytes = (int64_t)a.s_pad * kHeadDim * 2 - kPart * wave;
   {
-    const pf_bf16x8 *const k0 = tile_at(a.kr, 0), *const k1 = tile_at(a.kr, 1), *const v0 = tile_at(a.vt, 0);
-#pragma unroll
-    for (int i = 0; i < kPfOperands; ++i) kw[i] = k0[64 * i + lane];
-#pragma unroll
-    for (int i = 0; i < kPfOperands; ++i) k_second[i] = k1[64 * i + lane];
-#pragma unroll
-    for (int i = 0; i < kPfOperands; ++i) vw[i] = v0[64 * i + lane];
+    // (behind the queries, which are wanted first: loads return in order)
+    const ps_buffer k_tiles = buffer_of(a.kr + head_at + kPart / 2 * wave, tiles_bytes);
+    const ps_buffer v_tiles = buffer_of(a.vt + head_at + kPart / 2 * wave, tiles_bytes);
+    const uint32_t at = 2 * kPfTileElems * t_from;
+    load_to_lds(part_at + 2 * kBytes, k_tiles, at, lane16);
+    load_to_lds(part_at + 3 * kBytes, k_tiles, at + 2 * kPfTileElems, lane16);
+    load_to_lds(part_at + 3 * kBytes + kBytes / 2, v_tiles, at, lane16);
   }
+  const ps_buffer ask_k = buffer_of(a.kr + head_at + 2 * kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * 2 * kPfTileElems);
+  const ps_buffer ask_v = buffer_of(a.vt + head_at + kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * kPfTileElems);
+  uint32_t ask_at = 2 * kPfTileElems * t_from;  // of the next package to be asked for, in the staging area
+  auto ask_keys = [&](uint32_t buffer) __attribute__((always_inline)) { load_to_lds(part_at + buffer, ask_k, ask_at, lane16); };
+  auto ask_values = [&](uint32_t buffer) __attribute__((always_inline)) {
+    load_to_lds(part_at + buffer + kBytes / 2, ask_v, ask_at, lane16);
+    ask_at += 2 * kPfTileElems;
+  };
+  const int S = __builtin_amdgcn_readfirstlane(min(max(listed, 0), a.max_sel_len));
   const int shift = S - m;  // query row i sits at position shift + i and sees keys <= that
   const bool rope = a.rope_mode == TS_ROPE_LLAMA;
   // (as in the other kernel: without a soft cap the softmax scale and log2(e) go into the query)
@@ -141,34 +249,48 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
         const float pair = (float)(32 * (e >> 3) + 8 * g4 + (e & 7));
         const float freq = a.rope_rcp_scale * exp2f(-pair * (2.0f / kHeadDim) * a.log2_theta);
         sincos_reduced(pos * freq, sn[e >> 3][e & 7], cs[e >> 3][e & 7]);
+        sn[e >> 3][e & 7] *= qs;
+        cs[e >> 3][e & 7] *= qs;
       }
     };
     if (rope) rotation(row0[0]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
+      if (cb == CB / 2) {
+        // All queries are here: the loop's first packages are asked for now, and nothing waits for those with them.
+#pragma unroll
+        for (int late = CB / 2; late < CB; ++late)
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(raw[late][ks].x), "+v"(raw[late][ks].y), "+v"(raw[late][ks].z), "+v"(raw[late][ks].w));
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          ask_keys(t * kBytes);
+          ask_values(t * kBytes);
+        }
+      }
       if (rope && row0[cb] != rotated) rotation(row0[cb]);
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         const uint32_t lw[4] = {raw[cb][ks].x, raw[cb][ks].y, raw[cb][ks].z, raw[cb][ks].w};
         const uint32_t hw[4] = {raw[cb][ks + 2].x, raw[cb][ks + 2].y, raw[cb][ks + 2].z, raw[cb][ks + 2].w};
         uint32_t lp[4], hp[4];
+        if (rope) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          float lo[2] = {bf16_lo(lw[w]), bf16_hi(lw[w])}, hi[2] = {bf16_lo(hw[w]), bf16_hi(hw[w])};
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            if (rope) {
-              const float s = sn[ks][2 * w + x], c = cs[ks][2 * w + x];
-              const float l2 = lo[x] * c - hi[x] * s;
-              hi[x] = hi[x] * c + lo[x] * s;
-              lo[x] = l2;
-            }
-            lo[x] *= qs;
-            hi[x] *= qs;
+          for (int w = 0; w < 4; ++w) {
+            const float lo[2] = {bf16_lo(lw[w]), bf16_hi(lw[w])}, hi[2] = {bf16_lo(hw[w]), bf16_hi(hw[w])};
+            const float* const s = &sn[ks][2 * w];
+            const float* const c = &cs[ks][2 * w];
+            lp[w] = pack_bf16(lo[0] * c[0] - hi[0] * s[0], lo[1] * c[1] - hi[1] * s[1]);
+            hp[w] = pack_bf16(hi[0] * c[0] + lo[0] * s[0], hi[1] * c[1] + lo[1] * s[1]);
           }
-          lp[w] = pack_bf16(lo[0], lo[1]);
-          hp[w] = pack_bf16(hi[0], hi[1]);
+          asm volatile("" : "+v"(lp[0]));  // (two ways, not one with the results picked)
+        } else {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            lp[w] = pack_bf16(bf16_lo(lw[w]) * qs, bf16_hi(lw[w]) * qs);
+            hp[w] = pack_bf16(bf16_lo(hw[w]) * qs, bf16_hi(hw[w]) * qs);
+          }
         }
         qb[cb][ks] = __builtin_bit_cast(pf_bf16x8, make_uint4(lp[0], lp[1], lp[2], lp[3]));
         qb[cb][ks + 2] = __builtin_bit_cast(pf_bf16x8, make_uint4(hp[0], hp[1], hp[2], hp[3]));
@@ -182,7 +304,8 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   // reported a fault, S <= 0; rows at negative positions see no key of any: their sums stay zero, and so does
   // their output)
   const int last_visible = min(S, shift + row_end) - 1;
-  const int n_tiles = S > 0 && last_visible >= 0 ? last_visible / kPfKeys + 1 : 0;
+  const int visible = S > 0 && last_visible >= 0 ? last_visible / kPfKeys + 1 : 0;
+  const int n_tiles = t_to < job.tiles ? min(t_to, visible) : visible;  // (the last piece goes to the end, wherever that is)
   const int masked = max(shift + row_begin + 1, 0) / kPfKeys;  // the first tile that some row must not see whole
   // Running maximum of each column's row: m_run (kNegBig: none yet), minus that as the
   // four-register start value of the logits' accumulators (0 while there is none), and the
@@ -204,25 +327,12 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   }
   const pf_bf16x8 ones = __builtin_bit_cast(pf_bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 
-  // The software pipeline of the other kernel.  Package t, what the operands' registers are refilled with in
-  // iteration t, is the K tile t + 2 and the V^T tile t + 1: sixteen kilobytes, of which a wavefront asks
-  // for four, straight to LDS, in iteration t - 2 (L2 takes 0.6 to 0.85 us, an iteration 0.65), buffer t % 4.
+  // The software pipeline of the other kernel.  Package t is asked for in iteration t - 2 (L2 takes 0.6 to 0.85 us, an
+  // iteration 0.65), to buffer (t - t_from) % 4.
   // Before the barrier in the second half of iteration t a wavefront waits until its part of package t + 1
   // has come, which leaves that of package t + 2 under way, and until all but its last eight
   // reads of LDS are through.  The buffer that is asked for in iteration t had package t - 2: its reads
   // were issued in iteration t - 2 and, everybody's, through at the barrier of iteration t - 1.
-  constexpr uint32_t kBytes = kPsPackage * 16, kPart = kBytes / 2 / kPsWaves;
-  const int64_t tiles_bytes = (int64_t)a.s_pad * kHeadDim * 2 - kPart * wave;
-  const ps_buffer ask_k = buffer_of(a.kr + head_at + 2 * kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * 2 * kPfTileElems);
-  const ps_buffer ask_v = buffer_of(a.vt + head_at + kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * kPfTileElems);
-  uint32_t ask_at = 0;  // of the next package to be asked for, in the staging area
-  const uint32_t lane16 = 16 * lane, part_at = kPart * wave;
-  auto ask_keys = [&](uint32_t buffer) __attribute__((always_inline)) { load_to_lds(part_at + buffer, ask_k, ask_at, lane16); };
-  auto ask_values = [&](uint32_t buffer) __attribute__((always_inline)) {
-    load_to_lds(part_at + buffer + kBytes / 2, ask_v, ask_at, lane16);
-    ask_at += 2 * kPfTileElems;
-  };
-
   // The largest logit of the lane's eight.
   auto largest = [&](const pf_f32x4 (&s)[2]) __attribute__((always_inline)) {
     float mx = max3(s[0][0], s[0][1], s[0][2]);
@@ -292,6 +402,7 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     raise_any = bound();
   };
 
+  pf_bf16x8 kw[kPfOperands], vw[kPfOperands];  // the operands of the next K tile and of the current V^T tile
   // NEXT: there is a tile t + 1.  s_cur: the logits of tile t, which become its
   // weights; s_next: those of tile t + 1.
   uint32_t read_at = 0;  // the buffer of package t (that of package t + 2 is the one after the next)
@@ -366,12 +477,19 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     }
   };
 
-  if (n_tiles > 0) {
+  if (t_from < n_tiles) {
+    pf_bf16x8 k_second[kPfOperands];
     pf_f32x4 s_even[CB][2], s_odd[CB][2];  // the logits of the even and of the odd tiles: [column block][key block]
+    // The first operands, once everybody's parts have come.
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    {
+      const pf_bf16x8* const from = (const pf_bf16x8*)((const char*)ps_lds + lane16 + 2 * kBytes);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      ask_keys(t * kBytes);
-      ask_values(t * kBytes);
+      for (int i = 0; i < kPfOperands; ++i) {
+        kw[i] = from[64 * i];
+        k_second[i] = from[kPsPackage + 64 * i];
+        vw[i] = from[kPsPackage + 64 * (kPfOperands + i)];
+      }
     }
     // the first tile's logits: nothing comes before them
 #pragma unroll
@@ -385,7 +503,7 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
       if (CAP) soft_cap(s_even[cb], cb);
-      if (masked <= 0) mask(0, s_even[cb], cb);
+      if (masked <= t_from) mask(t_from, s_even[cb], cb);
       raise(s_even[cb], cb);
     }
     raise_any = bound();
@@ -395,7 +513,7 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     using Yes = std::true_type;
     using No = std::false_type;
-    int t = 0;
+    int t = t_from;
     for (; t + 2 < n_tiles; t += 2) {
       iteration(t, s_even, s_odd, Yes{});
       iteration(t + 1, s_odd, s_even, Yes{});
@@ -410,24 +528,110 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     }
     iteration(t, s_even, s_odd, No{});
     mfma_settled(o);
-    // What was asked for past the end comes before the space may be another workgroup's.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  // What was asked for past the end comes before the space may be another workgroup's.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // The length of a dense chunk, whose gather is through (nothing here reads it).
-  if (a.new_len && blockIdx.x == 0 && blockIdx.z == 0 && blockIdx.y + 1 == gridDim.y && threadIdx.x == 0)
-    *a.new_len = min(*a.new_len + m, a.len_cap);
-  // o[cb][db][r] = O[query qc][dim 16 db + 4 g4 + r]; the row sum is complete in every lane.
+  if (a.new_len && j == 0 && t_from == 0 && kvh == 0 && threadIdx.x == 0) *a.new_len = min(*a.new_len + m, a.len_cap);
+  bool write = true;
+  if (cut) {
+    // A wavefront leaves what it has of its columns and draws a ticket of the job's; the last to draw adds up the
+    // pieces.  Nobody waits.  (What is left is visible by the time the ticket is drawn: written past the L2, and waited
+    // for.)  Of two pieces the one that finds the other's ticket drawn is not left anywhere.
+    const int first_cut = (job_cost + kPsCost + kPsLeast + cuts.quantum - 1) / cuts.quantum;
+    const int pieces = (job_cost + kPsCost + job.tiles - kPsLeast) / cuts.quantum - first_cut + 2;
+    const int mine = own - first_cut + 1;
+    const int slot0 = kvh * cuts.streams + first_cut - 1;  // of the workgroup with the first piece
+    uint32_t* const ticket = cuts.tickets + slot0 * kPsWaves + wave;
+    auto piece = [&](int p) __attribute__((always_inline)) {
+      return __builtin_amdgcn_make_buffer_rsrc(
+          cuts.pieces + ((size_t)(2 * (slot0 + p) + (p == 0)) * kPsWaves + wave) * kPsPiece, 0, kPsPiece, 0x00020000);
+    };
+    const bool two = pieces == 2;
+    write = two && __hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+    if (!write) {
+      const auto to = piece(mine);
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    const int row = row0[cb] + qc;
-    if (row >= m) continue;
-    const float l = row_sum[cb][0], inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* const to = a.out + ((size_t)(first_row + row) * a.num_heads + head[cb]) * kHeadDim + 4 * g4;
+      for (int cb = 0; cb < CB; ++cb) {
 #pragma unroll
-    for (int db = 0; db < 8; ++db)
-      *(uint2*)(to + 16 * db) = make_uint2(pack_bf16(o[cb][db][0] * inv, o[cb][db][1] * inv),
-                                           pack_bf16(o[cb][db][2] * inv, o[cb][db][3] * inv));
+        for (int db = 0; db < 8; ++db)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ps_u32x4, o[cb][db]), to, lane16, (8 * cb + db) * 1024, kPsCoherent);
+        const ps_u32x2 ml = {__float_as_uint(m_run[cb]), __float_as_uint(row_sum[cb][0])};
+        __builtin_amdgcn_raw_buffer_store_b64(ml, to, 8 * lane, 32 * 1024 + cb * 512, kPsCoherent);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      uint32_t before = 0;
+      if (lane == 0) before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      write = __builtin_amdgcn_readfirstlane((int)before) + 1 == pieces;
+    }
+    if (write) {
+      // Two pieces: the other one to this one, the same sums whichever came last.  More: from the first on.
+      if (!two) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          m_run[cb] = kNegBig;
+          row_sum[cb][0] = 0.f;
+#pragma unroll
+          for (int db = 0; db < 8; ++db) {
+            o[cb][db] = pf_f32x4{0.f, 0.f, 0.f, 0.f};
+            keep_acc(o[cb][db]);
+          }
+        }
+      }
+      for (int p = two ? 1 - mine : 0; p < (two ? 2 - mine : pieces); ++p) {
+#pragma clang fp contract(off)
+        const auto from = piece(p);
+        pf_f32x4 x[CB][8];
+        ps_u32x2 ml[CB];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          ml[cb] = __builtin_bit_cast(ps_u32x2, __builtin_amdgcn_raw_buffer_load_b64(from, 8 * lane, 32 * 1024 + cb * 512, kPsCoherent));
+#pragma unroll
+          for (int db = 0; db < 8; ++db)
+            x[cb][db] = __builtin_bit_cast(pf_f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, lane16, (8 * cb + db) * 1024, kPsCoherent));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const float m_p = __uint_as_float(ml[cb].x), m_new = fmaxf(m_run[cb], m_p);
+          const float e0 = __builtin_amdgcn_exp2f(m_run[cb] - m_new), e1 = __builtin_amdgcn_exp2f(m_p - m_new);
+          m_run[cb] = m_new;
+          row_sum[cb][0] = row_sum[cb][0] * e0 + __uint_as_float(ml[cb].y) * e1;
+#pragma unroll
+          for (int db = 0; db < 8; ++db) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[cb][db][r] = o[cb][db][r] * e0 + x[cb][db][r] * e1;
+            keep_acc(o[cb][db]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  }
+  // o[cb][db][r] = O[query qc][dim 16 db + 4 g4 + r]; the row sum is complete in every lane.  Of two blocks of 16 dims the
+  // even lane groups take the first, the odd ones the second, so that a lane has eight dims in a row.
+  if (write) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      const int row = row0[cb] + qc;
+      const float l = row_sum[cb][0], inv = l > 0.f ? 1.0f / l : 0.f;
+      uint16_t* const to = a.out + ((size_t)(first_row + row) * a.num_heads + head[cb]) * kHeadDim + 16 * (g4 & 1) + 8 * (g4 >> 1);
+#pragma unroll
+      for (int db = 0; db < 8; db += 2) {
+        const auto first = [&](int at) { return pack_bf16(o[cb][db][at] * inv, o[cb][db][at + 1] * inv); };
+        const auto second = [&](int at) { return pack_bf16(o[cb][db + 1][at] * inv, o[cb][db + 1][at + 1] * inv); };
+        const ps_u32x2 x = __builtin_amdgcn_permlane16_swap(first(0), second(0), false, false);
+        const ps_u32x2 y = __builtin_amdgcn_permlane16_swap(first(2), second(2), false, false);
+        if (row < m) *(uint4*)(to + 16 * db) = make_uint4(x.x, y.x, x.y, y.y);
+      }
+    }
+  }
+  if (!more) return;
+  job_cost += kPsCost + job.tiles;
+  t_from = 0;
+  ++j;
+  __syncthreads();  // (everybody is through with the buffers)
   }
 }
 
@@ -435,16 +639,40 @@ int64_t prefill_shared_workgroups(int num_heads, int num_kv_heads, int chunk_row
   return ceil_div(ceil_div(chunk_rows, 16) * (num_heads / num_kv_heads), kPsUnits) * num_kv_heads;
 }
 
-int launch_prefill_shared(const PrefillArgs& a, int chunks, hipStream_t stream) {
-  const int64_t per_head = prefill_shared_workgroups(a.num_heads, a.num_kv_heads, a.chunk_rows) / a.num_kv_heads;
-  const dim3 grid((unsigned)a.num_kv_heads, (unsigned)per_head, (unsigned)chunks);
+PrefillCuts prefill_cuts(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys, void* workspace) {
+  PrefillCuts c{};
+  const int group = num_heads / num_kv_heads, streams = kPsSlots / num_kv_heads;
+  auto workgroups = [&](int m) { return (int)ceil_div(ceil_div(m, 16) * group, kPsUnits); };
+  c.chunks = (int)ceil_div(rows, chunk_rows);
+  c.per_chunk = workgroups(std::min(rows, chunk_rows));
+  c.jobs = (c.chunks - 1) * c.per_chunk + workgroups(rows - (c.chunks - 1) * chunk_rows);
+  c.keys = keys;
+  c.whole = c.jobs;
+  // Shares are of all jobs where these are of very different lengths (2048 rows of a dense chunk, a wave: 62 -> 56 us), and
+  // otherwise of what is left of whole waves and of one wave more (of what is left alone, 0.2 to 0.7 waves: six chunks
+  // of 32 heads 188 us, 183 so).  A last wave that is 0.85 full is left as it is.
+  const int rest = c.jobs % streams, m = std::min(rows, chunk_rows);
+  const bool even = 2 * job_tiles(keys, m, 0, group) >= job_tiles(keys, m, c.per_chunk - 1, group);
+  if (workspace == nullptr || (even && (rest == 0 || 100 * rest >= 85 * streams))) return c;
+  c.streams = streams;
+  c.whole = even ? std::max(c.jobs / streams - 1, 0) * streams : 0;
+  int64_t cost = 0;
+  for (int j = c.whole; j < c.jobs; ++j) cost += kPsCost + job_at(c, rows, chunk_rows, group, j).tiles;
+  c.quantum = (int)std::max<int64_t>(ceil_div(cost, c.streams), kPsCost + 2 * kPsLeast);
+  c.tickets = (uint32_t*)workspace;
+  c.pieces = (char*)workspace + kPsTicketBytes;
+  return c;
+}
+
+int launch_prefill_shared(const PrefillArgs& a, const PrefillCuts& cuts, hipStream_t stream) {
+  const dim3 grid((unsigned)a.num_kv_heads, (unsigned)(cuts.whole + cuts.streams));
   const auto kernel = a.logit_cap > 0.f ? prefill_shared_kernel<true> : prefill_shared_kernel<false>;
   static const hipError_t ok[2] = {
       hipFuncSetAttribute((const void*)prefill_shared_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPsLdsBytes),
       hipFuncSetAttribute((const void*)prefill_shared_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPsLdsBytes)};
   if (ok[0] != hipSuccess || ok[1] != hipSuccess)
     return fail(TS_EHIP, "prefill attention: %zu bytes of LDS refused", kPsLdsBytes);
-  hipLaunchKernelGGL(kernel, grid, dim3(kPsThreads), kPsLdsBytes, stream, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(kPsThreads), kPsLdsBytes, stream, a, cuts);
   return check_launch("prefill_shared_kernel");
 }
 

@@ -391,7 +391,7 @@ struct PromptWorkspace {
   int max_sel, blocks, tokens_per_block;
 };
 
-static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_t max_seq_len) {
+static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_t max_seq_len, bool cut = false) {
   PromptWorkspace w;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -418,6 +418,8 @@ static PromptWorkspace prompt_workspace(const ts_config* cfg, int chunks, int32_
   w.partials = take((size_t)(kPrWorkgroups + ceil_div(kPrGroup, kPrChunks)) * kPrChunks * H * token_groups * sizeof(float2));
   w.stats = take(C * H * sizeof(float2));
   w.topk = take(ts_topk_workspace_bytes(cfg, chunks, max_seq_len));
+  // (what the attention leaves of its jobs that are cut, where nobody reads the selection's any more)
+  if (cut) off = std::max(off, w.votes + align_up(prefill_cut_bytes(), 256));
   w.stage = take(C * ts_prefill_attn_workspace_bytes(cfg, w.max_sel));
   w.total = off;
   return w;
@@ -429,6 +431,15 @@ static int prompt_group(const ts_config* cfg, int32_t rows, int32_t chunk_rows, 
   while (group > 1 && prompt_workspace(cfg, group, max_seq_len).total > kPrBytes)  // (whole sets, while there are any)
     group = group > kPrChunks ? (group - 1) / kPrChunks * kPrChunks : group - 1;
   return group;
+}
+
+// Whether the attention of a call may cut jobs: some launch gains by it, and the bound leaves room for their pieces.
+static bool prompt_cuts(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
+  const int most = prompt_group(cfg, rows, chunk_rows, max_seq_len);
+  const int keys = std::min(cfg->n_init + cfg->top_k + cfg->n_local, max_seq_len);
+  return (prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, rows, rows, keys) ||
+          prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows, keys)) &&
+         prompt_workspace(cfg, most, max_seq_len, true).total <= std::max(kPrBytes, prompt_workspace(cfg, most, max_seq_len).total);
 }
 
 template <int HKV, int NB>
@@ -466,7 +477,8 @@ extern "C" {
 size_t ts_prefill_prompt_workspace_bytes(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
   if (validate_config(cfg) != TS_OK || rows < 1 || chunk_rows < 1 || chunk_rows > kPrRows || max_seq_len < 1)
     return 0;
-  return prompt_workspace(cfg, prompt_group(cfg, rows, chunk_rows, max_seq_len), max_seq_len).total;
+  return prompt_workspace(cfg, prompt_group(cfg, rows, chunk_rows, max_seq_len), max_seq_len,
+                          prompt_cuts(cfg, rows, chunk_rows, max_seq_len)).total;
 }
 
 int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv* kv, const void* q,
@@ -500,6 +512,8 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
   const size_t need = prompt_workspace(cfg, most, bt->max_seq_len).total;
   TS_REQUIRE(workspace_bytes >= need, TS_EWORKSPACE, "ts_prefill_prompt: workspace %zu bytes < required %zu",
              workspace_bytes, need);
+  const bool cut = prompt_cuts(cfg, rows, chunk_rows, bt->max_seq_len) &&
+                   workspace_bytes >= prompt_workspace(cfg, most, bt->max_seq_len, true).total;
 
   const hipStream_t st = (hipStream_t)stream;
   const int q_stride = q_row_stride ? q_row_stride : cfg->num_heads * cfg->head_dim;
@@ -532,7 +546,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     const int64_t row0 = (int64_t)first * chunk_rows;
     const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)std::min(merged, dense - first) * chunk_rows, rows - row0);
     const int32_t bound = bound_after(row0 + n_rows);
-    const PromptWorkspace w = prompt_workspace(cfg, 1, bound);
+    const PromptWorkspace w = prompt_workspace(cfg, 1, bound, cut);
     PrefillDense all{};
     all.table = table;
     all.seq_len = seq_len;
@@ -543,7 +557,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     all.store = rows_at(row0, n_rows);
     TS_TRY(launch_prefill_attn(cfg, (const uint16_t*)q + row0 * q_stride, q_stride, n_rows, k_pool, v_pool, pool_rows,
                                all.sel, all.sel_len, bound, (uint16_t*)out + row0 * cfg->num_heads * cfg->head_dim,
-                               ws + w.stage, w.total - w.stage, st, &all));
+                               ws + w.stage, w.total - w.stage, st, &all, cut ? ws + w.votes : nullptr));
   }
 
   if (dense == chunks) return TS_OK;
@@ -553,7 +567,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     const int64_t row0 = (int64_t)first * chunk_rows;
     const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)here * chunk_rows, rows - row0);
     const int32_t bound = bound_after(row0 + n_rows);
-    const PromptWorkspace w = prompt_workspace(cfg, here, bound);
+    const PromptWorkspace w = prompt_workspace(cfg, here, bound, cut);
     int32_t *const lens = (int32_t*)(ws + w.lens), *const sel = (int32_t*)(ws + w.sel),
                    *const sel_len = (int32_t*)(ws + w.sel_len);
     float *const votes = (float*)(ws + w.votes), *const pooled = cfg->pool_kernel > 0 ? (float*)(ws + w.pooled) : nullptr;
@@ -603,7 +617,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     TS_TRY(launch_prefill_attn_chunks(cfg, q0, q_stride, n_rows, std::min(chunk_rows, n_rows), k_pool, v_pool, pool_rows,
                                       sel, w.max_sel, sel_len, w.max_sel,
                                       (uint16_t*)out + row0 * cfg->num_heads * cfg->head_dim, ws + w.stage,
-                                      w.total - w.stage, st));
+                                      w.total - w.stage, st, nullptr, cut ? ws + w.votes : nullptr));
   }
   return TS_OK;
 }
