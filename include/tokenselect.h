@@ -130,14 +130,18 @@ typedef struct ts_batch {
                                that never arrive, so that every wait gives up
                                after wait_us while all kernels still exit (with a
                                threshold_hint, where there is no rendezvous: the
-                               waits of all but a request's first workgroup)     */
+                               waits of all but a request's first workgroup);
+                               < 0: of the attention, that many splits of each
+                               request and KV head (where it waits: below)       */
   int32_t workspace_clean;  /* ts_decode_layer and ts_decode_step.  1: the caller states that
                                this workspace was last used by one of these calls with
                                the same cfg, batch, max_seq_len (or one of the same
                                ts_decode_layer_layout) and cache == NULL that
                                completed without a give-up, and by nothing since (every
                                such call leaves the selection's counters zero again:
-                               its attention kernel clears them on the side).  The
+                               its attention kernel clears them on the side, and
+                               whoever waited for a word of the attention's that
+                               word).  The
                                layer then starts with the selection kernel, which
                                rotates the query itself (bit-identical to ts_rope_apply);
                                the launch that rotates and clears is not needed.  Honoured

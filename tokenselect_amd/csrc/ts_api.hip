@@ -182,8 +182,11 @@ int64_t ts_decode_layer_layout(const ts_config* cfg, int32_t batch, int32_t max_
   // are cleared (at most kSelMaxChunks); the offsets are multiples of 256.
   const int64_t at = (int64_t)(layer_workspace(cfg, batch, max_seq_len).select_ws / 256);
   const int64_t sync = (int64_t)(s.sync / 256);
-  if (at >= (int64_t)1 << 26 || sync >= (int64_t)1 << 26 || s.clear_chunks >= 1 << 11) return -1;
-  return (at << 37) | (sync << 11) | s.clear_chunks;
+  // (Nor does a call of a length that is attended to whole leave the words of the attention zero that a longer one
+  // waits for.)
+  const int64_t longer = max_seq_len > (int64_t)cfg->n_init + cfg->top_k + cfg->n_local;
+  if (at >= (int64_t)1 << 26 || sync >= (int64_t)1 << 25 || s.clear_chunks >= 1 << 11) return -1;
+  return (at << 37) | (longer << 36) | (sync << 11) | s.clear_chunks;
 }
 
 size_t ts_decode_layer_workspace_bytes(const ts_config* cfg, int32_t batch, int32_t max_seq_len) {
@@ -340,6 +343,28 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   // the query itself; this call's attention kernel clears the counters again.
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;
+  // So does the attention with the words by which its splits are merged (those who read them do), which lie where
+  // separate kernels have their scores and votes: cleared ahead of a first call, and behind
+  // a call that was on the separate kernels though the next one need not be.
+  ZeroSet after = zero;
+  AttnShare share{};
+  if (chunk_rows == 0 && !cache && bt->max_seq_len > w.max_sel) {
+    share = attn_share(cfg, bt->batch, w.max_sel, ws + w.scores, w.topk_ws - w.scores);
+    share.ticks = select_wait_ticks(bt);
+    share.absent = bt->absent_workgroups < 0 ? -bt->absent_workgroups : 0;
+    share.sel_len = sel_len;
+    share.fault_out = (uint32_t*)bt->fault;
+    const ZeroRegion words{(uint32_t*)share.words, (int64_t)(share.bytes / 4), (int)(share.bytes / 4), 1};
+    if (!one_launch) {
+      after = ZeroSet{};
+      if (share.words && select_workspace(cfg, bt->batch, bt->max_seq_len, true).tokens_per_block > 0) after.add(words);
+    } else if (share.words && !starts_with_selection) {
+      // (a launch of its own, once in some 64 steps: a fifth region in the others costs each of them)
+      ZeroSet first;
+      first.add(words);
+      TS_TRY(launch_select_zero(first, (hipStream_t)stream));
+    }
+  }
   // That selection also stores the step's new tokens, and the attention after it writes the lengths
   // (a layer of one request of 32K 38.0 -> 37.1 us, of 128K 71.8 -> 69.2).  Where a new token may be a
   // candidate the store stays ahead.
@@ -418,7 +443,8 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                                w.max_sel, out, ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream);
   return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch,
                      w.max_sel, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream,
-                     plain_decode ? &zero : nullptr, nullptr, commit.batch ? &commit : nullptr);
+                     chunk_rows == 0 && !cache ? &after : nullptr, nullptr, commit.batch ? &commit : nullptr,
+                     one_launch && share.words ? &share : nullptr);
 }
 
 int ts_decode_layer(const ts_config* cfg, const ts_batch* bt, const void* q, const float* q_cos,

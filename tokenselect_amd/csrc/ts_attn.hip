@@ -8,8 +8,11 @@
 // the query to S-1; softmax is online in fp32.  A dense decode step on a per-token or paged
 // table is this one launch (AttnDense): the list is the table itself.  Partial (max, sum, acc) triples are merged
 // across the wavefronts, written with device-coherent stores, and the workgroup that draws
-// the last ticket of its (request, KV head) merges the splits and writes the bf16 output.
+// the last ticket of its (request, KV head) merges the splits and writes the bf16 output; or, in a layer without a selection
+// cache, all of them merge a share each (attn_finish_shared).
 #include <math.h>
+
+#include <algorithm>
 
 #include <mutex>
 #include <type_traits>
@@ -45,6 +48,9 @@ struct AttnArgs {
   int list_shift, list_bound;
   AttnDense step;
   StepCommit commit;  // what the step's store left to be written (batch 0: nothing)
+};
+struct AttnSharedArgs : AttnArgs {
+  AttnShare share;  // the splits merged by everybody
 };
 
 // The last three wavefronts' share of the regions to clear.
@@ -257,8 +263,186 @@ __device__ __forceinline__ bool attn_finish(const AttnArgs& a, int b, int kvh, i
   return true;
 }
 
+// The end of a workgroup where the splits are merged by everybody (AttnShare): each sends its partial sums as
+// words that are not zero, so that each word is its own flag, and then merges, of one head, the columns that are its
+// own share: it asks for them until they have come.  A word has one reader, who leaves it zero again for the next
+// launch.  In place of the acknowledgement of the partials, the ticket and one workgroup that fetches the partials of all
+// there is the time that the last words take.  In-kernel clock, one request, us after the first workgroup's start: 32 heads
+// on 8, tiles done 5.3, partials sent 6.2, then ticket 7.3 (the last 8.3) and end 10.2, or all words seen 7.4 (8.0) and end
+// 8.5.  28 on 4: as before end 10.6; and since more splits cost the merge nothing now, with 64 entries each tiles done 3.9
+// in place of 5.2, sent 5.0, seen 6.4, end 7.4.
+// Nothing of a word is lost: the bits are sent inverted, and the one pattern that would be zero, two NaN that no
+// computation makes, as its neighbour.
+__device__ __forceinline__ uint64_t share_word(float x, float y) {
+  const uint64_t w = ~((uint64_t)__float_as_uint(x) | ((uint64_t)__float_as_uint(y) << 32));
+  return w ? w : 1ull;
+}
+__device__ __forceinline__ float2 shared_pair(uint64_t w) {
+  return make_float2(__uint_as_float(~(uint32_t)w), __uint_as_float(~(uint32_t)(w >> 32)));
+}
+template <int G>
+__device__ __forceinline__ void attn_finish_shared(const AttnSharedArgs& a, int b, int kvh, int split,
+                                                   float (*sm_acc)[G][kHeadDim], float (*sm_m)[G], float (*sm_l)[G],
+                                                   float2 (*sm_sum)[kHeadDim / 2]) {
+  constexpr int kColumns = kHeadDim / 2;  // two adjacent dims each
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ns = a.nsplit, parts = a.share.parts, cols = a.share.cols;
+  const int stride = G * (kColumns + parts);  // words of a split: its sums, then its (max, sum) for every reader
+  uint64_t* const words = a.share.words + (size_t)(b * a.num_kv_heads + kvh) * ns * stride;
+  auto head_of = [&](int reader) { return (int)((uint32_t)reader * a.share.parts_magic >> 16); };
+  __syncthreads();
+  auto merged = [&](int g, float (&sc)[kAttnWaves], float& mm) {
+    mm = kNegBig;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) mm = fmaxf(mm, sm_m[w][g]);
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) sc[w] = __expf(sm_m[w][g] - mm);
+  };
+  if (split >= a.share.absent) {
+    uint64_t* const to = words + (size_t)split * stride;
+    for (int idx = tid; idx < G * kColumns; idx += kAttnThreads) {
+      const int g = idx / kColumns, d = (idx % kColumns) * 2;
+      float sc[kAttnWaves], mm, o0 = 0.f, o1 = 0.f;
+      merged(g, sc, mm);
+#pragma unroll
+      for (int w = 0; w < kAttnWaves; ++w) {
+        o0 += sm_acc[w][g][d] * sc[w];
+        o1 += sm_acc[w][g][d + 1] * sc[w];
+      }
+      __hip_atomic_store(&to[idx], share_word(o0, o1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (tid < G * parts) {  // (at most kAttnShareSplits of them)
+      const int g = head_of(tid);
+      float sc[kAttnWaves], mm, ll = 0.f;
+      merged(g, sc, mm);
+#pragma unroll
+      for (int w = 0; w < kAttnWaves; ++w) ll += sm_l[w][g] * sc[w];
+      __hip_atomic_store(&to[G * kColumns + tid], share_word(mm, ll), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (tid >= 64) {
+    attn_clear_on_the_side(a);
+    if (tid >= kAttnThreads - 64 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) attn_commit(a.commit);
+  }
+  if (split >= G * parts) return;
+
+  // Sixteen lanes have a column each (and sixteen further on, the next), the sixteen groups of them a split each.
+  const int g = head_of(split), first = (split - g * parts) * cols, here = min(cols, kColumns - first);
+  const int c = lane & 15, group = tid >> 4;
+  uint64_t* const sums = words + g * kColumns + first;
+  uint64_t* const ml = words + G * kColumns + split;
+  float m_all = kNegBig, l_all = 0.f;
+  auto collect = [&](auto count_c, auto passes_c) __attribute__((always_inline)) {
+    constexpr int COUNT = decltype(count_c)::value, PASSES = decltype(passes_c)::value;
+    uint64_t w[COUNT][PASSES], x[COUNT];
+    const uint64_t t0 = wall_clock64();
+    bool lost = false;
+    for (uint32_t polls = 1;; ++polls) {
+      bool come = true;
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) {
+        const int mine = group + 16 * i, s = c + 16 * i;
+        x[i] = s < ns ? __hip_atomic_load(&ml[(size_t)s * stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : share_word(kNegBig, 0.f);
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+          w[i][p] = mine < ns && c + 16 * p < here
+                        ? __hip_atomic_load(&sums[(size_t)mine * stride + c + 16 * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : ~0ull;
+      }
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) {
+        come = come && x[i] != 0ull;
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) come = come && w[i][p] != 0ull;
+      }
+      if (__all(come)) break;
+      if ((polls & 15u) == 0 && wall_clock64() - t0 > a.share.ticks) {
+        lost = true;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    // What every wait of a layer does that gives up: the request has no result, and says so.
+    if (lost) {
+      if (lane == 0) {
+        __hip_atomic_store(&a.share.sel_len[b], -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.share.fault_out) __hip_atomic_store(a.share.fault_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) {
+        x[i] = share_word(kNegBig, 0.f);
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) w[i][p] = ~0ull;
+      }
+    }
+    float2 pair[COUNT];
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+      pair[i] = shared_pair(x[i]);
+      m_all = fmaxf(m_all, pair[i].x);
+    }
+    m_all = fmaxf(m_all, dpp_move<kRowRor8>(m_all));
+    m_all = fmaxf(m_all, dpp_move<kRowRor4>(m_all));
+    m_all = fmaxf(m_all, dpp_move<kRowRor2>(m_all));
+    m_all = fmaxf(m_all, dpp_move<kRowRor1>(m_all));
+    float o0[PASSES], o1[PASSES];
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) o0[p] = o1[p] = 0.f;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+      const float e = c + 16 * i < ns ? __expf(pair[i].x - m_all) : 0.f;
+      l_all += pair[i].y * e;
+      const float weight = __shfl(e, (lane & 48) | group);
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p) {
+        const float2 o = shared_pair(w[i][p]);
+        o0[p] += o.x * weight;
+        o1[p] += o.y * weight;
+      }
+    }
+    l_all = row16_sum(l_all);
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      o0[p] += __shfl_xor(o0[p], 16);
+      o1[p] += __shfl_xor(o1[p], 16);
+      o0[p] += __shfl_xor(o0[p], 32);
+      o1[p] += __shfl_xor(o1[p], 32);
+      if (lane < 16) sm_sum[wave][lane + 16 * p] = make_float2(o0[p], o1[p]);
+    }
+    __syncthreads();
+    if (tid < here) {
+      float2 o = sm_sum[0][tid];
+#pragma unroll
+      for (int v = 1; v < kAttnWaves; ++v) {
+        o.x += sm_sum[v][tid].x;
+        o.y += sm_sum[v][tid].y;
+      }
+      *(uint32_t*)(a.out + ((size_t)b * a.num_heads + kvh * G + g) * kHeadDim + 2 * (first + tid)) =
+          (uint32_t)f32_to_bf16(l_all > 0.f ? o.x / l_all : 0.f) | ((uint32_t)f32_to_bf16(l_all > 0.f ? o.y / l_all : 0.f) << 16);
+    }
+    // Zero again, for the next launch (nobody else reads them; the maxima are every wavefront's of this workgroup).
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+      const int mine = group + 16 * i;
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p)
+        if (mine < ns && c + 16 * p < here) sums[(size_t)mine * stride + c + 16 * p] = 0ull;
+    }
+    for (int s = tid; s < ns; s += kAttnThreads) ml[(size_t)s * stride] = 0ull;
+  };
+  auto for_columns = [&](auto count_c) __attribute__((always_inline)) {
+    if (cols <= 16) collect(count_c, std::integral_constant<int, 1>{});
+    else if (cols <= 32) collect(count_c, std::integral_constant<int, 2>{});
+    else collect(count_c, std::integral_constant<int, 4>{});
+  };
+  if (ns <= 16) for_columns(std::integral_constant<int, 1>{});
+  else if (ns <= 32) for_columns(std::integral_constant<int, 2>{});
+  else if (ns <= 48) for_columns(std::integral_constant<int, 3>{});
+  else for_columns(std::integral_constant<int, 5>{});
+}
+
 // ---------------------------------------------------------------------------------------
-// attn_kernel<G, ROPE, CAP, DENSE>: G = H / Hkv query heads per workgroup (1 to 8), on the matrix
+// attn_kernel<G, ROPE, CAP, FORM>: G = H / Hkv query heads per workgroup (1 to 8), on the matrix
 // cores.  A wavefront walks a contiguous quarter of the workgroup's range in tiles of 32
 // tokens.  v_mfma_f32_16x16x32_bf16 three times over:
 //   logits   S[token][head] = K' Q'^T : A = 16 rotated keys x 32 dims (lane (token l%16,
@@ -335,8 +519,13 @@ __device__ __forceinline__ int opaque_zero(uint32_t after) {
 
 // DENSE (AttnDense) is an instantiation of its own: with its few instructions in the one kernel the
 // attention over a list took 1 us more.
-template <int G, bool ROPE, bool CAP, bool DENSE>
-__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_kernel(AttnArgs a) {
+enum AttnForm { kAttnList, kAttnDenseStep, kAttnShared, kAttnSharedHalf };
+template <int G, bool ROPE, bool CAP, int FORM>
+__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_kernel(
+    std::conditional_t<(FORM >= kAttnShared), AttnSharedArgs, AttnArgs> a) {
+  constexpr bool DENSE = FORM == kAttnDenseStep, SHARED = FORM >= kAttnShared;
+  constexpr bool HALF = FORM == kAttnSharedHalf;  // a wavefront has 16 tokens: half a tile is all there is
+  constexpr int TILES = HALF ? 1 : 2;
   static_assert(G >= 1 && G <= 8, "the query heads of a KV head are columns of one tile");
   const int split = blockIdx.x, b = blockIdx.z, kvh = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -356,6 +545,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
   __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ uint32_t s_last;
+  __shared__ float2 sm_sum[SHARED ? kAttnWaves : 1][kHeadDim / 2];
 
   // Column n of the logits: query head n of the KV head (zeros beyond its heads).  Wavefront
   // kb2 < 2 prepares the dims [32 kb2, +32) and their partners 64 further on.
@@ -378,8 +568,8 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
     return ((uint32_t)sel[min(j, a.list_bound - 1) >> a.list_shift] << a.list_shift) +
            (uint32_t)(j & ((1 << a.list_shift) - 1));
   };
-  uint32_t slot_cur[2] = {raw_slot(wlo + n), raw_slot(wlo + 16 + n)};
-  uint32_t slot_next[2] = {raw_slot(wlo + kAttnTile + n), raw_slot(wlo + kAttnTile + 16 + n)};
+  uint32_t slot_cur[2] = {raw_slot(wlo + n), HALF ? 0u : raw_slot(wlo + 16 + n)};
+  uint32_t slot_next[2] = {HALF ? 0u : raw_slot(wlo + kAttnTile + n), HALF ? 0u : raw_slot(wlo + kAttnTile + 16 + n)};
   // A dense step's list is the table and, at the end, the new token, whose row is not in the pool
   // yet: it is read where the caller has it, as slot kNewRow.  (With no new token some word that can
   // be read is loaded in place of its slot.)
@@ -409,7 +599,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   // (from_new: elements from the pool to the new token's row)
   auto request = [&](const uint16_t* pool, int64_t from_new, const uint32_t* slots, uint4 (&dst)[2][4]) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < TILES; ++t) {
       size_t at = (size_t)slots[t] * row_elems;
       if (DENSE && slots[t] == kNewRow) at = (size_t)from_new;
       const uint16_t* row = pool + at + (size_t)kvh * kHeadDim + 8 * qd;
@@ -637,12 +827,16 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
     // (Lowering a wavefront's priority as it advances, which evens out the two workgroups of
     // a CU in the kernel above, evens them out here too and gains nothing: the rows arrive
     // as fast as the memory system delivers them either way.)
-    int j0 = wlo;
-    for (; j0 + kAttnTile < whi; j0 += kAttnTile) tile(j0, std::true_type{}, std::false_type{});
-    if (whi - j0 <= kAttnTile / 2)
-      tile(j0, std::false_type{}, std::true_type{});
-    else
-      tile(j0, std::false_type{}, std::false_type{});
+    if constexpr (HALF) {
+      tile(wlo, std::false_type{}, std::true_type{});
+    } else {
+      int j0 = wlo;
+      for (; j0 + kAttnTile < whi; j0 += kAttnTile) tile(j0, std::true_type{}, std::false_type{});
+      if (whi - j0 <= kAttnTile / 2)
+        tile(j0, std::false_type{}, std::true_type{});
+      else
+        tile(j0, std::false_type{}, std::false_type{});
+    }
   }
 
   l += __shfl_xor(l, 16);
@@ -656,8 +850,12 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
       sm_l[wave][n] = l;
     }
   }
-  const bool last = attn_finish<G>(a, b, kvh, split, sm_acc, sm_m, sm_l, &s_last);
-  if (DENSE) attn_dense_epilogue(a, b, kvh, split * chunk, (split + 1) * chunk, S, new_slot, length, appends, last);
+  if constexpr (SHARED) {
+    attn_finish_shared<G>(a, b, kvh, split, sm_acc, sm_m, sm_l, sm_sum);
+  } else {
+    const bool last = attn_finish<G>(a, b, kvh, split, sm_acc, sm_m, sm_l, &s_last);
+    if (DENSE) attn_dense_epilogue(a, b, kvh, split * chunk, (split + 1) * chunk, S, new_slot, length, appends, last);
+  }
 }
 
 __global__ __launch_bounds__(256) void attn_zero_kernel(uint32_t* tickets, int count) {
@@ -702,12 +900,38 @@ size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
   return attn_workspace(cfg, batch, max_sel_len).total;
 }
 
+// Splits that everybody merges: a workgroup for each as long as all are resident at once (two per CU), with 64
+// entries (16 a wavefront) where each has a CU to itself.  At most kAttnShareSplits, and at least one for each head of the
+// group, whose columns they share; otherwise, or where the words do not fit, none.  us a layer merged by one and by
+// all: one request of 20K, 28 heads on 4 36.1 and 32.3, 32 on 8 33.9 and 32.7 (with 336 workgroups of 64 entries in
+// place of 168 of 128, 33.4), 4 on 1 35.0 and 31.5; two of 8K, 28 on 4 37.9 and 35.3; eight, 14 splits each, 56.1 and
+// 55.5; eight of 32 on 8, seven splits, 68.2 and 68.4: so from ten splits on.
+constexpr int kAttnShareSplits = 80;
+AttnShare attn_share(const ts_config* cfg, int batch, int max_sel_len, void* words, size_t bytes) {
+  AttnShare s{};
+  const int64_t groups = (int64_t)batch * cfg->num_kv_heads, fine = ceil_div(max_sel_len, kAttnChunkUnit);
+  const int G = cfg->num_heads / cfg->num_kv_heads;
+  s.half = groups * fine <= 256;
+  const int64_t want = s.half ? fine : std::min<int64_t>(ceil_div(max_sel_len, kAttnRange), 512 / groups);
+  if (want < 2) return AttnShare{};
+  s.nsplit = (int)ceil_div(max_sel_len, attn_chunk(max_sel_len, (int)want));
+  if (s.nsplit < std::max(G, 10) || s.nsplit > kAttnShareSplits) return AttnShare{};
+  s.parts = std::min(s.nsplit / G, 32);
+  s.parts_magic = 65536u / (uint32_t)s.parts + 1u;
+  s.cols = (int)ceil_div(kHeadDim / 2, s.parts);
+  s.bytes = (size_t)groups * s.nsplit * G * (kHeadDim / 2 + s.parts) * 8;
+  if (s.bytes > bytes) return AttnShare{};
+  s.words = (uint64_t*)words;
+  return s;
+}
+
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
                 int batch, int max_sel_len, void* out, void* workspace, bool tickets_clear,
-                hipStream_t st, const ZeroSet* clear_after, const AttnDense* dense, const StepCommit* commit) {
+                hipStream_t st, const ZeroSet* clear_after, const AttnDense* dense, const StepCommit* commit,
+                const AttnShare* share) {
   const AttnWorkspace w = attn_workspace(cfg, batch, max_sel_len);
-  AttnArgs a;
+  AttnSharedArgs a;
   a.step = AttnDense{};
   a.commit = commit ? *commit : StepCommit{};
   a.list_shift = a.list_bound = 0;
@@ -744,6 +968,8 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
   a.part_ml = (float*)((char*)workspace + w.ml);
   a.tickets = (uint32_t*)((char*)workspace + w.tickets);
   a.out = (uint16_t*)out;
+  a.share = share ? *share : AttnShare{};
+  if (share) a.nsplit = share->nsplit;
 
   if (!tickets_clear) {
     const int count = batch * attn_tickets_per_request(cfg);
@@ -755,8 +981,10 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
   const bool rope = cfg->rope_mode == TS_ROPE_LLAMA, cap = cfg->logit_cap > 0.f;
 #define TS_ATTN_LAUNCH(G_, R_, C_)                                                                    \
   do {                                                                                                \
-    if (dense) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, true>), grid, dim3(kAttnThreads), 0, st, a);        \
-    else hipLaunchKernelGGL((attn_kernel<G_, R_, C_, false>), grid, dim3(kAttnThreads), 0, st, a);             \
+    if (dense) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, kAttnDenseStep>), grid, dim3(kAttnThreads), 0, st, a); \
+    else if (share && share->half) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, kAttnSharedHalf>), grid, dim3(kAttnThreads), 0, st, a); \
+    else if (share) hipLaunchKernelGGL((attn_kernel<G_, R_, C_, kAttnShared>), grid, dim3(kAttnThreads), 0, st, a); \
+    else hipLaunchKernelGGL((attn_kernel<G_, R_, C_, kAttnList>), grid, dim3(kAttnThreads), 0, st, a);         \
   } while (0)
 #define TS_ATTN_CASE(G_)                              \
   case G_:                                            \
