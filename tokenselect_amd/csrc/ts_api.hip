@@ -417,7 +417,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                          (hipStream_t)stream, select_wait_ticks(bt),
                          (uint32_t)(bt->absent_workgroups > 0 ? bt->absent_workgroups : 0),
                          starts_with_selection ? &unrotated : nullptr, commit.batch ? store : nullptr,
-                         commit.notes));
+                         commit.notes, /*late=*/true));
   } else if (vote_group > 0) {
     // With max-pooling the kernel writes the pooled votes (there is no un-pooled copy).
     TS_TRY(launch_score_votes(cfg, bt, qf, k_pool, pool_rows, hit, votes, w.score_stride, topk.ws,

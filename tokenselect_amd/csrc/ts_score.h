@@ -80,6 +80,7 @@ struct ScoreArgs {
   size_t hist_ws_stride;
   uint32_t* fault_word;   // votes-only: the word the kernels after this one consult
   uint32_t absent;        // team members that never arrive (tests of the give-up path)
+  int late;               // a layer's selection: the wide band and the late candidates in place of rounds
   uint32_t* fault_out;    // caller's word, set to 1 when a wait gave up, or NULL
   int32_t* hint;          // [B] threshold bin + 1 of the last selection (0: none), or NULL
   uint64_t* band;         // [B][kBandRows][kSelMaxChunks], zero at launch
@@ -155,6 +156,30 @@ constexpr uint64_t kBandFull = 1ull << 60, kBandSent = 1ull << 62;
 constexpr int kBandReplicas = 8;
 constexpr int kBandRows = kBandReplicas + 2 * kBandBins;  // the counts, then two words of candidates per bin
 __device__ __forceinline__ int band_piece_row(int bin, int half) { return kBandReplicas + 2 * bin + half; }
+// Where the band does not do, words sent later, in the place of words of the band that nobody reads any more
+// (all of a workgroup's candidates but those of the hint's bin and of the bin that was found): bit 63 set and bit 31 not,
+// which no word of candidates of the band is.
+// For a threshold outside the band the counts of kWideBins bins around it, in three words: the lowest eight bins, the four
+// on either side of the band, the highest eight and the tokens above.  (The queries of the next step move the
+// threshold by more than the band in a quarter of the steps of one request of 32K tokens, in half of those behind a
+// prompt of 31600.)  And for a bin that is known but whose candidates were not sent (outside the band, too many for its
+// slots, no hint) these, up to kLateSlots of a workgroup, two to a word; without a hint, when all words of the band are
+// free, behind a word with their number and the tokens above in place of the band's counts.
+constexpr uint64_t kLateMark = 1ull << 63;
+__device__ __forceinline__ bool late_come(uint64_t w) { return (w & (kLateMark | 0x80000000ull)) == kLateMark; }
+constexpr int kWideBins = 32, kWideBelow = 16, kWideWords = 3, kWideReplicas = 2;
+constexpr int kWideBand = kWideBelow - kBandBelow;  // the band's first bin
+__device__ __forceinline__ int wide_bin(int word, int field) {
+  return word == 0 ? field : word == 1 ? kWideBand - 4 + field + (field >= 4 ? kBandBins : 0) : kWideBins - 8 + field;
+}
+static_assert(kWideBand == 12 && kWideBins == 32, "24 bins in three words");
+// Fields of six bits, the last three behind bit 31; then the tokens above, and whether a field is 31.
+__device__ __forceinline__ int wide_field_at(int field) { return field * kBandCountBits + (field >= 5 ? 2 : 0); }
+constexpr int kWideOverAt = 50;
+constexpr uint64_t kWideFull = 1ull << 62;
+constexpr int kWideFirst = kBandReplicas;  // their rows: those of the first three bins' candidates
+constexpr int kLateSlots = 24, kLateSlotsWide = 16;
+constexpr int kLateFewAt = 16;  // of the word without a hint: below it the tokens above
 constexpr int kSelCounterWords = kSelListCount + kSelListParts * 32;
 
 // Workgroups of one request the workspace of ts_select is laid out for (the device keeps
@@ -239,6 +264,6 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
                   int64_t vote_stride, void* workspace, uint32_t* clear, int clear_per_req,
                   hipStream_t stream, uint64_t wait_ticks, uint32_t absent,
                   const UnrotatedQuery* unrotated = nullptr, const StepStore* append = nullptr,
-                  int4* notes = nullptr);
+                  int4* notes = nullptr, bool late = false);
 
 }  // namespace ts

@@ -1055,11 +1055,17 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // Over all workgroups: [0..3] the counts of two bins each, [4] the tokens above the band, [8] how many
     // bins from the lowest on hold one without room for its count, [9] a bin's candidates do not fit.
     __shared__ uint32_t band_sum[kBandBins + 2];
+    // Per bin of the wide band, and above them all; over all workgroups two bins each, the tokens above, and how many
+    // bins from the lowest on hold one without room for its count.
+    __shared__ uint32_t wide_count[kWideBins + 1], wide_sum[4 * kWideWords + 2];
+    static_assert(kLateSlots <= kBandBins * kBandSlots, "the late candidates take the place of the band's");
     for (int i = tid; i < kTopkBins; i += 256) lh[i] = 0u;
     if (tid < 16) scratch[tid] = 0u;
     if (tid < kBandBins * kBandSlots) band_lds[tid / kBandSlots][tid % kBandSlots] = 0u;
     if (tid <= kBandBins) band_count[tid] = 0u;
     if (tid < kBandBins + 2) band_sum[tid] = 0u;
+    if (tid <= kWideBins) wide_count[tid] = 0u;
+    if (tid < 4 * kWideWords + 2) wide_sum[tid] = 0u;
     TS_MARK(1);
     __syncthreads();  // scores, own maxima and the cleared histogram are in LDS for all
     TS_MARK(2);
@@ -1356,6 +1362,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     };
     bool found = false;     // the threshold bin is known
     bool from_band = false; // and its candidates are in `entries`
+    // Where it is known and they are not: what each workgroup holds in it, and above it.
+    uint32_t late_few[kBandLoads], late_above[kBandLoads];
+    int late_from = 0, late_skip0 = kBandBins, late_skip1 = kBandBins;  // the bins whose words are free: from the first, less two
     // The candidates that the last step ranks, in any order (in the place of the histogram's
     // last bins: with a hint it has not been counted yet, else it has been searched by then).
     uint2* const entries = (uint2*)(lh + kTopkBins - 2 * kSelListCap);
@@ -1471,6 +1480,130 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
           // (every candidate of the bin is in a slot: the count is that of the histogram)
           if (from_band && scratch[15] != in_bin0 && tid == 0) raise_fault(lp.sync);
         }
+        if (__builtin_expect(!from_band, 0)) {
+          late_skip0 = min(d0, kBandBelow);
+          late_skip1 = d0 == kBandBelow ? kBandBins : max(d0, kBandBelow);
+#pragma unroll
+          for (int r = 0; r < kBandLoads; ++r) {
+            late_few[r] = band_here(r, d0);
+            late_above[r] = (uint32_t)(band_counts[r] >> kBandOverAt) & kBandOverMask;
+            for (int d = d0 + 1; d < kBandBins; ++d) late_above[r] += band_here(r, d);
+          }
+        }
+      }
+    }
+    if (__builtin_expect(a.late && banded && !found && (band_sum[kBandBins / 2] >= k || band_sum[kBandBins] == 0u), 0)) {
+      // Not in the band: the counts of the bins around it, of every workgroup, on the side where it is.  (The tokens of
+      // the band are known where it has room for them all.)
+      const bool higher = band_sum[kBandBins / 2] >= k;
+      for (int i = tid; i < count; i += 256) {
+        const int e = (int)key_bin0(key_of(i)) - (hint_bin - kWideBelow);
+        if (e >= 0 && (higher ? e >= kWideBand + kBandBins : e < kWideBand)) atomicAdd(&wide_count[min(e, kWideBins)], 1u);
+      }
+      __syncthreads();
+      if (wave == 0 && lane < kWideWords * kWideReplicas) {
+        const int word = lane / kWideReplicas;
+        uint64_t fields = kLateMark | (word == 2 ? (uint64_t)wide_count[kWideBins] << kWideOverAt : 0ull);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+          const uint32_t n = wide_count[wide_bin(word, d)];
+          fields |= (uint64_t)min(n, kBandCountMost) << wide_field_at(d);
+          fields |= n >= kBandCountMost ? kWideFull : 0ull;
+        }
+        store_coherent(&band[(size_t)(kWideFirst + lane) * kSelMaxChunks + chunk], fields);
+      }
+      uint64_t sent[kBandLoads][kWideWords];
+      const uint64_t* from = &band[(size_t)(kWideFirst + team.index % kWideReplicas) * kSelMaxChunks];
+      until_come([&]() {
+        bool come = true;
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r)
+#pragma unroll
+          for (int w = 0; w < kWideWords; ++w) {
+            const int at = tid + 256 * r;
+            sent[r][w] = at < req_chunks ? load_coherent(&from[(size_t)w * kWideReplicas * kSelMaxChunks + at]) : 0ull;
+            come = come && (at >= req_chunks || late_come(sent[r][w]));
+          }
+        return come;
+      });
+      auto field = [&](int r, int w, int d) { return (uint32_t)(sent[r][w] >> wide_field_at(d)) & kBandCountMask; };
+#pragma unroll
+      for (int w = 0; w < kWideWords; ++w) {
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r)
+          if (__builtin_expect((sent[r][w] & kWideFull) != 0ull, 0))
+            for (int d = 0; d < 8; ++d)
+              if (field(r, w, d) == kBandCountMost) atomicMax(&wide_sum[4 * kWideWords + 1], (uint32_t)wide_bin(w, d) + 1u);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint32_t two = 0;
+#pragma unroll
+          for (int r = 0; r < kBandLoads; ++r) two += field(r, w, 2 * j) | field(r, w, 2 * j + 1) << 16;
+          two = row16_total(two);
+          if ((lane & 15) == 0) atomicAdd(&wide_sum[4 * w + j], two);
+        }
+      }
+      {
+        uint32_t over = 0;
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r) over += (uint32_t)(sent[r][2] >> kWideOverAt) & kBandOverMask;
+        over = row16_total(over);
+        if ((lane & 15) == 0) atomicAdd(&wide_sum[4 * kWideWords], over);
+      }
+      __syncthreads();
+      int e0 = -1;
+      uint32_t run = higher ? wide_sum[4 * kWideWords] : band_sum[kBandBins / 2];
+      uint32_t above[kBandLoads];
+#pragma unroll
+      for (int r = 0; r < kBandLoads; ++r) {
+        above[r] = higher ? (uint32_t)(sent[r][2] >> kWideOverAt) & kBandOverMask
+                          : (uint32_t)(band_counts[r] >> kBandOverAt) & kBandOverMask;
+        late_few[r] = late_above[r] = 0u;
+      }
+      auto search = [&](int w, int d) {
+        const uint32_t here = wide_sum[4 * w + d / 2] >> (16 * (d & 1)) & 0xffffu;
+        if (e0 >= 0) return;
+        const bool in = run < k && run + here >= k;
+        if (in) {
+          e0 = wide_bin(w, d);
+          in_bin0 = here;
+        } else {
+          run += here;
+        }
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r) {
+          const uint32_t own = field(r, w, d);
+          if (in) {
+            late_few[r] = own;
+            late_above[r] = above[r];
+          }
+          above[r] += own;
+        }
+      };
+      if (higher) {
+#pragma unroll
+        for (int d = 7; d >= 0; --d) search(2, d);
+#pragma unroll
+        for (int d = 7; d >= 4; --d) search(1, d);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kBandBins / 2; ++j) run += (band_sum[j] & 0xffffu) + (band_sum[j] >> 16);
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r)
+#pragma unroll
+          for (int d = 0; d < kBandBins; ++d) above[r] += band_here(r, d);
+#pragma unroll
+        for (int d = 3; d >= 0; --d) search(1, d);
+#pragma unroll
+        for (int d = 7; d >= 0; --d) search(0, d);
+      }
+      // (as in the band: above every bin without room)
+      if (e0 >= (int)wide_sum[4 * kWideWords + 1] && hint_bin - kWideBelow + e0 >= 0) {
+        found = true;
+        t0 = (uint32_t)(hint_bin - kWideBelow + e0);
+        above0 = run;
+        late_from = kWideWords * kWideReplicas / 2;  // (the others are the words just read)
+        late_skip0 = kBandBelow;
       }
     }
     if (banded && !found) {  // the hint was of no use: the histogram is needed after all
@@ -1583,7 +1716,126 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
       if (tid < 8) scratch[8 + tid] = 0u;
       __syncthreads();
     }
-    if (listed && !from_band) {
+    // The candidates of the threshold bin, wherever it was found, from word to word as those of the band: nobody meets.
+    // (A hint that failed altogether leaves no words free, a bin that was cut further no counts, and more candidates than
+    // kLateSlots of some workgroup no room.  Of pooled votes, whose peaks are as many equal keys as the window, a workgroup
+    // has more than one look brings: window 15, one request of 100K tokens 64.1 us a layer met, 64.6 so.)  us a layer,
+    // with two rounds, or one, met for in place of the wide band and this: eight requests of 3-16K 92.4 -> 88.0 (their
+    // bins are crowded, and whoever fails keeps all waiting), one of 32K 32.6 -> 32.2 in the mean over hints that hold and
+    // some that do not, four of 64K with a selection cache 75.4 -> 74.2, a chunk at 128K 100.0 -> 99.5.
+    // (Both behind __builtin_expect: in line with the path of a hint that holds they cost that 0.3 us.)
+    constexpr int kLatePool = 8;
+    bool late = a.late && a.pool_kernel <= kLatePool && listed && !from_band && (banded ? found && shift == 21 : true) && lp.tokens_per_block <= kBandMaxTokens &&
+                req_chunks <= kSelMaxChunks / 2;
+    if (__builtin_expect(late, 0)) {
+      const uint32_t slots = late_from ? (uint32_t)kLateSlotsWide : (uint32_t)kLateSlots;
+      auto piece_row = [&](int p) {  // of a workgroup's p-th word of candidates
+        int bin = late_from + (p >> 1);
+        bin += bin >= late_skip0 ? 1 : 0;
+        bin += bin >= late_skip1 ? 1 : 0;
+        return (size_t)band_piece_row(bin, p & 1) * kSelMaxChunks;
+      };
+      uint32_t* const own = &band_lds[0][0];
+      uint32_t above = 0;
+      for (int base = 0; base < count; base += 256) {
+        const int i = base + tid;
+        const uint32_t key = i < count ? key_of(i) : 0u;
+        const uint32_t top = key >> shift;
+        above += (i < count && top > prefix) ? 1u : 0u;
+        if (i < count && top == prefix) {
+          const uint32_t at = atomicAdd(&scratch[9], 1u);
+          if (at < slots) own[at] = ((key & 0x1fffffu) << 10) | (uint32_t)i;
+        }
+      }
+      if (!banded) {
+        above = wave_total(above);
+        if (lane == 0 && above) atomicAdd(&scratch[8], above);
+      }
+      if (tid == 0) band_sum[kBandBins + 1] = 0u;
+      __syncthreads();
+      TS_MARK(10);
+      if (wave == 0) {
+        const uint32_t n = scratch[9];
+        if (2u * (uint32_t)lane < n && n <= slots)
+          store_coherent(&band[piece_row(lane) + chunk],
+                         kLateMark | (uint64_t)own[2 * lane] | ((uint64_t)(2u * (uint32_t)lane + 1u < n ? own[2 * lane + 1] : 0u) << 32));
+        if (!banded && lane < kBandReplicas)
+          store_coherent(&band[(size_t)lane * kSelMaxChunks + chunk], kBandSent | ((uint64_t)n << kLateFewAt) | (uint64_t)scratch[8]);
+      }
+      if (!banded) {
+        uint64_t sent[kBandLoads];
+        const uint64_t* const words = &band[(size_t)(team.index % kBandReplicas) * kSelMaxChunks];
+        until_come([&]() {
+          bool come = true;
+#pragma unroll
+          for (int r = 0; r < kBandLoads; ++r) {
+            const int at = tid + 256 * r;
+            sent[r] = at < req_chunks ? load_coherent(&words[at]) : 0ull;
+            come = come && (at >= req_chunks || sent[r] != 0ull);
+          }
+          return come;
+        });
+#pragma unroll
+        for (int r = 0; r < kBandLoads; ++r) {
+          late_few[r] = (uint32_t)(sent[r] >> kLateFewAt) & 0xffffu;
+          late_above[r] = (uint32_t)sent[r] & 0xffffu;
+        }
+      }
+      uint32_t before = 0;
+#pragma unroll
+      for (int r = 0; r < kBandLoads; ++r) {
+        const uint32_t fits = late_few[r] <= slots ? late_few[r] : 0u;
+        before += tid + 256 * r < chunk ? late_above[r] : 0u;
+        if (late_few[r] != fits) band_sum[kBandBins + 1] = 1u;
+        const uint32_t from = (uint32_t)(tid + 256 * r) * (uint32_t)lp.tokens_per_block;
+        const uint64_t low = (1ull << lane) - 1ull;
+        constexpr int kBatch = 4;  // words asked for together: eight candidates
+        static_assert(kLateSlots % (2 * kBatch) == 0 && kLateSlotsWide % (2 * kBatch) == 0, "whole batches");
+        for (uint32_t p0 = 0; 2 * p0 < slots && __any(fits > 2 * p0); p0 += kBatch) {
+          uint64_t piece[kBatch];
+          until_come([&]() {
+            bool come = true;
+#pragma unroll
+            for (int p = 0; p < kBatch; ++p)
+              piece[p] = fits > 2 * (p0 + p) ? load_coherent(&band[piece_row((int)p0 + p) + tid + 256 * r]) : kLateMark;
+#pragma unroll
+            for (int p = 0; p < kBatch; ++p) come = come && late_come(piece[p]);
+            return come;
+          });
+          const uint32_t have = fits > 2 * p0 ? min(fits - 2 * p0, 2u * kBatch) : 0u;
+          // (places for the wavefront's candidates with one addition)
+          uint32_t total = 0, mine = 0;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint64_t bits = __ballot(have >> i & 1u);
+            total += (uint32_t)__popcll(bits) << i;
+            mine += (uint32_t)__popcll(bits & low) << i;
+          }
+          uint32_t at = 0;
+          if (lane == 0) at = atomicAdd(&scratch[15], total);
+          at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + mine;
+#pragma unroll
+          for (uint32_t h = 0; h < 2 * kBatch; ++h) {
+            const uint32_t packed = (uint32_t)(piece[h >> 1] >> (32 * (h & 1)));
+            if (h < have && at + h < (uint32_t)kSelListCap)
+              entries[at + h] = make_uint2((t0 << 21) | ((packed >> 10) & 0x1fffffu), from + (packed & 1023u));
+          }
+        }
+      }
+      before = wave_total(before);
+      if (lane == 0 && before) atomicAdd(&scratch[10], before);
+      __syncthreads();
+      TS_MARK(11);
+      late = band_sum[kBandBins + 1] == 0u;
+      // (every candidate is there: the count is the one that was found)
+      if (late && scratch[15] != in_bin && tid == 0) raise_fault(lp.sync);
+      if (!late) {  // (everybody has seen the same words)
+        __syncthreads();
+        if (tid < 8) scratch[8 + tid] = 0u;
+        __syncthreads();
+      }
+    }
+    if (listed && !from_band && !late) {
       // Last round, short form: the candidates of the threshold bin are appended to
       // the list (in kSelListParts parts with a counter each, a wavefront reserving
       // its entries with one add), and every workgroup publishes how many of its
@@ -2238,7 +2490,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
                   int32_t* sel_pos, int64_t sel_stride, int32_t* sel_len, float* votes,
                   int64_t vote_stride, void* workspace, uint32_t* clear, int clear_per_req,
                   hipStream_t stream, uint64_t wait_ticks, uint32_t absent,
-                  const UnrotatedQuery* unrotated, const StepStore* append, int4* notes) {
+                  const UnrotatedQuery* unrotated, const StepStore* append, int4* notes, bool late) {
   // (requests may be skipped when the caller brings hit flags: the selection cache)
   const SelectWorkspace w = select_workspace(cfg, bt->batch, bt->max_seq_len, false, hit != nullptr);
   TS_REQUIRE(w.tokens_per_block > 0, TS_ESHAPE, "fused selection: unsupported shape");
@@ -2280,6 +2532,7 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
   a.clear_per_req = clear_per_req;
   a.spin_ticks = wait_ticks;
   a.absent = absent;
+  a.late = late ? 1 : 0;
   a.fault_out = bt->fault;
   a.pool_kernel = cfg->pool_kernel;
   a.pool_votes = (float*)(ws + w.pool_votes);
