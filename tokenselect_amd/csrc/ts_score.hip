@@ -1492,7 +1492,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         }
       }
     }
-    if (__builtin_expect(a.late && banded && !found && (band_sum[kBandBins / 2] >= k || band_sum[kBandBins] == 0u), 0)) {
+    constexpr int kLatePool = 8;  // (wider windows fill fields and words too often: 9 of 0.9-7.5K, 58, 51.4 us a layer, and 49.1 met)
+    if (__builtin_expect(a.late && a.pool_kernel <= kLatePool && banded && !found && (band_sum[kBandBins / 2] >= k || band_sum[kBandBins] == 0u), 0)) {
       // Not in the band: the counts of the bins around it, of every workgroup, on the side where it is.  (The tokens of
       // the band are known where it has room for them all.)
       const bool higher = band_sum[kBandBins / 2] >= k;
@@ -1724,7 +1725,6 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // bins are crowded, and whoever fails keeps all waiting), one of 32K 32.6 -> 32.2 in the mean over hints that hold and
     // some that do not, four of 64K with a selection cache 75.4 -> 74.2, a chunk at 128K 100.0 -> 99.5.
     // (Both behind __builtin_expect: in line with the path of a hint that holds they cost that 0.3 us.)
-    constexpr int kLatePool = 8;
     bool late = a.late && a.pool_kernel <= kLatePool && listed && !from_band && (banded ? found && shift == 21 : true) && lp.tokens_per_block <= kBandMaxTokens &&
                 req_chunks <= kSelMaxChunks / 2;
     if (__builtin_expect(late, 0)) {
