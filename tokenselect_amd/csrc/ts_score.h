@@ -80,7 +80,6 @@ struct ScoreArgs {
   size_t hist_ws_stride;
   uint32_t* fault_word;   // votes-only: the word the kernels after this one consult
   uint32_t absent;        // team members that never arrive (tests of the give-up path)
-  int late;               // a layer's selection: the wide band and the late candidates in place of rounds
   uint32_t* fault_out;    // caller's word, set to 1 when a wait gave up, or NULL
   int32_t* hint;          // [B] threshold bin + 1 of the last selection (0: none), or NULL
   uint64_t* band;         // [B][kBandRows][kSelMaxChunks], zero at launch

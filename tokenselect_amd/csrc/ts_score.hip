@@ -90,6 +90,10 @@ constexpr int kScoreDirect = 0, kScoreTiled = 1, kScoreFused = 2;
 // The fused kernel's votes-only form (phases of requests in one launch): a kernel of its
 // own, so that the single-launch selection does not carry the bookkeeping.
 constexpr int kScorePacked = 3;
+// kScoreFused that meets wherever the band does not do: an instantiation of its own for ts_select by itself and for votes
+// pooled over wide windows, where what is sent late does not pay (kLatePool).  With that code in it, never taken, a
+// chunk of 250 rows on 24K tokens with a window of 124 took 64.2 us a layer, and 63.7 so (63.4 before there was such code).
+constexpr int kScoreMeeting = 4;
 constexpr int kMaxHeads = 128;
 
 // What a workgroup of the fused kernel serves: the whole launch, or one phase of a
@@ -650,7 +654,8 @@ template <int HKV, int G, bool OUT_BF16, int MODE>
 __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a) {
   extern __shared__ float stage[];  // tiled / fused: [tiles of the workgroup][tile_stride]
   constexpr bool TILED = MODE != kScoreDirect;
-  constexpr bool FUSED = MODE == kScoreFused || MODE == kScorePacked;
+  constexpr bool LATE = MODE == kScoreFused;
+  constexpr bool FUSED = LATE || MODE == kScoreMeeting || MODE == kScorePacked;
   constexpr bool PACKED = MODE == kScorePacked;
   constexpr int TG = 8 / HKV;
   constexpr int UNITS = 8;
@@ -1057,15 +1062,15 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     __shared__ uint32_t band_sum[kBandBins + 2];
     // Per bin of the wide band, and above them all; over all workgroups two bins each, the tokens above, and how many
     // bins from the lowest on hold one without room for its count.
-    __shared__ uint32_t wide_count[kWideBins + 1], wide_sum[4 * kWideWords + 2];
+    __shared__ uint32_t wide_count[LATE ? kWideBins + 1 : 1], wide_sum[LATE ? 4 * kWideWords + 2 : 1];
     static_assert(kLateSlots <= kBandBins * kBandSlots, "the late candidates take the place of the band's");
     for (int i = tid; i < kTopkBins; i += 256) lh[i] = 0u;
     if (tid < 16) scratch[tid] = 0u;
     if (tid < kBandBins * kBandSlots) band_lds[tid / kBandSlots][tid % kBandSlots] = 0u;
     if (tid <= kBandBins) band_count[tid] = 0u;
     if (tid < kBandBins + 2) band_sum[tid] = 0u;
-    if (tid <= kWideBins) wide_count[tid] = 0u;
-    if (tid < 4 * kWideWords + 2) wide_sum[tid] = 0u;
+    if (LATE && tid <= kWideBins) wide_count[tid] = 0u;
+    if (LATE && tid < 4 * kWideWords + 2) wide_sum[tid] = 0u;
     TS_MARK(1);
     __syncthreads();  // scores, own maxima and the cleared histogram are in LDS for all
     TS_MARK(2);
@@ -1480,7 +1485,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
           // (every candidate of the bin is in a slot: the count is that of the histogram)
           if (from_band && scratch[15] != in_bin0 && tid == 0) raise_fault(lp.sync);
         }
-        if (__builtin_expect(!from_band, 0)) {
+        if (LATE && __builtin_expect(!from_band, 0)) {
           late_skip0 = min(d0, kBandBelow);
           late_skip1 = d0 == kBandBelow ? kBandBins : max(d0, kBandBelow);
 #pragma unroll
@@ -1492,8 +1497,7 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
         }
       }
     }
-    constexpr int kLatePool = 8;  // (wider windows fill fields and words too often: 9 of 0.9-7.5K, 58, 51.4 us a layer, and 49.1 met)
-    if (__builtin_expect(a.late && a.pool_kernel <= kLatePool && banded && !found && (band_sum[kBandBins / 2] >= k || band_sum[kBandBins] == 0u), 0)) {
+    if (LATE && __builtin_expect(banded && !found && (band_sum[kBandBins / 2] >= k || band_sum[kBandBins] == 0u), 0)) {
       // Not in the band: the counts of the bins around it, of every workgroup, on the side where it is.  (The tokens of
       // the band are known where it has room for them all.)
       const bool higher = band_sum[kBandBins / 2] >= k;
@@ -1725,9 +1729,9 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // bins are crowded, and whoever fails keeps all waiting), one of 32K 32.6 -> 32.2 in the mean over hints that hold and
     // some that do not, four of 64K with a selection cache 75.4 -> 74.2, a chunk at 128K 100.0 -> 99.5.
     // (Both behind __builtin_expect: in line with the path of a hint that holds they cost that 0.3 us.)
-    bool late = a.late && a.pool_kernel <= kLatePool && listed && !from_band && (banded ? found && shift == 21 : true) && lp.tokens_per_block <= kBandMaxTokens &&
+    bool late = LATE && listed && !from_band && (banded ? found && shift == 21 : true) && lp.tokens_per_block <= kBandMaxTokens &&
                 req_chunks <= kSelMaxChunks / 2;
-    if (__builtin_expect(late, 0)) {
+    if (LATE && __builtin_expect(late, 0)) {
       const uint32_t slots = late_from ? (uint32_t)kLateSlotsWide : (uint32_t)kLateSlots;
       auto piece_row = [&](int p) {  // of a workgroup's p-th word of candidates
         int bin = late_from + (p >> 1);
@@ -2165,11 +2169,12 @@ static int launch_score(int hkv, int group, const ScoreArgs& a, dim3 grid, hipSt
 }
 
 // The fused kernel of a head shape (its packed votes-only form), or NULL.
-static const void* fused_kernel_of(int hkv, int group, bool packed = false) {
+static const void* fused_kernel_of(int hkv, int group, int mode) {
 #define TS_SCORE_CASE(HKV_, G_)                                                        \
   if (hkv == HKV_ && group == G_)                                                      \
-    return packed ? (const void*)&score_kernel<HKV_, G_, false, kScorePacked>          \
-                  : (const void*)&score_kernel<HKV_, G_, false, kScoreFused>;
+    return mode == kScorePacked  ? (const void*)&score_kernel<HKV_, G_, false, kScorePacked>  \
+         : mode == kScoreMeeting ? (const void*)&score_kernel<HKV_, G_, false, kScoreMeeting> \
+                                 : (const void*)&score_kernel<HKV_, G_, false, kScoreFused>;
 #define TS_SCORE_ROW(HKV_) \
   TS_SCORE_CASE(HKV_, 1) TS_SCORE_CASE(HKV_, 2) TS_SCORE_CASE(HKV_, 3) TS_SCORE_CASE(HKV_, 4) \
       TS_SCORE_CASE(HKV_, 5) TS_SCORE_CASE(HKV_, 6) TS_SCORE_CASE(HKV_, 7) TS_SCORE_CASE(HKV_, 8)
@@ -2207,13 +2212,13 @@ SeparateKernelsScope::SeparateKernelsScope(bool on) : was(g_separate_call) {
 }
 SeparateKernelsScope::~SeparateKernelsScope() { g_separate_call = was; }
 
-// Workgroups of the fused kernel that the current device keeps resident at once (0: the
+// Workgroups of a fused kernel that the current device keeps resident at once (0: the
 // shape has no fused kernel, or the runtime refused); depends on the kernel only.
-static int fused_capacity(const ts_config* cfg, bool packed, bool large) {
-  const void* fn = fused_kernel_of(cfg->num_kv_heads, cfg->num_heads / cfg->num_kv_heads, packed);
+static int kernel_capacity(const void* fn, bool large) {
   if (!fn) return 0;
   struct Entry { const void* fn; int device; bool large; int capacity; };
-  static thread_local Entry memo[16] = {};
+  constexpr int kMemo = 24;  // four shapes
+  static thread_local Entry memo[kMemo] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return 0;
   int capacity = 0;
@@ -2235,9 +2240,16 @@ static int fused_capacity(const ts_config* cfg, bool packed, bool large) {
     capacity = per_cu * cus;
     if (capacity <= 0) return 0;
     static thread_local int next = 0;
-    memo[next++ % 16] = Entry{fn, device, large, capacity};
+    memo[next++ % kMemo] = Entry{fn, device, large, capacity};
   }
   return capacity;
+}
+// ... of the kernel that a call may turn out to launch: of a selection's two forms the one that fewer fit of.
+static int fused_capacity(const ts_config* cfg, bool packed, bool large) {
+  const int hkv = cfg->num_kv_heads, group = cfg->num_heads / cfg->num_kv_heads;
+  if (packed) return kernel_capacity(fused_kernel_of(hkv, group, kScorePacked), large);
+  return std::min(kernel_capacity(fused_kernel_of(hkv, group, kScoreFused), large),
+                  kernel_capacity(fused_kernel_of(hkv, group, kScoreMeeting), large));
 }
 
 // With max-pooling a workgroup gathers its votes and kernel - 1 neighbours into the LDS
@@ -2532,12 +2544,13 @@ int launch_select(const ts_config* cfg, const ts_batch* bt, const void* qf, cons
   a.clear_per_req = clear_per_req;
   a.spin_ticks = wait_ticks;
   a.absent = absent;
-  a.late = late ? 1 : 0;
   a.fault_out = bt->fault;
   a.pool_kernel = cfg->pool_kernel;
   a.pool_votes = (float*)(ws + w.pool_votes);
   a.pool_stride = w.pool_stride;
-  const void* fn = fused_kernel_of(cfg->num_kv_heads, cfg->num_heads / cfg->num_kv_heads);
+  constexpr int kLatePool = 8;  // (wider windows fill fields and words too often: 9 of 0.9-7.5K, 58, 51.4 us a layer, and 49.1 met)
+  const void* fn = fused_kernel_of(cfg->num_kv_heads, cfg->num_heads / cfg->num_kv_heads,
+                                   late && cfg->pool_kernel <= kLatePool ? kScoreFused : kScoreMeeting);
   // One-dimensional: the kernel deals these workgroups over the requests that select.
   a.batch = bt->batch;
   const dim3 grid((unsigned)(w.blocks_per_req * bt->batch), 1u);
@@ -2646,7 +2659,7 @@ int launch_score_votes(const ts_config* cfg, const ts_batch* bt, const void* qf,
   // Offsets of the pieces: those of the whole batch's workspace, whatever the launches.
   const SelectWorkspace all = select_workspace(cfg, bt->batch, bt->max_seq_len, true);
   char* ws = (char*)workspace;
-  const void* fn = fused_kernel_of(cfg->num_kv_heads, cfg->num_heads / cfg->num_kv_heads, true);
+  const void* fn = fused_kernel_of(cfg->num_kv_heads, cfg->num_heads / cfg->num_kv_heads, kScorePacked);
   const int per_launch = kMaxPhases;
   for (size_t at = 0; at < plan.parts.size(); at += per_launch) {
     const VoteLaunch& v = plan.parts[at];
