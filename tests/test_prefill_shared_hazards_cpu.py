@@ -27,3 +27,17 @@ def test_output_products_keep_their_distance(tmp_path, kind):
     for name, kernel in kernels.items():
         assert sum(i[3] and i[4] for i in kernel) >= 4 * 32, name
         assert _hazards(kernel) == [], name
+
+
+def test_what_is_asked_for_ahead_is_bounded_by_the_lanes_offset(tmp_path):
+    """Tiles past the end of the staging area are asked for ahead: it is the buffer's size that keeps those loads off the
+    memory behind it, and a buffer's size bounds the lanes' offset and the instruction's, not the scalar one."""
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    out = tmp_path / "shared.s"
+    subprocess.run([build.HIPCC, *build.CXXFLAGS, *build.SOURCE_FLAGS["ts_prefill_shared.hip"], "-S", "--offload-device-only",
+                    os.path.join(build.CSRC, "ts_prefill_shared.hip"), "-o", str(out)], check=True, capture_output=True)
+    loads = [line.split() for line in out.read_text().splitlines() if re.match(r"\s*buffer_load\w* .*\blds\b", line)]
+    assert len(loads) >= 2 * 2 * 7                             # kernels, halves, and three and four packages' halves
+    for load in loads:
+        assert "offen" in load and load[3] == "0", " ".join(load)

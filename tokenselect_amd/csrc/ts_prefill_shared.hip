@@ -56,8 +56,10 @@ constexpr int kPsCost = 10;       // what a piece of a job costs besides its til
 constexpr int kPsLeast = 8;      // tiles of a piece of a job that is cut, at least
 constexpr size_t kPsLdsBytes = (size_t)kPsBuffers * kPsPackage * 16;  // 64 KB
 
-// Two kilobytes, 16 bytes per lane of each, from `at` bytes behind the start of `from` to `to` (a byte of LDS), past
-// the registers (the offset of the second counts on both sides; what lies past the end of `from` arrives as zeros).
+// Two kilobytes, 16 bytes per lane of each, from `at` (of the lane) bytes behind the start of `from` to `to` (a byte of
+// LDS), past the registers (the offset of the second counts on both sides).  All of the offset is the lanes' own: that is
+// the part of an address that a raw buffer's size bounds, so that what would lie past the end of `from` is not read (it
+// arrives as zeros, and nothing uses it), wherever the memory behind it ends.  A scalar offset is not part of that check.
 // Assembly, because the compiler would wait for it at the next read of LDS, wherever that reads; nothing is returned to
 // a register, and the waits are in the loop.
 typedef __attribute__((ext_vector_type(4))) uint32_t ps_buffer;  // a buffer resource: base, size, raw dwords
@@ -65,10 +67,10 @@ __device__ __forceinline__ ps_buffer buffer_of(const void* from, int64_t bytes) 
   const uint64_t at = (uint64_t)from;
   return ps_buffer{(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, (uint32_t)(bytes > 0 ? bytes : 0), 0x00020000u};
 }
-__device__ __forceinline__ void load_to_lds(uint32_t to, const ps_buffer& from, uint32_t at, uint32_t lane16) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\tbuffer_load_dwordx4 %1, %2, %3 offen offset:1024 lds"
+__device__ __forceinline__ void load_to_lds(uint32_t to, const ps_buffer& from, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\tbuffer_load_dwordx4 %1, %2, 0 offen offset:1024 lds"
                :
-               : "s"(to), "v"(lane16), "s"(from), "s"(at)
+               : "s"(to), "v"(at), "s"(from)
                : "m0", "memory");
 }
 
@@ -218,17 +220,17 @@ __global__ __launch_bounds__(kPsThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     // (behind the queries, which are wanted first: loads return in order)
     const ps_buffer k_tiles = buffer_of(a.kr + head_at + kPart / 2 * wave, tiles_bytes);
     const ps_buffer v_tiles = buffer_of(a.vt + head_at + kPart / 2 * wave, tiles_bytes);
-    const uint32_t at = 2 * kPfTileElems * t_from;
-    load_to_lds(part_at + 2 * kBytes, k_tiles, at, lane16);
-    load_to_lds(part_at + 3 * kBytes, k_tiles, at + 2 * kPfTileElems, lane16);
-    load_to_lds(part_at + 3 * kBytes + kBytes / 2, v_tiles, at, lane16);
+    const uint32_t at = lane16 + 2 * kPfTileElems * t_from;
+    load_to_lds(part_at + 2 * kBytes, k_tiles, at);
+    load_to_lds(part_at + 3 * kBytes, k_tiles, at + 2 * kPfTileElems);
+    load_to_lds(part_at + 3 * kBytes + kBytes / 2, v_tiles, at);
   }
   const ps_buffer ask_k = buffer_of(a.kr + head_at + 2 * kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * 2 * kPfTileElems);
   const ps_buffer ask_v = buffer_of(a.vt + head_at + kPfTileElems + kPart / 2 * wave, tiles_bytes - 2 * kPfTileElems);
-  uint32_t ask_at = 2 * kPfTileElems * t_from;  // of the next package to be asked for, in the staging area
-  auto ask_keys = [&](uint32_t buffer) __attribute__((always_inline)) { load_to_lds(part_at + buffer, ask_k, ask_at, lane16); };
+  uint32_t ask_at = lane16 + 2 * kPfTileElems * t_from;  // of the next package to be asked for, in the staging area
+  auto ask_keys = [&](uint32_t buffer) __attribute__((always_inline)) { load_to_lds(part_at + buffer, ask_k, ask_at); };
   auto ask_values = [&](uint32_t buffer) __attribute__((always_inline)) {
-    load_to_lds(part_at + buffer + kBytes / 2, ask_v, ask_at, lane16);
+    load_to_lds(part_at + buffer + kBytes / 2, ask_v, ask_at);
     ask_at += 2 * kPfTileElems;
   };
   const int S = __builtin_amdgcn_readfirstlane(min(max(listed, 0), a.max_sel_len));
