@@ -21,7 +21,6 @@
 
 namespace ts {
 
-constexpr int kAttnWaves = 4;  // wavefronts of a workgroup
 constexpr int kAttnThreads = 64 * kAttnWaves;
 
 struct AttnArgs {
@@ -472,8 +471,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 at_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float at_f32x4;
 constexpr float kAttnLog2e = 1.4426950408889634f, kAttnLn2 = 0.6931471805599453f;
 constexpr uint32_t kNewRow = 0xffffffffu;  // the slot of a row that is not in the pool (no pool has as many)
-constexpr int kAttnTile = 32;        // tokens per step of a wavefront
-constexpr int kAttnChunkUnit = 16 * kAttnWaves;  // a workgroup's range is a multiple of this
 
 __device__ __forceinline__ at_bf16x8 pack8(const float* x) {
   const uint4 w = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]),
@@ -500,12 +497,6 @@ __device__ __forceinline__ void split8(const float* x, at_bf16x8& hi, at_bf16x8&
                       x[4] - bf16_lo(h.z), x[5] - bf16_hi(h.z), x[6] - bf16_lo(h.w), x[7] - bf16_hi(h.w)};
   hi = __builtin_bit_cast(at_bf16x8, h);
   lo = pack8(r);
-}
-
-// Tokens per workgroup of the matrix-core kernel for a launch of nsplit splits.
-__host__ __device__ __forceinline__ int attn_chunk(int max_sel_len, int nsplit) {
-  const int even = (max_sel_len + nsplit - 1) / nsplit;
-  return (even + kAttnChunkUnit - 1) / kAttnChunkUnit * kAttnChunkUnit;
 }
 
 // An index offset of zero that the compiler cannot see through, produced after `after` is:
@@ -865,7 +856,6 @@ __global__ __launch_bounds__(256) void attn_zero_kernel(uint32_t* tickets, int c
 // Tickets per request (the words to clear): one per KV head, and one for the heads of a dense step.
 int attn_tickets_per_request(const ts_config* cfg) { return cfg->num_kv_heads + 1; }
 
-constexpr int kAttnRange = kAttnTile * kAttnWaves;  // list entries per workgroup as long as the device has room
 static int attn_splits(int batch, int num_kv_heads, int max_sel_len) {
   // One tile per wavefront (128 entries per workgroup) as long as the grid stays within the
   // 512 workgroups that are resident at once (two per CU): a second round of workgroups pays
@@ -900,27 +890,60 @@ size_t attn_workspace_bytes(const ts_config* cfg, int batch, int max_sel_len) {
   return attn_workspace(cfg, batch, max_sel_len).total;
 }
 
-// Splits that everybody merges: a workgroup for each as long as all are resident at once (two per CU), with 64
-// entries (16 a wavefront) where each has a CU to itself.  At most kAttnShareSplits, and at least one for each head of the
-// group, whose columns they share; otherwise, or where the words do not fit, none.  us a layer merged by one and by
-// all: one request of 20K, 28 heads on 4 36.1 and 32.3, 32 on 8 33.9 and 32.7 (with 336 workgroups of 64 entries in
-// place of 168 of 128, 33.4), 4 on 1 35.0 and 31.5; two of 8K, 28 on 4 37.9 and 35.3; eight, 14 splits each, 56.1 and
-// 55.5; eight of 32 on 8, seven splits, 68.2 and 68.4: so from ten splits on.
-constexpr int kAttnShareSplits = 80;
+// The kernel of a call whose splits are shared, 64 entries each or more.
+template <int G>
+static const void* shared_kernel_of(bool rope, bool cap, bool half) {
+  if (half)
+    return rope ? (cap ? (const void*)&attn_kernel<G, true, true, kAttnSharedHalf> : (const void*)&attn_kernel<G, true, false, kAttnSharedHalf>)
+                : (cap ? (const void*)&attn_kernel<G, false, true, kAttnSharedHalf> : (const void*)&attn_kernel<G, false, false, kAttnSharedHalf>);
+  return rope ? (cap ? (const void*)&attn_kernel<G, true, true, kAttnShared> : (const void*)&attn_kernel<G, true, false, kAttnShared>)
+              : (cap ? (const void*)&attn_kernel<G, false, true, kAttnShared> : (const void*)&attn_kernel<G, false, false, kAttnShared>);
+}
+static const void* shared_kernel_of(int group, bool rope, bool cap, bool half) {
+  switch (group) {
+    case 1: return shared_kernel_of<1>(rope, cap, half);
+    case 2: return shared_kernel_of<2>(rope, cap, half);
+    case 3: return shared_kernel_of<3>(rope, cap, half);
+    case 4: return shared_kernel_of<4>(rope, cap, half);
+    case 5: return shared_kernel_of<5>(rope, cap, half);
+    case 6: return shared_kernel_of<6>(rope, cap, half);
+    case 7: return shared_kernel_of<7>(rope, cap, half);
+    case 8: return shared_kernel_of<8>(rope, cap, half);
+    default: return nullptr;
+  }
+}
+// What the current device holds of them (nothing: it did not answer, and is asked again).
+static AttnRoom attn_room(int group, bool rope, bool cap) {
+  struct Entry { int device, kind; AttnRoom room; };
+  constexpr int kMemo = 8;
+  static thread_local Entry memo[kMemo] = {};
+  static thread_local int next = 0;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return AttnRoom{};
+  const int kind = group * 4 + rope * 2 + cap;
+  for (const Entry& e : memo)
+    if (e.kind == kind && e.device == device) return e.room;
+  int cus = 0, per_cu[2] = {0, 0};
+  bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess;
+  for (int half = 0; half < 2; ++half) {
+    const void* fn = shared_kernel_of(group, rope, cap, half != 0);
+    ok = ok && fn && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[half], fn, kAttnThreads, 0) == hipSuccess;
+  }
+  if (!ok) {
+    (void)hipGetLastError();
+    return AttnRoom{};
+  }
+  const AttnRoom room{cus, cus * per_cu[1], cus * per_cu[0]};
+  memo[next] = Entry{device, kind, room};
+  next = (next + 1) % kMemo;
+  return room;
+}
+
 AttnShare attn_share(const ts_config* cfg, int batch, int max_sel_len, void* words, size_t bytes) {
-  AttnShare s{};
-  const int64_t groups = (int64_t)batch * cfg->num_kv_heads, fine = ceil_div(max_sel_len, kAttnChunkUnit);
-  const int G = cfg->num_heads / cfg->num_kv_heads;
-  s.half = groups * fine <= 256;
-  const int64_t want = s.half ? fine : std::min<int64_t>(ceil_div(max_sel_len, kAttnRange), 512 / groups);
-  if (want < 2) return AttnShare{};
-  s.nsplit = (int)ceil_div(max_sel_len, attn_chunk(max_sel_len, (int)want));
-  if (s.nsplit < std::max(G, 10) || s.nsplit > kAttnShareSplits) return AttnShare{};
-  s.parts = std::min(s.nsplit / G, 32);
-  s.parts_magic = 65536u / (uint32_t)s.parts + 1u;
-  s.cols = (int)ceil_div(kHeadDim / 2, s.parts);
-  s.bytes = (size_t)groups * s.nsplit * G * (kHeadDim / 2 + s.parts) * 8;
-  if (s.bytes > bytes) return AttnShare{};
+  const AttnRoom room =
+      attn_room(cfg->num_heads / cfg->num_kv_heads, cfg->rope_mode == TS_ROPE_LLAMA, cfg->logit_cap > 0.f);
+  AttnShare s = plan_attn_share(batch, cfg->num_heads, cfg->num_kv_heads, max_sel_len, room);
+  if (s.nsplit == 0 || s.bytes > bytes) return AttnShare{};
   s.words = (uint64_t*)words;
   return s;
 }

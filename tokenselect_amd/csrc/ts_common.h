@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/tokenselect.h"
+#include "ts_share.h"
 
 namespace ts {
 
@@ -284,21 +285,7 @@ struct AttnDense {
   int32_t* seq_lens;
   int max_tokens;
 };
-// The splits of a request and KV head merged by all of their workgroups, which wait for each other's words
-// (bounded; on giving up sel_len[b] = -1 and *fault_out = 1), in place of the last one to draw a ticket.  The words
-// are zero at launch and again when the kernel ends without having given up.
-struct AttnShare {
-  uint64_t* words;  // [B, Hkv, split, G x 64 sums then G x parts (max, sum)], or NULL
-  size_t bytes;
-  int nsplit, half;          // splits; 64 entries each
-  int parts, cols;           // workgroups that share a head's 64 columns of two dims, and columns of each
-  uint32_t parts_magic;      // x / parts = x * parts_magic >> 16, for x below 2^8
-  int absent;                // tests of the give-up: the first splits that send nothing
-  uint64_t ticks;            // a wait at most (100 MHz)
-  int32_t* sel_len;
-  uint32_t* fault_out;
-};
-// How a call's splits would be shared, with words in `bytes` bytes (words == NULL: not at all).
+// How a call's splits are shared on the current device, with words in `bytes` bytes (words == NULL: not at all).
 AttnShare attn_share(const ts_config* cfg, int batch, int max_sel_len, void* words, size_t bytes);
 int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                 int64_t pool_rows, const int32_t* sel, int64_t sel_stride, const int32_t* sel_len,
@@ -306,7 +293,6 @@ int launch_attn(const ts_config* cfg, const void* q, int q_stride, const void* k
                 hipStream_t stream, const ZeroSet* clear_after = nullptr, const AttnDense* dense = nullptr,
                 const StepCommit* commit = nullptr, const AttnShare* share = nullptr);
 
-constexpr int kHeadDim = 128;
 constexpr float kNegBig = -3.0e38f;  // finite stand-in for -inf in running maxima
 
 // -------------------------------------------------------------- device side
