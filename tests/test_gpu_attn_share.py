@@ -103,3 +103,50 @@ def test_an_attention_that_gives_up(dev, absent):
     with pytest.raises(ops.SelectionGaveUp):
         other(wl.q, wl.k_pool, wl.v_pool, wl.batch)
     _close(wl, other(wl.q, wl.k_pool, wl.v_pool, wl.batch), wl.q)
+
+
+def _nodes(graph):
+    """Launches in a captured graph, of the runtime that captured it."""
+    with open("/proc/self/maps") as maps:
+        path = next(line.split()[-1] for line in maps if "libamdhip64.so" in line)
+    count = ctypes.c_size_t(0)
+    assert ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+@pytest.mark.parametrize("stated", [False, True], ids=["unstated", "stated clean"])
+@pytest.mark.parametrize("case", [(28, 4, [20000]), (32, 8, [9000, 3000])], ids=lambda c: "H%dkv%d" % c[:2])
+def test_a_captured_layer(dev, case, stated):
+    """At a model's sizes: the rotation (which clears the words where the caller states nothing), the selection and the attention,
+    and no launch besides; replays with other queries, eager work and synchronisations in between, give the eager call's bits."""
+    say(f"captured attention merged by everybody {case} stated={stated}")
+    wl = _workload(dev, *case, 128, 512, 2048)
+    B, longest = len(wl.seq_lens), max(wl.seq_lens)
+    bt = dataclasses.replace(wl.batch, workspace_clean=stated)
+    layer, eager = (ops.DecodeLayer(wl.cfg, B, longest, dev) for _ in range(2))
+    q = wl.q.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # the first calls load code objects and size the grids
+        for _ in range(2):
+            layer(q, wl.k_pool, wl.v_pool, wl.batch)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out, sel, _, sel_len = layer(q, wl.k_pool, wl.v_pool, bt)
+    assert _nodes(graph) == (2 if stated else 3)
+    g = torch.Generator(device=dev).manual_seed(43)
+    for replay in range(5):
+        q.copy_(torch.randn(q.shape, generator=g, device=dev))
+        if not stated and replay == 3:
+            layer.workspace.fill_(0xa5)  # whatever used it in between
+        graph.replay()
+        torch.cuda.synchronize()
+        layer.check()
+        want = eager(q, wl.k_pool, wl.v_pool, wl.batch)
+        torch.cuda.synchronize()
+        assert torch.equal(sel_len, want[3]), replay
+        for b, n in enumerate(sel_len.tolist()):
+            assert torch.equal(sel[b, :n], want[1][b, :n]), replay
+        assert torch.equal(out.view(torch.int16), want[0].view(torch.int16)), replay

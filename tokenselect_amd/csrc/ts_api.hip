@@ -344,9 +344,11 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
   const bool plain_decode = one_launch && chunk_rows == 0 && !cache;
   const bool starts_with_selection = plain_decode && bt->workspace_clean != 0;
   // So does the attention with the words by which its splits are merged (those who read them do), which lie where
-  // separate kernels have their scores and votes: cleared ahead of a first call, and behind
-  // a call that was on the separate kernels though the next one need not be.
-  ZeroSet after = zero;
+  // separate kernels have their scores and votes: cleared by the rotation of a call that is not known to find them zero,
+  // and behind a call that was on the separate kernels though the next one need not be.
+  ZeroSet after{};
+  if (plain_decode) after = zero;
+  ZeroRegion ahead{};
   AttnShare share{};
   if (chunk_rows == 0 && !cache && bt->max_seq_len > w.max_sel) {
     share = attn_share(cfg, bt->batch, w.max_sel, ws + w.scores, w.topk_ws - w.scores);
@@ -355,14 +357,10 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
     share.sel_len = sel_len;
     share.fault_out = (uint32_t*)bt->fault;
     const ZeroRegion words{(uint32_t*)share.words, (int64_t)(share.bytes / 4), (int)(share.bytes / 4), 1};
-    if (!one_launch) {
-      after = ZeroSet{};
-      if (share.words && select_workspace(cfg, bt->batch, bt->max_seq_len, true).tokens_per_block > 0) after.add(words);
+    if (share.words && !one_launch) {
+      if (select_workspace(cfg, bt->batch, bt->max_seq_len, true).tokens_per_block > 0) after.add(words);
     } else if (share.words && !starts_with_selection) {
-      // (a launch of its own, once in some 64 steps: a fifth region in the others costs each of them)
-      ZeroSet first;
-      first.add(words);
-      TS_TRY(launch_select_zero(first, (hipStream_t)stream));
+      ahead = words;
     }
   }
   // That selection also stores the step's new tokens, and the attention after it writes the lengths
@@ -406,7 +404,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                                 zero, (hipStream_t)stream, store));
   } else {
     TS_TRY(launch_rope(q, q_stride, qf, q_cos, q_sin, nullptr, 1, bt->batch, cfg->num_heads, cfg->head_dim,
-                       zero, (hipStream_t)stream, store, bt->batch));
+                       zero, (hipStream_t)stream, store, bt->batch, ahead));
   }
   if (cache && chunk_rows > 0)
     TS_TRY(launch_selcache(cfg, bt, qf, cache, hit, bt->rerun ? sel_len : nullptr, (hipStream_t)stream));
@@ -443,7 +441,7 @@ static int run_layer(const ts_config* cfg, const ts_batch* bt, const void* q, in
                                w.max_sel, out, ws + w.attn_ws, w.total - w.attn_ws, (hipStream_t)stream);
   return launch_attn(cfg, q, q_stride, k_pool, v_pool, pool_rows, sel, sel_stride, sel_len, bt->batch,
                      w.max_sel, out, ws + w.attn_ws, /*tickets_clear=*/true, (hipStream_t)stream,
-                     chunk_rows == 0 && !cache ? &after : nullptr, nullptr, commit.batch ? &commit : nullptr,
+                     after.used ? &after : nullptr, nullptr, commit.batch ? &commit : nullptr,
                      one_launch && share.words ? &share : nullptr);
 }
 

@@ -70,34 +70,36 @@ struct ZeroSet {
     return t;
   }
 };
-// Wavefront `wave` of `waves` clears its share of every region: word by word (16 bytes at a time)
-// where the pieces touch, else a wavefront per piece.  No index is divided by the length of a
+// Wavefront `wave` of `waves` clears its share of a region: word by word (16 bytes at a time)
+// where the pieces touch, else a wavefront per piece, beginning with wavefront `from`.  No index is divided by the length of a
 // piece: with a 64-bit division and remainder per word the 0.3 MB of one request's selection cost
 // every workgroup of the launch some 600 instructions ahead of its first load.
-__device__ __forceinline__ void clear_regions(const ZeroSet& zero, uint32_t wave, uint32_t waves) {
+__device__ __forceinline__ void clear_region(const ZeroRegion& z, uint32_t wave, uint32_t waves, uint32_t from) {
   const uint32_t lane = threadIdx.x & 63u;
+  if (z.count == 1 || z.stride == z.words) {
+    const int64_t total = (int64_t)z.count * z.words, step = (int64_t)waves * 64;
+    int64_t done = 0;
+    if (((uintptr_t)z.base & 15u) == 0) {
+      done = total & ~(int64_t)3;
+      for (int64_t w = (int64_t)wave * 64 + lane; w < done >> 2; w += step)
+        *(uint4*)(z.base + 4 * w) = make_uint4(0u, 0u, 0u, 0u);
+    }
+    for (int64_t w = done + (int64_t)wave * 64 + lane; w < total; w += step) z.base[w] = 0u;
+  } else {
+    uint32_t first = wave + from;
+    first -= first >= waves ? waves : 0u;
+    for (uint32_t piece = first; piece < (uint32_t)z.count; piece += waves) {
+      uint32_t* const at = z.base + (int64_t)piece * z.stride;
+      for (int w = (int)lane; w < z.words; w += 64) at[w] = 0u;
+    }
+  }
+}
+__device__ __forceinline__ void clear_regions(const ZeroSet& zero, uint32_t wave, uint32_t waves) {
 #pragma unroll
   for (int i = 0; i < kZeroRegions; ++i) {
     if (i >= zero.used) break;
-    const ZeroRegion& z = zero.r[i];
-    if (z.count == 1 || z.stride == z.words) {
-      const int64_t total = (int64_t)z.count * z.words, step = (int64_t)waves * 64;
-      int64_t done = 0;
-      if (((uintptr_t)z.base & 15u) == 0) {
-        done = total & ~(int64_t)3;
-        for (int64_t w = (int64_t)wave * 64 + lane; w < done >> 2; w += step)
-          *(uint4*)(z.base + 4 * w) = make_uint4(0u, 0u, 0u, 0u);
-      }
-      for (int64_t w = done + (int64_t)wave * 64 + lane; w < total; w += step) z.base[w] = 0u;
-    } else {
-      // (another first wavefront per region: a piece each, not all of them to the same few)
-      uint32_t first = wave + (uint32_t)i * (waves >> 2);
-      first -= first >= waves ? waves : 0u;
-      for (uint32_t piece = first; piece < (uint32_t)z.count; piece += waves) {
-        uint32_t* const at = z.base + (int64_t)piece * z.stride;
-        for (int w = (int)lane; w < z.words; w += 64) at[w] = 0u;
-      }
-    }
+    // (another first wavefront per region: a piece each, not all of them to the same few)
+    clear_region(zero.r[i], wave, waves, (uint32_t)i * (waves >> 2));
   }
 }
 // Chunk fingerprint (ts_prefill.hip) with the same side job as launch_rope: the
@@ -161,10 +163,12 @@ struct StepCommit {
 };
 constexpr int kCommitBatch = 64;  // requests that one wavefront writes for
 
-// x_stride: elements between the rows of x (out is contiguous).  store: rides in the launch.
+// x_stride: elements between the rows of x (out is contiguous).  store: rides in the launch.  zero, more: what it
+// clears, `more` in one piece (words == 0: nothing).
 int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
                 const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
-                const ZeroSet& zero, hipStream_t stream, const StepStore* store = nullptr, int store_batch = 0);
+                const ZeroSet& zero, hipStream_t stream, const StepStore* store = nullptr, int store_batch = 0,
+                const ZeroRegion& more = ZeroRegion{});
 
 // Selection-cache decision (ts_selcache.hip); gave_up_len: see ts_batch.rerun (NULL: an
 // ordinary step).

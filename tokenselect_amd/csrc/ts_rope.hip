@@ -18,7 +18,8 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
                                                          const float* __restrict__ sin_table,
                                                          const int64_t* __restrict__ position_ids,
                                                          int64_t table_rows, int64_t rows, int heads,
-                                                         int dim, ZeroSet zero, int blocks, StepStore st) {
+                                                         int dim, ZeroSet zero, int blocks, StepStore st,
+                                                         ZeroRegion more) {
 #pragma clang fp contract(off)
   if ((int)blockIdx.x >= blocks) {
     store_step(st, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
@@ -45,6 +46,7 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
   const float c1 = c[i], s1 = s[i], c2 = c[i + half], s2 = s[i + half];
   // Counters the later kernels of a decode step accumulate into.
   clear_regions(zero, blockIdx.x * 4 + (threadIdx.x >> 6), (uint32_t)blocks * 4);
+  if (more.words) clear_region(more, blockIdx.x * 4 + (threadIdx.x >> 6), (uint32_t)blocks * 4, 0u);
   if (gid >= pairs) return;
   const float lo = rotate_element(x1, x2, c1, s1, true);
   const float hi = rotate_element(x2, x1, c2, s2, false);
@@ -54,16 +56,16 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(const uint16_t* __restr
 
 int launch_rope(const void* x, int64_t x_stride, void* out, const float* cos_table, const float* sin_table,
                 const int64_t* position_ids, int64_t table_rows, int64_t rows, int heads, int dim,
-                const ZeroSet& zero, hipStream_t stream, const StepStore* store, int store_batch) {
+                const ZeroSet& zero, hipStream_t stream, const StepStore* store, int store_batch, const ZeroRegion& more) {
   TS_REQUIRE(!zero.overflow, TS_EINVAL, "internal: more than %d regions to clear in one launch", kZeroRegions);
   const int64_t pairs = rows * heads * (dim / 2);
   // Enough workgroups for the clearing on the side as well: four words per thread.
-  const int64_t to_clear = zero.total();
+  const int64_t to_clear = zero.total() + more.words;
   const int64_t blocks = std::max(ceil_div(pairs, 256), ceil_div(to_clear, 1024));
   TS_REQUIRE(blocks + store_batch <= 0x7fffffff, TS_EINVAL, "ts_rope_apply: too many rows");
   hipLaunchKernelGGL(rope_apply_kernel, dim3((unsigned)(blocks + (store ? store_batch : 0))), dim3(256), 0, stream,
                      (const uint16_t*)x, x_stride, (uint16_t*)out, cos_table, sin_table, position_ids,
-                     table_rows, rows, heads, dim, zero, (int)blocks, store ? *store : StepStore{});
+                     table_rows, rows, heads, dim, zero, (int)blocks, store ? *store : StepStore{}, more);
   return check_launch("rope_apply_kernel");
 }
 
