@@ -85,8 +85,9 @@ typedef struct ts_batch {
                                (device memory, or pinned host memory that the
                                device maps, which the host may read at any time
                                without synchronising): set to 1 when a grid-wide
-                               wait of a ts_select launch gave up, never cleared
-                               by the library                                   */
+                               wait of a ts_select launch gave up, or one of a
+                               layer's attention where that waits
+                               (ts_decode_layer), never cleared by the library  */
   const int32_t* host_seq_lens; /* NULL, or [B] in host memory: upper bounds of
                                seq_lens[] that the host knows (a serving
                                framework's CPU copy of the lengths), each <=
@@ -123,8 +124,9 @@ typedef struct ts_batch {
                                the array of that call): the selection cache takes a
                                request that gave up as a miss whatever it cached
                                meanwhile, and its counters do not advance again  */
-  uint32_t wait_us;         /* bound of a grid-wide wait of the fused kernels in
-                               microseconds; 0 = TS_DEFAULT_WAIT_US              */
+  uint32_t wait_us;         /* bound of a grid-wide wait of the fused kernels, and of
+                               a wait of a layer's attention (ts_decode_layer),
+                               in microseconds; 0 = TS_DEFAULT_WAIT_US           */
   int32_t absent_workgroups; /* tests of the give-up path only (0 in production):
                                workgroups counted as members of every rendezvous
                                that never arrive, so that every wait gives up
@@ -132,7 +134,8 @@ typedef struct ts_batch {
                                threshold_hint, where there is no rendezvous: the
                                waits of all but a request's first workgroup);
                                < 0: of the attention, that many splits of each
-                               request and KV head (where it waits: below)       */
+                               request and KV head (where it waits:
+                               ts_decode_layer)                                  */
   int32_t workspace_clean;  /* ts_decode_layer and ts_decode_step.  1: the caller states that
                                this workspace was last used by one of these calls with
                                the same cfg, batch, max_seq_len (or one of the same
@@ -574,7 +577,18 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
  * neither serves (pool_kernel above 256, a request that does not fit the device)
  * ts_score, ts_vote and ts_topk_ragged run as they do on their own.  All forms give
  * the same selection.
- * ts_set_fused_select(0) forces the separate kernels for the calling process
+ * The attention waits too, for the words by which all workgroups of a request and KV
+ * head merge its splits: in ts_decode_layer and ts_decode_step without a selection
+ * cache whose selection is the ts_select kernel, with max_seq_len > n_init + top_k +
+ * n_local, where the launch has ten to 80 splits per KV head (and one for each query
+ * head of the group) that the device holds all at once, and the workspace's area for the
+ * separate kernels' scores holds the words (for 64 entries a split, the form of few KV
+ * heads, from contexts of some 1.6 to 2.2 times n_init + top_k + n_local on).  A wait
+ * that gives up (bt->wait_us) leaves sel_len[b] = -1 for its request b, though the
+ * selection in sel was whole, and *bt->fault = 1 where that is given; the output of that
+ * request is not valid.  Everything else of the call is done, a ts_decode_step's store
+ * included, and the call is repeated as one whose selection gave up is.
+ * ts_set_fused_select(0) forces the separate kernels, which wait for nobody, for the calling process
  * (1 restores the default); it returns the previous setting and has no
  * counterpart in the reference. */
 int ts_set_fused_select(int enable);
