@@ -150,3 +150,66 @@ def test_a_captured_layer(dev, case, stated):
         for b, n in enumerate(sel_len.tolist()):
             assert torch.equal(sel[b, :n], want[1][b, :n]), replay
         assert torch.equal(out.view(torch.int16), want[0].view(torch.int16)), replay
+
+
+# the contexts from which the words fit where separate kernels have their scores (k = 2048), and one below
+LINE = [((28, 4, [4608]), False), ((28, 4, [4609]), True), ((12, 2, [4480]), False), ((12, 2, [4481]), True),
+        ((4, 1, [4096]), False), ((4, 1, [4097]), True), ((32, 8, [2689]), True), ((28, 4, [2700, 2689]), True)]
+
+
+@pytest.mark.parametrize("case,shares", LINE, ids=lambda c: "H%dkv%d-%d" % (c[0], c[1], c[2][0]) if isinstance(c, tuple) else str(c))
+def test_where_the_words_fit(dev, case, shares):
+    """Both sides of the line give the other attention's output; splits forced to be absent tell who waits."""
+    say(f"attention where the words fit: {case} {shares}")
+    wl = _workload(dev, *case, 128, 512, 2048)
+    B, longest = len(wl.seq_lens), max(wl.seq_lens)
+    layer = ops.DecodeLayer(wl.cfg, B, longest, dev)
+    for _ in range(3):
+        got = layer(wl.q, wl.k_pool, wl.v_pool, wl.batch)
+        _close(wl, got, wl.q)
+    layer(wl.q, wl.k_pool, wl.v_pool, dataclasses.replace(wl.batch, wait_us=20, absent_workgroups=-1))
+    torch.cuda.synchronize()
+    assert layer.gave_up() == shares
+
+
+@pytest.mark.parametrize("before", [0, 2], ids=["stored ahead", "stored by the selection"])
+def test_a_step_whose_attention_gives_up(dev, before):
+    """The store of a step that gives up has happened, whichever launch it rode in: recover() repeats selection and attention
+    alone, lengths advance once, and pools, table and output are those of an object that nothing disturbed."""
+    say(f"step whose attention gives up, {before} steps before it")
+    wl = _workload(dev, 28, 4, [7000, 6000], 128, 512, 2048)
+    g = torch.Generator(device=dev).manual_seed(44)
+    width, steps = 7000 + 8, before + 2
+    spare = torch.arange(wl.k_pool.shape[0], wl.k_pool.shape[0] + 2 * steps, dtype=torch.int32, device=dev).view(steps, 2)
+    qs = torch.randn((steps, *wl.q.shape), generator=g, device=dev).bfloat16()
+    kv = torch.randn((steps, 2, 2, 4, 128), generator=g, device=dev).bfloat16()
+
+    def serve(forced_at):
+        pools = [torch.cat((p, torch.zeros((2 * steps, 4, 128), dtype=p.dtype, device=dev))) for p in (wl.k_pool, wl.v_pool)]
+        table = torch.zeros((2, width), dtype=torch.int32, device=dev)
+        table[:, :wl.table.shape[1]] = wl.table
+        lens = wl.seq_lens_dev.clone()
+        layer = ops.DecodeLayer(wl.cfg, 2, 7000 + steps, dev)
+        for t in range(steps):
+            bt = ops.Batch(lens, table, 7000 + steps)
+            if t == forced_at:
+                bt = dataclasses.replace(bt, wait_us=20, absent_workgroups=-1)
+            assert (layer._clean_for is not None) == (t > 0 and not layer.separate)
+            got = layer.step(qs[t], kv[t, 0], kv[t, 1], spare[t], *pools, bt)
+            torch.cuda.synchronize()
+            assert lens.tolist() == [7000 + t + 1, 6000 + t + 1]
+            if t == forced_at:
+                assert layer.gave_up() and got[3].tolist() == [-1, -1]
+                got = layer.recover(qs[t], *pools, bt)
+                torch.cuda.synchronize()
+            assert not layer.gave_up() and lens.tolist() == [7000 + t + 1, 6000 + t + 1]
+        return [x.clone() for x in got], pools, table, lens
+
+    (got, pools, table, lens), (want, pools_w, table_w, lens_w) = serve(before), serve(None)
+    for a, b in ((pools[0], pools_w[0]), (pools[1], pools_w[1])):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert torch.equal(table, table_w) and torch.equal(lens, lens_w) and torch.equal(got[3], want[3])
+    for b, n in enumerate(got[3].tolist()):  # (the separate kernels' votes are added up in another order: ties only)
+        assert len(set(got[1][b, :n].tolist()) ^ set(want[1][b, :n].tolist())) <= 2
+    full = dataclasses.replace(wl, k_pool=pools[0], v_pool=pools[1])
+    _close(full, got, qs[-1])

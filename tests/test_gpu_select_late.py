@@ -102,3 +102,27 @@ def test_a_wait_for_late_words_that_gives_up(dev, off):
     torch.cuda.synchronize()
     assert got is not None and not layer.gave_up()
     _same(got, want, "recovered")
+
+
+def test_each_request_with_a_k_of_its_own(dev):
+    """The wide band finds each request's own k-th vote: hints off by bins on either side of it, a request among them that
+    attends to everything."""
+    say("late candidates, k per request")
+    lens, ks = [9000, 3000, 7000, 900], [700, 31, 512, 700]
+    wl = workloads.build("late", dict(num_heads=32, num_kv_heads=8, rope_theta=5e5), lens, ks, 1, dev, seed=53, n_init=64,
+                         n_local=128, top_k=700)
+    assert wl.batch.k_per_req is not None
+    layer = ops.DecodeLayer(wl.cfg, 4, 9000, dev)
+    hint = torch.zeros(4, dtype=torch.int32, device=dev)
+    bt = dataclasses.replace(wl.batch, hint=hint)
+    want = _met(wl, wl.q)
+    assert want[2].tolist() == [64 + 700 + 128, 64 + 31 + 128, 64 + 512 + 128, 64 + 700 + 128]
+    _same(layer(wl.q, wl.k_pool, wl.v_pool, bt), want, "no hint yet")
+    code = hint.clone()
+    for off in (0, -17, -16, -12, -9, -5, -4, 4, 5, 9, 12, 16, 17):
+        hint.copy_(torch.where(code > 0, code + off, code))
+        got = layer(wl.q, wl.k_pool, wl.v_pool, bt)
+        torch.cuda.synchronize()
+        assert not layer.gave_up(), off
+        _same(got, want, off)
+        assert torch.equal(hint, code), off
