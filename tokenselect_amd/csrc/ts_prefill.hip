@@ -893,13 +893,16 @@ int launch_prompt_fingerprint(const ts_config* cfg, const void* q, int q_stride,
   return check_launch("prompt_fingerprint_kernel");
 }
 
-// Chunks, from the first on, whose attention takes the workgroups of 256 columns.  A wave of those over the
-// device, a workgroup per CU, takes 75 us for 2688 keys, and one of the workgroups of 64 columns 20 where all
-// of them read the same 1.4 MB per head, 26 where each chunk has its own: so they get all chunks where
-// their last wave is at least 0.8 full, else as many as fill whole waves (20 chunks of 512 rows, 28 heads on 4,
-// are 1120: 18 of them four waves less 16, 300 us, and two chunks 52).  The rows of a long dense chunk
-// see fewer keys the earlier they are, and the early ones fill the last wave up: 115 us instead of 161 with
-// 1.5 waves, 159 instead of 192 with two, 107 instead of 77 with 0.75; 2560 rows that are all there is, 79 instead of 88 with 1.1.
+// Chunks, from the first on, whose attention takes the workgroups of 256 columns where no job is cut: for a workspace
+// without room for the pieces, or jobs too few.  A wave of those over the device, a workgroup per CU, takes 68 us for 2688 keys, and one
+// of the workgroups of 64 columns 20 where all of them read the same 1.4 MB per head, 26 where each chunk has its own: so they get all
+// chunks where their last wave is at least 0.8 full, else as many as fill whole waves.  us for a whole call of chunks of 512 rows in
+// workgroups of 64 columns, with whole waves, and with all: 28 heads on 4, two chunks (0.44 waves) 106, 106 and 125, four
+// (0.88) 152, 152 and 132, nine (1.97) 285, 269 and 224, 18 (3.94) 530, 447 and 402.  The line is that of a loop that took 75 us;
+// with this one it would lie at some 0.6 (three chunks, 0.66, 130, 130 and 128, eight, 1.75, 264, 247 and 219; 32 on 8, six,
+// 1.5, 219, 206 and 211), of use only to who has no room for pieces: jobs are cut from 0.59 waves on.  The rows of a long dense chunk see
+// fewer keys the earlier they are, and the early ones fill the last wave up: 28 heads on 4, 2048 rows (0.88) 66 and 66, 2336 (1) 83 and
+// 73, 2688 (1.16) 96 and 83.
 static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_rows) {
   const int64_t each = prefill_shared_workgroups(num_heads, num_kv_heads, chunk_rows), chunks = ceil_div(rows, chunk_rows);
   // (small chunks would leave most of a workgroup without columns)
@@ -911,7 +914,7 @@ static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_ro
 
 // Whether the workgroups of 256 columns take all rows, with jobs that are cut: one long dense chunk from 0.87 waves of
 // jobs on, several chunks from 0.59.  us for a whole call, in workgroups of 64 columns and so: 28 heads on 4, 1536
-// dense rows (0.66) 46 and 45, 2048 (0.87) 61 and 54; 32 on 8, 1536 (0.75) 46 and 48, 2048 (1) 62 and 60; two full chunks of
+// dense rows (0.66) 46 and 45, 2048 (0.87) 61 and 54 (of another box, 66 and 60); 32 on 8, 1536 (0.75) 46 and 48, 2048 (1) 62 and 60; two full chunks of
 // 28 heads (0.44) 95 and 96, of 32 (0.5) 99 and 103; 1436 rows in chunks of 512 of 28 heads (0.61) 117 and 110, of 32
 // (0.7) 124 and 122, 1948 of 24 on 8 (0.72) 149 and 125.  And from 1024 keys on: the start of a piece costs ten tiles of 32.
 bool prefill_cuts_pay(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys) {

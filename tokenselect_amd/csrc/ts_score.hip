@@ -1727,7 +1727,8 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // has more than one look brings: window 15, one request of 100K tokens 64.1 us a layer met, 64.6 so.)  us a layer,
     // with two rounds, or one, met for in place of the wide band and this: eight requests of 3-16K 92.4 -> 88.0 (their
     // bins are crowded, and whoever fails keeps all waiting), one of 32K 32.6 -> 32.2 in the mean over hints that hold and
-    // some that do not, four of 64K with a selection cache 75.4 -> 74.2, a chunk at 128K 100.0 -> 99.5.
+    // some that do not; four of 64K with a selection cache and a chunk at 128K, of which hardly one comes here, the same within
+    // their runs' spread (612 and 606 us for eight steps, 198.1 and 198.2 for two layers).
     // (Both behind __builtin_expect: in line with the path of a hint that holds they cost that 0.3 us.)
     bool late = LATE && listed && !from_band && (banded ? found && shift == 21 : true) && lp.tokens_per_block <= kBandMaxTokens &&
                 req_chunks <= kSelMaxChunks / 2;
