@@ -126,3 +126,22 @@ def test_each_request_with_a_k_of_its_own(dev):
         assert not layer.gave_up(), off
         _same(got, want, off)
         assert torch.equal(hint, code), off
+
+
+def test_every_head_shape_selects_in_one_launch(dev):
+    """A single request, and a few, of any head shape the library serves."""
+    for kv_heads in (1, 2, 4, 8):
+        for group in range(1, 9):
+            c = ops.LayerConfig(num_heads=group * kv_heads, num_kv_heads=kv_heads, page_size=1, n_init=64, n_local=128, top_k=512)
+            for batch, longest in ((1, 1000), (1, 60000), (4, 9000)):
+                say(f"selection form of {group * kv_heads} heads on {kv_heads}, {batch} of {longest}")
+                assert ops.layer_selection_form(c, batch, longest) == 2 and ops.select_supported(c, batch, longest)
+
+
+@pytest.mark.parametrize("case", [dict(heads=64, kv_heads=8, lens=[40000], top_k=512),
+                                  dict(heads=40, kv_heads=8, lens=[9000, 3000, 700], top_k=700),
+                                  dict(heads=48, kv_heads=8, lens=[7000, 6000], top_k=400, same=9)],
+                         ids=lambda c: "H%dkv%d-%d" % (c["heads"], c["kv_heads"], sum(c["lens"])))
+def test_five_to_eight_heads_on_each_of_eight(dev, case):
+    """The shapes whose kernels take the most of a CU."""
+    test_a_layers_selection_without_meetings(dev, case)
