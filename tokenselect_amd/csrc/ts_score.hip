@@ -1061,18 +1061,22 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     // bins from the lowest on hold one without room for its count, [9] a bin's candidates do not fit.
     __shared__ uint32_t band_sum[kBandBins + 2];
     // Per bin of the wide band, and above them all; over all workgroups two bins each, the tokens above, and how many
-    // bins from the lowest on hold one without room for its count.  In the place of the histogram's first bins, which a
-    // workgroup with a hint has not counted when it wants them: words of their own (208 bytes) took the kernels of 40 to 64 heads on
-    // 8 past the 160 KB of a CU, with the stage that a workgroup with a CU to itself may ask for, and those shapes had no fused selection.
-    constexpr int kWideLds = kWideBins + 1 + 4 * kWideWords + 2;
-    uint32_t *const wide_count = lh, *const wide_sum = lh + kWideBins + 1;
-    static_assert(kWideLds <= kTopkBins - 2 * kSelListCap, "the entries take the place of the last bins");
+    // bins from the lowest on hold one without room for its count.  (Of 40 to 64 heads on 8 behind the histogram, where their query
+    // operands have left room: with 208 bytes more, and the stage that a workgroup with a CU to itself may ask for, their kernels
+    // were past the 160 KB of a CU, and those shapes had no fused selection.  In the place of the histogram's first bins for all shapes: one request of
+    // 32K 501 -> 505 us, a chunk at 128K 199.0 -> 200.)
+    constexpr bool kWideInRoom = LATE && LH >= kTopkBins + kWideBins + 1 + 4 * kWideWords + 2;
+    __shared__ uint32_t wide_count_own[LATE && !kWideInRoom ? kWideBins + 1 : 1], wide_sum_own[LATE && !kWideInRoom ? 4 * kWideWords + 2 : 1];
+    uint32_t *const wide_count = kWideInRoom ? lh + kTopkBins : wide_count_own,
+             *const wide_sum = kWideInRoom ? lh + kTopkBins + kWideBins + 1 : wide_sum_own;
     static_assert(kLateSlots <= kBandBins * kBandSlots, "the late candidates take the place of the band's");
     for (int i = tid; i < kTopkBins; i += 256) lh[i] = 0u;
     if (tid < 16) scratch[tid] = 0u;
     if (tid < kBandBins * kBandSlots) band_lds[tid / kBandSlots][tid % kBandSlots] = 0u;
     if (tid <= kBandBins) band_count[tid] = 0u;
     if (tid < kBandBins + 2) band_sum[tid] = 0u;
+    if (LATE && tid <= kWideBins) wide_count[tid] = 0u;
+    if (LATE && tid < 4 * kWideWords + 2) wide_sum[tid] = 0u;
     TS_MARK(1);
     __syncthreads();  // scores, own maxima and the cleared histogram are in LDS for all
     TS_MARK(2);
@@ -1616,7 +1620,6 @@ __global__ __launch_bounds__(256, (G > 4 ? 1 : 2)) void score_kernel(ScoreArgs a
     if (banded && !found) {  // the hint was of no use: the histogram is needed after all
       __syncthreads();
       for (int i = tid; i < 2 * kSelListCap; i += 256) lh[kTopkBins - 2 * kSelListCap + i] = 0u;  // (the entries)
-      if (LATE && tid < kWideLds) lh[tid] = 0u;
       __syncthreads();
       count_bins();
       publish_histogram();
