@@ -47,13 +47,13 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 # Each figure carries the commit of the kernels it was measured on: a later change to the
 # kernel makes it stale until the two counter runs are repeated.
 MEASURED_TRAFFIC = {  # workload -> (bytes per launch of its dominant kernel, commit); profiles/decode_layer_hbm_traffic.txt
-    "C2": (269404338, "1f23e95"),        # ts_select, score_kernel<8,4,false,2>
-    "C3": (2229759047, "1f23e95"),       # the votes-only launch, score_kernel<8,4,false,3>
-    "C5-layer": (2154451912, "1f23e95"),  # likewise
-    "MODEL": (2158924619, "1f23e95"),     # likewise, inside the 32-layer decoder (page 1)
+    "C2": (269432169, "93f4fda"),        # ts_select, score_kernel<8,4,false,4>
+    "C3": (2230531986, "93f4fda"),       # the votes-only launch, score_kernel<8,4,false,3>
+    "C5-layer": (2155118032, "93f4fda"),  # likewise
+    "MODEL": (2159277691, "93f4fda"),     # likewise, inside the 32-layer decoder (page 1)
 }
 # attn_kernel<4>, same runs
-MEASURED_ATTN_TRAFFIC = {"C2": 12288543, "C3": 180834151, "C5-layer": 82201640}
+MEASURED_ATTN_TRAFFIC = {"C2": 12149239, "C3": 180860735, "C5-layer": 82214348}
 
 
 def event_time_us(fn, launches: int, warmup: int, before=None, burst: int = 1):
@@ -155,7 +155,7 @@ def kernel_rooflines(ops, wl, k_pools, v_pools, layer, steps, warmup):
         dom_us, dom_min = event_time_us(run_select, steps, warmup, before=clear_all, burst=burst)
         if any(ops.select_fault(c, bt, space) for space in spaces):
             sys.exit("bench.py: a grid-wide wait of the selection kernel gave up")
-        dom_kernel = "ts::score_kernel<Hkv,G,false,2> (ts_select: score + vote + top-k in one launch)"
+        dom_kernel = "ts::score_kernel<Hkv,G,false,4> (ts_select: score + vote + top-k in one launch)"
     elif ops.layer_selection_form(c, bt) == 1:
         # Scores and votes request by request, the scores never in memory: the fused kernel
         # in its votes-only form (+ one small clearing kernel), one launch whose phases are
