@@ -154,7 +154,7 @@ def test_a_captured_layer(dev, case, stated):
 
 # the contexts from which the words fit where separate kernels have their scores (k = 2048), and one below
 LINE = [((28, 4, [4608]), False), ((28, 4, [4609]), True), ((12, 2, [4480]), False), ((12, 2, [4481]), True),
-        ((4, 1, [4096]), False), ((4, 1, [4097]), True), ((32, 8, [2689]), True), ((28, 4, [2700, 2689]), True)]
+        ((4, 1, [4096]), False), ((4, 1, [4097]), True), ((32, 8, [2689]), True), ((28, 4, [2700, 2689]), True), ((64, 8, [2689]), True), ((56, 8, [5000, 900]), True)]
 
 
 @pytest.mark.parametrize("case,shares", LINE, ids=lambda c: "H%dkv%d-%d" % (c[0], c[1], c[2][0]) if isinstance(c, tuple) else str(c))
