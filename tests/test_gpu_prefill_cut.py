@@ -99,3 +99,22 @@ def test_jobs_that_are_cut(dev, case):
     p.check(out, lists)
     assert torch.equal(out, p.together()[0])
     p.check(p.together(room=0)[0], lists)
+
+
+@pytest.mark.parametrize("heads,kv_heads,rows,top_k,cap,cut",
+                         [(40, 8, 1584, 1024, 0.0, True), (32, 8, 1664, 1024, 0.0, False), (64, 8, 1024, 1024, 0.0, False),
+                          (56, 8, 1664, 1024, 0.0, False), (24, 8, 2560, 2048, 0.0, True), (32, 8, 2688, 2048, 0.0, True),
+                          (56, 8, 2560, 2048, 30.0, True), (40, 8, 2560, 2048, 0.0, False)])
+def test_dense_rows_that_are_cut(dev, monkeypatch, heads, kv_heads, rows, top_k, cap, cut):
+    """Dense rows alone, where sharing their jobs out pays (less than a wave, more, more than two) and where it does not (too few, jobs too
+    short, so many that the longest is the launch either way): cut, some sums are added up in pieces; otherwise the bits are those
+    without room."""
+    say(f"dense rows, cut or not: {heads} on {kv_heads}, {rows}, top-k {top_k}")
+    monkeypatch.setitem(globals(), "TOP_K", top_k)
+    p = _Prompt(dev, heads, kv_heads, 0, rows, cap)
+    lists = p.one_by_one()
+    out, _, _ = p.together()
+    p.check(out, lists)
+    without = p.together(room=0)[0]
+    p.check(without, lists)
+    assert torch.equal(out, without) != cut

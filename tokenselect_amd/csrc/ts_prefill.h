@@ -105,6 +105,7 @@ constexpr int kPsSlots = 256;   // workgroups that share jobs, of all KV heads: 
 constexpr int kPsTicketBytes = kPsSlots * 4 * 4;
 // (without a workspace of prefill_cut_bytes() no job is cut)
 PrefillCuts prefill_cuts(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys, void* workspace);
+bool prefill_dense_cuts_pay(int num_heads, int num_kv_heads, int rows, int keys);
 int launch_prefill_shared(const PrefillArgs& a, const PrefillCuts& cuts, hipStream_t stream);
 // The same in workgroups of 64 columns, for several chunks (ts_prefill_chunks.hip).
 int launch_prefill_several(const PrefillArgs& a, int chunks, hipStream_t stream);

@@ -912,17 +912,17 @@ static int shared_chunks(int num_heads, int num_kv_heads, int rows, int chunk_ro
   return (int)(full * 256 / each);
 }
 
-// Whether the workgroups of 256 columns take all rows, with jobs that are cut: one long dense chunk from 0.87 waves of
-// jobs on, several chunks from 0.59.  us for a whole call, in workgroups of 64 columns and so: 28 heads on 4, 1536
-// dense rows (0.66) 46 and 45, 2048 (0.87) 61 and 54 (of another box, 66 and 60); 32 on 8, 1536 (0.75) 46 and 48, 2048 (1) 62 and 60; two full chunks of
-// 28 heads (0.44) 95 and 96, of 32 (0.5) 99 and 103; 1436 rows in chunks of 512 of 28 heads (0.61) 117 and 110, of 32
+// Whether the workgroups of 256 columns take all rows, with jobs that are cut: one long dense chunk by what it would take
+// either way (prefill_dense_cuts_pay), several chunks from 0.59 waves of jobs on.  us for a whole call, in workgroups of 64 columns
+// and so: two full chunks of 28 heads (0.44) 95 and 96, of 32 (0.5) 99 and 103; 1436 rows in chunks of 512 of 28 heads (0.61) 117 and 110, of 32
 // (0.7) 124 and 122, 1948 of 24 on 8 (0.72) 149 and 125.  And from 1024 keys on: the start of a piece costs ten tiles of 32.
 bool prefill_cuts_pay(int num_heads, int num_kv_heads, int rows, int chunk_rows, int keys) {
   if (keys < 1024) return false;
   const PrefillCuts c = prefill_cuts(num_heads, num_kv_heads, rows, chunk_rows, 1, nullptr);
   // (small chunks would leave most of a workgroup without columns)
   if (4 * (int64_t)std::min(rows, chunk_rows) * num_heads < 3 * (int64_t)c.per_chunk * num_kv_heads * 256) return false;
-  return c.jobs * num_kv_heads >= (c.chunks == 1 ? 224 : 152);
+  if (c.chunks == 1) return prefill_dense_cuts_pay(num_heads, num_kv_heads, rows, keys);
+  return c.jobs * num_kv_heads >= 152;
 }
 
 static int prefill_s_pad(int max_sel_len) { return (int)ceil_div(max_sel_len, kPfPadKeys) * kPfPadKeys; }

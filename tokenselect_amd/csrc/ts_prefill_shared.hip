@@ -666,6 +666,29 @@ PrefillCuts prefill_cuts(int num_heads, int num_kv_heads, int rows, int chunk_ro
   return c;
 }
 
+// Whether the jobs of one long dense chunk are shared out, by what the launch would take either way, in tiles.  Cut, all
+// of a head's jobs and ten tiles each divided by its workgroups, and 26 for what is cut on top.  As they are, the longest start
+// first and whoever is through takes the next, sixteen tiles each besides their own: within a wave the longest, within
+// two also two from the middle (whose lengths go down evenly, so that any such two are as long), within three the longest
+// of the third on top of these; with more, and below 0.87 waves, sharing pays nowhere.  By four tiles at least, this says the
+// right thing for all of 73 sizes of 16 to 64 heads, 1024 to 4700 rows.  us for a whole call uncut and cut, where it says cut: 24 on 8, 2560
+// rows (0.94 waves) 75 and 65, 32 on 8, 2048 (1) 63 and 59, 2688 (1.31) 79 and 75, 28 on 4, 2560 (1.09) 73 and 68, 64 on 8, 2304 (2.25) 104 and
+// 101; where it says not: 64 on 8, 1024 rows (1) 44.5 and 50, 1536 (1.5) 59 and 67, 40 on 8, 1792 (1.09) 59 and 61, 32 on 8, 3200 (1.56) 92.5 and 97,
+// 4000 (1.97) 127 and 135, 28 on 4, 4000 (1.72) 115 and 124, 56 on 8, 4000 (3.44) 213 and 224.
+bool prefill_dense_cuts_pay(int num_heads, int num_kv_heads, int rows, int keys) {
+  const int group = num_heads / num_kv_heads, streams = kPsSlots / num_kv_heads;
+  const int jobs = (int)ceil_div(ceil_div(rows, 16) * group, kPsUnits);
+  if (jobs * num_kv_heads < 224 || jobs > 3 * streams) return false;
+  auto tiles = [&](int j) { return job_tiles(keys, rows, jobs - 1 - j, group); };  // of the j-th to start
+  constexpr int kUncut = 16, kCut = 26, kLeastGain = 4;
+  int64_t cost = 0;
+  for (int j = 0; j < jobs; ++j) cost += kPsCost + tiles(j);
+  int whole = tiles(0) + kUncut;
+  if (jobs > streams) whole = std::max(whole, tiles(streams - 1) + tiles(streams) + 2 * kUncut);
+  if (jobs > 2 * streams) whole += tiles(2 * streams) + kUncut;
+  return ceil_div(cost, streams) + kCut + kLeastGain <= whole;
+}
+
 int launch_prefill_shared(const PrefillArgs& a, const PrefillCuts& cuts, hipStream_t stream) {
   const dim3 grid((unsigned)a.num_kv_heads, (unsigned)(cuts.whole + cuts.streams));
   const auto kernel = a.logit_cap > 0.f ? prefill_shared_kernel<true> : prefill_shared_kernel<false>;

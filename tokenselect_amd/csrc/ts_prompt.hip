@@ -437,7 +437,11 @@ static int prompt_group(const ts_config* cfg, int32_t rows, int32_t chunk_rows, 
 static bool prompt_cuts(const ts_config* cfg, int32_t rows, int32_t chunk_rows, int32_t max_seq_len) {
   const int most = prompt_group(cfg, rows, chunk_rows, max_seq_len);
   const int keys = std::min(cfg->n_init + cfg->top_k + cfg->n_local, max_seq_len);
-  return (prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, rows, rows, keys) ||
+  // The rows that are one dense chunk, and the keys of its last.
+  const int before = std::max(max_seq_len - rows, 0);
+  int dense = std::min(rows, std::max(keys - before, 0));
+  if (dense < rows) dense = dense / chunk_rows * chunk_rows;
+  return ((dense > 0 && prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, dense, dense, before + dense)) ||
           prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, rows, chunk_rows, keys)) &&
          prompt_workspace(cfg, most, max_seq_len, true).total <= std::max(kPrBytes, prompt_workspace(cfg, most, max_seq_len).total);
 }
@@ -546,7 +550,8 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     const int64_t row0 = (int64_t)first * chunk_rows;
     const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)std::min(merged, dense - first) * chunk_rows, rows - row0);
     const int32_t bound = bound_after(row0 + n_rows);
-    const PromptWorkspace w = prompt_workspace(cfg, 1, bound, cut);
+    const bool cut_here = cut && prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, n_rows, n_rows, bound);
+    const PromptWorkspace w = prompt_workspace(cfg, 1, bound, cut_here);
     PrefillDense all{};
     all.table = table;
     all.seq_len = seq_len;
@@ -557,7 +562,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     all.store = rows_at(row0, n_rows);
     TS_TRY(launch_prefill_attn(cfg, (const uint16_t*)q + row0 * q_stride, q_stride, n_rows, k_pool, v_pool, pool_rows,
                                all.sel, all.sel_len, bound, (uint16_t*)out + row0 * cfg->num_heads * cfg->head_dim,
-                               ws + w.stage, w.total - w.stage, st, &all, cut ? ws + w.votes : nullptr));
+                               ws + w.stage, w.total - w.stage, st, &all, cut_here ? ws + w.votes : nullptr));
   }
 
   if (dense == chunks) return TS_OK;
@@ -567,7 +572,10 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     const int64_t row0 = (int64_t)first * chunk_rows;
     const int32_t n_rows = (int32_t)std::min<int64_t>((int64_t)here * chunk_rows, rows - row0);
     const int32_t bound = bound_after(row0 + n_rows);
-    const PromptWorkspace w = prompt_workspace(cfg, here, bound, cut);
+    const int max_sel = cfg->n_init + cfg->top_k + cfg->n_local;
+    const bool cut_here =
+        cut && prefill_cuts_pay(cfg->num_heads, cfg->num_kv_heads, n_rows, std::min(chunk_rows, n_rows), max_sel);
+    const PromptWorkspace w = prompt_workspace(cfg, here, bound, cut_here);
     int32_t *const lens = (int32_t*)(ws + w.lens), *const sel = (int32_t*)(ws + w.sel),
                    *const sel_len = (int32_t*)(ws + w.sel_len);
     float *const votes = (float*)(ws + w.votes), *const pooled = cfg->pool_kernel > 0 ? (float*)(ws + w.pooled) : nullptr;
@@ -617,7 +625,7 @@ int ts_prefill_prompt(const ts_config* cfg, const ts_batch* bt, const ts_new_kv*
     TS_TRY(launch_prefill_attn_chunks(cfg, q0, q_stride, n_rows, std::min(chunk_rows, n_rows), k_pool, v_pool, pool_rows,
                                       sel, w.max_sel, sel_len, w.max_sel,
                                       (uint16_t*)out + row0 * cfg->num_heads * cfg->head_dim, ws + w.stage,
-                                      w.total - w.stage, st, nullptr, cut ? ws + w.votes : nullptr));
+                                      w.total - w.stage, st, nullptr, cut_here ? ws + w.votes : nullptr));
   }
   return TS_OK;
 }
